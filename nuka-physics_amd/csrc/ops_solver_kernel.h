@@ -780,6 +780,41 @@ __device__ __forceinline__ void add_head(const Tile& c, uint32_t h, bool coordin
     }
 }
 
+// The heads' curvature on the matrix cores, for blocks of at most 32 coordinates: H += sum over heads and axes of
+// (C J)_r^T J_r, four heads a pass.  The wavefront's four groups of sixteen lanes take a head each; a lane holds, for
+// its head, the three entries of a coordinate of every sixteen (column = lane & 15 of tile t), forms the entries of C J
+// from them and hands both to v_mfma_f32_16x16x4, whose four products of one instruction are the four heads.  Three
+// instructions (the axes) a tile and pass, T x T tiles.  The same loads give the heads' part of the force and its
+// rounding scale, in double, a partial sum a group.
+//   The block's rows need the tiles as lane = row, a register a column.  Tile (J, I) holds H[16 J + 4 g + r][16 I + x] in
+// register r of lane 16 g + x; H is symmetric, so that is entry 16 J + 4 g + r of row 16 I + x, and one exchange of lane
+// rows between tiles (J, 0) and (J, 1) (v_permlane16_swap) puts rows 0-15 and 16-31 side by side: g = 0 and 1 in the
+// lower half of the wavefront, g = 2 and 3 in the upper, which v_permlane32_swap brings down.
+//   Bound by the latency of one wave (LDS words of a pass, then the matrix instructions in line).  It takes the place of
+// a loop that added heads to register rows by broadcast reads of their Jacobian words, a head a pass with unit heads present
+// and two to four without: 1000 servo-driven quadrupeds, four steps, 2.58 -> 2.23 ms; 4096 walkers 1.06 -> 1.01 ms.
+typedef float Vec4 __attribute__((ext_vector_type(4)));
+template <int N>
+constexpr int kTileSpan = (N + 15) / 16;   // tiles of sixteen coordinates a side
+__device__ __forceinline__ float lane_permute(int source, float v) {   // v of lane `source`, a byte address (4 x lane)
+    return __int_as_float(__builtin_amdgcn_ds_bpermute(source, __float_as_int(v)));
+}
+// rows of sixteen lanes: {a0, b0, a2, b2} in a and {a1, b1, a3, b3} in b
+__device__ __forceinline__ void swap_lane_rows(float& a, float& b) {
+    const auto pair = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    a = __uint_as_float(pair[0]); b = __uint_as_float(pair[1]);
+}
+__device__ __forceinline__ void swap_lane_rows(double& a, double& b) {
+    const uint64_t x = uint64_t(__double_as_longlong(a)), y = uint64_t(__double_as_longlong(b));
+    const auto low = __builtin_amdgcn_permlane16_swap(uint32_t(x), uint32_t(y), false, false);
+    const auto high = __builtin_amdgcn_permlane16_swap(uint32_t(x >> 32u), uint32_t(y >> 32u), false, false);
+    a = __longlong_as_double((long long)((uint64_t(high[0]) << 32u) | uint64_t(low[0])));
+    b = __longlong_as_double((long long)((uint64_t(high[1]) << 32u) | uint64_t(low[1])));
+}
+// v[32 + (lane & 31)] in every lane
+__device__ __forceinline__ float upper_half(float v) {
+    return __uint_as_float(__builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false)[1]);
+}
 // v[lane & 31] + v[32 + (lane & 31)] in every lane: the two halves of the wavefront swapped against each other
 __device__ __forceinline__ float halves_sum(float v) {
     const auto pair = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
@@ -792,7 +827,82 @@ __device__ __forceinline__ double halves_sum(double v) {
     return __longlong_as_double((long long)((uint64_t(high[0]) << 32u) | uint64_t(low[0]))) +
            __longlong_as_double((long long)((uint64_t(high[1]) << 32u) | uint64_t(low[1])));
 }
+// lane = head on the way in (mf, mc, mn, my_first; `heads` the uniform mask of those to add), lane = row on return
+template <int N>
+__device__ __forceinline__ void add_heads_by_tiles(const Tile& c, uint64_t heads, const float (&mf)[3], const float (&mc)[6], const float (&mn)[3],
+                                                   uint32_t my_first, float (&hrow)[N], TileSum& g, float& scale) {
+    static_assert(N <= 32, "two tiles a side at most");
+    constexpr int T = kTileSpan<N>;
+    const uint32_t group = c.lane >> 4u, x = c.lane & 15u;
+    uint32_t column[T];
+#pragma unroll
+    for (int t = 0; t < T; ++t) column[t] = min(uint32_t(16 * t) + x, uint32_t(N - 1));   // (entries past the width are never read back)
+    Vec4 tile[T][T] = {};
+    double force[T] = {};
+    float bound[T] = {};
+    while (heads != 0ull) {
+        uint32_t mine = kInvalid;
+#pragma unroll
+        for (uint32_t k = 0u; k < 4u; ++k) {
+            const uint32_t h = heads != 0ull ? uint32_t(__builtin_ctzll(heads)) : kInvalid;
+            heads &= heads - 1ull;   // zero stays zero
+            mine = group == k ? h : mine;
+        }
+        const bool live = mine != kInvalid;
+        const int source = int((live ? mine : 0u) * 4u);
+        const float* rows = c.jac + uint32_t(__builtin_amdgcn_ds_bpermute(source, int(my_first))) * uint32_t(N);
+        float f[3], cv[6], noise[3];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) { f[k] = lane_permute(source, mf[k]); noise[k] = lane_permute(source, mn[k]); }
+#pragma unroll
+        for (int k = 0; k < 6; ++k) cv[k] = lane_permute(source, mc[k]);
+        float j[T][3], a[T][3];
+#pragma unroll
+        for (int t = 0; t < T; ++t) {
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                const float word = rows[uint32_t(k) * uint32_t(N) + column[t]];
+                j[t][k] = live ? word : 0.0f;
+            }
+            a[t][0] = fmaf(j[t][2], cv[4], fmaf(j[t][1], cv[3], j[t][0] * cv[0]));
+            a[t][1] = fmaf(j[t][2], cv[5], fmaf(j[t][0], cv[3], j[t][1] * cv[1]));
+            a[t][2] = fmaf(j[t][1], cv[5], fmaf(j[t][0], cv[4], j[t][2] * cv[2]));
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                force[t] = fma(double(j[t][k]), double(f[k]), force[t]);
+                bound[t] = fmaf(fabsf(j[t][k]), noise[k], bound[t]);
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < 3; ++k)
+#pragma unroll
+            for (int J = 0; J < T; ++J)
+#pragma unroll
+                for (int I = 0; I < T; ++I) tile[J][I] = __builtin_amdgcn_mfma_f32_16x16x4f32(j[J][k], a[I][k], tile[J][I], 0, 0, 0);
+    }
+#pragma unroll
+    for (int J = 0; J < T; ++J) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            if (16 * J + r >= N) continue;
+            float low = tile[J][0][r], high = tile[J][T - 1][r];
+            swap_lane_rows(low, high);
+            hrow[16 * J + r] += low;
+            if (16 * J + 4 + r < N) hrow[16 * J + 4 + r] += high;
+            if (16 * J + 8 + r < N) hrow[16 * J + 8 + r] += upper_half(low);
+            if (16 * J + 12 + r < N) hrow[16 * J + 12 + r] += upper_half(high);
+        }
+    }
+    double force_low = force[0], force_high = force[T - 1];
+    float bound_low = bound[0], bound_high = bound[T - 1];
+    swap_lane_rows(force_low, force_high); swap_lane_rows(bound_low, bound_high);
+    g.value += halves_sum(force_low + force_high);
+    scale += halves_sum(bound_low + bound_high);
+}
 
+// A reduced block adds its heads to register rows instead, in an order of its own (below): its worlds are robots on two
+// many-sphered feet, of which some do not converge within their sweeps, and an environment that has not converged hands
+// a last place of its Hessian on as the fourth decimal of its velocities.
 // Two heads in one pass, for blocks of at most 32 coordinates: lanes 0..31 add head `ha` to their rows, lanes 32..63
 // add head `hb` (kInvalid: none) to rows of their own that start at zero, row = lane & 31 in both halves; the caller
 // sums the halves afterwards (halves_sum).  A head's values come from its own lane (lane = head) through the lane
@@ -1384,151 +1494,123 @@ __device__ __forceinline__ bool assemble_block(const Tile& c, const float (&mrow
     TileSum g{-inertial.value};
     PROF_END(c, 11);
     PROF_BEGIN(c, 12);
-    bool paired = false, grouped = false;
-    if constexpr (N <= 32) {
-        // two or more contributing heads (all of them staged, one a lane): two a pass, the second half of the
-        // wavefront collecting its heads in rows of its own
-        const uint64_t all = __ballot(mine);
-        paired = !c.units && c.heads <= uint32_t(kWave) && (all & (all - 1ull)) != 0ull;
-        if constexpr (N <= 20 && N <= kTwoWaveWidth) {
-            // where three or four copies of the rows fit the wavefront, that many heads a pass - when it takes fewer
-            // passes than two a pass would (adding the groups' rows together costs more than adding two halves)
-            const int contributing = __popcll(all);
-            if (paired && (contributing + kGroups<N> - 1) / kGroups<N> < (contributing + 1) / 2) {
-                if (lane >= uint32_t(N)) {
-#pragma unroll
-                    for (int k = 0; k < N; ++k) hrow[k] = 0.0f;
-                    g.value = 0.0; scale = 0.0f;
-                }
-                const uint32_t my_first = lane < c.heads ? c.U(hRow, lane) : 0u;
-                for (uint64_t rest = all; rest != 0ull;) {
-                    uint32_t taken[4] = {kInvalid, kInvalid, kInvalid, kInvalid};
-#pragma unroll
-                    for (int k = 0; k < kGroups<N>; ++k) {
-                        if (rest == 0ull) break;
-                        taken[k] = uint32_t(__builtin_ctzll(rest));
-                        rest &= rest - 1ull;
-                    }
-                    add_head_group<N>(c, taken, mf, mc, mn, my_first, my_low, my_high, hrow, g, scale);
-                }
-#pragma unroll
-                for (int k = 0; k < N; ++k) hrow[k] = groups_sum<N>(lane, hrow[k]);
-                g.value = groups_sum<N>(lane, g.value); scale = groups_sum<N>(lane, scale);
-                grouped = true;
-            }
-        }
-        if (paired && !grouped) {
-            if (lane >= 32u) {
-#pragma unroll
-                for (int k = 0; k < N; ++k) hrow[k] = 0.0f;
-                g.value = 0.0; scale = 0.0f;
-            }
-            const uint32_t my_first = lane < c.heads ? c.U(hRow, lane) : 0u;
-            for (uint64_t rest = all; rest != 0ull;) {
-                const uint32_t ha = uint32_t(__builtin_ctzll(rest));
-                rest &= rest - 1ull;
-                const uint32_t hb = rest != 0ull ? uint32_t(__builtin_ctzll(rest)) : kInvalid;
-                rest &= rest - 1ull;   // zero stays zero
-                add_head_pair<N>(c, ha, hb, mf, mc, mn, my_first, my_low, my_high, hrow, g, scale);
-            }
-#pragma unroll
-            for (int k = 0; k < N; ++k) hrow[k] = halves_sum(hrow[k]);
-            g.value = halves_sum(g.value); scale = halves_sum(scale);
-        }
-    }
-    if (paired) {
-    } else if (N > kTwoWaveWidth && c.from_links) {
-        if (__ballot(mine) != 0ull) {
+    // heads beyond the first 64 hold their responses in the fields
+    auto add_later_head = [&](uint32_t h) {
+        const float f[3] = {c.F(hF, h), c.F(hF + 1, h), c.F(hF + 2, h)};
+        const float cv[6] = {c.F(hC, h), c.F(hC + 1, h), c.F(hC + 2, h), c.F(hC + 3, h), c.F(hC + 4, h), c.F(hC + 5, h)};
+        const float noise[3] = {c.F(hNoise, h), c.F(hNoise + 1, h), c.F(hNoise + 2, h)};
+        const uint64_t columns = (uint64_t(__builtin_amdgcn_readfirstlane(c.U(hColumnsHigh, h))) << 32u) |
+                                 uint64_t(__builtin_amdgcn_readfirstlane(c.U(hColumnsLow, h)));
+        add_head<N>(c, h, coordinate, f, cv, noise, c.U(hAxes, h), columns, hrow, g, scale);
+    };
+    // the staged ones of the first 64
+    const uint64_t staged = __ballot(mine && (!c.units || c.U(hUnit, lane) == kInvalid));
+    if (N > kTwoWaveWidth && c.from_links) {
+        if (staged != 0ull) {
             float weighted = 0.0f;
-            g.value += rows_transposed_times<true>(c, __ballot(mine), mf, mn, &weighted);
+            g.value += rows_transposed_times<true>(c, staged, mf, mn, &weighted);
             scale += weighted;
             add_heads_through_links<N>(c, mine, mc, hrow);
         }
-    } else if (N > kTwoWaveWidth && c.through_links && __popcll(__ballot(mine)) >= int(kLinkHeads)) {
+    } else if (N > kTwoWaveWidth && c.through_links && __popcll(staged) >= int(kLinkHeads)) {
         // enough heads that their curvature is cheaper by way of the links; the force takes the staged rows as ever
-        add_heads_force<N>(c, __ballot(mine), mf, mn, lane < c.heads ? c.U(hRow, lane) : 0u, g, scale);
+        add_heads_force<N>(c, staged, mf, mn, lane < c.heads ? c.U(hRow, lane) : 0u, g, scale);
         add_heads_through_links<N>(c, mine, mc, hrow);
-    } else if (!c.units) {   // staged heads only: plain head order
-        for (uint64_t rest = __ballot(mine); rest != 0ull; rest &= rest - 1ull) {
-            const uint32_t h = uint32_t(__builtin_ctzll(rest));
-            float f[3], cv[6], noise[3];
-#pragma unroll
-            for (int k = 0; k < 3; ++k) { f[k] = uniform_lane_value(mf[k], h); noise[k] = uniform_lane_value(mn[k], h); }
-#pragma unroll
-            for (int k = 0; k < 6; ++k) cv[k] = uniform_lane_value(mc[k], h);
-            const uint32_t axes = uint32_t(__builtin_amdgcn_readlane(int(my_axes), int(h)));
-            const uint64_t columns = (uint64_t(uint32_t(__builtin_amdgcn_readlane(int(my_high), int(h)))) << 32u) |
-                                     uint64_t(uint32_t(__builtin_amdgcn_readlane(int(my_low), int(h))));
-            add_head<N>(c, h, coordinate, f, cv, noise, axes, columns, hrow, g, scale);
-        }
-        for (uint32_t h = kWave; h < c.heads; ++h) {
-            if (c.U(hContrib, h) == 0u) continue;
-            const float f[3] = {c.F(hF, h), c.F(hF + 1, h), c.F(hF + 2, h)};
-            const float cv[6] = {c.F(hC, h), c.F(hC + 1, h), c.F(hC + 2, h), c.F(hC + 3, h), c.F(hC + 4, h), c.F(hC + 5, h)};
-            const float noise[3] = {c.F(hNoise, h), c.F(hNoise + 1, h), c.F(hNoise + 2, h)};
-            const uint64_t columns = (uint64_t(__builtin_amdgcn_readfirstlane(c.U(hColumnsHigh, h))) << 32u) |
-                                     uint64_t(__builtin_amdgcn_readfirstlane(c.U(hColumnsLow, h)));
-            add_head<N>(c, h, coordinate, f, cv, noise, c.U(hAxes, h), columns, hrow, g, scale);
-        }
     } else {
-        // The heads add in the reference's order (:1533-1603): 32 at a time, and within each 32 the unit heads - a row on
-        // one coordinate adds to that coordinate's diagonal and force only - before the staged ones.  Chunks past the
-        // last staged head hold unit heads only and go in one pass.
+        bool added = false;
+        if constexpr (N <= 32 && !kFollow) {
+            if (staged != 0ull) add_heads_by_tiles<N>(c, staged, mf, mc, mn, lane < c.heads ? c.U(hRow, lane) : 0u, hrow, g, scale);
+            added = true;
+        }
+        if constexpr (N <= 32 && kFollow) {
+            // two or more contributing heads (all of them staged, one a lane): two a pass, the second half of the
+            // wavefront collecting its heads in rows of its own
+            if ((staged & (staged - 1ull)) != 0ull) {
+                const uint32_t my_first = lane < c.heads ? c.U(hRow, lane) : 0u;
+                if constexpr (N <= 20) {
+                    // where three or four copies of the rows fit the wavefront, that many heads a pass - when it takes fewer
+                    // passes than two a pass would (adding the groups' rows together costs more than adding two halves)
+                    const int contributing = __popcll(staged);
+                    if ((contributing + kGroups<N> - 1) / kGroups<N> < (contributing + 1) / 2) {
+                        if (lane >= uint32_t(N)) {
+#pragma unroll
+                            for (int k = 0; k < N; ++k) hrow[k] = 0.0f;
+                            g.value = 0.0; scale = 0.0f;
+                        }
+                        for (uint64_t rest = staged; rest != 0ull;) {
+                            uint32_t taken[4] = {kInvalid, kInvalid, kInvalid, kInvalid};
+#pragma unroll
+                            for (int k = 0; k < kGroups<N>; ++k) {
+                                if (rest == 0ull) break;
+                                taken[k] = uint32_t(__builtin_ctzll(rest));
+                                rest &= rest - 1ull;
+                            }
+                            add_head_group<N>(c, taken, mf, mc, mn, my_first, my_low, my_high, hrow, g, scale);
+                        }
+#pragma unroll
+                        for (int k = 0; k < N; ++k) hrow[k] = groups_sum<N>(lane, hrow[k]);
+                        g.value = groups_sum<N>(lane, g.value); scale = groups_sum<N>(lane, scale);
+                        added = true;
+                    }
+                }
+                if (!added) {
+                    if (lane >= 32u) {
+#pragma unroll
+                        for (int k = 0; k < N; ++k) hrow[k] = 0.0f;
+                        g.value = 0.0; scale = 0.0f;
+                    }
+                    for (uint64_t rest = staged; rest != 0ull;) {
+                        const uint32_t ha = uint32_t(__builtin_ctzll(rest));
+                        rest &= rest - 1ull;
+                        const uint32_t hb = rest != 0ull ? uint32_t(__builtin_ctzll(rest)) : kInvalid;
+                        rest &= rest - 1ull;   // zero stays zero
+                        add_head_pair<N>(c, ha, hb, mf, mc, mn, my_first, my_low, my_high, hrow, g, scale);
+                    }
+#pragma unroll
+                    for (int k = 0; k < N; ++k) hrow[k] = halves_sum(hrow[k]);
+                    g.value = halves_sum(g.value); scale = halves_sum(scale);
+                    added = true;
+                }
+            }
+        }
+        if (!added) {
+            for (uint64_t rest = staged; rest != 0ull; rest &= rest - 1ull) {
+                const uint32_t h = uint32_t(__builtin_ctzll(rest));
+                float f[3], cv[6], noise[3];
+#pragma unroll
+                for (int k = 0; k < 3; ++k) { f[k] = uniform_lane_value(mf[k], h); noise[k] = uniform_lane_value(mn[k], h); }
+#pragma unroll
+                for (int k = 0; k < 6; ++k) cv[k] = uniform_lane_value(mc[k], h);
+                const uint32_t axes = uint32_t(__builtin_amdgcn_readlane(int(my_axes), int(h)));
+                const uint64_t columns = (uint64_t(uint32_t(__builtin_amdgcn_readlane(int(my_high), int(h)))) << 32u) |
+                                         uint64_t(uint32_t(__builtin_amdgcn_readlane(int(my_low), int(h))));
+                add_head<N>(c, h, coordinate, f, cv, noise, axes, columns, hrow, g, scale);
+            }
+        }
+        for (uint32_t h = kWave; h < (c.units ? c.staged_end : c.heads); ++h) {
+            if (c.U(hContrib, h) == 0u || (c.units && c.U(hUnit, h) != kInvalid)) continue;
+            add_later_head(h);
+        }
+    }
+    if (c.units) {
+        // a unit head - a row on one coordinate - adds to that coordinate's diagonal and force only: lane = coordinate walks
+        // its own short list, or, when some coordinate's list overflowed, the wave walks every unit head in turn
         float diagonal = 0.0f;
-        uint32_t next = 0u;
-        const uint64_t contributing = __ballot(mine);
-        const uint64_t unit_heads = __ballot(lane < c.heads && c.U(hUnit, lane) != kInvalid);
         auto add_unit = [&](uint32_t h) {
             const float v = c.F(hUnitValue, h);
             diagonal += v * c.F(hC, h) * v;
             tile_add_product(g, v, c.F(hF, h));
             scale += fabsf(v) * c.F(hNoise, h);
         };
-        // unit heads below `below`: lane = coordinate walks its own short list, or, when some coordinate's list
-        // overflowed, the wave walks every unit head in turn
-        auto add_units = [&](uint32_t from, uint32_t below) {
-            if (c.unit_lists) {
-                while (next < c.unit_count) {
-                    const uint32_t h = c.unit_list[next * uint32_t(kWave) + lane];
-                    if (h >= below) break;
-                    ++next;
-                    if (c.U(hContrib, h) != 0u) add_unit(h);
-                }
-                return;
+        if (c.unit_lists) {
+            for (uint32_t k = 0u; k < c.unit_count; ++k) {
+                const uint32_t h = c.unit_list[k * uint32_t(kWave) + lane];
+                if (c.U(hContrib, h) != 0u) add_unit(h);
             }
-            for (uint32_t h = from; h < below; ++h)
+        } else {
+            for (uint32_t h = 0u; h < c.heads; ++h)
                 if (c.U(hContrib, h) != 0u && c.U(hUnit, h) == lane) add_unit(h);
-        };
-        for (uint32_t chunk = 0u; chunk < c.staged_end; chunk += 32u) {
-            const uint32_t end = min(chunk + 32u, c.heads);
-            add_units(chunk, end);
-            if (chunk < uint32_t(kWave)) {
-                for (uint64_t rest = contributing & ~unit_heads & (0xFFFFFFFFull << chunk); rest != 0ull; rest &= rest - 1ull) {
-                    const uint32_t h = uint32_t(__builtin_ctzll(rest));
-                    float f[3], cv[6], noise[3];
-#pragma unroll
-                    for (int k = 0; k < 3; ++k) { f[k] = uniform_lane_value(mf[k], h); noise[k] = uniform_lane_value(mn[k], h); }
-#pragma unroll
-                    for (int k = 0; k < 6; ++k) cv[k] = uniform_lane_value(mc[k], h);
-                    const uint32_t axes = uint32_t(__builtin_amdgcn_readlane(int(my_axes), int(h)));
-                    const uint64_t columns = (uint64_t(uint32_t(__builtin_amdgcn_readlane(int(my_high), int(h)))) << 32u) |
-                                             uint64_t(uint32_t(__builtin_amdgcn_readlane(int(my_low), int(h))));
-                    add_head<N>(c, h, coordinate, f, cv, noise, axes, columns, hrow, g, scale);
-                }
-            } else {
-                for (uint32_t h = chunk; h < end; ++h) {
-                    if (c.U(hContrib, h) == 0u || c.U(hUnit, h) != kInvalid) continue;
-                    const float f[3] = {c.F(hF, h), c.F(hF + 1, h), c.F(hF + 2, h)};
-                    const float cv[6] = {c.F(hC, h), c.F(hC + 1, h), c.F(hC + 2, h), c.F(hC + 3, h), c.F(hC + 4, h), c.F(hC + 5, h)};
-                    const float noise[3] = {c.F(hNoise, h), c.F(hNoise + 1, h), c.F(hNoise + 2, h)};
-                    const uint64_t columns = (uint64_t(__builtin_amdgcn_readfirstlane(c.U(hColumnsHigh, h))) << 32u) |
-                                             uint64_t(__builtin_amdgcn_readfirstlane(c.U(hColumnsLow, h)));
-                    add_head<N>(c, h, coordinate, f, cv, noise, c.U(hAxes, h), columns, hrow, g, scale);
-                }
-            }
         }
-        add_units((c.staged_end + 31u) & ~31u, c.heads);
-        // the unit heads' curvature lands on the diagonal after every staged head (:1605-1606)
 #pragma unroll
         for (int k = 0; k < N; ++k) hrow[k] += local_lane(lane) == uint32_t(k) ? diagonal : 0.0f;
     }
@@ -2368,6 +2450,10 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
         if (points < points_lo || points > points_hi) return;
     }
     const uint32_t R = p.rows_per_env, md = p.max_dof, n = m.dof, nl = m.links_per_env, S = p.contact_slots_per_env;
+    // A narrow block would leave registers free and let more waves share a SIMD than the launch is sized for; one name of
+    // the last register holds the kernel to its two (dense build: three) waves.
+    if constexpr (WavesPerSimd(W) == 3) asm volatile("" ::: "v163");
+    else if constexpr (WavesPerSimd(W) == 2) asm volatile("" ::: "v255");
     Tile c;
     c.env = env; c.lane = lane; c.n = kReduced ? uint32_t(K) : n; c.n_all = n; c.ldj = uint32_t(W); c.cap = cap; c.narrow = staged_cap; c.heads = 0u; c.iteration = 0u;
     c.tolerance = p.velocity_tolerance; c.failed = false; c.momentum = 0.0f; c.residual = 0.0f;
