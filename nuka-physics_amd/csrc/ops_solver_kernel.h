@@ -303,6 +303,7 @@ struct Tile {
     float* fields;   // cap x kWideStride, then (narrow + 1) x kNarrowStride
     float* vec;      // 4 x 64 scratch vectors, 16-byte aligned
     float mass_inverse;   // 1 / diagonal of the mass factor, lane = row
+    mutable float factor_root;       // the diagonal of that factor, lane = row
     mutable bool factor_current;     // no head's curvature has changed since hfac was factored: the Hessian is the same
     mutable uint32_t work;   // Newton steps and line probes of this solve, the next solve's scheduling key
     bool mass_valid;
@@ -368,23 +369,26 @@ __device__ __forceinline__ void head_response(const Tile& c, uint32_t h, float m
 __device__ __forceinline__ float pivot_scale(float pivot) { return __builtin_amdgcn_rsqf(pivot); }
 
 // FactorTileBlock (:1622-1645) on register rows: lane i holds row i of the symmetric matrix; on return its entries
-// k <= i are row i of the Cholesky factor.  Element (i, j) loses L_ik L_jk for k = 0, 1, ... in that order, as the
-// reference's serial inner loop does; each product and subtraction is one fused multiply-add (the reference is
-// built with its compiler's default contraction, so it fuses these too).  Uniform result: false on a bad pivot.
+// k < i are row i of the strict lower triangle of the Cholesky factor and every other entry is zero, so that a
+// substitution takes each entry without a condition; the diagonal is `root`, with `inverse` the scale its pivot gave.
+// Element (i, j) loses L_ik L_jk for k = 0, 1, ... in that order, as the reference's serial inner loop does; each product
+// and subtraction is one fused multiply-add (the reference is built with its compiler's default contraction, so it fuses
+// these too).  A pivot that is not positive and finite gives a scale that is not: one look at the scales at the end
+// (uniform result, false on a bad pivot) instead of a test a pivot.  A lane takes the scale of every pivot up to its
+// own and keeps the last, so one comparison a pivot serves the mask and, a pivot later, the diagonal.
+__device__ __forceinline__ bool pivots_valid(uint32_t lane, uint32_t N, float inverse) {
+    return __all(lane >= N || (inverse > 0.0f && inverse <= FLT_MAX));
+}
 template <int N>
-__device__ __forceinline__ bool factor_rows(uint32_t lane, float (&row)[N], float* inverse_out) {
+__device__ __forceinline__ bool factor_rows(uint32_t lane, float (&row)[N], float* inverse_out, float* root_out) {
     lane = local_lane(lane);
-    bool valid = true;
-    float inverse = 0.0f;
+    float inverse = 0.0f, root = 0.0f;
 #pragma unroll
     for (int k = 0; k < N; ++k) {
-        // the pivot's square root and reciprocal
-        const float pivot = lane_value(row[k], k);
-        valid = valid && pivot > 0.0f && pivot <= FLT_MAX;
-        const float scale = pivot_scale(valid ? pivot : 1.0f);
-        const float root = pivot * scale;
-        row[k] = lane == uint32_t(k) ? root : row[k] * scale;
-        if (lane == uint32_t(k)) inverse = scale;
+        const float scale = pivot_scale(lane_value(row[k], k));
+        const float scaled = row[k] * scale;
+        if (lane >= uint32_t(k)) { inverse = scale; root = scaled; }
+        row[k] = lane > uint32_t(k) ? scaled : 0.0f;
         // lane reads in batches of eight ahead of their multiply-adds: a scalar read has to settle for two cycles
         // before an arithmetic instruction may use it, and the next reads fill that gap
 #pragma unroll
@@ -397,8 +401,8 @@ __device__ __forceinline__ bool factor_rows(uint32_t lane, float (&row)[N], floa
                 if (j0 + t < N) row[j0 + t] = fmaf(-row[k], l[t], row[j0 + t]);
         }
     }
-    *inverse_out = inverse;
-    return valid;
+    *inverse_out = inverse; *root_out = root;
+    return pivots_valid(lane, uint32_t(N), inverse);
 }
 
 // Past 32 coordinates the reference's tile is "wide" (TileSpan > 1, :71-73) and factors H = U U^T from the last
@@ -408,35 +412,32 @@ __device__ __forceinline__ bool factor_rows(uint32_t lane, float (&row)[N], floa
 template <int N>
 constexpr bool kLeavesFirst = N > 32;
 
-// Where a factor is kept for its transposed reads.  Root first: rows of N + 1 words.  Leaves first: lane i's row of
-// U holds the entries k >= i only, and the rows are packed - row i starts at i N - i (i - 1) / 2 and is N - i words
-// long - which halves the storage; a column's words for consecutive lanes are consecutive.
-__host__ __device__ constexpr uint32_t FactorFloats(uint32_t N) { return N > 32u ? (N * (N + 1u) / 2u + 3u) & ~3u : N * (N + 1u); }
+// Where a factor is kept for its transposed reads, the diagonal's place holding zero.  Root first: rows of N words, moved
+// sixteen bytes at a time.  Leaves first: lane i's row of U holds the entries k >= i only, and the rows are packed - row i
+// starts at i N - i (i - 1) / 2 and is N - i words long - which halves the storage; a column's words for consecutive
+// lanes are consecutive.
+__host__ __device__ constexpr uint32_t FactorFloats(uint32_t N) { return N > 32u ? (N * (N + 1u) / 2u + 3u) & ~3u : N * N; }
 template <int N>
 __device__ __forceinline__ uint32_t factor_at(uint32_t i, uint32_t k) {   // leaves first: k >= i
     if constexpr (kLeavesFirst<N>) return i * uint32_t(N) - (i * (i - 1u)) / 2u + (k - i);
-    else return i * uint32_t(N + 1) + k;
+    else return i * uint32_t(N) + k;
 }
 
-// FactorTileColumns on register rows: lane i holds row i of the symmetric matrix; on return its entries k >= i are
-// row i of U.  Column k leaves exact zeros in the rows of other branches of the tree, and the update of a column by
-// an exact zero changes nothing: such columns are skipped four at a time.
-// With kStop > 0 the elimination ends after pivot kStop: rows and columns below it then hold the Schur complement of the
-// eliminated coordinates, rows below it hold their coupling to them in the columns from kStop on.
-template <int N, int kStop = 0>
-__device__ __forceinline__ bool factor_rows_up(uint32_t lane, float (&row)[N], float* inverse_out) {
+// FactorTileColumns on register rows: lane i holds row i of the symmetric matrix; on return its entries k > i are
+// row i of U, every other entry is zero, and `root` is the diagonal.  Column k leaves exact zeros in the rows of other
+// branches of the tree, and the update of a column by an exact zero changes nothing: such columns are skipped four at a
+// time.
+template <int N>
+__device__ __forceinline__ bool factor_rows_up(uint32_t lane, float (&row)[N], float* inverse_out, float* root_out) {
     lane = local_lane(lane);
-    bool valid = true;
-    float inverse = 0.0f;
+    float inverse = 0.0f, root = 0.0f;
 #pragma unroll
-    for (int k = N - 1; k >= kStop; --k) {
-        const float pivot = lane_value(row[k], k);
-        valid = valid && pivot > 0.0f && pivot <= FLT_MAX;
-        const float scale = pivot_scale(valid ? pivot : 1.0f);
-        const float root = pivot * scale;
-        row[k] = lane == uint32_t(k) ? root : row[k] * scale;
-        if (lane == uint32_t(k)) inverse = scale;
-        const uint64_t reach = __ballot(lane < uint32_t(k) && row[k] != 0.0f);
+    for (int k = N - 1; k >= 0; --k) {
+        const float scale = pivot_scale(lane_value(row[k], k));
+        const float scaled = row[k] * scale;
+        if (lane <= uint32_t(k)) { inverse = scale; root = scaled; }
+        row[k] = lane < uint32_t(k) ? scaled : 0.0f;
+        const uint64_t reach = __ballot(row[k] != 0.0f);
 #pragma unroll
         for (int q = (k - 1) / 4; q >= 0 && k >= 1; --q) {
             if (((reach >> (4 * q)) & 0xFull) == 0ull) continue;
@@ -448,79 +449,82 @@ __device__ __forceinline__ bool factor_rows_up(uint32_t lane, float (&row)[N], f
                 if (4 * q + t <= k - 1) row[4 * q + t] = fmaf(-row[k], u[t], row[4 * q + t]);
         }
     }
-    *inverse_out = inverse;
-    return valid;
+    *inverse_out = inverse; *root_out = root;
+    return pivots_valid(lane, uint32_t(N), inverse);
 }
 
 // SolveWideTileBlock: U w = g with lane's own row (entries right of the diagonal), then U^T d = w with the columns,
-// read from the factor in LDS eight at a time.
+// read from the factor in LDS eight at a time.  The rows hold zeros from the diagonal on, so no step asks which lanes it
+// is for: a lane whose entry is final loses an exact zero.
 template <int N>
 __device__ __forceinline__ float substitute_up(uint32_t lane, const float (&row)[N], const float* factor, float inverse, float g) {
     lane = local_lane(lane);
     float r = g;
 #pragma unroll
-    for (int j = N - 1; j >= 0; --j) {
-        const float y = lane_value(r * inverse, j);
-        r = lane < uint32_t(j) ? fmaf(-row[j], y, r) : r;
-    }
+    for (int j = N - 1; j >= 0; --j) r = fmaf(-row[j], lane_value(r * inverse, j), r);
     r *= inverse;
     const uint32_t mine = lane < uint32_t(N) ? lane : 0u;
 #pragma unroll
     for (int j0 = 0; j0 < N; j0 += 8) {
         float u[8];
 #pragma unroll
-        for (int t = 0; t < 8; ++t)   // U[j][lane] for the lanes past j; the others read a word they do not use
+        for (int t = 0; t < 8; ++t)   // U[j][lane] for the lanes past j; the others read the first diagonal's word, a zero
             u[t] = j0 + t < N ? factor[mine >= uint32_t(j0 + t) ? factor_at<N>(uint32_t(j0 + t), mine) : 0u] : 0.0f;
 #pragma unroll
-        for (int t = 0; t < 8; ++t) {
-            if (j0 + t >= N) continue;
-            const float x = lane_value(r * inverse, j0 + t);
-            r = lane > uint32_t(j0 + t) && lane < uint32_t(N) ? fmaf(-u[t], x, r) : r;
-        }
+        for (int t = 0; t < 8; ++t)
+            if (j0 + t < N) r = fmaf(-u[t], lane_value(r * inverse, j0 + t), r);
     }
     return r * inverse;
 }
 
-// SolveTileBlock (:1647-1666): forward with the factor's rows, backward with its columns (col[j] = L_j,lane).
+// SolveTileBlock (:1647-1666): forward with the factor's rows, backward with its columns (col[j] = L_j,lane), both zero
+// from the diagonal on.
 template <int N>
-__device__ __forceinline__ float substitute(uint32_t lane, const float (&row)[N], const float (&col)[N], float inverse, float g) {
+__device__ __forceinline__ float substitute(const float (&row)[N], const float (&col)[N], float inverse, float g) {
     // Lane j's entry is final once the steps before it have run, so it is scaled by its reciprocal pivot where it is
     // read (the same product that would be stored back) and the lanes take it in one multiplication after the sweep.
-    lane = local_lane(lane);
     float r = g;
 #pragma unroll
-    for (int j = 0; j < N; ++j) {
-        const float y = lane_value(r * inverse, j);
-        r = lane > uint32_t(j) ? fmaf(-row[j], y, r) : r;
-    }
+    for (int j = 0; j < N; ++j) r = fmaf(-row[j], lane_value(r * inverse, j), r);
     r *= inverse;
 #pragma unroll
-    for (int j = N - 1; j >= 0; --j) {
-        const float x = lane_value(r * inverse, j);
-        r = lane < uint32_t(j) ? fmaf(-col[j], x, r) : r;
-    }
+    for (int j = N - 1; j >= 0; --j) r = fmaf(-col[j], lane_value(r * inverse, j), r);
     return r * inverse;
 }
 
 template <int N>
 __device__ __forceinline__ void store_rows(float* a, uint32_t lane, const float (&row)[N]) {
     lane = local_lane(lane);
-    if (lane < uint32_t(N)) {
+    if (lane >= uint32_t(N)) return;
+    if constexpr (kLeavesFirst<N>) {
 #pragma unroll
         for (int k = 0; k < N; ++k)
-            if (!kLeavesFirst<N> || uint32_t(k) >= lane) a[factor_at<N>(lane, uint32_t(k))] = row[k];
+            if (uint32_t(k) >= lane) a[factor_at<N>(lane, uint32_t(k))] = row[k];
+    } else {
+        float4* words = reinterpret_cast<float4*>(a + lane * uint32_t(N));
+#pragma unroll
+        for (int q = 0; q < N / 4; ++q) words[q] = float4{row[4 * q], row[4 * q + 1], row[4 * q + 2], row[4 * q + 3]};
     }
 }
-// (Every word is read whether or not the lane keeps it - a read under a condition compiles to a branch a word - from
-// a place inside the factor: a lane past the rows reads the last row's, and a packed row's words left of its diagonal
-// fall in the rows before it.)
+// (A packed row's words are read whether or not the lane keeps them - a read under a condition compiles to a branch a
+// word - from a place inside the factor: a lane past the rows reads the last row's, and a packed row's words left of its
+// diagonal fall in the rows before it.)
 template <int N>
 __device__ __forceinline__ void load_rows(const float* a, uint32_t lane, float (&row)[N]) {
     lane = local_lane(lane);
     const uint32_t from = lane < uint32_t(N) ? lane : uint32_t(N - 1);
+    if constexpr (!kLeavesFirst<N>) {
+        const float4* words = reinterpret_cast<const float4*>(a + from * uint32_t(N));
+#pragma unroll
+        for (int q = 0; q < N / 4; ++q) {
+            const float4 w = words[q];
+            row[4 * q] = w.x; row[4 * q + 1] = w.y; row[4 * q + 2] = w.z; row[4 * q + 3] = w.w;
+        }
+        return;
+    }
 #pragma unroll
     for (int k = 0; k < N; ++k) {
-        const bool kept = lane < uint32_t(N) && (!kLeavesFirst<N> || uint32_t(k) >= lane);
+        const bool kept = lane < uint32_t(N) && uint32_t(k) >= lane;
         if constexpr (N > kTwoWaveWidth) {   // such a block's mass factor is in device memory: only the words that are kept
             row[k] = kept ? a[factor_at<N>(lane, uint32_t(k))] : 0.0f;
         } else {
@@ -534,21 +538,17 @@ __device__ __forceinline__ void load_columns(const float* a, uint32_t lane, floa
     lane = local_lane(lane);
     const uint32_t from = lane < uint32_t(N) ? lane : uint32_t(N - 1);
 #pragma unroll
-    for (int j = 0; j < N; ++j) {
-        const float word = a[j * (N + 1) + from];
-        col[j] = lane < uint32_t(N) ? word : 0.0f;
-    }
+    for (int j = 0; j < N; ++j) col[j] = a[uint32_t(j) * uint32_t(N) + from];
 }
 
 // Cholesky of the Newton Hessian held in `hrow`, then d = H^-1 g.  The factor passes through LDS once, for the
 // transposed read of the backward substitution.
 template <int N>
 __device__ __forceinline__ bool cholesky_solve(const Tile& c, float (&hrow)[N], float g, float* d_out) {
-    const uint32_t row = local_lane(c.lane);
     float inverse = 0.0f;
     if (!c.factor_current) {   // otherwise the Hessian is the one factored last: its factor is still in hfac
         PROF_BEGIN(c, 14);
-        const bool valid = kLeavesFirst<N> ? factor_rows_up<N>(c.lane, hrow, &inverse) : factor_rows<N>(c.lane, hrow, &inverse);
+        const bool valid = kLeavesFirst<N> ? factor_rows_up<N>(c.lane, hrow, &inverse, &c.factor_root) : factor_rows<N>(c.lane, hrow, &inverse, &c.factor_root);
         PROF_END(c, 14);
         if (!valid) return false;
         PROF_BEGIN(c, 24);
@@ -558,9 +558,8 @@ __device__ __forceinline__ bool cholesky_solve(const Tile& c, float (&hrow)[N], 
         c.factor_current = true;
     } else {
         PROF_COUNT(c, 3);
-        // rows and the reciprocal diagonal come back from hfac (the factor's own reciprocal is 1 / its diagonal
-        // entry, the same division)
-        inverse = row < uint32_t(N) ? 1.0f / c.hfac[factor_at<N>(row, row)] : 0.0f;
+        // the rows come back from hfac; the reciprocal of the diagonal is its quotient
+        inverse = 1.0f / c.factor_root;
         load_rows<N>(c.hfac, c.lane, hrow);
     }
     PROF_BEGIN(c, 15);
@@ -569,7 +568,7 @@ __device__ __forceinline__ bool cholesky_solve(const Tile& c, float (&hrow)[N], 
     } else {
         float col[N];
         load_columns<N>(c.hfac, c.lane, col);
-        *d_out = substitute<N>(c.lane, hrow, col, inverse, c.lane < c.n ? g : 0.0f);
+        *d_out = substitute<N>(hrow, col, inverse, c.lane < c.n ? g : 0.0f);
     }
     __syncthreads();
     PROF_END(c, 15);
@@ -583,8 +582,8 @@ __device__ __forceinline__ bool factor_mass(Tile& c, const float (&mrow)[N]) {
     float row[N];
 #pragma unroll
     for (int k = 0; k < N; ++k) row[k] = mrow[k];
-    float inverse = 0.0f;
-    const bool valid = kLeavesFirst<N> ? factor_rows_up<N>(c.lane, row, &inverse) : factor_rows<N>(c.lane, row, &inverse);
+    float inverse = 0.0f, root = 0.0f;
+    const bool valid = kLeavesFirst<N> ? factor_rows_up<N>(c.lane, row, &inverse, &root) : factor_rows<N>(c.lane, row, &inverse, &root);
     c.mass_inverse = inverse;
     store_rows<N>(c.mfac, c.lane, row);
     __syncthreads();
@@ -597,7 +596,7 @@ __device__ __forceinline__ float solve_tile_mass(const Tile& c, float force) {
     if constexpr (kLeavesFirst<N>) return substitute_up<N>(c.lane, row, c.mfac, c.mass_inverse, c.lane < c.n ? force : 0.0f);
     float col[N];
     load_columns<N>(c.mfac, c.lane, col);
-    return substitute<N>(c.lane, row, col, c.mass_inverse, c.lane < c.n ? force : 0.0f);
+    return substitute<N>(row, col, c.mass_inverse, c.lane < c.n ? force : 0.0f);
 }
 
 // The LDS byte address of a pointer into the block's shared memory.
@@ -1618,18 +1617,20 @@ __device__ __forceinline__ bool assemble_block(const Tile& c, const float (&mrow
     PROF_BEGIN(c, 13);
     *force = coordinate ? float(g.value) : 0.0f;
     *inertia = coordinate ? float(inertial.value) : 0.0f;
-    bool finite = isfinite(*force);
     const float4* u4 = reinterpret_cast<const float4*>(uvec);
 #pragma unroll
     for (int q = 0; q < N / 4; ++q) {
         const float4 uv = u4[q];
         const float uk[4] = {uv.x, uv.y, uv.z, uv.w};
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
-            const float entry = hrow[4 * q + t];
-            finite = finite && isfinite(entry);
-            scale += fabsf(entry) * uk[t];
-        }
+        for (int t = 0; t < 4; ++t) scale += fabsf(hrow[4 * q + t]) * uk[t];
+    }
+    // a row entry that is not finite leaves its scale not finite: the entries themselves are looked at only then
+    bool finite = isfinite(*force) && isfinite(scale);
+    if (!__all(!coordinate || finite)) {
+        finite = isfinite(*force);
+#pragma unroll
+        for (int k = 0; k < N; ++k) finite = finite && isfinite(hrow[k]);
     }
     *converged = __all(!coordinate || fabsf(*force) <= kRoundings * FLT_EPSILON * scale);
     const bool ok = __all(!coordinate || finite);
@@ -2458,7 +2459,7 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
     c.env = env; c.lane = lane; c.n = kReduced ? uint32_t(K) : n; c.n_all = n; c.ldj = uint32_t(W); c.cap = cap; c.narrow = staged_cap; c.heads = 0u; c.iteration = 0u;
     c.tolerance = p.velocity_tolerance; c.failed = false; c.momentum = 0.0f; c.residual = 0.0f;
     c.mass_inverse = 0.0f; c.mass_valid = false; c.work = 0u; c.units = false; c.elliptic = false;
-    c.factor_current = false;
+    c.factor_current = false; c.factor_root = 1.0f;
 #ifdef NKH_SOLVER_PROFILE
     for (int i = 0; i < 32; ++i) c.prof[i] = 0;
     for (int i = 0; i < 4; ++i) c.prof_count[i] = 0u;
