@@ -125,6 +125,15 @@ __device__ __forceinline__ float wave_total(TileSum s, bool first_row_only = fal
     if (first_row_only) return float(a);
     return float((a + row_value_d(v, 1)) + (row_value_d(v, 2) + row_value_d(v, 3)));
 }
+// the same where only the first N lanes carry terms: the rows past them would add exact zeros
+template <int N>
+__device__ __forceinline__ float coordinate_total(TileSum s) {
+    const double v = row_total_d(s.value);
+    const double first = row_value_d(v, 0);
+    if constexpr (N <= 16) return float(first);
+    else if constexpr (N <= 32) return float(first + row_value_d(v, 1));
+    else return float((first + row_value_d(v, 1)) + (row_value_d(v, 2) + row_value_d(v, 3)));
+}
 __device__ __forceinline__ float first_row_sum(float v) {
     v += dpp_move<kDppXor1>(v); v += dpp_move<kDppXor2>(v); v += dpp_move<kDppHalfMirror>(v); v += dpp_move<kDppMirror>(v);
     return row_value(v, 0);
@@ -303,6 +312,7 @@ struct Tile {
     float* fields;   // cap x kWideStride, then (narrow + 1) x kNarrowStride
     float* vec;      // 4 x 64 scratch vectors, 16-byte aligned
     float mass_inverse;   // 1 / diagonal of the mass factor, lane = row
+    mutable float curvature[6];      // of lane's own head at the last assembly
     mutable float factor_root;       // the diagonal of that factor, lane = row
     mutable bool factor_current;     // no head's curvature has changed since hfac was factored: the Hessian is the same
     mutable uint32_t work;   // Newton steps and line probes of this solve, the next solve's scheduling key
@@ -461,7 +471,7 @@ __device__ __forceinline__ float substitute_up(uint32_t lane, const float (&row)
     lane = local_lane(lane);
     float r = g;
 #pragma unroll
-    for (int j = N - 1; j >= 0; --j) r = fmaf(-row[j], lane_value(r * inverse, j), r);
+    for (int j = N - 1; j >= 0; --j) r = fmaf(row[j], -lane_value(r * inverse, j), r);
     r *= inverse;
     const uint32_t mine = lane < uint32_t(N) ? lane : 0u;
 #pragma unroll
@@ -472,7 +482,7 @@ __device__ __forceinline__ float substitute_up(uint32_t lane, const float (&row)
             u[t] = j0 + t < N ? factor[mine >= uint32_t(j0 + t) ? factor_at<N>(uint32_t(j0 + t), mine) : 0u] : 0.0f;
 #pragma unroll
         for (int t = 0; t < 8; ++t)
-            if (j0 + t < N) r = fmaf(-u[t], lane_value(r * inverse, j0 + t), r);
+            if (j0 + t < N) r = fmaf(u[t], -lane_value(r * inverse, j0 + t), r);
     }
     return r * inverse;
 }
@@ -485,10 +495,10 @@ __device__ __forceinline__ float substitute(const float (&row)[N], const float (
     // read (the same product that would be stored back) and the lanes take it in one multiplication after the sweep.
     float r = g;
 #pragma unroll
-    for (int j = 0; j < N; ++j) r = fmaf(-row[j], lane_value(r * inverse, j), r);
+    for (int j = 0; j < N; ++j) r = fmaf(row[j], -lane_value(r * inverse, j), r);
     r *= inverse;
 #pragma unroll
-    for (int j = N - 1; j >= 0; --j) r = fmaf(-col[j], lane_value(r * inverse, j), r);
+    for (int j = N - 1; j >= 0; --j) r = fmaf(col[j], -lane_value(r * inverse, j), r);
     return r * inverse;
 }
 
@@ -1169,15 +1179,22 @@ constexpr bool kKeepLine = N <= 24 || N > kTwoWaveWidth;
 __device__ __forceinline__ PlainLine own_line(const Tile& c) {
     return plain_line(load_head_line(c, c.heads <= 16u ? (c.lane & 15u) : c.lane));
 }
+// (read whether or not the lane has a head, from the first one's place then, and taken as zero: a read under a condition
+// compiles to a branch)
 __device__ __forceinline__ void refresh_moves(const Tile& c, PlainLine& p) {
-    if (p.head == kInvalid) return;
+    const bool live = p.head != kInvalid;
+    const uint32_t h = live ? p.head : 0u;
 #pragma unroll
-    for (int k = 0; k < 3; ++k) p.move[k] = c.F(hMove + k, p.head);
+    for (int k = 0; k < 3; ++k) { const float move = c.F(hMove + k, h); p.move[k] = live ? move : 0.0f; }
 }
 __device__ __forceinline__ void refresh_steps(const Tile& c, PlainLine& p) {
-    if (p.head == kInvalid) return;
+    const bool live = p.head != kInvalid;
+    const uint32_t h = live ? p.head : 0u;
 #pragma unroll
-    for (int k = 0; k < 3; ++k) { p.move[k] = c.F(hMove + k, p.head); p.step[k] = c.F(hStep + k, p.head); }
+    for (int k = 0; k < 3; ++k) {
+        const float move = c.F(hMove + k, h), step = c.F(hStep + k, h);
+        p.move[k] = live ? move : 0.0f; p.step[k] = live ? step : 0.0f;
+    }
 }
 // A head's response at its current move with the rounding noise of each axis; false when nothing of it is non-zero.
 __device__ __forceinline__ bool head_terms(const Tile& c, uint32_t h, float (&f)[3], float (&cv)[6], float (&noise)[3]) {
@@ -1435,30 +1452,30 @@ __device__ __forceinline__ bool assemble_block(const Tile& c, const float (&mrow
         for (int k = 0; k < 3; ++k) mn[k] = fabsf(mf[k]) + mc[k] * (fabsf(own.res[k]) + fabsf(own.move[k]));
     }
     if (c.elliptic) head_terms(c, lane, mf, mc, mn);   // the cone's own response; the same values as above for every other head
-    // (lanes from the heads' count on hold copies of the first sixteen heads when there are no more than that)
-    const bool mine = lane < c.heads && (mf[0] != 0.0f || mf[1] != 0.0f || mf[2] != 0.0f || mc[0] != 0.0f || mc[1] != 0.0f || mc[2] != 0.0f || mc[5] != 0.0f ||
-                      mc[3] != 0.0f || mc[4] != 0.0f || mn[0] != 0.0f || mn[1] != 0.0f || mn[2] != 0.0f);
-    const uint32_t my_axes = lane < c.heads ? c.U(hAxes, lane) : 0u;
-    const uint32_t my_low = lane < c.heads ? c.U(hColumnsLow, lane) : 0u, my_high = lane < c.heads ? c.U(hColumnsHigh, lane) : 0u;
-    // The Hessian M + sum J^T C J changes only through the heads' curvatures: every head keeps the curvature of its
-    // last assembly in its fields, and while none differs the factor of the last factorisation still stands.
-    bool changed = false;
+    // whether anything of the head is not zero (lanes from the heads' count on hold copies of the first sixteen heads when
+    // there are no more than that)
+    const auto bits = [](float v) { return __float_as_uint(v); };
+    const uint32_t any_bits = ((bits(mf[0]) | bits(mf[1]) | bits(mf[2])) | (bits(mc[0]) | bits(mc[1]) | bits(mc[2]))) |
+                              ((bits(mc[3]) | bits(mc[4]) | bits(mc[5])) | (bits(mn[0]) | bits(mn[1]) | bits(mn[2])));
+    const bool mine = lane < c.heads && (any_bits << 1u) != 0u;
+    // The Hessian M + sum J^T C J changes only through the heads' curvatures: the curvature of a head's last assembly is
+    // kept (in the lane of a head below 64, in the fields beyond), and while none differs the factor of the last
+    // factorisation still stands.
+    uint32_t differs = 0u;
     for (uint32_t h = lane + kWave; h < c.heads; h += kWave) {
         float f[3], cv[6], noise[3];
         const bool contributes = head_terms(c, h, f, cv, noise);
 #pragma unroll
         for (int k = 0; k < 3; ++k) { c.F(hF + k, h) = f[k]; c.F(hNoise + k, h) = noise[k]; }
 #pragma unroll
-        for (int k = 0; k < 6; ++k) { changed = changed || __float_as_uint(c.F(hC + k, h)) != __float_as_uint(cv[k]); c.F(hC + k, h) = cv[k]; }
+        for (int k = 0; k < 6; ++k) { differs |= bits(c.F(hC + k, h)) ^ bits(cv[k]); c.F(hC + k, h) = cv[k]; }
         c.U(hContrib, h) = contributes ? 1u : 0u;
     }
-    if (lane < c.heads) {
 #pragma unroll
-        for (int k = 0; k < 6; ++k) { changed = changed || __float_as_uint(c.F(hC + k, lane)) != __float_as_uint(mc[k]); c.F(hC + k, lane) = mc[k]; }
-    }
-    if (__any(changed)) c.factor_current = false;
+    for (int k = 0; k < 6; ++k) { differs |= bits(c.curvature[k]) ^ bits(mc[k]); c.curvature[k] = mc[k]; }
+    if (__any(lane < c.heads && differs != 0u)) c.factor_current = false;
     if (c.units && lane < c.heads && c.U(hUnit, lane) != kInvalid) {   // a coordinate reads its unit heads' responses from the fields
-        c.F(hF, lane) = mf[0]; c.F(hNoise, lane) = mn[0];
+        c.F(hF, lane) = mf[0]; c.F(hNoise, lane) = mn[0]; c.F(hC, lane) = mc[0];
         c.U(hContrib, lane) = mine ? 1u : 0u;
     }
     __syncthreads();
@@ -1518,14 +1535,15 @@ __device__ __forceinline__ bool assemble_block(const Tile& c, const float (&mrow
     } else {
         bool added = false;
         if constexpr (N <= 32 && !kFollow) {
-            if (staged != 0ull) add_heads_by_tiles<N>(c, staged, mf, mc, mn, lane < c.heads ? c.U(hRow, lane) : 0u, hrow, g, scale);
+            if (staged != 0ull) add_heads_by_tiles<N>(c, staged, mf, mc, mn, c.U(hRow, lane < c.heads ? lane : 0u), hrow, g, scale);
             added = true;
         }
         if constexpr (N <= 32 && kFollow) {
             // two or more contributing heads (all of them staged, one a lane): two a pass, the second half of the
             // wavefront collecting its heads in rows of its own
             if ((staged & (staged - 1ull)) != 0ull) {
-                const uint32_t my_first = lane < c.heads ? c.U(hRow, lane) : 0u;
+                const uint32_t own_head = lane < c.heads ? lane : 0u;
+                const uint32_t my_first = c.U(hRow, own_head), my_low = c.U(hColumnsLow, own_head), my_high = c.U(hColumnsHigh, own_head);
                 if constexpr (N <= 20) {
                     // where three or four copies of the rows fit the wavefront, that many heads a pass - when it takes fewer
                     // passes than two a pass would (adding the groups' rows together costs more than adding two halves)
@@ -1572,7 +1590,9 @@ __device__ __forceinline__ bool assemble_block(const Tile& c, const float (&mrow
                 }
             }
         }
-        if (!added) {
+        if (!added && staged != 0ull) {
+            const uint32_t own_head = lane < c.heads ? lane : 0u;
+            const uint32_t my_axes = c.U(hAxes, own_head), my_low = c.U(hColumnsLow, own_head), my_high = c.U(hColumnsHigh, own_head);
             for (uint64_t rest = staged; rest != 0ull; rest &= rest - 1ull) {
                 const uint32_t h = uint32_t(__builtin_ctzll(rest));
                 float f[3], cv[6], noise[3];
@@ -1723,6 +1743,15 @@ __device__ __forceinline__ void row_steps(const Tile& c, float d) {
     float* dvec = c.vec;
     dvec[c.lane] = c.lane < c.n ? d : 0.0f;
     __syncthreads();
+    if (c.heads <= 16u && !c.units && !c.from_links) {
+        // a lane a row: the first three rows of sixteen lanes take an axis each, lane & 15 = head (a head on one axis has
+        // zeros in the rows of the others)
+        const uint32_t axis = c.lane >> 4u, h = c.lane & 15u;
+        if (axis < 3u && h < c.heads && c.U(hRow, h) != kInvalid)
+            c.fields[axis == 0u ? c.at(hStep, h) : c.at(hStep + 1, h) + axis - 1u] = row_dot_fma<N>(c.jac + (c.U(hRow, h) + axis) * uint32_t(N), dvec);
+        __syncthreads();
+        return;
+    }
     for (uint32_t h = c.lane; h < c.heads; h += kWave) {
         if (c.U(hOwned, h) == 0u) continue;
         const uint32_t unit = c.U(hUnit, h);
@@ -1926,7 +1955,7 @@ __device__ __forceinline__ void descend_block(Tile& c, const float (&mrow)[N], c
         if (follower) dd = mass_step;
         TileSum curvature{0.0};
         if (coordinate) tile_add_product(curvature, dd, mass_step);
-        const float inertial_curvature = wave_total(curvature);
+        const float inertial_curvature = coordinate_total<N>(curvature);
         if (inertial_curvature > 0.0f && isfinite(inertial_curvature)) {
             row_steps<N>(c, dd);
             const float alpha = search_line<kKeepLine<N>>(c, line, -inertial_curvature, inertial_curvature);
@@ -1957,9 +1986,9 @@ __device__ __forceinline__ void descend_block(Tile& c, const float (&mrow)[N], c
             tile_add_product(slope, inertia, dd);
             tile_add_product(curvature, dd, mass_step);
         }
-        const float total_decrement = wave_total(decrement);
-        const float inertial_slope = wave_total(slope);
-        const float inertial_curvature = wave_total(curvature);
+        const float total_decrement = coordinate_total<N>(decrement);
+        const float inertial_slope = coordinate_total<N>(slope);
+        const float inertial_curvature = coordinate_total<N>(curvature);
         if (!isfinite(total_decrement) || !isfinite(inertial_slope) || !isfinite(inertial_curvature)) { failure = kFailDirection; break; }
         if (!(total_decrement > 0.0f)) break;
         PROF_END(c, 27);
@@ -2394,13 +2423,13 @@ __device__ __forceinline__ bool reduce_block(uint32_t lane, uint32_t n, const fl
         }
     }
     double* coupling = reinterpret_cast<double*>(lds);   // [follower][coordinate below K]: U_TU transposed
-    double* corner = coupling + kFollowers * K;           // [follower i][follower k]: U_UU[i][k], zero below the diagonal
+    double* corner = coupling + kFollowers * K;           // [follower i][follower k]: U_UU[i][k], zero from the diagonal down
     if (lane < uint32_t(K)) {
 #pragma unroll
         for (int k = K; k < N; ++k) coupling[(k - K) * K + int(lane)] = full[k];
     } else if (lane < uint32_t(N)) {
 #pragma unroll
-        for (int k = K; k < N; ++k) corner[(int(lane) - K) * kFollowers + (k - K)] = uint32_t(k) >= lane ? full[k] : 0.0;
+        for (int k = K; k < N; ++k) corner[(int(lane) - K) * kFollowers + (k - K)] = uint32_t(k) > lane ? full[k] : 0.0;
     }
     __syncthreads();
     const uint32_t slot = lane >= uint32_t(K) && lane < uint32_t(N) ? lane - uint32_t(K) : 0u;
@@ -2420,7 +2449,7 @@ __device__ __forceinline__ bool reduce_block(uint32_t lane, uint32_t n, const fl
 #pragma unroll
         for (int i = K; i < N; ++i) {
             const double y = lane_value_d(prow[c0] * own_scale, i);
-            prow[c0] = at > uint32_t(i) ? fma(-column[i - K], y, prow[c0]) : prow[c0];
+            prow[c0] = fma(column[i - K], -y, prow[c0]);   // (the column holds zeros for the followers up to i)
         }
     }
 #pragma unroll
@@ -2460,6 +2489,7 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
     c.tolerance = p.velocity_tolerance; c.failed = false; c.momentum = 0.0f; c.residual = 0.0f;
     c.mass_inverse = 0.0f; c.mass_valid = false; c.work = 0u; c.units = false; c.elliptic = false;
     c.factor_current = false; c.factor_root = 1.0f;
+    for (float& entry : c.curvature) entry = 0.0f;
 #ifdef NKH_SOLVER_PROFILE
     for (int i = 0; i < 32; ++i) c.prof[i] = 0;
     for (int i = 0; i < 4; ++i) c.prof_count[i] = 0u;
@@ -2859,7 +2889,7 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
             }
         }
         for (uint32_t h0 = 0u; h0 < (by_heads ? 0u : share_units ? c.individual_end : heads); h0 += 4u) {
-            float a[4], term[4], total[4];
+            float a[4], total[4];
             bool second[4], apart[4], skip[4];
 #pragma unroll
             for (uint32_t t = 0u; t < 4u; ++t) {
@@ -2890,16 +2920,29 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
             if (skip[0] && skip[1] && skip[2] && skip[3]) continue;
 #pragma unroll
             for (int j = 0; j < N; ++j) {
+                float y[4];
 #pragma unroll
-                for (int t = 0; t < 4; ++t) a[t] -= lrow[j] * lane_value(a[t], j);
+                for (int t = 0; t < 4; ++t) y[t] = lane_value(a[t], j);
+#pragma unroll
+                for (int t = 0; t < 4; ++t) a[t] -= lrow[j] * y[t];
             }
+            // the ordered sums, a lane a head: the terms pass through LDS (where the factors will stand, not built yet)
+            float* terms = c.hfac;
 #pragma unroll
-            for (int t = 0; t < 4; ++t) { term[t] = coordinate ? a[t] * a[t] / pivot : 0.0f; total[t] = 0.0f; }
-#pragma unroll
-            for (int i = 0; i < N; ++i) {
-#pragma unroll
-                for (int t = 0; t < 4; ++t) total[t] += lane_value(term[t], i);
+            for (int t = 0; t < 4; ++t) {
+                const float term = coordinate ? a[t] * a[t] / pivot : 0.0f;
+                if (lane < uint32_t(N)) terms[uint32_t(t * N) + lane] = term;
             }
+            __syncthreads();
+            float mine = 0.0f;
+            {
+                const float4* words = reinterpret_cast<const float4*>(terms + (lane & 3u) * uint32_t(N));
+#pragma unroll
+                for (int q = 0; q < N / 4; ++q) { const float4 w = words[q]; mine += w.x; mine += w.y; mine += w.z; mine += w.w; }
+            }
+            __syncthreads();
+#pragma unroll
+            for (int t = 0; t < 4; ++t) total[t] = lane_value(mine, t);
 #pragma unroll
             for (uint32_t t = 0u; t < 4u; ++t) {
                 const uint32_t h = h0 + t;
@@ -2916,7 +2959,7 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
             float mine = 0.0f;
             for (uint64_t rest = __ballot(c.unit_count > 0u); rest != 0ull;) {
                 uint32_t target[4];
-                float a[4], term[4], total[4];
+                float a[4], total[4];
 #pragma unroll
                 for (int t = 0; t < 4; ++t) {
                     target[t] = rest != 0ull ? uint32_t(__builtin_ctzll(rest)) : kInvalid;
@@ -2928,17 +2971,28 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
 #pragma unroll
                 for (int j = 0; j < N; ++j) {
                     if (j < first) continue;
+                    float y[4];
 #pragma unroll
-                    for (int t = 0; t < 4; ++t) a[t] -= lrow[j] * lane_value(a[t], j);
+                    for (int t = 0; t < 4; ++t) y[t] = lane_value(a[t], j);
+#pragma unroll
+                    for (int t = 0; t < 4; ++t) a[t] -= lrow[j] * y[t];
                 }
+                float* terms = c.hfac;
 #pragma unroll
-                for (int t = 0; t < 4; ++t) { term[t] = coordinate ? a[t] * a[t] / pivot : 0.0f; total[t] = 0.0f; }
-#pragma unroll
-                for (int i = 0; i < N; ++i) {
-                    if (i < first) continue;
-#pragma unroll
-                    for (int t = 0; t < 4; ++t) total[t] += lane_value(term[t], i);
+                for (int t = 0; t < 4; ++t) {
+                    const float term = coordinate ? a[t] * a[t] / pivot : 0.0f;
+                    if (lane < uint32_t(N)) terms[uint32_t(t * N) + lane] = term;
                 }
+                __syncthreads();
+                float sum = 0.0f;
+                {
+                    const float4* words = reinterpret_cast<const float4*>(terms + (lane & 3u) * uint32_t(N));
+#pragma unroll
+                    for (int q = 0; q < N / 4; ++q) { const float4 w = words[q]; sum += w.x; sum += w.y; sum += w.z; sum += w.w; }
+                }
+                __syncthreads();
+#pragma unroll
+                for (int t = 0; t < 4; ++t) total[t] = lane_value(sum, t);
 #pragma unroll
                 for (int t = 0; t < 4; ++t) if (lane == target[t]) mine = total[t];
             }
