@@ -21,7 +21,6 @@
 // Not built: free rigid 6x6 blocks, mimic couplings.
 #pragma once
 
-#include <utility>
 #include "nk_device_math.h"
 #include "backend.h"
 #include "nk_ops.h"
@@ -311,9 +310,12 @@ struct Tile {
     float* jac;      // 3 * staged capacity rows x ldj, ldj = N
     float* fields;   // cap x kWideStride, then (narrow + 1) x kNarrowStride
     float* vec;      // 4 x 64 scratch vectors, 16-byte aligned
+    float* hrows;    // blocks of at most 32 coordinates: N x N words, the Hessian of the last assembly in full
+    float* low;      // a reduced block: N x N words, the second floats of its mass rows
     float mass_inverse;   // 1 / diagonal of the mass factor, lane = row
     mutable float curvature[6];      // of lane's own head at the last assembly
     mutable float factor_root;       // the diagonal of that factor, lane = row
+    mutable bool rows_current;       // ... and since hrows was written
     mutable bool factor_current;     // no head's curvature has changed since hfac was factored: the Hessian is the same
     mutable uint32_t work;   // Newton steps and line probes of this solve, the next solve's scheduling key
     bool mass_valid;
@@ -352,6 +354,10 @@ struct Tile {
     __device__ __forceinline__ float& F(uint32_t field, uint32_t h) const { return fields[at(field, h)]; }
     __device__ __forceinline__ uint32_t& U(uint32_t field, uint32_t h) const { return reinterpret_cast<uint32_t*>(fields)[at(field, h)]; }
 };
+
+// lane's row of Tile::low, as sixteen-byte words
+template <int N>
+__device__ __forceinline__ const float4* low_row(const Tile& c) { return reinterpret_cast<const float4*>(c.low + min(c.lane, uint32_t(N - 1)) * uint32_t(N)); }
 
 // TileResponse (block_descent_tile.cuh:678-681) with the Coulomb branch of EvaluateAugmentedResponse (block_descent.cu:1593-1621)
 __device__ __forceinline__ void head_response(const Tile& c, uint32_t h, float mx, float my, float mz, float* f, float* cv) {
@@ -609,166 +615,73 @@ __device__ __forceinline__ float solve_tile_mass(const Tile& c, float force) {
     return substitute<N>(row, col, c.mass_inverse, c.lane < c.n ? force : 0.0f);
 }
 
-// The LDS byte address of a pointer into the block's shared memory.
-__device__ __forceinline__ uint32_t lds_address(const float* p) {
-    return uint32_t(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const float*)p));
+typedef float Vec4 __attribute__((ext_vector_type(4)));
+// Columns 4 q .. 4 q + 3 of a head's Hessian term in lane's row, on the matrix cores: v_mfma_f32_4x4x1 multiplies, in each
+// of the wavefront's sixteen blocks of four lanes, four values a block with one a lane, so with the Jacobian row's words
+// 4 q + (lane & 3) on the one side and the lane's entry of C J on the other, register r of a lane comes out as the
+// term's entry (lane's row, 4 q + r) - the register rows' own layout, whatever head each block of lanes is at.  An axis an
+// instruction, each the fused multiply-add it would be on the vector unit (bit for bit), then one sum into the row.  A
+// head's words come in one round trip of fifteen four-byte reads; written as vector code the columns took four times
+// the arithmetic and a wait for three sixteen-byte reads each (12 heads of 20 columns: 5.7 k cycles a Newton step).
+template <int N>
+__device__ __forceinline__ void add_columns(int q, const float* rows, float a0, float a1, float a2, float (&hrow)[N]) {
+    const float* x = rows + 4 * q;
+    Vec4 term = {};
+    term = __builtin_amdgcn_mfma_f32_4x4x1f32(x[0], a0, term, 0, 0, 0);
+    term = __builtin_amdgcn_mfma_f32_4x4x1f32(x[N], a1, term, 0, 0, 0);
+    term = __builtin_amdgcn_mfma_f32_4x4x1f32(x[2 * N], a2, term, 0, 0, 0);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) hrow[4 * q + r] += term[r];
 }
+// the same for a head on one axis, straight into the row
+template <int N>
+__device__ __forceinline__ void add_columns_single(int q, const float* rows, float a0, float (&hrow)[N]) {
+    Vec4 term = {hrow[4 * q], hrow[4 * q + 1], hrow[4 * q + 2], hrow[4 * q + 3]};
+    term = __builtin_amdgcn_mfma_f32_4x4x1f32(rows[4 * q], a0, term, 0, 0, 0);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) hrow[4 * q + r] = term[r];
+}
+// The column groups a block's contacts reach when they leave the later ones alone: taken without a test a group.
+template <int N>
+constexpr int kFirstColumns = N > 20 ? 5 : N / 4;
 
-// Four columns of a head's Hessian term, taken or left as a whole on a uniform mask, with the products and sums the
-// plain loops of add_head form.  Three rows: h += a0 x0 + a1 x1 + a2 x2 as a product, two fused multiply-adds and a
-// sum.  A single row: one fused multiply-add into h.  Written out because the compiled form of such a conditional
-// update carries the whole row through the head loop twice and copies one set of registers into the other at every
-// branch, about as many moves as the update has arithmetic.  Here the row's registers change in place, and the words
-// come from LDS (`kFirst`, `kSecond`, `kThird` bytes past `row_address`) into twelve registers that the block takes for
-// itself, v244-v255.  Only for widths that run two waves a SIMD: their kernels leave those registers free.  The waits
-// count LDS reads only as far as those return in order; scalar loads in flight make them wait longer, never shorter.
-#ifdef NKH_SOLVER_DENSE   // the same block on registers inside the dense build's 168: v152-v163
-template <int kFirst, int kSecond, int kThird>
-__device__ __forceinline__ void add_columns_if(uint32_t live, uint32_t single, uint32_t row_address, float a0, float a1, float a2, float& h0,
-                                               float& h1, float& h2, float& h3) {
-    asm volatile(
-        "s_cmp_eq_u32 %[live], 0\n\t"
-        "s_cbranch_scc1 .Lcolumns_done_%=\n\t"
-        "s_cmp_eq_u32 %[single], 0\n\t"
-        "s_cbranch_scc0 .Lcolumns_single_%=\n\t"
-        "ds_read_b128 v[152:155], %[at] offset:%[first]\n\t"
-        "ds_read_b128 v[156:159], %[at] offset:%[second]\n\t"
-        "ds_read_b128 v[160:163], %[at] offset:%[third]\n\t"
-        "s_waitcnt lgkmcnt(2)\n\t"
-        "v_mul_f32 v152, %[a0], v152\n\t"
-        "v_mul_f32 v153, %[a0], v153\n\t"
-        "v_mul_f32 v154, %[a0], v154\n\t"
-        "v_mul_f32 v155, %[a0], v155\n\t"
-        "s_waitcnt lgkmcnt(1)\n\t"
-        "v_fmac_f32 v152, %[a1], v156\n\t"
-        "v_fmac_f32 v153, %[a1], v157\n\t"
-        "v_fmac_f32 v154, %[a1], v158\n\t"
-        "v_fmac_f32 v155, %[a1], v159\n\t"
-        "s_waitcnt lgkmcnt(0)\n\t"
-        "v_fmac_f32 v152, %[a2], v160\n\t"
-        "v_fmac_f32 v153, %[a2], v161\n\t"
-        "v_fmac_f32 v154, %[a2], v162\n\t"
-        "v_fmac_f32 v155, %[a2], v163\n\t"
-        "v_add_f32 %[h0], %[h0], v152\n\t"
-        "v_add_f32 %[h1], %[h1], v153\n\t"
-        "v_add_f32 %[h2], %[h2], v154\n\t"
-        "v_add_f32 %[h3], %[h3], v155\n\t"
-        "s_branch .Lcolumns_done_%=\n"
-        ".Lcolumns_single_%=:\n\t"
-        "ds_read_b128 v[152:155], %[at] offset:%[first]\n\t"
-        "s_waitcnt lgkmcnt(0)\n\t"
-        "v_fmac_f32 %[h0], %[a0], v152\n\t"
-        "v_fmac_f32 %[h1], %[a0], v153\n\t"
-        "v_fmac_f32 %[h2], %[a0], v154\n\t"
-        "v_fmac_f32 %[h3], %[a0], v155\n"
-        ".Lcolumns_done_%=:"
-        : [h0] "+v"(h0), [h1] "+v"(h1), [h2] "+v"(h2), [h3] "+v"(h3)
-        : [live] "s"(live), [single] "s"(single), [at] "v"(row_address), [a0] "v"(a0), [a1] "v"(a1), [a2] "v"(a2), [first] "n"(kFirst),
-          [second] "n"(kSecond), [third] "n"(kThird)
-        : "v152", "v153", "v154", "v155", "v156", "v157", "v158", "v159", "v160", "v161", "v162", "v163", "scc");
-}
-#else
-template <int kFirst, int kSecond, int kThird>
-__device__ __forceinline__ void add_columns_if(uint32_t live, uint32_t single, uint32_t row_address, float a0, float a1, float a2, float& h0,
-                                               float& h1, float& h2, float& h3) {
-    asm volatile(
-        "s_cmp_eq_u32 %[live], 0\n\t"
-        "s_cbranch_scc1 .Lcolumns_done_%=\n\t"
-        "s_cmp_eq_u32 %[single], 0\n\t"
-        "s_cbranch_scc0 .Lcolumns_single_%=\n\t"
-        "ds_read_b128 v[244:247], %[at] offset:%[first]\n\t"
-        "ds_read_b128 v[248:251], %[at] offset:%[second]\n\t"
-        "ds_read_b128 v[252:255], %[at] offset:%[third]\n\t"
-        "s_waitcnt lgkmcnt(2)\n\t"
-        "v_mul_f32 v244, %[a0], v244\n\t"
-        "v_mul_f32 v245, %[a0], v245\n\t"
-        "v_mul_f32 v246, %[a0], v246\n\t"
-        "v_mul_f32 v247, %[a0], v247\n\t"
-        "s_waitcnt lgkmcnt(1)\n\t"
-        "v_fmac_f32 v244, %[a1], v248\n\t"
-        "v_fmac_f32 v245, %[a1], v249\n\t"
-        "v_fmac_f32 v246, %[a1], v250\n\t"
-        "v_fmac_f32 v247, %[a1], v251\n\t"
-        "s_waitcnt lgkmcnt(0)\n\t"
-        "v_fmac_f32 v244, %[a2], v252\n\t"
-        "v_fmac_f32 v245, %[a2], v253\n\t"
-        "v_fmac_f32 v246, %[a2], v254\n\t"
-        "v_fmac_f32 v247, %[a2], v255\n\t"
-        "v_add_f32 %[h0], %[h0], v244\n\t"
-        "v_add_f32 %[h1], %[h1], v245\n\t"
-        "v_add_f32 %[h2], %[h2], v246\n\t"
-        "v_add_f32 %[h3], %[h3], v247\n\t"
-        "s_branch .Lcolumns_done_%=\n"
-        ".Lcolumns_single_%=:\n\t"
-        "ds_read_b128 v[244:247], %[at] offset:%[first]\n\t"
-        "s_waitcnt lgkmcnt(0)\n\t"
-        "v_fmac_f32 %[h0], %[a0], v244\n\t"
-        "v_fmac_f32 %[h1], %[a0], v245\n\t"
-        "v_fmac_f32 %[h2], %[a0], v246\n\t"
-        "v_fmac_f32 %[h3], %[a0], v247\n"
-        ".Lcolumns_done_%=:"
-        : [h0] "+v"(h0), [h1] "+v"(h1), [h2] "+v"(h2), [h3] "+v"(h3)
-        : [live] "s"(live), [single] "s"(single), [at] "v"(row_address), [a0] "v"(a0), [a1] "v"(a1), [a2] "v"(a2), [first] "n"(kFirst),
-          [second] "n"(kSecond), [third] "n"(kThird)
-        : "v244", "v245", "v246", "v247", "v248", "v249", "v250", "v251", "v252", "v253", "v254", "v255", "scc");
-}
-#endif
-template <int N, int... Q>
-__device__ __forceinline__ void add_column_groups(std::integer_sequence<int, Q...>, uint64_t columns, uint32_t single, uint32_t row_address,
-                                                  float a0, float a1, float a2, float (&hrow)[N]) {
-    // the mask and the flag are uniform; the lane read says so where they come out of LDS
-    const uint32_t low = uint32_t(__builtin_amdgcn_readfirstlane(int(uint32_t(columns))));
-    const uint32_t high = uint32_t(__builtin_amdgcn_readfirstlane(int(uint32_t(columns >> 32u))));
-    const uint64_t uniform_columns = (uint64_t(high) << 32u) | uint64_t(low);
-    single = uint32_t(__builtin_amdgcn_readfirstlane(int(single)));
-    (add_columns_if<16 * Q, 16 * Q + 4 * N, 16 * Q + 8 * N>(uint32_t(uniform_columns >> (4 * Q)) & 0xFu, single, row_address, a0, a1, a2, hrow[4 * Q],
-                                                            hrow[4 * Q + 1], hrow[4 * Q + 2], hrow[4 * Q + 3]), ...);
-}
-
-// One head's part of the block: g += J^T f and H += J^T C J for lane's row, skipping the column blocks the head's
-// Jacobian rows leave at exact zero.  All head values are uniform.  Widths that run two waves a SIMD update the row
-// through add_columns_if, wider ones through the plain loops.
+// One head's part of the block: g += J^T f and H += J^T C J for lane's row, skipping the column blocks past the first
+// twenty coordinates that the head's Jacobian rows leave at exact zero.  All head values are uniform.
 template <int N>
 __device__ __forceinline__ void add_head(const Tile& c, uint32_t h, bool coordinate, const float (&f)[3], const float (&cv)[6],
                                          const float (&noise)[3], uint32_t axes, uint64_t columns, float (&hrow)[N], TileSum& g,
                                          float& scale) {
     const float* j0r = c.jac + c.U(hRow, h) * uint32_t(N);
+    const float* words = j0r + (c.lane & 3u);
     // (the lane's words read whether or not it is a coordinate: a read under a condition compiles to a branch a word)
     const uint32_t column = c.lane < uint32_t(N) ? c.lane : uint32_t(N - 1);
     const float w0 = j0r[column];
     const float j0 = coordinate ? w0 : 0.0f;
     tile_add_product(g, j0, f[0]);
     scale += fabsf(j0) * noise[0];
-    const float4* r0 = reinterpret_cast<const float4*>(j0r);
-    if constexpr (N <= kTwoWaveWidth) {
-        float a0 = j0 * cv[0], a1 = 0.0f, a2 = 0.0f;
-        if (axes != 1u) {
-            const float w1 = j0r[N + column], w2 = j0r[2 * N + column];
-            const float j1 = coordinate ? w1 : 0.0f, j2 = coordinate ? w2 : 0.0f;
-            const float cxx = cv[0], cyy = cv[1], czz = cv[2], cxy = cv[3], cxz = cv[4], cyz = cv[5];
-            tile_add_product(g, j1, f[1]);
-            tile_add_product(g, j2, f[2]);
-            scale += fabsf(j1) * noise[1] + fabsf(j2) * noise[2];
-            a0 = (j0 * cxx + j1 * cxy) + j2 * cxz;
-            a1 = (j1 * cyy + j2 * cyz) + j0 * cxy;
-            a2 = (j2 * czz + j1 * cyz) + j0 * cxz;
-        }
-        add_column_groups<N>(std::make_integer_sequence<int, N / 4>{}, columns, axes == 1u ? 1u : 0u, lds_address(j0r), a0, a1, a2, hrow);
-        return;
-    }
     if (axes == 1u) {
         const float a0 = j0 * cv[0];
+        if constexpr (N > kTwoWaveWidth) {
+            const float4* r0 = reinterpret_cast<const float4*>(j0r);
 #pragma unroll
-        for (int q = 0; q < N / 4; ++q) {
-            if (((columns >> (4 * q)) & 0xFull) == 0ull) continue;
-            const float4 x0 = r0[q];
-            hrow[4 * q] = fmaf(a0, x0.x, hrow[4 * q]); hrow[4 * q + 1] = fmaf(a0, x0.y, hrow[4 * q + 1]);
-            hrow[4 * q + 2] = fmaf(a0, x0.z, hrow[4 * q + 2]); hrow[4 * q + 3] = fmaf(a0, x0.w, hrow[4 * q + 3]);
+            for (int q = 0; q < N / 4; ++q) {
+                if (((columns >> (4 * q)) & 0xFull) == 0ull) continue;
+                const float4 x0 = r0[q];
+                hrow[4 * q] = fmaf(a0, x0.x, hrow[4 * q]); hrow[4 * q + 1] = fmaf(a0, x0.y, hrow[4 * q + 1]);
+                hrow[4 * q + 2] = fmaf(a0, x0.z, hrow[4 * q + 2]); hrow[4 * q + 3] = fmaf(a0, x0.w, hrow[4 * q + 3]);
+            }
+            return;
         }
+#pragma unroll
+        for (int q = 0; q < kFirstColumns<N>; ++q) add_columns_single<N>(q, words, a0, hrow);
+        if ((columns >> (4 * kFirstColumns<N>)) == 0ull) return;
+#pragma unroll
+        for (int q = kFirstColumns<N>; q < N / 4; ++q)
+            if (((columns >> (4 * q)) & 0xFull) != 0ull) add_columns_single<N>(q, words, a0, hrow);
         return;
     }
-    const float* j1r = j0r + N, *j2r = j0r + 2 * N;
-    const float j1 = coordinate ? j1r[c.lane] : 0.0f, j2 = coordinate ? j2r[c.lane] : 0.0f;
+    const float w1 = j0r[N + column], w2 = j0r[2 * N + column];
+    const float j1 = coordinate ? w1 : 0.0f, j2 = coordinate ? w2 : 0.0f;
     const float cxx = cv[0], cyy = cv[1], czz = cv[2], cxy = cv[3], cxz = cv[4], cyz = cv[5];
     tile_add_product(g, j1, f[1]);
     tile_add_product(g, j2, f[2]);
@@ -776,17 +689,27 @@ __device__ __forceinline__ void add_head(const Tile& c, uint32_t h, bool coordin
     const float a0 = (j0 * cxx + j1 * cxy) + j2 * cxz;
     const float a1 = (j1 * cyy + j2 * cyz) + j0 * cxy;
     const float a2 = (j2 * czz + j1 * cyz) + j0 * cxz;
-    const float4* r1 = reinterpret_cast<const float4*>(j1r);
-    const float4* r2 = reinterpret_cast<const float4*>(j2r);
+    if constexpr (N > kTwoWaveWidth) {   // with the whole register file in use, the terms' registers would spill
+        const float4* r0 = reinterpret_cast<const float4*>(j0r);
+        const float4* r1 = reinterpret_cast<const float4*>(j0r + N);
+        const float4* r2 = reinterpret_cast<const float4*>(j0r + 2 * N);
 #pragma unroll
-    for (int q = 0; q < N / 4; ++q) {
-        if (((columns >> (4 * q)) & 0xFull) == 0ull) continue;
-        const float4 x0 = r0[q], x1 = r1[q], x2 = r2[q];
-        hrow[4 * q] += fmaf(a2, x2.x, fmaf(a1, x1.x, a0 * x0.x));
-        hrow[4 * q + 1] += fmaf(a2, x2.y, fmaf(a1, x1.y, a0 * x0.y));
-        hrow[4 * q + 2] += fmaf(a2, x2.z, fmaf(a1, x1.z, a0 * x0.z));
-        hrow[4 * q + 3] += fmaf(a2, x2.w, fmaf(a1, x1.w, a0 * x0.w));
+        for (int q = 0; q < N / 4; ++q) {
+            if (((columns >> (4 * q)) & 0xFull) == 0ull) continue;
+            const float4 x0 = r0[q], x1 = r1[q], x2 = r2[q];
+            hrow[4 * q] += fmaf(a2, x2.x, fmaf(a1, x1.x, a0 * x0.x));
+            hrow[4 * q + 1] += fmaf(a2, x2.y, fmaf(a1, x1.y, a0 * x0.y));
+            hrow[4 * q + 2] += fmaf(a2, x2.z, fmaf(a1, x1.z, a0 * x0.z));
+            hrow[4 * q + 3] += fmaf(a2, x2.w, fmaf(a1, x1.w, a0 * x0.w));
+        }
+        return;
     }
+#pragma unroll
+    for (int q = 0; q < kFirstColumns<N>; ++q) add_columns<N>(q, words, a0, a1, a2, hrow);
+    if ((columns >> (4 * kFirstColumns<N>)) == 0ull) return;
+#pragma unroll
+    for (int q = kFirstColumns<N>; q < N / 4; ++q)
+        if (((columns >> (4 * q)) & 0xFull) != 0ull) add_columns<N>(q, words, a0, a1, a2, hrow);
 }
 
 // The heads' curvature on the matrix cores, for blocks of at most 32 coordinates: H += sum over heads and axes of
@@ -802,7 +725,6 @@ __device__ __forceinline__ void add_head(const Tile& c, uint32_t h, bool coordin
 //   Bound by the latency of one wave (LDS words of a pass, then the matrix instructions in line).  It takes the place of
 // a loop that added heads to register rows by broadcast reads of their Jacobian words, a head a pass with unit heads present
 // and two to four without: 1000 servo-driven quadrupeds, four steps, 2.58 -> 2.23 ms; 4096 walkers 1.06 -> 1.01 ms.
-typedef float Vec4 __attribute__((ext_vector_type(4)));
 template <int N>
 constexpr int kTileSpan = (N + 15) / 16;   // tiles of sixteen coordinates a side
 __device__ __forceinline__ float lane_permute(int source, float v) {   // v of lane `source`, a byte address (4 x lane)
@@ -837,7 +759,7 @@ __device__ __forceinline__ double halves_sum(double v) {
            __longlong_as_double((long long)((uint64_t(high[1]) << 32u) | uint64_t(low[1])));
 }
 // lane = head on the way in (mf, mc, mn, my_first; `heads` the uniform mask of those to add), lane = row on return
-template <int N>
+template <int N, bool kRows>
 __device__ __forceinline__ void add_heads_by_tiles(const Tile& c, uint64_t heads, const float (&mf)[3], const float (&mc)[6], const float (&mn)[3],
                                                    uint32_t my_first, float (&hrow)[N], TileSum& g, float& scale) {
     static_assert(N <= 32, "two tiles a side at most");
@@ -860,11 +782,13 @@ __device__ __forceinline__ void add_heads_by_tiles(const Tile& c, uint64_t heads
         const bool live = mine != kInvalid;
         const int source = int((live ? mine : 0u) * 4u);
         const float* rows = c.jac + uint32_t(__builtin_amdgcn_ds_bpermute(source, int(my_first))) * uint32_t(N);
-        float f[3], cv[6], noise[3];
+        float f[3], cv[6] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f}, noise[3];
 #pragma unroll
         for (int k = 0; k < 3; ++k) { f[k] = lane_permute(source, mf[k]); noise[k] = lane_permute(source, mn[k]); }
+        if constexpr (kRows) {
 #pragma unroll
-        for (int k = 0; k < 6; ++k) cv[k] = lane_permute(source, mc[k]);
+            for (int k = 0; k < 6; ++k) cv[k] = lane_permute(source, mc[k]);
+        }
         float j[T][3], a[T][3];
 #pragma unroll
         for (int t = 0; t < T; ++t) {
@@ -882,6 +806,7 @@ __device__ __forceinline__ void add_heads_by_tiles(const Tile& c, uint64_t heads
                 bound[t] = fmaf(fabsf(j[t][k]), noise[k], bound[t]);
             }
         }
+        if constexpr (!kRows) continue;
 #pragma unroll
         for (int k = 0; k < 3; ++k)
 #pragma unroll
@@ -890,7 +815,7 @@ __device__ __forceinline__ void add_heads_by_tiles(const Tile& c, uint64_t heads
                 for (int I = 0; I < T; ++I) tile[J][I] = __builtin_amdgcn_mfma_f32_16x16x4f32(j[J][k], a[I][k], tile[J][I], 0, 0, 0);
     }
 #pragma unroll
-    for (int J = 0; J < T; ++J) {
+    for (int J = 0; J < (kRows ? T : 0); ++J) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             if (16 * J + r >= N) continue;
@@ -912,112 +837,21 @@ __device__ __forceinline__ void add_heads_by_tiles(const Tile& c, uint64_t heads
 // A reduced block adds its heads to register rows instead, in an order of its own (below): its worlds are robots on two
 // many-sphered feet, of which some do not converge within their sweeps, and an environment that has not converged hands
 // a last place of its Hessian on as the fourth decimal of its velocities.
-// Two heads in one pass, for blocks of at most 32 coordinates: lanes 0..31 add head `ha` to their rows, lanes 32..63
-// add head `hb` (kInvalid: none) to rows of their own that start at zero, row = lane & 31 in both halves; the caller
-// sums the halves afterwards (halves_sum).  A head's values come from its own lane (lane = head) through the lane
-// permute, its Jacobian words from the head's own rows in LDS; a column group is taken when either head reaches it
-// (the other then adds exact zeros).  The sums add in another order than head after head: the last place may differ.
-template <int N>
-__device__ __forceinline__ void add_head_pair(const Tile& c, uint32_t ha, uint32_t hb, const float (&mf)[3], const float (&mc)[6], const float (&mn)[3],
-                                              uint32_t my_first, uint32_t my_low, uint32_t my_high, float (&hrow)[N], TileSum& g, float& scale) {
-    static_assert(N <= 32, "both halves of the wavefront hold every row");
-    const uint32_t row = c.lane & 31u;
-    const bool none = c.lane >= 32u && hb == kInvalid;
-    const int source = int(c.lane >= 32u ? (hb == kInvalid ? ha : hb) : ha);
-    float f[3], cv[6], noise[3];
-#pragma unroll
-    for (int k = 0; k < 3; ++k) { f[k] = __shfl(mf[k], source, kWave); noise[k] = __shfl(mn[k], source, kWave); }
-#pragma unroll
-    for (int k = 0; k < 6; ++k) cv[k] = __shfl(mc[k], source, kWave);
-    const uint32_t first = uint32_t(__shfl(int(my_first), source, kWave));
-    const float* j0r = c.jac + first * uint32_t(N);
-    const bool live = !none && row < c.n;
-    // (read whether or not the lane uses them: a read under a condition compiles to a branch a word)
-    const uint32_t column = row < uint32_t(N) ? row : uint32_t(N - 1);
-    const float w0 = j0r[column], w1 = j0r[N + column], w2 = j0r[2 * N + column];
-    const float j0 = live ? w0 : 0.0f, j1 = live ? w1 : 0.0f, j2 = live ? w2 : 0.0f;
-    tile_add_product(g, j0, f[0]);
-    tile_add_product(g, j1, f[1]);
-    tile_add_product(g, j2, f[2]);
-    scale += (fabsf(j0) * noise[0] + fabsf(j1) * noise[1]) + fabsf(j2) * noise[2];
-    const float cxx = cv[0], cyy = cv[1], czz = cv[2], cxy = cv[3], cxz = cv[4], cyz = cv[5];
-    const float a0 = (j0 * cxx + j1 * cxy) + j2 * cxz;
-    const float a1 = (j1 * cyy + j2 * cyz) + j0 * cxy;
-    const float a2 = (j2 * czz + j1 * cyz) + j0 * cxz;
-    uint64_t columns = (uint64_t(uint32_t(__builtin_amdgcn_readlane(int(my_high), int(ha)))) << 32u) |
-                       uint64_t(uint32_t(__builtin_amdgcn_readlane(int(my_low), int(ha))));
-    if (hb != kInvalid)
-        columns |= (uint64_t(uint32_t(__builtin_amdgcn_readlane(int(my_high), int(hb)))) << 32u) |
-                   uint64_t(uint32_t(__builtin_amdgcn_readlane(int(my_low), int(hb))));
-    if constexpr (N <= kTwoWaveWidth) {
-        add_column_groups<N>(std::make_integer_sequence<int, N / 4>{}, columns, 0u, lds_address(j0r), a0, a1, a2, hrow);
-    } else {
-        const float4* r0 = reinterpret_cast<const float4*>(j0r);
-        const float4* r1 = reinterpret_cast<const float4*>(j0r + N);
-        const float4* r2 = reinterpret_cast<const float4*>(j0r + 2 * N);
-#pragma unroll
-        for (int q = 0; q < N / 4; ++q) {
-            if (((columns >> (4 * q)) & 0xFull) == 0ull) continue;
-            const float4 x0 = r0[q], x1 = r1[q], x2 = r2[q];
-            hrow[4 * q] += fmaf(a2, x2.x, fmaf(a1, x1.x, a0 * x0.x));
-            hrow[4 * q + 1] += fmaf(a2, x2.y, fmaf(a1, x1.y, a0 * x0.y));
-            hrow[4 * q + 2] += fmaf(a2, x2.z, fmaf(a1, x1.z, a0 * x0.z));
-            hrow[4 * q + 3] += fmaf(a2, x2.w, fmaf(a1, x1.w, a0 * x0.w));
-        }
-    }
-}
-
-// Heads a pass where three or four copies of the block's rows fit the wavefront (kGroups<N> of N lanes each): the
-// lanes of group g add head `heads[g]` (kInvalid: none) to rows of their own, row = lane - g N; groups past the first
-// start at zero and the caller adds the groups' rows together afterwards (groups_sum).  Otherwise as add_head_pair.
+// Heads a pass: as many copies of the block's rows as fit the wavefront, kGroups<N> of them, a group of lanes kGroupLanes
+// wide each - or two where that takes as few passes, or the one that contributes.  The lanes of group k add head
+// `taken[k]` to rows of their own, which start at zero past the first group; a head's values come from its own lane
+// (lane = head) through the lane permute.  The groups' rows are added together at the end, in group order, through LDS
+// (hrows and hfac, which a changed Hessian frees), and stay in hrows.  With kRows false only the force and its scale are
+// taken: the Hessian of the last assembly stands.
 template <int N>
 constexpr int kGroups = N <= 16 ? 4 : (N <= 20 ? 3 : 2);
 template <int N>
-__device__ __forceinline__ void add_head_group(const Tile& c, const uint32_t (&heads)[4], const float (&mf)[3], const float (&mc)[6],
-                                               const float (&mn)[3], uint32_t my_first, uint32_t my_low, uint32_t my_high, float (&hrow)[N],
-                                               TileSum& g, float& scale) {
-    constexpr int G = kGroups<N>;
-    static_assert(G >= 3 && G * N <= 64, "three or four copies of the rows fit the wavefront");
-    const uint32_t group = c.lane / uint32_t(N), row = c.lane - group * uint32_t(N);
-    uint32_t mine = kInvalid;
-#pragma unroll
-    for (int k = 0; k < G; ++k) mine = group == uint32_t(k) ? heads[k] : mine;
-    const bool none = mine == kInvalid;   // also the lanes past the last group
-    const int source = int(none ? heads[0] : mine);
-    float f[3], cv[6], noise[3];
-#pragma unroll
-    for (int k = 0; k < 3; ++k) { f[k] = __shfl(mf[k], source, kWave); noise[k] = __shfl(mn[k], source, kWave); }
-#pragma unroll
-    for (int k = 0; k < 6; ++k) cv[k] = __shfl(mc[k], source, kWave);
-    const uint32_t first = uint32_t(__shfl(int(my_first), source, kWave));
-    const float* j0r = c.jac + first * uint32_t(N);
-    const bool live = !none && row < c.n;
-    const uint32_t column = row < uint32_t(N) ? row : uint32_t(N - 1);
-    const float w0 = j0r[column], w1 = j0r[N + column], w2 = j0r[2 * N + column];
-    const float j0 = live ? w0 : 0.0f, j1 = live ? w1 : 0.0f, j2 = live ? w2 : 0.0f;
-    tile_add_product(g, j0, f[0]);
-    tile_add_product(g, j1, f[1]);
-    tile_add_product(g, j2, f[2]);
-    scale += (fabsf(j0) * noise[0] + fabsf(j1) * noise[1]) + fabsf(j2) * noise[2];
-    const float cxx = cv[0], cyy = cv[1], czz = cv[2], cxy = cv[3], cxz = cv[4], cyz = cv[5];
-    const float a0 = (j0 * cxx + j1 * cxy) + j2 * cxz;
-    const float a1 = (j1 * cyy + j2 * cyz) + j0 * cxy;
-    const float a2 = (j2 * czz + j1 * cyz) + j0 * cxz;
-    uint64_t columns = 0ull;
-#pragma unroll
-    for (int k = 0; k < G; ++k) {
-        if (heads[k] == kInvalid) continue;
-        columns |= (uint64_t(uint32_t(__builtin_amdgcn_readlane(int(my_high), int(heads[k])))) << 32u) |
-                   uint64_t(uint32_t(__builtin_amdgcn_readlane(int(my_low), int(heads[k]))));
-    }
-    add_column_groups<N>(std::make_integer_sequence<int, N / 4>{}, columns, 0u, lds_address(j0r), a0, a1, a2, hrow);
-}
-// v[lane] + v[lane + N] + ... over the groups of add_head_group, in the lanes of the first group
+constexpr uint32_t kGroupLanes = kGroups<N> == 2 ? 32u : uint32_t(N);
 template <int N>
 __device__ __forceinline__ float groups_sum(uint32_t lane, float v) {
     float total = v;
 #pragma unroll
-    for (int k = 1; k < kGroups<N>; ++k) total += __shfl(v, int(lane) + k * N, kWave);
+    for (int k = 1; k < kGroups<N>; ++k) total += __shfl(v, int(lane + uint32_t(k) * kGroupLanes<N>), kWave);
     return total;
 }
 template <int N>
@@ -1026,11 +860,91 @@ __device__ __forceinline__ double groups_sum(uint32_t lane, double v) {
     double total = v;
 #pragma unroll
     for (int k = 1; k < kGroups<N>; ++k) {
-        const uint32_t low = uint32_t(__shfl(int(uint32_t(bits)), int(lane) + k * N, kWave));
-        const uint32_t high = uint32_t(__shfl(int(uint32_t(bits >> 32u)), int(lane) + k * N, kWave));
+        const int from = int(lane + uint32_t(k) * kGroupLanes<N>);
+        const uint32_t low = uint32_t(__shfl(int(uint32_t(bits)), from, kWave));
+        const uint32_t high = uint32_t(__shfl(int(uint32_t(bits >> 32u)), from, kWave));
         total += __longlong_as_double((long long)((uint64_t(high) << 32u) | uint64_t(low)));
     }
     return total;
+}
+template <int N, bool kRows>
+__device__ __forceinline__ void add_heads_by_groups(const Tile& c, uint64_t heads, const float (&mf)[3], const float (&mc)[6], const float (&mn)[3],
+                                                    uint32_t my_first, float (&hrow)[N], TileSum& g, float& scale) {
+    static_assert(N <= 32, "two copies of the rows fit the wavefront");
+    constexpr int G = kGroups<N>;
+    const uint32_t lane = c.lane, group = lane / kGroupLanes<N>, row = lane - group * kGroupLanes<N>;
+    const int contributing = __popcll(heads);
+    const int taken_a_pass = contributing == 1 ? 1 : ((contributing + G - 1) / G < (contributing + 1) / 2 ? G : 2);
+    const bool single = contributing == 1 && c.U(hAxes, uint32_t(__builtin_ctzll(heads))) == 1u;
+    const uint32_t column = min(row, uint32_t(N - 1));
+    if (group != 0u) {
+        if constexpr (kRows) {
+#pragma unroll
+            for (int k = 0; k < N; ++k) hrow[k] = 0.0f;
+        }
+        g.value = 0.0; scale = 0.0f;
+    }
+    while (heads != 0ull) {
+        uint32_t mine = kInvalid;
+#pragma unroll
+        for (int k = 0; k < G; ++k) {
+            const uint32_t h = heads != 0ull && k < taken_a_pass ? uint32_t(__builtin_ctzll(heads)) : kInvalid;
+            if (k < taken_a_pass) heads &= heads - 1ull;   // zero stays zero
+            mine = group == uint32_t(k) ? h : mine;
+        }
+        const bool none = mine == kInvalid;   // also the lanes past the last group
+        const int source = int((none ? 0u : mine) * 4u);
+        const float* rows = c.jac + uint32_t(__builtin_amdgcn_ds_bpermute(source, int(my_first))) * uint32_t(N);
+        float f[3], noise[3];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) { f[k] = lane_permute(source, mf[k]); noise[k] = lane_permute(source, mn[k]); }
+        const bool live = !none && row < c.n;
+        // (read whether or not the lane uses them: a read under a condition compiles to a branch a word)
+        const float w0 = rows[column], w1 = rows[N + column], w2 = rows[2 * N + column];
+        const float j0 = live ? w0 : 0.0f, j1 = live ? w1 : 0.0f, j2 = live ? w2 : 0.0f;
+        tile_add_product(g, j0, f[0]);
+        tile_add_product(g, j1, f[1]);
+        tile_add_product(g, j2, f[2]);
+        scale += (fabsf(j0) * noise[0] + fabsf(j1) * noise[1]) + fabsf(j2) * noise[2];
+        if constexpr (kRows) {
+            float cv[6];
+#pragma unroll
+            for (int k = 0; k < 6; ++k) cv[k] = lane_permute(source, mc[k]);
+            const float cxx = cv[0], cyy = cv[1], czz = cv[2], cxy = cv[3], cxz = cv[4], cyz = cv[5];
+            const float a0 = (j0 * cxx + j1 * cxy) + j2 * cxz;
+            const float a1 = (j1 * cyy + j2 * cyz) + j0 * cxy;
+            const float a2 = (j2 * czz + j1 * cyz) + j0 * cxz;
+            if (single) {
+#pragma unroll
+                for (int q = 0; q < N / 4; ++q) add_columns_single<N>(q, rows + (lane & 3u), a0, hrow);
+            } else {
+#pragma unroll
+                for (int q = 0; q < N / 4; ++q) add_columns<N>(q, rows + (lane & 3u), a0, a1, a2, hrow);
+            }
+        }
+    }
+    if (contributing == 1) return;
+    g.value = groups_sum<N>(lane, g.value); scale = groups_sum<N>(lane, scale);
+    if constexpr (kRows) {
+#pragma unroll
+        for (int k = 1; k < G; ++k) {
+            float* exchange = k % 2 == 1 ? c.hrows : c.hfac;
+            if (group == uint32_t(k) && row < uint32_t(N)) {
+                float4* words = reinterpret_cast<float4*>(exchange + row * uint32_t(N));
+#pragma unroll
+                for (int q = 0; q < N / 4; ++q) words[q] = float4{hrow[4 * q], hrow[4 * q + 1], hrow[4 * q + 2], hrow[4 * q + 3]};
+            }
+            __syncthreads();
+            const float4* words = reinterpret_cast<const float4*>(exchange + column * uint32_t(N));
+#pragma unroll
+            for (int q = 0; q < N / 4; ++q) {
+                const float4 w = words[q];
+                if (group != 0u) continue;
+                hrow[4 * q] += w.x; hrow[4 * q + 1] += w.y; hrow[4 * q + 2] += w.z; hrow[4 * q + 3] += w.w;
+            }
+            __syncthreads();
+        }
+    }
 }
 
 // One head's line-search inputs in registers: nothing in them changes between the probes of one search, and neither
@@ -1429,11 +1343,11 @@ __device__ __forceinline__ void add_heads_through_links(const Tile& c, bool mine
 // AssembleTileBlock (:1507-1618): lane i assembles row i of H = M + sum J^T C J in `hrow` and its force g_i.  The
 // first 64 heads evaluate their response one per lane and hand it to the row lanes as scalar lane reads; heads beyond
 // 64 pass theirs through the head fields.
-// In a reduced block (kFollow) the mass row is the sum of two floats, `mrow` and `mlow`: the Schur complement as it comes
+// In a reduced block (kFollow) the mass row is the sum of two floats, `mrow` and low_row: the Schur complement as it comes
 // out of the double-precision elimination.  The force takes both parts, so that the velocity the block converges to
 // balances the momentum against the mass matrix itself; the Hessian takes the first.
 template <int N, bool kFollow>
-__device__ __forceinline__ bool assemble_block(const Tile& c, const float (&mrow)[N], const float (&mlow)[N], PlainLine& own, float u, float free_v,
+__device__ __forceinline__ bool assemble_block(const Tile& c, const float (&mrow)[N], PlainLine& own, float u, float free_v,
                                float (&hrow)[N], float* force, float* inertia, bool* converged) {
     const uint32_t lane = c.lane;
     const bool coordinate = lane < c.n;
@@ -1473,7 +1387,8 @@ __device__ __forceinline__ bool assemble_block(const Tile& c, const float (&mrow
     }
 #pragma unroll
     for (int k = 0; k < 6; ++k) { differs |= bits(c.curvature[k]) ^ bits(mc[k]); c.curvature[k] = mc[k]; }
-    if (__any(lane < c.heads && differs != 0u)) c.factor_current = false;
+    if (__any(lane < c.heads && differs != 0u)) { c.factor_current = false; c.rows_current = false; }
+    const bool rows_kept = N <= 32 && c.rows_current && c.heads <= uint32_t(kWave);   // only the force is to be summed
     if (c.units && lane < c.heads && c.U(hUnit, lane) != kInvalid) {   // a coordinate reads its unit heads' responses from the fields
         c.F(hF, lane) = mf[0]; c.F(hNoise, lane) = mn[0]; c.F(hC, lane) = mc[0];
         c.U(hContrib, lane) = mine ? 1u : 0u;
@@ -1486,6 +1401,8 @@ __device__ __forceinline__ bool assemble_block(const Tile& c, const float (&mrow
     TileSum inertial{0.0};
     double inertial_scale = 0.0;
     const double2* d2 = reinterpret_cast<const double2*>(dvec);
+    const float4* low4 = low_row<N>(c);
+    float4 low{};
 #pragma unroll
     for (int q = 0; q < N / 2; ++q) {
         const double2 dv = d2[q];
@@ -1498,10 +1415,9 @@ __device__ __forceinline__ bool assemble_block(const Tile& c, const float (&mrow
         inertial.value = fma(m0, dv.x, inertial.value);
         inertial.value = fma(m1, dv.y, inertial.value);
         if constexpr (kFollow) {
-            // (the low parts widened here, at every assembly: held widened over the solve beside the high parts they
-            // take the block past its registers)
-            inertial.value = fma(double(opaque_with(mlow[2 * q], u)), dv.x, inertial.value);
-            inertial.value = fma(double(opaque_with(mlow[2 * q + 1], u)), dv.y, inertial.value);
+            if (q % 2 == 0) low = low4[q / 2];
+            inertial.value = fma(double(q % 2 == 0 ? low.x : low.z), dv.x, inertial.value);
+            inertial.value = fma(double(q % 2 == 0 ? low.y : low.w), dv.y, inertial.value);
         }
         inertial_scale = fma(fabs(m0), fabs(dv.x), inertial_scale);
         inertial_scale = fma(fabs(m1), fabs(dv.y), inertial_scale);
@@ -1533,64 +1449,18 @@ __device__ __forceinline__ bool assemble_block(const Tile& c, const float (&mrow
         add_heads_force<N>(c, staged, mf, mn, lane < c.heads ? c.U(hRow, lane) : 0u, g, scale);
         add_heads_through_links<N>(c, mine, mc, hrow);
     } else {
-        bool added = false;
-        if constexpr (N <= 32 && !kFollow) {
-            if (staged != 0ull) add_heads_by_tiles<N>(c, staged, mf, mc, mn, c.U(hRow, lane < c.heads ? lane : 0u), hrow, g, scale);
-            added = true;
-        }
-        if constexpr (N <= 32 && kFollow) {
-            // two or more contributing heads (all of them staged, one a lane): two a pass, the second half of the
-            // wavefront collecting its heads in rows of its own
-            if ((staged & (staged - 1ull)) != 0ull) {
-                const uint32_t own_head = lane < c.heads ? lane : 0u;
-                const uint32_t my_first = c.U(hRow, own_head), my_low = c.U(hColumnsLow, own_head), my_high = c.U(hColumnsHigh, own_head);
-                if constexpr (N <= 20) {
-                    // where three or four copies of the rows fit the wavefront, that many heads a pass - when it takes fewer
-                    // passes than two a pass would (adding the groups' rows together costs more than adding two halves)
-                    const int contributing = __popcll(staged);
-                    if ((contributing + kGroups<N> - 1) / kGroups<N> < (contributing + 1) / 2) {
-                        if (lane >= uint32_t(N)) {
-#pragma unroll
-                            for (int k = 0; k < N; ++k) hrow[k] = 0.0f;
-                            g.value = 0.0; scale = 0.0f;
-                        }
-                        for (uint64_t rest = staged; rest != 0ull;) {
-                            uint32_t taken[4] = {kInvalid, kInvalid, kInvalid, kInvalid};
-#pragma unroll
-                            for (int k = 0; k < kGroups<N>; ++k) {
-                                if (rest == 0ull) break;
-                                taken[k] = uint32_t(__builtin_ctzll(rest));
-                                rest &= rest - 1ull;
-                            }
-                            add_head_group<N>(c, taken, mf, mc, mn, my_first, my_low, my_high, hrow, g, scale);
-                        }
-#pragma unroll
-                        for (int k = 0; k < N; ++k) hrow[k] = groups_sum<N>(lane, hrow[k]);
-                        g.value = groups_sum<N>(lane, g.value); scale = groups_sum<N>(lane, scale);
-                        added = true;
-                    }
-                }
-                if (!added) {
-                    if (lane >= 32u) {
-#pragma unroll
-                        for (int k = 0; k < N; ++k) hrow[k] = 0.0f;
-                        g.value = 0.0; scale = 0.0f;
-                    }
-                    for (uint64_t rest = staged; rest != 0ull;) {
-                        const uint32_t ha = uint32_t(__builtin_ctzll(rest));
-                        rest &= rest - 1ull;
-                        const uint32_t hb = rest != 0ull ? uint32_t(__builtin_ctzll(rest)) : kInvalid;
-                        rest &= rest - 1ull;   // zero stays zero
-                        add_head_pair<N>(c, ha, hb, mf, mc, mn, my_first, my_low, my_high, hrow, g, scale);
-                    }
-#pragma unroll
-                    for (int k = 0; k < N; ++k) hrow[k] = halves_sum(hrow[k]);
-                    g.value = halves_sum(g.value); scale = halves_sum(scale);
-                    added = true;
+        if constexpr (N <= 32) {
+            if (staged != 0ull) {
+                const uint32_t my_first = c.U(hRow, lane < c.heads ? lane : 0u);
+                if constexpr (kFollow) {
+                    if (rows_kept) add_heads_by_groups<N, false>(c, staged, mf, mc, mn, my_first, hrow, g, scale);
+                    else add_heads_by_groups<N, true>(c, staged, mf, mc, mn, my_first, hrow, g, scale);
+                } else {
+                    if (rows_kept) add_heads_by_tiles<N, false>(c, staged, mf, mc, mn, my_first, hrow, g, scale);
+                    else add_heads_by_tiles<N, true>(c, staged, mf, mc, mn, my_first, hrow, g, scale);
                 }
             }
-        }
-        if (!added && staged != 0ull) {
+        } else {
             const uint32_t own_head = lane < c.heads ? lane : 0u;
             const uint32_t my_axes = c.U(hAxes, own_head), my_low = c.U(hColumnsLow, own_head), my_high = c.U(hColumnsHigh, own_head);
             for (uint64_t rest = staged; rest != 0ull; rest &= rest - 1ull) {
@@ -1630,8 +1500,27 @@ __device__ __forceinline__ bool assemble_block(const Tile& c, const float (&mrow
             for (uint32_t h = 0u; h < c.heads; ++h)
                 if (c.U(hContrib, h) != 0u && c.U(hUnit, h) == lane) add_unit(h);
         }
+        if (!rows_kept) {
 #pragma unroll
-        for (int k = 0; k < N; ++k) hrow[k] += local_lane(lane) == uint32_t(k) ? diagonal : 0.0f;
+            for (int k = 0; k < N; ++k) hrow[k] += local_lane(lane) == uint32_t(k) ? diagonal : 0.0f;
+        }
+    }
+    if constexpr (N <= 32) {   // the rows as they stand, for the assemblies that find no curvature changed
+        if (!rows_kept) {
+            if (lane < uint32_t(N)) {
+                float4* words = reinterpret_cast<float4*>(c.hrows + lane * uint32_t(N));
+#pragma unroll
+                for (int q = 0; q < N / 4; ++q) words[q] = float4{hrow[4 * q], hrow[4 * q + 1], hrow[4 * q + 2], hrow[4 * q + 3]};
+            }
+            c.rows_current = true;
+        } else {
+            const float4* words = reinterpret_cast<const float4*>(c.hrows + min(lane, uint32_t(N - 1)) * uint32_t(N));
+#pragma unroll
+            for (int q = 0; q < N / 4; ++q) {
+                const float4 w = words[q];
+                hrow[4 * q] = w.x; hrow[4 * q + 1] = w.y; hrow[4 * q + 2] = w.z; hrow[4 * q + 3] = w.w;
+            }
+        }
     }
     PROF_END(c, 12);
     PROF_BEGIN(c, 13);
@@ -1693,13 +1582,13 @@ __device__ __forceinline__ float mass_times(const Tile& c, const float (&mrow)[N
 // convergence test because its mass factor overwrites the Hessian storage; here the two live apart and the
 // assembled row, force and inertia (which the second assembly would reproduce bit for bit) are simply kept.
 template <int N, bool kFollow>
-__device__ __forceinline__ Failure newton_direction(const Tile& c, const float (&mrow)[N], const float (&mlow)[N], PlainLine& line, float u, float free_v,
+__device__ __forceinline__ Failure newton_direction(const Tile& c, const float (&mrow)[N], PlainLine& line, float u, float free_v,
                                     float* force, float* inertia, float* d, bool* converged) {
     PROF_COUNT(c, 0);
     c.work += 16u;
     float hrow[N];
     PROF_BEGIN(c, 1);
-    const bool assembled = assemble_block<N, kFollow>(c, mrow, mlow, line, u, free_v, hrow, force, inertia, converged);
+    const bool assembled = assemble_block<N, kFollow>(c, mrow, line, u, free_v, hrow, force, inertia, converged);
     PROF_END(c, 1);
     if (!assembled) return kFailEquation;
     if (*converged && c.tolerance > 0.0f) {
@@ -1927,7 +1816,7 @@ __device__ __forceinline__ void apply_moves(const Tile& c, float alpha) {
 
 // DescendTileBlock (:2145-2301).  `u` is lane i's block coordinate; `has_free` is false in the position pass.
 template <int N, bool kFollow>
-__device__ __forceinline__ void descend_block(Tile& c, const float (&mrow)[N], const float (&mlow)[N], float* u_io, float free_in, bool has_free,
+__device__ __forceinline__ void descend_block(Tile& c, const float (&mrow)[N], float* u_io, float free_in, bool has_free,
                                               DataView d) {
     const uint32_t lane = c.lane, n = c.n;
     const bool coordinate = lane < n;
@@ -1971,7 +1860,7 @@ __device__ __forceinline__ void descend_block(Tile& c, const float (&mrow)[N], c
     for (uint32_t step = 0u; step < kNewtonSteps; ++step) {
         float force = 0.0f, inertia = 0.0f, dd = 0.0f;
         bool converged = false;
-        failure = newton_direction<N, kFollow>(c, mrow, mlow, line, u, free_v, &force, &inertia, &dd, &converged);
+        failure = newton_direction<N, kFollow>(c, mrow, line, u, free_v, &force, &inertia, &dd, &converged);
         if (converged) primal = 0.0f;
         if (failure != kFailNone || converged) break;
         if (!coordinate) dd = 0.0f;
@@ -2032,7 +1921,7 @@ __device__ __forceinline__ void descend_block(Tile& c, const float (&mrow)[N], c
 
 // MeasureTilePrimal (:2378-2489): the mass-normalised momentum balance in double
 template <int N, bool kFollow>
-__device__ __forceinline__ void measure_primal(Tile& c, const float (&mrow)[N], const float (&mlow)[N], float* velocity_io, float free_v,
+__device__ __forceinline__ void measure_primal(Tile& c, const float (&mrow)[N], float* velocity_io, float free_v,
                                const float* lambda_env, uint32_t R, bool reconstruct, DataView d) {
     const uint32_t lane = c.lane, n = c.n;
     const bool coordinate = lane < n;
@@ -2044,6 +1933,8 @@ __device__ __forceinline__ void measure_primal(Tile& c, const float (&mrow)[N], 
     __syncthreads();
     double balance = 0.0;
     const double2* apart2 = reinterpret_cast<const double2*>(apart);
+    const float4* low4 = low_row<N>(c);
+    float4 low{};
 #pragma unroll
     for (int q = 0; q < N / 2; ++q) {
         // the mass row does not change over the solve: left to itself the compiler widens all of it to double once,
@@ -2052,8 +1943,9 @@ __device__ __forceinline__ void measure_primal(Tile& c, const float (&mrow)[N], 
         balance = fma(-double(opaque_with(mrow[2 * q], here)), dv.x, balance);
         balance = fma(-double(opaque_with(mrow[2 * q + 1], here)), dv.y, balance);
         if constexpr (kFollow) {
-            balance = fma(-double(opaque_with(mlow[2 * q], here)), dv.x, balance);
-            balance = fma(-double(opaque_with(mlow[2 * q + 1], here)), dv.y, balance);
+            if (q % 2 == 0) low = low4[q / 2];
+            balance = fma(-double(q % 2 == 0 ? low.x : low.z), dv.x, balance);
+            balance = fma(-double(q % 2 == 0 ? low.y : low.w), dv.y, balance);
         }
     }
     // heads with an impulse add J^T lambda in head order (:2402-2436).  A unit head touches one coordinate: that
@@ -2340,6 +2232,11 @@ __host__ __device__ inline uint32_t ReductionScratchFloats(uint32_t full, uint32
 }
 // the coordinates' motion axes of a wide block (Tile::axes), twelve words a coordinate
 __host__ __device__ inline uint32_t LinkAxisFloats(uint32_t n) { return PaddedWidth(n) > uint32_t(kTwoWaveWidth) ? 12u * uint32_t(kWave) : 0u; }
+// the kept Hessian rows of a narrow block (Tile::hrows), and the second floats of a reduced block's mass rows (Tile::low)
+__host__ __device__ inline uint32_t KeptRowFloats(uint32_t n, bool reduced) {
+    const uint32_t N = PaddedWidth(n);
+    return N > 32u ? 0u : (reduced ? 2u : 1u) * N * N;
+}
 __host__ __device__ inline uint32_t HeadFieldFloats(uint32_t cap, uint32_t narrow) {
     return (kWideStride * cap + kNarrowStride * (narrow + 1u) + 3u) & ~3u;
 }
@@ -2352,15 +2249,15 @@ __host__ __device__ inline bool RowsFromLinks(uint32_t n, bool contacts_only, ui
 __host__ __device__ inline uint32_t RowFloats(uint32_t N, uint32_t staged, bool from_links) {
     return from_links ? (kWrenchStride * staged + 3u) & ~3u : 3u * staged * N;
 }
-__host__ __device__ inline uint32_t SolverLdsFloats(uint32_t n, uint32_t cap, uint32_t staged, bool from_links = false) {
+__host__ __device__ inline uint32_t SolverLdsFloats(uint32_t n, uint32_t cap, uint32_t staged, bool from_links = false, bool reduced = false) {
     const uint32_t N = PaddedWidth(n);
     // the per-coordinate unit lists exist only when some head beyond the staged ones can be listed; without joint rows
     // the block keeps the footprint that lets eight of them share a compute unit's LDS
     return FactorRegionFloats(n) + RowFloats(N, staged, from_links) + HeadFieldFloats(cap, staged) + 256u +
-           (cap > staged ? kUnitSlots * uint32_t(kWave) : 0u) + LinkAxisFloats(n);
+           (cap > staged ? kUnitSlots * uint32_t(kWave) : 0u) + LinkAxisFloats(n) + KeptRowFloats(n, reduced);
 }
 __host__ __device__ inline uint32_t ReducedSolverLdsFloats(uint32_t full, uint32_t reduced, uint32_t cap, uint32_t staged, bool from_links = false) {
-    const uint32_t solve = SolverLdsFloats(reduced, cap, staged, from_links), scratch = ReductionScratchFloats(full, reduced);
+    const uint32_t solve = SolverLdsFloats(reduced, cap, staged, from_links, reduced < full), scratch = ReductionScratchFloats(full, reduced);
     return solve > scratch ? solve : scratch;
 }
 
@@ -2372,11 +2269,12 @@ __host__ __device__ inline uint32_t ReducedSolverLdsFloats(uint32_t full, uint32
 // their rows of the Schur complement S = M_TT - M_TU M_UU^-1 M_UT and of U_TU = M_TU U_UU^-T, the followers with their
 // rows of the factor M_UU = U_UU U_UU^T.  P = M_UU^-1 M_UT = U_UU^-T U_TU^T then follows by forward substitution over the
 // followers in ascending order, its two operands passing through LDS to be read transposed.  On return a lane below K
-// holds its row of S as the sum mrow + mlow of two floats, a follower its row of -P rounded to float in mrow.
+// holds its row of S as the sum of two floats, mrow in registers and the second in LDS at `low` (read by low_row), a
+// follower its row of -P rounded to float in mrow.
 // Double because these rows stand in for the mass matrix over the whole solve: a Schur complement eliminated in
 // single precision moves the velocities the solve converges to by a few 1e-5 of the contact impulse's effect.
 template <int N, int K>
-__device__ __forceinline__ bool reduce_block(uint32_t lane, uint32_t n, const float* mass, uint32_t md, float* lds, float (&mrow)[K], float (&mlow)[K]) {
+__device__ __forceinline__ bool reduce_block(uint32_t lane, uint32_t n, const float* mass, uint32_t md, float* lds, float* low, float (&mrow)[K]) {
     constexpr int kFollowers = N - K;
     const bool row_lane = lane < n;
     double full[N];
@@ -2452,11 +2350,17 @@ __device__ __forceinline__ bool reduce_block(uint32_t lane, uint32_t n, const fl
             prow[c0] = fma(column[i - K], -y, prow[c0]);   // (the column holds zeros for the followers up to i)
         }
     }
+    float rest[K];
 #pragma unroll
     for (int k = 0; k < K; ++k) {
         const double entry = lane < uint32_t(K) ? full[k] : (lane < n ? -(prow[k] * own_scale) : 0.0);
         mrow[k] = float(entry);
-        mlow[k] = lane < uint32_t(K) ? float(entry - double(mrow[k])) : 0.0f;
+        rest[k] = float(entry - double(mrow[k]));
+    }
+    if (lane < uint32_t(K)) {   // (the scratch above has been read: its words may be these)
+        float4* words = reinterpret_cast<float4*>(low + lane * uint32_t(K));
+#pragma unroll
+        for (int q = 0; q < K / 4; ++q) words[q] = float4{rest[4 * q], rest[4 * q + 1], rest[4 * q + 2], rest[4 * q + 3]};
     }
     __syncthreads();
     return valid;
@@ -2488,7 +2392,7 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
     c.env = env; c.lane = lane; c.n = kReduced ? uint32_t(K) : n; c.n_all = n; c.ldj = uint32_t(W); c.cap = cap; c.narrow = staged_cap; c.heads = 0u; c.iteration = 0u;
     c.tolerance = p.velocity_tolerance; c.failed = false; c.momentum = 0.0f; c.residual = 0.0f;
     c.mass_inverse = 0.0f; c.mass_valid = false; c.work = 0u; c.units = false; c.elliptic = false;
-    c.factor_current = false; c.factor_root = 1.0f;
+    c.factor_current = false; c.rows_current = false; c.factor_root = 1.0f;
     for (float& entry : c.curvature) entry = 0.0f;
 #ifdef NKH_SOLVER_PROFILE
     for (int i = 0; i < 32; ++i) c.prof[i] = 0;
@@ -2509,23 +2413,22 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
     c.wrench = c.jac;   // one or the other
     c.fields = c.jac + RowFloats(uint32_t(W), staged_cap, c.from_links);
     c.vec = c.fields + HeadFieldFloats(cap, staged_cap);
+    c.hrows = c.vec + 256 + (cap > staged_cap ? kUnitSlots * uint32_t(kWave) : 0u);
+    c.low = c.hrows + uint32_t(W) * uint32_t(W);
     // The block's mass rows: lane's row of M, or in a reduced block lane's row of the Schur complement (lanes below K)
     // and of -P (the followers).
-    float mrow[W], mlow[W];
+    float mrow[W];
     bool reduction_valid = true;
     if constexpr (kReduced) {
         PROF_BEGIN(c, 30);
-        reduction_valid = reduce_block<N, K>(lane, n, d.m + size_t{env} * md * md + size_t{lane < n ? lane : 0u} * md, md, lds, mrow, mlow);
+        reduction_valid = reduce_block<N, K>(lane, n, d.m + size_t{env} * md * md + size_t{lane < n ? lane : 0u} * md, md, lds, c.low, mrow);
         PROF_END(c, 30);
-    } else {
-#pragma unroll
-        for (int k = 0; k < W; ++k) mlow[k] = 0.0f;   // never read
     }
     if (lane < kNarrowFields) c.fields[kWideStride * cap + staged_cap * kNarrowStride + lane] = 0.0f;   // what a narrow field reads beyond its heads
     c.unit_list = reinterpret_cast<uint32_t*>(c.vec + 256);
     c.unit_lists = true; c.unit_count = 0u; c.staged_end = 0u; c.individual_end = 0u;
     c.through_links = false;
-    c.axes = c.vec + 256 + (cap > staged_cap ? kUnitSlots * uint32_t(kWave) : 0u);
+    c.axes = c.vec + 256 + (cap > staged_cap ? kUnitSlots * uint32_t(kWave) : 0u);   // a wide block's; a narrow one keeps rows here
     c.path_low = c.path_high = c.under_low = c.under_high = 0u;
     c.rows = d.urows; c.row_point_a = d.row_cj_point; c.row_point_b = d.row_cj_point_b; c.row_link_a = d.row_cj_link; c.row_link_b = d.row_cj_link_b;
     c.link_paths = m.link_dof_mask; c.first_link = env * nl;
@@ -3078,22 +2981,22 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
         c.iteration = sweeps++;
         c.momentum = 0.0f; c.residual = 0.0f;
         PROF_COUNT(c, 2);
-        descend_block<W, kReduced>(c, mrow, mlow, &velocity, free_v, true, d);
+        descend_block<W, kReduced>(c, mrow, &velocity, free_v, true, d);
         float rowsr[3];
         PROF_BEGIN(c, 6);
         update_duals(c, lambda_env, R, urows, &momentum, true, true, rowsr);
         PROF_END(c, 6);
         PROF_BEGIN(c, 7);
         if (sweeps == p.iterations || fmaxf(fmaxf(rowsr[0], rowsr[1]), fmaxf(rowsr[2], c.residual)) < tol)
-            measure_primal<W, kReduced>(c, mrow, mlow, &velocity, free_v, lambda_env, R, false, d);
+            measure_primal<W, kReduced>(c, mrow, &velocity, free_v, lambda_env, R, false, d);
         PROF_END(c, 7);
         if (fmaxf(fmaxf(rowsr[0], rowsr[1]), rowsr[2]) < tol && c.residual >= tol && c.residual < FLT_MAX) {
-            measure_primal<W, kReduced>(c, mrow, mlow, &velocity, free_v, lambda_env, R, true, d);
+            measure_primal<W, kReduced>(c, mrow, &velocity, free_v, lambda_env, R, true, d);
             if (c.residual < FLT_MAX) {
                 initialize_residuals<W>(c, velocity, urows, p.dt);
                 update_duals(c, lambda_env, R, urows, nullptr, true, false, rowsr);
                 c.residual = 0.0f;
-                measure_primal<W, kReduced>(c, mrow, mlow, &velocity, free_v, lambda_env, R, false, d);
+                measure_primal<W, kReduced>(c, mrow, &velocity, free_v, lambda_env, R, false, d);
             }
         }
         residual4[0] = rowsr[0]; residual4[1] = rowsr[1]; residual4[2] = rowsr[2]; residual4[3] = c.residual;
@@ -3212,7 +3115,7 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
             const uint32_t positions = 1u;   // no head couples two moving blocks here, so one solve (:2716)
             for (uint32_t iteration = 0u; iteration < positions; ++iteration) {
                 c.iteration = sweeps + iteration;
-                descend_block<W, kReduced>(c, mrow, mlow, &pseudo, 0.0f, false, d);
+                descend_block<W, kReduced>(c, mrow, &pseudo, 0.0f, false, d);
             }
         }
         // FinishTilePositions (:2720-2744)
