@@ -468,7 +468,11 @@ struct World {   // src/c_abi/internal.hpp:153-165 WorldRecord + nk::World
     std::vector<std::string> link_names, joint_names;   // per template link; a joint's name sits at its child link
     nuka_phi_execution_error last_error{};
 
+    uint32_t* reset_ids = nullptr;       // nuka_world_reset_envs: pinned host memory, env_count words, from its first call on
+    std::vector<uint8_t> reset_seen;     // and the environments that call has met
+
     ~World() {
+        if (reset_ids != nullptr) (void)hipHostFree(reset_ids);
         if (be != nullptr && plan != nullptr) be->plan_free(backend, plan);
         if (arena != nullptr) reinterpret_cast<nuka_phi_buffer_head*>(arena)->iface->free(arena);
         if (initial != nullptr) reinterpret_cast<nuka_phi_buffer_head*>(initial)->iface->free(initial);
@@ -1263,21 +1267,29 @@ nuka_result_t nuka_world_reset_envs(nuka_world_handle world, const uint32_t* env
     if (count == 0u) return NUKA_RESULT_OK;
     if (env_ids == nullptr) return Error(NUKA_RESULT_INVALID_ARG, "env_ids is null");
     // an invalid id changes nothing; duplicates are dropped so that no two workgroups write one slice
-    std::vector<uint8_t> seen(w->env_count, 0u);
-    std::vector<uint32_t> unique;
-    for (uint32_t i = 0u; i < count; ++i) {
+    for (uint32_t i = 0u; i < count; ++i)
         if (env_ids[i] >= w->env_count) return Error(NUKA_RESULT_INVALID_ARG, "environment id out of range");
-        if (seen[env_ids[i]] == 0u) { seen[env_ids[i]] = 1u; unique.push_back(env_ids[i]); }
+    // The upload is from pinned memory of the world's own, so it is enqueued like the kernel, and the one wait at the end is
+    // the call's contract.  A first wait, before an upload from pageable memory, left the device idle between the steps
+    // already submitted and the reset.
+    if (w->reset_ids == nullptr &&
+        hipHostMalloc(reinterpret_cast<void**>(&w->reset_ids), size_t{w->env_count} * sizeof(uint32_t), hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
+        w->reset_ids = nullptr;
+        return Error(NUKA_RESULT_OUT_OF_MEMORY, "reset ids");
     }
     ResetSegments segments{};
     if (ResetSegmentsOf(w, &segments) != NUKA_RESULT_OK) return Error(NUKA_RESULT_INTERNAL, "too many reset segments");
-    if (nuka_world_synchronize(world) != NUKA_RESULT_OK) return NUKA_RESULT_DEVICE_ERROR;
-    if (hipMemcpyAsync(w->data.reset_env_ids, unique.data(), unique.size() * sizeof(uint32_t), hipMemcpyHostToDevice,
-                       BackendStream(w->device->backend)) != hipSuccess) return Error(NUKA_RESULT_DEVICE_ERROR, "id upload failed");
-    hipLaunchKernelGGL(ResetEnvsKernel, dim3(uint32_t(unique.size()), segments.count), dim3(256), 0, BackendStream(w->device->backend),
-                       segments, w->data.reset_env_ids, w->env_count);
+    w->reset_seen.assign(w->env_count, 0u);
+    uint32_t unique = 0u;
+    for (uint32_t i = 0u; i < count; ++i)
+        if (w->reset_seen[env_ids[i]] == 0u) { w->reset_seen[env_ids[i]] = 1u; w->reset_ids[unique++] = env_ids[i]; }
+    hipStream_t stream = BackendStream(w->device->backend);
+    if (hipMemcpyAsync(w->data.reset_env_ids, w->reset_ids, size_t{unique} * sizeof(uint32_t), hipMemcpyHostToDevice, stream) != hipSuccess)
+        return Error(NUKA_RESULT_DEVICE_ERROR, "id upload failed");
+    hipLaunchKernelGGL(ResetEnvsKernel, dim3(unique, segments.count), dim3(256), 0, stream, segments, w->data.reset_env_ids, w->env_count);
     if (hipGetLastError() != hipSuccess) return Error(NUKA_RESULT_DEVICE_ERROR, "reset launch failed");
-    return nuka_world_synchronize(world);   // the host copy of the ids must outlive the upload
+    return nuka_world_synchronize(world);   // the ids may be written again
 }
 
 // nuka_world_reset_envs for callers that cannot allocate: same kernel, same result, but the ids are staged in the
