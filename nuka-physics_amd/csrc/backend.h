@@ -11,6 +11,8 @@ namespace nkh {
 // A backend on `device`; `borrowed_stream` non-null is used as is, else an owned stream at default priority.
 void* CreateBackend(int device, void* borrowed_stream);
 hipStream_t BackendStream(void* backend);
+// one launch for the first op of the list, or for the first few where a merged kernel runs them (`served` of them), as in a plan
+Status BackendDispatchNext(void* backend, const ModelView& m, const DataView& d, const nuka_phi_op_call* calls, int n, int* served);
 nuka_phi_buffer_type* BackendDeviceBufferType(void* backend);
 nuka_phi_buffer_type* BackendHostBufferType(void* backend);
 bool BackendSupportsOp(NkOp op);

@@ -180,6 +180,18 @@ int MergeCollisionHead(Backend* be, const ModelView& m, const DataView& d, const
     return status == Status::Ok ? 5 : 0;
 }
 
+// The next launch of an op list: the ops after the solve, and those between the dynamics and the row assembly, each take
+// about a launch's time, so where the list holds them in a row one kernel runs them (StepTailKernel, CollisionHeadKernel);
+// where it cannot, the first op goes alone.  `served` is the number of ops that the launch covers.
+Status DispatchNext(Backend* be, const ModelView& m, const DataView& d, const nuka_phi_op_call* calls, int n, int* served) {
+    Status status = Status::Ok;
+    *served = MergeStepTail(be, m, d, calls, n, &status);
+    if (*served == 0 && status == Status::Ok) *served = MergeCollisionHead(be, m, d, calls, n, &status);
+    if (*served > 0 || status != Status::Ok) return status;
+    *served = 1;
+    return DispatchOn(be, m, d, calls[0]);
+}
+
 uint8_t BeDispatch(nuka_phi_backend* b, const nuka_phi_model_view* m, const nuka_phi_data_view* d, const nuka_phi_op_call* call) {
     if (b == nullptr || m == nullptr || d == nullptr || call == nullptr) return uint8_t(Status::InvalidArgument);
     return uint8_t(DispatchOn(reinterpret_cast<Backend*>(b), *reinterpret_cast<const ModelView*>(m),
@@ -216,15 +228,8 @@ nuka_phi_plan* BePlanCreate(nuka_phi_backend* b, const nuka_phi_model_view* m, c
     uint16_t failed = uint16_t(NkOp::Count);
     const ModelView& model = *reinterpret_cast<const ModelView*>(m);
     const DataView& data = *reinterpret_cast<const DataView*>(d);
-    for (int i = 0; i < n_calls && status == Status::Ok; ++i) {
-        // The ops after the solve, and those between the dynamics and the row assembly, each take about a launch's time:
-        // where the list holds them in a row, one kernel runs them (StepTailKernel, CollisionHeadKernel); where it cannot,
-        // they go one by one as dispatched.
-        int merged = MergeStepTail(be, model, data, calls + i, n_calls - i, &status);
-        if (merged == 0 && status == Status::Ok) merged = MergeCollisionHead(be, model, data, calls + i, n_calls - i, &status);
-        if (status != Status::Ok) { failed = calls[i].op; break; }
-        if (merged > 0) { i += merged - 1; continue; }
-        status = DispatchOn(be, model, data, calls[i]);
+    for (int i = 0, served = 0; i < n_calls && status == Status::Ok; i += served) {
+        status = DispatchNext(be, model, data, calls + i, n_calls - i, &served);
         if (status != Status::Ok) failed = calls[i].op;
     }
     hipGraph_t graph = nullptr;
@@ -383,6 +388,9 @@ void* CreateBackend(int device, void* borrowed_stream) {
     return be;
 }
 
+Status BackendDispatchNext(void* backend, const ModelView& m, const DataView& d, const nuka_phi_op_call* calls, int n, int* served) {
+    return DispatchNext(static_cast<Backend*>(backend), m, d, calls, n, served);
+}
 hipStream_t BackendStream(void* backend) { return static_cast<Backend*>(backend)->stream; }
 nuka_phi_buffer_type* BackendDeviceBufferType(void* backend) { return reinterpret_cast<nuka_phi_buffer_type*>(&static_cast<Backend*>(backend)->device_type); }
 nuka_phi_buffer_type* BackendHostBufferType(void* backend) { return reinterpret_cast<nuka_phi_buffer_type*>(&static_cast<Backend*>(backend)->host_type); }
