@@ -149,6 +149,7 @@ struct DataView {
     uint64_t *ucontact_id_pair, *ucontact_id_feature;
     float *urows, *lambda, *row_penetration, *row_cj_point, *row_cj_point_b, *chain_jacobian, *chain_jacobian_b;
     uint32_t *row_cj_link, *row_cj_link_b, *row_count, *contact_count, *contact_row_extent;
+    uint32_t *row_clear_extent;             // contact rows from here (less one) on are clear in memory, whatever contact_row_extent says
     uint32_t *env_status, *vbd_velocity_sweep_count;
     float *solver_residual, *solver_penalty;
     float *solver_velocity, *solver_free;   // block velocities kept between solves (carried constraint velocity)

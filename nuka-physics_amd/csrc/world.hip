@@ -376,7 +376,7 @@ struct Field { const char* name; Dtype dtype; uint32_t elem_bytes; size_t count;
     X(urows, kF32, E * R * 26) X(lambda, kF32, E * R) X(row_penetration, kF32, E * R) X(row_cj_point, kF32, E * R * 3) \
     X(row_cj_point_b, kF32, E * R * 3) X(chain_jacobian, kF32, E * R * md) X(chain_jacobian_b, kF32, E * R * md) \
     X(row_cj_link, kU32, E * R) X(row_cj_link_b, kU32, E * R) X(row_count, kU32, E) X(contact_count, kU32, E) \
-    X(contact_row_extent, kU32, E * 2) X(env_status, kU32, E) X(vbd_velocity_sweep_count, kU32, E) \
+    X(contact_row_extent, kU32, E * 2) X(row_clear_extent, kU32, E) X(env_status, kU32, E) X(vbd_velocity_sweep_count, kU32, E) \
     X(solver_residual, kF32, E * 4) X(solver_penalty, kF32, E * R) X(solver_velocity, kF32, E * md) X(solver_free, kF32, E * md) \
     X(solver_cost, kU32, E) X(tile_order, kU32, E) X(row_unit, kU32, E * R) X(row_unit_value, kF32, E * R) \
     X(solver_mass_factor, kF32, E * mf) \
