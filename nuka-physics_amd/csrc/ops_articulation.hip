@@ -130,12 +130,28 @@ __device__ void motion_subspace(uint8_t type, V3 axis, float* s) {
 }
 
 // ---- FkWorldPoses ---------------------------------------------------------------------------------------
-// One wavefront, one environment; `pose` holds nl * 7 words of LDS
-__device__ __forceinline__ void world_poses_of_env(const ModelView& m, const DataView& d, uint32_t env, uint32_t lane, float* pose) {
-    const uint32_t nl = m.links_per_env;
-    const float* q = d.q + size_t{env} * nl;
-    // A link's frame in its parent does not wait on the tree: every lane computes its own link's before the sweep, which
-    // then only composes a depth at a time (links past the 64th compute theirs when their depth comes).
+// The sweeps down the tree give a link a lane, and an environment `G` lanes of a wavefront: where its links need no more
+// than half, a quarter or an eighth of one, as many environments share it, and each instruction serves them all
+// (the poses of 31 links: 127 us a wavefront each, 70 us two a wavefront, at 65536 environments; of 8 links: 32 and 9 us at
+// 20011).  The sharing stops where it would leave one of the chip's 1024 SIMDs without a wavefront.  More than 64 links take
+// two each ("128 lanes"): prepared ahead like the first, where a link that is prepared again at every depth of a 65-link
+// chain doubled its sweep (227 and 106 us at 8192).
+constexpr uint32_t kSimds = 1024u;
+inline uint32_t LanesAnEnvironment(uint32_t links, uint32_t envs) {
+    if (links > 64u) return 128u;
+    uint32_t lanes = 64u;
+    while (lanes > 8u && links <= lanes / 2u && uint64_t{envs} * (lanes / 2u) >= uint64_t{kSimds} * 64u) lanes /= 2u;
+    return lanes;
+}
+
+// One environment by `G` lanes of one wavefront (128: by all 64, two links each); `pose` holds nl * 7 words of LDS.  Every lane of the wavefront is in the
+// call, those without an environment with `there` false.
+template <int G>
+__device__ __forceinline__ void world_poses_of_env(const ModelView& m, const DataView& d, uint32_t env, uint32_t lane, bool there, float* pose) {
+    const uint32_t nl = there ? m.links_per_env : 0u;
+    const float* q = d.q + size_t{env} * m.links_per_env;
+    // A link's frame in its parent does not wait on the tree: every lane computes its own links' before the sweep, which
+    // then only composes a depth at a time (links past the second a lane compute theirs when their depth comes).
     struct Placed { uint32_t depth, parent; Xf frame; };
     auto place = [&](uint32_t l) {
         const uint8_t type = m.joint_type[l];
@@ -147,23 +163,33 @@ __device__ __forceinline__ void world_poses_of_env(const ModelView& m, const Dat
     auto compose = [&](uint32_t l, const Placed& t) {
         store_xf(pose + 7u * l, t.parent == kInvalid ? t.frame : compose_frame(load_xf(pose + 7u * t.parent), t.frame));
     };
-    Placed own{kInvalid, kInvalid, Xf{}};
-    if (lane < nl) own = place(lane);
+    constexpr int kOwn = G > kWave ? 2 : 1, kLanes = G / kOwn;   // fewer links than nl only past the second a lane
+    Placed own[kOwn];
+#pragma unroll
+    for (int i = 0; i < kOwn; ++i) {
+        own[i] = Placed{kInvalid, kInvalid, Xf{}};
+        if (lane + uint32_t(i * kLanes) < nl) own[i] = place(lane + uint32_t(i * kLanes));
+    }
     for (uint32_t depth = 0u; depth <= m.max_depth; ++depth) {
-        if (own.depth == depth) compose(lane, own);
-        for (uint32_t l = lane + kWave; l < nl; l += kWave) {
-            const Placed t = place(l);
-            if (t.depth == depth) compose(l, t);
-        }
+#pragma unroll
+        for (int i = 0; i < kOwn; ++i)
+            if (own[i].depth == depth) compose(lane + uint32_t(i * kLanes), own[i]);
+        if (G > kWave)
+            for (uint32_t l = lane + 2u * kWave; l < nl; l += kWave) {
+                const Placed t = place(l);
+                if (t.depth == depth) compose(l, t);
+            }
         wave_sync();
     }
-    float* out = d.link_pose + size_t{env} * nl * 7u;
-    for (uint32_t e = lane; e < nl * 7u; e += kWave) out[e] = pose[e];
+    float* out = d.link_pose + size_t{env} * m.links_per_env * 7u;
+    for (uint32_t e = lane; e < nl * 7u; e += kLanes) out[e] = pose[e];
 }
+template <int G>
 __global__ void __launch_bounds__(kWave) FkWorldPosesKernel(ModelView m, DataView d, uint32_t env_count) {
     extern __shared__ float lds[];
-    if (blockIdx.x >= env_count) return;
-    world_poses_of_env(m, d, blockIdx.x, threadIdx.x, lds);
+    constexpr uint32_t kLanes = G < kWave ? G : kWave;
+    const uint32_t group = threadIdx.x / kLanes, env = blockIdx.x * (kWave / kLanes) + group;
+    world_poses_of_env<G>(m, d, env, threadIdx.x % kLanes, env < env_count, lds + group * m.links_per_env * 7u);
 }
 
 // ---- ArticulationDynamics -------------------------------------------------------------------------------
@@ -590,13 +616,15 @@ __global__ void IntegratePositionKernel(ModelView m, DataView d, IntegratePositi
 }
 
 // ---- FkLinkVelocities (articulation.cu:647-689) ---------------------------------------------------------
-// One wavefront, one environment; `v` holds nl * 6 words of LDS
-__device__ __forceinline__ void link_velocities_of_env(const ModelView& m, const DataView& d, uint32_t env, uint32_t lane, float* v) {
-    const uint32_t nl = m.links_per_env;
-    const size_t lbase = size_t{env} * nl;
-    for (uint32_t e = lane; e < nl * 6u; e += kWave) v[e] = d.link_velocity[lbase * 6u + e];
+// One environment by `G` lanes of one wavefront, as world_poses_of_env; `v` holds nl * 6 words of LDS
+template <int G>
+__device__ __forceinline__ void link_velocities_of_env(const ModelView& m, const DataView& d, uint32_t env, uint32_t lane, bool there, float* v) {
+    const uint32_t nl = there ? m.links_per_env : 0u;
+    const size_t lbase = size_t{env} * m.links_per_env;
+    constexpr int kOwn = G > kWave ? 2 : 1, kLanes = G / kOwn;
+    for (uint32_t e = lane; e < nl * 6u; e += kLanes) v[e] = d.link_velocity[lbase * 6u + e];
     wave_sync();
-    // the joint transform and the joint's own twist do not wait on the tree: a lane prepares its link's before the sweep
+    // the joint transform and the joint's own twist do not wait on the tree: a lane prepares its links' before the sweep
     struct Jointed { uint32_t depth, parent; bool state; float X[36], own[6]; };
     auto prepare = [&](uint32_t l, Jointed& t) {
         const uint8_t type = m.joint_type[l];
@@ -621,44 +649,67 @@ __device__ __forceinline__ void link_velocities_of_env(const ModelView& m, const
 #pragma unroll
         for (int c = 0; c < 6; ++c) v[6u * l + c] = vl[c] + t.own[c];
     };
-    Jointed own;
-    own.depth = kInvalid; own.parent = kInvalid; own.state = true;
-    if (lane < nl) prepare(lane, own);
+    Jointed own[kOwn];
+#pragma unroll
+    for (int i = 0; i < kOwn; ++i) {
+        own[i].depth = kInvalid; own[i].parent = kInvalid; own[i].state = true;
+        if (lane + uint32_t(i * kLanes) < nl) prepare(lane + uint32_t(i * kLanes), own[i]);
+    }
     for (uint32_t depth = 0u; depth <= m.max_depth; ++depth) {
-        if (own.depth == depth) propagate(lane, own);
-        for (uint32_t l = lane + kWave; l < nl; l += kWave) {
-            Jointed t;
-            prepare(l, t);
-            if (t.depth == depth) propagate(l, t);
-        }
+#pragma unroll
+        for (int i = 0; i < kOwn; ++i)
+            if (own[i].depth == depth) propagate(lane + uint32_t(i * kLanes), own[i]);
+        if (G > kWave)
+            for (uint32_t l = lane + 2u * kWave; l < nl; l += kWave) {
+                Jointed t;
+                prepare(l, t);
+                if (t.depth == depth) propagate(l, t);
+            }
         wave_sync();
     }
-    for (uint32_t e = lane; e < nl * 6u; e += kWave) d.link_velocity[lbase * 6u + e] = v[e];
+    for (uint32_t e = lane; e < nl * 6u; e += kLanes) d.link_velocity[lbase * 6u + e] = v[e];
 }
+template <int G>
 __global__ void __launch_bounds__(kWave) FkLinkVelocitiesKernel(ModelView m, DataView d, uint32_t env_count) {
     extern __shared__ float lds[];
-    if (blockIdx.x >= env_count) return;
-    link_velocities_of_env(m, d, blockIdx.x, threadIdx.x, lds);
+    constexpr uint32_t kLanes = G < kWave ? G : kWave;
+    const uint32_t group = threadIdx.x / kLanes, env = blockIdx.x * (kWave / kLanes) + group;
+    link_velocities_of_env<G>(m, d, env, threadIdx.x % kLanes, env < env_count, lds + group * m.links_per_env * 6u);
 }
 
 // What follows the solve in a step - positions integrated, world poses, link twists, the bodies' poses - as one kernel,
-// one wavefront an environment: four kernels that each take about the time of a launch become one, running the same
-// device code in the same order (IntegratePosition, FkWorldPoses, FkLinkVelocities, SyncLinkBodyPose).  A plan takes this
-// route when its op list holds the four in a row (backend.hip); an op dispatched by itself runs its own kernel.
+// `G` lanes of two wavefronts an environment: four kernels that each take about the time of a launch become one, running
+// the same device code in the same order (IntegratePosition, FkWorldPoses, FkLinkVelocities, SyncLinkBodyPose).  A plan
+// takes this route when its op list holds the four in a row (backend.hip); an op dispatched by itself runs its own kernel.
+template <int G>
 __global__ void __launch_bounds__(2 * kWave) StepTailKernel(ModelView m, DataView d, IntegratePositionParams p, uint32_t env_count,
                                                             uint32_t sync_bodies) {
     extern __shared__ float lds[];
-    const uint32_t env = blockIdx.x, lane = threadIdx.x % kWave, nl = m.links_per_env;
+    constexpr uint32_t kLanes = G < kWave ? G : kWave, kEnvs = kWave / kLanes;
+    const uint32_t lane = threadIdx.x % kLanes, group = threadIdx.x % kWave / kLanes, env = blockIdx.x * kEnvs + group, nl = m.links_per_env;
     const bool twists = threadIdx.x >= uint32_t(kWave);   // world poses and link twists do not depend on each other: a wavefront each
-    if (env >= env_count) return;
-    if (!twists) for (uint32_t l = lane; l < nl; l += kWave) integrate_position_of_link(m, d, p, env, l);
+    const bool there = env < env_count;
+    if (!twists && there) for (uint32_t l = lane; l < nl; l += kLanes) integrate_position_of_link(m, d, p, env, l);
     __syncthreads();   // the new coordinates, base pose and root twist are in memory for both wavefronts
-    if (twists) { link_velocities_of_env(m, d, env, lane, lds + nl * 7u); return; }
-    world_poses_of_env(m, d, env, lane, lds);
-    if (sync_bodies == 0u) return;
+    if (twists) { link_velocities_of_env<G>(m, d, env, lane, there, lds + kEnvs * nl * 7u + group * nl * 6u); return; }
+    float* pose = lds + group * nl * 7u;
+    world_poses_of_env<G>(m, d, env, lane, there, pose);
+    if (sync_bodies == 0u || !there) return;
     wave_sync();
-    for (uint32_t b = lane; b < m.bodies_per_env; b += kWave) sync_body_pose(m, d, env, b, lds);
+    for (uint32_t b = lane; b < m.bodies_per_env; b += kLanes) sync_body_pose(m, d, env, b, pose);
 }
+
+// The instantiation for `lanes` lanes an environment and the number of its workgroups
+#define NKH_LAUNCH_LANES(lanes, kernel, envs, threads, lds_words_an_env, stream, ...)                                                          \
+    do {                                                                                                                                       \
+        const uint32_t envs_a_block = (lanes) < 64u ? 64u / (lanes) : 1u, blocks = ((envs) + envs_a_block - 1u) / envs_a_block;                                      \
+        const size_t lds_bytes = size_t{envs_a_block} * (lds_words_an_env) * sizeof(float);                                                     \
+        if ((lanes) == 8u) hipLaunchKernelGGL(kernel<8>, dim3(blocks), dim3(threads), lds_bytes, stream, __VA_ARGS__);                          \
+        else if ((lanes) == 16u) hipLaunchKernelGGL(kernel<16>, dim3(blocks), dim3(threads), lds_bytes, stream, __VA_ARGS__);                   \
+        else if ((lanes) == 32u) hipLaunchKernelGGL(kernel<32>, dim3(blocks), dim3(threads), lds_bytes, stream, __VA_ARGS__);                   \
+        else if ((lanes) == 64u) hipLaunchKernelGGL(kernel<64>, dim3(blocks), dim3(threads), lds_bytes, stream, __VA_ARGS__);                   \
+        else hipLaunchKernelGGL(kernel<128>, dim3(blocks), dim3(threads), lds_bytes, stream, __VA_ARGS__);                                       \
+    } while (false)
 
 }  // namespace
 
@@ -668,8 +719,8 @@ Status OpFkWorldPoses(const ModelView& m, const DataView& d, const void* params,
     if (p == nullptr) return Status::Failed;
     if (p->articulation_count == 0u || p->total_link_count == 0u) return Status::Ok;
     if (m.links_per_env == 0u || p->total_link_count != p->articulation_count * m.links_per_env) return Status::InvalidArgument;
-    const size_t lds = size_t{m.links_per_env} * 7u * sizeof(float);
-    hipLaunchKernelGGL(FkWorldPosesKernel, dim3(p->articulation_count), dim3(kWave), lds, stream, m, d, p->articulation_count);
+    const uint32_t lanes = LanesAnEnvironment(m.links_per_env, p->articulation_count);
+    NKH_LAUNCH_LANES(lanes, FkWorldPosesKernel, p->articulation_count, kWave, m.links_per_env * 7u, stream, m, d, p->articulation_count);
     return hipGetLastError() == hipSuccess ? Status::Ok : Status::Failed;
 }
 
@@ -684,8 +735,8 @@ Status OpStepTail(const ModelView& m, const DataView& d, const IntegratePosition
         twists->total_link_count != links) return Status::Unsupported;
     if (bodies != nullptr && (bodies->env_count != E || bodies->bodies_per_env != m.bodies_per_env || bodies->bodies_per_env == 0u ||
                               bodies->selected_env_count != 0u)) return Status::Unsupported;
-    const size_t lds = size_t{m.links_per_env} * 13u * sizeof(float);
-    hipLaunchKernelGGL(StepTailKernel, dim3(E), dim3(2 * kWave), lds, stream, m, d, *integrate, E, bodies != nullptr ? 1u : 0u);
+    const uint32_t lanes = LanesAnEnvironment(m.links_per_env, E);
+    NKH_LAUNCH_LANES(lanes, StepTailKernel, E, 2 * kWave, m.links_per_env * 13u, stream, m, d, *integrate, E, bodies != nullptr ? 1u : 0u);
     return hipGetLastError() == hipSuccess ? Status::Ok : Status::Failed;
 }
 
@@ -929,8 +980,8 @@ Status OpFkLinkVelocities(const ModelView& m, const DataView& d, const void* par
     const auto* p = static_cast<const FkLinkVelocitiesParams*>(params);
     if (p == nullptr) return Status::InvalidArgument;
     if (p->articulation_count == 0u || p->total_link_count == 0u) return Status::Ok;
-    const size_t lds = size_t{m.links_per_env} * 6u * sizeof(float);
-    hipLaunchKernelGGL(FkLinkVelocitiesKernel, dim3(p->articulation_count), dim3(kWave), lds, stream, m, d, p->articulation_count);
+    const uint32_t lanes = LanesAnEnvironment(m.links_per_env, p->articulation_count);
+    NKH_LAUNCH_LANES(lanes, FkLinkVelocitiesKernel, p->articulation_count, kWave, m.links_per_env * 6u, stream, m, d, p->articulation_count);
     return hipGetLastError() == hipSuccess ? Status::Ok : Status::Failed;
 }
 
