@@ -395,27 +395,52 @@ __device__ __forceinline__ float pivot_scale(float pivot) { return __builtin_amd
 __device__ __forceinline__ bool pivots_valid(uint32_t lane, uint32_t N, float inverse) {
     return __all(lane >= N || (inverse > 0.0f && inverse <= FLT_MAX));
 }
-template <int N>
-__device__ __forceinline__ bool factor_rows(uint32_t lane, float (&row)[N], float* inverse_out, float* root_out) {
+// From sixteen coordinates on four columns of a full block go as a panel: within it a column's update takes lane reads, and the columns
+// past it lose the panel's four on the matrix cores - v_mfma_f32_4x4x1 with the panel's words of rows 4 q .. 4 q + 3 (from
+// LDS, `panel`: 4 N words) on the one side and the lane's own on the other gives the rows' layout, an instruction a column
+// where a lane read and a multiply-add an entry went before, each the fused multiply-add it was and in the same order, bit
+// for bit.  4096 quadrupeds 538 -> 519 us a step, 1000 servo-driven ones 2228 -> 2070 us for four.  Narrower factors have too
+// few columns past a panel to pay for its way through LDS, and a reduced block, which keeps more in registers, lost by it
+// (333 humanoids 576 -> 588 us, 4096 823 -> 838 us).
+typedef float Vec4 __attribute__((ext_vector_type(4)));
+template <int N, bool kFollow>
+constexpr bool kPanels = N >= 16 && !kFollow;
+template <int N, bool kFollow>
+__device__ __forceinline__ bool factor_rows(uint32_t lane, float (&row)[N], float* panel, float* inverse_out, float* root_out) {
     lane = local_lane(lane);
     float inverse = 0.0f, root = 0.0f;
+    Vec4* words = reinterpret_cast<Vec4*>(panel);
 #pragma unroll
     for (int k = 0; k < N; ++k) {
         const float scale = pivot_scale(lane_value(row[k], k));
         const float scaled = row[k] * scale;
         if (lane >= uint32_t(k)) { inverse = scale; root = scaled; }
         row[k] = lane > uint32_t(k) ? scaled : 0.0f;
+        const int end = kPanels<N, kFollow> ? k / 4 * 4 + 4 : N;
         // lane reads in batches of eight ahead of their multiply-adds: a scalar read has to settle for two cycles
         // before an arithmetic instruction may use it, and the next reads fill that gap
 #pragma unroll
-        for (int j0 = k + 1; j0 < N; j0 += 8) {
+        for (int j0 = k + 1; j0 < end; j0 += 8) {
             float l[8];
 #pragma unroll
-            for (int t = 0; t < 8; ++t) l[t] = j0 + t < N ? lane_value(row[k], j0 + t) : 0.0f;
+            for (int t = 0; t < 8; ++t) l[t] = j0 + t < end ? lane_value(row[k], j0 + t) : 0.0f;
 #pragma unroll
             for (int t = 0; t < 8; ++t)
-                if (j0 + t < N) row[j0 + t] = fmaf(-row[k], l[t], row[j0 + t]);
+                if (j0 + t < end) row[j0 + t] = fmaf(-row[k], l[t], row[j0 + t]);
         }
+        if (!kPanels<N, kFollow> || k % 4 != 3 || k == N - 1) continue;
+        if (lane < uint32_t(N)) words[lane] = Vec4{row[k - 3], row[k - 2], row[k - 1], row[k]};
+        __syncthreads();
+#pragma unroll
+        for (int q = k / 4 + 1; q < N / 4; ++q) {
+            const Vec4 l = words[4u * uint32_t(q) + (lane & 3u)];
+            Vec4 four = {row[4 * q], row[4 * q + 1], row[4 * q + 2], row[4 * q + 3]};
+#pragma unroll
+            for (int t = 0; t < 4; ++t) four = __builtin_amdgcn_mfma_f32_4x4x1f32(l[t], -row[k - 3 + t], four, 0, 0, 0);
+#pragma unroll
+            for (int t = 0; t < 4; ++t) row[4 * q + t] = four[t];
+        }
+        __syncthreads();
     }
     *inverse_out = inverse; *root_out = root;
     return pivots_valid(lane, uint32_t(N), inverse);
@@ -440,13 +465,9 @@ __device__ __forceinline__ uint32_t factor_at(uint32_t i, uint32_t k) {   // lea
 }
 
 // FactorTileColumns on register rows: lane i holds row i of the symmetric matrix; on return its entries k > i are
-// row i of U, every other entry is zero, and `root` is the diagonal.  Four columns a panel: within it a column's update goes
-// through lane reads, and the columns left of it lose the panel's four on the matrix cores - v_mfma_f32_4x4x1 with the
-// panel's words of rows 4 q .. 4 q + 3 (from LDS, `panel`: 4 x 64 words) on the one side and the lane's own on the other
-// gives the rows' layout, an instruction a column where a lane read and a multiply-add an entry went before, each the
-// fused multiply-add it was and in the same order, bit for bit.  A step of 8192 ropes (64 coordinates):
-// 24.7 -> 21.9 ms, of 4096 servo-driven humanoids (36 coordinates) 2.30 -> 2.16 ms.
-typedef float Vec4 __attribute__((ext_vector_type(4)));
+// row i of U, every other entry is zero, and `root` is the diagonal.  Panels of four columns as above (`panel`: 4 x 64
+// words).  A step of 8192 ropes (64 coordinates, 4032 instructions of updates before): 24.7 -> 21.9 ms, of 4096 servo-driven
+// humanoids (36 coordinates) 2.30 -> 2.16 ms.
 template <int N>
 __device__ __forceinline__ bool factor_rows_up(uint32_t lane, float (&row)[N], float* panel, float* inverse_out, float* root_out) {
     lane = local_lane(lane);
@@ -571,12 +592,12 @@ __device__ __forceinline__ void load_columns(const float* a, uint32_t lane, floa
 
 // Cholesky of the Newton Hessian held in `hrow`, then d = H^-1 g.  The factor passes through LDS once, for the
 // transposed read of the backward substitution.
-template <int N>
+template <int N, bool kFollow>
 __device__ __forceinline__ bool cholesky_solve(const Tile& c, float (&hrow)[N], float g, float* d_out) {
     float inverse = 0.0f;
     if (!c.factor_current) {   // otherwise the Hessian is the one factored last: its factor is still in hfac
         PROF_BEGIN(c, 14);
-        const bool valid = kLeavesFirst<N> ? factor_rows_up<N>(c.lane, hrow, c.hfac, &inverse, &c.factor_root) : factor_rows<N>(c.lane, hrow, &inverse, &c.factor_root);
+        const bool valid = kLeavesFirst<N> ? factor_rows_up<N>(c.lane, hrow, c.hfac, &inverse, &c.factor_root) : factor_rows<N, kFollow>(c.lane, hrow, c.hfac, &inverse, &c.factor_root);
         PROF_END(c, 14);
         if (!valid) return false;
         PROF_BEGIN(c, 24);
@@ -605,13 +626,13 @@ __device__ __forceinline__ bool cholesky_solve(const Tile& c, float (&hrow)[N], 
 
 // SolveTileMass (:1898-1931).  The mass matrix does not change during a solve, so its factor (same arithmetic as the
 // reference's per-call factorisation, hence the same numbers) is built once by factor_mass and reused here.
-template <int N>
+template <int N, bool kFollow>
 __device__ __forceinline__ bool factor_mass(Tile& c, const float (&mrow)[N]) {
     float row[N];
 #pragma unroll
     for (int k = 0; k < N; ++k) row[k] = mrow[k];
     float inverse = 0.0f, root = 0.0f;
-    const bool valid = kLeavesFirst<N> ? factor_rows_up<N>(c.lane, row, c.hfac, &inverse, &root) : factor_rows<N>(c.lane, row, &inverse, &root);
+    const bool valid = kLeavesFirst<N> ? factor_rows_up<N>(c.lane, row, c.hfac, &inverse, &root) : factor_rows<N, kFollow>(c.lane, row, c.hfac, &inverse, &root);
     c.mass_inverse = inverse;
     store_rows<N>(c.mfac, c.lane, row);
     __syncthreads();
@@ -1618,7 +1639,7 @@ __device__ __forceinline__ Failure newton_direction(const Tile& c, const float (
     }
     if (*converged) return kFailNone;
     PROF_BEGIN(c, 2);
-    const bool factored = cholesky_solve<N>(c, hrow, *force, d);
+    const bool factored = cholesky_solve<N, kFollow>(c, hrow, *force, d);
     PROF_END(c, 2);
     if (!factored) return kFailFactor;
     return kFailNone;
@@ -2978,7 +2999,7 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
     PROF_END(c, 19);
     PROF_BEGIN(c, 20);
     // the one factorisation of the mass matrix
-    c.mass_valid = factor_mass<W>(c, mrow) && reduction_valid;
+    c.mass_valid = factor_mass<W, kReduced>(c, mrow) && reduction_valid;
     PROF_END(c, 20);
     PROF_BEGIN(c, 21);
     initialize_residuals<W>(c, velocity, urows, p.dt);
