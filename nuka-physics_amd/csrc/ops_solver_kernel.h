@@ -335,12 +335,12 @@ struct Tile {
     float* axes;              // 64 x 12: a coordinate's motion axis about `pivot`, then the contact stiffness it carries times that axis
     uint32_t path_low, path_high;     // lane = coordinate: the coordinates on the way from its link to the root, itself included
     uint32_t under_low, under_high;   // the coordinates whose way to the root passes through lane's
+    uint32_t over_low, over_high;     // the heads whose way to the root passes through lane's coordinate
+    float* spread;            // from_links: 8 x 68 words, what the lanes hand each other as heads and take as coordinates
+    mutable bool stiffness_current;   // no head's curvature has changed since the stiffness in `axes` was summed
     V3 pivot;                 // the point the axes and the heads' wrenches are taken about: the root link's origin
-    const float* rows;        // the environment-major row records, row points and row links of device memory
+    const float* rows;        // the environment-major row records and row points of device memory
     const float* row_point_a, *row_point_b;
-    const uint32_t* row_link_a, *row_link_b;
-    const uint64_t* link_paths;
-    uint32_t first_link;      // index of the environment's first link
 #ifdef NKH_SOLVER_PROFILE
     mutable long long prof[32];
     mutable uint32_t prof_count[4];
@@ -403,6 +403,9 @@ __device__ __forceinline__ bool pivots_valid(uint32_t lane, uint32_t N, float in
 // few columns past a panel to pay for its way through LDS, and a reduced block, which keeps more in registers, lost by it
 // (333 humanoids 576 -> 588 us, 4096 823 -> 838 us).
 typedef float Vec4 __attribute__((ext_vector_type(4)));
+// v where bit `at` of the mask is set, else zero: two instructions, no comparison
+__device__ __forceinline__ uint32_t bit_spread(uint32_t mask, uint32_t at) { return uint32_t(__builtin_amdgcn_sbfe(int(mask), at, 1u)); }
+__device__ __forceinline__ float kept_if(uint32_t mask, uint32_t at, float v) { return __uint_as_float(bit_spread(mask, at) & __float_as_uint(v)); }
 template <int N, bool kFollow>
 constexpr bool kPanels = N >= 16 && !kFollow;
 template <int N, bool kFollow>
@@ -1192,25 +1195,28 @@ __device__ __forceinline__ void add_heads_force(const Tile& c, uint64_t heads, c
 // lane = head: the motion of the head's link, sum over the coordinates j on its way of s_j x_j, for a vector x in LDS.
 template <int N>
 __device__ __forceinline__ void link_motion(const Tile& c, uint64_t way, const float* x, float (&motion)[6]) {
-    const float4* table = reinterpret_cast<const float4*>(c.axes);
+    // Every lane of the wavefront, those without a head with a way of none: v_mfma_f32_4x4x1 takes a coordinate's axis, a
+    // component a lane of four, against the lane's own weight, and register r of a lane is the sum of component r - the
+    // multiply-adds that six vector instructions and two sixteen-byte reads a coordinate made before, bit for bit.
+    const float* words = c.axes + (c.lane & 3u);
     const float4* x4 = reinterpret_cast<const float4*>(x);
-#pragma unroll
-    for (int k = 0; k < 6; ++k) motion[k] = 0.0f;
+    const uint32_t on_low = uint32_t(way), on_high = uint32_t(way >> 32u);
+    Vec4 low = {}, high = {};
     // a loop that stays a loop: unrolled, all of the table is fetched ahead of the first product, into registers the
     // block does not have
-#pragma unroll 1
+#pragma unroll 2
     for (uint32_t q = 0u; q < uint32_t(N / 4); ++q) {
         const float4 xq = x4[q];
         const float xs[4] = {xq.x, xq.y, xq.z, xq.w};
-        const uint32_t four = uint32_t(way >> (4u * q)) & 0xFu;
+        const uint32_t four = q < 8u ? on_low >> (4u * q) : on_high >> (4u * q - 32u);
 #pragma unroll
         for (uint32_t t = 0u; t < 4u; ++t) {
-            const float4 a = table[3u * (4u * q + t)], b = table[3u * (4u * q + t) + 1u];
-            const float on = ((four >> t) & 1u) != 0u ? xs[t] : 0.0f;
-            motion[0] = fmaf(a.x, on, motion[0]); motion[1] = fmaf(a.y, on, motion[1]); motion[2] = fmaf(a.z, on, motion[2]);
-            motion[3] = fmaf(a.w, on, motion[3]); motion[4] = fmaf(b.x, on, motion[4]); motion[5] = fmaf(b.y, on, motion[5]);
+            const float on = kept_if(four, t, xs[t]);
+            low = __builtin_amdgcn_mfma_f32_4x4x1f32(words[12u * (4u * q + t)], on, low, 0, 0, 0);
+            high = __builtin_amdgcn_mfma_f32_4x4x1f32(words[12u * (4u * q + t) + 4u], on, high, 0, 0, 0);   // (and two components nobody reads)
         }
     }
+    motion[0] = low[0]; motion[1] = low[1]; motion[2] = low[2]; motion[3] = low[3]; motion[4] = high[0]; motion[5] = high[1];
 }
 // lane = head: row `axis` of head h times the vector whose link motion is `motion`
 __device__ __forceinline__ float wrench_dot(const Tile& c, uint32_t h, uint32_t axis, const float (&motion)[6]) {
@@ -1221,6 +1227,41 @@ __device__ __forceinline__ uint64_t way_of(const Tile& c, uint32_t h) {
     const uint32_t* w = reinterpret_cast<const uint32_t*>(c.wrench + h * kWrenchStride + 18u);
     return (uint64_t(w[1]) << 32u) | uint64_t(w[0]);
 }
+// lane = head holds 4 kGroups values; lane = coordinate comes back with their sums over the heads of `heads` (a uniform mask of
+// the first 64) whose way holds the coordinate, added to `sum` in head order.  The values go through LDS (`words`,
+// 4 kGroups x (kHeads + 4) of them) kHeads heads at a time, and v_mfma_f32_4x4x1 multiplies a head's four words of a group, a
+// lane of four each, with the coordinates' own ones and zeros: an instruction a head and group, each the four
+// multiply-adds by one or zero it replaces with their lane reads.  The lanes of heads outside `heads` hold zeros.
+template <int kGroups, uint32_t kHeads>
+__device__ __forceinline__ void sums_over_ways(const Tile& c, uint64_t heads, const float (&v)[4 * kGroups], float* words, Vec4 (&sum)[kGroups]) {
+    constexpr uint32_t kStride = kHeads + 4u;   // sixteen-byte words, the four lanes' in different banks
+    const uint32_t end = heads == 0ull ? 0u : uint32_t(64 - __builtin_clzll(heads));
+#pragma unroll 1
+    for (uint32_t first = 0u; first < end; first += kHeads) {
+        const uint32_t at = c.lane - first;
+        if (at < kHeads) {
+#pragma unroll
+            for (uint32_t e = 0u; e < 4u * kGroups; ++e) words[e * kStride + at] = v[e];
+        }
+        __syncthreads();
+        const float* mine = words + (c.lane & 3u) * kStride;
+        const uint32_t here = min(end - first, kHeads);
+#pragma unroll 2
+        for (uint32_t h = 0u; h < here; h += 4u) {
+            const uint32_t four = first + h < 32u ? c.over_low >> (first + h) : c.over_high >> (first + h - 32u);
+            Vec4 word[kGroups];
+#pragma unroll
+            for (uint32_t g = 0u; g < uint32_t(kGroups); ++g) word[g] = *reinterpret_cast<const Vec4*>(mine + 4u * g * kStride + h);
+#pragma unroll
+            for (uint32_t t = 0u; t < 4u; ++t) {
+                const float through = kept_if(four, t, 1.0f);
+#pragma unroll
+                for (uint32_t g = 0u; g < uint32_t(kGroups); ++g) sum[g] = __builtin_amdgcn_mfma_f32_4x4x1f32(word[g][t], through, sum[g], 0, 0, 0);
+            }
+        }
+        __syncthreads();
+    }
+}
 // lane = coordinate: sum over the heads `heads` (a uniform mask of the first 64) of J^T x, x one value an axis held by
 // lane = head, in double: the heads' wrenches weighted by x summed over the heads whose way holds the coordinate, then
 // taken against the coordinate's motion axis.  With `weights` (the magnitudes that go with x) also the rounding scale
@@ -1228,8 +1269,7 @@ __device__ __forceinline__ uint64_t way_of(const Tile& c, uint32_t h) {
 template <bool kScale>
 __device__ __forceinline__ double rows_transposed_times(const Tile& c, uint64_t heads, const float (&x)[3], const float (&weights)[3], float* scale) {
     const uint32_t lane = c.lane;
-    float sum[6] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f}, bound[6] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
-    uint32_t way_low = 0u, way_high = 0u;
+    float sum[6] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f}, bound[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
     if (lane < c.heads && ((heads >> lane) & 1ull) != 0ull) {
         const float* w = c.wrench + lane * kWrenchStride;
 #pragma unroll
@@ -1237,22 +1277,21 @@ __device__ __forceinline__ double rows_transposed_times(const Tile& c, uint64_t 
             sum[k] = (w[k] * x[0] + w[6 + k] * x[1]) + w[12 + k] * x[2];
             if constexpr (kScale) bound[k] = (fabsf(w[k]) * weights[0] + fabsf(w[6 + k]) * weights[1]) + fabsf(w[12 + k]) * weights[2];
         }
-        const uint64_t way = way_of(c, lane);
-        way_low = uint32_t(way); way_high = uint32_t(way >> 32u);
     }
     double carried[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-    float carried_bound[6] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
-    for (uint64_t rest = heads; rest != 0ull; rest &= rest - 1ull) {
-        const int h = __builtin_ctzll(rest);
-        const uint64_t way = (uint64_t(uint32_t(__builtin_amdgcn_readlane(int(way_high), h))) << 32u) |
-                             uint64_t(uint32_t(__builtin_amdgcn_readlane(int(way_low), h)));
-        const float through = ((way >> lane) & 1ull) != 0ull ? 1.0f : 0.0f;
+    const auto add_from = [&](uint32_t mask, uint32_t rest, int first) {
+        for (; rest != 0u; rest &= rest - 1u) {
+            const int h = __builtin_ctz(rest);
+            // one or zero, its low word zero
+            const double through = __hiloint2double(int(bit_spread(mask, uint32_t(h)) & 0x3ff00000u), 0);
 #pragma unroll
-        for (int k = 0; k < 6; ++k) {
-            carried[k] = fma(double(through), double(uniform_lane_value(sum[k], uint32_t(h))), carried[k]);
-            if constexpr (kScale) carried_bound[k] = fmaf(through, uniform_lane_value(bound[k], uint32_t(h)), carried_bound[k]);
+            for (int k = 0; k < 6; ++k) carried[k] = fma(through, double(uniform_lane_value(sum[k], uint32_t(first + h))), carried[k]);
         }
-    }
+    };
+    add_from(c.over_low, uint32_t(heads), 0);
+    add_from(c.over_high, uint32_t(heads >> 32u), 32);
+    Vec4 carried_bound[2] = {};
+    if constexpr (kScale) sums_over_ways<2, 64u>(c, heads, bound, c.spread, carried_bound);
     const float4* table = reinterpret_cast<const float4*>(c.axes);
     const float4 a = table[3u * lane], b = table[3u * lane + 1u];
     const float s[6] = {a.x, a.y, a.z, a.w, b.x, b.y};
@@ -1262,7 +1301,7 @@ __device__ __forceinline__ double rows_transposed_times(const Tile& c, uint64_t 
     if constexpr (kScale) {
         float magnitude = 0.0f;
 #pragma unroll
-        for (int k = 0; k < 6; ++k) magnitude = fmaf(fabsf(s[k]), carried_bound[k], magnitude);
+        for (int k = 0; k < 6; ++k) magnitude = fmaf(fabsf(s[k]), carried_bound[k / 4][k % 4], magnitude);
         *scale += magnitude;
     }
     return total;
@@ -1278,73 +1317,71 @@ __device__ __forceinline__ double rows_transposed_times(const Tile& c, uint64_t 
 //     H_ij += (K_i s_i) . s_j   for j on i's way to the root,      (K_j s_j) . s_i   for i on j's,
 // which takes 21 words a head and 12 a column where the plain sum over heads takes 3 N words a head.  The two forms
 // of one entry multiply and add the same numbers in the same order: the rows stay each other's transposes to the bit.
-// lane = head on the way in (mc: its curvature, `mine`: it contributes), lane = coordinate from the sums on.
+// lane = head on the way in (mc: its curvature, `mine`: it contributes), lane = coordinate from the sums on.  Both products
+// run on the matrix cores with the multiply-adds of the vector form, bit for bit; while no curvature has changed the
+// stiffness of the last assembly, left in the table beside the axes, stands.  A
+// step of 8192 ropes: 22.1 -> 18.5 ms with the sums of rows_transposed_times and link_motion in the same form.
+// heads a pass of the stiffness sums: 24 words a head (21 and padding), within the factor's place
+template <int N>
+constexpr uint32_t kLinkPass = FactorFloats(N) >= 24u * 68u ? 64u : (FactorFloats(N) >= 24u * 36u ? 32u : 16u);
 template <int N>
 __device__ __forceinline__ void add_heads_through_links(const Tile& c, bool mine, const float (&mc)[6], float (&hrow)[N]) {
     const uint32_t lane = c.lane;
-    float k[21];
-#pragma unroll
-    for (int e = 0; e < 21; ++e) k[e] = 0.0f;
-    uint32_t way_low = 0u, way_high = 0u;
-    if (mine) {
-        const uint32_t slot = c.U(hSlot, lane), stride = c.U(hStride, lane), axes = c.U(hAxes, lane);
-        const bool second = c.U(hSourceA, lane) == kInvalid;   // the side that moves is the row's second
-        const uint64_t way = c.from_links ? way_of(c, lane) : c.link_paths[(second ? c.row_link_b : c.row_link_a)[slot] - c.first_link];
-        way_low = uint32_t(way); way_high = uint32_t(way >> 32u);
-        float w[3][6];
-#pragma unroll
-        for (uint32_t a = 0u; a < 3u; ++a) {
-            if (c.from_links) {
-#pragma unroll
-                for (int t = 0; t < 6; ++t) w[a][t] = c.wrench[lane * kWrenchStride + 6u * a + uint32_t(t)];
-                continue;
-            }
-#pragma unroll
-            for (int t = 0; t < 6; ++t) w[a][t] = 0.0f;
-            if (a != 0u && axes == 1u) continue;
-            const size_t rs = size_t{slot} + a * stride;
-            const float* row = c.rows + rs * kRowWords + 12u;          // the first side's direction; the second side's is its negative,
-            const float* at = (second ? c.row_point_b : c.row_point_a) + 3u * rs;   // and W C W^T does not see the sign
-            const V3 n{row[0], row[1], row[2]};
-            const V3 arm = sub3(V3{at[0], at[1], at[2]}, c.pivot);
-            const V3 moment = cross3(arm, n);
-            w[a][0] = moment.x; w[a][1] = moment.y; w[a][2] = moment.z; w[a][3] = n.x; w[a][4] = n.y; w[a][5] = n.z;
-        }
-        const float cxx = mc[0], cyy = mc[1], czz = mc[2], cxy = mc[3], cxz = mc[4], cyz = mc[5];
-        float u[3][6];
-#pragma unroll
-        for (int t = 0; t < 6; ++t) {
-            u[0][t] = (cxx * w[0][t] + cxy * w[1][t]) + cxz * w[2][t];
-            u[1][t] = (cxy * w[0][t] + cyy * w[1][t]) + cyz * w[2][t];
-            u[2][t] = (cxz * w[0][t] + cyz * w[1][t]) + czz * w[2][t];
-        }
-        int e = 0;
-#pragma unroll
-        for (int r = 0; r < 6; ++r) {
-#pragma unroll
-            for (int t = r; t < 6; ++t) k[e++] = (w[0][r] * u[0][t] + w[1][r] * u[1][t]) + w[2][r] * u[2][t];
-        }
-    }
-    // lane = coordinate: the stiffness of every head whose way to the root passes through it
-    float carried[21];
-#pragma unroll
-    for (int e = 0; e < 21; ++e) carried[e] = 0.0f;
-    for (uint64_t rest = __ballot(mine); rest != 0ull; rest &= rest - 1ull) {
-        const int h = __builtin_ctzll(rest);
-        const uint64_t way = (uint64_t(uint32_t(__builtin_amdgcn_readlane(int(way_high), h))) << 32u) |
-                             uint64_t(uint32_t(__builtin_amdgcn_readlane(int(way_low), h)));
-        // one multiply-add an entry with a weight of one or zero: a conditional sum compiles to an add and two copies
-        const float through = ((way >> lane) & 1ull) != 0ull ? 1.0f : 0.0f;
-#pragma unroll
-        for (int e = 0; e < 21; ++e) carried[e] = fmaf(through, uniform_lane_value(k[e], uint32_t(h)), carried[e]);
-    }
     float4* table = reinterpret_cast<float4*>(c.axes);
-    float s[6], y[6];
-    {
+    if (!c.stiffness_current) {
+        float k[24];
+#pragma unroll
+        for (int e = 0; e < 24; ++e) k[e] = 0.0f;
+        if (mine) {
+            const uint32_t slot = c.U(hSlot, lane), stride = c.U(hStride, lane), axes = c.U(hAxes, lane);
+            const bool second = c.U(hSourceA, lane) == kInvalid;   // the side that moves is the row's second
+            float w[3][6];
+#pragma unroll
+            for (uint32_t a = 0u; a < 3u; ++a) {
+                if (c.from_links) {
+#pragma unroll
+                    for (int t = 0; t < 6; ++t) w[a][t] = c.wrench[lane * kWrenchStride + 6u * a + uint32_t(t)];
+                    continue;
+                }
+#pragma unroll
+                for (int t = 0; t < 6; ++t) w[a][t] = 0.0f;
+                if (a != 0u && axes == 1u) continue;
+                const size_t rs = size_t{slot} + a * stride;
+                const float* row = c.rows + rs * kRowWords + 12u;          // the first side's direction; the second side's is its negative,
+                const float* at = (second ? c.row_point_b : c.row_point_a) + 3u * rs;   // and W C W^T does not see the sign
+                const V3 n{row[0], row[1], row[2]};
+                const V3 arm = sub3(V3{at[0], at[1], at[2]}, c.pivot);
+                const V3 moment = cross3(arm, n);
+                w[a][0] = moment.x; w[a][1] = moment.y; w[a][2] = moment.z; w[a][3] = n.x; w[a][4] = n.y; w[a][5] = n.z;
+            }
+            const float cxx = mc[0], cyy = mc[1], czz = mc[2], cxy = mc[3], cxz = mc[4], cyz = mc[5];
+            float u[3][6];
+#pragma unroll
+            for (int t = 0; t < 6; ++t) {
+                u[0][t] = (cxx * w[0][t] + cxy * w[1][t]) + cxz * w[2][t];
+                u[1][t] = (cxy * w[0][t] + cyy * w[1][t]) + cyz * w[2][t];
+                u[2][t] = (cxz * w[0][t] + cyz * w[1][t]) + czz * w[2][t];
+            }
+            int e = 0;
+#pragma unroll
+            for (int r = 0; r < 6; ++r) {
+#pragma unroll
+                for (int t = r; t < 6; ++t) k[e++] = (w[0][r] * u[0][t] + w[1][r] * u[1][t]) + w[2][r] * u[2][t];
+            }
+        }
+        // lane = coordinate: the stiffness of every head whose way to the root passes through it.  By way of the factor's
+        // place, which a changed Hessian frees; where the factor still stood it is made again.
+        c.factor_current = false;
+        Vec4 carried[6] = {};
+        sums_over_ways<6, kLinkPass<N>>(c, __ballot(mine), k, c.hfac, carried);
         const float4 a = table[3u * lane], b = table[3u * lane + 1u];
-        s[0] = a.x; s[1] = a.y; s[2] = a.z; s[3] = a.w; s[4] = b.x; s[5] = b.y;
+        const float s[6] = {a.x, a.y, a.z, a.w, b.x, b.y};
+        float y[6];
         // y = K s, K symmetric with its upper triangle in `carried`, rows first
-        auto entry = [&](int r, int t) { return r <= t ? carried[r * 6 - r * (r - 1) / 2 + (t - r)] : carried[t * 6 - t * (t - 1) / 2 + (r - t)]; };
+        const auto entry = [&](int r, int t) {
+            const int e = r <= t ? r * 6 - r * (r - 1) / 2 + (t - r) : t * 6 - t * (t - 1) / 2 + (r - t);
+            return carried[e / 4][e % 4];
+        };
 #pragma unroll
         for (int r = 0; r < 6; ++r) {
             float sum = entry(r, 0) * s[0];
@@ -1354,20 +1391,34 @@ __device__ __forceinline__ void add_heads_through_links(const Tile& c, bool mine
         }
         table[3u * lane + 1u] = float4{b.x, b.y, y[0], y[1]};
         table[3u * lane + 2u] = float4{y[2], y[3], y[4], y[5]};
+        c.stiffness_current = true;
     }
     __syncthreads();
+    const float4 la = table[3u * lane], lb = table[3u * lane + 1u], lc = table[3u * lane + 2u];
+    const float s[6] = {la.x, la.y, la.z, la.w, lb.x, lb.y}, y[6] = {lb.z, lb.w, lc.x, lc.y, lc.z, lc.w};
     // (through the barrier so that the sixty-four lane masks of each are made here, two instructions a column, instead of
     // ahead of the sweeps and kept in scalar registers the kernel does not have)
-    const uint64_t path = (uint64_t(opaque_word(c.path_high)) << 32u) | uint64_t(opaque_word(c.path_low));
-    const uint64_t under = (uint64_t(opaque_word(c.under_high)) << 32u) | uint64_t(opaque_word(c.under_low));
+    const uint32_t path[2] = {opaque_word(c.path_low), opaque_word(c.path_high)};
+    const uint32_t under[2] = {opaque_word(c.under_low) & ~path[0], opaque_word(c.under_high) & ~path[1]};
 #pragma unroll
-    for (int j = 0; j < N; ++j) {
-        const float4 a = table[3 * j], b = table[3 * j + 1], d = table[3 * j + 2];
-        // (K_i s_i) . s_j and (K_j s_j) . s_i, each the stiffness-times-axis of the coordinate further from the root first
-        const float mine_first = fmaf(y[5], b.y, fmaf(y[4], b.x, fmaf(y[3], a.w, fmaf(y[2], a.z, fmaf(y[1], a.y, y[0] * a.x)))));
-        const float other_first = fmaf(d.w, s[5], fmaf(d.z, s[4], fmaf(d.y, s[3], fmaf(d.x, s[2], fmaf(b.w, s[1], b.z * s[0])))));
-        const bool on_my_way = ((path >> j) & 1ull) != 0ull, through_me = ((under >> j) & 1ull) != 0ull;
-        hrow[j] += on_my_way ? mine_first : (through_me ? other_first : 0.0f);
+    for (int q = 0; q < N / 4; ++q) {
+        // (K_i s_i) . s_j and (K_j s_j) . s_i, each the stiffness-times-axis of the coordinate further from the root first:
+        // four columns an instruction and component, v_mfma_f32_4x4x1 with the columns' words a lane of four each
+        const float4* column = table + 3u * (4u * uint32_t(q) + (lane & 3u));
+        const float4 a = column[0], b = column[1], d = column[2];
+        const float cs[6] = {a.x, a.y, a.z, a.w, b.x, b.y}, cy[6] = {b.z, b.w, d.x, d.y, d.z, d.w};
+        Vec4 mine_first = {}, other_first = {};
+#pragma unroll
+        for (int t = 0; t < 6; ++t) {
+            mine_first = __builtin_amdgcn_mfma_f32_4x4x1f32(cs[t], y[t], mine_first, 0, 0, 0);
+            other_first = __builtin_amdgcn_mfma_f32_4x4x1f32(cy[t], s[t], other_first, 0, 0, 0);
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const uint32_t at = uint32_t(4 * q + r) & 31u;
+            const uint32_t bits = (bit_spread(path[q / 8], at) & __float_as_uint(mine_first[r])) | (bit_spread(under[q / 8], at) & __float_as_uint(other_first[r]));
+            hrow[4 * q + r] += __uint_as_float(bits);
+        }
     }
     __syncthreads();
 }
@@ -1419,7 +1470,7 @@ __device__ __forceinline__ bool assemble_block(const Tile& c, const float (&mrow
     }
 #pragma unroll
     for (int k = 0; k < 6; ++k) { differs |= bits(c.curvature[k]) ^ bits(mc[k]); c.curvature[k] = mc[k]; }
-    if (__any(lane < c.heads && differs != 0u)) { c.factor_current = false; c.rows_current = false; }
+    if (__any(lane < c.heads && differs != 0u)) { c.factor_current = false; c.rows_current = false; c.stiffness_current = false; }
     const bool rows_kept = N <= 32 && c.rows_current && c.heads <= uint32_t(kWave);   // only the force is to be summed
     if (c.units && lane < c.heads && c.U(hUnit, lane) != kInvalid) {   // a coordinate reads its unit heads' responses from the fields
         c.F(hF, lane) = mf[0]; c.F(hNoise, lane) = mn[0]; c.F(hC, lane) = mc[0];
@@ -1673,6 +1724,21 @@ __device__ __forceinline__ void row_steps(const Tile& c, float d) {
         __syncthreads();
         return;
     }
+    if constexpr (N > kTwoWaveWidth) {
+        if (c.from_links) {   // contact heads, one a lane at most, none of them a unit head
+            const bool owned = c.lane < c.heads && c.U(hOwned, c.lane < c.heads ? c.lane : 0u) != 0u;
+            const uint32_t h = owned ? c.lane : 0u, axes = c.U(hAxes, h);
+            float motion[6];
+            link_motion<N>(c, owned ? way_of(c, h) : 0ull, dvec, motion);
+            if (owned) {
+                c.F(hStep, h) = wrench_dot(c, h, 0u, motion);
+                c.F(hStep + 1, h) = axes > 1u ? wrench_dot(c, h, 1u, motion) : 0.0f;
+                c.F(hStep + 2, h) = axes > 2u ? wrench_dot(c, h, 2u, motion) : 0.0f;
+            }
+            __syncthreads();
+            return;
+        }
+    }
     for (uint32_t h = c.lane; h < c.heads; h += kWave) {
         if (c.U(hOwned, h) == 0u) continue;
         const uint32_t unit = c.U(hUnit, h);
@@ -1681,16 +1747,6 @@ __device__ __forceinline__ void row_steps(const Tile& c, float d) {
             continue;
         }
         const uint32_t axes = c.U(hAxes, h);
-        if constexpr (N > kTwoWaveWidth) {
-            if (c.from_links) {
-                float motion[6];
-                link_motion<N>(c, way_of(c, h), dvec, motion);
-                c.F(hStep, h) = wrench_dot(c, h, 0u, motion);
-                c.F(hStep + 1, h) = axes > 1u ? wrench_dot(c, h, 1u, motion) : 0.0f;
-                c.F(hStep + 2, h) = axes > 2u ? wrench_dot(c, h, 2u, motion) : 0.0f;
-                continue;
-            }
-        }
         const float* j = c.jac + c.U(hRow, h) * uint32_t(N);
         c.F(hStep, h) = row_dot_fma<N>(j, dvec);
         c.F(hStep + 1, h) = axes > 1u ? row_dot_fma<N>(j + N, dvec) : 0.0f;
@@ -2063,6 +2119,10 @@ __device__ __forceinline__ void initialize_residuals(const Tile& c, float veloci
     dvec[c.lane] = c.lane < c.n ? velocity : 0.0f;
     __syncthreads();
     const float4* d4 = reinterpret_cast<const float4*>(dvec);
+    float motion[6] = {};   // of the link of lane's head, where the rows follow from the links
+    if constexpr (N > kTwoWaveWidth) {
+        if (c.from_links) link_motion<N>(c, c.lane < c.heads ? way_of(c, c.lane) : 0ull, dvec, motion);
+    }
     for (uint32_t h = c.lane; h < c.heads; h += kWave) {
         const uint32_t slot = c.U(hSlot, h), stride = c.U(hStride, h), axes = c.U(hAxes, h);
         const uint32_t unit = c.U(hUnit, h), first = c.U(hRow, h);
@@ -2074,8 +2134,6 @@ __device__ __forceinline__ void initialize_residuals(const Tile& c, float veloci
         }
         if constexpr (N > kTwoWaveWidth) {
             if (c.from_links) {
-                float motion[6];
-                link_motion<N>(c, way_of(c, h), dvec, motion);
                 for (uint32_t axis = 0u; axis < 3u; ++axis)
                     c.F(hRes + axis, h) = axis < axes ? urows[size_t{slot + axis * stride} * kRowWords + 4u] * dt - wrench_dot(c, h, axis, motion) : 0.0f;
                 continue;
@@ -2281,12 +2339,14 @@ __host__ __device__ inline bool RowsFromLinks(uint32_t n, bool contacts_only, ui
 __host__ __device__ inline uint32_t RowFloats(uint32_t N, uint32_t staged, bool from_links) {
     return from_links ? (kWrenchStride * staged + 3u) & ~3u : 3u * staged * N;
 }
+// what a block that keeps no contact rows sums over its heads' ways through LDS (Tile::spread)
+__host__ __device__ inline uint32_t SpreadFloats(bool from_links) { return from_links ? 8u * 68u : 0u; }
 __host__ __device__ inline uint32_t SolverLdsFloats(uint32_t n, uint32_t cap, uint32_t staged, bool from_links = false, bool reduced = false) {
     const uint32_t N = PaddedWidth(n);
     // the per-coordinate unit lists exist only when some head beyond the staged ones can be listed; without joint rows
     // the block keeps the footprint that lets eight of them share a compute unit's LDS
     return FactorRegionFloats(n) + RowFloats(N, staged, from_links) + HeadFieldFloats(cap, staged) + 256u +
-           (cap > staged ? kUnitSlots * uint32_t(kWave) : 0u) + LinkAxisFloats(n) + KeptRowFloats(n, reduced);
+           (cap > staged ? kUnitSlots * uint32_t(kWave) : 0u) + LinkAxisFloats(n) + SpreadFloats(from_links) + KeptRowFloats(n, reduced);
 }
 __host__ __device__ inline uint32_t ReducedSolverLdsFloats(uint32_t full, uint32_t reduced, uint32_t cap, uint32_t staged, bool from_links = false) {
     const uint32_t solve = SolverLdsFloats(reduced, cap, staged, from_links, reduced < full), scratch = ReductionScratchFloats(full, reduced);
@@ -2461,9 +2521,10 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
     c.unit_lists = true; c.unit_count = 0u; c.staged_end = 0u; c.individual_end = 0u;
     c.through_links = false;
     c.axes = c.vec + 256 + (cap > staged_cap ? kUnitSlots * uint32_t(kWave) : 0u);   // a wide block's; a narrow one keeps rows here
-    c.path_low = c.path_high = c.under_low = c.under_high = 0u;
-    c.rows = d.urows; c.row_point_a = d.row_cj_point; c.row_point_b = d.row_cj_point_b; c.row_link_a = d.row_cj_link; c.row_link_b = d.row_cj_link_b;
-    c.link_paths = m.link_dof_mask; c.first_link = env * nl;
+    c.spread = c.axes + 12u * uint32_t(kWave);   // a block without contact rows has it
+    c.path_low = c.path_high = c.under_low = c.under_high = c.over_low = c.over_high = 0u;
+    c.stiffness_current = false;
+    c.rows = d.urows; c.row_point_a = d.row_cj_point; c.row_point_b = d.row_cj_point_b;
     c.pivot = V3{0.0f, 0.0f, 0.0f};
     const bool coordinate = lane < n;
     const float* urows = d.urows;
@@ -2633,12 +2694,18 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
         table[3u * lane + 1u] = float4{axis[4], axis[5], 0.0f, 0.0f};
         table[3u * lane + 2u] = float4{0.0f, 0.0f, 0.0f, 0.0f};
         c.path_low = uint32_t(path); c.path_high = uint32_t(path >> 32u);
-        uint64_t under = 0ull;
-        for (uint32_t i = 0u; i < n; ++i) {
-            const uint64_t holders = __ballot(((path >> i) & 1ull) != 0ull);   // the coordinates whose way to the root holds i
-            if (lane == i) under = holders;
+        uint64_t head_way = 0ull;   // lane = head: the way to the root of the one side that moves
+        if (lane < heads) {
+            const bool side_a = c.U(hSourceA, lane) != kInvalid, side_b = c.U(hSourceB, lane) != kInvalid;
+            if (side_a != side_b) head_way = m.link_dof_mask[(side_a ? d.row_cj_link : d.row_cj_link_b)[c.U(hSlot, lane)] - env * nl];
+        }
+        uint64_t under = 0ull, over = 0ull;
+        for (uint32_t i = 0u; i < n; ++i) {   // the coordinates, and the heads, whose way to the root holds i
+            const uint64_t holders = __ballot(((path >> i) & 1ull) != 0ull), met = __ballot(((head_way >> i) & 1ull) != 0ull);
+            if (lane == i) { under = holders; over = met; }
         }
         c.under_low = uint32_t(under); c.under_high = uint32_t(under >> 32u);
+        c.over_low = uint32_t(over); c.over_high = uint32_t(over >> 32u);
         // every staged head with exactly one side that moves
         bool one_link = true;
         if (lane < heads) {
@@ -2660,8 +2727,6 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
                 const uint32_t axes = (__float_as_uint(row[0]) & kRowBlockNormal) != 0u ? 3u : 1u;
                 const bool side_a = c.U(hSourceA, lane) != kInvalid, side_b = c.U(hSourceB, lane) != kInvalid;
                 const bool second = !side_a;
-                uint64_t way = 0ull;
-                if (side_a != side_b) way = m.link_dof_mask[(second ? d.row_cj_link_b : d.row_cj_link)[slot] - env * nl];
                 for (uint32_t a = 0u; a < 3u; ++a) {
                     float w[6] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
                     if (a < axes && side_a != side_b) {
@@ -2675,9 +2740,9 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
 #pragma unroll
                     for (int t = 0; t < 6; ++t) record[6u * a + uint32_t(t)] = w[t];
                 }
-                reinterpret_cast<uint32_t*>(record)[18] = uint32_t(way);
-                reinterpret_cast<uint32_t*>(record)[19] = uint32_t(way >> 32u);
-                c.U(hColumnsLow, lane) = uint32_t(way); c.U(hColumnsHigh, lane) = uint32_t(way >> 32u);
+                reinterpret_cast<uint32_t*>(record)[18] = uint32_t(head_way);
+                reinterpret_cast<uint32_t*>(record)[19] = uint32_t(head_way >> 32u);
+                c.U(hColumnsLow, lane) = uint32_t(head_way); c.U(hColumnsHigh, lane) = uint32_t(head_way >> 32u);
             }
         }
         __syncthreads();
