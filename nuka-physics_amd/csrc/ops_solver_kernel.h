@@ -72,6 +72,8 @@ constexpr uint32_t kUnitSlots = 6u;
 constexpr uint32_t kLinkHeads = 4u;
 // words a head of Tile::wrench: 3 x 6 wrench components, the two words of its way to the root, one more for an odd stride
 constexpr uint32_t kWrenchStride = 21u;
+// words a component of Tile::motions: sixteen-byte words, the components of four lanes in different banks
+constexpr uint32_t kMotionStride = 68u;
 
 // Phase timers for development builds (-DNKH_SOLVER_PROFILE): cycles per phase and event counts per environment,
 // written over the environment's solver_penalty words at the end of the solve.
@@ -337,6 +339,7 @@ struct Tile {
     uint32_t under_low, under_high;   // the coordinates whose way to the root passes through lane's
     uint32_t over_low, over_high;     // the heads whose way to the root passes through lane's coordinate
     float* spread;            // from_links: 8 x 68 words, what the lanes hand each other as heads and take as coordinates
+    float* motions;           // from_links: 8 x 68 words, the coordinates' motion axes once more, component by component (two of them idle)
     mutable bool stiffness_current;   // no head's curvature has changed since the stiffness in `axes` was summed
     V3 pivot;                 // the point the axes and the heads' wrenches are taken about: the root link's origin
     const float* rows;        // the environment-major row records and row points of device memory
@@ -406,6 +409,12 @@ typedef float Vec4 __attribute__((ext_vector_type(4)));
 // v where bit `at` of the mask is set, else zero: two instructions, no comparison
 __device__ __forceinline__ uint32_t bit_spread(uint32_t mask, uint32_t at) { return uint32_t(__builtin_amdgcn_sbfe(int(mask), at, 1u)); }
 __device__ __forceinline__ float kept_if(uint32_t mask, uint32_t at, float v) { return __uint_as_float(bit_spread(mask, at) & __float_as_uint(v)); }
+template <int N>
+__device__ __forceinline__ void subtract_product(int q, float other, float own, float (&row)[N]) {   // columns 4 q .. 4 q + 3 lose own x other
+    const Vec4 four = __builtin_amdgcn_mfma_f32_4x4x1f32(other, -own, Vec4{row[4 * q], row[4 * q + 1], row[4 * q + 2], row[4 * q + 3]}, 0, 0, 0);
+#pragma unroll
+    for (int t = 0; t < 4; ++t) row[4 * q + t] = four[t];
+}
 template <int N, bool kFollow>
 constexpr bool kPanels = N >= 16 && !kFollow;
 template <int N, bool kFollow>
@@ -413,6 +422,7 @@ __device__ __forceinline__ bool factor_rows(uint32_t lane, float (&row)[N], floa
     lane = local_lane(lane);
     float inverse = 0.0f, root = 0.0f;
     Vec4* words = reinterpret_cast<Vec4*>(panel);
+    Vec4 others[N / 4];   // the last panel's words of the rows past it
 #pragma unroll
     for (int k = 0; k < N; ++k) {
         const float scale = pivot_scale(lane_value(row[k], k));
@@ -431,18 +441,18 @@ __device__ __forceinline__ bool factor_rows(uint32_t lane, float (&row)[N], floa
             for (int t = 0; t < 8; ++t)
                 if (j0 + t < end) row[j0 + t] = fmaf(-row[k], l[t], row[j0 + t]);
         }
-        if (!kPanels<N, kFollow> || k % 4 != 3 || k == N - 1) continue;
+        if (!kPanels<N, kFollow>) continue;
+        if (k >= 4) {   // under this pivot's chain: what the columns past this panel still lose to the last one
+#pragma unroll
+            for (int q = k / 4 + 1; q < N / 4; ++q) subtract_product<N>(q, others[q][k % 4], row[k / 4 * 4 - 4 + k % 4], row);
+        }
+        if (k % 4 != 3 || k == N - 1) continue;
         if (lane < uint32_t(N)) words[lane] = Vec4{row[k - 3], row[k - 2], row[k - 1], row[k]};
         __syncthreads();
 #pragma unroll
-        for (int q = k / 4 + 1; q < N / 4; ++q) {
-            const Vec4 l = words[4u * uint32_t(q) + (lane & 3u)];
-            Vec4 four = {row[4 * q], row[4 * q + 1], row[4 * q + 2], row[4 * q + 3]};
+        for (int q = k / 4 + 1; q < N / 4; ++q) others[q] = words[4u * uint32_t(q) + (lane & 3u)];
 #pragma unroll
-            for (int t = 0; t < 4; ++t) four = __builtin_amdgcn_mfma_f32_4x4x1f32(l[t], -row[k - 3 + t], four, 0, 0, 0);
-#pragma unroll
-            for (int t = 0; t < 4; ++t) row[4 * q + t] = four[t];
-        }
+        for (int t = 0; t < 4; ++t) subtract_product<N>(k / 4 + 1, others[k / 4 + 1][t], row[k - 3 + t], row);   // the next panel's own
         __syncthreads();
     }
     *inverse_out = inverse; *root_out = root;
@@ -476,29 +486,30 @@ __device__ __forceinline__ bool factor_rows_up(uint32_t lane, float (&row)[N], f
     lane = local_lane(lane);
     float inverse = 0.0f, root = 0.0f;
     Vec4* words = reinterpret_cast<Vec4*>(panel);
+    Vec4 others[N / 4];   // the last panel's words of the rows left of it
 #pragma unroll
     for (int p = N / 4 - 1; p >= 0; --p) {
 #pragma unroll
-        for (int k = 4 * p + 3; k >= 4 * p; --k) {
+        for (int t = 3; t >= 0; --t) {
+            const int k = 4 * p + t;
             const float scale = pivot_scale(lane_value(row[k], k));
             const float scaled = row[k] * scale;
             if (lane <= uint32_t(k)) { inverse = scale; root = scaled; }
             row[k] = lane < uint32_t(k) ? scaled : 0.0f;
 #pragma unroll
             for (int j = k - 1; j >= 4 * p; --j) row[j] = fmaf(-row[k], lane_value(row[k], j), row[j]);
+            if (p < N / 4 - 1) {   // under this pivot's chain: what the columns left of this panel still lose to the last one
+#pragma unroll
+                for (int q = p - 1; q >= 0; --q) subtract_product<N>(q, others[q][t], row[4 * p + 4 + t], row);
+            }
         }
         if (p == 0) break;
         words[lane] = Vec4{row[4 * p], row[4 * p + 1], row[4 * p + 2], row[4 * p + 3]};
         __syncthreads();
 #pragma unroll
-        for (int q = p - 1; q >= 0; --q) {
-            const Vec4 u = words[4u * uint32_t(q) + (lane & 3u)];
-            Vec4 four = {row[4 * q], row[4 * q + 1], row[4 * q + 2], row[4 * q + 3]};
+        for (int q = p - 1; q >= 0; --q) others[q] = words[4u * uint32_t(q) + (lane & 3u)];
 #pragma unroll
-            for (int t = 3; t >= 0; --t) four = __builtin_amdgcn_mfma_f32_4x4x1f32(u[t], -row[4 * p + t], four, 0, 0, 0);
-#pragma unroll
-            for (int t = 0; t < 4; ++t) row[4 * q + t] = four[t];
-        }
+        for (int t = 3; t >= 0; --t) subtract_product<N>(p - 1, others[p - 1][t], row[4 * p + t], row);   // the next panel's own
         __syncthreads();
     }
     *inverse_out = inverse; *root_out = root;
@@ -506,7 +517,7 @@ __device__ __forceinline__ bool factor_rows_up(uint32_t lane, float (&row)[N], f
 }
 
 // SolveWideTileBlock: U w = g with lane's own row (entries right of the diagonal), then U^T d = w with the columns,
-// read from the factor in LDS eight at a time.  The rows hold zeros from the diagonal on, so no step asks which lanes it
+// read from the factor several at a time.  The rows hold zeros from the diagonal on, so no step asks which lanes it
 // is for: a lane whose entry is final loses an exact zero.
 template <int N>
 __device__ __forceinline__ float substitute_up(uint32_t lane, const float (&row)[N], const float* factor, float inverse, float g) {
@@ -516,14 +527,15 @@ __device__ __forceinline__ float substitute_up(uint32_t lane, const float (&row)
     for (int j = N - 1; j >= 0; --j) r = fmaf(row[j], -lane_value(r * inverse, j), r);
     r *= inverse;
     const uint32_t mine = lane < uint32_t(N) ? lane : 0u;
+    constexpr int kAhead = N > kTwoWaveWidth ? 16 : 8;   // a wide block has the registers for twice the reads in flight
 #pragma unroll
-    for (int j0 = 0; j0 < N; j0 += 8) {
-        float u[8];
+    for (int j0 = 0; j0 < N; j0 += kAhead) {
+        float u[kAhead];
 #pragma unroll
-        for (int t = 0; t < 8; ++t)   // U[j][lane] for the lanes past j; the others read the first diagonal's word, a zero
+        for (int t = 0; t < kAhead; ++t)   // U[j][lane] for the lanes past j; the others read the first diagonal's word, a zero
             u[t] = j0 + t < N ? factor[mine >= uint32_t(j0 + t) ? factor_at<N>(uint32_t(j0 + t), mine) : 0u] : 0.0f;
 #pragma unroll
-        for (int t = 0; t < 8; ++t)
+        for (int t = 0; t < kAhead; ++t)
             if (j0 + t < N) r = fmaf(u[t], -lane_value(r * inverse, j0 + t), r);
     }
     return r * inverse;
@@ -549,18 +561,18 @@ __device__ __forceinline__ void store_rows(float* a, uint32_t lane, const float 
     lane = local_lane(lane);
     if (lane >= uint32_t(N)) return;
     if constexpr (kLeavesFirst<N>) {
+        // the entries left of the diagonal are zeros and go to the diagonal's place, a zero too: no condition a word
+        float* diagonal = a + factor_at<N>(lane, lane);
 #pragma unroll
-        for (int k = 0; k < N; ++k)
-            if (uint32_t(k) >= lane) a[factor_at<N>(lane, uint32_t(k))] = row[k];
+        for (int k = 0; k < N; ++k) diagonal[max(k - int(lane), 0)] = row[k];
     } else {
         float4* words = reinterpret_cast<float4*>(a + lane * uint32_t(N));
 #pragma unroll
         for (int q = 0; q < N / 4; ++q) words[q] = float4{row[4 * q], row[4 * q + 1], row[4 * q + 2], row[4 * q + 3]};
     }
 }
-// (A packed row's words are read whether or not the lane keeps them - a read under a condition compiles to a branch a
-// word - from a place inside the factor: a lane past the rows reads the last row's, and a packed row's words left of its
-// diagonal fall in the rows before it.)
+// (A packed row's words are read without a condition, which compiles to a branch a word: left of the diagonal the
+// diagonal's place answers, a zero; a lane past the rows reads the last row's.)
 template <int N>
 __device__ __forceinline__ void load_rows(const float* a, uint32_t lane, float (&row)[N]) {
     lane = local_lane(lane);
@@ -574,16 +586,9 @@ __device__ __forceinline__ void load_rows(const float* a, uint32_t lane, float (
         }
         return;
     }
+    const float* diagonal = a + factor_at<N>(from, from);
 #pragma unroll
-    for (int k = 0; k < N; ++k) {
-        const bool kept = lane < uint32_t(N) && uint32_t(k) >= lane;
-        if constexpr (N > kTwoWaveWidth) {   // such a block's mass factor is in device memory: only the words that are kept
-            row[k] = kept ? a[factor_at<N>(lane, uint32_t(k))] : 0.0f;
-        } else {
-            const float word = a[factor_at<N>(from, uint32_t(k))];
-            row[k] = kept ? word : 0.0f;
-        }
-    }
+    for (int k = 0; k < N; ++k) row[k] = diagonal[max(k - int(from), 0)];
 }
 template <int N>
 __device__ __forceinline__ void load_columns(const float* a, uint32_t lane, float (&col)[N]) {
@@ -1198,22 +1203,21 @@ __device__ __forceinline__ void link_motion(const Tile& c, uint64_t way, const f
     // Every lane of the wavefront, those without a head with a way of none: v_mfma_f32_4x4x1 takes a coordinate's axis, a
     // component a lane of four, against the lane's own weight, and register r of a lane is the sum of component r - the
     // multiply-adds that six vector instructions and two sixteen-byte reads a coordinate made before, bit for bit.
-    const float* words = c.axes + (c.lane & 3u);
-    const float4* x4 = reinterpret_cast<const float4*>(x);
+    const Vec4* words = reinterpret_cast<const Vec4*>(c.motions + (c.lane & 3u) * kMotionStride);
+    const Vec4* x4 = reinterpret_cast<const Vec4*>(x);
     const uint32_t on_low = uint32_t(way), on_high = uint32_t(way >> 32u);
     Vec4 low = {}, high = {};
     // a loop that stays a loop: unrolled, all of the table is fetched ahead of the first product, into registers the
     // block does not have
 #pragma unroll 2
     for (uint32_t q = 0u; q < uint32_t(N / 4); ++q) {
-        const float4 xq = x4[q];
-        const float xs[4] = {xq.x, xq.y, xq.z, xq.w};
+        const Vec4 xs = x4[q], first = words[q], last = words[kMotionStride + q];
         const uint32_t four = q < 8u ? on_low >> (4u * q) : on_high >> (4u * q - 32u);
 #pragma unroll
         for (uint32_t t = 0u; t < 4u; ++t) {
             const float on = kept_if(four, t, xs[t]);
-            low = __builtin_amdgcn_mfma_f32_4x4x1f32(words[12u * (4u * q + t)], on, low, 0, 0, 0);
-            high = __builtin_amdgcn_mfma_f32_4x4x1f32(words[12u * (4u * q + t) + 4u], on, high, 0, 0, 0);   // (and two components nobody reads)
+            low = __builtin_amdgcn_mfma_f32_4x4x1f32(first[t], on, low, 0, 0, 0);
+            high = __builtin_amdgcn_mfma_f32_4x4x1f32(last[t], on, high, 0, 0, 0);   // (and two components nobody reads)
         }
     }
     motion[0] = low[0]; motion[1] = low[1]; motion[2] = low[2]; motion[3] = low[3]; motion[4] = high[0]; motion[5] = high[1];
@@ -1279,17 +1283,22 @@ __device__ __forceinline__ double rows_transposed_times(const Tile& c, uint64_t 
         }
     }
     double carried[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-    const auto add_from = [&](uint32_t mask, uint32_t rest, int first) {
-        for (; rest != 0u; rest &= rest - 1u) {
-            const int h = __builtin_ctz(rest);
-            // one or zero, its low word zero
-            const double through = __hiloint2double(int(bit_spread(mask, uint32_t(h)) & 0x3ff00000u), 0);
+    // (in double from here: two lane reads a component and head, where one and its widening took a quarter-rate conversion;
+    // eight heads a turn at constant lanes, those outside `heads` holding zeros)
+    double wide[6];
 #pragma unroll
-            for (int k = 0; k < 6; ++k) carried[k] = fma(through, double(uniform_lane_value(sum[k], uint32_t(first + h))), carried[k]);
+    for (int k = 0; k < 6; ++k) wide[k] = double(sum[k]);
+#pragma unroll
+    for (int first = 0; first < int(kWave); first += 8) {
+        if (((heads >> first) & 0xFFull) == 0ull) continue;
+        const uint32_t eight = (first < 32 ? c.over_low : c.over_high) >> (first & 31);
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+            const double through = __hiloint2double(int(bit_spread(eight, uint32_t(t)) & 0x3ff00000u), 0);   // one or zero
+#pragma unroll
+            for (int k = 0; k < 6; ++k) carried[k] = fma(through, lane_value_d(wide[k], first + t), carried[k]);
         }
-    };
-    add_from(c.over_low, uint32_t(heads), 0);
-    add_from(c.over_high, uint32_t(heads >> 32u), 32);
+    }
     Vec4 carried_bound[2] = {};
     if constexpr (kScale) sums_over_ways<2, 64u>(c, heads, bound, c.spread, carried_bound);
     const float4* table = reinterpret_cast<const float4*>(c.axes);
@@ -2339,8 +2348,8 @@ __host__ __device__ inline bool RowsFromLinks(uint32_t n, bool contacts_only, ui
 __host__ __device__ inline uint32_t RowFloats(uint32_t N, uint32_t staged, bool from_links) {
     return from_links ? (kWrenchStride * staged + 3u) & ~3u : 3u * staged * N;
 }
-// what a block that keeps no contact rows sums over its heads' ways through LDS (Tile::spread)
-__host__ __device__ inline uint32_t SpreadFloats(bool from_links) { return from_links ? 8u * 68u : 0u; }
+// what a block that keeps no contact rows sums over its heads' ways through LDS (Tile::spread), and Tile::motions
+__host__ __device__ inline uint32_t SpreadFloats(bool from_links) { return from_links ? 16u * kMotionStride : 0u; }
 __host__ __device__ inline uint32_t SolverLdsFloats(uint32_t n, uint32_t cap, uint32_t staged, bool from_links = false, bool reduced = false) {
     const uint32_t N = PaddedWidth(n);
     // the per-coordinate unit lists exist only when some head beyond the staged ones can be listed; without joint rows
@@ -2521,7 +2530,8 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
     c.unit_lists = true; c.unit_count = 0u; c.staged_end = 0u; c.individual_end = 0u;
     c.through_links = false;
     c.axes = c.vec + 256 + (cap > staged_cap ? kUnitSlots * uint32_t(kWave) : 0u);   // a wide block's; a narrow one keeps rows here
-    c.spread = c.axes + 12u * uint32_t(kWave);   // a block without contact rows has it
+    c.spread = c.axes + 12u * uint32_t(kWave);   // a block without contact rows has it, and the next
+    c.motions = c.spread + 8u * kMotionStride;
     c.path_low = c.path_high = c.under_low = c.under_high = c.over_low = c.over_high = 0u;
     c.stiffness_current = false;
     c.rows = d.urows; c.row_point_a = d.row_cj_point; c.row_point_b = d.row_cj_point_b;
@@ -2693,6 +2703,10 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
         table[3u * lane] = float4{axis[0], axis[1], axis[2], axis[3]};
         table[3u * lane + 1u] = float4{axis[4], axis[5], 0.0f, 0.0f};
         table[3u * lane + 2u] = float4{0.0f, 0.0f, 0.0f, 0.0f};
+        if (c.from_links) {
+#pragma unroll
+            for (uint32_t k = 0u; k < 6u; ++k) c.motions[k * kMotionStride + lane] = axis[k];
+        }
         c.path_low = uint32_t(path); c.path_high = uint32_t(path >> 32u);
         uint64_t head_way = 0ull;   // lane = head: the way to the root of the one side that moves
         if (lane < heads) {
