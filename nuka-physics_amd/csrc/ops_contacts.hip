@@ -986,7 +986,9 @@ __global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(4, 4
     // zeroes since it brings impulses back, the rest by what this world's own steps have left in memory, which a restore
     // does not touch: 192 flags cleared, a line of memory each, were 197 us of the 641 us this kernel took at 65536 humanoids
     // stepped from a checkpoint.
-    const uint32_t impulse_bound = contact_row_bound(previous_extent, 1u, CR), clear_bound = contact_row_bound(d.row_clear_extent[env], 1u, CR);
+    // (a caller that binds its own buffers may leave the field out: the previous extent then bounds both)
+    const uint32_t left = d.row_clear_extent != nullptr ? d.row_clear_extent[env] : previous_extent;
+    const uint32_t impulse_bound = contact_row_bound(previous_extent, 1u, CR), clear_bound = contact_row_bound(left, 1u, CR);
     for (uint32_t local = lane; local < impulse_bound; local += kWave) lambda[local] = 0.0f;
     for (uint32_t local = lane; local < clear_bound; local += kWave) {
         pen[local] = 0.0f; cj_link[local] = kInvalid; cj_link_b[local] = kInvalid;
@@ -996,7 +998,7 @@ __global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(4, 4
     if (lane == 0u) {
         d.contact_row_extent[2u * env] = previous_extent;
         d.contact_row_extent[2u * env + 1u] = extent;
-        d.row_clear_extent[env] = extent;
+        if (d.row_clear_extent != nullptr) d.row_clear_extent[env] = extent;
     }
     // padded generalized velocity tile (:200-214)
     if (lane < md) {

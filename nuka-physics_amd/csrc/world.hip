@@ -1354,7 +1354,7 @@ const char* ReferenceName(const char* name) {
     static const char* const own[] = {"joint_law", "link_push_order", "sweep_links", "link_dof", "link_dof_mask", "pairable_rows", "profile_mu",
                                       "profile_law", "profile_solref", "profile_solimp", "profile_margin", "profile_mix", "articulation_qdd",
                                       "solver_penalty", "solver_velocity", "solver_free", "solver_cost", "tile_order", "row_unit",
-                                      "row_unit_value", "solver_mass_factor", "contact_cache_match"};
+                                      "row_unit_value", "solver_mass_factor", "contact_cache_match", "row_clear_extent"};
     for (const auto& pair : renamed) if (std::strcmp(name, pair[0]) == 0) return pair[1];
     for (const char* mine : own) if (std::strcmp(name, mine) == 0) return nullptr;
     return name;
