@@ -402,7 +402,8 @@ __device__ __forceinline__ bool pivots_valid(uint32_t lane, uint32_t N, float in
 // past it lose the panel's four on the matrix cores - v_mfma_f32_4x4x1 with the panel's words of rows 4 q .. 4 q + 3 (from
 // LDS, `panel`: 4 N words) on the one side and the lane's own on the other gives the rows' layout, an instruction a column
 // where a lane read and a multiply-add an entry went before, each the fused multiply-add it was and in the same order, bit
-// for bit.  4096 quadrupeds 538 -> 519 us a step, 1000 servo-driven ones 2228 -> 2070 us for four.  Narrower factors have too
+// for bit.  4096 quadrupeds 538 -> 519 us a step (514 with the products under the next pivots), 1000 servo-driven ones
+// 2228 -> 2070 us for four.  Narrower factors have too
 // few columns past a panel to pay for its way through LDS, and a reduced block, which keeps more in registers, lost by it
 // (333 humanoids 576 -> 588 us, 4096 823 -> 838 us).
 typedef float Vec4 __attribute__((ext_vector_type(4)));
@@ -480,7 +481,8 @@ __device__ __forceinline__ uint32_t factor_at(uint32_t i, uint32_t k) {   // lea
 // FactorTileColumns on register rows: lane i holds row i of the symmetric matrix; on return its entries k > i are
 // row i of U, every other entry is zero, and `root` is the diagonal.  Panels of four columns as above (`panel`: 4 x 64
 // words).  A step of 8192 ropes (64 coordinates, 4032 instructions of updates before): 24.7 -> 21.9 ms, of 4096 servo-driven
-// humanoids (36 coordinates) 2.30 -> 2.16 ms.
+// humanoids (36 coordinates) 2.30 -> 2.16 ms; with the products that the next panel does not wait for under its pivots, in
+// either direction, and the packed rows stored without conditions 2.10 ms.
 template <int N>
 __device__ __forceinline__ bool factor_rows_up(uint32_t lane, float (&row)[N], float* panel, float* inverse_out, float* root_out) {
     lane = local_lane(lane);
