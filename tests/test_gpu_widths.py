@@ -212,3 +212,23 @@ def test_large_batches_take_the_dense_kernels_and_give_the_same_bits(oracle_py, 
     small.close()
     big.close()
     oracle.close()
+
+
+@pytest.mark.parametrize("dof,limb_joints,heads", [(40, 2, 34), (44, 2, 38), (48, 2, 42), (60, 2, 54)])
+def test_more_heads_than_a_pass_of_the_link_sums_match_the_oracle(oracle_py, device, dof, limb_joints, heads):
+    """A wide block sums its heads over the links 16 heads a pass at 40 coordinates, 32 from 44 and 64 from 60: limbs of two
+    joints give every joint's link a sphere, and so two passes or three with a last one in part full (one, at 60)."""
+    E = 32
+    tree, desc, state = tree_case(oracle_py, dof, True, True, seed=13 * dof, E=E, limb_joints=limb_joints)
+    assert len(tree.sphere_links) == heads
+    oracle = oracle_py.OracleWorld(tree.template, desc, threads=8)
+    world = nk.World(device, tree.template, desc)
+    assert world.dof == dof
+    oracle.set_state(state)
+    world.set_state(state)
+    sens = one_ulp_sensitivity(oracle_py, tree.template, desc, state)
+    compare_ops(oracle, world, E, sens, state)
+    assert oracle.download("contact_count").max() > heads // 2, "the passes past the first must hold live heads"
+    close(world, oracle, "link_velocity", tol=bar(sens, "velocity"))
+    world.close()
+    oracle.close()
