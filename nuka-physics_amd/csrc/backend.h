@@ -20,7 +20,7 @@ bool BackendSupportsOp(NkOp op);
 void InitArticulationKernels();
 void InitSolverKernels();
 void InitContactKernels();
-uint32_t SolverHeadCapacity(const ModelView& m, uint32_t slots, size_t lds_budget_bytes);
+uint32_t SolverHeadCapacity(const ModelView& m, uint32_t slots);
 // the width the sweeps of the world's block-descent solve run at: its coordinates, or fewer for a reduced block
 uint32_t SolverSweepWidth(const ModelView& m);
 // blocks of the world's full-capacity solve launch that one compute unit holds at once (runtime occupancy query for

@@ -34,14 +34,19 @@ NKH_DECLARE_DENSE(24, 12) NKH_DECLARE_DENSE(28, 16) NKH_DECLARE_DENSE(32, 16) NK
 
 
 // Heads the solver's LDS holds: the contact heads (each stages three Jacobian rows) plus one unit head per joint row
-// slot.  Returns the contact-head capacity that fits `lds_budget_bytes`, 0 when not even one does.
-uint32_t SolverHeadCapacity(const ModelView& m, uint32_t slots, size_t lds_budget_bytes) {
+// slot.  Returns the contact-head capacity that fits the budget, 0 when not even one does.  The Hessian rows that a block
+// of at most 32 coordinates keeps (KeptRowFloats, 4 KB at most) are not counted against the budget: they save time and
+// would cost a full world heads (six of 230 at 32 coordinates), and a compute unit has room for both.
+constexpr size_t kHeadLdsBytes = 150u * 1024u;
+static_assert(kHeadLdsBytes + 32u * 32u * sizeof(float) <= 160u * 1024u, "the largest tile and its kept rows fit a compute unit");
+uint32_t SolverHeadCapacity(const ModelView& m, uint32_t slots) {
     // a contact point is one head, or four under the pyramidal cone of the MuJoCo law (one scalar head an edge)
     const uint32_t heads_per_point = m.any_mujoco != 0u && m.contact_cone == 0u ? kRowsPerPoint : 1u;
     const uint32_t want = slots * (m.max_points_per_slot == 0u ? kPointsPerSlot : m.max_points_per_slot) * heads_per_point;
     const uint32_t joint_heads = m.joint_limit_rows + m.joint_friction_rows + m.joint_drive_rows;
     for (uint32_t staged = want; staged >= 1u; --staged)
-        if (size_t{solver::SolverLdsFloats(m.dof, staged + joint_heads, staged)} * sizeof(float) <= lds_budget_bytes) return staged;
+        if (size_t{solver::SolverLdsFloats(m.dof, staged + joint_heads, staged) - solver::KeptRowFloats(m.dof, false)} * sizeof(float) <=
+            kHeadLdsBytes) return staged;
     return 0u;
 }
 
@@ -176,7 +181,7 @@ static SolverKernel KernelOfWidth(const ModelView& m, bool contacts_only, uint32
 // once, as the runtime's occupancy query answers for the kernel and the LDS the launch asks for; 0 without a solve.
 uint32_t SolverBlocksPerUnit(const ModelView& m, uint32_t env_count) {
     if (m.rows_per_env == 0u || m.dof == 0u) return 0u;
-    const uint32_t staged = SolverHeadCapacity(m, std::max(m.contact_slots, 1u), 150u * 1024u);
+    const uint32_t staged = SolverHeadCapacity(m, std::max(m.contact_slots, 1u));
     if (staged == 0u) return 0u;
     const uint32_t joint_heads = m.joint_limit_rows + m.joint_friction_rows + m.joint_drive_rows;
     const bool contacts_only = ContactHeadsOnly(m, staged);
@@ -198,7 +203,7 @@ uint32_t SolverMassFactorFloats(const ModelView& m) {
 }
 uint32_t SolverSweepWidth(const ModelView& m) {
     if (m.rows_per_env == 0u || m.dof == 0u) return m.dof;
-    const uint32_t staged = SolverHeadCapacity(m, std::max(m.contact_slots, 1u), 150u * 1024u);
+    const uint32_t staged = SolverHeadCapacity(m, std::max(m.contact_slots, 1u));
     return SolverWorkingWidth(m, staged != 0u && ContactHeadsOnly(m, staged));
 }
 
@@ -208,8 +213,7 @@ Status OpBlockDescentSolve(const ModelView& m, const DataView& d, const void* pa
     if (p->env_count == 0u || p->rows_per_env == 0u || p->articulation_count == 0u) return Status::Ok;
     if (p->articulation_count != p->env_count || m.dof == 0u || m.dof > kMaxDof || p->max_dof != m.max_dof ||
         p->iterations == 0u) return Status::InvalidArgument;
-    const size_t budget = 150u * 1024u;
-    const uint32_t staged = SolverHeadCapacity(m, p->contact_slots_per_env == 0u ? 1u : p->contact_slots_per_env, budget);
+    const uint32_t staged = SolverHeadCapacity(m, p->contact_slots_per_env == 0u ? 1u : p->contact_slots_per_env);
     if (staged == 0u) return Status::InvalidArgument;
     const uint32_t joint_heads = m.joint_limit_rows + m.joint_friction_rows + m.joint_drive_rows;
     const bool contacts_only = ContactHeadsOnly(m, staged);

@@ -911,7 +911,7 @@ nuka_result_t CreateWorld(nuka_device_handle device, const nuka_template_desc_t*
         const size_t mf = SolverMassFactorFloats(hc);
         const size_t fb = hc.free_body != 0u ? nb : 0u;   // the rigid-body fields have their rows in a world of free bodies only
         if (E * std::max<size_t>(R, 1u) > 0xFFFFFFFFull / 2u || E * nl * 7u > 0xFFFFFFFFull) throw std::invalid_argument("world too large for 32-bit row indices");
-        if (hc.rows_per_env > 0u && SolverHeadCapacity(hc, std::max(hc.contact_slots, 1u), 150u * 1024u) == 0u) throw std::invalid_argument("solver tile does not fit LDS");
+        if (hc.rows_per_env > 0u && SolverHeadCapacity(hc, std::max(hc.contact_slots, 1u)) == 0u) throw std::invalid_argument("solver tile does not fit LDS");
         // arena layout: template tables first, then the env-major fields, each on a 256-byte boundary (buffer.hpp:39)
         size_t cursor = 0u;
 #define X(name, dtype) Place<int>(w.fields, #name, dtype, w.host.name.size(), &cursor, true);
