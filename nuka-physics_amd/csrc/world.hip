@@ -468,8 +468,8 @@ struct World {   // src/c_abi/internal.hpp:153-165 WorldRecord + nk::World
     std::vector<std::string> link_names, joint_names;   // per template link; a joint's name sits at its child link
     nuka_phi_execution_error last_error{};
 
-    uint32_t* reset_ids = nullptr;       // nuka_world_reset_envs: pinned host memory, env_count words, from its first call on
-    std::vector<uint8_t> reset_seen;     // and the environments that call has met
+    uint32_t* reset_ids = nullptr;       // nuka_world_reset_envs: pinned host memory, env_count words
+    std::vector<uint8_t> reset_seen;     // and the environments that a call has met, env_count of them
 
     ~World() {
         if (reset_ids != nullptr) (void)hipHostFree(reset_ids);
@@ -927,6 +927,12 @@ nuka_result_t CreateWorld(nuka_device_handle device, const nuka_template_desc_t*
         if (w.arena == nullptr) return Error(NUKA_RESULT_OUT_OF_MEMORY, "arena allocation failed");
         w.initial = reinterpret_cast<nuka_phi_buffer_type_head*>(type)->iface->alloc(type, w.arena_bytes, &status);
         if (w.initial == nullptr) return Error(NUKA_RESULT_OUT_OF_MEMORY, "reset snapshot allocation failed");
+        w.reset_seen.resize(E);
+        if (hipHostMalloc(reinterpret_cast<void**>(&w.reset_ids), E * sizeof(uint32_t), hipHostMallocDefault) != hipSuccess) {
+            (void)hipGetLastError();
+            w.reset_ids = nullptr;
+            return Error(NUKA_RESULT_OUT_OF_MEMORY, "reset id allocation failed");
+        }
         if (Iface(w.arena)->memset(w.arena, 0u, 0u, w.arena_bytes) != uint8_t(Status::Ok)) return Error(NUKA_RESULT_DEVICE_ERROR, "arena clear failed");
         char* base = static_cast<char*>(Iface(w.arena)->base(w.arena));
         w.model = hc;
@@ -1273,16 +1279,11 @@ nuka_result_t nuka_world_reset_envs(nuka_world_handle world, const uint32_t* env
         if (env_ids[i] >= w->env_count) return Error(NUKA_RESULT_INVALID_ARG, "environment id out of range");
     // The upload is from pinned memory of the world's own, so it is enqueued like the kernel, and the one wait at the end is
     // the call's contract.  A first wait, before an upload from pageable memory, left the device idle between the steps
-    // already submitted and the reset.
-    if (w->reset_ids == nullptr &&
-        hipHostMalloc(reinterpret_cast<void**>(&w->reset_ids), size_t{w->env_count} * sizeof(uint32_t), hipHostMallocDefault) != hipSuccess) {
-        (void)hipGetLastError();
-        w->reset_ids = nullptr;
-        return Error(NUKA_RESULT_OUT_OF_MEMORY, "reset ids");
-    }
+    // already submitted and the reset.  That memory and the list of environments met come with the world: no call in a step
+    // loop allocates, the first one included.
     ResetSegments segments{};
     if (ResetSegmentsOf(w, &segments) != NUKA_RESULT_OK) return Error(NUKA_RESULT_INTERNAL, "too many reset segments");
-    w->reset_seen.assign(w->env_count, 0u);
+    std::fill(w->reset_seen.begin(), w->reset_seen.end(), uint8_t{0});
     uint32_t unique = 0u;
     for (uint32_t i = 0u; i < count; ++i)
         if (w->reset_seen[env_ids[i]] == 0u) { w->reset_seen[env_ids[i]] = 1u; w->reset_ids[unique++] = env_ids[i]; }
@@ -1290,8 +1291,9 @@ nuka_result_t nuka_world_reset_envs(nuka_world_handle world, const uint32_t* env
     if (hipMemcpyAsync(w->data.reset_env_ids, w->reset_ids, size_t{unique} * sizeof(uint32_t), hipMemcpyHostToDevice, stream) != hipSuccess)
         return Error(NUKA_RESULT_DEVICE_ERROR, "id upload failed");
     hipLaunchKernelGGL(ResetEnvsKernel, dim3(unique, segments.count), dim3(256), 0, stream, segments, w->data.reset_env_ids, w->env_count);
-    if (hipGetLastError() != hipSuccess) return Error(NUKA_RESULT_DEVICE_ERROR, "reset launch failed");
-    return nuka_world_synchronize(world);   // the ids may be written again
+    const bool launched = hipGetLastError() == hipSuccess;
+    const nuka_result_t waited = nuka_world_synchronize(world);   // the ids may be written again
+    return launched ? waited : Error(NUKA_RESULT_DEVICE_ERROR, "reset launch failed");
 }
 
 // nuka_world_reset_envs for callers that cannot allocate: same kernel, same result, but the ids are staged in the
