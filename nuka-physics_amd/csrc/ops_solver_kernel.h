@@ -814,6 +814,7 @@ __device__ __forceinline__ void add_heads_by_tiles(const Tile& c, uint64_t heads
     double force[T] = {};
     float bound[T] = {};
     while (heads != 0ull) {
+        const uint32_t first = uint32_t(__builtin_ctzll(heads));   // what a group without a head reads: its rows are staged
         uint32_t mine = kInvalid;
 #pragma unroll
         for (uint32_t k = 0u; k < 4u; ++k) {
@@ -822,7 +823,7 @@ __device__ __forceinline__ void add_heads_by_tiles(const Tile& c, uint64_t heads
             mine = group == k ? h : mine;
         }
         const bool live = mine != kInvalid;
-        const int source = int((live ? mine : 0u) * 4u);
+        const int source = int((live ? mine : first) * 4u);
         const float* rows = c.jac + uint32_t(__builtin_amdgcn_ds_bpermute(source, int(my_first))) * uint32_t(N);
         float f[3], cv[6] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f}, noise[3];
 #pragma unroll
@@ -927,6 +928,9 @@ __device__ __forceinline__ void add_heads_by_groups(const Tile& c, uint64_t head
         g.value = 0.0; scale = 0.0f;
     }
     while (heads != 0ull) {
+        // what lanes without a head read: its rows are staged, and add_columns multiplies a word of theirs by zero, which must
+        // be a finite word
+        const uint32_t first = uint32_t(__builtin_ctzll(heads));
         uint32_t mine = kInvalid;
 #pragma unroll
         for (int k = 0; k < G; ++k) {
@@ -935,7 +939,7 @@ __device__ __forceinline__ void add_heads_by_groups(const Tile& c, uint64_t head
             mine = group == uint32_t(k) ? h : mine;
         }
         const bool none = mine == kInvalid;   // also the lanes past the last group
-        const int source = int((none ? 0u : mine) * 4u);
+        const int source = int((none ? first : mine) * 4u);
         const float* rows = c.jac + uint32_t(__builtin_amdgcn_ds_bpermute(source, int(my_first))) * uint32_t(N);
         float f[3], noise[3];
 #pragma unroll
