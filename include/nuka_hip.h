@@ -301,7 +301,7 @@ typedef struct nuka_world_execution_info_t {
     uint64_t capture_attempts;
     uint64_t graph_replays;
     nuka_result_t last_result;
-    uint32_t failed_op;
+    uint32_t failed_op;   /* the op that failed; where a step runs several as one launch and that fails, the first of them (the message names all) */
     int32_t native_error;
     char message[256];
 } nuka_world_execution_info_t;

@@ -152,9 +152,10 @@ Status DispatchOn(Backend* be, const ModelView& m, const DataView& d, const nuka
 }
 
 // IntegratePosition, FkWorldPoses, FkLinkVelocities and, if it follows, SyncLinkBodyPose at the head of `calls` as one
-// launch: the number of calls served, 0 when the head is something else or the merged kernel does not serve these
-// parameters (Unsupported: the ops then run one by one).  Any other failure of the merged launch is the plan's
-// failure and comes back through `status`, never as a quiet fall back that would dispatch the ops a second time.
+// launch: the number of calls it covers, 0 when the head is something else or the merged kernel does not serve these
+// parameters (Unsupported: the ops then run one by one, and each names its own parameters' errors).  Any other failure of
+// the merged launch is the step's or the plan's and comes back through `failure`, never as a quiet fall back that would
+// dispatch the ops a second time.
 int MergeStepTail(Backend* be, const ModelView& m, const DataView& d, const nuka_phi_op_call* calls, int n, Status* failure) {
     if (n < 3 || calls[0].op != uint16_t(NkOp::IntegratePosition) || calls[1].op != uint16_t(NkOp::FkWorldPoses) ||
         calls[2].op != uint16_t(NkOp::FkLinkVelocities)) return 0;
@@ -163,8 +164,9 @@ int MergeStepTail(Backend* be, const ModelView& m, const DataView& d, const nuka
                                      static_cast<const FkWorldPosesParams*>(calls[1].params),
                                      static_cast<const FkLinkVelocitiesParams*>(calls[2].params),
                                      bodies ? static_cast<const SyncLinkBodyPoseParams*>(calls[3].params) : nullptr, be->stream);
-    if (status != Status::Ok && status != Status::Unsupported) *failure = status;
-    return status == Status::Ok ? (bodies ? 4 : 3) : 0;
+    if (status == Status::Unsupported) return 0;
+    *failure = status;
+    return bodies ? 4 : 3;
 }
 
 // SyncLinkBodyPose, BuildAabbs, LbvhBuild, LbvhQueryPairs, NarrowphasePrimitives at the head of `calls` as one launch
@@ -176,18 +178,19 @@ int MergeCollisionHead(Backend* be, const ModelView& m, const DataView& d, const
                                           static_cast<const BuildAabbsParams*>(calls[1].params),
                                           static_cast<const LbvhQueryPairsParams*>(calls[3].params),
                                           static_cast<const NarrowphasePrimitivesParams*>(calls[4].params), be->stream);
-    if (status != Status::Ok && status != Status::Unsupported) *failure = status;
-    return status == Status::Ok ? 5 : 0;
+    if (status == Status::Unsupported) return 0;
+    *failure = status;
+    return 5;
 }
 
 // The next launch of an op list: the ops after the solve, and those between the dynamics and the row assembly, each take
 // about a launch's time, so where the list holds them in a row one kernel runs them (StepTailKernel, CollisionHeadKernel);
-// where it cannot, the first op goes alone.  `served` is the number of ops that the launch covers.
+// where it cannot, the first op goes alone.  `served` is the number of ops that the launch covers, also one that failed.
 Status DispatchNext(Backend* be, const ModelView& m, const DataView& d, const nuka_phi_op_call* calls, int n, int* served) {
     Status status = Status::Ok;
     *served = MergeStepTail(be, m, d, calls, n, &status);
-    if (*served == 0 && status == Status::Ok) *served = MergeCollisionHead(be, m, d, calls, n, &status);
-    if (*served > 0 || status != Status::Ok) return status;
+    if (*served == 0) *served = MergeCollisionHead(be, m, d, calls, n, &status);
+    if (*served > 0) return status;
     *served = 1;
     return DispatchOn(be, m, d, calls[0]);
 }

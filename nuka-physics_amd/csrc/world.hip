@@ -744,7 +744,11 @@ nuka_result_t StepEager(World& w) {
         if (status != uint8_t(Status::Ok)) {
             w.last_error = {};
             w.last_error.status = status; w.last_error.failed_op = call.op;
-            std::snprintf(w.last_error.message, sizeof(w.last_error.message), "step failed in op %s", OpName(static_cast<NkOp>(call.op)));
+            char* message = w.last_error.message;
+            size_t length = size_t(std::snprintf(message, sizeof(w.last_error.message), "step failed in op %s", OpName(static_cast<NkOp>(call.op))));
+            for (int k = 1; k < served; ++k)   // the ops of one launch fail together: failed_op is the first of them
+                length += size_t(std::snprintf(message + length, sizeof(w.last_error.message) - length, "%s%s", k == 1 ? ", one launch with " : ", ",
+                                               OpName(static_cast<NkOp>(w.calls[i + k].op))));
             return Error(MapStatus(status), w.last_error.message);
         }
     }
