@@ -101,3 +101,37 @@ def test_link_wrenches_are_the_sums_of_the_rows(device, robot, envs):
     # a row's terms round a handful of times each, and as many sums as the link has rows follow: some tens of half an ulp of their size
     assert np.all(np.abs(got - wrench / dt) <= 64 * 6e-8 / dt * size[:, None] + 1e-12)
     world.close()
+
+
+@pytest.mark.parametrize("robot,envs", [("quadruped", 65), ("rope", 33), ("walker", 65)])
+def test_steps_after_restores_are_those_of_a_world_never_restored(device, robot, envs):
+    """From the ground to the air and back, several steps each, a plan's replays and eager steps in turn: what the rows of
+    one leave behind must not reach the other."""
+    world, _, low, high = made(device, robot, envs)
+    world.download("link_contact_wrench")
+    held, points = {}, {}
+    for name, state in (("low", low), ("high", high)):
+        world.set_state(state)
+        held[name] = world.checkpoint()
+    world.restore(held["low"])
+    world.set_execution_mode(True)
+    world.step(3)
+    for name, state, modes in (("high", high, (False, True, True)), ("low", low, (True, False, False, True)), ("high", high, (True, False)),
+                               ("low", low, (False, True))):
+        world.restore(held[name])
+        for graph in modes:
+            world.set_execution_mode(graph)
+            world.step()
+        fresh = made(device, robot, envs)[0]
+        fresh.download("link_contact_wrench")
+        fresh.set_state(state)
+        fresh.step(len(modes))
+        after, expect = rows_of(world), rows_of(fresh)
+        points[name] = int(expect["contact_count"].sum())
+        for field, value in expect.items():
+            assert np.array_equal(after[field], value), (name, modes, field)
+        fresh.close()
+    assert points["low"] > 2 * points["high"]
+    for checkpoint in held.values():
+        nk.lib().nuka_checkpoint_destroy(checkpoint)
+    world.close()
