@@ -38,7 +38,7 @@ def crowded(dof, heads, friction, E, seed):
     return t, dict(q=q, qdot=qd, tau=tau, base_pose=base, root_twist=g.normal(0.0, 0.3, (E, 6)).astype(np.float32))
 
 
-# (coordinates, joint friction, contact heads): what 150 KB of LDS hold of heads (a contact head 59 words and three rows of
+# (coordinates, joint friction, contact heads): what 150 KB of LDS hold of heads (a contact head 60 words and three rows of
 # the block's width, a joint row's unit head 31) beside the block's two factors
 CASES = [(12, 0.0, 393), (16, 0.0, 347), (20, 0.0, 310), (24, 0.0, 279), (28, 0.0, 253), (32, 0.0, 230), (20, 0.1, 303), (32, 0.1, 222),
          (36, 0.0, 218)]
