@@ -39,10 +39,10 @@ NKH_DECLARE_DENSE(24, 12) NKH_DECLARE_DENSE(28, 16) NKH_DECLARE_DENSE(32, 16) NK
 // would cost a full world heads (six of 230 at 32 coordinates), and a compute unit has room for both.
 constexpr size_t kHeadLdsBytes = 150u * 1024u;
 static_assert(kHeadLdsBytes + 32u * 32u * sizeof(float) <= 160u * 1024u, "the largest tile and its kept rows fit a compute unit");
+// a contact point is one head, or four under the pyramidal cone of the MuJoCo law (one scalar head an edge)
+static uint32_t HeadsAPoint(const ModelView& m) { return m.any_mujoco != 0u && m.contact_cone == 0u ? kRowsPerPoint : 1u; }
 uint32_t SolverHeadCapacity(const ModelView& m, uint32_t slots) {
-    // a contact point is one head, or four under the pyramidal cone of the MuJoCo law (one scalar head an edge)
-    const uint32_t heads_per_point = m.any_mujoco != 0u && m.contact_cone == 0u ? kRowsPerPoint : 1u;
-    const uint32_t want = slots * (m.max_points_per_slot == 0u ? kPointsPerSlot : m.max_points_per_slot) * heads_per_point;
+    const uint32_t want = slots * (m.max_points_per_slot == 0u ? kPointsPerSlot : m.max_points_per_slot) * HeadsAPoint(m);
     const uint32_t joint_heads = m.joint_limit_rows + m.joint_friction_rows + m.joint_drive_rows;
     for (uint32_t staged = want; staged >= 1u; --staged)
         if (size_t{solver::SolverLdsFloats(m.dof, staged + joint_heads, staged) - solver::KeptRowFloats(m.dof, false)} * sizeof(float) <=
@@ -163,7 +163,7 @@ static bool ContactHeadsOnly(const ModelView& m, uint32_t staged) {
     const uint32_t joint_heads = m.joint_limit_rows + m.joint_friction_rows + m.joint_drive_rows;
     return joint_heads == 0u && staged <= uint32_t(solver::kWave) && !(m.any_mujoco != 0u && m.contact_cone == 1u);
 }
-// `dense_out`: whether the kernel is a dense one (three waves a SIMD)
+// `dense_out`: whether the kernel is a dense one
 static SolverKernel KernelOfWidth(const ModelView& m, bool contacts_only, uint32_t width, uint32_t env_count, bool* dense_out = nullptr) {
     if (dense_out != nullptr) *dense_out = false;
     if (contacts_only && env_count >= kDenseBatch)
@@ -231,23 +231,25 @@ Status OpBlockDescentSolve(const ModelView& m, const DataView& d, const void* pa
     // The LDS a block needs grows with the contact heads it can stage, and a scene's slots (every pair that may ever
     // touch, at its largest manifold) outnumber the contacts an environment usually has.  Where a smaller capacity
     // lets more blocks share a compute unit, environments with few contact points go to a launch of that capacity:
-    // up to three such launches, for eight, four and two blocks a unit, before the full one.  Each launch takes the
+    // a launch each for twelve, eight, four and two blocks a unit, those the waves allow, before the full one.  Each launch takes the
     // environments whose contact points fall in its range; an environment's results do not depend on its launch.
+    // A contact point is at most `a_point` heads, so `few` heads hold few / a_point points whatever their friction: four
+    // edges a point under the pyramidal cone.  (While those worlds went to the one full launch, a walker's 304 heads left a
+    // compute unit one block for environments of a handful of points: a step of 4096 with a twentieth reset 768 -> 438 us.)
     hipLaunchKernelGGL(OrderTilesKernel, dim3(1), dim3(1024), 0, stream, d, p->env_count);
     uint32_t first_points = 0u;
-    // (a launch takes its environments by their contact points, one head a point: not under the pyramidal cone, whose
-    // worlds go to the one full launch)
-    const bool one_head_a_point = !(m.any_mujoco != 0u && m.contact_cone == 0u);
-    if (p->contact_slots_per_env != 0u && one_head_a_point) {
+    const uint32_t a_point = HeadsAPoint(m);
+    if (p->contact_slots_per_env != 0u) {
         for (const size_t blocks : {size_t{12u}, size_t{8u}, size_t{4u}, size_t{2u}}) {
             if (blocks > most_blocks) continue;                            // more blocks than the waves allow
             if (blocks_per_unit(staged) >= blocks) break;                  // the full capacity does as well
             uint32_t few = staged;
             while (few > 8u && blocks_per_unit(few) < blocks) --few;
-            if (blocks_per_unit(few) < blocks || few < first_points) continue;   // not even eight heads fit that often
+            const uint32_t points = few / a_point;
+            if (blocks_per_unit(few) < blocks || points < first_points) continue;   // not even eight heads fit that often
             hipLaunchKernelGGL(kernel, dim3(p->env_count), dim3(solver::kWave), lds_bytes(few), stream, m, d, *p, few + joint_heads, few,
-                               first_points, few);
-            first_points = few + 1u;
+                               first_points, points);
+            first_points = points + 1u;
         }
     }
     hipLaunchKernelGGL(kernel, dim3(p->env_count), dim3(solver::kWave), lds_bytes(staged), stream, m, d, *p, staged + joint_heads, staged,
