@@ -19,7 +19,7 @@ NKH_DECLARE_REDUCED(24, 12) NKH_DECLARE_REDUCED(28, 16) NKH_DECLARE_REDUCED(32, 
 NKH_DECLARE_REDUCED(44, 24) NKH_DECLARE_REDUCED(48, 24) NKH_DECLARE_REDUCED(52, 28) NKH_DECLARE_REDUCED(56, 28) NKH_DECLARE_REDUCED(60, 32)
 NKH_DECLARE_REDUCED(64, 32)
 #undef NKH_DECLARE_REDUCED
-// The dense build of the same template (ops_solver_kernel.h compiled with NKH_SOLVER_DENSE: three waves a SIMD), for the
+// The dense build of the same template (ops_solver_kernel.h compiled with NKH_SOLVER_DENSE: three or four waves a SIMD), for the
 // widths it is instantiated at in ops_solver_d*.hip.
 namespace dense {
 template <int N, bool kContactsOnly, int K = N>
@@ -224,14 +224,14 @@ Status OpBlockDescentSolve(const ModelView& m, const DataView& d, const void* pa
     };
     bool dense = false;
     const SolverKernel kernel = KernelOfWidth(m, contacts_only, width, p->env_count, &dense);
-    // widths past kTwoWaveWidth run one wave a SIMD: four blocks a compute unit at most, whatever their LDS; the dense
-    // kernels run three, twelve blocks
-    const size_t most_blocks = dense ? 12u : solver::PaddedWidth(width) > uint32_t(solver::kTwoWaveWidth) ? 4u : 8u;
+    // blocks a compute unit holds at most, whatever their LDS: four a wave of a SIMD
+    const int padded = int(solver::PaddedWidth(width));
+    const size_t most_blocks = 4u * size_t(dense ? solver::DenseWavesPerSimd(padded) : solver::WavesPerSimd(padded));
     const auto blocks_per_unit = [&](uint32_t contact_heads) { return std::min<size_t>(most_blocks, (160u * 1024u) / lds_bytes(contact_heads)); };
     // The LDS a block needs grows with the contact heads it can stage, and a scene's slots (every pair that may ever
     // touch, at its largest manifold) outnumber the contacts an environment usually has.  Where a smaller capacity
     // lets more blocks share a compute unit, environments with few contact points go to a launch of that capacity:
-    // a launch each for twelve, eight, four and two blocks a unit, those the waves allow, before the full one.  Each launch takes the
+    // a launch each for sixteen, twelve, eight, four and two blocks a unit, those the waves allow, before the full one.  Each launch takes the
     // environments whose contact points fall in its range; an environment's results do not depend on its launch.
     // A contact point is at most `a_point` heads, so `few` heads hold few / a_point points whatever their friction: four
     // edges a point under the pyramidal cone.  (While those worlds went to the one full launch, a walker's 304 heads left a
@@ -240,7 +240,7 @@ Status OpBlockDescentSolve(const ModelView& m, const DataView& d, const void* pa
     uint32_t first_points = 0u;
     const uint32_t a_point = HeadsAPoint(m);
     if (p->contact_slots_per_env != 0u) {
-        for (const size_t blocks : {size_t{12u}, size_t{8u}, size_t{4u}, size_t{2u}}) {
+        for (const size_t blocks : {size_t{16u}, size_t{12u}, size_t{8u}, size_t{4u}, size_t{2u}}) {
             if (blocks > most_blocks) continue;                            // more blocks than the waves allow
             if (blocks_per_unit(staged) >= blocks) break;                  // the full capacity does as well
             uint32_t few = staged;

@@ -1,4 +1,4 @@
-// Dense instantiations of the block-descent kernel (three waves a SIMD, contact heads only) for padded widths 4 ... 20.
+// Dense instantiations of the block-descent kernel (three or four waves a SIMD, contact heads only) for padded widths 4 ... 20.
 #define NKH_SOLVER_DENSE
 #include "ops_solver_kernel.h"
 namespace nkh {

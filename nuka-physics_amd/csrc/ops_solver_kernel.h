@@ -29,8 +29,8 @@ namespace nkh {
 namespace solver {
 // This header compiles two ways.  Plainly, a block of up to kTwoWaveWidth coordinates runs two waves a SIMD with up to 256
 // registers each.  With NKH_SOLVER_DENSE defined (ops_solver_d*.hip) everything below sits in namespace `dense` and a block
-// of up to kThreeWaveWidth coordinates is compiled for three waves a SIMD: 168 registers, a few dozen values a lane in
-// scratch memory, the same arithmetic.  A long environment runs a tenth slower that way and a full machine gets a tenth
+// of up to twenty coordinates is compiled for three waves a SIMD, of up to eight for four (DenseWavesPerSimd): 168 or 128
+// registers, a few dozen values a lane in scratch memory at some widths, the same arithmetic.  A long environment runs a tenth slower that way and a full machine gets a tenth
 // more done, so the launcher takes the dense kernels for batches that fill the machine several times over.
 #ifdef NKH_SOLVER_DENSE
 namespace dense {
@@ -42,13 +42,15 @@ constexpr int kWave = 64;
 #define NKH_TWO_WAVE_WIDTH 36
 #endif
 constexpr int kTwoWaveWidth = NKH_TWO_WAVE_WIDTH;
-// Widths up to this run three waves per SIMD in the dense build (none in the plain one).
+// Waves per SIMD of the dense build at widths it is instantiated at: four where 128 registers hold the block without
+// scratch memory (eight coordinates need 126, twelve spill 12 bytes a lane), else three.  A step of 16384 free boxes
+// (six coordinates) 642 -> 588 us, of 65536 2128 -> 1904 us, with a fourth wave.
+constexpr int DenseWavesPerSimd(int width) { return width <= 8 ? 4 : width <= 20 ? 3 : 0; }
 #ifdef NKH_SOLVER_DENSE
-constexpr int kThreeWaveWidth = 20;
+constexpr int WavesPerSimd(int width) { return DenseWavesPerSimd(width) != 0 ? DenseWavesPerSimd(width) : (width <= kTwoWaveWidth ? 2 : 1); }
 #else
-constexpr int kThreeWaveWidth = 0;
+constexpr int WavesPerSimd(int width) { return width <= kTwoWaveWidth ? 2 : 1; }
 #endif
-constexpr int WavesPerSimd(int width) { return width <= kThreeWaveWidth ? 3 : (width <= kTwoWaveWidth ? 2 : 1); }
 // From this width on a block widens its mass rows to double where it uses them; below it the widened rows are kept over
 // the solve (two registers an entry), which pays while they fit.  In the dense build's 168 registers they never do:
 // kept, they are what spills (96 B a lane at 20 coordinates, none widened at use; 65536 quadrupeds 6.74 -> 6.48 ms).
@@ -2521,8 +2523,9 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
     }
     const uint32_t R = p.rows_per_env, md = p.max_dof, n = m.dof, nl = m.links_per_env, S = p.contact_slots_per_env;
     // A narrow block would leave registers free and let more waves share a SIMD than the launch is sized for; one name of
-    // the last register holds the kernel to its two (dense build: three) waves.
-    if constexpr (WavesPerSimd(W) == 3) asm volatile("" ::: "v163");
+    // the last register holds the kernel to its two (dense build: three or four) waves.
+    if constexpr (WavesPerSimd(W) == 4) asm volatile("" ::: "v127");
+    else if constexpr (WavesPerSimd(W) == 3) asm volatile("" ::: "v163");
     else if constexpr (WavesPerSimd(W) == 2) asm volatile("" ::: "v255");
     Tile c;
     c.env = env; c.lane = lane; c.n = kReduced ? uint32_t(K) : n; c.n_all = n; c.ldj = uint32_t(W); c.cap = cap; c.narrow = staged_cap; c.heads = 0u; c.iteration = 0u;
