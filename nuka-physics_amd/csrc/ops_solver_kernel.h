@@ -400,64 +400,58 @@ __device__ __forceinline__ float pivot_scale(float pivot) { return __builtin_amd
 __device__ __forceinline__ bool pivots_valid(uint32_t lane, uint32_t N, float inverse) {
     return __all(lane >= N || (inverse > 0.0f && inverse <= FLT_MAX));
 }
-// From sixteen coordinates on four columns of a full block go as a panel: within it a column's update takes lane reads, and the columns
-// past it lose the panel's four on the matrix cores - v_mfma_f32_4x4x1 with the panel's words of rows 4 q .. 4 q + 3 (from
-// LDS, `panel`: 4 N words) on the one side and the lane's own on the other gives the rows' layout, an instruction a column
-// where a lane read and a multiply-add an entry went before, each the fused multiply-add it was and in the same order, bit
-// for bit.  4096 quadrupeds 538 -> 519 us a step (514 with the products under the next pivots), 1000 servo-driven ones
-// 2228 -> 2070 us for four.  Narrower factors have too
-// few columns past a panel to pay for its way through LDS, and a reduced block, which keeps more in registers, lost by it
-// (333 humanoids 576 -> 588 us, 4096 823 -> 838 us).
+// Four columns go as a panel: within it a column's update takes lane reads, and the columns past it lose each of the
+// panel's four on the matrix cores.  v_mfma_f32_4x4x1 multiplies, in each block of four lanes, four values a block with one a
+// lane, and its broadcast of one block's four to all sixteen (cbsz 4, abid q) takes the column's own register for both
+// sides: the words of rows 4 q .. 4 q + 3 against the lane's own come out in the rows' layout, columns 4 q .. 4 q + 3 of
+// the lane's row, with nothing passed through LDS.  An instruction for four columns where a lane read and a multiply-add an entry
+// go otherwise, each the fused multiply-add it was and in the same order, bit for bit.  (With the panel's words handed round
+// through LDS, an exchange and two waits a panel, a step of 8192 ropes took 17.45 ms, 16.62 as it is; 1000 servo-driven
+// quadrupeds, four steps, 2062 and 2026 us; 4096 humanoids, whose reduced blocks took lane reads throughout, 784 and 780.)
 typedef float Vec4 __attribute__((ext_vector_type(4)));
 // v where bit `at` of the mask is set, else zero: two instructions, no comparison
 __device__ __forceinline__ uint32_t bit_spread(uint32_t mask, uint32_t at) { return uint32_t(__builtin_amdgcn_sbfe(int(mask), at, 1u)); }
 __device__ __forceinline__ float kept_if(uint32_t mask, uint32_t at, float v) { return __uint_as_float(bit_spread(mask, at) & __float_as_uint(v)); }
-template <int N>
-__device__ __forceinline__ void subtract_product(int q, float other, float own, float (&row)[N]) {   // columns 4 q .. 4 q + 3 lose own x other
-    const Vec4 four = __builtin_amdgcn_mfma_f32_4x4x1f32(other, -own, Vec4{row[4 * q], row[4 * q + 1], row[4 * q + 2], row[4 * q + 3]}, 0, 0, 0);
+// columns 4 Q .. 4 Q + 3 lose own x the `column` of rows 4 Q .. 4 Q + 3
+template <int Q, int N>
+__device__ __forceinline__ void subtract_product(float column, float own, float (&row)[N]) {
+    const Vec4 four = __builtin_amdgcn_mfma_f32_4x4x1f32(column, -own, Vec4{row[4 * Q], row[4 * Q + 1], row[4 * Q + 2], row[4 * Q + 3]}, 4, Q, 0);
 #pragma unroll
-    for (int t = 0; t < 4; ++t) row[4 * q + t] = four[t];
+    for (int t = 0; t < 4; ++t) row[4 * Q + t] = four[t];
 }
-template <int N, bool kFollow>
-constexpr bool kPanels = N >= 16 && !kFollow;
-template <int N, bool kFollow>
-__device__ __forceinline__ bool factor_rows(uint32_t lane, float (&row)[N], float* panel, float* inverse_out, float* root_out) {
+// the groups of columns First .. End - 1 (a matrix instruction names the block it broadcasts in its encoding)
+template <int First, int End, int N>
+__device__ __forceinline__ void subtract_products(float column, float own, float (&row)[N]) {
+    if constexpr (First < End) {
+        subtract_product<First>(column, own, row);
+        subtract_products<First + 1, End>(column, own, row);
+    }
+}
+template <int Q, int N>   // from group Q down to the first
+__device__ __forceinline__ void subtract_products_down(float column, float own, float (&row)[N]) {
+    if constexpr (Q >= 0) {
+        subtract_product<Q>(column, own, row);
+        subtract_products_down<Q - 1>(column, own, row);
+    }
+}
+template <int K, int N>
+__device__ __forceinline__ void factor_pivots(uint32_t lane, float (&row)[N], float* inverse, float* root) {
+    if constexpr (K < N) {
+        const float scale = pivot_scale(lane_value(row[K], K));
+        const float scaled = row[K] * scale;
+        if (lane >= uint32_t(K)) { *inverse = scale; *root = scaled; }
+        row[K] = lane > uint32_t(K) ? scaled : 0.0f;
+#pragma unroll
+        for (int j = K + 1; j < K / 4 * 4 + 4; ++j) row[j] = fmaf(-row[K], lane_value(row[K], j), row[j]);
+        subtract_products<K / 4 + 1, N / 4>(row[K], row[K], row);
+        factor_pivots<K + 1>(lane, row, inverse, root);
+    }
+}
+template <int N>
+__device__ __forceinline__ bool factor_rows(uint32_t lane, float (&row)[N], float* inverse_out, float* root_out) {
     lane = local_lane(lane);
     float inverse = 0.0f, root = 0.0f;
-    Vec4* words = reinterpret_cast<Vec4*>(panel);
-    Vec4 others[N / 4];   // the last panel's words of the rows past it
-#pragma unroll
-    for (int k = 0; k < N; ++k) {
-        const float scale = pivot_scale(lane_value(row[k], k));
-        const float scaled = row[k] * scale;
-        if (lane >= uint32_t(k)) { inverse = scale; root = scaled; }
-        row[k] = lane > uint32_t(k) ? scaled : 0.0f;
-        const int end = kPanels<N, kFollow> ? k / 4 * 4 + 4 : N;
-        // lane reads in batches of eight ahead of their multiply-adds: a scalar read has to settle for two cycles
-        // before an arithmetic instruction may use it, and the next reads fill that gap
-#pragma unroll
-        for (int j0 = k + 1; j0 < end; j0 += 8) {
-            float l[8];
-#pragma unroll
-            for (int t = 0; t < 8; ++t) l[t] = j0 + t < end ? lane_value(row[k], j0 + t) : 0.0f;
-#pragma unroll
-            for (int t = 0; t < 8; ++t)
-                if (j0 + t < end) row[j0 + t] = fmaf(-row[k], l[t], row[j0 + t]);
-        }
-        if (!kPanels<N, kFollow>) continue;
-        if (k >= 4) {   // under this pivot's chain: what the columns past this panel still lose to the last one
-#pragma unroll
-            for (int q = k / 4 + 1; q < N / 4; ++q) subtract_product<N>(q, others[q][k % 4], row[k / 4 * 4 - 4 + k % 4], row);
-        }
-        if (k % 4 != 3 || k == N - 1) continue;
-        if (lane < uint32_t(N)) words[lane] = Vec4{row[k - 3], row[k - 2], row[k - 1], row[k]};
-        __syncthreads();
-#pragma unroll
-        for (int q = k / 4 + 1; q < N / 4; ++q) others[q] = words[4u * uint32_t(q) + (lane & 3u)];
-#pragma unroll
-        for (int t = 0; t < 4; ++t) subtract_product<N>(k / 4 + 1, others[k / 4 + 1][t], row[k - 3 + t], row);   // the next panel's own
-        __syncthreads();
-    }
+    factor_pivots<0>(lane, row, &inverse, &root);
     *inverse_out = inverse; *root_out = root;
     return pivots_valid(lane, uint32_t(N), inverse);
 }
@@ -481,41 +475,25 @@ __device__ __forceinline__ uint32_t factor_at(uint32_t i, uint32_t k) {   // lea
 }
 
 // FactorTileColumns on register rows: lane i holds row i of the symmetric matrix; on return its entries k > i are
-// row i of U, every other entry is zero, and `root` is the diagonal.  Panels of four columns as above (`panel`: 4 x 64
-// words).  A step of 8192 ropes (64 coordinates, 4032 instructions of updates before): 24.7 -> 21.9 ms, of 4096 servo-driven
-// humanoids (36 coordinates) 2.30 -> 2.16 ms; with the products that the next panel does not wait for under its pivots, in
-// either direction, and the packed rows stored without conditions 2.10 ms.
+// row i of U, every other entry is zero, and `root` is the diagonal.  Panels of four columns as above.
+template <int K, int N>
+__device__ __forceinline__ void factor_pivots_up(uint32_t lane, float (&row)[N], float* inverse, float* root) {
+    if constexpr (K >= 0) {
+        const float scale = pivot_scale(lane_value(row[K], K));
+        const float scaled = row[K] * scale;
+        if (lane <= uint32_t(K)) { *inverse = scale; *root = scaled; }
+        row[K] = lane < uint32_t(K) ? scaled : 0.0f;
+#pragma unroll
+        for (int j = K - 1; j >= K / 4 * 4; --j) row[j] = fmaf(-row[K], lane_value(row[K], j), row[j]);
+        subtract_products_down<K / 4 - 1>(row[K], row[K], row);
+        factor_pivots_up<K - 1>(lane, row, inverse, root);
+    }
+}
 template <int N>
-__device__ __forceinline__ bool factor_rows_up(uint32_t lane, float (&row)[N], float* panel, float* inverse_out, float* root_out) {
+__device__ __forceinline__ bool factor_rows_up(uint32_t lane, float (&row)[N], float* inverse_out, float* root_out) {
     lane = local_lane(lane);
     float inverse = 0.0f, root = 0.0f;
-    Vec4* words = reinterpret_cast<Vec4*>(panel);
-    Vec4 others[N / 4];   // the last panel's words of the rows left of it
-#pragma unroll
-    for (int p = N / 4 - 1; p >= 0; --p) {
-#pragma unroll
-        for (int t = 3; t >= 0; --t) {
-            const int k = 4 * p + t;
-            const float scale = pivot_scale(lane_value(row[k], k));
-            const float scaled = row[k] * scale;
-            if (lane <= uint32_t(k)) { inverse = scale; root = scaled; }
-            row[k] = lane < uint32_t(k) ? scaled : 0.0f;
-#pragma unroll
-            for (int j = k - 1; j >= 4 * p; --j) row[j] = fmaf(-row[k], lane_value(row[k], j), row[j]);
-            if (p < N / 4 - 1) {   // under this pivot's chain: what the columns left of this panel still lose to the last one
-#pragma unroll
-                for (int q = p - 1; q >= 0; --q) subtract_product<N>(q, others[q][t], row[4 * p + 4 + t], row);
-            }
-        }
-        if (p == 0) break;
-        words[lane] = Vec4{row[4 * p], row[4 * p + 1], row[4 * p + 2], row[4 * p + 3]};
-        __syncthreads();
-#pragma unroll
-        for (int q = p - 1; q >= 0; --q) others[q] = words[4u * uint32_t(q) + (lane & 3u)];
-#pragma unroll
-        for (int t = 3; t >= 0; --t) subtract_product<N>(p - 1, others[p - 1][t], row[4 * p + t], row);   // the next panel's own
-        __syncthreads();
-    }
+    factor_pivots_up<N - 1>(lane, row, &inverse, &root);
     *inverse_out = inverse; *root_out = root;
     return pivots_valid(lane, uint32_t(N), inverse);
 }
@@ -609,7 +587,7 @@ __device__ __forceinline__ bool cholesky_solve(const Tile& c, float (&hrow)[N], 
     float inverse = 0.0f;
     if (!c.factor_current) {   // otherwise the Hessian is the one factored last: its factor is still in hfac
         PROF_BEGIN(c, 14);
-        const bool valid = kLeavesFirst<N> ? factor_rows_up<N>(c.lane, hrow, c.hfac, &inverse, &c.factor_root) : factor_rows<N, kFollow>(c.lane, hrow, c.hfac, &inverse, &c.factor_root);
+        const bool valid = kLeavesFirst<N> ? factor_rows_up<N>(c.lane, hrow, &inverse, &c.factor_root) : factor_rows<N>(c.lane, hrow, &inverse, &c.factor_root);
         PROF_END(c, 14);
         if (!valid) return false;
         PROF_BEGIN(c, 24);
@@ -644,7 +622,7 @@ __device__ __forceinline__ bool factor_mass(Tile& c, const float (&mrow)[N]) {
 #pragma unroll
     for (int k = 0; k < N; ++k) row[k] = mrow[k];
     float inverse = 0.0f, root = 0.0f;
-    const bool valid = kLeavesFirst<N> ? factor_rows_up<N>(c.lane, row, c.hfac, &inverse, &root) : factor_rows<N, kFollow>(c.lane, row, c.hfac, &inverse, &root);
+    const bool valid = kLeavesFirst<N> ? factor_rows_up<N>(c.lane, row, &inverse, &root) : factor_rows<N>(c.lane, row, &inverse, &root);
     c.mass_inverse = inverse;
     store_rows<N>(c.mfac, c.lane, row);
     __syncthreads();
