@@ -201,6 +201,35 @@ __host__ __device__ inline uint32_t DynamicsLdsFloats(uint32_t nl, uint32_t n, u
     return nl * (36u + 36u + 5u * 6u) + n * (n + 1u) + 2u * n + 64u + nl * 7u + sweep_passes * kSweepLinks;
 }
 
+// LDL^T of the matrix whose row `lane` is `row`: the strict lower triangle becomes L and the diagonal D (:269-335).  Entry
+// (i, j) loses (L_ik L_jk) D_k for k = 0, 1, ... with the three roundings of the serial loop (fused into one multiply-add an
+// entry the factor differs in its last place, which an environment that does not converge in its sweeps hands on: one of 256
+// driven humanoids then ends 2.5e-4 from the oracle's).  The products L_ik L_jk come four columns an instruction, columns
+// 4 Q .. 4 Q + 3 of lane's row at a time: v_mfma_f32_4x4x1 multiplies four values a block of four lanes with one a lane,
+// and its broadcast of block Q's four to all blocks (cbsz 4, abid Q) takes the multipliers' own register for them, where a
+// lane read and a product an entry went before.  What a lane computes above its diagonal is never read.
+typedef float Vec4 __attribute__((ext_vector_type(4)));
+template <int Q, int K, int N>
+__device__ __forceinline__ void subtract_products(float lik, float diagonal, float (&row)[N]) {
+    if constexpr (4 * Q < N) {
+        const Vec4 product = __builtin_amdgcn_mfma_f32_4x4x1f32(lik, lik, Vec4{}, 4, Q, 0);
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+            if (4 * Q + t > K) row[4 * Q + t] -= product[t] * diagonal;
+        subtract_products<Q + 1, K>(lik, diagonal, row);
+    }
+}
+template <int K, int N>
+__device__ __forceinline__ void ldlt_pivots(uint32_t lane, float (&row)[N]) {
+    if constexpr (K < N) {
+        const float diagonal = fmaxf(lane_value(row[K], K), 1.0e-6f);
+        const float lik = row[K] / diagonal;
+        row[K] = lane > uint32_t(K) ? lik : (lane == uint32_t(K) ? diagonal : row[K]);
+        subtract_products<(K + 1) / 4, K>(lik, diagonal, row);
+        ldlt_pivots<K + 1>(lane, row);
+    }
+}
+
 // Compiled per padded DoF width N (a multiple of 4): the LDL^T factorisation and the solve keep one matrix row per
 // lane in registers, fully unrolled, and pass pivots and multipliers between lanes as scalar lane reads.
 // The tree sweeps run six lanes a link - a lane a row of the link's 6x6 products - and ten links a pass, a depth at a
@@ -462,11 +491,7 @@ __global__ void __launch_bounds__(2 * kWave) ArticulationDynamicsKernel(ModelVie
             }
         }
         __syncthreads();   // the mass matrix stands in LDS: the first wavefront carries it to HBM while this one factors it
-        // LDL^T, right-looking, lane = row in registers; the strict lower triangle becomes L and the diagonal D (:269-335).
-        // Rows and columns n..N-1 are those of the identity.  Entry (i, j) loses (L_ik L_jk) D_k for k = 0, 1, ... as the
-        // serial loop does (the products in the reference's order: fused into one multiply-add an entry the factor
-        // differs in its last place, and of 4096 humanoids one then ends its eight sweeps 2e-4 from the oracle's);
-        // what a lane computes above its diagonal is never read.
+        // LDL^T, right-looking, lane = row in registers; rows and columns n..N-1 are those of the identity
         {
             // (every word read whether or not the lane keeps it, from a place inside the matrix: a read under a condition
             // compiles to a branch a word)
@@ -479,23 +504,9 @@ __global__ void __launch_bounds__(2 * kWave) ArticulationDynamicsKernel(ModelVie
             }
         }
         {
-            const uint32_t ll = local_lane(lane);
-#pragma unroll
-            for (int k = 0; k < N; ++k) {
-                const float diagonal = fmaxf(lane_value(row[k], k), 1.0e-6f);
-                const float lik = row[k] / diagonal;
-                row[k] = ll > uint32_t(k) ? lik : (ll == uint32_t(k) ? diagonal : row[k]);
-#pragma unroll
-                for (int j0 = k + 1; j0 < N; j0 += 8) {
-                    float l[8];
-#pragma unroll
-                    for (int t = 0; t < 8; ++t) l[t] = j0 + t < N ? lane_value(lik, j0 + t) : 0.0f;
-#pragma unroll
-                    for (int t = 0; t < 8; ++t)
-                        if (j0 + t < N) row[j0 + t] -= lik * l[t] * diagonal;
-                }
-            }
+            ldlt_pivots<0>(local_lane(lane), row);
             __syncthreads();   // the first wavefront has read the mass matrix: its words take the factor
+            const uint32_t ll = local_lane(lane);
             if (ll < n) {
 #pragma unroll
                 for (int k = 0; k < N; ++k)
