@@ -13,6 +13,8 @@
 #include "backend.h"
 #include "nk_ops.h"
 
+#include <type_traits>
+
 namespace nkh {
 
 namespace {
@@ -193,372 +195,694 @@ __global__ void __launch_bounds__(kWave) FkWorldPosesKernel(ModelView m, DataVie
 }
 
 // ---- ArticulationDynamics -------------------------------------------------------------------------------
-// Two wavefronts an environment.  The bias forces (velocities, bias accelerations, the leaf-to-root force pass) and the
-// mass matrix with its factor (composite inertias, columns, LDL^T) do not depend on each other, and each is a chain of
-// tree sweeps that keeps a few lanes busy: the first wavefront takes the one, the second the other, side by side, and
-// they meet before the solve.  Each keeps to its own words of LDS in between.
-__host__ __device__ inline uint32_t DynamicsLdsFloats(uint32_t nl, uint32_t n, uint32_t sweep_passes) {
-    return nl * (36u + 36u + 5u * 6u) + n * (n + 1u) + 2u * n + 64u + nl * 7u + sweep_passes * kSweepLinks;
+// Two wavefronts a workgroup, and G lanes of each an environment, so that a workgroup takes 64 / G environments.  The bias
+// forces (velocities, bias accelerations, the leaf-to-root force pass) and the mass matrix (composite inertias, columns) do
+// not depend on each other, and each is a chain of tree sweeps that keeps a few lanes an environment busy: the first
+// wavefront takes the one, the second the other, side by side, each for all environments of the workgroup.  Then they meet,
+// and each factors and solves half of the environments, 2 G lanes each (of a workgroup's only one, the second wavefront
+// does, while the first carries the matrix and its factor to memory).  Every instruction of a sweep serves 64 / G
+// environments: the kernel is bound by the instructions it issues where environments outnumber the wavefronts, not by
+// memory.  Fewer lanes give the sweeps fewer links a pass; DynamicsLanes says where that pays.
+__host__ __device__ constexpr uint32_t DynamicsSlots(uint32_t lanes) { return lanes >= 64u ? kSweepLinks : lanes >= 32u ? 5u : lanes >= 16u ? 2u : 1u; }
+// three places past the links: what a root hangs from, what a floating root does, and one for lanes without a link
+constexpr uint32_t kGround = 0u, kBase = 1u, kNobody = 2u, kPlaces = 3u;
+// a link's record and its place in the children's list, and the sweeps' list with its length and steps past its end
+__host__ __device__ inline uint32_t DynamicsTreeWords(uint32_t nl, uint32_t sweep_passes) {
+    return (nl + kPlaces) * 2u + nl + (sweep_passes + 3u) * kSweepLinks + 1u;
+}
+// links a lane has in the pass over the mass columns, and whether the matrix may take the composite inertias' place: when
+// every link's inertia has been read by then
+__host__ __device__ constexpr uint32_t DynamicsLinksALane(uint32_t lanes) { return lanes >= 64u ? 2u : 1u; }
+__host__ __device__ inline uint32_t DynamicsMatrixWords(uint32_t nl, uint32_t n, uint32_t envs) {   // the inertias and the matrix
+    const uint32_t inertias = nl * 36u, matrix = n * (n | 1u), lanes = 64u / envs;
+    return nl <= lanes * DynamicsLinksALane(lanes) ? (inertias > matrix ? inertias : matrix) : inertias + matrix;
+}
+__host__ __device__ inline uint32_t DynamicsEnvWords(uint32_t nl, uint32_t n, uint32_t envs) {
+    const uint32_t words = (nl + kPlaces) * (18u + 5u * 6u) + nl + DynamicsMatrixWords(nl, n, envs) + 2u * n + 36u;
+    const uint32_t apart = 64u / envs;   // one place of the environments in different banks
+    return envs == 1u ? words : (words + 63u - apart) / 64u * 64u + apart;
 }
 
-// LDL^T of the matrix whose row `lane` is `row`: the strict lower triangle becomes L and the diagonal D (:269-335).  Entry
-// (i, j) loses (L_ik L_jk) D_k for k = 0, 1, ... with the three roundings of the serial loop (fused into one multiply-add an
-// entry the factor differs in its last place, which an environment that does not converge in its sweeps hands on: one of 256
-// driven humanoids then ends 2.5e-4 from the oracle's).  The products L_ik L_jk come four columns an instruction, columns
-// 4 Q .. 4 Q + 3 of lane's row at a time: v_mfma_f32_4x4x1 multiplies four values a block of four lanes with one a lane,
-// and its broadcast of block Q's four to all blocks (cbsz 4, abid Q) takes the multipliers' own register for them, where a
-// lane read and a product an entry went before.  What a lane computes above its diagonal is never read.
+// v of lane K of the L lanes an environment has
+template <int L, int K>
+__device__ __forceinline__ float group_value(float v) {
+    typedef float Vec4 __attribute__((ext_vector_type(4)));
+    if constexpr (L == 64) return lane_value(v, K);
+    else if constexpr (L == 16) return dpp_move<0x150 + K>(v);   // a row's lane K to the whole row
+    else return __builtin_amdgcn_mfma_f32_4x4x1f32(v, 1.0f, Vec4{}, 3, K / 4, 0)[K % 4];   // a block's four to eight blocks
+}
+// LDL^T of the matrix whose row `lane` is `row`, L lanes a matrix: the strict lower triangle becomes L and the diagonal D
+// (:269-335).  Entry (i, j) loses (L_ik L_jk) D_k for k = 0, 1, ... with the three roundings of the serial loop (fused into
+// one multiply-add an entry the factor differs in its last place, which an environment that does not converge in its sweeps
+// hands on: one of 256 driven humanoids then ends 2.5e-4 from the oracle's).  The products L_ik L_jk come four columns an
+// instruction, columns 4 Q .. 4 Q + 3 of lane's row at a time: v_mfma_f32_4x4x1 multiplies four values a block of four lanes
+// with one a lane, and its broadcast of block Q's four to the L / 4 blocks (cbsz, abid) takes the multipliers' own register
+// for them, where a lane read and a product an entry went before.  What a lane computes above its diagonal is never read.
 typedef float Vec4 __attribute__((ext_vector_type(4)));
-template <int Q, int K, int N>
+template <int L>
+constexpr int kBlocksLog = L == 64 ? 4 : L == 32 ? 3 : 2;
+template <int L, int Q, int K, int N>
 __device__ __forceinline__ void subtract_products(float lik, float diagonal, float (&row)[N]) {
     if constexpr (4 * Q < N) {
-        const Vec4 product = __builtin_amdgcn_mfma_f32_4x4x1f32(lik, lik, Vec4{}, 4, Q, 0);
+        const Vec4 product = __builtin_amdgcn_mfma_f32_4x4x1f32(lik, lik, Vec4{}, kBlocksLog<L>, Q, 0);
 #pragma unroll
         for (int t = 0; t < 4; ++t)
             if (4 * Q + t > K) row[4 * Q + t] -= product[t] * diagonal;
-        subtract_products<Q + 1, K>(lik, diagonal, row);
+        subtract_products<L, Q + 1, K>(lik, diagonal, row);
     }
 }
-template <int K, int N>
+template <int L, int K, int N>
 __device__ __forceinline__ void ldlt_pivots(uint32_t lane, float (&row)[N]) {
     if constexpr (K < N) {
-        const float diagonal = fmaxf(lane_value(row[K], K), 1.0e-6f);
-        const float lik = row[K] / diagonal;
+        const float diagonal = fmaxf(group_value<L, K>(row[K]), 1.0e-6f);
+        const float lik = div_by(row[K], make_recip(diagonal));   // the quotient to the bit, masses lying far inside its range
         row[K] = lane > uint32_t(K) ? lik : (lane == uint32_t(K) ? diagonal : row[K]);
-        subtract_products<(K + 1) / 4, K>(lik, diagonal, row);
-        ldlt_pivots<K + 1>(lane, row);
+        subtract_products<L, (K + 1) / 4, K>(lik, diagonal, row);
+        ldlt_pivots<L, K + 1>(lane, row);
     }
 }
+template <int L, int J, int N>
+__device__ __forceinline__ void forward_rows(uint32_t lane, uint32_t n, const float (&row)[N], float* x) {
+    if constexpr (J < N) {
+        const float solved = group_value<L, J>(*x);
+        if (lane > uint32_t(J) && lane < n) *x -= row[J] * solved;
+        forward_rows<L, J + 1>(lane, n, row, x);
+    }
+}
+template <int L, int I, int N>
+__device__ __forceinline__ void backward_columns(uint32_t lane, const float (&col)[N], float* x) {
+    if constexpr (I >= 0) {
+        const float value = group_value<L, I>(*x);
+        if (lane < uint32_t(I)) *x -= col[I] * value;
+        backward_columns<L, I - 1>(lane, col, x);
+    }
+}
+// A matrix of LDS to its stride x stride words of memory by a whole wavefront: all of it, or (kLower) the lower triangle of
+// a factor, as sixteen-byte words (kWide) where the rows start on them.  Rows and columns past n are zero, but for a factor's
+// diagonal.  Row and column of a lane's words step with it, a division by the stride a word costing more than the word.
+struct TilePlace {
+    uint32_t wide, row, word, rows_a_step, words_a_step;
+    __device__ __forceinline__ TilePlace(uint32_t wide_, uint32_t stride, uint32_t lane) : wide(wide_) {
+        const uint32_t words = stride / wide;
+        row = lane / words; word = lane - row * words;
+        rows_a_step = uint32_t(kWave) / words; words_a_step = uint32_t(kWave) - rows_a_step * words;
+    }
+};
+template <bool kLower, bool kWide>
+__device__ __forceinline__ void store_tile(const TilePlace& place, float* out, const float* A, uint32_t n, uint32_t ld, uint32_t stride, uint32_t lane) {
+    auto word = [&](uint32_t i, uint32_t j) {
+        if (kLower) return i < n ? A[i * ld + min(j, i)] : (i == j ? 1.0e-6f : 0.0f);
+        const float v = A[min(i, n - 1u) * ld + min(j, n - 1u)];
+        return i < n && j < n ? v : 0.0f;
+    };
+    const uint32_t wide = kWide ? place.wide : 1u, words = stride / wide;
+    uint32_t i = place.row, q = place.word;
+    for (uint32_t e = lane; e < stride * words; e += kWave) {
+        const uint32_t j = wide * q;
+        if (wide == 1u) {
+            if (!kLower || j <= i) out[e] = word(i, j);
+        } else if (!kLower || j + 3u <= i) {
+            reinterpret_cast<float4*>(out)[e] = float4{word(i, j), word(i, j + 1u), word(i, j + 2u), word(i, j + 3u)};
+        } else {
+            for (uint32_t t = 0u; j + t <= i; ++t) out[i * stride + j + t] = word(i, j + t);
+        }
+        i += place.rows_a_step; q += place.words_a_step;
+        if (q >= words) { q -= words; ++i; }
+    }
+}
+// A link's motion transform X = [[E, 0], [L, E]] as its two blocks, E then L (the products with the zeros add nothing).
+// X^T f, each entry summed in the order of the whole product
+__device__ __forceinline__ void push_force(const float* X, const float (&f)[6], float (&out)[6]) {
+#pragma unroll
+    for (int r = 0; r < 3; ++r) {
+        float upper = 0.0f, lower = 0.0f;
+#pragma unroll
+        for (int c = 0; c < 3; ++c) upper += X[3 * c + r] * f[c];
+#pragma unroll
+        for (int c = 0; c < 3; ++c) { upper += X[9 + 3 * c + r] * f[3 + c]; lower += X[3 * c + r] * f[3 + c]; }
+        out[r] = upper; out[3 + r] = lower;
+    }
+}
+// A row of X as a lane of the sweeps holds it: the words its first three terms take and those of the other three, which
+// an angular row does not have; row times x (six words), likewise
+struct TransformRow { float first[3], second[3]; };
+__device__ __forceinline__ TransformRow load_transform_row(const float* X, uint32_t row) {
+    const float* first = X + 3u * row, *second = X + 3u * (row < 3u ? row : row - 3u);   // L's rows follow E's
+    return TransformRow{{first[0], first[1], first[2]}, {second[0], second[1], second[2]}};
+}
+__device__ __forceinline__ float transform_row(const TransformRow& X, uint32_t row, const float (&x)[6]) {
+    float value = 0.0f;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) value += X.first[c] * x[c];
+    const float angular = value;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) value += X.second[c] * x[3 + c];
+    return row < 3u ? angular : value;
+}
+
+// A link's record in LDS: its parent's place (a root's is one past the links), joint type and first coordinate; the place of
+// its children in their list and their number.
+struct LinkRecord {
+    uint32_t low, high;
+    __device__ __forceinline__ uint32_t parent() const { return low & 0xFFFFu; }
+    __device__ __forceinline__ uint8_t type() const { return uint8_t(low >> 16u); }
+    __device__ __forceinline__ uint32_t dof() const { return low >> 24u; }
+    __device__ __forceinline__ uint32_t child_begin() const { return high & 0xFFFFu; }
+    __device__ __forceinline__ uint32_t children() const { return high >> 16u; }
+};
+__device__ __forceinline__ uint32_t times(uint32_t words, uint32_t link) { return __umul24(words, link); }
 
 // Compiled per padded DoF width N (a multiple of 4): the LDL^T factorisation and the solve keep one matrix row per
-// lane in registers, fully unrolled, and pass pivots and multipliers between lanes as scalar lane reads.
-// The tree sweeps run six lanes a link - a lane a row of the link's 6x6 products - and ten links a pass, a depth at a
+// lane in registers, fully unrolled, and hand pivots and multipliers round the environment's lanes.
+// The tree sweeps run six lanes a link - a lane a row of the link's 6x6 products - and up to ten links a pass, a depth at a
 // time from the cooked pass list (ModelView::sweep_links): a pass costs about a third of the instructions of a lane a
-// link carrying all six rows, and each row sums in the order the whole product does.
-template <int N>
+// link carrying all six rows, and each row sums in the order the whole product does.  A lone wavefront is bound by the chain
+// of a pass, and each dependent read of LDS on it is some 130 cycles: what a pass reads beside the values of the pass before -
+// the links, their records, their rows of X - is read a pass or two ahead, roots and lanes without a link have places of
+// their own so that no read stands under a condition, and the matrix takes the inertias' place (a pass of 64 arms 900 -> 400
+// cycles, the kernel 19.4 -> 16.9 us; 4096 humanoids 118 -> 98 us, 65536 1405 -> 1133 us, 8192 ropes 1633 -> 1031 us).
+template <int N, int G>
 __global__ void __launch_bounds__(2 * kWave) ArticulationDynamicsKernel(ModelView m, DataView d, ArticulationDynamicsParams p,
                                                                        uint32_t env_count) {
     extern __shared__ float lds[];
-    const uint32_t env = blockIdx.x, lane = threadIdx.x % kWave, nl = m.links_per_env, n = m.dof, stride = m.max_dof;
-    const bool forces = threadIdx.x < uint32_t(kWave);   // the first wavefront: bias forces; the second: mass matrix, factor, solve
-    if (env >= env_count) return;
-    float* xup = lds;
-    float* S = xup + nl * 36u;
-    float* vb = S + nl * 6u;
-    float* v = vb + nl * 6u;
-    float* ic = v + nl * 6u;          // composite inertias (second wavefront)
-    float* a = ic + nl * 36u;         // link accelerations: bias pass (first wavefront), and again the final pass (second)
-    float* pf = a + nl * 6u;          // bias forces (first wavefront)
-    float* A = pf + nl * 6u;          // n x (n + 1): mass matrix, then its factor (second wavefront)
-    float* vel = A + n * (n + 1u);
-    float* acc = vel + n;
-    float* tmp = acc + n;             // 36 floats of the inertia push, padded to 64
-    // the tree as the sweeps read it, a word a link each: parent, joint type, first coordinate, child range, children, rate
-    uint32_t* t_parent = reinterpret_cast<uint32_t*>(tmp + 64u);
-    uint32_t* t_type = t_parent + nl;
-    uint32_t* t_dof = t_type + nl;
-    uint32_t* t_child_begin = t_dof + nl;
-    uint32_t* t_child_end = t_child_begin + nl;
-    uint32_t* t_children = t_child_end + nl;
-    float* t_rate = reinterpret_cast<float*>(t_children + nl);
-    uint32_t* sweep = reinterpret_cast<uint32_t*>(t_rate + nl);   // sweep_passes x kSweepLinks links, kInvalid where a pass ends early
+    constexpr uint32_t kEnvs = kWave / G, kRowLanes = G < 32 ? 2u * G : 64u;
+    static_assert(N <= int(kRowLanes), "a lane a row");
+    const uint32_t wave = threadIdx.x / kWave, lane = threadIdx.x % kWave, nl = m.links_per_env, n = m.dof, stride = m.max_dof;
+    const bool forces = wave == 0u;
+    // the tree as the sweeps read it: a record a link, the children's list, and the sweeps' list, kSlots places a step, nobody's
+    // where a step has fewer links and in three steps past the end, with its number of steps
+    constexpr uint32_t kSlots = DynamicsSlots(G);
+    LinkRecord* records = reinterpret_cast<LinkRecord*>(lds);
+    uint32_t* t_children = reinterpret_cast<uint32_t*>(records + nl + kPlaces);
+    uint32_t* sweep_steps = t_children + nl;
+    uint32_t* sweep = sweep_steps + 1u;
     const uint32_t passes = m.sweep_passes;
-    const uint32_t ld = n + 1u;
-    const size_t lbase = size_t{env} * nl;
-    const float* q = d.q + lbase;
-    float* qd = d.qdot + lbase;
+    const uint32_t ld = n | 1u;
+    struct Words { float *xup, *S, *vb, *v, *ic, *a, *pf, *A, *vel, *acc, *tmp, *rate; };
+    auto words_of = [&](uint32_t index) {
+        float* base = lds + DynamicsTreeWords(nl, passes) + index * DynamicsEnvWords(nl, n, kEnvs);
+        Words w;
+        const uint32_t places = nl + kPlaces;
+        w.xup = base;                    // motion transforms, eighteen words a link
+        w.S = w.xup + places * 18u;
+        w.vb = w.S + places * 6u;
+        w.v = w.vb + places * 6u;
+        w.a = w.v + places * 6u;         // link accelerations: bias pass (first wavefront), and again the final pass
+        w.pf = w.a + places * 6u;        // bias forces (first wavefront)
+        w.ic = w.pf + places * 6u;       // composite inertias (second wavefront)
+        // n x ld: mass matrix, then its factor (second wavefront), in the inertias' place where they are read by then
+        w.A = nl <= uint32_t(G) * DynamicsLinksALane(G) ? w.ic : w.ic + nl * 36u;
+        w.vel = w.ic + DynamicsMatrixWords(nl, n, kEnvs);
+        w.acc = w.vel + n;
+        w.rate = w.acc + n;
+        w.tmp = w.rate + nl;         // 36 words of the inertia push
+        return w;
+    };
     const V3 gravity{p.gravity[0], p.gravity[1], p.gravity[2]};
-    const Q4 base_rot = load_xf(d.base_pose + size_t{env} * 7u).r;
-    const uint32_t slot = lane / 6u, srow = lane - 6u * slot;   // of the sweeps: lanes 60..63 sit them out
-    const uint32_t ri = srow % 3u, rj = (ri + 1u) % 3u, rk = (ri + 2u) % 3u;
-    auto link_of_pass = [&](uint32_t pass) { return lane < 6u * kSweepLinks ? sweep[pass * kSweepLinks + slot] : kInvalid; };
-    const V3 gravity_in_base = rotate_inverse(base_rot, gravity);
-    const float gravity_in_base_row = srow < 3u ? 0.0f : (srow == 3u ? gravity_in_base.x : srow == 4u ? gravity_in_base.y : gravity_in_base.z);
-
-    if (!forces) {   // what the mass matrix starts from and the sweeps' tables, while the first wavefront builds the joint transforms
-        for (uint32_t e = lane; e < nl * 36u; e += kWave) ic[e] = m.link_inertia[e];
-        for (uint32_t e = lane; e < n * ld; e += kWave) A[e] = 0.0f;
-        for (uint32_t l = lane; l < nl; l += kWave) {
-            t_parent[l] = m.parent_link[l]; t_type[l] = m.joint_type[l]; t_dof[l] = m.link_dof[l];
-            t_child_begin[l] = m.link_child_range[2u * l]; t_child_end[l] = m.link_child_range[2u * l + 1u];
-            t_children[l] = m.link_children[l]; t_rate[l] = qd[l];
-        }
-        for (uint32_t e = lane; e < passes * kSweepLinks; e += kWave) sweep[e] = m.sweep_links[e];
-    }
-    // link twists of the state enter LDS (a floating root's twist is state; the rest is rebuilt)
-    for (uint32_t e = lane; forces && e < nl * 6u; e += kWave) v[e] = d.link_velocity[lbase * 6u + e];
-    // joint transforms and motion subspaces (articulation.cu:318-332)
-    for (uint32_t l = lane; forces && l < nl; l += kWave) {
-        if (m.parent_link[l] == kInvalid && m.joint_type[l] == kFloatingBase) {
-            const float id[9] = {1, 0, 0, 0, 1, 0, 0, 0, 1};
-            store_motion_transform(id, V3{0.0f, 0.0f, 0.0f}, xup + 36u * l);
-#pragma unroll
-            for (int i = 0; i < 6; ++i) { S[6u * l + i] = 0.0f; vb[6u * l + i] = 0.0f; }
-            continue;
-        }
-        joint_transform(m, l, q[l], xup + 36u * l);
-        motion_subspace(m.joint_type[l], load3(m.joint_axis + 3u * l), S + 6u * l);
-    }
-    __syncthreads();
-    const bool floating_root = m.floating_root != 0u;
-    float row[N];   // the second wavefront's row of the mass matrix, then of its factor
-    if (forces) {
-        // velocities root to leaf (:334-363)
-        for (uint32_t pass = 0u; pass < passes; ++pass) {
-            const uint32_t l = link_of_pass(pass);
-            const bool moves = l != kInvalid && !(t_parent[l] == kInvalid && t_type[l] == kFloatingBase);   // a floating root's twist is state
-            if (moves) {
-                const uint32_t parent = t_parent[l];
-                const float* X = xup + 36u * l + 6u * srow;
-                float through = 0.0f;
-#pragma unroll
-                for (int c = 0; c < 6; ++c) through += X[c] * (parent != kInvalid ? v[6u * parent + c] : 0.0f);
-                v[6u * l + srow] = through + S[6u * l + srow] * t_rate[l];
-            }
+    // Step by step down the sweeps' list: `fetch` a link's constants one step ahead, `use` them with the values of the step
+    // before.  A lane without a link sweeps nobody's place, so that no step asks which lanes it is for.
+    const uint32_t nobody = nl + kNobody;
+    auto sweep_down = [&](uint32_t steps, uint32_t slot, auto&& fetch, auto&& use) {
+        const bool takes = slot < kSlots;
+        const uint32_t* list = sweep + (takes ? slot : 0u);
+        auto link_at = [&](uint32_t step) { const uint32_t l = list[step * kSlots]; return takes ? l : nobody; };
+        uint32_t here = link_at(0u), next = link_at(1u);
+        auto constants = fetch(here);
+#pragma unroll 1
+        for (uint32_t step = 0u; step < steps; ++step) {
+            const uint32_t after = link_at(step + 2u);
+            const auto ahead = fetch(next);
+            use(here, constants);
             wave_sync();
-            if (moves) {   // the link's twist crossed with its joint's own twist, row by row (motion_cross)
-                const float* vl = v + 6u * l, *s6 = S + 6u * l;
-                const float rate = t_rate[l];
+            here = next; next = after; constants = ahead;
+        }
+    };
+    // (where a lane's words of a matrix lie takes divisions: ahead of the first barrier they wait beside reads of memory)
+    const uint32_t aligned = uint32_t((reinterpret_cast<uintptr_t>(d.m) | reinterpret_cast<uintptr_t>(d.m_factor)) & 15u);
+    const TilePlace place(N > 16 && (stride & 3u) == 0u && aligned == 0u ? 4u : 1u, stride, lane);
+    {
+        // the tree phase: G lanes an environment; a group past the last environment repeats it and writes nothing
+        const uint32_t gl = lane % G, group = lane / G;
+        const bool there = blockIdx.x * kEnvs + group < env_count;
+        const uint32_t env = min(blockIdx.x * kEnvs + group, env_count - 1u);
+        const Words w = words_of(group);
+        const size_t lbase = size_t{env} * nl;
+        const float* q = d.q + lbase;
+        const float* qd = d.qdot + lbase;
+        const uint32_t slot = gl / 6u, srow = gl - 6u * slot;   // of the sweeps: lanes past the slots' sit them out
+        const uint32_t ri = srow % 3u, rj = (ri + 1u) % 3u, rk = (ri + 2u) % 3u;
+        if (!forces) {   // what the mass matrix starts from and the sweeps' tables, while the first wavefront builds the joint transforms
+            for (uint32_t e = gl; e < nl * 36u; e += G) w.ic[e] = m.link_inertia[e];
+            for (uint32_t l = gl; l < nl; l += G) w.rate[l] = qd[l];
+            for (uint32_t l = lane; l < nl; l += kWave) {
+                const uint32_t begin = m.link_child_range[2u * l];
+                const uint32_t parent = m.parent_link[l], type = m.joint_type[l];
+                const uint32_t hangs = parent != kInvalid ? parent : nl + (type == kFloatingBase ? kBase : kGround);
+                records[l] = LinkRecord{hangs | (type << 16u) | (m.link_dof[l] << 24u), (begin & 0xFFFFu) | ((m.link_child_range[2u * l + 1u] - begin) << 16u)};
+                t_children[l] = m.link_children[l];
+            }
+            if (lane < kPlaces) records[nl + lane] = LinkRecord{nobody | (kFixed << 16u), 0u};
+            if constexpr (G == 64) {
+                for (uint32_t e = lane; e < (passes + 3u) * kSweepLinks; e += kWave) sweep[e] = e < passes * kSweepLinks ? min(m.sweep_links[e], nobody) : nobody;
+                if (lane == 0u) *sweep_steps = passes;
+            } else {   // lane = pass: a pass of `count` links is as many steps as they fill
+                uint32_t links[kSweepLinks], count = 0u;
+#pragma unroll
+                for (uint32_t k = 0u; k < kSweepLinks; ++k) {
+                    links[k] = lane < passes ? m.sweep_links[lane * kSweepLinks + k] : kInvalid;
+                    count += links[k] != kInvalid ? 1u : 0u;
+                }
+                const uint32_t mine = (count + kSlots - 1u) / kSlots;
+                uint32_t through = mine;
+#pragma unroll
+                for (int o = 1; o < kWave; o <<= 1) {
+                    const uint32_t other = __shfl_up(through, o, kWave);
+                    if (int(lane) >= o) through += other;
+                }
+#pragma unroll
+                for (uint32_t k = 0u; k < kSweepLinks; ++k)
+                    if (k < mine * kSlots) sweep[(through - mine) * kSlots + k] = min(links[k], nobody);
+                const uint32_t all = __shfl(through, kWave - 1, kWave);
+                if (lane < 3u * kSlots) sweep[all * kSlots + lane] = nobody;
+                if (lane == 0u) *sweep_steps = all;
+            }
+        } else {
+            const V3 base_gravity = rotate_inverse(load_xf(d.base_pose + size_t{env} * 7u).r, gravity);
+            // what the roots hang from: at rest, and accelerating against gravity (in the base's own frame for a floating one)
+            if (gl < 6u) {
+                const uint32_t k = gl % 3u;
+                const float world = k == 0u ? gravity.x : k == 1u ? gravity.y : gravity.z, local = k == 0u ? base_gravity.x : k == 1u ? base_gravity.y : base_gravity.z;
+                w.v[6u * (nl + kGround) + gl] = 0.0f; w.v[6u * (nl + kBase) + gl] = 0.0f;
+                w.a[6u * (nl + kGround) + gl] = gl < 3u ? 0.0f : -world; w.a[6u * (nl + kBase) + gl] = gl < 3u ? 0.0f : -local;
+            }
+            // link twists of the state enter LDS (a floating root's twist is state; the rest is rebuilt)
+            for (uint32_t e = gl; e < nl * 6u; e += G) w.v[e] = d.link_velocity[lbase * 6u + e];
+            // joint transforms and motion subspaces (articulation.cu:318-332)
+            for (uint32_t l = gl; l < nl; l += G) {
+                float X[36];
+                if (m.parent_link[l] == kInvalid && m.joint_type[l] == kFloatingBase) {
+                    const float id[9] = {1, 0, 0, 0, 1, 0, 0, 0, 1};
+                    store_motion_transform(id, V3{0.0f, 0.0f, 0.0f}, X);
+#pragma unroll
+                    for (int i = 0; i < 6; ++i) { w.S[6u * l + i] = 0.0f; w.vb[6u * l + i] = 0.0f; }
+                } else {
+                    joint_transform(m, l, q[l], X);
+                    motion_subspace(m.joint_type[l], load3(m.joint_axis + 3u * l), w.S + 6u * l);
+                }
+#pragma unroll
+                for (int e = 0; e < 9; ++e) { w.xup[18u * l + e] = X[(e / 3) * 6 + e % 3]; w.xup[18u * l + 9u + e] = X[(e / 3 + 3) * 6 + e % 3]; }
+            }
+        }
+        __syncthreads();
+        const uint32_t steps = *sweep_steps;
+        if (forces) {
+            struct Constants { LinkRecord record; TransformRow X; float add; };
+            // velocities root to leaf (:334-363)
+            // (a floating root's twist is state: its joint moves nothing, and its own words are what is added)
+            sweep_down(steps, slot, [&](uint32_t l) {
+                const LinkRecord record = records[l];
+                const float state = w.v[times(6u, l) + srow], moved = w.S[times(6u, l) + srow] * w.rate[min(l, nl - 1u)];
+                return Constants{record, load_transform_row(w.xup + times(18u, l), srow), record.parent() == nl + kBase ? state : moved};
+            }, [&](uint32_t l, const Constants& k) {
+                float x[6];
+                const float* parent = w.v + times(6u, k.record.parent());
+#pragma unroll
+                for (int c = 0; c < 6; ++c) x[c] = parent[c];
+                w.v[times(6u, l) + srow] = transform_row(k.X, srow, x) + k.add;
+            });
+            // each link's twist crossed with its joint's own twist, row by row (motion_cross); a floating root has none
+            for (uint32_t l = slot; l < (slot < kSlots ? nl : 0u); l += kSlots) {
+                const float* vl = w.v + 6u * l, *s6 = w.S + 6u * l;
+                const float rate = w.rate[l];
                 const float first = vl[rj] * (s6[(srow < 3u ? 0u : 3u) + rk] * rate) - vl[rk] * (s6[(srow < 3u ? 0u : 3u) + rj] * rate);
                 const float second = vl[3u + rj] * (s6[rk] * rate) - vl[3u + rk] * (s6[rj] * rate);
-                vb[6u * l + srow] = srow < 3u ? first : first + second;
-            }
-        }
-        wave_sync();
-        // p = v x* (I v) - external wrench (:364-374, 279-295)
-        for (uint32_t l = lane; l < nl; l += kWave) {
-            float vl[6], iv[6], bf[6];
-#pragma unroll
-            for (int i = 0; i < 6; ++i) vl[i] = v[6u * l + i];
-            mat66_vec(m.link_inertia + 36u * l, vl, iv);
-            force_cross(vl, iv, bf);
-            if (p.apply_link_wrench != 0u) {
-                const float* wr = d.link_wrench + (lbase + l) * 6u;
-                if (wr[0] != 0.0f || wr[1] != 0.0f || wr[2] != 0.0f || wr[3] != 0.0f || wr[4] != 0.0f || wr[5] != 0.0f) {
-                    const Q4 rot = load_xf(d.link_pose + (lbase + l) * 7u).r;
-                    const V3 force = rotate_inverse(rot, V3{wr[0], wr[1], wr[2]});
-                    const V3 torque = rotate_inverse(rot, V3{wr[3], wr[4], wr[5]});
-                    const V3 moment = add3(torque, cross3(load_xf(m.link_inertial_frame + 7u * l).p, force));
-                    bf[0] -= moment.x; bf[1] -= moment.y; bf[2] -= moment.z; bf[3] -= force.x; bf[4] -= force.y; bf[5] -= force.z;
-                }
-            }
-#pragma unroll
-            for (int i = 0; i < 6; ++i) pf[6u * l + i] = bf[i];
-        }
-        wave_sync();
-        // bias accelerations with gravity as base acceleration (:526-547)
-        for (uint32_t pass = 0u; pass < passes; ++pass) {
-            const uint32_t l = link_of_pass(pass);
-            if (l != kInvalid) {
-                const uint32_t parent = t_parent[l];
-                float al;
-                if (parent == kInvalid && t_type[l] == kFloatingBase) al = srow < 3u ? 0.0f : -gravity_in_base_row;
-                else {
-                    const float* X = xup + 36u * l + 6u * srow;
-                    al = 0.0f;
-#pragma unroll
-                    for (int c = 0; c < 6; ++c) al += X[c] * (parent != kInvalid ? a[6u * parent + c] : (c < 3 ? 0.0f : (c == 3 ? -gravity.x : c == 4 ? -gravity.y : -gravity.z)));
-                }
-                a[6u * l + srow] = al + vb[6u * l + srow];
+                const bool state = records[l].parent() == nl + kBase;
+                w.vb[6u * l + srow] = state ? 0.0f : (srow < 3u ? first : first + second);
             }
             wave_sync();
-        }
-        // p += I a (:548-555)
-        for (uint32_t l = lane; l < nl; l += kWave) {
-            float al[6], f[6];
+            // p = v x* (I v) - external wrench (:364-374, 279-295)
+            for (uint32_t l = gl; l < nl; l += G) {
+                float vl[6], iv[6], bf[6];
 #pragma unroll
-            for (int i = 0; i < 6; ++i) al[i] = a[6u * l + i];
-            mat66_vec(m.link_inertia + 36u * l, al, f);
-#pragma unroll
-            for (int i = 0; i < 6; ++i) pf[6u * l + i] += f[i];
-        }
-        wave_sync();
-        // leaf to root, children in CSR order (:557-569): the passes backwards, a lane a row of every child's X^T p
-        for (uint32_t pass = passes; pass-- > 0u;) {
-            const uint32_t l = link_of_pass(pass);
-            if (l != kInvalid) {
-                float total = pf[6u * l + srow];
-                for (uint32_t i = t_child_begin[l]; i < t_child_end[l]; ++i) {
-                    const uint32_t child = t_children[i];
-                    const float* X = xup + 36u * child + srow, *pc = pf + 6u * child;
-                    float pushed = 0.0f;
-#pragma unroll
-                    for (int c = 0; c < 6; ++c) pushed += X[6 * c] * pc[c];
-                    total += pushed;
+                for (int i = 0; i < 6; ++i) vl[i] = w.v[6u * l + i];
+                mat66_vec(m.link_inertia + 36u * l, vl, iv);
+                force_cross(vl, iv, bf);
+                if (p.apply_link_wrench != 0u) {
+                    const float* wr = d.link_wrench + (lbase + l) * 6u;
+                    if (wr[0] != 0.0f || wr[1] != 0.0f || wr[2] != 0.0f || wr[3] != 0.0f || wr[4] != 0.0f || wr[5] != 0.0f) {
+                        const Q4 rot = load_xf(d.link_pose + (lbase + l) * 7u).r;
+                        const V3 force = rotate_inverse(rot, V3{wr[0], wr[1], wr[2]});
+                        const V3 torque = rotate_inverse(rot, V3{wr[3], wr[4], wr[5]});
+                        const V3 moment = add3(torque, cross3(load_xf(m.link_inertial_frame + 7u * l).p, force));
+                        bf[0] -= moment.x; bf[1] -= moment.y; bf[2] -= moment.z; bf[3] -= force.x; bf[4] -= force.y; bf[5] -= force.z;
+                    }
                 }
-                pf[6u * l + srow] = total;
+#pragma unroll
+                for (int i = 0; i < 6; ++i) w.pf[6u * l + i] = bf[i];
             }
             wave_sync();
-        }
-        // generalized bias and right-hand side, lane = DoF (:570-585)
-        float* bias = d.articulation_bias + size_t{env} * stride;
-        if (lane < stride) {
-            if (lane >= n) bias[lane] = 0.0f;
-            else {
-                const uint32_t link = m.dof_link[lane], component = m.dof_component[lane];
+            // bias accelerations with gravity as base acceleration (:526-547)
+            sweep_down(steps, slot, [&](uint32_t l) {
+                return Constants{records[l], load_transform_row(w.xup + times(18u, l), srow), w.vb[times(6u, l) + srow]};
+            }, [&](uint32_t l, const Constants& k) {
+                float x[6];
+                const float* parent = w.a + times(6u, k.record.parent());
+#pragma unroll
+                for (int c = 0; c < 6; ++c) x[c] = parent[c];
+                w.a[times(6u, l) + srow] = transform_row(k.X, srow, x) + k.add;
+            });
+            // p += I a (:548-555)
+            for (uint32_t l = gl; l < nl; l += G) {
+                float al[6], f[6];
+#pragma unroll
+                for (int i = 0; i < 6; ++i) al[i] = w.a[6u * l + i];
+                mat66_vec(m.link_inertia + 36u * l, al, f);
+#pragma unroll
+                for (int i = 0; i < 6; ++i) w.pf[6u * l + i] += f[i];
+            }
+            wave_sync();
+            // leaf to root, children in CSR order (:557-569): the passes backwards, a lane a row of every child's X^T p
+            {
+                const bool takes = slot < kSlots;
+                const uint32_t* list = sweep + (takes ? slot : 0u);
+                auto link_at = [&](uint32_t back) { const uint32_t l = list[(back < steps ? steps - 1u - back : steps) * kSlots]; return takes ? l : nobody; };
+                struct Child { float E[3], L[3]; };
+                auto child_of = [&](const LinkRecord& record) { return t_children[min(record.child_begin(), nl - 1u)]; };
+                auto push_of = [&](uint32_t child) {
+                    const float* E = w.xup + times(18u, child) + ri;
+                    return Child{{E[0], E[3], E[6]}, {E[9], E[12], E[15]}};
+                };
+                auto pushed = [&](uint32_t child, const Child& X) {
+                    const float* pc = w.pf + times(6u, child), *first = pc + (srow < 3u ? 0u : 3u);
+                    float value = 0.0f;
+#pragma unroll
+                    for (int c = 0; c < 3; ++c) value += X.E[c] * first[c];
+                    const float linear = value;
+#pragma unroll
+                    for (int c = 0; c < 3; ++c) value += X.L[c] * pc[3 + c];
+                    return srow < 3u ? value : linear;
+                };
+                // two steps ahead the record, one step ahead its first child's columns of X and its own force
+                uint32_t here = link_at(0u), next = link_at(1u), after = link_at(2u);
+                LinkRecord record = records[here], next_record = records[next];
+                uint32_t child = child_of(record), next_child = child_of(next_record);
+                Child X = push_of(child);
+                float own = w.pf[times(6u, here) + srow];
+#pragma unroll 1
+                for (uint32_t back = 0u; back < steps; ++back) {
+                    const uint32_t later = link_at(back + 3u);
+                    const LinkRecord after_record = records[after];
+                    const uint32_t after_child = child_of(after_record);
+                    const Child next_X = push_of(next_child);
+                    const float next_own = w.pf[times(6u, next) + srow];
+                    if (record.children() != 0u) {
+                        float total = own + pushed(child, X);
+                        for (uint32_t i = 1u; i < record.children(); ++i) {
+                            const uint32_t other = t_children[record.child_begin() + i];
+                            total += pushed(other, push_of(other));
+                        }
+                        w.pf[times(6u, here) + srow] = total;
+                    }
+                    wave_sync();
+                    here = next; next = after; after = later;
+                    record = next_record; next_record = after_record;
+                    child = next_child; next_child = after_child;
+                    X = next_X; own = next_own;
+                }
+            }
+            // generalized bias and right-hand side, lane = DoF (:570-585)
+            float* bias = d.articulation_bias + size_t{env} * stride;
+            for (uint32_t i = gl; i < stride; i += G) {
+                if (i >= n) { if (there) bias[i] = 0.0f; continue; }
+                const uint32_t link = m.dof_link[i], component = m.dof_component[i];
                 const bool scalar = component == kInvalid;
-                const float velocity = scalar ? qd[link] : v[6u * link + component];
-                float b = scalar ? dot6(S + 6u * link, pf + 6u * link) : pf[6u * link + component];
+                const float velocity = scalar ? qd[link] : w.v[6u * link + component];
+                float b = scalar ? dot6(w.S + 6u * link, w.pf + 6u * link) : w.pf[6u * link + component];
                 if (scalar) b += d.joint_gravity_force[lbase + link];   // zero unless uploaded
                 const float damping = scalar ? m.joint_damping[link] + (p.fold_drive_damping != 0u ? d.drive_dissipation[lbase + link] : 0.0f) : 0.0f;
                 const float spring = scalar ? m.joint_stiffness[link] * (q[link] - m.joint_spring_reference[link]) : 0.0f;
-                vel[lane] = velocity;
-                bias[lane] = b;
-                acc[lane] = (scalar ? d.tau[lbase + link] : 0.0f) - b - damping * velocity - spring;
+                w.vel[i] = velocity;
+                if (there) bias[i] = b;
+                w.acc[i] = (scalar ? d.tau[lbase + link] : 0.0f) - b - damping * velocity - spring;
             }
-        }
-        __syncthreads();   // the second wavefront has the mass matrix in LDS
-        // the dense mass tile reaches HBM once, in row-major runs (row and column of a lane's word step with it: a
-        // division by the stride a word costs more than the word)
-        float* M = d.m + size_t{env} * stride * stride;
-        const uint32_t rows_a_step = uint32_t(kWave) / stride, columns_a_step = uint32_t(kWave) % stride;
-        {
-            uint32_t i = lane / stride, j = lane % stride;
-            for (uint32_t e = lane; e < stride * stride; e += kWave) {
-                M[e] = i < n && j < n ? A[i * ld + j] : 0.0f;
-                i += rows_a_step; j += columns_a_step;
-                if (j >= stride) { j -= stride; ++i; }
-            }
-        }
-        __syncthreads();   // ... and may now overwrite it with the factor
-    } else {
-        // CRBA: composite inertias leaf to root; the push X^T Ic X runs entry-parallel on 36 lanes (articulation_mass.cuh:146-165)
-        // deepest parents first, parents of one depth in link order, a parent's children in list order: the cooked visiting
-        // list, sixty-four visits at a time - a lane reads one visit's child and parent, the visits take theirs as lane reads
-        for (uint32_t first = 0u; first < nl; first += kWave) {
-            uint32_t my_child = kInvalid, my_parent = 0u;
-            if (first + lane < nl) {
-                my_child = m.link_push_order[first + lane];
-                if (my_child != kInvalid) my_parent = m.parent_link[my_child];
-            }
-            for (uint32_t visit = 0u; visit < uint32_t(kWave); ++visit) {
-                const uint32_t child = uint32_t(__builtin_amdgcn_readlane(int(my_child), int(visit)));
-                if (child == kInvalid) break;
-                const uint32_t l = uint32_t(__builtin_amdgcn_readlane(int(my_parent), int(visit)));
-                const float* X = xup + 36u * child;
-                const float* C = ic + 36u * child;
-                const uint32_t entry_row = lane / 6u, entry_col = lane % 6u;
-                if (lane < 36u) {
-                    float value = 0.0f;
-#pragma unroll
-                    for (int k = 0; k < 6; ++k) value += C[entry_row * 6u + k] * X[k * 6u + entry_col];
-                    tmp[lane] = value;
+        } else {
+            // CRBA: composite inertias leaf to root, the push X^T Ic X (articulation_mass.cuh:146-165).
+            // deepest parents first, parents of one depth in link order, a parent's children in list order: the cooked visiting
+            // list, sixty-four visits at a time - a lane reads one visit's child and parent, the visits take theirs as lane reads.
+            // Thirty-six lanes take an entry of each product, or eighteen two that share their words (column c and c + 3 of a
+            // row, row r and r + 3 of a column), or six a row and a column each.
+            // (lanes past the entries repeat the last one: the same words, the same values)
+            const uint32_t push_lane = min(lane, 35u), push_row = push_lane / 6u, push_column = push_lane - 6u * push_row;
+            for (uint32_t first = 0u; first < nl; first += kWave) {
+                uint32_t my_child = kInvalid, my_parent = 0u;
+                if (first + lane < nl) {
+                    my_child = m.link_push_order[first + lane];
+                    if (my_child != kInvalid) my_parent = m.parent_link[my_child];
                 }
-                wave_sync();
-                if (lane < 36u) {
-                    float value = 0.0f;
+                for (uint32_t visit = 0u; visit < uint32_t(kWave); ++visit) {
+                    const uint32_t child = uint32_t(__builtin_amdgcn_readlane(int(my_child), int(visit)));
+                    if (child == kInvalid) break;
+                    const uint32_t l = uint32_t(__builtin_amdgcn_readlane(int(my_parent), int(visit)));
+                    const float* E = w.xup + times(18u, child), *C = w.ic + times(36u, child);
+                    float* into = w.ic + times(36u, l);
+                    if constexpr (G == 64) {
+                        // a lane an entry (a pair's second is three products of the six); what does not wait for the first product
+                        // is read ahead of it
+                        const uint32_t row = push_row, c = push_column, at = c < 3u ? c : c - 3u, out = row < 3u ? row : row - 3u;
+                        const float* other = E + (c < 3u ? 9u : 0u), *beside = E + (row < 3u ? 9u : 0u);
+                        float left[6], right[6], entry[6];
 #pragma unroll
-                    for (int k = 0; k < 6; ++k) value += X[k * 6u + entry_row] * tmp[k * 6u + entry_col];
-                    ic[36u * l + lane] += value;
+                        for (int k = 0; k < 6; ++k) left[k] = C[row * 6u + uint32_t(k)];
+#pragma unroll
+                        for (int k = 0; k < 3; ++k) {
+                            right[k] = E[3 * k + at]; right[3 + k] = other[3 * k + at];
+                            entry[k] = E[3 * k + out]; entry[3 + k] = beside[3 * k + out];
+                        }
+                        const float before = into[push_lane];
+                        float value = 0.0f;
+#pragma unroll
+                        for (int k = 0; k < 3; ++k) value += left[k] * right[k];
+                        value = c < 3u ? value : 0.0f;
+#pragma unroll
+                        for (int k = 3; k < 6; ++k) value += left[k] * right[k];
+                        w.tmp[push_lane] = value;
+                        wave_sync();
+                        value = 0.0f;
+#pragma unroll
+                        for (int k = 0; k < 3; ++k) value += entry[k] * w.tmp[k * 6 + c];
+                        value = row < 3u ? value : 0.0f;
+#pragma unroll
+                        for (int k = 3; k < 6; ++k) value += entry[k] * w.tmp[k * 6 + c];
+                        into[push_lane] = before + value;
+                    } else {
+                        constexpr int kPairs = G == 32 ? 1 : 3;   // a lane
+                        constexpr uint32_t kLanes = G == 32 ? 18u : 6u;
+                        const uint32_t row = G == 32 ? gl / 3u : gl, column = G == 32 ? gl % 3u : 0u;
+                        if (gl < kLanes) {
+#pragma unroll
+                            for (int t = 0; t < kPairs; ++t) {
+                                const uint32_t c = column + uint32_t(t);
+                                float left = 0.0f, right = 0.0f;
+#pragma unroll
+                                for (int k = 0; k < 3; ++k) left += C[row * 6u + k] * E[3 * k + c];
+#pragma unroll
+                                for (int k = 0; k < 3; ++k) {
+                                    left += C[row * 6u + 3u + k] * E[9 + 3 * k + c];
+                                    right += C[row * 6u + 3u + k] * E[3 * k + c];
+                                }
+                                w.tmp[row * 6u + c] = left; w.tmp[row * 6u + 3u + c] = right;
+                            }
+                        }
+                        wave_sync();
+                        const uint32_t out_row = G == 32 ? gl / 6u : 0u, out_column = G == 32 ? gl % 6u : gl;
+                        if (gl < kLanes) {
+#pragma unroll
+                            for (int t = 0; t < kPairs; ++t) {
+                                const uint32_t r = out_row + uint32_t(t);
+                                float upper = 0.0f, lower = 0.0f;
+#pragma unroll
+                                for (int k = 0; k < 3; ++k) upper += E[3 * k + r] * w.tmp[k * 6 + out_column];
+#pragma unroll
+                                for (int k = 0; k < 3; ++k) {
+                                    upper += E[9 + 3 * k + r] * w.tmp[(3 + k) * 6 + out_column];
+                                    lower += E[3 * k + r] * w.tmp[(3 + k) * 6 + out_column];
+                                }
+                                into[r * 6u + out_column] += upper; into[(r + 3u) * 6u + out_column] += lower;
+                            }
+                        }
+                    }
+                    wave_sync();
                 }
-                wave_sync();
             }
-        }
-        if (floating_root && lane < 36u) A[(lane / 6u) * ld + lane % 6u] = ic[lane];
-        wave_sync();
-        // mass columns: each jointed link pushes Ic S to the root (:183-252)
-        for (uint32_t l = lane; l < nl; l += kWave) {
-            if (joint_dof(uint8_t(t_type[l])) == 0u) continue;
-            if (l == 0u && floating_root) continue;
-            const uint32_t dof_i = t_dof[l];
-            float force[6], sl[6];
+            // mass columns: each jointed link pushes Ic S to the root (:183-252).  First every link's Ic S and its diagonal entry,
+            // and the root's own block, after which the matrix may take the inertias' place.
+            const bool floating_root = m.floating_root != 0u;
+            constexpr uint32_t kLinks = DynamicsLinksALane(G);
+            auto jointed = [&](uint32_t l) { return l < nl && joint_dof(records[l].type()) != 0u && !(l == 0u && floating_root); };
+            // (loops that stay loops, one copy of their code each: a lone wavefront waits on instructions it fetches once)
+#pragma unroll 1
+            for (uint32_t chunk = 0u; chunk < nl; chunk += kLinks * G) {   // past the first the matrix stands apart from the inertias
+                float start[kLinks][6], diagonals[kLinks];
+#pragma unroll 1
+                for (uint32_t o = 0u; o < kLinks; ++o) {
+                    const uint32_t l = chunk + o * G + gl;
+                    float force[6] = {}, diagonal = 0.0f;
+                    if (jointed(l)) {
+                        float sl[6];
 #pragma unroll
-            for (int i = 0; i < 6; ++i) sl[i] = S[6u * l + i];
-            mat66_vec(ic + 36u * l, sl, force);
-            float diagonal = dot6(sl, force);
-            diagonal += m.joint_armature[l];
-            if (p.fold_drive_damping != 0u) diagonal += p.dt * d.drive_dissipation[lbase + l];   // articulation_mass.cuh:206-208
-            A[dof_i * ld + dof_i] = diagonal;
-            uint32_t walk = l;
-            for (;;) {
-                const uint32_t parent = t_parent[walk];   // the walk reads the tree from LDS: a table load a hop would be its latency
-                if (parent == kInvalid) break;
-                float pushed[6];
-                mat66t_vec(xup + 36u * walk, force, pushed);
+                        for (int i = 0; i < 6; ++i) sl[i] = w.S[6u * l + i];
+                        mat66_vec(w.ic + 36u * l, sl, force);
+                        diagonal = dot6(sl, force);
+                        diagonal += m.joint_armature[l];
+                        if (p.fold_drive_damping != 0u) diagonal += p.dt * d.drive_dissipation[lbase + l];   // articulation_mass.cuh:206-208
+                    }
 #pragma unroll
-                for (int i = 0; i < 6; ++i) force[i] = pushed[i];
-                walk = parent;
-                if (joint_dof(uint8_t(t_type[walk])) == 0u) continue;
-                const uint32_t dof_j = t_dof[walk];
-                if (walk == 0u && floating_root) {
+                    for (uint32_t k = 0u; k < kLinks; ++k) {
+                        if (o != k) continue;
 #pragma unroll
-                    for (int b = 0; b < 6; ++b) { A[dof_i * ld + b] = force[b]; A[b * ld + dof_i] = force[b]; }
-                    continue;
+                        for (int i = 0; i < 6; ++i) start[k][i] = force[i];
+                        diagonals[k] = diagonal;
+                    }
+                    if (chunk + (o + 1u) * G >= nl) break;
                 }
-                const float entry = dot6(S + 6u * walk, force);
-                A[dof_i * ld + dof_j] = entry;
-                A[dof_j * ld + dof_i] = entry;
-            }
-        }
-        __syncthreads();   // the mass matrix stands in LDS: the first wavefront carries it to HBM while this one factors it
-        // LDL^T, right-looking, lane = row in registers; rows and columns n..N-1 are those of the identity
-        {
-            // (every word read whether or not the lane keeps it, from a place inside the matrix: a read under a condition
-            // compiles to a branch a word)
-            const uint32_t ll = local_lane(lane);
-            const uint32_t from = (ll < n ? ll : 0u) * ld;
+                if (chunk == 0u) {
+                    float root_block[(36 + G - 1) / G];
 #pragma unroll
-            for (int k = 0; k < N; ++k) {
-                const float word = A[from + (uint32_t(k) < n ? uint32_t(k) : 0u)];
-                row[k] = ll < n && uint32_t(k) < n ? word : (ll == uint32_t(k) ? 1.0f : 0.0f);
-            }
-        }
-        {
-            ldlt_pivots<0>(local_lane(lane), row);
-            __syncthreads();   // the first wavefront has read the mass matrix: its words take the factor
-            const uint32_t ll = local_lane(lane);
-            if (ll < n) {
+                    for (int o = 0; o < (36 + G - 1) / G; ++o) root_block[o] = w.ic[min(gl + uint32_t(o * G), 35u)];
+                    wave_sync();
+                    for (uint32_t e = gl; e < n * ld; e += G) w.A[e] = 0.0f;
+                    wave_sync();
+                    if (floating_root) {
 #pragma unroll
-                for (int k = 0; k < N; ++k)
-                    if (uint32_t(k) < n) A[ll * ld + k] = row[k];
+                        for (int o = 0; o < (36 + G - 1) / G; ++o) {
+                            const uint32_t e = gl + uint32_t(o * G);
+                            if (e < 36u) w.A[(e / 6u) * ld + e % 6u] = root_block[o];
+                        }
+                    }
+                    wave_sync();
+                }
+#pragma unroll 1
+                for (uint32_t o = 0u; o < kLinks; ++o) {
+                    const uint32_t l = chunk + o * G + gl;
+                    if (chunk + o * G >= nl) break;
+                    if (!jointed(l)) continue;
+                    float force[6], diagonal = diagonals[0];
+#pragma unroll
+                    for (int i = 0; i < 6; ++i) force[i] = start[0][i];
+                    if (kLinks > 1u && o != 0u) {
+#pragma unroll
+                        for (int i = 0; i < 6; ++i) force[i] = start[kLinks - 1u][i];
+                        diagonal = diagonals[kLinks - 1u];
+                    }
+                    // a hop ahead: the parent's record, its axis and its transform
+                    LinkRecord record = records[l];
+                    const uint32_t dof_i = record.dof();
+                    w.A[dof_i * ld + dof_i] = diagonal;
+                    float X[18];
+                    auto fetch_X = [&](uint32_t link) {
+#pragma unroll
+                        for (int e = 0; e < 18; ++e) X[e] = w.xup[times(18u, link) + e];
+                    };
+                    fetch_X(l);
+                    uint32_t parent = record.parent();
+                    record = records[parent];
+                    while (parent < nl) {
+                        float pushed[6], axis[6];
+#pragma unroll
+                        for (int i = 0; i < 6; ++i) axis[i] = w.S[times(6u, parent) + i];
+                        push_force(X, force, pushed);
+                        fetch_X(parent);
+                        const LinkRecord further = records[record.parent()];
+#pragma unroll
+                        for (int i = 0; i < 6; ++i) force[i] = pushed[i];
+                        const uint32_t dof_j = record.dof();
+                        if (parent == 0u && floating_root) {
+#pragma unroll
+                            for (int b = 0; b < 6; ++b) { w.A[dof_i * ld + b] = force[b]; w.A[b * ld + dof_i] = force[b]; }
+                        } else if (joint_dof(record.type()) != 0u) {
+                            const float entry = dot6(axis, force);
+                            w.A[dof_i * ld + dof_j] = entry;
+                            w.A[dof_j * ld + dof_i] = entry;
+                        }
+                        parent = record.parent();
+                        record = further;
+                    }
+                }
             }
         }
     }
-    __syncthreads();   // the factor stands in LDS, and the right-hand side (first wavefront) meets it (second)
-    if (forces) {
-        float* factor = d.m_factor + size_t{env} * stride * stride;
-        const uint32_t rows_a_step = uint32_t(kWave) / stride, columns_a_step = uint32_t(kWave) % stride;
-        uint32_t i = lane / stride, j = lane % stride;
-        for (uint32_t e = lane; e < stride * stride; e += kWave) {
-            if (j <= i) factor[e] = i < n ? A[i * ld + j] : (i == j ? 1.0e-6f : 0.0f);
-            i += rows_a_step; j += columns_a_step;
-            if (j >= stride) { j -= stride; ++i; }
+    __syncthreads();   // the mass matrix (second wavefront) and the right-hand side (first) stand in LDS
+    // The matrix phase: kRowLanes lanes an environment, half of the workgroup's environments a wavefront.  A wavefront carries
+    // its environments' matrices to memory before their words take the factors.
+    constexpr uint32_t kOwn = kEnvs == 1u ? 1u : kEnvs / 2u;
+    const uint32_t own_first = kEnvs == 1u ? 0u : wave * kOwn;
+    auto store_own = [&](auto lower, float* field) {
+        for (uint32_t e = 0u; e < kOwn; ++e) {
+            const uint32_t at = blockIdx.x * kEnvs + own_first + e;
+            if (at < env_count) store_tile<decltype(lower)::value, (N > 16)>(place, field + size_t{at} * stride * stride, words_of(own_first + e).A, n, ld, stride, lane);
         }
+    };
+    if (kEnvs > 1u || forces) store_own(std::false_type{}, d.m);
+    if (kEnvs == 1u && forces) {
+        __syncthreads();   // the other wavefront may now overwrite the matrix with the factor
+        __syncthreads();   // ... and has
+        store_own(std::true_type{}, d.m_factor);
         return;
     }
-    // solve L D L^T x = rhs: forward by rows, scale, backward by columns (:357-396)
-    float x = lane < n ? acc[lane] : 0.0f;
+    const uint32_t ml = lane % kRowLanes;
+    const bool there = blockIdx.x * kEnvs + own_first + lane / kRowLanes < env_count;
+    const uint32_t env = min(blockIdx.x * kEnvs + own_first + lane / kRowLanes, env_count - 1u);
+    const Words w = words_of(own_first + lane / kRowLanes);
+    float row[N];
     {
-        const uint32_t ll = local_lane(lane);
+        // rows and columns n..N-1 are those of the identity
+        // (every word read whether or not the lane keeps it, from a place inside the matrix: a read under a condition
+        // compiles to a branch a word)
+        const uint32_t ll = local_lane(ml);
+        const uint32_t from = (ll < n ? ll : 0u) * ld;
+#pragma unroll
+        for (int k = 0; k < N; ++k) {
+            const float word = w.A[from + (uint32_t(k) < n ? uint32_t(k) : 0u)];
+            row[k] = ll < n && uint32_t(k) < n ? word : (ll == uint32_t(k) ? 1.0f : 0.0f);
+        }
+    }
+    ldlt_pivots<int(kRowLanes), 0>(local_lane(ml), row);
+    if (kEnvs == 1u) __syncthreads(); else wave_sync();   // the matrix has been read: its words take the factor
+    {
+        const uint32_t ll = local_lane(ml);
+        if (ll < n) {
+#pragma unroll
+            for (int k = 0; k < N; ++k)
+                if (uint32_t(k) < n) w.A[ll * ld + k] = row[k];
+        }
+    }
+    if (kEnvs == 1u) __syncthreads(); else { wave_sync(); store_own(std::true_type{}, d.m_factor); }
+    // solve L D L^T x = rhs: forward by rows, scale, backward by columns (:357-396)
+    float x = ml < n ? w.acc[ml] : 0.0f;
+    {
+        const uint32_t ll = local_lane(ml);
         float col[N];
 #pragma unroll
         for (int i = 0; i < N; ++i) {
-            const float word = A[(uint32_t(i) < n ? uint32_t(i) : 0u) * ld + (ll < n ? ll : 0u)];
+            const float word = w.A[(uint32_t(i) < n ? uint32_t(i) : 0u) * ld + (ll < n ? ll : 0u)];
             col[i] = ll < uint32_t(i) && uint32_t(i) < n ? word : 0.0f;
         }
-#pragma unroll
-        for (int j = 0; j < N; ++j) {
-            const float solved = lane_value(x, j);
-            if (ll > uint32_t(j) && ll < n) x -= row[j] * solved;
-        }
-        if (ll < n) x = x / A[ll * ld + ll];
-#pragma unroll
-        for (int i = N - 1; i >= 0; --i) {
-            const float value = lane_value(x, i);
-            if (ll < uint32_t(i)) x -= col[i] * value;
-        }
+        forward_rows<int(kRowLanes), 0>(ll, n, row, &x);
+        if (ll < n) x = x / w.A[ll * ld + ll];
+        backward_columns<int(kRowLanes), N - 1>(ll, col, &x);
     }
-    if (lane < stride) d.articulation_qdd[size_t{env} * stride + lane] = lane < n ? x : 0.0f;
-    if (lane < n) acc[lane] = x;
+    if (there)
+        for (uint32_t i = ml; i < stride; i += kRowLanes) d.articulation_qdd[size_t{env} * stride + i] = i < n ? x : 0.0f;
+    if (ml < n) w.acc[ml] = x;
     wave_sync();
     // write back accelerations and the unconstrained velocity update (:597-615)
-    for (uint32_t l = lane; l < nl; l += kWave) {
-        const uint8_t type = m.joint_type[l];
+    const size_t lbase = size_t{env} * nl;
+    for (uint32_t l = ml; l < (there ? nl : 0u); l += kRowLanes) {
         float qdd = 0.0f;
-        if (joint_dof(type) == 1u) {
-            const uint32_t dof = m.link_dof[l];
-            qdd = acc[dof];
-            if (p.integrate_velocity != 0u) qd[l] = vel[dof] + p.dt * qdd;
+        if (joint_dof(records[l].type()) == 1u) {
+            const uint32_t dof = records[l].dof();
+            qdd = w.acc[dof];
+            if (p.integrate_velocity != 0u) d.qdot[lbase + l] = w.vel[dof] + p.dt * qdd;
         }
         d.qddot[lbase + l] = qdd;
         if (p.integrate_velocity != 0u) {
@@ -567,34 +891,36 @@ __global__ void __launch_bounds__(2 * kWave) ArticulationDynamicsKernel(ModelVie
             for (int i = 0; i < 6; ++i) wr[i] = 0.0f;
         }
     }
-    if (floating_root && p.integrate_velocity != 0u && lane < 6u) {
-        const uint32_t component = lane, i = component % 3u, j = (i + 1u) % 3u, k = (i + 2u) % 3u;
-        const float transport = component < 3u ? 0.0f : vel[j] * vel[3u + k] - vel[k] * vel[3u + j];
-        v[component] = vel[lane] + p.dt * (acc[lane] + transport);
+    if (m.floating_root != 0u && p.integrate_velocity != 0u && ml < 6u) {
+        const uint32_t component = ml, i = component % 3u, j = (i + 1u) % 3u, k = (i + 2u) % 3u;
+        const float transport = component < 3u ? 0.0f : w.vel[j] * w.vel[3u + k] - w.vel[k] * w.vel[3u + j];
+        w.v[component] = w.vel[ml] + p.dt * (w.acc[ml] + transport);
     }
     wave_sync();
     // final link accelerations (:617-644)
-    for (uint32_t pass = 0u; pass < passes; ++pass) {
-        const uint32_t l = link_of_pass(pass);
-        if (l != kInvalid) {
-            const uint32_t parent = t_parent[l], type = t_type[l];
-            float al;
-            if (type == kFloatingBase) al = srow < 3u ? acc[srow] : acc[srow] - gravity_in_base_row;
-            else {
-                const float* X = xup + 36u * l + 6u * srow;
-                al = 0.0f;
+    {
+        const uint32_t slot = ml / 6u, srow = ml - 6u * slot;
+        struct Constants { LinkRecord record; TransformRow X; float bias, axis, qdd; };
+        sweep_down(*sweep_steps, slot, [&](uint32_t l) {
+            const LinkRecord record = records[l];
+            const float solved = w.acc[min(record.type() == kFloatingBase ? srow : record.dof(), n - 1u)];
+            return Constants{record, load_transform_row(w.xup + times(18u, l), srow), w.vb[times(6u, l) + srow], w.S[times(6u, l) + srow],
+                             joint_dof(record.type()) == 1u || record.type() == kFloatingBase ? solved : 0.0f};
+        }, [&](uint32_t l, const Constants& k) {
+            float x6[6];
+            const float* parent = w.a + times(6u, k.record.parent());
 #pragma unroll
-                for (int c = 0; c < 6; ++c) al += X[c] * (parent != kInvalid ? a[6u * parent + c] : (c < 3 ? 0.0f : (c == 3 ? -gravity.x : c == 4 ? -gravity.y : -gravity.z)));
-                const float qdd = joint_dof(uint8_t(type)) == 1u ? acc[t_dof[l]] : 0.0f;
-                al += vb[6u * l + srow] + S[6u * l + srow] * qdd;
-            }
-            a[6u * l + srow] = al;
-        }
-        wave_sync();
+            for (int c = 0; c < 6; ++c) x6[c] = parent[c];
+            float al = transform_row(k.X, srow, x6);
+            // a floating root accelerates as solved, in the base's frame
+            if (k.record.type() == kFloatingBase) al = srow < 3u ? k.qdd : k.qdd + w.a[6u * (nl + kBase) + srow];
+            else al += k.bias + k.axis * k.qdd;
+            w.a[times(6u, l) + srow] = al;
+        });
     }
-    for (uint32_t e = lane; e < nl * 6u; e += kWave) {
-        d.link_velocity[lbase * 6u + e] = v[e];
-        d.link_acceleration[lbase * 6u + e] = a[e];
+    for (uint32_t e = ml; e < (there ? nl * 6u : 0u); e += kRowLanes) {
+        d.link_velocity[lbase * 6u + e] = w.v[e];
+        d.link_acceleration[lbase * 6u + e] = w.a[e];
     }
 }
 
@@ -752,11 +1078,28 @@ Status OpStepTail(const ModelView& m, const DataView& d, const IntegratePosition
 }
 
 using DynamicsKernel = void (*)(ModelView, DataView, ArticulationDynamicsParams, uint32_t);
-static const DynamicsKernel kDynamicsKernels[16] = {
-    ArticulationDynamicsKernel<4>, ArticulationDynamicsKernel<8>, ArticulationDynamicsKernel<12>, ArticulationDynamicsKernel<16>,
-    ArticulationDynamicsKernel<20>, ArticulationDynamicsKernel<24>, ArticulationDynamicsKernel<28>, ArticulationDynamicsKernel<32>,
-    ArticulationDynamicsKernel<36>, ArticulationDynamicsKernel<40>, ArticulationDynamicsKernel<44>, ArticulationDynamicsKernel<48>,
-    ArticulationDynamicsKernel<52>, ArticulationDynamicsKernel<56>, ArticulationDynamicsKernel<60>, ArticulationDynamicsKernel<64>};
+struct DynamicsEntry { uint32_t width, lanes; DynamicsKernel kernel; };
+// by lanes an environment, then by width: the first that holds an environment's links and coordinates is the one
+#define NKH_DYNAMICS(N, G) {N##u, G##u, ArticulationDynamicsKernel<N, G>}
+static const DynamicsEntry kDynamicsKernels[] = {
+    NKH_DYNAMICS(8, 8), NKH_DYNAMICS(16, 8),
+    NKH_DYNAMICS(12, 16), NKH_DYNAMICS(16, 16), NKH_DYNAMICS(20, 16), NKH_DYNAMICS(24, 16),
+    NKH_DYNAMICS(4, 64), NKH_DYNAMICS(8, 64), NKH_DYNAMICS(12, 64), NKH_DYNAMICS(16, 64), NKH_DYNAMICS(20, 64), NKH_DYNAMICS(24, 64),
+    NKH_DYNAMICS(28, 64), NKH_DYNAMICS(32, 64), NKH_DYNAMICS(36, 64), NKH_DYNAMICS(40, 64), NKH_DYNAMICS(44, 64), NKH_DYNAMICS(48, 64),
+    NKH_DYNAMICS(52, 64), NKH_DYNAMICS(56, 64), NKH_DYNAMICS(60, 64), NKH_DYNAMICS(64, 64)};
+#undef NKH_DYNAMICS
+// Lanes an environment: all 64 while every environment fits the chip at once (ten workgroups a compute unit and more), when
+// the one chain an environment has is what counts and fewer lanes lengthen its sweeps; past that as few as hold its links
+// and coordinates.  When the line was drawn a step of 20011 arms (8 links, 7 coordinates) took 187 us with 64 lanes, 115
+// with 16 and 104 with 8 (92 since the sweeps read ahead; 181 with two wavefronts an environment before); 4000 arms 72, 60
+// and 59 us, 3000 56 us any way, 1000 47, 52 and 53; 4096 quadrupeds (13 links, 18 coordinates) 504 us with 64 and 496 with
+// 16, 16384 1308 and 1264, 1000 380 and 390.  Thirty-two lanes gain nothing: two environments of 31 links and 36 coordinates
+// ask for the LDS that two workgroups with 64 lanes each do (65536 humanoids 8435 and 8490 us).
+constexpr uint32_t kDynamicsResident = 3072u;
+static uint32_t DynamicsLanes(uint32_t links, uint32_t dof, uint32_t envs) {
+    if (envs < kDynamicsResident) return 64u;
+    return links <= 8u && dof <= 16u ? 8u : links <= 16u && dof <= 24u ? 16u : 64u;
+}
 
 Status OpArticulationDynamics(const ModelView& m, const DataView& d, const void* params, hipStream_t stream) {
     const auto* p = static_cast<const ArticulationDynamicsParams*>(params);
@@ -764,10 +1107,14 @@ Status OpArticulationDynamics(const ModelView& m, const DataView& d, const void*
     if (p->articulation_count == 0u || p->total_link_count == 0u) return Status::Ok;
     if (m.dof > kMaxDof || m.dof == 0u || p->max_dof != m.max_dof ||
         p->total_link_count != p->articulation_count * m.links_per_env) return Status::InvalidArgument;
-    const size_t lds = size_t{DynamicsLdsFloats(m.links_per_env, m.dof, m.sweep_passes)} * sizeof(float);
-    if (lds > 160u * 1024u) return Status::InvalidArgument;
-    hipLaunchKernelGGL(kDynamicsKernels[((m.dof + 3u) & ~3u) / 4u - 1u], dim3(p->articulation_count), dim3(2 * kWave), lds, stream, m, d,
-                       *p, p->articulation_count);
+    // the links a world may have: those whose working state, with its transforms in full, fits a compute unit's LDS
+    if (size_t{m.links_per_env * 109u + m.dof * (m.dof + 3u) + 64u + m.sweep_passes * kSweepLinks} * sizeof(float) > 160u * 1024u) return Status::InvalidArgument;
+    const uint32_t lanes = DynamicsLanes(m.links_per_env, m.dof, p->articulation_count);
+    const DynamicsEntry* entry = kDynamicsKernels;
+    while (entry->lanes < lanes || entry->width < m.dof) ++entry;
+    const uint32_t envs = kWave / entry->lanes;
+    const size_t lds = size_t{DynamicsTreeWords(m.links_per_env, m.sweep_passes) + envs * DynamicsEnvWords(m.links_per_env, m.dof, envs)} * sizeof(float);
+    hipLaunchKernelGGL(entry->kernel, dim3((p->articulation_count + envs - 1u) / envs), dim3(2 * kWave), lds, stream, m, d, *p, p->articulation_count);
     return hipGetLastError() == hipSuccess ? Status::Ok : Status::Failed;
 }
 
@@ -997,8 +1344,8 @@ Status OpFkLinkVelocities(const ModelView& m, const DataView& d, const void* par
 }
 
 void InitArticulationKernels() {
-    for (DynamicsKernel kernel : kDynamicsKernels) {
-        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    for (const DynamicsEntry& entry : kDynamicsKernels) {
+        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(entry.kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
         (void)hipGetLastError();
     }
 }
