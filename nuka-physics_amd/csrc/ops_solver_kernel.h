@@ -325,6 +325,7 @@ struct Tile {
     bool mass_valid;
     bool elliptic;   // some head is under the elliptic cone: every response goes through the general functions
     bool units;      // some head is a unit head
+    bool near_heads; // no staged head's rows reach past the coordinates two tiles hold (add_heads_by_tiles)
     bool unit_lists; // every coordinate's unit heads fit its list
     uint32_t* unit_list;      // kUnitSlots x 64: lane's unit heads in head order, slot-major
     uint32_t unit_count;      // lane's own count
@@ -738,7 +739,8 @@ __device__ __forceinline__ void add_head(const Tile& c, uint32_t h, bool coordin
         if (((columns >> (4 * q)) & 0xFull) != 0ull) add_columns<N>(q, words, a0, a1, a2, hrow);
 }
 
-// The heads' curvature on the matrix cores, for blocks of at most 32 coordinates: H += sum over heads and axes of
+// The heads' curvature on the matrix cores, for blocks of at most 32 coordinates and those of 36 whose heads reach no further
+// than 32 (Tile::near_heads: a robot on two feet, whose arms come last): H += sum over heads and axes of
 // (C J)_r^T J_r, four heads a pass.  The wavefront's four groups of sixteen lanes take a head each; a lane holds, for
 // its head, the three entries of a coordinate of every sixteen (column = lane & 15 of tile t), forms the entries of C J
 // from them and hands both to v_mfma_f32_16x16x4, whose four products of one instruction are the four heads.  Three
@@ -758,7 +760,7 @@ __device__ __forceinline__ void add_head(const Tile& c, uint32_t h, bool coordin
 // a loop that added heads to register rows by broadcast reads of their Jacobian words, a head a pass with unit heads present
 // and two to four without: 1000 servo-driven quadrupeds, four steps, 2.58 -> 2.23 ms; 4096 walkers 1.06 -> 1.01 ms.
 template <int N>
-constexpr int kTileSpan = (N + 15) / 16;   // tiles of sixteen coordinates a side
+constexpr int kTileSpan = N > 32 ? 2 : (N + 15) / 16;   // tiles of sixteen coordinates a side
 __device__ __forceinline__ float lane_permute(int source, float v) {   // v of lane `source`, a byte address (4 x lane)
     return __int_as_float(__builtin_amdgcn_ds_bpermute(source, __float_as_int(v)));
 }
@@ -798,9 +800,9 @@ __device__ __forceinline__ double halves_sum(double v) {
 template <int N, bool kRows>
 __device__ __forceinline__ void add_heads_by_tiles(const Tile& c, uint64_t heads, const float (&mf)[3], const float (&mc)[6], const float (&mn)[3],
                                                    uint32_t my_first, float (&hrow)[N], TileSum& g, float& scale) {
-    static_assert(N <= 32, "two tiles a side at most");
-    constexpr int T = kTileSpan<N>;
+    constexpr int T = kTileSpan<N>, kReach = N < 16 * T ? N : 16 * T;   // the coordinates the tiles hold
     const uint32_t group = c.lane >> 4u, x = c.lane & 15u;
+    const bool reached = N <= 16 * T || c.lane < uint32_t(kReach);   // a wider block: its last rows are no tile's
     uint32_t column[T];
 #pragma unroll
     for (int t = 0; t < T; ++t) column[t] = min(uint32_t(16 * t) + x, uint32_t(N - 1));   // (entries past the width are never read back)
@@ -810,7 +812,7 @@ __device__ __forceinline__ void add_heads_by_tiles(const Tile& c, uint64_t heads
         for (int J = 0; J < T; ++J) {
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const auto entry = [&](int k) { return k < N ? hrow[k < N ? k : 0] : 0.0f; };
+                const auto entry = [&](int k) { return k < kReach ? hrow[k < kReach ? k : 0] : 0.0f; };
                 float low = halves_beside(entry(16 * J + r), entry(16 * J + 8 + r)), high = halves_beside(entry(16 * J + 4 + r), entry(16 * J + 12 + r));
                 swap_lane_rows(low, high);
                 tile[J][0][r] = low;
@@ -818,7 +820,7 @@ __device__ __forceinline__ void add_heads_by_tiles(const Tile& c, uint64_t heads
             }
         }
 #pragma unroll
-        for (int k = 0; k < N; ++k) hrow[k] = 0.0f;
+        for (int k = 0; k < kReach; ++k) hrow[k] = reached ? 0.0f : hrow[k];
     }
     double force[T] = {};
     float bound[T] = {};
@@ -870,20 +872,23 @@ __device__ __forceinline__ void add_heads_by_tiles(const Tile& c, uint64_t heads
     for (int J = 0; J < (kRows ? T : 0); ++J) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            if (16 * J + r >= N) continue;
+            if (16 * J + r >= kReach) continue;
             float low = tile[J][0][r], high = tile[J][T - 1][r];
             swap_lane_rows(low, high);
-            hrow[16 * J + r] += low;
-            if (16 * J + 4 + r < N) hrow[16 * J + 4 + r] += high;
-            if (16 * J + 8 + r < N) hrow[16 * J + 8 + r] += upper_half(low);
-            if (16 * J + 12 + r < N) hrow[16 * J + 12 + r] += upper_half(high);
+            const auto add = [&](int k, float v) { if (k < kReach) hrow[k < kReach ? k : 0] += reached ? v : 0.0f; };
+            add(16 * J + r, low);
+            add(16 * J + 4 + r, high);
+            add(16 * J + 8 + r, upper_half(low));
+            add(16 * J + 12 + r, upper_half(high));
         }
     }
     double force_low = force[0], force_high = force[T - 1];
     float bound_low = bound[0], bound_high = bound[T - 1];
     swap_lane_rows(force_low, force_high); swap_lane_rows(bound_low, bound_high);
-    g.value += halves_sum(force_low + force_high);
-    scale += halves_sum(bound_low + bound_high);
+    const double force_sum = halves_sum(force_low + force_high);
+    const float bound_sum = halves_sum(bound_low + bound_high);
+    g.value += reached ? force_sum : 0.0;
+    scale += reached ? bound_sum : 0.0f;
 }
 
 // A reduced block adds its heads to register rows instead, in an order of its own (below): its worlds are robots on two
@@ -1556,10 +1561,10 @@ __device__ __forceinline__ bool assemble_block(const Tile& c, const float (&mrow
         add_heads_force<N>(c, staged, mf, mn, lane < c.heads ? c.U(hRow, lane) : 0u, g, scale);
         add_heads_through_links<N>(c, mine, mc, hrow);
     } else {
-        if constexpr (N <= 32) {
-            if (staged != 0ull) {
+        if (N <= 32 || (N <= kTwoWaveWidth && c.near_heads)) {
+            if constexpr (N <= kTwoWaveWidth) if (staged != 0ull) {
                 const uint32_t my_first = c.U(hRow, lane < c.heads ? lane : 0u);
-                if constexpr (kFollow) {
+                if constexpr (kFollow && N <= 32) {
                     if (rows_kept) add_heads_by_groups<N, false>(c, staged, mf, mc, mn, my_first, hrow, g, scale);
                     else add_heads_by_groups<N, true>(c, staged, mf, mc, mn, my_first, hrow, g, scale);
                 } else {
@@ -2780,6 +2785,7 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
     // CopyTileRows (:836-869): the staged heads' rows, their loads in flight together
 
     bool stray = false;   // a reduced block: an entry past the block's coordinates
+    c.near_heads = true;
     for (uint32_t h0 = 0u; h0 < (c.from_links ? 0u : c.staged_end); h0 += 4u) {   // four heads at a time: 24 reads in flight
         uint32_t first[4];
         float value[4][3];
@@ -2811,6 +2817,7 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
                 stray = stray || (columns >> uint32_t(W)) != 0ull;
                 columns &= (uint64_t{1} << uint32_t(W)) - 1ull;
             }
+            c.near_heads = c.near_heads && (columns >> 32u) == 0ull;
             if (lane == 0u) { c.U(hColumnsLow, h) = uint32_t(columns); c.U(hColumnsHigh, h) = uint32_t(columns >> 32u); }
         }
     }
