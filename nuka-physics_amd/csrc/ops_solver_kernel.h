@@ -325,6 +325,7 @@ struct Tile {
     bool mass_valid;
     bool elliptic;   // some head is under the elliptic cone: every response goes through the general functions
     bool units;      // some head is a unit head
+    bool scalar_later;   // the heads past the first 64 are on one axis, and two a lane hold them
     bool near_heads; // no staged head's rows reach past the coordinates two tiles hold (add_heads_by_tiles)
     bool unit_lists; // every coordinate's unit heads fit its list
     uint32_t* unit_list;      // kUnitSlots x 64: lane's unit heads in head order, slot-major
@@ -1142,6 +1143,29 @@ __device__ __forceinline__ void plain_response(const PlainLine& p, float mx, flo
     r[3] = 0.0f; r[4] = 0.0f;
     r[5] = inside ? 0.0f : -cs * p.mu_y * p.mu_z * dy * dz;
 }
+// A head on one axis as numbers: what of a PlainLine such a head has.  Lanes keep their later heads (the second and third
+// sixty-four) so where all of those are on one axis, as joint rows are: a probe of 97 heads 3.7 k cycles with the later
+// ones' fields read and their general response taken each time, and a step of 4096 servo-driven humanoids, whose longest
+// environment makes 340 probes, 2002 -> 1832 us with it and with the row steps below (row_steps).
+struct ScalarLine { float k, k_bounded, dual_part, lower, upper, res, move, step; };
+constexpr uint32_t kLaterHeads = 2u;   // a lane
+__device__ __forceinline__ ScalarLine scalar_line(const Tile& c, uint32_t h) {
+    const uint32_t at = min(h, c.heads - 1u);   // (read whether or not there is such a head)
+    const float rho = c.F(hRho, at), dual = c.F(hDual, at), compliance = c.F(hCompliance, at), lower = c.F(hLower, at), upper = c.F(hUpper, at);
+    const float k = c.F(hResidualScale, at), scaled = c.F(hDualScale, at) * dual, res = c.F(hRes, at), move = c.F(hMove, at), step = c.F(hStep, at);
+    const bool live = h < c.heads && c.U(hOwned, at) != 0u && !(rho <= 0.0f);
+    ScalarLine s{};
+    s.k = live ? k : 0.0f; s.k_bounded = live && lower < upper ? k : 0.0f;
+    s.dual_part = live ? scaled : 0.0f; s.lower = live ? lower : 0.0f; s.upper = live ? upper : 0.0f;
+    s.res = live ? res : 0.0f; s.move = live ? move : 0.0f; s.step = live ? step : 0.0f;
+    if (live && !(rho == rho && dual == dual && compliance == compliance && lower == lower && upper == upper)) s.dual_part = nanf("");
+    return s;
+}
+__device__ __forceinline__ void scalar_line_response(const ScalarLine& s, float move, float* f, float* r) {
+    const float x = fmaf(s.k, s.res - move, s.dual_part);
+    *f = x < s.lower ? s.lower : (x > s.upper ? s.upper : x);
+    *r = x >= s.lower && x <= s.upper ? s.k_bounded : 0.0f;
+}
 // The constants of lane's own head for one block descent.  With at most sixteen heads the four rows of sixteen lanes
 // hold copies of the heads (lane & 15), which the line search uses to evaluate several points of a line in one pass;
 // the block assembly then takes the copies of the first row only.  `move` and `step` change with every Newton step
@@ -1488,7 +1512,16 @@ __device__ __forceinline__ bool assemble_block(const Tile& c, const float (&mrow
     // kept (in the lane of a head below 64, in the fields beyond), and while none differs the factor of the last
     // factorisation still stands.
     uint32_t differs = 0u;
-    for (uint32_t h = lane + kWave; h < c.heads; h += kWave) {
+    for (uint32_t h = lane + kWave; c.scalar_later && h < c.heads; h += kWave) {
+        const ScalarLine s = scalar_line(c, h);
+        float f, cv;
+        scalar_line_response(s, s.move, &f, &cv);
+        const float noise = fabsf(f) + cv * (fabsf(s.res) + fabsf(s.move));
+        differs |= bits(c.F(hC, h)) ^ bits(cv);
+        c.F(hF, h) = f; c.F(hNoise, h) = noise; c.F(hC, h) = cv;
+        c.U(hContrib, h) = ((bits(f) | bits(cv) | bits(noise)) << 1u) != 0u ? 1u : 0u;
+    }
+    for (uint32_t h = lane + kWave; !c.scalar_later && h < c.heads; h += kWave) {
         float f[3], cv[6], noise[3];
         const bool contributes = head_terms(c, h, f, cv, noise);
 #pragma unroll
@@ -1768,18 +1801,18 @@ __device__ __forceinline__ void row_steps(const Tile& c, float d) {
             return;
         }
     }
-    for (uint32_t h = c.lane; h < c.heads; h += kWave) {
-        if (c.U(hOwned, h) == 0u) continue;
-        const uint32_t unit = c.U(hUnit, h);
-        if (unit != kInvalid) {   // :2028-2032
-            c.F(hStep, h) = c.F(hUnitValue, h) * dvec[unit]; c.F(hStep + 1, h) = 0.0f; c.F(hStep + 2, h) = 0.0f;
-            continue;
+    // a lane a row of the staged heads (a head on one axis has zeros in its other rows), then a lane a unit head, which all
+    // come after them.  (A lane a head, its three rows in turn, held the unit heads up behind a dozen contacts.)
+    for (uint32_t r = c.lane; r < 3u * c.staged_end; r += kWave) {
+        const uint32_t h = r / 3u, axis = r - 3u * h, first = c.U(hRow, h);
+        if (first == kInvalid || c.U(hOwned, h) == 0u) continue;
+        c.fields[axis == 0u ? c.at(hStep, h) : c.at(hStep + 1, h) + axis - 1u] = row_dot_fma<N>(c.jac + (first + axis) * uint32_t(N), dvec);
+    }
+    if (c.units) {
+        for (uint32_t h = c.lane; h < c.heads; h += kWave) {
+            const uint32_t unit = c.U(hUnit, h);
+            if (c.U(hOwned, h) != 0u && unit != kInvalid) c.F(hStep, h) = c.F(hUnitValue, h) * dvec[unit];   // :2028-2032
         }
-        const uint32_t axes = c.U(hAxes, h);
-        const float* j = c.jac + c.U(hRow, h) * uint32_t(N);
-        c.F(hStep, h) = row_dot_fma<N>(j, dvec);
-        c.F(hStep + 1, h) = axes > 1u ? row_dot_fma<N>(j + N, dvec) : 0.0f;
-        c.F(hStep + 2, h) = axes > 2u ? row_dot_fma<N>(j + 2 * N, dvec) : 0.0f;
     }
     __syncthreads();
 }
@@ -1795,12 +1828,13 @@ __device__ __forceinline__ void plain_line_terms(const PlainLine& p, float alpha
     row_magnitude += fabsf(f[0] * sx) + fabsf(f[1] * sy) + fabsf(f[2] * sz) + line_noise(r, p.res[0], p.res[1], p.res[2], mx, my, mz, sx, sy, sz);
     row_curvature += r[0] * sx * sx + r[1] * sy * sy + r[2] * sz * sz + 2.0f * r[5] * sy * sz;
 }
-// The line search runs in one of three modes, the same for every probe of a solve: general (the block has more heads
-// than lanes, or some head is under the elliptic cone), plain with the terms in the first sixteen lanes (narrow), plain
-// over the whole wavefront.  The mode is a template argument so that the probes carry no branch on it.
-enum LineMode : int { kLineGeneral = 0, kLineWide = 1, kLineNarrow = 2 };
+// The line search runs in one of four modes, the same for every probe of a solve: general (some head is under the elliptic
+// cone, or later heads need more than a number a field), plain with the terms in the first sixteen lanes (narrow), plain
+// over the whole wavefront, plain with the heads past the first 64 as numbers beside it (later).  The mode is a template
+// argument so that the probes carry no branch on it.
+enum LineMode : int { kLineGeneral = 0, kLineWide = 1, kLineNarrow = 2, kLineLater = 3 };
 template <LineMode kMode>
-__device__ __forceinline__ void line_derivatives(const Tile& c, const HeadLine& mine, const PlainLine& plain, float alpha,
+__device__ __forceinline__ void line_derivatives(const Tile& c, const HeadLine& mine, const PlainLine& plain, const ScalarLine (&later)[kLaterHeads], float alpha,
                                  float inertial_slope, float inertial_curvature, float* slope, float* curvature, float* magnitude) {
     PROF_COUNT(c, 1);
     c.work += 1u;
@@ -1814,6 +1848,19 @@ __device__ __forceinline__ void line_derivatives(const Tile& c, const HeadLine& 
         }
     } else {
         plain_line_terms(plain, alpha, row_slope, row_curvature, row_magnitude);
+        if constexpr (kMode == kLineLater) {
+#pragma unroll
+            for (uint32_t e = 0u; e < kLaterHeads; ++e) {
+                if (c.heads <= kWave * (e + 1u)) break;
+                const ScalarLine& s = later[e];
+                float f, r;
+                const float move = fmaf(alpha, s.step, s.move);
+                scalar_line_response(s, move, &f, &r);
+                tile_add_product(row_slope, f, s.step);
+                row_magnitude += fabsf(f * s.step) + r * (fabsf(s.res) + fabsf(move)) * fabsf(s.step);
+                row_curvature += r * s.step * s.step;
+            }
+        }
     }
     PROF_BEGIN(c, 25);
     TileSum total{-row_slope.value};
@@ -1871,6 +1918,12 @@ __device__ __forceinline__ float search_line_in(const Tile& c, PlainLine& plain,
     constexpr bool kPaired = kMode == kLineNarrow;
     float slope = 0.0f, curvature = 0.0f, magnitude = 0.0f;
     HeadLine mine{};
+    ScalarLine later[kLaterHeads] = {};
+    if constexpr (kMode == kLineLater) {
+#pragma unroll
+        for (uint32_t e = 0u; e < kLaterHeads; ++e)
+            if (c.heads > kWave * (e + 1u)) later[e] = scalar_line(c, c.lane + kWave * (e + 1u));
+    }
     if constexpr (kMode == kLineGeneral) mine = load_head_line(c, c.lane);
     else if constexpr (kKept) refresh_steps(c, plain);
     else plain = own_line(c);
@@ -1905,18 +1958,19 @@ __device__ __forceinline__ float search_line_in(const Tile& c, PlainLine& plain,
         if (turn(&answer)) return answer;
         step = 1u;
     } else {
-        line_derivatives<kMode>(c, mine, plain, 0.0f, inertial_slope, inertial_curvature, &slope, &curvature, &magnitude);
+        line_derivatives<kMode>(c, mine, plain, later, 0.0f, inertial_slope, inertial_curvature, &slope, &curvature, &magnitude);
         initial = slope;
         if (!(initial < 0.0f)) return 0.0f;
     }
     for (; step < kLineSearchSteps; ++step) {
-        line_derivatives<kMode>(c, mine, plain, alpha, inertial_slope, inertial_curvature, &slope, &curvature, &magnitude);
+        line_derivatives<kMode>(c, mine, plain, later, alpha, inertial_slope, inertial_curvature, &slope, &curvature, &magnitude);
         if (turn(&answer)) return answer;
     }
     return low;
 }
 template <bool kKept>
 __device__ __forceinline__ float search_line(const Tile& c, PlainLine& line, float inertial_slope, float inertial_curvature) {
+    if (c.scalar_later) return search_line_in<kLineLater, kKept>(c, line, inertial_slope, inertial_curvature);
     if (c.heads > uint32_t(kWave) || c.elliptic) return search_line_in<kLineGeneral, kKept>(c, line, inertial_slope, inertial_curvature);
     if (c.heads <= 16u) return search_line_in<kLineNarrow, kKept>(c, line, inertial_slope, inertial_curvature);
     return search_line_in<kLineWide, kKept>(c, line, inertial_slope, inertial_curvature);
@@ -2513,7 +2567,7 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
     Tile c;
     c.env = env; c.lane = lane; c.n = kReduced ? uint32_t(K) : n; c.n_all = n; c.ldj = uint32_t(W); c.cap = cap; c.narrow = staged_cap; c.heads = 0u; c.iteration = 0u;
     c.tolerance = p.velocity_tolerance; c.failed = false; c.momentum = 0.0f; c.residual = 0.0f;
-    c.mass_inverse = 0.0f; c.mass_valid = false; c.work = 0u; c.units = false; c.elliptic = false;
+    c.scalar_later = false; c.near_heads = false; c.mass_inverse = 0.0f; c.mass_valid = false; c.work = 0u; c.units = false; c.elliptic = false;
     c.factor_current = false; c.rows_current = false; c.factor_root = 1.0f;
     for (float& entry : c.curvature) entry = 0.0f;
 #ifdef NKH_SOLVER_PROFILE
@@ -3098,6 +3152,9 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
     }
     c.elliptic = !kContactsOnly && __any(any_elliptic);
     __syncthreads();
+    bool later_axes = false;   // a later head on more axes than one
+    for (uint32_t h = lane + kWave; h < heads; h += kWave) later_axes = later_axes || c.U(hAxes, h) != 1u;
+    c.scalar_later = !kContactsOnly && !c.elliptic && heads > uint32_t(kWave) && heads <= uint32_t(kWave) * (kLaterHeads + 1u) && !__any(later_axes);
     PROF_END(c, 19);
     PROF_BEGIN(c, 20);
     // the one factorisation of the mass matrix
