@@ -330,6 +330,7 @@ struct Tile {
     bool unit_lists; // every coordinate's unit heads fit its list
     uint32_t* unit_list;      // kUnitSlots x 64: lane's unit heads in head order, slot-major
     uint32_t unit_count;      // lane's own count
+    uint32_t unit_most;       // the largest
     uint32_t staged_end;      // one past the last staged head
     uint32_t individual_end;  // one past the last head whose inertial response is computed for itself
     float momentum, residual;
@@ -1170,10 +1171,8 @@ __device__ __forceinline__ void scalar_line_response(const ScalarLine& s, float 
 // hold copies of the heads (lane & 15), which the line search uses to evaluate several points of a line in one pass;
 // the block assembly then takes the copies of the first row only.  `move` and `step` change with every Newton step
 // and are read again where they are used.
-// Widths whose register rows leave room keep the constants in registers over the whole block descent; the others
-// (28 to 36, at two waves a SIMD) compute them again at each use, which costs less than the spills would.
-template <int N>
-constexpr bool kKeepLine = N <= 24 || N > kTwoWaveWidth;
+// The constants stay in registers over the whole block descent (while the factor's panels went through registers of their
+// own, widths of 28 to 36 had no room for them and computed them again at each use).
 __device__ __forceinline__ PlainLine own_line(const Tile& c) {
     return plain_line(load_head_line(c, c.heads <= 16u ? (c.lane & 15u) : c.lane));
 }
@@ -1495,8 +1494,7 @@ __device__ __forceinline__ bool assemble_block(const Tile& c, const float (&mrow
     // lane's own head (the first 64 heads) from its constants, without a branch; a lane without an owned head gets zeros
     float mf[3], mc[6], mn[3];
     {
-        if constexpr (kKeepLine<N>) refresh_moves(c, own);
-        else own = own_line(c);
+        refresh_moves(c, own);
         plain_response(own, own.move[0], own.move[1], own.move[2], mf, mc);
 #pragma unroll
         for (int k = 0; k < 3; ++k) mn[k] = fabsf(mf[k]) + mc[k] * (fabsf(own.res[k]) + fabsf(own.move[k]));
@@ -1629,21 +1627,36 @@ __device__ __forceinline__ bool assemble_block(const Tile& c, const float (&mrow
     if (c.units) {
         // a unit head - a row on one coordinate - adds to that coordinate's diagonal and force only: lane = coordinate walks
         // its own short list, or, when some coordinate's list overflowed, the wave walks every unit head in turn
+        // (the list and then its heads' words read whether or not the lane has so many, all in flight together: a head that does
+        // not contribute holds zeros)
         float diagonal = 0.0f;
-        auto add_unit = [&](uint32_t h) {
-            const float v = c.F(hUnitValue, h);
-            diagonal += v * c.F(hC, h) * v;
-            tile_add_product(g, v, c.F(hF, h));
-            scale += fabsf(v) * c.F(hNoise, h);
+        auto add_unit = [&](float v, float curvature, float force, float noise) {
+            diagonal += v * curvature * v;
+            tile_add_product(g, v, force);
+            scale += fabsf(v) * noise;
         };
         if (c.unit_lists) {
-            for (uint32_t k = 0u; k < c.unit_count; ++k) {
-                const uint32_t h = c.unit_list[k * uint32_t(kWave) + lane];
-                if (c.U(hContrib, h) != 0u) add_unit(h);
+            uint32_t h[kUnitSlots];
+            float v[kUnitSlots], words[kUnitSlots][3];
+#pragma unroll
+            for (uint32_t k = 0u; k < kUnitSlots; ++k) {
+                const uint32_t listed = c.unit_list[k * uint32_t(kWave) + lane];
+                h[k] = k < c.unit_count ? listed : 0u;
+            }
+#pragma unroll
+            for (uint32_t k = 0u; k < kUnitSlots; ++k) {
+                if (k >= c.unit_most) break;
+                v[k] = c.F(hUnitValue, h[k]); words[k][0] = c.F(hC, h[k]); words[k][1] = c.F(hF, h[k]); words[k][2] = c.F(hNoise, h[k]);
+            }
+#pragma unroll
+            for (uint32_t k = 0u; k < kUnitSlots; ++k) {
+                if (k >= c.unit_most) break;
+                const bool on = k < c.unit_count;
+                add_unit(on ? v[k] : 0.0f, on ? words[k][0] : 0.0f, on ? words[k][1] : 0.0f, on ? words[k][2] : 0.0f);
             }
         } else {
             for (uint32_t h = 0u; h < c.heads; ++h)
-                if (c.U(hContrib, h) != 0u && c.U(hUnit, h) == lane) add_unit(h);
+                if (c.U(hContrib, h) != 0u && c.U(hUnit, h) == lane) add_unit(c.F(hUnitValue, h), c.F(hC, h), c.F(hF, h), c.F(hNoise, h));
         }
         if (!rows_kept) {
 #pragma unroll
@@ -1913,7 +1926,7 @@ __device__ __forceinline__ void line_derivatives_pair(const Tile& c, const Plain
 }
 
 // SearchTileLine (:2089-2125)
-template <LineMode kMode, bool kKept>
+template <LineMode kMode>
 __device__ __forceinline__ float search_line_in(const Tile& c, PlainLine& plain, float inertial_slope, float inertial_curvature) {
     constexpr bool kPaired = kMode == kLineNarrow;
     float slope = 0.0f, curvature = 0.0f, magnitude = 0.0f;
@@ -1925,8 +1938,7 @@ __device__ __forceinline__ float search_line_in(const Tile& c, PlainLine& plain,
             if (c.heads > kWave * (e + 1u)) later[e] = scalar_line(c, c.lane + kWave * (e + 1u));
     }
     if constexpr (kMode == kLineGeneral) mine = load_head_line(c, c.lane);
-    else if constexpr (kKept) refresh_steps(c, plain);
-    else plain = own_line(c);
+    else refresh_steps(c, plain);
     float low = 0.0f, high = 0.0f, alpha = 1.0f;
     bool bounded = false;
     float initial;
@@ -1968,12 +1980,11 @@ __device__ __forceinline__ float search_line_in(const Tile& c, PlainLine& plain,
     }
     return low;
 }
-template <bool kKept>
 __device__ __forceinline__ float search_line(const Tile& c, PlainLine& line, float inertial_slope, float inertial_curvature) {
-    if (c.scalar_later) return search_line_in<kLineLater, kKept>(c, line, inertial_slope, inertial_curvature);
-    if (c.heads > uint32_t(kWave) || c.elliptic) return search_line_in<kLineGeneral, kKept>(c, line, inertial_slope, inertial_curvature);
-    if (c.heads <= 16u) return search_line_in<kLineNarrow, kKept>(c, line, inertial_slope, inertial_curvature);
-    return search_line_in<kLineWide, kKept>(c, line, inertial_slope, inertial_curvature);
+    if (c.scalar_later) return search_line_in<kLineLater>(c, line, inertial_slope, inertial_curvature);
+    if (c.heads > uint32_t(kWave) || c.elliptic) return search_line_in<kLineGeneral>(c, line, inertial_slope, inertial_curvature);
+    if (c.heads <= 16u) return search_line_in<kLineNarrow>(c, line, inertial_slope, inertial_curvature);
+    return search_line_in<kLineWide>(c, line, inertial_slope, inertial_curvature);
 }
 
 __device__ __forceinline__ void apply_moves(const Tile& c, float alpha) {
@@ -2000,8 +2011,7 @@ __device__ __forceinline__ void descend_block(Tile& c, const float (&mrow)[N], f
         c.F(hMove, h) = 0.0f; c.F(hMove + 1, h) = 0.0f; c.F(hMove + 2, h) = 0.0f;
     }
     __syncthreads();
-    PlainLine line{};   // the heads' constants over this block descent
-    if constexpr (kKeepLine<N>) line = own_line(c);
+    PlainLine line = own_line(c);   // the heads' constants over this block descent
     float start = coordinate ? *u_io : 0.0f;
     const float free_v = moving && has_free ? free_in : 0.0f;
     if constexpr (kFollow) {   // the followers start where the block's coordinates put them
@@ -2018,7 +2028,7 @@ __device__ __forceinline__ void descend_block(Tile& c, const float (&mrow)[N], f
         const float inertial_curvature = coordinate_total<N>(curvature);
         if (inertial_curvature > 0.0f && isfinite(inertial_curvature)) {
             row_steps<N>(c, dd);
-            const float alpha = search_line<kKeepLine<N>>(c, line, -inertial_curvature, inertial_curvature);
+            const float alpha = search_line(c, line, -inertial_curvature, inertial_curvature);
             if (alpha > 0.0f) {
                 u = fmaf(alpha, dd, u);
                 apply_moves(c, alpha);
@@ -2056,7 +2066,7 @@ __device__ __forceinline__ void descend_block(Tile& c, const float (&mrow)[N], f
         row_steps<N>(c, dd);
         PROF_END(c, 4);
         PROF_BEGIN(c, 5);
-        const float alpha = search_line<kKeepLine<N>>(c, line, inertial_slope, inertial_curvature);
+        const float alpha = search_line(c, line, inertial_slope, inertial_curvature);
         PROF_END(c, 5);
         PROF_BEGIN(c, 28);
         const float after = fmaf(alpha, dd, u);
@@ -2602,7 +2612,7 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
     }
     if (lane < kNarrowFields) c.fields[kWideStride * cap + staged_cap * kNarrowStride + lane] = 0.0f;   // what a narrow field reads beyond its heads
     c.unit_list = reinterpret_cast<uint32_t*>(c.vec + 256);
-    c.unit_lists = true; c.unit_count = 0u; c.staged_end = 0u; c.individual_end = 0u;
+    c.unit_lists = true; c.unit_count = 0u; c.unit_most = 0u; c.staged_end = 0u; c.individual_end = 0u;
     c.through_links = false;
     c.axes = c.vec + 256 + (cap > staged_cap ? kUnitSlots * uint32_t(kWave) : 0u);   // a wide block's; a narrow one keeps rows here
     c.spread = c.axes + 12u * uint32_t(kWave);   // a block without contact rows has it, and the next
@@ -2730,13 +2740,21 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
         __syncthreads();
         // every coordinate lists its own unit heads, in head order
         if (c.units) {
-            for (uint32_t h = 0u; h < heads; ++h) {
-                if (c.U(hUnit, h) != lane) continue;
-                if (my_units < kUnitSlots) c.unit_list[my_units * uint32_t(kWave) + lane] = h;
-                ++my_units;
+            constexpr uint32_t kAhead = 16u;   // reads in flight
+            for (uint32_t h0 = 0u; h0 < heads; h0 += kAhead) {
+                uint32_t unit[kAhead];
+#pragma unroll
+                for (uint32_t t = 0u; t < kAhead; ++t) unit[t] = c.U(hUnit, min(h0 + t, heads - 1u));
+#pragma unroll
+                for (uint32_t t = 0u; t < kAhead; ++t) {
+                    if (unit[t] != lane || h0 + t >= heads) continue;
+                    if (my_units < kUnitSlots) c.unit_list[my_units * uint32_t(kWave) + lane] = h0 + t;
+                    ++my_units;
+                }
             }
             c.unit_lists = !__any(my_units > kUnitSlots);
             c.unit_count = min(my_units, kUnitSlots);
+            c.unit_most = wave_max_u(c.unit_count);
         }
         PROF_END(c, 23);
     }
