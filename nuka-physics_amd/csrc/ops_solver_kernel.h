@@ -2643,7 +2643,7 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
     const uint32_t current = d.contact_row_extent[2u * env + 1u];
     const uint32_t bound = current == 0u ? p.contact_rows_per_env : min(current - 1u, p.contact_rows_per_env);
     const uint32_t total = bound + (R - p.contact_rows_per_env);
-    uint32_t heads = 0u;
+    uint32_t heads = 0u, contact_heads = 0u;   // the latter among the former
     bool overflow = false;
     for (uint32_t base = 0u; base < total; base += kWave) {
         const uint32_t index = base + lane;
@@ -2659,9 +2659,11 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
             if (at < cap) c.U(hSlot, at) = slot; else overflow = true;
         }
         heads += __popcll(mask);
+        contact_heads += __popcll(mask & (bound >= base + kWave ? ~uint64_t{0} : bound > base ? (uint64_t{1} << (bound - base)) - 1u : uint64_t{0}));
     }
     if (__any(overflow)) {   // more heads than the staged LDS holds: fail loudly, solve the ones that fit
         heads = cap;
+        contact_heads = min(contact_heads, cap);
         if (lane == 0u) d.env_status[env] |= kEnvStatusSolverFailure;
     }
     if constexpr (kContactsOnly) __builtin_assume(heads <= uint32_t(kWave));
@@ -2672,12 +2674,15 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
     // stage Jacobian rows: the sum of the articulated sides' chain rows (TileBlock::Jacobian :555-573, CopyTileRows :836-869).
     // First every (head, axis) row finds its source rows, one per lane; then the copies run with their loads in flight
     // together instead of one row's latency after another.
-    for (uint32_t r = lane; r < 3u * heads; r += kWave) {
-        const uint32_t h = r / 3u, axis = r - 3u * h;
+    // (the contact rows' heads have up to three rows, those of the joint rows, which all come after them, one)
+    const uint32_t fan_out = 3u * contact_heads, sources = fan_out + (heads - contact_heads);
+    for (uint32_t r = lane; r < sources; r += kWave) {
+        const bool contact = r < fan_out;
+        const uint32_t h = contact ? r / 3u : r - 2u * contact_heads, axis = contact ? r - 3u * h : 0u;
         const uint32_t slot = c.U(hSlot, h);
         const uint32_t flags = __float_as_uint(urows[size_t{slot} * kRowWords]);
         const uint32_t stride = __float_as_uint(urows[size_t{slot} * kRowWords + 2u]);
-        const uint32_t axes = (flags & kRowBlockNormal) != 0u ? 3u : 1u;
+        const uint32_t axes = contact && (flags & kRowBlockNormal) != 0u ? 3u : 1u;
         uint32_t source_a = kInvalid, source_b = kInvalid;
         if (axis < axes) {
             const uint32_t rs = slot + axis * stride;
@@ -2685,6 +2690,9 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
             if (__float_as_uint(urows[size_t{rs} * kRowWords + 18u]) == kSideArtic) source_b = rs;
         }
         c.U(hSourceA + axis, h) = source_a; c.U(hSourceB + axis, h) = source_b;
+        if (contact) continue;
+#pragma unroll
+        for (uint32_t k = 1u; k < 3u; ++k) { c.U(hSourceA + k, h) = kInvalid; c.U(hSourceB + k, h) = kInvalid; }
     }
     __syncthreads();
     PROF_BEGIN(c, 22);
@@ -3064,46 +3072,20 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
                 if (lane == 0u) { c.F(hStep, h) = shares[0]; c.F(hMove, h) = shares[1]; }
             }
         }
-        if (share_units) {   // (M^-1)_uu of every coordinate that has unit heads, four coordinates at a time
-            float mine = 0.0f;
-            for (uint64_t rest = __ballot(c.unit_count > 0u); rest != 0ull;) {
-                uint32_t target[4];
-                float a[4], total[4];
+        if (share_units) {
+            // (M^-1)_uu of every coordinate at once, lane = coordinate u: y = L^-1 e_u down the rows with the factor's entries the
+            // same for every lane, and the ordered sum of y^2 / D, with the operations of the loop above (four coordinates a
+            // pass of that loop took 40 k cycles of a servo-driven humanoid's set-up, this takes 9 k)
+            const Recip by_pivot = make_recip(pivot);   // the quotients to the bit wherever their sum can see them
+            float mine = 0.0f, y[N];
 #pragma unroll
-                for (int t = 0; t < 4; ++t) {
-                    target[t] = rest != 0ull ? uint32_t(__builtin_ctzll(rest)) : kInvalid;
-                    rest &= rest - 1ull;   // zero stays zero
-                    a[t] = lane == target[t] ? 1.0f : 0.0f;
-                }
-                // below the group's first coordinate every y_j is an exact zero: those steps subtract and add nothing
-                const int first = int(target[0]);
+            for (int i = 0; i < N; ++i) {
+                float v = lane == uint32_t(i) ? 1.0f : 0.0f;
 #pragma unroll
-                for (int j = 0; j < N; ++j) {
-                    if (j < first) continue;
-                    float y[4];
-#pragma unroll
-                    for (int t = 0; t < 4; ++t) y[t] = lane_value(a[t], j);
-#pragma unroll
-                    for (int t = 0; t < 4; ++t) a[t] -= lrow[j] * y[t];
-                }
-                float* terms = c.hfac;
-#pragma unroll
-                for (int t = 0; t < 4; ++t) {
-                    const float term = coordinate ? a[t] * a[t] / pivot : 0.0f;
-                    if (lane < uint32_t(N)) terms[uint32_t(t * N) + lane] = term;
-                }
-                __syncthreads();
-                float sum = 0.0f;
-                {
-                    const float4* words = reinterpret_cast<const float4*>(terms + (lane & 3u) * uint32_t(N));
-#pragma unroll
-                    for (int q = 0; q < N / 4; ++q) { const float4 w = words[q]; sum += w.x; sum += w.y; sum += w.z; sum += w.w; }
-                }
-                __syncthreads();
-#pragma unroll
-                for (int t = 0; t < 4; ++t) total[t] = lane_value(sum, t);
-#pragma unroll
-                for (int t = 0; t < 4; ++t) if (lane == target[t]) mine = total[t];
+                for (int j = 0; j < i; ++j) v -= lane_value(lrow[j], i) * y[j];
+                y[i] = v;
+                const float term = div_by(v * v, Recip{lane_value(pivot, i), lane_value(by_pivot.value, i)});
+                mine += uint32_t(i) < n ? term : 0.0f;
             }
             for (uint32_t k = 0u; k < c.unit_count; ++k) {   // lane = coordinate hands its response to its own unit heads
                 const uint32_t h = c.unit_list[k * uint32_t(kWave) + lane];
