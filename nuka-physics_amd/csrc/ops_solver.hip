@@ -34,19 +34,24 @@ NKH_DECLARE_DENSE(24, 12) NKH_DECLARE_DENSE(28, 16) NKH_DECLARE_DENSE(32, 16) NK
 
 
 // Heads the solver's LDS holds: the contact heads (each stages three Jacobian rows) plus one unit head per joint row
-// slot.  Returns the contact-head capacity that fits the budget, 0 when not even one does.  The Hessian rows that a block
-// of at most 32 coordinates keeps (KeptRowFloats, 4 KB at most) are not counted against the budget: they save time and
-// would cost a full world heads (six of 230 at 32 coordinates), and a compute unit has room for both.
+// slot.  Returns the contact-head capacity that fits the budget, 0 when not even one does.  The line lies where it was when a
+// contact head took 60 words beside its rows, a joint row's 31 and the unit heads' lists a word a place: an environment
+// past it is flagged and solved with the heads that fit, and stays so though the records have shrunk since.
 constexpr size_t kHeadLdsBytes = 150u * 1024u;
+static uint32_t CapacityFloats(uint32_t dof, uint32_t staged, uint32_t joint_heads) {
+    const uint32_t fields = (31u * (staged + joint_heads) + 29u * (staged + 1u) + 3u) & ~3u;
+    return solver::FactorRegionFloats(dof) + solver::RowFloats(solver::PaddedWidth(dof), staged, false) + fields + 256u +
+           (joint_heads != 0u ? solver::kUnitSlots * uint32_t(solver::kWave) : 0u) + solver::LinkAxisFloats(dof);
+}
 static_assert(kHeadLdsBytes + 32u * 32u * sizeof(float) <= 160u * 1024u, "the largest tile and its kept rows fit a compute unit");
+static_assert(solver::kWideStride <= 31u && solver::kWideStride + solver::kNarrowStride <= 60u, "a head takes no more than the capacity allows for");
 // a contact point is one head, or four under the pyramidal cone of the MuJoCo law (one scalar head an edge)
 static uint32_t HeadsAPoint(const ModelView& m) { return m.any_mujoco != 0u && m.contact_cone == 0u ? kRowsPerPoint : 1u; }
 uint32_t SolverHeadCapacity(const ModelView& m, uint32_t slots) {
     const uint32_t want = slots * (m.max_points_per_slot == 0u ? kPointsPerSlot : m.max_points_per_slot) * HeadsAPoint(m);
     const uint32_t joint_heads = m.joint_limit_rows + m.joint_friction_rows + m.joint_drive_rows;
     for (uint32_t staged = want; staged >= 1u; --staged)
-        if (size_t{solver::SolverLdsFloats(m.dof, staged + joint_heads, staged) - solver::KeptRowFloats(m.dof, false)} * sizeof(float) <=
-            kHeadLdsBytes) return staged;
+        if (size_t{CapacityFloats(m.dof, staged, joint_heads)} * sizeof(float) <= kHeadLdsBytes) return staged;
     return 0u;
 }
 
@@ -232,7 +237,9 @@ Status OpBlockDescentSolve(const ModelView& m, const DataView& d, const void* pa
     // touch, at its largest manifold) outnumber the contacts an environment usually has.  Where a smaller capacity
     // lets more blocks share a compute unit, environments with few contact points go to a launch of that capacity:
     // a launch each for sixteen, twelve, eight, four and two blocks a unit, those the waves allow, before the full one.  Each launch takes the
-    // environments whose contact points fall in its range; an environment's results do not depend on its launch.
+    // environments whose contact points fall in its range; an environment's results do not depend on its launch.  It has to
+    // let half as many blocks again share a unit: 4096 servo-driven humanoids take 2525 us a step in launches of eight and of
+    // seven blocks a unit, one after the other's longest environment, and 1476 us in one of seven.
     // A contact point is at most `a_point` heads, so `few` heads hold few / a_point points whatever their friction: four
     // edges a point under the pyramidal cone.  (While those worlds went to the one full launch, a walker's 304 heads left a
     // compute unit one block for environments of a handful of points: a step of 4096 with a twentieth reset 768 -> 438 us.)
@@ -242,7 +249,8 @@ Status OpBlockDescentSolve(const ModelView& m, const DataView& d, const void* pa
     if (p->contact_slots_per_env != 0u) {
         for (const size_t blocks : {size_t{16u}, size_t{12u}, size_t{8u}, size_t{4u}, size_t{2u}}) {
             if (blocks > most_blocks) continue;                            // more blocks than the waves allow
-            if (blocks_per_unit(staged) >= blocks) break;                  // the full capacity does as well
+            if (blocks_per_unit(staged) >= blocks) break;                  // the full capacity does as well,
+            if (2u * blocks < 3u * blocks_per_unit(staged)) continue;      // or nearly: a launch more ends with a longest environment more
             uint32_t few = staged;
             while (few > 8u && blocks_per_unit(few) < blocks) --few;
             const uint32_t points = few / a_point;

@@ -264,14 +264,20 @@ __device__ __forceinline__ float along_axis(float impulse, float velocity) { ret
 
 // Per-head state in LDS, head-major with an odd stride so lane = head reads without bank conflicts.
 enum HeadField : uint32_t {
-    hSlot, hStride, hAxes, hOwned, hRho, hCompliance, hLower, hUpper, hMu1, hMu2, hNormalBound,
+    hSlot,               // the head's row of the environment-major records; kUnowned beside it: the head acts on nothing
+    hStride, hAxes, hRho, hCompliance, hLower, hUpper, hMu1, hMu2, hNormalBound,
     hRes, hDual = hRes + 3, hMove = hDual + 3, hStep = hMove + 3, hBase = hStep + 3, hDualScale = hBase + 3, hResidualScale,
-    hRelaxStep, hRelaxWeight = hRelaxStep + 3, hRelaxPoint, hF = hRelaxPoint + 3, hC = hF + 3, hNoise = hC + 6, hContrib = hNoise + 3, hColumnsLow, hColumnsHigh, hSourceA, hSourceB = hSourceA + 3, hSourceEnd = hSourceB + 3,
-    hRow = hSourceEnd,   // first of the head's three staged Jacobian rows; kInvalid for a unit head
+    hRelaxStep, hRelaxWeight = hRelaxStep + 3, hRelaxPoint, hC = hRelaxPoint + 3, hColumnsLow = hC + 6, hColumnsHigh,
+    hRow,                // first of the head's three staged Jacobian rows; kInvalid for a unit head
+    hSecond,             // the side that moves is the row's second
     hUnit,               // the one coordinate a unit head acts on; kInvalid for a staged head
     hUnitValue,          // its Jacobian entry there
     hFieldCount
 };
+// Fields that share their words: the rows' sources are done with when a head's residual and base are first written, and an
+// assembly's impulses when the next steps are.
+constexpr uint32_t hSourceA = hRes, hSourceB = hBase, hF = hStep;
+constexpr uint32_t kUnowned = 0x80000000u;
 
 // A contact head under the elliptic cone of the MuJoCo law (block_descent_tile.cuh:645, 778) carries 4 in hAxes: three
 // axes, answered by elliptic_impulse.  Such a head has no relaxation state (its dual update takes the projection as it
@@ -283,18 +289,22 @@ __device__ __forceinline__ bool block_axes(uint32_t axes) { return axes >= 3u; }
 // A head on one axis uses the first component of every three-component field and none of the block-only fields;
 // only block heads (three axes: contact points, which are listed first) use the rest.  The fields are therefore kept
 // in two tables: "wide" fields have room for every head, "narrow" fields for the first `narrow` heads and one more
-// word that every later head shares.  That word reads as zero and swallows what is written to it, which is always
-// zero: a single-axis head keeps its second and third components, its relaxation state and its column masks at zero
-// throughout.  A head's place in a narrow field is min(h, narrow), one operation whatever the number of fields read.
+// word that every later head shares.  What is written to that word is the same for all of them: zero for the second and third
+// components, the relaxation state, the friction and the column masks, one for the axes and the stride, no row (the
+// normal bound apart, which no head on one axis reads).  A head's place in a narrow field is min(h, narrow), one operation
+// whatever the number of fields read.
+//   A joint row's head takes fifteen words so, and with joint rows on every coordinate the tables are most of a block's LDS:
+// 31 words a head (and words where its unit heads are listed) let five blocks of the servo-driven humanoid share a
+// compute unit, where fifteen let seven: a step of 4096 of them 1749 -> 1476 us.
 __host__ __device__ constexpr uint32_t clamped_span(uint32_t f, uint32_t first, uint32_t end) {   // fields of [first, end) below f
     return f <= first ? 0u : (f >= end ? end - first : f - first);
 }
 // the narrow fields are these ranges of field ids
 __host__ __device__ constexpr uint32_t narrow_below(uint32_t f) {
-    return clamped_span(f, hRes + 1, hRes + 3) + clamped_span(f, hDual + 1, hDual + 3) + clamped_span(f, hMove + 1, hMove + 3) +
-           clamped_span(f, hStep + 1, hStep + 3) + clamped_span(f, hBase + 1, hBase + 3) + clamped_span(f, hRelaxStep, hF) +
-           clamped_span(f, hF + 1, hF + 3) + clamped_span(f, hC + 1, hNoise) + clamped_span(f, hNoise + 1, hNoise + 3) +
-           clamped_span(f, hColumnsLow, hColumnsHigh + 1);
+    return clamped_span(f, hStride, hAxes + 1) + clamped_span(f, hMu1, hNormalBound + 1) +
+           clamped_span(f, hRes + 1, hRes + 3) + clamped_span(f, hDual + 1, hDual + 3) + clamped_span(f, hMove + 1, hMove + 3) +
+           clamped_span(f, hStep + 1, hStep + 3) + clamped_span(f, hBase + 1, hBase + 3) + clamped_span(f, hRelaxStep, hC) +
+           clamped_span(f, hC + 1, hC + 6) + clamped_span(f, hColumnsLow, hSecond + 1);
 }
 __host__ __device__ constexpr bool narrow_field(uint32_t f) { return narrow_below(f + 1u) != narrow_below(f); }
 constexpr uint32_t kNarrowFields = narrow_below(hFieldCount);
@@ -328,7 +338,7 @@ struct Tile {
     bool scalar_later;   // the heads past the first 64 are on one axis, and two a lane hold them
     bool near_heads; // no staged head's rows reach past the coordinates two tiles hold (add_heads_by_tiles)
     bool unit_lists; // every coordinate's unit heads fit its list
-    uint32_t* unit_list;      // kUnitSlots x 64: lane's unit heads in head order, slot-major
+    uint16_t* unit_list;      // kUnitSlots x 64: lane's unit heads in head order, slot-major
     uint32_t unit_count;      // lane's own count
     uint32_t unit_most;       // the largest
     uint32_t staged_end;      // one past the last staged head
@@ -361,6 +371,8 @@ struct Tile {
     }
     __device__ __forceinline__ float& F(uint32_t field, uint32_t h) const { return fields[at(field, h)]; }
     __device__ __forceinline__ uint32_t& U(uint32_t field, uint32_t h) const { return reinterpret_cast<uint32_t*>(fields)[at(field, h)]; }
+    __device__ __forceinline__ uint32_t slot(uint32_t h) const { return U(hSlot, h) & ~kUnowned; }
+    __device__ __forceinline__ bool owned(uint32_t h) const { return (U(hSlot, h) & kUnowned) == 0u; }
 };
 
 // lane's row of Tile::low, as sixteen-byte words
@@ -1025,7 +1037,7 @@ struct HeadLine {
 __device__ __forceinline__ HeadLine load_head_line(const Tile& c, uint32_t h) {
     HeadLine l{};
     l.head = h;
-    l.owned = h < c.heads && c.U(hOwned, h) != 0u;
+    l.owned = h < c.heads && c.owned(h);
     if (!l.owned) return l;
     l.contact = block_axes(c.U(hAxes, h));
     l.elliptic = c.elliptic && c.U(hAxes, h) == kAxesElliptic;
@@ -1154,7 +1166,7 @@ __device__ __forceinline__ ScalarLine scalar_line(const Tile& c, uint32_t h) {
     const uint32_t at = min(h, c.heads - 1u);   // (read whether or not there is such a head)
     const float rho = c.F(hRho, at), dual = c.F(hDual, at), compliance = c.F(hCompliance, at), lower = c.F(hLower, at), upper = c.F(hUpper, at);
     const float k = c.F(hResidualScale, at), scaled = c.F(hDualScale, at) * dual, res = c.F(hRes, at), move = c.F(hMove, at), step = c.F(hStep, at);
-    const bool live = h < c.heads && c.U(hOwned, at) != 0u && !(rho <= 0.0f);
+    const bool live = h < c.heads && c.owned(at) && !(rho <= 0.0f);
     ScalarLine s{};
     s.k = live ? k : 0.0f; s.k_bounded = live && lower < upper ? k : 0.0f;
     s.dual_part = live ? scaled : 0.0f; s.lower = live ? lower : 0.0f; s.upper = live ? upper : 0.0f;
@@ -1199,7 +1211,7 @@ __device__ __forceinline__ bool head_terms(const Tile& c, uint32_t h, float (&f)
     for (int k = 0; k < 3; ++k) { f[k] = 0.0f; noise[k] = 0.0f; }
 #pragma unroll
     for (int k = 0; k < 6; ++k) cv[k] = 0.0f;
-    if (h >= c.heads || c.U(hOwned, h) == 0u) return false;
+    if (h >= c.heads || !c.owned(h)) return false;
     head_response(c, h, c.F(hMove, h), c.F(hMove + 1, h), c.F(hMove + 2, h), f, cv);
 #pragma unroll
     for (int k = 0; k < 3; ++k) noise[k] = fabsf(f[k]) + cv[k] * (fabsf(c.F(hRes + k, h)) + fabsf(c.F(hMove + k, h)));
@@ -1385,8 +1397,8 @@ __device__ __forceinline__ void add_heads_through_links(const Tile& c, bool mine
 #pragma unroll
         for (int e = 0; e < 24; ++e) k[e] = 0.0f;
         if (mine) {
-            const uint32_t slot = c.U(hSlot, lane), stride = c.U(hStride, lane), axes = c.U(hAxes, lane);
-            const bool second = c.U(hSourceA, lane) == kInvalid;   // the side that moves is the row's second
+            const uint32_t slot = c.slot(lane), stride = c.U(hStride, lane), axes = c.U(hAxes, lane);
+            const bool second = c.U(hSecond, lane) != 0u;
             float w[3][6];
 #pragma unroll
             for (uint32_t a = 0u; a < 3u; ++a) {
@@ -1514,27 +1526,23 @@ __device__ __forceinline__ bool assemble_block(const Tile& c, const float (&mrow
         const ScalarLine s = scalar_line(c, h);
         float f, cv;
         scalar_line_response(s, s.move, &f, &cv);
-        const float noise = fabsf(f) + cv * (fabsf(s.res) + fabsf(s.move));
         differs |= bits(c.F(hC, h)) ^ bits(cv);
-        c.F(hF, h) = f; c.F(hNoise, h) = noise; c.F(hC, h) = cv;
-        c.U(hContrib, h) = ((bits(f) | bits(cv) | bits(noise)) << 1u) != 0u ? 1u : 0u;
+        c.F(hF, h) = f; c.F(hC, h) = cv;
     }
     for (uint32_t h = lane + kWave; !c.scalar_later && h < c.heads; h += kWave) {
         float f[3], cv[6], noise[3];
-        const bool contributes = head_terms(c, h, f, cv, noise);
+        head_terms(c, h, f, cv, noise);
 #pragma unroll
-        for (int k = 0; k < 3; ++k) { c.F(hF + k, h) = f[k]; c.F(hNoise + k, h) = noise[k]; }
+        for (int k = 0; k < 3; ++k) c.F(hF + k, h) = f[k];
 #pragma unroll
         for (int k = 0; k < 6; ++k) { differs |= bits(c.F(hC + k, h)) ^ bits(cv[k]); c.F(hC + k, h) = cv[k]; }
-        c.U(hContrib, h) = contributes ? 1u : 0u;
     }
 #pragma unroll
     for (int k = 0; k < 6; ++k) { differs |= bits(c.curvature[k]) ^ bits(mc[k]); c.curvature[k] = mc[k]; }
     if (__any(lane < c.heads && differs != 0u)) { c.factor_current = false; c.rows_current = false; c.stiffness_current = false; }
     const bool rows_kept = N <= 32 && c.rows_current && c.heads <= uint32_t(kWave);   // only the force is to be summed
     if (c.units && lane < c.heads && c.U(hUnit, lane) != kInvalid) {   // a coordinate reads its unit heads' responses from the fields
-        c.F(hF, lane) = mf[0]; c.F(hNoise, lane) = mn[0]; c.F(hC, lane) = mc[0];
-        c.U(hContrib, lane) = mine ? 1u : 0u;
+        c.F(hF, lane) = mf[0]; c.F(hC, lane) = mc[0];
     }
     __syncthreads();
     PROF_END(c, 10);
@@ -1569,11 +1577,15 @@ __device__ __forceinline__ bool assemble_block(const Tile& c, const float (&mrow
     TileSum g{-inertial.value};
     PROF_END(c, 11);
     PROF_BEGIN(c, 12);
-    // heads beyond the first 64 hold their responses in the fields
+    // heads beyond the first 64 hold their responses in the fields, unit heads theirs
+    auto noise_of = [&](float f, float curvature, uint32_t h, uint32_t axis) {
+        return fabsf(f) + curvature * (fabsf(c.F(hRes + axis, h)) + fabsf(c.F(hMove + axis, h)));
+    };
     auto add_later_head = [&](uint32_t h) {
         const float f[3] = {c.F(hF, h), c.F(hF + 1, h), c.F(hF + 2, h)};
         const float cv[6] = {c.F(hC, h), c.F(hC + 1, h), c.F(hC + 2, h), c.F(hC + 3, h), c.F(hC + 4, h), c.F(hC + 5, h)};
-        const float noise[3] = {c.F(hNoise, h), c.F(hNoise + 1, h), c.F(hNoise + 2, h)};
+        if (f[0] == 0.0f && f[1] == 0.0f && f[2] == 0.0f && cv[0] == 0.0f && cv[1] == 0.0f && cv[2] == 0.0f && cv[3] == 0.0f && cv[4] == 0.0f && cv[5] == 0.0f) return;
+        const float noise[3] = {noise_of(f[0], cv[0], h, 0u), noise_of(f[1], cv[1], h, 1u), noise_of(f[2], cv[2], h, 2u)};
         const uint64_t columns = (uint64_t(__builtin_amdgcn_readfirstlane(c.U(hColumnsHigh, h))) << 32u) |
                                  uint64_t(__builtin_amdgcn_readfirstlane(c.U(hColumnsLow, h)));
         add_head<N>(c, h, coordinate, f, cv, noise, c.U(hAxes, h), columns, hrow, g, scale);
@@ -1592,7 +1604,7 @@ __device__ __forceinline__ bool assemble_block(const Tile& c, const float (&mrow
         add_heads_force<N>(c, staged, mf, mn, lane < c.heads ? c.U(hRow, lane) : 0u, g, scale);
         add_heads_through_links<N>(c, mine, mc, hrow);
     } else {
-        if (N <= 32 || (N <= kTwoWaveWidth && c.near_heads)) {
+        if (N <= 32 || (N <= kTwoWaveWidth && c.near_heads && !c.units)) {
             if constexpr (N <= kTwoWaveWidth) if (staged != 0ull) {
                 const uint32_t my_first = c.U(hRow, lane < c.heads ? lane : 0u);
                 if constexpr (kFollow && N <= 32) {
@@ -1620,7 +1632,7 @@ __device__ __forceinline__ bool assemble_block(const Tile& c, const float (&mrow
             }
         }
         for (uint32_t h = kWave; h < (c.units ? c.staged_end : c.heads); ++h) {
-            if (c.U(hContrib, h) == 0u || (c.units && c.U(hUnit, h) != kInvalid)) continue;
+            if (c.units && c.U(hUnit, h) != kInvalid) continue;
             add_later_head(h);
         }
     }
@@ -1630,14 +1642,14 @@ __device__ __forceinline__ bool assemble_block(const Tile& c, const float (&mrow
         // (the list and then its heads' words read whether or not the lane has so many, all in flight together: a head that does
         // not contribute holds zeros)
         float diagonal = 0.0f;
-        auto add_unit = [&](float v, float curvature, float force, float noise) {
+        auto add_unit = [&](float v, float curvature, float force, float res, float move) {
             diagonal += v * curvature * v;
             tile_add_product(g, v, force);
-            scale += fabsf(v) * noise;
+            scale += fabsf(v) * (fabsf(force) + curvature * (fabsf(res) + fabsf(move)));
         };
         if (c.unit_lists) {
             uint32_t h[kUnitSlots];
-            float v[kUnitSlots], words[kUnitSlots][3];
+            float v[kUnitSlots], words[kUnitSlots][4];
 #pragma unroll
             for (uint32_t k = 0u; k < kUnitSlots; ++k) {
                 const uint32_t listed = c.unit_list[k * uint32_t(kWave) + lane];
@@ -1646,17 +1658,18 @@ __device__ __forceinline__ bool assemble_block(const Tile& c, const float (&mrow
 #pragma unroll
             for (uint32_t k = 0u; k < kUnitSlots; ++k) {
                 if (k >= c.unit_most) break;
-                v[k] = c.F(hUnitValue, h[k]); words[k][0] = c.F(hC, h[k]); words[k][1] = c.F(hF, h[k]); words[k][2] = c.F(hNoise, h[k]);
+                v[k] = c.F(hUnitValue, h[k]); words[k][0] = c.F(hC, h[k]); words[k][1] = c.F(hF, h[k]);
+                words[k][2] = c.F(hRes, h[k]); words[k][3] = c.F(hMove, h[k]);
             }
 #pragma unroll
             for (uint32_t k = 0u; k < kUnitSlots; ++k) {
                 if (k >= c.unit_most) break;
                 const bool on = k < c.unit_count;
-                add_unit(on ? v[k] : 0.0f, on ? words[k][0] : 0.0f, on ? words[k][1] : 0.0f, on ? words[k][2] : 0.0f);
+                add_unit(on ? v[k] : 0.0f, on ? words[k][0] : 0.0f, on ? words[k][1] : 0.0f, on ? words[k][2] : 0.0f, on ? words[k][3] : 0.0f);
             }
         } else {
             for (uint32_t h = 0u; h < c.heads; ++h)
-                if (c.U(hContrib, h) != 0u && c.U(hUnit, h) == lane) add_unit(c.F(hUnitValue, h), c.F(hC, h), c.F(hF, h), c.F(hNoise, h));
+                if (c.U(hUnit, h) == lane) add_unit(c.F(hUnitValue, h), c.F(hC, h), c.F(hF, h), c.F(hRes, h), c.F(hMove, h));
         }
         if (!rows_kept) {
 #pragma unroll
@@ -1801,7 +1814,7 @@ __device__ __forceinline__ void row_steps(const Tile& c, float d) {
     }
     if constexpr (N > kTwoWaveWidth) {
         if (c.from_links) {   // contact heads, one a lane at most, none of them a unit head
-            const bool owned = c.lane < c.heads && c.U(hOwned, c.lane < c.heads ? c.lane : 0u) != 0u;
+            const bool owned = c.lane < c.heads && c.owned(c.lane < c.heads ? c.lane : 0u);
             const uint32_t h = owned ? c.lane : 0u, axes = c.U(hAxes, h);
             float motion[6];
             link_motion<N>(c, owned ? way_of(c, h) : 0ull, dvec, motion);
@@ -1818,13 +1831,13 @@ __device__ __forceinline__ void row_steps(const Tile& c, float d) {
     // come after them.  (A lane a head, its three rows in turn, held the unit heads up behind a dozen contacts.)
     for (uint32_t r = c.lane; r < 3u * c.staged_end; r += kWave) {
         const uint32_t h = r / 3u, axis = r - 3u * h, first = c.U(hRow, h);
-        if (first == kInvalid || c.U(hOwned, h) == 0u) continue;
+        if (first == kInvalid || !c.owned(h)) continue;
         c.fields[axis == 0u ? c.at(hStep, h) : c.at(hStep + 1, h) + axis - 1u] = row_dot_fma<N>(c.jac + (first + axis) * uint32_t(N), dvec);
     }
     if (c.units) {
         for (uint32_t h = c.lane; h < c.heads; h += kWave) {
             const uint32_t unit = c.U(hUnit, h);
-            if (c.U(hOwned, h) != 0u && unit != kInvalid) c.F(hStep, h) = c.F(hUnitValue, h) * dvec[unit];   // :2028-2032
+            if (c.owned(h) && unit != kInvalid) c.F(hStep, h) = c.F(hUnitValue, h) * dvec[unit];   // :2028-2032
         }
     }
     __syncthreads();
@@ -1989,7 +2002,7 @@ __device__ __forceinline__ float search_line(const Tile& c, PlainLine& line, flo
 
 __device__ __forceinline__ void apply_moves(const Tile& c, float alpha) {
     for (uint32_t h = c.lane; h < c.heads; h += kWave) {
-        if (c.U(hOwned, h) == 0u) continue;
+        if (!c.owned(h)) continue;
 #pragma unroll
         for (int k = 0; k < 3; ++k) c.F(hMove + k, h) = fmaf(alpha, c.F(hStep + k, h), c.F(hMove + k, h));
     }
@@ -2006,7 +2019,7 @@ __device__ __forceinline__ void descend_block(Tile& c, const float (&mrow)[N], f
     const bool moving = coordinate || follower;
     PROF_BEGIN(c, 26);
     for (uint32_t h = lane; h < c.heads; h += kWave) {   // StartTileBlock (:1386-1397)
-        if (c.U(hOwned, h) == 0u) continue;
+        if (!c.owned(h)) continue;
         c.F(hNormalBound, h) = c.F(hDual, h);
         c.F(hMove, h) = 0.0f; c.F(hMove + 1, h) = 0.0f; c.F(hMove + 2, h) = 0.0f;
     }
@@ -2082,7 +2095,7 @@ __device__ __forceinline__ void descend_block(Tile& c, const float (&mrow)[N], f
     }
     PROF_BEGIN(c, 29);
     for (uint32_t h = lane; h < c.heads; h += kWave) {   // EndTileBlock (:1400-1409)
-        if (c.U(hOwned, h) == 0u) continue;
+        if (!c.owned(h)) continue;
 #pragma unroll
         for (int k = 0; k < 3; ++k) c.F(hRes + k, h) = c.F(hRes + k, h) - c.F(hMove + k, h);
     }
@@ -2139,20 +2152,20 @@ __device__ __forceinline__ void measure_primal(Tile& c, const float (&mrow)[N], 
                 const uint32_t h = c.unit_list[next * uint32_t(kWave) + lane];
                 if (h >= below) break;
                 ++next;
-                if (c.U(hOwned, h) != 0u) balance += double(c.F(hUnitValue, h)) * lambda_env[c.U(hSlot, h) - c.env * R];
+                if (c.owned(h)) balance += double(c.F(hUnitValue, h)) * lambda_env[c.slot(h) - c.env * R];
             }
             return;
         }
         for (uint32_t h = from; h < below; ++h)
-            if (c.U(hOwned, h) != 0u && c.U(hUnit, h) == lane) balance += double(c.F(hUnitValue, h)) * lambda_env[c.U(hSlot, h) - c.env * R];
+            if (c.owned(h) && c.U(hUnit, h) == lane) balance += double(c.F(hUnitValue, h)) * lambda_env[c.slot(h) - c.env * R];
     };
     uint32_t done = 0u;
     bool rows_taken = false;
     if constexpr (N > kTwoWaveWidth) {
         if (c.from_links) {   // lane = head holds its impulse; the sum goes by way of the links
             float impulse[3] = {0.0f, 0.0f, 0.0f};
-            if (lane < c.heads && c.U(hOwned, lane) != 0u) {
-                const uint32_t local = c.U(hSlot, lane) - c.env * R, stride = c.U(hStride, lane), axes = c.U(hAxes, lane);
+            if (lane < c.heads && c.owned(lane)) {
+                const uint32_t local = c.slot(lane) - c.env * R, stride = c.U(hStride, lane), axes = c.U(hAxes, lane);
                 impulse[0] = lambda_env[local];
                 if (block_axes(axes)) { impulse[1] = lambda_env[local + stride]; impulse[2] = lambda_env[local + 2u * stride]; }
             }
@@ -2163,10 +2176,10 @@ __device__ __forceinline__ void measure_primal(Tile& c, const float (&mrow)[N], 
     }
     for (uint32_t h = 0u; h < (rows_taken ? 0u : c.staged_end); ++h) {
         const uint32_t first = c.U(hRow, h);
-        if (first == kInvalid || c.U(hOwned, h) == 0u) continue;
+        if (first == kInvalid || !c.owned(h)) continue;
         add_units(done, h);
         done = h + 1u;
-        const uint32_t local = c.U(hSlot, h) - c.env * R, stride = c.U(hStride, h), axes = c.U(hAxes, h);
+        const uint32_t local = c.slot(h) - c.env * R, stride = c.U(hStride, h), axes = c.U(hAxes, h);
         const float ix = lambda_env[local], iy = block_axes(axes) ? lambda_env[local + stride] : 0.0f,
                     iz = block_axes(axes) ? lambda_env[local + 2u * stride] : 0.0f;
         if (!(ix != 0.0f || iy != 0.0f || iz != 0.0f)) continue;
@@ -2217,7 +2230,7 @@ __device__ __forceinline__ void initialize_residuals(const Tile& c, float veloci
         if (c.from_links) link_motion<N>(c, c.lane < c.heads ? way_of(c, c.lane) : 0ull, dvec, motion);
     }
     for (uint32_t h = c.lane; h < c.heads; h += kWave) {
-        const uint32_t slot = c.U(hSlot, h), stride = c.U(hStride, h), axes = c.U(hAxes, h);
+        const uint32_t slot = c.slot(h), stride = c.U(hStride, h), axes = c.U(hAxes, h);
         const uint32_t unit = c.U(hUnit, h), first = c.U(hRow, h);
         if (unit != kInvalid || first == kInvalid) {   // one coordinate (or none): every other product is an exact zero
             const float along = unit != kInvalid ? c.F(hUnitValue, h) * dvec[unit] : 0.0f;
@@ -2259,7 +2272,7 @@ __device__ __forceinline__ void update_duals(const Tile& c, float* lambda_env, u
     uint32_t steps[3] = {0u, 0u, 0u};
     double restart = 0.0;
     for (uint32_t h = c.lane; h < c.heads; h += kWave) {
-        const uint32_t slot = c.U(hSlot, h), local = slot - c.env * R, stride = c.U(hStride, h), axes = c.U(hAxes, h);
+        const uint32_t slot = c.slot(h), local = slot - c.env * R, stride = c.U(hStride, h), axes = c.U(hAxes, h);
         const bool contact = block_axes(axes);
         const bool elliptic = c.elliptic && axes == kAxesElliptic;
         const float rho = c.F(hRho, h), compliance = c.F(hCompliance, h), lower = c.F(hLower, h), upper = c.F(hUpper, h);
@@ -2420,6 +2433,8 @@ __host__ __device__ inline uint32_t KeptRowFloats(uint32_t n, bool reduced) {
     const uint32_t N = PaddedWidth(n);
     return N > 32u ? 0u : (reduced ? 2u : 1u) * N * N;
 }
+// the coordinates' lists of their unit heads, sixteen bits a place
+__host__ __device__ inline uint32_t UnitListFloats(uint32_t cap, uint32_t staged) { return cap > staged ? kUnitSlots * uint32_t(kWave) / 2u : 0u; }
 __host__ __device__ inline uint32_t HeadFieldFloats(uint32_t cap, uint32_t narrow) {
     return (kWideStride * cap + kNarrowStride * (narrow + 1u) + 3u) & ~3u;
 }
@@ -2439,7 +2454,7 @@ __host__ __device__ inline uint32_t SolverLdsFloats(uint32_t n, uint32_t cap, ui
     // the per-coordinate unit lists exist only when some head beyond the staged ones can be listed; without joint rows
     // the block keeps the footprint that lets eight of them share a compute unit's LDS
     return FactorRegionFloats(n) + RowFloats(N, staged, from_links) + HeadFieldFloats(cap, staged) + 256u +
-           (cap > staged ? kUnitSlots * uint32_t(kWave) : 0u) + LinkAxisFloats(n) + SpreadFloats(from_links) + KeptRowFloats(n, reduced);
+           UnitListFloats(cap, staged) + LinkAxisFloats(n) + SpreadFloats(from_links) + KeptRowFloats(n, reduced);
 }
 __host__ __device__ inline uint32_t ReducedSolverLdsFloats(uint32_t full, uint32_t reduced, uint32_t cap, uint32_t staged, bool from_links = false) {
     const uint32_t solve = SolverLdsFloats(reduced, cap, staged, from_links, reduced < full), scratch = ReductionScratchFloats(full, reduced);
@@ -2599,7 +2614,7 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
     c.wrench = c.jac;   // one or the other
     c.fields = c.jac + RowFloats(uint32_t(W), staged_cap, c.from_links);
     c.vec = c.fields + HeadFieldFloats(cap, staged_cap);
-    c.hrows = c.vec + 256 + (cap > staged_cap ? kUnitSlots * uint32_t(kWave) : 0u);
+    c.hrows = c.vec + 256 + UnitListFloats(cap, staged_cap);
     c.low = c.hrows + uint32_t(W) * uint32_t(W);
     // The block's mass rows: lane's row of M, or in a reduced block lane's row of the Schur complement (lanes below K)
     // and of -P (the followers).
@@ -2611,10 +2626,10 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
         PROF_END(c, 30);
     }
     if (lane < kNarrowFields) c.fields[kWideStride * cap + staged_cap * kNarrowStride + lane] = 0.0f;   // what a narrow field reads beyond its heads
-    c.unit_list = reinterpret_cast<uint32_t*>(c.vec + 256);
+    c.unit_list = reinterpret_cast<uint16_t*>(c.vec + 256);
     c.unit_lists = true; c.unit_count = 0u; c.unit_most = 0u; c.staged_end = 0u; c.individual_end = 0u;
     c.through_links = false;
-    c.axes = c.vec + 256 + (cap > staged_cap ? kUnitSlots * uint32_t(kWave) : 0u);   // a wide block's; a narrow one keeps rows here
+    c.axes = c.vec + 256 + UnitListFloats(cap, staged_cap);   // a wide block's; a narrow one keeps rows here
     c.spread = c.axes + 12u * uint32_t(kWave);   // a block without contact rows has it, and the next
     c.motions = c.spread + 8u * kMotionStride;
     c.path_low = c.path_high = c.under_low = c.under_high = c.over_low = c.over_high = 0u;
@@ -2679,10 +2694,10 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
     for (uint32_t r = lane; r < sources; r += kWave) {
         const bool contact = r < fan_out;
         const uint32_t h = contact ? r / 3u : r - 2u * contact_heads, axis = contact ? r - 3u * h : 0u;
-        const uint32_t slot = c.U(hSlot, h);
+        const uint32_t slot = c.slot(h);
         const uint32_t flags = __float_as_uint(urows[size_t{slot} * kRowWords]);
         const uint32_t stride = __float_as_uint(urows[size_t{slot} * kRowWords + 2u]);
-        const uint32_t axes = contact && (flags & kRowBlockNormal) != 0u ? 3u : 1u;
+        const uint32_t axes = contact && h < staged_cap && (flags & kRowBlockNormal) != 0u ? 3u : 1u;   // (one past the staged heads' room)
         uint32_t source_a = kInvalid, source_b = kInvalid;
         if (axis < axes) {
             const uint32_t rs = slot + axis * stride;
@@ -2702,6 +2717,7 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
         // a single-axis head acting on one coordinate is a unit head; the rows carry that coordinate and its entry
         // from where they were emitted (row_unit, row_unit_value), which is what a scan of the head's Jacobian row
         // for its entries would find
+        bool overflow_rows = false;
         for (uint32_t base = 0u; base < heads; base += kWave) {
             const uint32_t h = base + lane;
             if (h >= heads) continue;
@@ -2709,31 +2725,26 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
             const bool owned = source_a != kInvalid || source_b != kInvalid;
             // a block head has found the sources of its tangent rows on the sides that move
             const bool single_axis = c.U(hSourceA + 1u, h) == kInvalid && c.U(hSourceB + 1u, h) == kInvalid;
-            const uint32_t slot = c.U(hSlot, h);
+            const uint32_t slot = c.slot(h);
             uint32_t unit = kInvalid;
             float unit_value = 0.0f;
             if (owned && single_axis && d.row_unit[slot] != kInvalid) { unit = d.row_unit[slot]; unit_value = d.row_unit_value[slot]; }
+            else if (owned && h >= staged_cap) { overflow_rows = true; unit = 0u; }   // no room for its rows: it acts on nothing, and the solve is flagged
             c.U(hUnit, h) = unit; c.F(hUnitValue, h) = unit_value; c.U(hRow, h) = owned && unit == kInvalid ? 0u : kInvalid;
             c.U(hColumnsLow, h) = 0u; c.U(hColumnsHigh, h) = 0u;
         }
+        if (__any(overflow_rows) && lane == 0u) d.env_status[env] |= kEnvStatusSolverFailure;
         __syncthreads();
         PROF_END(c, 22);
         PROF_BEGIN(c, 23);
         // PlaceTileRows: the staged heads take their rows in head order
         uint32_t staged = 0u, staged_end = 0u, individual_end = 0u, my_units = 0u;
-        bool overflow_rows = false, any_unit = false;
+        bool any_unit = false;
         for (uint32_t base = 0u; base < heads; base += kWave) {
             const uint32_t h = base + lane;
             const bool stage = h < heads && c.U(hRow, h) != kInvalid;
             const uint64_t mask = __ballot(stage);
-            if (stage) {
-                const uint32_t at = staged + uint32_t(__popcll(mask & ((uint64_t{1} << lane) - 1ull)));
-                if (at < staged_cap) c.U(hRow, h) = 3u * at;
-                else {   // no room: the head acts on nothing, and the solve is flagged
-                    overflow_rows = true;
-                    c.U(hRow, h) = kInvalid; c.U(hUnit, h) = 0u; c.F(hUnitValue, h) = 0.0f;
-                }
-            }
+            if (stage) c.U(hRow, h) = 3u * (staged + uint32_t(__popcll(mask & ((uint64_t{1} << lane) - 1ull))));   // no more than h
             staged += uint32_t(__popcll(mask));
             if (mask != 0ull) staged_end = base + uint32_t(64 - __builtin_clzll(mask));
             any_unit = any_unit || (h < heads && c.U(hUnit, h) != kInvalid);
@@ -2744,7 +2755,6 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
         c.units = !kContactsOnly && __any(any_unit) && cap > staged_cap;   // the lists have room only when the world has joint heads
         c.staged_end = staged_end;
         c.individual_end = individual_end;
-        if (__any(overflow_rows) && lane == 0u) d.env_status[env] |= kEnvStatusSolverFailure;
         __syncthreads();
         // every coordinate lists its own unit heads, in head order
         if (c.units) {
@@ -2756,7 +2766,7 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
 #pragma unroll
                 for (uint32_t t = 0u; t < kAhead; ++t) {
                     if (unit[t] != lane || h0 + t >= heads) continue;
-                    if (my_units < kUnitSlots) c.unit_list[my_units * uint32_t(kWave) + lane] = h0 + t;
+                    if (my_units < kUnitSlots) c.unit_list[my_units * uint32_t(kWave) + lane] = uint16_t(h0 + t);
                     ++my_units;
                 }
             }
@@ -2812,7 +2822,7 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
         uint64_t head_way = 0ull;   // lane = head: the way to the root of the one side that moves
         if (lane < heads) {
             const bool side_a = c.U(hSourceA, lane) != kInvalid, side_b = c.U(hSourceB, lane) != kInvalid;
-            if (side_a != side_b) head_way = m.link_dof_mask[(side_a ? d.row_cj_link : d.row_cj_link_b)[c.U(hSlot, lane)] - env * nl];
+            if (side_a != side_b) head_way = m.link_dof_mask[(side_a ? d.row_cj_link : d.row_cj_link_b)[c.slot(lane)] - env * nl];
         }
         uint64_t under = 0ull, over = 0ull;
         for (uint32_t i = 0u; i < n; ++i) {   // the coordinates, and the heads, whose way to the root holds i
@@ -2836,7 +2846,7 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
             // moves, and its way to the root
             if (lane < heads) {
                 float* record = c.wrench + lane * kWrenchStride;
-                const uint32_t slot = c.U(hSlot, lane);
+                const uint32_t slot = c.slot(lane);
                 const float* row = urows + size_t{slot} * kRowWords;
                 const uint32_t stride = __float_as_uint(row[2]);
                 const uint32_t axes = (__float_as_uint(row[0]) & kRowBlockNormal) != 0u ? 3u : 1u;
@@ -3015,7 +3025,7 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
                 if (h >= heads) continue;
                 const bool artic_a = c.U(hSourceA, h) != kInvalid, artic_b = c.U(hSourceB, h) != kInvalid;
                 if (artic_a && artic_b) {
-                    const float* row = urows + size_t{c.U(hSlot, h)} * kRowWords;
+                    const float* row = urows + size_t{c.slot(h)} * kRowWords;
                     apart[t] = __float_as_uint(row[11]) != __float_as_uint(row[19]);
                 }
                 second[t] = artic_b && !artic_a;
@@ -3092,7 +3102,7 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
                 if (fabsf(c.F(hUnitValue, h)) != 1.0f) continue;
                 const bool artic_a = c.U(hSourceA, h) != kInvalid, artic_b = c.U(hSourceB, h) != kInvalid;
                 if (artic_a && artic_b) {   // both sides on one owner (two owners were answered above)
-                    const float* row = urows + size_t{c.U(hSlot, h)} * kRowWords;
+                    const float* row = urows + size_t{c.slot(h)} * kRowWords;
                     if (__float_as_uint(row[11]) != __float_as_uint(row[19])) continue;
                 }
                 const bool second = artic_b && !artic_a;
@@ -3108,10 +3118,12 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
     for (uint32_t base = 0u; base < heads; base += kWave) {
         const uint32_t h = base + lane;
         if (h < heads) {
-            const uint32_t slot = c.U(hSlot, h);
+            const uint32_t slot = c.slot(h);
             const float* row = urows + size_t{slot} * kRowWords;
-            const uint32_t flags = __float_as_uint(row[0]), stride = __float_as_uint(row[2]);
-            const uint32_t axes = (flags & kRowBlockNormal) != 0u ? 3u : 1u;
+            // (a head past the staged ones' room shares its narrow words with the joint rows' heads, which are on one axis)
+            const bool joint = h >= staged_cap;
+            const uint32_t flags = __float_as_uint(row[0]), stride = joint ? 1u : __float_as_uint(row[2]);
+            const uint32_t axes = !joint && (flags & kRowBlockNormal) != 0u ? 3u : 1u;
             const uint32_t kind_a = __float_as_uint(row[10]), kind_b = __float_as_uint(row[18]);
             const float shares[2] = {c.F(hStep, h), c.F(hMove, h)};
             const bool valid = shares[0] >= 0.0f && isfinite(shares[0]) && shares[1] >= 0.0f && isfinite(shares[1]);
@@ -3133,9 +3145,10 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
             const bool elliptic = !kContactsOnly && axes == 3u && (flags & kRowMuJoCo) != 0u;
             any_elliptic = any_elliptic || elliptic;
             c.U(hStride, h) = stride; c.U(hAxes, h) = elliptic ? kAxesElliptic : axes;
-            c.U(hOwned, h) = (kind_a == kSideArtic || kind_b == kSideArtic) ? 1u : 0u;
+            c.U(hSlot, h) = slot | (kind_a == kSideArtic || kind_b == kSideArtic ? 0u : kUnowned);
+            c.U(hSecond, h) = joint || kind_a == kSideArtic ? 0u : 1u;
             c.F(hRho, h) = rho; c.F(hCompliance, h) = compliance; c.F(hLower, h) = row[6]; c.F(hUpper, h) = row[7];
-            c.F(hMu1, h) = row[8]; c.F(hMu2, h) = row[9]; c.F(hNormalBound, h) = 0.0f;
+            c.F(hMu1, h) = joint ? 0.0f : row[8]; c.F(hMu2, h) = joint ? 0.0f : row[9]; c.F(hNormalBound, h) = 0.0f;
             c.F(hDualScale, h) = sr.dual_scale; c.F(hResidualScale, h) = sr.residual_scale;
             const float dx = lambda_env[local], dy = axes == 3u ? lambda_env[local + stride] : 0.0f,
                         dz = axes == 3u ? lambda_env[local + 2u * stride] : 0.0f;
@@ -3246,7 +3259,7 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
         __syncthreads();
         bool push = false;
         for (uint32_t h = lane; h < heads; h += kWave) {
-            const uint32_t slot = c.U(hSlot, h);
+            const uint32_t slot = c.slot(h);
             const float* row = urows + size_t{slot} * kRowWords;
             const uint32_t flags = __float_as_uint(row[0]);
             const float penetration = d.row_penetration[slot];
@@ -3290,7 +3303,7 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
                     bias = fminf(correction / p.dt, p.position_max_velocity);
                 }
             }
-            if (!position) c.U(hOwned, h) = 0u;
+            if (!position) c.U(hSlot, h) = slot | kUnowned;
             const Response sr = scalar_response(c.F(hRho, h), 0.0f);
             c.U(hAxes, h) = 1u;
             c.F(hCompliance, h) = 0.0f; c.F(hLower, h) = 0.0f; c.F(hUpper, h) = FLT_MAX;
