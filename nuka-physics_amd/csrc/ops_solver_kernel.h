@@ -336,6 +336,7 @@ struct Tile {
     bool elliptic;   // some head is under the elliptic cone: every response goes through the general functions
     bool units;      // some head is a unit head
     bool scalar_later;   // the heads past the first 64 are on one axis, and two a lane hold them
+    bool block_heads;   // every staged head of the first 64 has three axes and reaches no further than the first columns (add_block_heads)
     bool near_heads; // no staged head's rows reach past the coordinates two tiles hold (add_heads_by_tiles)
     bool unit_lists; // every coordinate's unit heads fit its list
     uint16_t* unit_list;      // kUnitSlots x 64: lane's unit heads in head order, slot-major
@@ -661,14 +662,18 @@ __device__ __forceinline__ float solve_tile_mass(const Tile& c, float force) {
 // head's words come in one round trip of fifteen four-byte reads; written as vector code the columns took four times
 // the arithmetic and a wait for three sixteen-byte reads each (12 heads of 20 columns: 5.7 k cycles a Newton step).
 template <int N>
-__device__ __forceinline__ void add_columns(int q, const float* rows, float a0, float a1, float a2, float (&hrow)[N]) {
-    const float* x = rows + 4 * q;
+__device__ __forceinline__ void add_columns(int q, float x0, float x1, float x2, float a0, float a1, float a2, float (&hrow)[N]) {
     Vec4 term = {};
-    term = __builtin_amdgcn_mfma_f32_4x4x1f32(x[0], a0, term, 0, 0, 0);
-    term = __builtin_amdgcn_mfma_f32_4x4x1f32(x[N], a1, term, 0, 0, 0);
-    term = __builtin_amdgcn_mfma_f32_4x4x1f32(x[2 * N], a2, term, 0, 0, 0);
+    term = __builtin_amdgcn_mfma_f32_4x4x1f32(x0, a0, term, 0, 0, 0);
+    term = __builtin_amdgcn_mfma_f32_4x4x1f32(x1, a1, term, 0, 0, 0);
+    term = __builtin_amdgcn_mfma_f32_4x4x1f32(x2, a2, term, 0, 0, 0);
 #pragma unroll
     for (int r = 0; r < 4; ++r) hrow[4 * q + r] += term[r];
+}
+template <int N>
+__device__ __forceinline__ void add_columns(int q, const float* rows, float a0, float a1, float a2, float (&hrow)[N]) {
+    const float* x = rows + 4 * q;
+    add_columns<N>(q, x[0], x[N], x[2 * N], a0, a1, a2, hrow);
 }
 // the same for a head on one axis, straight into the row
 template <int N>
@@ -903,6 +908,62 @@ __device__ __forceinline__ void add_heads_by_tiles(const Tile& c, uint64_t heads
     const float bound_sum = halves_sum(bound_low + bound_high);
     g.value += reached ? force_sum : 0.0;
     scale += reached ? bound_sum : 0.0f;
+}
+
+// The same as add_head for the heads of `heads` (a uniform mask of the first 64), in head order, where all of them have three
+// axes and reach no further than the first columns (Tile::block_heads): nothing is asked of a head, and the next one's words
+// are on their way while this one's are worked on.  About half of add_head's instructions, which with its three waits made
+// 1.1 k cycles a head: 1000 servo-driven humanoids 1262 -> 1210 us a step, 4096 1432 -> 1409.
+template <int N>
+__device__ __forceinline__ void add_block_heads(const Tile& c, uint64_t heads, bool coordinate, const float (&mf)[3], const float (&mc)[6], const float (&mn)[3],
+                                                uint32_t my_first, float (&hrow)[N], TileSum& g, float& scale) {
+    constexpr int kFirst = kFirstColumns<N>;
+    const uint32_t column = min(c.lane, uint32_t(N - 1));
+    struct Words { float own[3], x[kFirst][3]; };
+    auto fetch = [&](uint32_t h) {
+        const float* rows = c.jac + uint32_t(__builtin_amdgcn_readlane(int(my_first), int(h))) * uint32_t(N);
+        Words w;
+#pragma unroll
+        for (int k = 0; k < 3; ++k) w.own[k] = rows[uint32_t(k * N) + column];
+#pragma unroll
+        for (int q = 0; q < kFirst; ++q)
+#pragma unroll
+            for (int k = 0; k < 3; ++k) w.x[q][k] = rows[uint32_t(k * N + 4 * q) + (c.lane & 3u)];
+        return w;
+    };
+    // (widened once: a lane's two words are read for a conversion a head, which takes four times an instruction's time)
+    const double wide[3] = {double(mf[0]), double(mf[1]), double(mf[2])};
+    auto force_of = [&](int k, uint32_t h) {
+        const uint64_t bits = uint64_t(__double_as_longlong(wide[k]));
+        const uint32_t low = uint32_t(__builtin_amdgcn_readlane(int(uint32_t(bits)), int(h))), high = uint32_t(__builtin_amdgcn_readlane(int(uint32_t(bits >> 32u)), int(h)));
+        return __longlong_as_double((long long)((uint64_t(high) << 32u) | uint64_t(low)));
+    };
+    auto value_of = [&](float v, uint32_t h) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), int(h))); };
+    uint32_t h = uint32_t(__builtin_ctzll(heads));
+    Words next = fetch(h);
+#pragma unroll 1
+    for (;;) {
+        heads &= heads - 1ull;
+        const Words w = next;
+        const uint32_t after = heads != 0ull ? uint32_t(__builtin_ctzll(heads)) : h;
+        next = fetch(after);
+        float j[3];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            j[k] = coordinate ? w.own[k] : 0.0f;
+            g.value = fma(double(j[k]), force_of(k, h), g.value);
+        }
+        scale += fabsf(j[0]) * value_of(mn[0], h);
+        scale += fabsf(j[1]) * value_of(mn[1], h) + fabsf(j[2]) * value_of(mn[2], h);
+        const float cxx = value_of(mc[0], h), cyy = value_of(mc[1], h), czz = value_of(mc[2], h), cxy = value_of(mc[3], h), cxz = value_of(mc[4], h), cyz = value_of(mc[5], h);
+        const float a0 = (j[0] * cxx + j[1] * cxy) + j[2] * cxz;
+        const float a1 = (j[1] * cyy + j[2] * cyz) + j[0] * cxy;
+        const float a2 = (j[2] * czz + j[1] * cyz) + j[0] * cxz;
+#pragma unroll
+        for (int q = 0; q < kFirst; ++q) add_columns<N>(q, w.x[q][0], w.x[q][1], w.x[q][2], a0, a1, a2, hrow);
+        if (heads == 0ull) break;
+        h = after;
+    }
 }
 
 // A reduced block adds its heads to register rows instead, in an order of its own (below): its worlds are robots on two
@@ -1615,6 +1676,9 @@ __device__ __forceinline__ bool assemble_block(const Tile& c, const float (&mrow
                     else add_heads_by_tiles<N, true>(c, staged, mf, mc, mn, my_first, hrow, g, scale);
                 }
             }
+        } else if (N <= kTwoWaveWidth && c.block_heads) {
+            if constexpr (N <= kTwoWaveWidth)
+                if (staged != 0ull) add_block_heads<N>(c, staged, coordinate, mf, mc, mn, c.U(hRow, lane < c.heads ? lane : 0u), hrow, g, scale);
         } else {
             const uint32_t own_head = lane < c.heads ? lane : 0u;
             const uint32_t my_axes = c.U(hAxes, own_head), my_low = c.U(hColumnsLow, own_head), my_high = c.U(hColumnsHigh, own_head);
@@ -2592,7 +2656,7 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
     Tile c;
     c.env = env; c.lane = lane; c.n = kReduced ? uint32_t(K) : n; c.n_all = n; c.ldj = uint32_t(W); c.cap = cap; c.narrow = staged_cap; c.heads = 0u; c.iteration = 0u;
     c.tolerance = p.velocity_tolerance; c.failed = false; c.momentum = 0.0f; c.residual = 0.0f;
-    c.scalar_later = false; c.near_heads = false; c.mass_inverse = 0.0f; c.mass_valid = false; c.work = 0u; c.units = false; c.elliptic = false;
+    c.scalar_later = false; c.near_heads = false; c.block_heads = false; c.mass_inverse = 0.0f; c.mass_valid = false; c.work = 0u; c.units = false; c.elliptic = false;
     c.factor_current = false; c.rows_current = false; c.factor_root = 1.0f;
     for (float& entry : c.curvature) entry = 0.0f;
 #ifdef NKH_SOLVER_PROFILE
@@ -3165,6 +3229,12 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
     }
     c.elliptic = !kContactsOnly && __any(any_elliptic);
     __syncthreads();
+    {
+        const uint32_t own = min(lane, heads == 0u ? 0u : heads - 1u);
+        const bool staged = lane < heads && c.U(hRow, own) != kInvalid;
+        const bool within = block_axes(c.U(hAxes, own)) && c.U(hColumnsHigh, own) == 0u && (uint64_t(c.U(hColumnsLow, own)) >> (4 * kFirstColumns<W>)) == 0ull;
+        c.block_heads = !__any(staged && !within);
+    }
     bool later_axes = false;   // a later head on more axes than one
     for (uint32_t h = lane + kWave; h < heads; h += kWave) later_axes = later_axes || c.U(hAxes, h) != 1u;
     c.scalar_later = !kContactsOnly && !c.elliptic && heads > uint32_t(kWave) && heads <= uint32_t(kWave) * (kLaterHeads + 1u) && !__any(later_axes);
@@ -3313,6 +3383,7 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
             push = push || bias > rounding;
         }
         push = __any(push);
+        c.block_heads = false;   // on one axis now
         __syncthreads();
         float pseudo = 0.0f;
         if (push) {
