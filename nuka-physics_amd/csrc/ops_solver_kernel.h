@@ -354,7 +354,8 @@ struct Tile {
     uint32_t path_low, path_high;     // lane = coordinate: the coordinates on the way from its link to the root, itself included
     uint32_t under_low, under_high;   // the coordinates whose way to the root passes through lane's
     uint32_t over_low, over_high;     // the heads whose way to the root passes through lane's coordinate
-    bool over_runs;                   // those are neighbours in the list of heads, for every coordinate
+    bool over_runs;                   // those are neighbours in the list of heads, for every coordinate (a chain, or limbs in turn)
+    bool way_runs;                    // and every head's way to the root is a run of coordinates (a chain)
     float* spread;            // from_links: 8 x 68 words, what the lanes hand each other as heads and take as coordinates
     float* motions;           // from_links: 8 x 68 words, the coordinates' motion axes once more, component by component (two of them idle)
     mutable bool stiffness_current;   // no head's curvature has changed since the stiffness in `axes` was summed
@@ -1312,11 +1313,65 @@ __device__ __forceinline__ void add_heads_force(const Tile& c, uint64_t heads, c
     }
 }
 
+// Sums over runs of neighbouring lanes, as differences of the running sum over the wavefront, in double.  A running sum takes
+// eighteen instructions, where the sum of every lane's own choice of 64 takes three a lane: a step of 8192 ropes 15.98 ->
+// 13.64 ms with the force so (rows_transposed_times), where the heads past every coordinate are neighbours in their list
+// (Tile::over_runs), and 13.64 -> 13.31 with the motion of the links (link_motion), where every way to the root is a run of
+// coordinates.  The motions are rounded once where 64 single-precision multiply-adds were; how near a step ends to a
+// double-precision solve is the same (12288 environments: 0.993 +- 0.011 and 1.001 +- 0.007 of the mean errors before).
+template <int Ctrl, int Rows>
+__device__ __forceinline__ double dpp_rows_d(double v) {   // lanes without a source, and rows outside the mask, get zero
+    const uint64_t bits = uint64_t(__double_as_longlong(v));
+    const uint32_t low = uint32_t(__builtin_amdgcn_update_dpp(0, int(uint32_t(bits)), Ctrl, Rows, 0xF, true));
+    const uint32_t high = uint32_t(__builtin_amdgcn_update_dpp(0, int(uint32_t(bits >> 32u)), Ctrl, Rows, 0xF, true));
+    return __longlong_as_double((long long)((uint64_t(high) << 32u) | uint64_t(low)));
+}
+__device__ __forceinline__ double running_sum(double v) {
+    v += dpp_rows_d<0x111, 0xF>(v); v += dpp_rows_d<0x112, 0xF>(v); v += dpp_rows_d<0x114, 0xF>(v); v += dpp_rows_d<0x118, 0xF>(v);   // within sixteen lanes
+    v += dpp_rows_d<0x142, 0xA>(v);   // lane 15 of a row to the next row,
+    v += dpp_rows_d<0x143, 0xC>(v);   // lane 31 to the upper two
+    return v;
+}
+__device__ __forceinline__ bool one_run(uint64_t lanes) {
+    const uint64_t from = lanes == 0ull ? 0ull : lanes >> __builtin_ctzll(lanes);
+    return (from & (from + 1ull)) == 0ull;
+}
+struct LaneRun {   // the lanes of a mask that are one run
+    bool some, from_start;
+    int before, last;      // byte addresses (4 x lane) of the lane ahead of the run and of its last
+    __device__ __forceinline__ LaneRun(uint32_t low, uint32_t high) {
+        const uint64_t lanes = (uint64_t(high) << 32u) | uint64_t(low);
+        some = lanes != 0ull;
+        const uint32_t first = some ? uint32_t(__builtin_ctzll(lanes)) : 0u, end = some ? 64u - uint32_t(__builtin_clzll(lanes)) : 1u;
+        from_start = first == 0u;
+        before = int(4u * (from_start ? 0u : first - 1u)); last = int(4u * (end - 1u));
+    }
+    __device__ __forceinline__ double sum(double v) const {
+        const uint64_t bits = uint64_t(__double_as_longlong(running_sum(v)));
+        auto at = [&](int source) {
+            const uint32_t low = uint32_t(__builtin_amdgcn_ds_bpermute(source, int(uint32_t(bits)))), high = uint32_t(__builtin_amdgcn_ds_bpermute(source, int(uint32_t(bits >> 32u))));
+            return __longlong_as_double((long long)((uint64_t(high) << 32u) | uint64_t(low)));
+        };
+        const double through = at(last), ahead = at(before);
+        return some ? (from_start ? through : through - ahead) : 0.0;
+    }
+};
+
 // Blocks that keep no contact rows (Tile::from_links).  Entry j of a head's row is s_j . w where j lies on the head's
 // way to the root, s_j the coordinate's motion axis (Tile::axes) and w the row's wrench (Tile::wrench); elsewhere zero.
 // lane = head: the motion of the head's link, sum over the coordinates j on its way of s_j x_j, for a vector x in LDS.
 template <int N>
 __device__ __forceinline__ void link_motion(const Tile& c, uint64_t way, const float* x, float (&motion)[6]) {
+    if (c.way_runs) {
+        const LaneRun run(uint32_t(way), uint32_t(way >> 32u));
+        const float4* table = reinterpret_cast<const float4*>(c.axes);
+        const float4 a = table[3u * c.lane], b = table[3u * c.lane + 1u];
+        const float s[6] = {a.x, a.y, a.z, a.w, b.x, b.y};
+        const double own = double(x[c.lane]);   // (a lane past the coordinates holds zeros on both sides)
+#pragma unroll
+        for (int k = 0; k < 6; ++k) motion[k] = float(run.sum(double(s[k]) * own));
+        return;
+    }
     // Every lane of the wavefront, those without a head with a way of none: v_mfma_f32_4x4x1 takes a coordinate's axis, a
     // component a lane of four, against the lane's own weight, and register r of a lane is the sum of component r - the
     // multiply-adds that six vector instructions and two sixteen-byte reads a coordinate made before, bit for bit.
@@ -1383,43 +1438,6 @@ __device__ __forceinline__ void sums_over_ways(const Tile& c, uint64_t heads, co
         __syncthreads();
     }
 }
-// Sums over the heads whose way holds a coordinate, where those heads are neighbours for every coordinate (Tile::over_runs:
-// contacts listed along a chain, or limb by limb): differences of the running sums over the lanes, in double.  A running sum
-// takes eighteen instructions a component where the sum of every lane's own choice of 64 took three a head: a step of 8192
-// ropes 15.98 -> 13.64 ms.
-template <int Ctrl, int Rows>
-__device__ __forceinline__ double dpp_rows_d(double v) {   // lanes without a source, and rows outside the mask, get zero
-    const uint64_t bits = uint64_t(__double_as_longlong(v));
-    const uint32_t low = uint32_t(__builtin_amdgcn_update_dpp(0, int(uint32_t(bits)), Ctrl, Rows, 0xF, true));
-    const uint32_t high = uint32_t(__builtin_amdgcn_update_dpp(0, int(uint32_t(bits >> 32u)), Ctrl, Rows, 0xF, true));
-    return __longlong_as_double((long long)((uint64_t(high) << 32u) | uint64_t(low)));
-}
-__device__ __forceinline__ double running_sum(double v) {
-    v += dpp_rows_d<0x111, 0xF>(v); v += dpp_rows_d<0x112, 0xF>(v); v += dpp_rows_d<0x114, 0xF>(v); v += dpp_rows_d<0x118, 0xF>(v);   // within sixteen lanes
-    v += dpp_rows_d<0x142, 0xA>(v);   // lane 15 of a row to the next row,
-    v += dpp_rows_d<0x143, 0xC>(v);   // lane 31 to the upper two
-    return v;
-}
-struct HeadRun {
-    bool some, from_start;
-    int before, last;      // byte addresses (4 x lane) of the lane ahead of the run and of its last
-    __device__ __forceinline__ explicit HeadRun(const Tile& c) {
-        const uint64_t heads = (uint64_t(c.over_high) << 32u) | uint64_t(c.over_low);
-        some = heads != 0ull;
-        const uint32_t first = some ? uint32_t(__builtin_ctzll(heads)) : 0u, end = some ? 64u - uint32_t(__builtin_clzll(heads)) : 1u;
-        from_start = first == 0u;
-        before = int(4u * (from_start ? 0u : first - 1u)); last = int(4u * (end - 1u));
-    }
-    __device__ __forceinline__ double sum(double v) const {
-        const uint64_t bits = uint64_t(__double_as_longlong(running_sum(v)));
-        auto at = [&](int source) {
-            const uint32_t low = uint32_t(__builtin_amdgcn_ds_bpermute(source, int(uint32_t(bits)))), high = uint32_t(__builtin_amdgcn_ds_bpermute(source, int(uint32_t(bits >> 32u))));
-            return __longlong_as_double((long long)((uint64_t(high) << 32u) | uint64_t(low)));
-        };
-        const double through = at(last), ahead = at(before);
-        return some ? (from_start ? through : through - ahead) : 0.0;
-    }
-};
 // lane = coordinate: sum over the heads `heads` (a uniform mask of the first 64) of J^T x, x one value an axis held by
 // lane = head, in double: the heads' wrenches weighted by x summed over the heads whose way holds the coordinate, then
 // taken against the coordinate's motion axis.  With `weights` (the magnitudes that go with x) also the rounding scale
@@ -1439,7 +1457,7 @@ __device__ __forceinline__ double rows_transposed_times(const Tile& c, uint64_t 
     double carried[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
     Vec4 carried_bound[2] = {};
     if (c.over_runs) {
-        const HeadRun run(c);
+        const LaneRun run(c.over_low, c.over_high);
 #pragma unroll
         for (int k = 0; k < 6; ++k) carried[k] = run.sum(double(sum[k]));
         if constexpr (kScale) {
@@ -2740,7 +2758,7 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
     if (lane < kNarrowFields) c.fields[kWideStride * cap + staged_cap * kNarrowStride + lane] = 0.0f;   // what a narrow field reads beyond its heads
     c.unit_list = reinterpret_cast<uint16_t*>(c.vec + 256);
     c.unit_lists = true; c.unit_count = 0u; c.unit_most = 0u; c.staged_end = 0u; c.individual_end = 0u;
-    c.through_links = false; c.over_runs = false;
+    c.through_links = false; c.over_runs = false; c.way_runs = false;
     c.axes = c.vec + 256 + UnitListFloats(cap, staged_cap);   // a wide block's; a narrow one keeps rows here
     c.spread = c.axes + 12u * uint32_t(kWave);   // a block without contact rows has it, and the next
     c.motions = c.spread + 8u * kMotionStride;
@@ -2943,8 +2961,8 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
         }
         c.under_low = uint32_t(under); c.under_high = uint32_t(under >> 32u);
         c.over_low = uint32_t(over); c.over_high = uint32_t(over >> 32u);
-        const uint64_t run = over == 0ull ? 0ull : over >> __builtin_ctzll(over);
-        c.over_runs = __all((run & (run + 1ull)) == 0ull);
+        c.over_runs = __all(one_run(over));
+        c.way_runs = __all(one_run(head_way));
         // every staged head with exactly one side that moves
         bool one_link = true;
         if (lane < heads) {
