@@ -936,23 +936,26 @@ __device__ __forceinline__ float uniform_value(float v, uint32_t lane) {   // `l
 }
 
 // ---- AssembleRows: one wavefront per environment (assemble_rows.cu:325-394, 200-214, 406-801, 122-186) ----
-// four waves a SIMD (128 registers a lane): sixteen environments a compute unit are resident at once at 4096 environments
-__global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(4, 4))) AssembleRowsKernel(ModelView m, DataView d, AssembleRowsParams p) {
-    extern __shared__ uint32_t lds_u[];
+// A lane a contact point, 64 points at a time: it writes the point's rows, and then the points go by in turn, lane = DoF,
+// with what their rows share - links, point, directions - handed round as lane reads, so that the moment arm of a point is
+// formed once for its rows and nothing of a row waits in LDS (ten words a row slot were 42 KB of it for 64 slots, three
+// blocks a compute unit).  Two instantiations: worlds without compliant contacts need neither their spring-dampers and pyramids
+// nor the registers these take, and run six waves a SIMD where the others run four.
+__host__ __device__ inline uint32_t AssembleTermStride(uint32_t md) { return md | 1u; }   // rows of terms in different banks
+constexpr uint32_t kTermRows = 32u;   // sixteen rows, both sides
+__host__ __device__ inline uint32_t AssembleLdsWords(uint32_t slots, uint32_t links, uint32_t md, bool compliant) {
+    return 2u * slots + 2u * links + (compliant ? kTermRows * AssembleTermStride(md) : 0u);
+}
+template <bool kCompliant>
+__global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(kCompliant ? 4 : 6, kCompliant ? 4 : 6))) AssembleRowsKernel(ModelView m, DataView d, AssembleRowsParams p) {
+    extern __shared__ __align__(8) uint32_t lds_u[];
     const uint32_t env = blockIdx.x, lane = threadIdx.x;
     const uint32_t R = p.rows_per_env, S = p.union_slot_count, CR = p.contact_rows_per_env, md = p.max_dof, nl = m.links_per_env;
-    uint32_t* range_first = lds_u;        // S
-    uint32_t* range_points = lds_u + S;   // S
-    // what the chain Jacobian pass needs of each row, kept here so that it does not read back what this block wrote
-    uint32_t* row_link_a = lds_u + 2u * S;             // CR (contact rows only; joint rows need no chain walk)
-    uint32_t* row_link_b = row_link_a + CR;             // CR
-    uint32_t* row_merge = row_link_b + CR;              // CR: both sides articulated with the same owner
-    float* row_point = reinterpret_cast<float*>(row_merge + CR);   // 3 CR
-    float* row_dir = row_point + 3u * CR;                // 3 CR, side A's direction (side B's is its negative)
-    float* row_gain = row_dir + 3u * CR;                 // CR: a compliant row's gain on the start velocity along it, else 0
-    // nl: the coordinates on each link's path to the root (2 S + 10 CR words come before: an even count, so 8-byte aligned);
-    // the chain Jacobian pass asks for a link's mask once a row and side and would wait on the table each time
-    uint64_t* link_mask = reinterpret_cast<uint64_t*>(row_gain + CR);
+    // nl: the coordinates on each link's path to the root; a point asks for its links' masks and would wait on the table each time
+    uint64_t* link_mask = reinterpret_cast<uint64_t*>(lds_u);
+    uint32_t* range_first = lds_u + 2u * nl;   // S
+    uint32_t* range_points = range_first + S;   // S
+    float* terms = reinterpret_cast<float*>(range_points + S);   // kTermRows rows of what a compliant row's start velocity sums
     for (uint32_t l = lane; l < nl; l += kWave) link_mask[l] = m.link_dof_mask[l];
     Row* rows = reinterpret_cast<Row*>(d.urows) + size_t{env} * R;
     float* lambda = d.lambda + size_t{env} * R;
@@ -962,6 +965,7 @@ __global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(4, 4
     // row ranges: exclusive prefix of the slots' point counts, four rows a point (:336-360)
     const uint32_t previous_extent = d.contact_row_extent[2u * env + 1u];
     uint32_t carry = 0u, extent = 1u;
+    bool many = false;   // some slot has more than one point
     for (uint32_t base = 0u; base < S; base += kWave) {
         const uint32_t slot = base + lane;
         const uint32_t points = slot < S ? d.ucontact_count[size_t{env} * S + slot] : 0u;
@@ -974,6 +978,7 @@ __global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(4, 4
         if (slot < S) {
             const uint32_t first = (carry + through - points) * kRowsPerPoint;
             range_first[slot] = first; range_points[slot] = points;
+            many = many || points > 1u;
             d.ucontact_row_range[(size_t{env} * S + slot) * 2u] = env * R + first;
             d.ucontact_row_range[(size_t{env} * S + slot) * 2u + 1u] = points;
             if (first < contact_row_bound(previous_extent, 1u, CR)) d.contact_material[size_t{env} * S + slot] = 0ull;   // :358
@@ -994,7 +999,6 @@ __global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(4, 4
         pen[local] = 0.0f; cj_link[local] = kInvalid; cj_link_b[local] = kInvalid;
         rows[local].flags = 0u;
     }
-    for (uint32_t local = lane; local < CR; local += kWave) { row_link_a[local] = kInvalid; row_link_b[local] = kInvalid; row_merge[local] = 0u; row_gain[local] = 0.0f; }
     if (lane == 0u) {
         d.contact_row_extent[2u * env] = previous_extent;
         d.contact_row_extent[2u * env + 1u] = extent;
@@ -1010,17 +1014,59 @@ __global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(4, 4
         d.qdot_flat[size_t{env} * md + lane] = value;
     }
     __syncthreads();
+    // lane = DoF: the coordinate's axis, where it lies and whether it turns
+    V3 axis_world{0, 0, 0}, origin{0, 0, 0};
+    uint32_t mode = 0u;   // 0 none, 1 revolute, 2 prismatic, 3 base angular, 4 base linear
+    if (lane < m.dof) {
+        const uint32_t link = m.dof_link[lane], component = m.dof_component[lane];
+        if (component == kInvalid) {
+            const Xf pose = load_xf(d.link_pose + (size_t{env} * nl + link) * 7u);
+            axis_world = rotate_normalized(pose.r, V3{m.joint_axis[3u * link], m.joint_axis[3u * link + 1u], m.joint_axis[3u * link + 2u]});
+            origin = pose.p;
+            mode = m.joint_type[link] == kPrismatic ? 2u : 1u;
+        } else {
+            const Xf base = load_xf(d.base_pose + size_t{env} * 7u);
+            const uint32_t k = component % 3u;
+            const V3 unit{k == 0u ? 1.0f : 0.0f, k == 1u ? 1.0f : 0.0f, k == 2u ? 1.0f : 0.0f};
+            if (m.free_body != 0u) {
+                // a free body's coordinates: linear velocity, then angular velocity about the centre of mass, world axes -
+                // the row's jlin and jang = (point - com) x jlin (assemble_rows.cu:537-538, 680-681)
+                axis_world = unit;
+                const float* frame = d.body_inertial_frame + (size_t{env} * m.bodies_per_env + m.link_body[0]) * 7u;
+                origin = add3(base.p, rotate_normalized(base.r, V3{frame[0], frame[1], frame[2]}));
+                mode = component < 3u ? 4u : 3u;
+            } else {
+                axis_world = rotate_normalized(base.r, unit);
+                origin = base.p;
+                mode = component < 3u ? 3u : 4u;
+            }
+        }
+    }
+    const float start_velocity = kCompliant && m.any_mujoco != 0u && lane < md ? d.step_qdot_flat[size_t{env} * md + lane] : 0.0f;
+    auto uniform_word = [](uint32_t v, uint32_t from) { return uint32_t(__builtin_amdgcn_readlane(int(v), int(from))); };
     // contact rows (:453-801; speculative law, condim 3): a lane a slot where every slot has one point at most, else a
     // lane a (slot, point) - a slot's points share nothing but the slot's own values, which each of their lanes works
     // out for itself
     uint32_t active_rows = 0u;
     bool invalid_endpoint = false;
-    const uint32_t fan = m.max_points_per_slot > 1u ? 4u : 1u;
-    for (uint32_t item = lane; item < S * fan; item += kWave) {
+    const uint32_t fan = __any(many) ? 4u : 1u;
+    constexpr int kAxes = kCompliant ? 4 : 3;   // rows a point
+    for (uint32_t chunk = 0u; chunk < S * fan; chunk += kWave) {
+        // what the chain Jacobians need of lane's point: its first row and the stride of its rows, which of them it has, its
+        // links, whether they have one owner, the point, the rows' directions (side A's; side B's are their negatives) and
+        // a compliant row's gain on the start velocity along it
+        uint32_t my_row = 0u, my_stride = 0u, my_axes = 0u, my_link[2] = {kInvalid, kInvalid}, my_merge = 0u;
+        V3 my_point{0, 0, 0}, my_dir[kAxes];
+        float my_gain[kAxes], my_rhs[kAxes];
+#pragma unroll
+        for (int axis = 0; axis < kAxes; ++axis) { my_dir[axis] = V3{0, 0, 0}; my_gain[axis] = 0.0f; my_rhs[axis] = 0.0f; }
+        const auto emit_point = [&]() {
+        const uint32_t item = chunk + lane;
+        if (item >= S * fan) return;
         const uint32_t slot = item / fan, own_point = item - slot * fan;
         const size_t gid = size_t{env} * S + slot;
         const uint32_t base = range_first[slot], P = range_points[slot];
-        if (P == 0u || (fan > 1u && own_point >= P)) continue;
+        if (own_point >= P) return;
         const bool slot_lane = own_point == 0u;   // the one lane that writes what belongs to the slot as a whole
         uint32_t n_active = P;
         const uint32_t local_a = d.ucontact_a[gid * 4u], local_b = d.ucontact_b[gid * 4u];
@@ -1039,7 +1085,7 @@ __global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(4, 4
         if (kind_b == kSideStatic) idx_b = kInvalid;
         // the two sides' profiles merged (:540-594; scene/contact_filter.hpp:100-137); a side without one has the defaults
         const uint32_t law = d.ucontact_law[gid];
-        const bool mujoco = law == kContactLawCompliant;   // :480
+        const bool mujoco = kCompliant && law == kContactLawCompliant;   // :480
         float side_a[14], side_b[14], merged[12];
         profile_terms(m, sa.profile, side_a); profile_terms(m, sb.profile, side_b);
         merge_contact_params(side_a, side_b, merged);
@@ -1062,7 +1108,8 @@ __global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(4, 4
         V3 frame_axis{0, 0, 0};   // :601-605: a capsule on a plane aligns the pyramid with the capsule's axis
         if (pyramidal && sa.kind == 1u && sb.kind == 3u) frame_axis = make_prim(sa, load_xf(d.body_pose + (size_t{env} * m.bodies_per_env + local_a) * 7u)).cz;
         if (pyramidal && sb.kind == 1u && sa.kind == 3u) frame_axis = make_prim(sb, load_xf(d.body_pose + (size_t{env} * m.bodies_per_env + local_b) * 7u)).cz;
-        for (uint32_t pt = fan > 1u ? own_point : 0u; pt < (fan > 1u ? own_point + 1u : P); ++pt) {
+        {
+            const uint32_t pt = own_point;
             const size_t mp = gid * 4u + pt;
             // the velocity laws keep every point; a compliant point lives inside its margin (:625-626)
             const bool live = pt < n_active && pt < 4u && (!mujoco || d.ucontact_depth[mp] + margin > 0.0f);
@@ -1076,7 +1123,7 @@ __global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(4, 4
                 const float len = sqrtf(raw.x * raw.x + raw.y * raw.y + raw.z * raw.z);
                 n = len < 1e-12f ? V3{0, 0, 0} : V3{raw.x / len, raw.y / len, raw.z / len};
                 point = V3{d.ucontact_point[3u * mp], d.ucontact_point[3u * mp + 1u], d.ucontact_point[3u * mp + 2u]};
-                if (pyramidal) mujoco_contact_frame(raw, frame_axis, &t0, &t1);
+                if (kCompliant && pyramidal) mujoco_contact_frame(raw, frame_axis, &t0, &t1);
                 else contact_tangent_basis(raw, &t0, &t1);
                 d0 = d.ucontact_depth[mp];
             }
@@ -1092,10 +1139,15 @@ __global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(4, 4
                 dir0 = add3(n, scale3(t0, mu1)); dir1 = add3(n, scale3(t0, -mu1));
                 dir2 = add3(n, scale3(t1, mu2)); dir3 = add3(n, scale3(t1, -mu2));
             } else { dir0 = n; dir1 = t0; dir2 = t1; }
+            my_row = base + pt; my_stride = P; my_point = point;
+            if (kind_a == kSideArtic) my_link[0] = link_a;
+            if (kind_b == kSideArtic) my_link[1] = link_b;
+            my_merge = kind_a == kSideArtic && kind_b == kSideArtic && idx_a == idx_b ? 1u : 0u;
+            my_dir[0] = dir0; my_dir[1] = dir1; my_dir[2] = dir2;
+            if constexpr (kCompliant) my_dir[kAxes - 1] = pyramidal ? dir3 : dir2;
             for (uint32_t axis = 0u; axis < row_count; ++axis) {
                 const uint32_t rs = base + axis * P + pt;
                 lambda[rs] = 0.0f; pen[rs] = 0.0f; cj_link[rs] = kInvalid; cj_link_b[rs] = kInvalid;
-                row_gain[rs] = 0.0f;
                 if (!(pyramidal ? live : emits[axis == 0u ? 0 : 1])) {
                     if (pyramidal) rows[rs] = Row{}; else rows[rs].flags = 0u;
                     continue;
@@ -1148,19 +1200,104 @@ __global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(4, 4
                 if (mujoco) {
                     d.row_reference_velocity_gain[size_t{env} * R + rs] = gain;
                     d.row_invweight[size_t{env} * R + rs] = weight;
-                    row_gain[rs] = gain;
                 }
-                row_point[3u * rs] = point.x; row_point[3u * rs + 1u] = point.y; row_point[3u * rs + 2u] = point.z;
-                row_dir[3u * rs] = dir.x; row_dir[3u * rs + 1u] = dir.y; row_dir[3u * rs + 2u] = dir.z;
-                if (kind_a == kSideArtic) row_link_a[rs] = link_a;
-                if (kind_b == kSideArtic) row_link_b[rs] = link_b;
-                row_merge[rs] = kind_a == kSideArtic && kind_b == kSideArtic && idx_a == idx_b ? 1u : 0u;
+                my_axes |= 1u << axis;
+#pragma unroll
+                for (int k = 0; k < kAxes; ++k)
+                    if (axis == uint32_t(k)) { my_gain[k] = gain; my_rhs[k] = row.rhs; }
                 if (kind_a == kSideArtic) { cj_link[rs] = link_a; cj_point[3u * rs] = point.x; cj_point[3u * rs + 1u] = point.y; cj_point[3u * rs + 2u] = point.z; }
                 if (kind_b == kSideArtic) { cj_link_b[rs] = link_b; cj_point_b[3u * rs] = point.x; cj_point_b[3u * rs + 1u] = point.y; cj_point_b[3u * rs + 2u] = point.z; }
                 rows[rs] = row;
                 ++active_rows;
             }
         }
+        };
+        emit_point();
+        if (md == 0u) continue;
+        // chain Jacobians, lane = DoF: every row entry is the joint's own column when the joint lies on the path from
+        // the row's link to the root, which the cooked per-link DoF mask answers (assemble_rows.cu:122-169,
+        // articulation_types.cuh:193-238); both sides, then the shared-owner merge (:172-186)
+        uint32_t my_mask[2][2] = {{0u, 0u}, {0u, 0u}};
+#pragma unroll
+        for (int side = 0; side < 2; ++side) {
+            if (my_link[side] == kInvalid) continue;
+            const uint64_t mask = link_mask[my_link[side] - env * nl];
+            my_mask[side][0] = uint32_t(mask); my_mask[side][1] = uint32_t(mask >> 32u);
+        }
+        uint32_t staged_terms = 0u;   // compliant rows whose terms stand in LDS
+        uint32_t term_row = kInvalid;   // lane = one of those: the row, its right-hand side and its gain
+        float term_rhs = 0.0f, term_gain = 0.0f;
+        bool term_sides[2] = {false, false};
+        // PrepareContactRowsKernel (:1134-1140): a compliant row's reference acceleration includes the damping of the velocity
+        // the step started from along the row, ContactReferenceVelocity (:1072-1100): side A's coordinates in order, then side
+        // B's.  Sixteen rows at a time, a lane a row.  (A lane read and a sum a coordinate and row took half of the kernel
+        // with 36 coordinates under the elliptic cone.)
+        auto add_velocities = [&]() {
+            __syncthreads();   // the rows, which other lanes wrote, and the terms stand
+            if (lane < staged_terms) {
+                float velocity = 0.0f;
+#pragma unroll
+                for (uint32_t side = 0u; side < 2u; ++side) {
+                    if (!term_sides[side]) continue;
+                    const float* own = terms + (16u * side + lane) * AssembleTermStride(md);
+                    for (uint32_t k = 0u; k < md; ++k) velocity += own[k];
+                }
+                rows[term_row].rhs = term_rhs + term_gain * velocity;
+            }
+            __syncthreads();
+            staged_terms = 0u;
+        };
+        for (uint64_t rest = __ballot(my_axes != 0u && (my_link[0] != kInvalid || my_link[1] != kInvalid)); rest != 0ull; rest &= rest - 1ull) {
+            const uint32_t i = uint32_t(__builtin_ctzll(rest));
+            const uint32_t links[2] = {uniform_word(my_link[0], i), uniform_word(my_link[1], i)}, axes = uniform_word(my_axes, i);
+            const uint32_t first_row = uniform_word(my_row, i), stride = uniform_word(my_stride, i), merge = uniform_word(my_merge, i);
+            const V3 point{uniform_value(my_point.x, i), uniform_value(my_point.y, i), uniform_value(my_point.z, i)};
+            const V3 arm = cross3(axis_world, sub3(point, origin));
+            bool on_path[2];
+#pragma unroll
+            for (int side = 0; side < 2; ++side) {
+                const uint64_t mask = (uint64_t(uniform_word(my_mask[side][1], i)) << 32u) | uint64_t(uniform_word(my_mask[side][0], i));
+                on_path[side] = lane < m.dof && ((mask >> lane) & 1ull) != 0ull;
+            }
+#pragma unroll
+            for (int axis = 0; axis < kAxes; ++axis) {
+                if (((axes >> axis) & 1u) == 0u) continue;
+                const V3 dir_a{uniform_value(my_dir[axis].x, i), uniform_value(my_dir[axis].y, i), uniform_value(my_dir[axis].z, i)};
+                float entries[2] = {0.0f, 0.0f};
+#pragma unroll
+                for (int side = 0; side < 2; ++side) {
+                    if (links[side] == kInvalid) continue;
+                    const V3 dir = side == 0 ? dir_a : V3{-dir_a.x, -dir_a.y, -dir_a.z};
+                    // a turning coordinate (hinge, base angular) takes the moment of the direction about its axis, a sliding
+                    // one (prismatic, base linear) the direction along it: both evaluated, one selected, so that lanes of
+                    // different kinds do not take turns
+                    const float turning = dot3(arm, dir) + dot3(axis_world, V3{0, 0, 0});
+                    const float sliding = dot3(axis_world, dir);
+                    entries[side] = !on_path[side] || mode == 0u ? 0.0f : ((mode & 1u) != 0u ? turning : sliding);
+                }
+                if (merge != 0u) { entries[0] += entries[1]; entries[1] = 0.0f; }   // shared owner (:172-186)
+                const uint32_t r = first_row + uint32_t(axis) * stride;
+                if (lane < md) {
+                    if (links[0] != kInvalid) d.chain_jacobian[(size_t{env} * R + r) * md + lane] = entries[0];
+                    if (links[1] != kInvalid) d.chain_jacobian_b[(size_t{env} * R + r) * md + lane] = entries[1];
+                }
+                if constexpr (kCompliant) {
+                    const float gain = uniform_value(my_gain[axis], i);
+                    if (gain == 0.0f) continue;
+                    if (lane < md) {
+#pragma unroll
+                        for (uint32_t side = 0u; side < 2u; ++side)
+                            terms[(16u * side + staged_terms) * AssembleTermStride(md) + lane] = entries[side] * start_velocity;
+                    }
+                    if (lane == staged_terms) {
+                        term_row = r; term_rhs = uniform_value(my_rhs[axis], i); term_gain = gain;
+                        term_sides[0] = links[0] != kInvalid; term_sides[1] = links[1] != kInvalid;
+                    }
+                    if (++staged_terms == kTermRows / 2u) add_velocities();
+                }
+            }
+        }
+        if (kCompliant && staged_terms != 0u) add_velocities();
     }
     // joint rows (EmitJointRowsKernel, assemble_rows.cu:803-1026): stable per-link slots after the contact rows - lower
     // and upper limit (two a link), dry friction, drive.  Each acts on one coordinate, J = +-e_joint; the rest of
@@ -1191,7 +1328,7 @@ __global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(4, 4
                     jacobian = side == 0u ? 1.0f : -1.0f;
                     pen[rs] = fmaxf(-signed_distance, 0.0f);
                     impulse = lambda[rs];   // an active limit row keeps its multiplier
-                    if (m.joint_law[l] == 1u) {   // :860-877: a compliant row inside its margin, on the nearer bound only
+                    if (kCompliant && m.joint_law[l] == 1u) {   // :860-877: a compliant row inside its margin, on the nearer bound only
                         const float pos = signed_distance - m.joint_limit_margin[l];
                         const float* reference = m.joint_limit_reference + 7u * l;
                         const float invweight = d.dof_invweight0[size_t{env} * md + m.link_dof[l]];
@@ -1210,7 +1347,7 @@ __global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(4, 4
                     row.flags = kRowActive | kRowVelocityOnly;
                     row.lower = -friction * p.dt; row.upper = friction * p.dt;
                     jacobian = 1.0f;
-                    if (m.joint_law[l] == 1u) {   // :921-931: dry friction regularised by its own solref / solimp
+                    if (kCompliant && m.joint_law[l] == 1u) {   // :921-931: dry friction regularised by its own solref / solimp
                         const float* reference = m.joint_friction_reference + 7u * l;
                         const float invweight = d.dof_invweight0[size_t{env} * md + m.link_dof[l]];
                         const CompliantRow c = compliant_row(reference, reference + 2u, 0.0f, 0.0f, 0.0f, invweight, p.dt, p.refsafe);
@@ -1254,101 +1391,6 @@ __global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(4, 4
     if (lane == 0u) {
         d.row_count[env] = active_rows;
         if (invalid_endpoint) d.env_status[env] |= kEnvStatusInvalidEndpoint;
-    }
-    __syncthreads();
-    // chain Jacobians, lane = DoF: every row entry is the joint's own column when the joint lies on the path from
-    // the row's link to the root, which the cooked per-link DoF mask answers (assemble_rows.cu:122-169,
-    // articulation_types.cuh:193-238); both sides, then the shared-owner merge (:172-186).
-    if (md == 0u) return;
-    V3 axis_world{0, 0, 0}, origin{0, 0, 0};
-    uint32_t mode = 0u;   // 0 none, 1 revolute, 2 prismatic, 3 base angular, 4 base linear
-    if (lane < m.dof) {
-        const uint32_t link = m.dof_link[lane], component = m.dof_component[lane];
-        if (component == kInvalid) {
-            const Xf pose = load_xf(d.link_pose + (size_t{env} * nl + link) * 7u);
-            axis_world = rotate_normalized(pose.r, V3{m.joint_axis[3u * link], m.joint_axis[3u * link + 1u], m.joint_axis[3u * link + 2u]});
-            origin = pose.p;
-            mode = m.joint_type[link] == kPrismatic ? 2u : 1u;
-        } else {
-            const Xf base = load_xf(d.base_pose + size_t{env} * 7u);
-            const uint32_t k = component % 3u;
-            const V3 unit{k == 0u ? 1.0f : 0.0f, k == 1u ? 1.0f : 0.0f, k == 2u ? 1.0f : 0.0f};
-            if (m.free_body != 0u) {
-                // a free body's coordinates: linear velocity, then angular velocity about the centre of mass, world axes -
-                // the row's jlin and jang = (point - com) x jlin (assemble_rows.cu:537-538, 680-681)
-                axis_world = unit;
-                const float* frame = d.body_inertial_frame + (size_t{env} * m.bodies_per_env + m.link_body[0]) * 7u;
-                origin = add3(base.p, rotate_normalized(base.r, V3{frame[0], frame[1], frame[2]}));
-                mode = component < 3u ? 4u : 3u;
-            } else {
-                axis_world = rotate_normalized(base.r, unit);
-                origin = base.p;
-                mode = component < 3u ? 3u : 4u;
-            }
-        }
-    }
-    // only the rows below this step's extent can have a link; the rows up to the previous extent were cleared above
-    const uint32_t bound = min(extent - 1u, CR);
-    const float start_velocity = m.any_mujoco != 0u && lane < md ? d.step_qdot_flat[size_t{env} * md + lane] : 0.0f;
-    // Sixty-four rows at a time: every lane first fetches one row's endpoints, point, direction, gain and its links' masks
-    // (one round of LDS reads, all in flight together), then the rows go by in turn with their values handed round as
-    // lane reads - a row no longer waits on its own chain of dependent reads.
-    auto uniform_word = [](uint32_t v, uint32_t from) { return uint32_t(__builtin_amdgcn_readlane(int(v), int(from))); };
-    for (uint32_t first = 0u; first < bound; first += kWave) {
-        const uint32_t mine = first + lane;
-        uint32_t my_link[2] = {kInvalid, kInvalid}, my_merge = 0u, my_mask[2][2] = {{0u, 0u}, {0u, 0u}};
-        float my_point[3] = {0.0f, 0.0f, 0.0f}, my_dir[3] = {0.0f, 0.0f, 0.0f}, my_gain = 0.0f;
-        if (mine < bound) {
-            my_link[0] = row_link_a[mine]; my_link[1] = row_link_b[mine]; my_merge = row_merge[mine]; my_gain = row_gain[mine];
-#pragma unroll
-            for (int k = 0; k < 3; ++k) { my_point[k] = row_point[3u * mine + k]; my_dir[k] = row_dir[3u * mine + k]; }
-#pragma unroll
-            for (int side = 0; side < 2; ++side) {
-                if (my_link[side] == kInvalid) continue;
-                const uint64_t mask = link_mask[my_link[side] - env * nl];
-                my_mask[side][0] = uint32_t(mask); my_mask[side][1] = uint32_t(mask >> 32u);
-            }
-        }
-        const uint32_t count = min(uint32_t(kWave), bound - first);
-        for (uint32_t i = 0u; i < count; ++i) {
-            const uint32_t r = first + i;
-            const uint32_t links[2] = {uniform_word(my_link[0], i), uniform_word(my_link[1], i)};
-            if (links[0] == kInvalid && links[1] == kInvalid) continue;
-            const V3 point{uniform_value(my_point[0], i), uniform_value(my_point[1], i), uniform_value(my_point[2], i)};
-            const V3 dir_a{uniform_value(my_dir[0], i), uniform_value(my_dir[1], i), uniform_value(my_dir[2], i)};
-            float entries[2] = {0.0f, 0.0f};
-#pragma unroll
-            for (int side = 0; side < 2; ++side) {
-                if (links[side] == kInvalid) continue;
-                const uint64_t mask = (uint64_t(uniform_word(my_mask[side][1], i)) << 32u) | uint64_t(uniform_word(my_mask[side][0], i));
-                const V3 dir = side == 0 ? dir_a : V3{-dir_a.x, -dir_a.y, -dir_a.z};
-                // a turning coordinate (hinge, base angular) takes the moment of the direction about its axis, a sliding
-                // one (prismatic, base linear) the direction along it: both evaluated, one selected, so that lanes of
-                // different kinds do not take turns
-                const float turning = dot3(cross3(axis_world, sub3(point, origin)), dir) + dot3(axis_world, V3{0, 0, 0});
-                const float sliding = dot3(axis_world, dir);
-                const bool on_path = lane < m.dof && ((mask >> lane) & 1ull) != 0ull;
-                entries[side] = !on_path || mode == 0u ? 0.0f : ((mode & 1u) != 0u ? turning : sliding);
-            }
-            if (uniform_word(my_merge, i) != 0u) { entries[0] += entries[1]; entries[1] = 0.0f; }   // shared owner (:172-186)
-            if (lane < md) {
-                if (links[0] != kInvalid) d.chain_jacobian[(size_t{env} * R + r) * md + lane] = entries[0];
-                if (links[1] != kInvalid) d.chain_jacobian_b[(size_t{env} * R + r) * md + lane] = entries[1];
-            }
-            // PrepareContactRowsKernel (:1134-1140): a compliant row's reference acceleration includes the damping of the
-            // velocity the step started from along the row, ContactReferenceVelocity (:1072-1100): side A's coordinates
-            // in order, then side B's
-            const float gain = uniform_value(my_gain, i);
-            if (gain != 0.0f) {
-                float velocity = 0.0f;
-                for (uint32_t side = 0u; side < 2u; ++side) {
-                    if (links[side] == kInvalid) continue;
-                    const float term = entries[side] * start_velocity;
-                    for (uint32_t k = 0u; k < md; ++k) velocity += uniform_value(term, k);
-                }
-                if (lane == 0u) rows[r].rhs += gain * velocity;
-            }
-        }
     }
 }
 
@@ -1427,9 +1469,12 @@ Status OpAssembleRows(const ModelView& m, const DataView& d, const void* params,
     if (p == nullptr) return Status::Failed;
     if (p->env_count == 0u || p->rows_per_env == 0u) return Status::Ok;
     if (p->max_dof > kMaxDof) return Status::InvalidArgument;
-    const size_t lds = (size_t{p->union_slot_count} * 2u + size_t{p->contact_rows_per_env} * 10u + size_t{m.links_per_env} * 2u) * sizeof(uint32_t);
-    if (lds > 150u * 1024u) return Status::InvalidArgument;
-    hipLaunchKernelGGL(AssembleRowsKernel, dim3(p->env_count), dim3(kWave), lds, stream, m, d, *p);
+    // (the slots a world may have: those whose row words fitted a compute unit's LDS when the rows were kept there)
+    if ((size_t{p->union_slot_count} * 2u + size_t{p->contact_rows_per_env} * 10u + size_t{m.links_per_env} * 2u) * sizeof(uint32_t) > 150u * 1024u)
+        return Status::InvalidArgument;
+    const bool compliant = m.any_mujoco != 0u;
+    const size_t lds = size_t{AssembleLdsWords(p->union_slot_count, m.links_per_env, p->max_dof, compliant)} * sizeof(uint32_t);
+    hipLaunchKernelGGL(compliant ? AssembleRowsKernel<true> : AssembleRowsKernel<false>, dim3(p->env_count), dim3(kWave), lds, stream, m, d, *p);
     return hipGetLastError() == hipSuccess ? Status::Ok : Status::Failed;
 }
 
@@ -1831,7 +1876,8 @@ Status OpSnapshotStepVelocity(const ModelView& m, const DataView& d, const void*
 }
 
 void InitContactKernels() {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(AssembleRowsKernel), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    for (const void* kernel : {reinterpret_cast<const void*>(AssembleRowsKernel<false>), reinterpret_cast<const void*>(AssembleRowsKernel<true>)})
+        (void)hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
     (void)hipGetLastError();
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(WarmStartPrepareKernel), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
     (void)hipGetLastError();
