@@ -22,9 +22,6 @@ __device__ __forceinline__ float dot3(V3 a, V3 b) { return a.x * b.x + a.y * b.y
 __device__ __forceinline__ V3 cross3(V3 a, V3 b) {
     return V3{a.y * b.z - a.z * b.y, a.z * b.x - a.x * b.z, a.x * b.y - a.y * b.x};
 }
-// Full-precision reciprocal square root: v_rsq_f32 alone is 1 ulp-approximate, sqrt then divide is exact-rounded.
-__device__ __forceinline__ float rsqrt_exact(float x) { return 1.0f / sqrtf(x); }
-
 // Correctly rounded square root and quotient for operands in the normal range, without the range scaling, special-value
 // fix-ups and second reciprocal that the general sqrtf and operator/ carry.  sqrt_rn_normal corrects v_sqrt_f32 (at
 // most one ulp off) by the residuals of its two neighbours; make_recip / div_by are the Newton reciprocal and the two
@@ -53,6 +50,11 @@ __device__ __forceinline__ float div_by(float a, Recip d) {
     e = fmaf(-d.divisor, q, a);
     return fmaf(e, d.value, q);
 }
+
+// Full-precision reciprocal square root: v_rsq_f32 alone is 1 ulp-approximate, sqrt then divide is exact-rounded.  The bits of
+// 1.0f / sqrtf(x) for x between 2^-90 and 2^90 - squared lengths of axes, normals and quaternions - in a third of its
+// instructions, which stand twice on the chain from a link's pose to its child's.
+__device__ __forceinline__ float rsqrt_exact(float x) { return div_by(1.0f, make_recip(sqrt_rn_normal(x))); }
 
 __device__ __forceinline__ Xf load_xf(const float* p) { return Xf{V3{p[0], p[1], p[2]}, Q4{p[3], p[4], p[5], p[6]}}; }
 __device__ __forceinline__ void store_xf(float* p, Xf t) {
