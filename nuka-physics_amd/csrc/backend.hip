@@ -169,18 +169,20 @@ int MergeStepTail(Backend* be, const ModelView& m, const DataView& d, const nuka
     return bodies ? 4 : 3;
 }
 
-// SyncLinkBodyPose, BuildAabbs, LbvhBuild, LbvhQueryPairs, NarrowphasePrimitives at the head of `calls` as one launch
+// SyncLinkBodyPose, BuildAabbs, LbvhBuild, LbvhQueryPairs and, where it follows and the world's manifolds are of one point,
+// NarrowphasePrimitives at the head of `calls` as one launch
 int MergeCollisionHead(Backend* be, const ModelView& m, const DataView& d, const nuka_phi_op_call* calls, int n, Status* failure) {
-    if (n < 5 || calls[0].op != uint16_t(NkOp::SyncLinkBodyPose) || calls[1].op != uint16_t(NkOp::BuildAabbs) ||
-        calls[2].op != uint16_t(NkOp::LbvhBuild) || calls[3].op != uint16_t(NkOp::LbvhQueryPairs) ||
-        calls[4].op != uint16_t(NkOp::NarrowphasePrimitives) || calls[2].params == nullptr) return 0;
+    if (n < 4 || calls[0].op != uint16_t(NkOp::SyncLinkBodyPose) || calls[1].op != uint16_t(NkOp::BuildAabbs) ||
+        calls[2].op != uint16_t(NkOp::LbvhBuild) || calls[3].op != uint16_t(NkOp::LbvhQueryPairs) || calls[2].params == nullptr) return 0;
+    const bool narrow = n >= 5 && calls[4].op == uint16_t(NkOp::NarrowphasePrimitives);
+    bool manifolds = false;
     const Status status = OpCollisionHead(m, d, static_cast<const SyncLinkBodyPoseParams*>(calls[0].params),
                                           static_cast<const BuildAabbsParams*>(calls[1].params),
                                           static_cast<const LbvhQueryPairsParams*>(calls[3].params),
-                                          static_cast<const NarrowphasePrimitivesParams*>(calls[4].params), be->stream);
+                                          narrow ? static_cast<const NarrowphasePrimitivesParams*>(calls[4].params) : nullptr, be->stream, &manifolds);
     if (status == Status::Unsupported) return 0;
     *failure = status;
-    return 5;
+    return manifolds ? 5 : 4;
 }
 
 // The next launch of an op list: the ops after the solve, and those between the dynamics and the row assembly, each take

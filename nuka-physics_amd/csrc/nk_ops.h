@@ -42,6 +42,6 @@ Status OpStepTail(const ModelView&, const DataView&, const IntegratePositionPara
                   const FkLinkVelocitiesParams*, const SyncLinkBodyPoseParams*, hipStream_t);
 // SyncLinkBodyPose, BuildAabbs, LbvhBuild, LbvhQueryPairs and NarrowphasePrimitives as one launch, likewise.
 Status OpCollisionHead(const ModelView&, const DataView&, const SyncLinkBodyPoseParams*, const BuildAabbsParams*,
-                       const LbvhQueryPairsParams*, const NarrowphasePrimitivesParams*, hipStream_t);
+                       const LbvhQueryPairsParams*, const NarrowphasePrimitivesParams*, hipStream_t, bool* manifolds_done);
 
 }  // namespace nkh

@@ -749,8 +749,11 @@ __global__ void __launch_bounds__(64) NarrowphasePackedKernel(ModelView m, DataV
 
 // What stands between the dynamics and the row assembly - the bodies' poses, their boxes, the candidate pairs, the
 // manifolds - as one kernel, one wavefront an environment: four kernels of about a launch's time each become one, running
-// the same device code in the same order.  Single-point worlds only (the general manifolds keep their candidate lists in
-// scratch memory).  A plan takes this route when its op list holds the ops in a row (backend.hip).
+// the same device code in the same order.  The general manifolds keep their candidate lists in scratch memory and, in
+// small worlds, several environments a wavefront, so with kManifolds false the kernel ends with the pairs: 13 us for the
+// three ops before them at 4096 walkers, 17 and two launches' gaps dispatched one by one (a step 353 -> 349 us).  A plan takes
+// this route when its op list holds the ops in a row (backend.hip).
+template <bool kManifolds>
 __global__ void __launch_bounds__(kWave) CollisionHeadKernel(ModelView m, DataView d, BuildAabbsParams boxes, LbvhQueryPairsParams query,
                                                              NarrowphasePrimitivesParams narrow) {
     const uint32_t env = blockIdx.x, lane = threadIdx.x, nb = m.bodies_per_env;
@@ -760,6 +763,7 @@ __global__ void __launch_bounds__(kWave) CollisionHeadKernel(ModelView m, DataVi
     for (uint32_t b = lane; b < nb; b += kWave) build_aabb_of_body(m, d, boxes, env * nb + b);
     __syncthreads();
     query_pairs_of_env(m, d, query, env, lane);
+    if constexpr (!kManifolds) return;
     __syncthreads();
     narrowphase_of_env<true>(m, d, narrow, env, lane);
 }
@@ -1445,17 +1449,22 @@ Status OpNarrowphasePrimitives(const ModelView& m, const DataView& d, const void
     return hipGetLastError() == hipSuccess ? Status::Ok : Status::Failed;
 }
 
-// SyncLinkBodyPose, BuildAabbs, LbvhBuild (no tree is built on this path), LbvhQueryPairs and NarrowphasePrimitives as one
-// launch; Unsupported when any of them would not run its kernel as dispatched, or the world has many-point manifolds.
+// SyncLinkBodyPose, BuildAabbs, LbvhBuild (no tree is built on this path), LbvhQueryPairs and, in worlds of single-point
+// manifolds, NarrowphasePrimitives as one launch, `manifolds_done` telling whether it made them; Unsupported when any of
+// them would not run its kernel as dispatched.
 Status OpCollisionHead(const ModelView& m, const DataView& d, const SyncLinkBodyPoseParams* bodies, const BuildAabbsParams* boxes,
-                       const LbvhQueryPairsParams* query, const NarrowphasePrimitivesParams* narrow, hipStream_t stream) {
-    if (bodies == nullptr || boxes == nullptr || query == nullptr || narrow == nullptr || m.max_points_per_slot > 1u) return Status::Unsupported;
+                       const LbvhQueryPairsParams* query, const NarrowphasePrimitivesParams* narrow, hipStream_t stream, bool* manifolds_done) {
+    *manifolds_done = false;
+    if (bodies == nullptr || boxes == nullptr || query == nullptr) return Status::Unsupported;
     const uint32_t E = bodies->env_count, nb = m.bodies_per_env;
     if (E == 0u || nb == 0u || bodies->bodies_per_env != nb || bodies->selected_env_count != 0u || boxes->env_count != E ||
-        boxes->bodies_per_env != nb || query->env_count != E || query->bodies_per_env != nb || query->excluded_count != 0u ||
-        narrow->env_count != E || narrow->bodies_per_env != nb || narrow->union_slot_count == 0u || narrow->rigid_slot_cap == 0u)
+        boxes->bodies_per_env != nb || query->env_count != E || query->bodies_per_env != nb || query->excluded_count != 0u)
         return Status::Unsupported;
-    hipLaunchKernelGGL(CollisionHeadKernel, dim3(E), dim3(kWave), 0, stream, m, d, *boxes, *query, *narrow);
+    const bool manifolds = narrow != nullptr && m.max_points_per_slot <= 1u && narrow->env_count == E && narrow->bodies_per_env == nb &&
+                           narrow->union_slot_count != 0u && narrow->rigid_slot_cap != 0u;
+    if (manifolds) hipLaunchKernelGGL(CollisionHeadKernel<true>, dim3(E), dim3(kWave), 0, stream, m, d, *boxes, *query, *narrow);
+    else hipLaunchKernelGGL(CollisionHeadKernel<false>, dim3(E), dim3(kWave), 0, stream, m, d, *boxes, *query, NarrowphasePrimitivesParams{});
+    *manifolds_done = manifolds;
     return hipGetLastError() == hipSuccess ? Status::Ok : Status::Failed;
 }
 
