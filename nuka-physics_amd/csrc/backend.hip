@@ -169,6 +169,20 @@ int MergeStepTail(Backend* be, const ModelView& m, const DataView& d, const nuka
     return bodies ? 4 : 3;
 }
 
+// FkWorldPoses and ArticulationDynamics with ApplyDrives between them: the last, which neither reads nor writes what the first
+// does, is dispatched ahead of the other two's one launch
+int MergePosesAndDynamics(Backend* be, const ModelView& m, const DataView& d, const nuka_phi_op_call* calls, int n, Status* failure) {
+    if (n < 3 || calls[0].op != uint16_t(NkOp::FkWorldPoses) || calls[1].op != uint16_t(NkOp::ApplyDrives) ||
+        calls[2].op != uint16_t(NkOp::ArticulationDynamics)) return 0;
+    const auto* poses = static_cast<const FkWorldPosesParams*>(calls[0].params);
+    const auto* dynamics = static_cast<const ArticulationDynamicsParams*>(calls[2].params);
+    if (!PosesAndDynamicsServed(m, poses, dynamics)) return 0;
+    const Status drives = DispatchOn(be, m, d, calls[1]);
+    if (drives == Status::InvalidArgument || drives == Status::Unsupported) return 0;   // nothing launched: it names its own error
+    *failure = drives != Status::Ok ? drives : OpPosesAndDynamics(m, d, dynamics, be->stream);
+    return 3;
+}
+
 // SyncLinkBodyPose, BuildAabbs, LbvhBuild, LbvhQueryPairs and, where it follows and the world's manifolds are of one point,
 // NarrowphasePrimitives at the head of `calls` as one launch
 int MergeCollisionHead(Backend* be, const ModelView& m, const DataView& d, const nuka_phi_op_call* calls, int n, Status* failure) {
@@ -185,12 +199,13 @@ int MergeCollisionHead(Backend* be, const ModelView& m, const DataView& d, const
     return manifolds ? 5 : 4;
 }
 
-// The next launch of an op list: the ops after the solve, and those between the dynamics and the row assembly, each take
-// about a launch's time, so where the list holds them in a row one kernel runs them (StepTailKernel, CollisionHeadKernel);
-// where it cannot, the first op goes alone.  `served` is the number of ops that the launch covers, also one that failed.
+// The next launch of an op list: the ops after the solve, those between the dynamics and the row assembly, and the poses ahead
+// of the dynamics each take about a launch's time, so where the list holds them in a row one kernel runs them (StepTailKernel,
+// CollisionHeadKernel, ArticulationDynamicsKernel with a third wavefront); where it cannot, the first op goes alone.  `served` is the number of ops that the launch covers, also one that failed.
 Status DispatchNext(Backend* be, const ModelView& m, const DataView& d, const nuka_phi_op_call* calls, int n, int* served) {
     Status status = Status::Ok;
     *served = MergeStepTail(be, m, d, calls, n, &status);
+    if (*served == 0) *served = MergePosesAndDynamics(be, m, d, calls, n, &status);
     if (*served == 0) *served = MergeCollisionHead(be, m, d, calls, n, &status);
     if (*served > 0) return status;
     *served = 1;

@@ -40,6 +40,9 @@ Status BodyIntegratePosition(const ModelView&, const DataView&, const IntegrateP
 // a plan whose op list holds them in a row; Unsupported when they must run one by one.
 Status OpStepTail(const ModelView&, const DataView&, const IntegratePositionParams*, const FkWorldPosesParams*,
                   const FkLinkVelocitiesParams*, const SyncLinkBodyPoseParams*, hipStream_t);
+// FkWorldPoses and ArticulationDynamics as one launch, where PosesAndDynamicsServed.
+bool PosesAndDynamicsServed(const ModelView&, const FkWorldPosesParams*, const ArticulationDynamicsParams*);
+Status OpPosesAndDynamics(const ModelView&, const DataView&, const ArticulationDynamicsParams*, hipStream_t);
 // SyncLinkBodyPose, BuildAabbs, LbvhBuild, LbvhQueryPairs and NarrowphasePrimitives as one launch, likewise.
 Status OpCollisionHead(const ModelView&, const DataView&, const SyncLinkBodyPoseParams*, const BuildAabbsParams*,
                        const LbvhQueryPairsParams*, const NarrowphasePrimitivesParams*, hipStream_t, bool* manifolds_done);

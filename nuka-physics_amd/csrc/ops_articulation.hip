@@ -361,10 +361,13 @@ __device__ __forceinline__ uint32_t times(uint32_t words, uint32_t link) { retur
 // the links, their records, their rows of X - is read a pass or two ahead, roots and lanes without a link have places of
 // their own so that no read stands under a condition, and the matrix takes the inertias' place (a pass of 64 arms 900 -> 400
 // cycles, the kernel 19.4 -> 16.9 us; 4096 humanoids 118 -> 98 us, 65536 1405 -> 1133 us, 8192 ropes 1633 -> 1031 us).
+// With a third wavefront the kernel is FkWorldPoses too (OpPosesAndDynamics): that one places the links beside the other two,
+// which ask for a pose only where a link has a wrench on it.
 template <int N, int G>
-__global__ void __launch_bounds__(2 * kWave) ArticulationDynamicsKernel(ModelView m, DataView d, ArticulationDynamicsParams p,
+__global__ void __launch_bounds__(3 * kWave) ArticulationDynamicsKernel(ModelView m, DataView d, ArticulationDynamicsParams p,
                                                                        uint32_t env_count) {
     extern __shared__ float lds[];
+    const bool places = blockDim.x > 2u * kWave;
     constexpr uint32_t kEnvs = kWave / G, kRowLanes = G < 32 ? 2u * G : 64u;
     static_assert(N <= int(kRowLanes), "a lane a row");
     const uint32_t wave = threadIdx.x / kWave, lane = threadIdx.x % kWave, nl = m.links_per_env, n = m.dof, stride = m.max_dof;
@@ -398,6 +401,20 @@ __global__ void __launch_bounds__(2 * kWave) ArticulationDynamicsKernel(ModelVie
         w.tmp = w.rate + nl;         // 36 words of the inertia push
         return w;
     };
+    // of a third wavefront: the links' poses, and whether they stand (a word, its place the environments' poses' last)
+    float* poses = lds + DynamicsTreeWords(nl, passes) + kEnvs * DynamicsEnvWords(nl, n, kEnvs);
+    volatile uint32_t* posed = reinterpret_cast<uint32_t*>(poses + kEnvs * nl * 7u);
+    if (wave == 2u) {
+        const uint32_t group = lane / G, env = blockIdx.x * kEnvs + group;
+        if (lane == 0u) *posed = 0u;
+        __syncthreads();
+        world_poses_of_env<G>(m, d, env, lane % G, env < env_count, poses + group * nl * 7u);   // G holds an environment's links
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+        if (lane == 0u) *posed = 1u;
+        __syncthreads();
+        if constexpr (kEnvs == 1u) { __syncthreads(); __syncthreads(); }
+        return;
+    }
     const V3 gravity{p.gravity[0], p.gravity[1], p.gravity[2]};
     // Step by step down the sweeps' list: `fetch` a link's constants one step ahead, `use` them with the values of the step
     // before.  A lane without a link sweeps nobody's place, so that no step asks which lanes it is for.
@@ -530,7 +547,10 @@ __global__ void __launch_bounds__(2 * kWave) ArticulationDynamicsKernel(ModelVie
                 if (p.apply_link_wrench != 0u) {
                     const float* wr = d.link_wrench + (lbase + l) * 6u;
                     if (wr[0] != 0.0f || wr[1] != 0.0f || wr[2] != 0.0f || wr[3] != 0.0f || wr[4] != 0.0f || wr[5] != 0.0f) {
-                        const Q4 rot = load_xf(d.link_pose + (lbase + l) * 7u).r;
+                        // (the third wavefront waits for nothing between the barrier above and its word)
+                        if (places) while (*posed == 0u) __builtin_amdgcn_s_sleep(1);
+                        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+                        const Q4 rot = load_xf(places ? poses + (group * nl + l) * 7u : d.link_pose + (lbase + l) * 7u).r;
                         const V3 force = rotate_inverse(rot, V3{wr[0], wr[1], wr[2]});
                         const V3 torque = rotate_inverse(rot, V3{wr[3], wr[4], wr[5]});
                         const V3 moment = add3(torque, cross3(load_xf(m.link_inertial_frame + 7u * l).p, force));
@@ -1101,21 +1121,53 @@ static uint32_t DynamicsLanes(uint32_t links, uint32_t dof, uint32_t envs) {
     return links <= 8u && dof <= 16u ? 8u : links <= 16u && dof <= 24u ? 16u : 64u;
 }
 
+// LDS of a workgroup of `entry`, with a third wavefront's poses where it `places`
+static size_t DynamicsBytes(const ModelView& m, const DynamicsEntry& entry, bool places) {
+    const uint32_t envs = kWave / entry.lanes;
+    return size_t{DynamicsTreeWords(m.links_per_env, m.sweep_passes) + envs * DynamicsEnvWords(m.links_per_env, m.dof, envs) +
+                  (places ? envs * m.links_per_env * 7u + 1u : 0u)} * sizeof(float);
+}
+// nullptr where the op refuses the world or the parameters
+static const DynamicsEntry* DynamicsEntryOf(const ModelView& m, const ArticulationDynamicsParams& p) {
+    if (m.dof > kMaxDof || m.dof == 0u || p.max_dof != m.max_dof || p.total_link_count != p.articulation_count * m.links_per_env) return nullptr;
+    // the links a world may have: those whose working state, with its transforms in full, fits a compute unit's LDS
+    if (size_t{m.links_per_env * 109u + m.dof * (m.dof + 3u) + 64u + m.sweep_passes * kSweepLinks} * sizeof(float) > 160u * 1024u) return nullptr;
+    const uint32_t lanes = DynamicsLanes(m.links_per_env, m.dof, p.articulation_count);
+    const DynamicsEntry* entry = kDynamicsKernels;
+    while (entry->lanes < lanes || entry->width < m.dof) ++entry;
+    return entry;
+}
+static Status LaunchDynamics(const ModelView& m, const DataView& d, const ArticulationDynamicsParams& p, const DynamicsEntry& entry, bool places, hipStream_t stream) {
+    const uint32_t envs = kWave / entry.lanes;
+    hipLaunchKernelGGL(entry.kernel, dim3((p.articulation_count + envs - 1u) / envs), dim3((places ? 3 : 2) * kWave), DynamicsBytes(m, entry, places), stream, m, d, p,
+                       p.articulation_count);
+    return hipGetLastError() == hipSuccess ? Status::Ok : Status::Failed;
+}
 Status OpArticulationDynamics(const ModelView& m, const DataView& d, const void* params, hipStream_t stream) {
     const auto* p = static_cast<const ArticulationDynamicsParams*>(params);
     if (p == nullptr) return Status::Failed;
     if (p->articulation_count == 0u || p->total_link_count == 0u) return Status::Ok;
-    if (m.dof > kMaxDof || m.dof == 0u || p->max_dof != m.max_dof ||
-        p->total_link_count != p->articulation_count * m.links_per_env) return Status::InvalidArgument;
-    // the links a world may have: those whose working state, with its transforms in full, fits a compute unit's LDS
-    if (size_t{m.links_per_env * 109u + m.dof * (m.dof + 3u) + 64u + m.sweep_passes * kSweepLinks} * sizeof(float) > 160u * 1024u) return Status::InvalidArgument;
-    const uint32_t lanes = DynamicsLanes(m.links_per_env, m.dof, p->articulation_count);
-    const DynamicsEntry* entry = kDynamicsKernels;
-    while (entry->lanes < lanes || entry->width < m.dof) ++entry;
-    const uint32_t envs = kWave / entry->lanes;
-    const size_t lds = size_t{DynamicsTreeWords(m.links_per_env, m.sweep_passes) + envs * DynamicsEnvWords(m.links_per_env, m.dof, envs)} * sizeof(float);
-    hipLaunchKernelGGL(entry->kernel, dim3((p->articulation_count + envs - 1u) / envs), dim3(2 * kWave), lds, stream, m, d, *p, p->articulation_count);
-    return hipGetLastError() == hipSuccess ? Status::Ok : Status::Failed;
+    const DynamicsEntry* entry = DynamicsEntryOf(m, *p);
+    return entry == nullptr ? Status::InvalidArgument : LaunchDynamics(m, d, *p, *entry, false, stream);
+}
+
+// The poses in the dynamics' launch: a launch and its gap less, and the sweep of the poses beside the dynamics' longer ones.
+// Always where environments share a wavefront (a step of 4000 and fewer arms 49 -> 45 us, of 64 37.3 -> 32.8, of 65536 229 -> 223;
+// 4096 walkers 343 -> 339, 16384 quadrupeds 1240 -> 1243).  An environment a wavefront, up to six workgroups a compute unit:
+// past that the third wavefront, which has a lane a link and waits on every depth, takes the others' turns (64 humanoids 517
+// -> 511 us, 1024 641 -> 637, 1500 621 -> 616, 1800 639 -> 645, 3000 714 -> 723, 65536 7818 -> 8180; 1800 quadrupeds 410 ->
+// 408, 2900 435 -> 440).  Not the 65 links of a rope, two a lane (256 of them 2321 -> 2288 us, 1000 2535 -> 2577).
+constexpr uint32_t kPlacedBeside = 1536u;
+bool PosesAndDynamicsServed(const ModelView& m, const FkWorldPosesParams* poses, const ArticulationDynamicsParams* dynamics) {
+    if (poses == nullptr || dynamics == nullptr || dynamics->articulation_count == 0u || m.links_per_env == 0u) return false;
+    if (poses->articulation_count != dynamics->articulation_count || poses->total_link_count != dynamics->total_link_count) return false;
+    const DynamicsEntry* entry = DynamicsEntryOf(m, *dynamics);
+    if (entry == nullptr || DynamicsBytes(m, *entry, true) > 160u * 1024u) return false;
+    return m.links_per_env <= entry->lanes && (entry->lanes < uint32_t(kWave) || dynamics->articulation_count <= kPlacedBeside);
+}
+Status OpPosesAndDynamics(const ModelView& m, const DataView& d, const ArticulationDynamicsParams* dynamics, hipStream_t stream) {
+    const DynamicsEntry* entry = DynamicsEntryOf(m, *dynamics);
+    return entry == nullptr ? Status::InvalidArgument : LaunchDynamics(m, d, *dynamics, *entry, true, stream);
 }
 
 namespace {

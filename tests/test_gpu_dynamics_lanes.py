@@ -81,3 +81,36 @@ def test_many_links_match_the_oracle(oracle_py, device, links):
         assert error <= bar, (name, error)
     world.close()
     oracle.close()
+
+
+@pytest.mark.parametrize("dof,floating,branched,limb_joints,E", [
+    (16, False, True, 3, 1), (16, False, True, 3, 1536), (16, False, True, 3, 1537),   # a wavefront each: one, the most, one more
+    (7, False, False, 7, 48), (7, False, False, 7, 3077),                              # a chain alone, and eight a workgroup
+    (21, True, True, 4, 1000), (21, True, True, 4, 3077),                              # a floating robot alone, and four a workgroup
+])
+def test_poses_beside_the_dynamics_are_those_ahead_of_it(oracle_py, device, dof, floating, branched, limb_joints, E):
+    """A step places the links in the dynamics' launch, where a link with a wrench on it turns that by its own new pose: the
+    state after the step has the bits the ops leave one by one, from poses and wrenches that were uploaded."""
+    tree, _, state = tree_case(oracle_py, dof, floating, branched, seed=dof, E=48, limb_joints=limb_joints)
+    rows, g = np.arange(E) % 48, np.random.default_rng(dof)
+    nl = tree.link_count
+    wrench = g.normal(0.0, 2.0, (E, nl, 6)).astype(np.float32) * (g.random((E, nl, 1)) < 0.3)
+    out = []
+    for single in (True, False):
+        world = nk.World(device, tree.template, abi.world_desc(E, 1.0 / 240.0, vel_iters=8, contact_margin=0.1))
+        world.set_state({k: v[rows] for k, v in state.items()})
+        world.upload("link_pose", np.full((E, nl, 7), np.nan, np.float32))
+        world.upload("link_wrench", wrench)
+        if single:
+            for op in ("FkWorldPoses", "ApplyDrives", "ArticulationDynamics", "SyncLinkBodyPose", "BuildAabbs", "LbvhBuild", "LbvhQueryPairs",
+                       "NarrowphasePrimitives", "AssembleRows", ("ContactWarmStart", 0), "BlockDescentSolve", ("ContactWarmStart", 1),
+                       "IntegratePosition", "FkWorldPoses", "FkLinkVelocities", "SyncLinkBodyPose"):
+                world.op(*(op if isinstance(op, tuple) else (op,)))
+        else:
+            world.step()
+        world.synchronize()
+        out.append({name: world.download(name).reshape(E, -1) for name in FIELDS + ("q", "link_pose")})
+        world.close()
+    assert np.abs(out[0]["articulation_qdd"]).max() > 0.1 and np.isfinite(out[0]["qddot"]).all()
+    for name in out[0]:
+        assert np.array_equal(out[0][name], out[1][name]), name
