@@ -151,26 +151,41 @@ Status DispatchOn(Backend* be, const ModelView& m, const DataView& d, const nuka
     return fn(m, d, call.params, be->stream);
 }
 
-// IntegratePosition, FkWorldPoses, FkLinkVelocities and, if it follows, SyncLinkBodyPose at the head of `calls` as one
-// launch: the number of calls it covers, 0 when the head is something else or the merged kernel does not serve these
-// parameters (Unsupported: the ops then run one by one, and each names its own parameters' errors).  Any other failure of
-// the merged launch is the step's or the plan's and comes back through `failure`, never as a quiet fall back that would
-// dispatch the ops a second time.
-int MergeStepTail(Backend* be, const ModelView& m, const DataView& d, const nuka_phi_op_call* calls, int n, Status* failure) {
+// IntegratePosition, FkWorldPoses, FkLinkVelocities and, if it follows, SyncLinkBodyPose at the head of an op list: how many
+// they are (0: the head is something else) and their parameters
+struct Tail {
+    const IntegratePositionParams* integrate;
+    const FkWorldPosesParams* poses;
+    const FkLinkVelocitiesParams* twists;
+    const SyncLinkBodyPoseParams* bodies;
+};
+int TailOf(const nuka_phi_op_call* calls, int n, Tail* tail) {
     if (n < 3 || calls[0].op != uint16_t(NkOp::IntegratePosition) || calls[1].op != uint16_t(NkOp::FkWorldPoses) ||
         calls[2].op != uint16_t(NkOp::FkLinkVelocities)) return 0;
     const bool bodies = n >= 4 && calls[3].op == uint16_t(NkOp::SyncLinkBodyPose);
-    const Status status = OpStepTail(m, d, static_cast<const IntegratePositionParams*>(calls[0].params),
-                                     static_cast<const FkWorldPosesParams*>(calls[1].params),
-                                     static_cast<const FkLinkVelocitiesParams*>(calls[2].params),
-                                     bodies ? static_cast<const SyncLinkBodyPoseParams*>(calls[3].params) : nullptr, be->stream);
-    if (status == Status::Unsupported) return 0;
-    *failure = status;
+    *tail = Tail{static_cast<const IntegratePositionParams*>(calls[0].params), static_cast<const FkWorldPosesParams*>(calls[1].params),
+                 static_cast<const FkLinkVelocitiesParams*>(calls[2].params),
+                 bodies ? static_cast<const SyncLinkBodyPoseParams*>(calls[3].params) : nullptr};
     return bodies ? 4 : 3;
 }
 
+// Those ops as one launch: the number of calls it covers, 0 when the head is something else or the merged kernel does not
+// serve these parameters (Unsupported: the ops then run one by one, and each names its own parameters' errors).  Any other
+// failure of the merged launch is the step's or the plan's and comes back through `failure`, never as a quiet fall back that
+// would dispatch the ops a second time.
+int MergeStepTail(Backend* be, const ModelView& m, const DataView& d, const nuka_phi_op_call* calls, int n, Status* failure) {
+    Tail tail;
+    const int ops = TailOf(calls, n, &tail);
+    if (ops == 0) return 0;
+    const Status status = OpStepTail(m, d, tail.integrate, tail.poses, tail.twists, tail.bodies, be->stream);
+    if (status == Status::Unsupported) return 0;
+    *failure = status;
+    return ops;
+}
+
 // FkWorldPoses and ArticulationDynamics with ApplyDrives between them: the last, which neither reads nor writes what the first
-// does, is dispatched ahead of the other two's one launch
+// does, is dispatched ahead of the other two's one launch; with IntegrateVelocity, which leaves an articulation alone, and the
+// step's tail right behind them, those too
 int MergePosesAndDynamics(Backend* be, const ModelView& m, const DataView& d, const nuka_phi_op_call* calls, int n, Status* failure) {
     if (n < 3 || calls[0].op != uint16_t(NkOp::FkWorldPoses) || calls[1].op != uint16_t(NkOp::ApplyDrives) ||
         calls[2].op != uint16_t(NkOp::ArticulationDynamics)) return 0;
@@ -179,7 +194,14 @@ int MergePosesAndDynamics(Backend* be, const ModelView& m, const DataView& d, co
     if (!PosesAndDynamicsServed(m, poses, dynamics)) return 0;
     const Status drives = DispatchOn(be, m, d, calls[1]);
     if (drives == Status::InvalidArgument || drives == Status::Unsupported) return 0;   // nothing launched: it names its own error
-    *failure = drives != Status::Ok ? drives : OpPosesAndDynamics(m, d, dynamics, be->stream);
+    *failure = drives;
+    Tail tail;
+    const int ops = n > 4 && calls[3].op == uint16_t(NkOp::IntegrateVelocity) && calls[3].params != nullptr && m.free_body == 0u ? TailOf(calls + 4, n - 4, &tail) : 0;
+    if (ops != 0 && StepServed(m, *dynamics, tail.integrate, tail.poses, tail.twists, tail.bodies)) {
+        if (drives == Status::Ok) *failure = OpStep(m, d, dynamics, tail.integrate, tail.poses, tail.twists, tail.bodies, be->stream);
+        return 4 + ops;
+    }
+    if (drives == Status::Ok) *failure = OpPosesAndDynamics(m, d, dynamics, be->stream);
     return 3;
 }
 
@@ -201,7 +223,8 @@ int MergeCollisionHead(Backend* be, const ModelView& m, const DataView& d, const
 
 // The next launch of an op list: the ops after the solve, those between the dynamics and the row assembly, and the poses ahead
 // of the dynamics each take about a launch's time, so where the list holds them in a row one kernel runs them (StepTailKernel,
-// CollisionHeadKernel, ArticulationDynamicsKernel with a third wavefront); where it cannot, the first op goes alone.  `served` is the number of ops that the launch covers, also one that failed.
+// CollisionHeadKernel, ArticulationDynamicsKernel with a third wavefront, which in a world without rows goes on with the tail);
+// where it cannot, the first op goes alone.  `served` is the number of ops that the launch covers, also one that failed.
 Status DispatchNext(Backend* be, const ModelView& m, const DataView& d, const nuka_phi_op_call* calls, int n, int* served) {
     Status status = Status::Ok;
     *served = MergeStepTail(be, m, d, calls, n, &status);

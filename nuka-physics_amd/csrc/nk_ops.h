@@ -43,6 +43,11 @@ Status OpStepTail(const ModelView&, const DataView&, const IntegratePositionPara
 // FkWorldPoses and ArticulationDynamics as one launch, where PosesAndDynamicsServed.
 bool PosesAndDynamicsServed(const ModelView&, const FkWorldPosesParams*, const ArticulationDynamicsParams*);
 Status OpPosesAndDynamics(const ModelView&, const DataView&, const ArticulationDynamicsParams*, hipStream_t);
+// Both and the ops of OpStepTail as one launch, where PosesAndDynamicsServed and StepServed.
+bool StepServed(const ModelView&, const ArticulationDynamicsParams&, const IntegratePositionParams*, const FkWorldPosesParams*,
+                const FkLinkVelocitiesParams*, const SyncLinkBodyPoseParams*);
+Status OpStep(const ModelView&, const DataView&, const ArticulationDynamicsParams*, const IntegratePositionParams*,
+              const FkWorldPosesParams*, const FkLinkVelocitiesParams*, const SyncLinkBodyPoseParams*, hipStream_t);
 // SyncLinkBodyPose, BuildAabbs, LbvhBuild, LbvhQueryPairs and NarrowphasePrimitives as one launch, likewise.
 Status OpCollisionHead(const ModelView&, const DataView&, const SyncLinkBodyPoseParams*, const BuildAabbsParams*,
                        const LbvhQueryPairsParams*, const NarrowphasePrimitivesParams*, hipStream_t, bool* manifolds_done);

@@ -364,9 +364,7 @@ __device__ __forceinline__ uint32_t times(uint32_t words, uint32_t link) { retur
 // With a third wavefront the kernel is FkWorldPoses too (OpPosesAndDynamics): that one places the links beside the other two,
 // which ask for a pose only where a link has a wrench on it.
 template <int N, int G>
-__global__ void __launch_bounds__(3 * kWave) ArticulationDynamicsKernel(ModelView m, DataView d, ArticulationDynamicsParams p,
-                                                                       uint32_t env_count) {
-    extern __shared__ float lds[];
+__device__ __forceinline__ void dynamics_of_block(const ModelView& m, const DataView& d, const ArticulationDynamicsParams& p, uint32_t env_count, float* lds) {
     const bool places = blockDim.x > 2u * kWave;
     constexpr uint32_t kEnvs = kWave / G, kRowLanes = G < 32 ? 2u * G : 64u;
     static_assert(N <= int(kRowLanes), "a lane a row");
@@ -1038,22 +1036,37 @@ __global__ void __launch_bounds__(kWave) FkLinkVelocitiesKernel(ModelView m, Dat
 // `G` lanes of two wavefronts an environment: four kernels that each take about the time of a launch become one, running
 // the same device code in the same order (IntegratePosition, FkWorldPoses, FkLinkVelocities, SyncLinkBodyPose).  A plan
 // takes this route when its op list holds the four in a row (backend.hip); an op dispatched by itself runs its own kernel.
+struct StepTail { IntegratePositionParams integrate; uint32_t runs, sync_bodies; };
 template <int G>
-__global__ void __launch_bounds__(2 * kWave) StepTailKernel(ModelView m, DataView d, IntegratePositionParams p, uint32_t env_count,
-                                                            uint32_t sync_bodies) {
-    extern __shared__ float lds[];
+__device__ __forceinline__ void step_tail_of_block(const ModelView& m, const DataView& d, const StepTail& t, uint32_t env_count, float* lds) {
     constexpr uint32_t kLanes = G < kWave ? G : kWave, kEnvs = kWave / kLanes;
     const uint32_t lane = threadIdx.x % kLanes, group = threadIdx.x % kWave / kLanes, env = blockIdx.x * kEnvs + group, nl = m.links_per_env;
-    const bool twists = threadIdx.x >= uint32_t(kWave);   // world poses and link twists do not depend on each other: a wavefront each
+    const uint32_t wave = threadIdx.x / kWave;   // world poses and link twists do not depend on each other: a wavefront each
     const bool there = env < env_count;
-    if (!twists && there) for (uint32_t l = lane; l < nl; l += kLanes) integrate_position_of_link(m, d, p, env, l);
+    if (wave == 0u && there) for (uint32_t l = lane; l < nl; l += kLanes) integrate_position_of_link(m, d, t.integrate, env, l);
     __syncthreads();   // the new coordinates, base pose and root twist are in memory for both wavefronts
-    if (twists) { link_velocities_of_env<G>(m, d, env, lane, there, lds + kEnvs * nl * 7u + group * nl * 6u); return; }
+    if (wave == 1u) link_velocities_of_env<G>(m, d, env, lane, there, lds + kEnvs * nl * 7u + group * nl * 6u);
+    if (wave != 0u) return;
     float* pose = lds + group * nl * 7u;
     world_poses_of_env<G>(m, d, env, lane, there, pose);
-    if (sync_bodies == 0u || !there) return;
+    if (t.sync_bodies == 0u || !there) return;
     wave_sync();
     for (uint32_t b = lane; b < m.bodies_per_env; b += kLanes) sync_body_pose(m, d, env, b, pose);
+}
+template <int G>
+__global__ void __launch_bounds__(2 * kWave) StepTailKernel(ModelView m, DataView d, StepTail t, uint32_t env_count) {
+    extern __shared__ float lds[];
+    step_tail_of_block<G>(m, d, t, env_count, lds);
+}
+// Where nothing stands between the dynamics and the step's tail, as in a world without rows, the workgroup goes on with its own
+// environments: their state is its own.
+template <int N, int G>
+__global__ void __launch_bounds__(3 * kWave) ArticulationDynamicsKernel(ModelView m, DataView d, ArticulationDynamicsParams p, uint32_t env_count, StepTail t) {
+    extern __shared__ float lds[];
+    dynamics_of_block<N, G>(m, d, p, env_count, lds);
+    if (t.runs == 0u) return;
+    __syncthreads();
+    step_tail_of_block<G>(m, d, t, env_count, lds);
 }
 
 // The instantiation for `lanes` lanes an environment and the number of its workgroups
@@ -1081,23 +1094,31 @@ Status OpFkWorldPoses(const ModelView& m, const DataView& d, const void* params,
     return hipGetLastError() == hipSuccess ? Status::Ok : Status::Failed;
 }
 
+// false when any of the four would not run its kernel as dispatched
+static bool StepTailOf(const ModelView& m, const IntegratePositionParams* integrate, const FkWorldPosesParams* poses, const FkLinkVelocitiesParams* twists,
+                       const SyncLinkBodyPoseParams* bodies, StepTail* tail) {
+    if (integrate == nullptr || poses == nullptr || twists == nullptr) return false;
+    const uint32_t E = poses->articulation_count, links = E * m.links_per_env;
+    if (E == 0u || m.links_per_env == 0u || integrate->dt <= 0.0f || integrate->total_link_count != links ||
+        poses->total_link_count != links || poses->selected_env_count != 0u || twists->articulation_count != E ||
+        twists->total_link_count != links) return false;
+    if (bodies != nullptr && (bodies->env_count != E || bodies->bodies_per_env != m.bodies_per_env || bodies->bodies_per_env == 0u ||
+                              bodies->selected_env_count != 0u)) return false;
+    *tail = StepTail{*integrate, 1u, bodies != nullptr ? 1u : 0u};
+    return true;
+}
 // The four ops after the solve as one launch; Unsupported when any of them would not run its kernel as dispatched
 // (the caller then dispatches them one by one).
 Status OpStepTail(const ModelView& m, const DataView& d, const IntegratePositionParams* integrate, const FkWorldPosesParams* poses,
                   const FkLinkVelocitiesParams* twists, const SyncLinkBodyPoseParams* bodies, hipStream_t stream) {
-    if (integrate == nullptr || poses == nullptr || twists == nullptr) return Status::Unsupported;
-    const uint32_t E = poses->articulation_count, links = E * m.links_per_env;
-    if (E == 0u || m.links_per_env == 0u || integrate->dt <= 0.0f || integrate->total_link_count != links ||
-        poses->total_link_count != links || poses->selected_env_count != 0u || twists->articulation_count != E ||
-        twists->total_link_count != links) return Status::Unsupported;
-    if (bodies != nullptr && (bodies->env_count != E || bodies->bodies_per_env != m.bodies_per_env || bodies->bodies_per_env == 0u ||
-                              bodies->selected_env_count != 0u)) return Status::Unsupported;
-    const uint32_t lanes = LanesAnEnvironment(m.links_per_env, E);
-    NKH_LAUNCH_LANES(lanes, StepTailKernel, E, 2 * kWave, m.links_per_env * 13u, stream, m, d, *integrate, E, bodies != nullptr ? 1u : 0u);
+    StepTail tail;
+    if (!StepTailOf(m, integrate, poses, twists, bodies, &tail)) return Status::Unsupported;
+    const uint32_t E = poses->articulation_count, lanes = LanesAnEnvironment(m.links_per_env, E);
+    NKH_LAUNCH_LANES(lanes, StepTailKernel, E, 2 * kWave, m.links_per_env * 13u, stream, m, d, tail, E);
     return hipGetLastError() == hipSuccess ? Status::Ok : Status::Failed;
 }
 
-using DynamicsKernel = void (*)(ModelView, DataView, ArticulationDynamicsParams, uint32_t);
+using DynamicsKernel = void (*)(ModelView, DataView, ArticulationDynamicsParams, uint32_t, StepTail);
 struct DynamicsEntry { uint32_t width, lanes; DynamicsKernel kernel; };
 // by lanes an environment, then by width: the first that holds an environment's links and coordinates is the one
 #define NKH_DYNAMICS(N, G) {N##u, G##u, ArticulationDynamicsKernel<N, G>}
@@ -1137,10 +1158,11 @@ static const DynamicsEntry* DynamicsEntryOf(const ModelView& m, const Articulati
     while (entry->lanes < lanes || entry->width < m.dof) ++entry;
     return entry;
 }
-static Status LaunchDynamics(const ModelView& m, const DataView& d, const ArticulationDynamicsParams& p, const DynamicsEntry& entry, bool places, hipStream_t stream) {
+static Status LaunchDynamics(const ModelView& m, const DataView& d, const ArticulationDynamicsParams& p, const DynamicsEntry& entry, bool places, const StepTail& tail,
+                             hipStream_t stream) {
     const uint32_t envs = kWave / entry.lanes;
     hipLaunchKernelGGL(entry.kernel, dim3((p.articulation_count + envs - 1u) / envs), dim3((places ? 3 : 2) * kWave), DynamicsBytes(m, entry, places), stream, m, d, p,
-                       p.articulation_count);
+                       p.articulation_count, tail);
     return hipGetLastError() == hipSuccess ? Status::Ok : Status::Failed;
 }
 Status OpArticulationDynamics(const ModelView& m, const DataView& d, const void* params, hipStream_t stream) {
@@ -1148,12 +1170,12 @@ Status OpArticulationDynamics(const ModelView& m, const DataView& d, const void*
     if (p == nullptr) return Status::Failed;
     if (p->articulation_count == 0u || p->total_link_count == 0u) return Status::Ok;
     const DynamicsEntry* entry = DynamicsEntryOf(m, *p);
-    return entry == nullptr ? Status::InvalidArgument : LaunchDynamics(m, d, *p, *entry, false, stream);
+    return entry == nullptr ? Status::InvalidArgument : LaunchDynamics(m, d, *p, *entry, false, StepTail{}, stream);
 }
 
 // The poses in the dynamics' launch: a launch and its gap less, and the sweep of the poses beside the dynamics' longer ones.
-// Always where environments share a wavefront (a step of 4000 and fewer arms 49 -> 45 us, of 64 37.3 -> 32.8, of 65536 229 -> 223;
-// 4096 walkers 343 -> 339, 16384 quadrupeds 1240 -> 1243).  An environment a wavefront, up to six workgroups a compute unit:
+// Always where environments share a wavefront or have few links (a step of 64 arms 37.3 -> 32.8 us, 2000 and 3500 49 -> 45,
+// 65536 229 -> 223; 4096 walkers 343 -> 339, 16384 quadrupeds 1240 -> 1243).  An environment a wavefront, up to six workgroups a compute unit:
 // past that the third wavefront, which has a lane a link and waits on every depth, takes the others' turns (64 humanoids 517
 // -> 511 us, 1024 641 -> 637, 1500 621 -> 616, 1800 639 -> 645, 3000 714 -> 723, 65536 7818 -> 8180; 1800 quadrupeds 410 ->
 // 408, 2900 435 -> 440).  Not the 65 links of a rope, two a lane (256 of them 2321 -> 2288 us, 1000 2535 -> 2577).
@@ -1163,11 +1185,29 @@ bool PosesAndDynamicsServed(const ModelView& m, const FkWorldPosesParams* poses,
     if (poses->articulation_count != dynamics->articulation_count || poses->total_link_count != dynamics->total_link_count) return false;
     const DynamicsEntry* entry = DynamicsEntryOf(m, *dynamics);
     if (entry == nullptr || DynamicsBytes(m, *entry, true) > 160u * 1024u) return false;
-    return m.links_per_env <= entry->lanes && (entry->lanes < uint32_t(kWave) || dynamics->articulation_count <= kPlacedBeside);
+    return m.links_per_env <= entry->lanes && (m.links_per_env <= 8u || entry->lanes < uint32_t(kWave) || dynamics->articulation_count <= kPlacedBeside);
 }
 Status OpPosesAndDynamics(const ModelView& m, const DataView& d, const ArticulationDynamicsParams* dynamics, hipStream_t stream) {
     const DynamicsEntry* entry = DynamicsEntryOf(m, *dynamics);
-    return entry == nullptr ? Status::InvalidArgument : LaunchDynamics(m, d, *dynamics, *entry, true, stream);
+    return entry == nullptr ? Status::InvalidArgument : LaunchDynamics(m, d, *dynamics, *entry, true, StepTail{}, stream);
+}
+// The step's tail in the dynamics' launch, up to five workgroups a compute unit: past that the shorter kernels fill the chip
+// better than one whose workgroups hold the dynamics' LDS to the end (a step of 64 arms 32.8 -> 30.6 us, 1000 37.8 -> 35.4, 8000
+// in 1000 workgroups 51.0 -> 46.7, 12000 67.2 -> 67.5, 20011 86 -> 88, 65536 223 -> 234).
+constexpr uint32_t kTailWorkgroups = 1280u;
+bool StepServed(const ModelView& m, const ArticulationDynamicsParams& dynamics, const IntegratePositionParams* integrate, const FkWorldPosesParams* poses,
+                const FkLinkVelocitiesParams* twists, const SyncLinkBodyPoseParams* bodies) {
+    StepTail tail;
+    const DynamicsEntry* entry = DynamicsEntryOf(m, dynamics);
+    if (entry == nullptr || !StepTailOf(m, integrate, poses, twists, bodies, &tail) || poses->articulation_count != dynamics.articulation_count) return false;
+    return uint64_t{dynamics.articulation_count} * entry->lanes <= uint64_t{kTailWorkgroups} * kWave;
+}
+Status OpStep(const ModelView& m, const DataView& d, const ArticulationDynamicsParams* dynamics, const IntegratePositionParams* integrate,
+              const FkWorldPosesParams* poses, const FkLinkVelocitiesParams* twists, const SyncLinkBodyPoseParams* bodies, hipStream_t stream) {
+    const DynamicsEntry* entry = DynamicsEntryOf(m, *dynamics);
+    StepTail tail;
+    if (entry == nullptr || !StepTailOf(m, integrate, poses, twists, bodies, &tail)) return Status::InvalidArgument;
+    return LaunchDynamics(m, d, *dynamics, *entry, true, tail, stream);
 }
 
 namespace {

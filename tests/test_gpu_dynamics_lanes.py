@@ -114,3 +114,42 @@ def test_poses_beside_the_dynamics_are_those_ahead_of_it(oracle_py, device, dof,
     assert np.abs(out[0]["articulation_qdd"]).max() > 0.1 and np.isfinite(out[0]["qddot"]).all()
     for name in out[0]:
         assert np.array_equal(out[0][name], out[1][name]), name
+
+
+@pytest.mark.parametrize("links,E", [(2, 1), (8, 48), (8, 3077), (8, 10240), (8, 10241), (17, 1280), (17, 1281)])
+def test_a_step_without_rows_is_one_launch_with_the_bits_of_its_ops(device, links, E):
+    """A world without rows goes on from the dynamics to the step's tail in the same workgroup, up to 1280 of them: the state after
+    two steps, the second from poses and twists the first left, has the bits the ops leave one by one."""
+    g = np.random.default_rng(links)
+    t = abi.Template()
+    t.add_link(abi.JOINT_FIXED, None, mass=2.0, diag_inertia=(0.02, 0.03, 0.02))
+    for k in range(links - 1):
+        t.add_link(abi.JOINT_REVOLUTE, max(0, k - k % 3 // 2), axis=((1, 0, 0), (0, 1, 0), (0, 0, 1))[k % 3], local_pos=(0.1, 0.02, -0.05),
+                   mass=g.uniform(0.1, 0.5), diag_inertia=tuple(g.uniform(1e-3, 5e-3, 3)), com=(0.0, 0.01, -0.03), armature=0.02)
+    for link in range(t.link_count):
+        t.add_body(abi.ROLE_LINK_BODY, link=link, kind=abi.SHAPE_NONE, contype=0, conaffinity=0)
+    rows = np.arange(E) % 48
+    state = {name: g.normal(0.0, sigma, (48, links)).astype(np.float32)[rows] for name, sigma in (("q", 0.5), ("qdot", 1.0), ("tau", 0.5))}
+    base = np.zeros((E, 7), np.float32)
+    base[:, 3] = 1.0
+    state.update(base_pose=base, root_twist=np.zeros((E, 6), np.float32))
+    for name in ("q", "qdot", "tau"):
+        state[name][:, 0] = 0.0
+    wrench = g.normal(0.0, 0.5, (48, links, 6)).astype(np.float32)[rows]
+    out = []
+    for single in (True, False):
+        world = nk.World(device, t, abi.world_desc(E, 1.0 / 240.0))
+        world.set_state(state)
+        for _ in range(2):
+            world.upload("link_wrench", wrench)
+            if single:
+                for op in ("FkWorldPoses", "ApplyDrives", "ArticulationDynamics", "IntegrateVelocity", "IntegratePosition", "FkWorldPoses", "FkLinkVelocities", "SyncLinkBodyPose"):
+                    world.op(op)
+            else:
+                world.step()
+        world.synchronize()
+        out.append({name: world.download(name).reshape(E, -1) for name in FIELDS + ("q", "link_pose", "body_pose")})
+        world.close()
+    assert np.isfinite(out[0]["link_pose"]).all() and np.abs(out[0]["qdot"]).max() > 0.1
+    for name in out[0]:
+        assert np.array_equal(out[0][name], out[1][name]), name
