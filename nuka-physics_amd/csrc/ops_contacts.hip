@@ -54,12 +54,9 @@ __device__ V3 rot_abs(Q4 q, V3 v) {
 
 // ---- BuildAabbs (broadphase.cu:173-270).  Link-owned collidables carry no body velocity on this path, so the
 // motion term of the margin is zero; a free body's row carries the body's velocities. ----
-__device__ __forceinline__ void build_aabb_of_body(const ModelView& m, const DataView& d, const BuildAabbsParams& p, uint32_t gid) {
-    const uint32_t b = gid % p.bodies_per_env;
+struct Aabb { float lo[3], hi[3]; };
+__device__ __forceinline__ Aabb aabb_of_body(const ModelView& m, const DataView& d, const BuildAabbsParams& p, uint32_t gid, uint32_t b, const Xf& xf) {
     const ShapeRow s = load_shape(m.shape_table, b);
-    const Xf xf = load_xf(d.body_pose + size_t{gid} * 7u);
-    float* lo = d.body_aabb_lo + size_t{gid} * 3u;
-    float* hi = d.body_aabb_hi + size_t{gid} * 3u;
     V3 he{0, 0, 0};
     if (s.kind == kShapeSphere) he = V3{s.p[0], s.p[0], s.p[0]};
     else if (s.kind == kShapeCapsule) he = rot_abs(xf.r, V3{s.p[0], s.p[0], s.p[0] + s.p[1]});
@@ -72,11 +69,9 @@ __device__ __forceinline__ void build_aabb_of_body(const ModelView& m, const Dat
                 s.p[1] * fabsf(a.y) + s.p[0] * sqrtf(fmaxf(0.0f, 1.0f - a.y * a.y)),
                 s.p[1] * fabsf(a.z) + s.p[0] * sqrtf(fmaxf(0.0f, 1.0f - a.z * a.z))};
     } else if (s.kind == kShapePlane) {
-        lo[0] = lo[1] = lo[2] = -FLT_MAX; hi[0] = hi[1] = hi[2] = FLT_MAX;
-        return;
+        return Aabb{{-FLT_MAX, -FLT_MAX, -FLT_MAX}, {FLT_MAX, FLT_MAX, FLT_MAX}};
     } else {
-        lo[0] = lo[1] = lo[2] = FLT_MAX; hi[0] = hi[1] = hi[2] = -FLT_MAX;
-        return;
+        return Aabb{{FLT_MAX, FLT_MAX, FLT_MAX}, {-FLT_MAX, -FLT_MAX, -FLT_MAX}};
     }
     // (:262-264) a free body's own row moves with it - its speed, and its turning rate over the shape's radius
     float speed = 0.0f;
@@ -87,13 +82,16 @@ __device__ __forceinline__ void build_aabb_of_body(const ModelView& m, const Dat
     }
     const float mg = fmaxf(p.margin, fminf(motion_radius(p.margin, p.dt, speed, 0.0f, 0.9f), p.query_reach));
     const V3 c = xf.p;
-    lo[0] = c.x - he.x - mg; lo[1] = c.y - he.y - mg; lo[2] = c.z - he.z - mg;
-    hi[0] = c.x + he.x + mg; hi[1] = c.y + he.y + mg; hi[2] = c.z + he.z + mg;
+    return Aabb{{c.x - he.x - mg, c.y - he.y - mg, c.z - he.z - mg}, {c.x + he.x + mg, c.y + he.y + mg, c.z + he.z + mg}};
+}
+__device__ __forceinline__ void store_aabb(const DataView& d, uint32_t gid, const Aabb& box) {
+#pragma unroll
+    for (int k = 0; k < 3; ++k) { d.body_aabb_lo[size_t{gid} * 3u + k] = box.lo[k]; d.body_aabb_hi[size_t{gid} * 3u + k] = box.hi[k]; }
 }
 __global__ void BuildAabbsKernel(ModelView m, DataView d, BuildAabbsParams p) {
     const uint32_t gid = blockIdx.x * blockDim.x + threadIdx.x;
     if (gid >= p.env_count * p.bodies_per_env) return;
-    build_aabb_of_body(m, d, p, gid);
+    store_aabb(d, gid, aabb_of_body(m, d, p, gid, gid % p.bodies_per_env, load_xf(d.body_pose + size_t{gid} * 7u)));
 }
 
 // collision/shape_kind.hpp:26-33
@@ -104,43 +102,50 @@ __device__ __forceinline__ bool shape_filter_admits(uint32_t ta, uint32_t aa, ui
 }
 
 // broadphase.cu:87-99 IsExcluded: binary search of the sorted (a << 32 | b) keys, a < b
-__device__ bool pair_excluded(const ModelView& m, uint32_t a, uint32_t b) {
+__device__ __forceinline__ bool pair_excluded(const uint64_t* excluded, uint32_t count, uint32_t a, uint32_t b) {
     const uint64_t key = (uint64_t{a} << 32u) | uint64_t{b};
-    uint32_t lo = 0u, hi = m.excluded_pair_count;
+    uint32_t lo = 0u, hi = count;
     while (lo < hi) {
         const uint32_t mid = lo + (hi - lo) / 2u;
-        if (m.excluded_pairs[mid] < key) lo = mid + 1u; else hi = mid;
+        if (excluded[mid] < key) lo = mid + 1u; else hi = mid;
     }
-    return lo < m.excluded_pair_count && m.excluded_pairs[lo] == key;
+    return lo < count && excluded[lo] == key;
 }
 
-// ---- candidate pairs: one wavefront per env walks the (i, j) grid in row-major order; the ballot rank of an
+// ---- candidate pairs: one wavefront per env walks the pairs i < j in row-major order; the ballot rank of an
 // emitting lane is its slot, which is the ascending (a, b) order the reference reaches by sorting.  The grid runs over
 // the rows that can pass the shape filter at all (a row with empty type and affinity masks pairs with nothing): a
-// humanoid's 31 shapeless link rows leave a grid of 13 x 13 out of 44 x 44. ----
+// humanoid's 31 shapeless link rows leave the 78 pairs of 13 out of 44 rows.  `boxes` and `excluded` are the field's and the
+// model's own words or copies of them in LDS: a pair is a chain of reads, a binary search of the exclusions among them. ----
+template <class Boxes>
 __device__ __forceinline__ void query_pairs_of_env(const ModelView& m, const DataView& d, const LbvhQueryPairsParams& p, uint32_t env,
-                                                    uint32_t lane) {
+                                                    uint32_t lane, const Boxes& boxes, const uint64_t* excluded) {
     const uint32_t N = m.pairable_count;
-    const size_t bbase = size_t{env} * p.bodies_per_env;
+    const uint32_t items = N < 2u ? 0u : N * (N - 1u) / 2u;
+    const auto first_of = [&](uint32_t row) { return row * (2u * N - row - 1u) / 2u; };   // pairs ahead of a row's
     const uint32_t capacity = min(p.rigid_slot_cap, p.max_pairs);
     uint32_t* pairs = d.candidate_pairs + size_t{env} * p.max_contacts_per_env * 2u;
     uint32_t count = 0u;
     bool overflow = false;
-    for (uint32_t base = 0u; base < N * N; base += kWave) {
-        const uint32_t item = base + lane, at_i = item / N, at_j = item % N;
+    for (uint32_t base = 0u; base < items; base += kWave) {
+        const uint32_t item = base + lane;
         bool emit = false;
         uint32_t i = 0u, j = 0u;
-        if (at_i < at_j && at_i < N) {
+        if (item < items) {
+            const float middle = float(N) - 0.5f;
+            uint32_t at_i = min(uint32_t(middle - sqrtf(fmaxf(middle * middle - 2.0f * float(item), 0.0f))), N - 2u);   // a row off at most
+            while (first_of(at_i) > item) --at_i;
+            while (first_of(at_i + 1u) <= item) ++at_i;
+            const uint32_t at_j = item - first_of(at_i) + at_i + 1u;
             i = m.pairable_rows[at_i]; j = m.pairable_rows[at_j];
-            const float* alo = d.body_aabb_lo + (bbase + i) * 3u, *ahi = d.body_aabb_hi + (bbase + i) * 3u;
-            const float* blo = d.body_aabb_lo + (bbase + j) * 3u, *bhi = d.body_aabb_hi + (bbase + j) * 3u;
-            const bool overlap = !(ahi[0] < blo[0] || alo[0] > bhi[0] || ahi[1] < blo[1] || alo[1] > bhi[1] ||
-                                   ahi[2] < blo[2] || alo[2] > bhi[2]);
+            const Aabb a = boxes(i), b = boxes(j);
+            const bool overlap = !(a.hi[0] < b.lo[0] || a.lo[0] > b.hi[0] || a.hi[1] < b.lo[1] || a.lo[1] > b.hi[1] ||
+                                   a.hi[2] < b.lo[2] || a.lo[2] > b.hi[2]);
             if (overlap) {
                 const ShapeRow sa = load_shape(m.shape_table, i), sb = load_shape(m.shape_table, j);
                 emit = !(sa.body_id < 0 && sb.body_id < 0) &&
                        shape_filter_admits(sa.contype, sa.conaffinity, sa.group, sb.contype, sb.conaffinity, sb.group) &&
-                       !pair_excluded(m, i, j);
+                       !pair_excluded(excluded, m.excluded_pair_count, i, j);
             }
         }
         const uint64_t mask = __ballot(emit);
@@ -159,7 +164,13 @@ __device__ __forceinline__ void query_pairs_of_env(const ModelView& m, const Dat
     }
 }
 __global__ void __launch_bounds__(kWave) QueryPairsKernel(ModelView m, DataView d, LbvhQueryPairsParams p) {
-    query_pairs_of_env(m, d, p, blockIdx.x, threadIdx.x);
+    const size_t first = size_t{blockIdx.x} * p.bodies_per_env;
+    query_pairs_of_env(m, d, p, blockIdx.x, threadIdx.x, [&](uint32_t b) {
+        Aabb box;
+#pragma unroll
+        for (int k = 0; k < 3; ++k) { box.lo[k] = d.body_aabb_lo[(first + b) * 3u + k]; box.hi[k] = d.body_aabb_hi[(first + b) * 3u + k]; }
+        return box;
+    }, m.excluded_pairs);
 }
 
 // ---- manifolds (collision/analytical_manifold.hpp) ------------------------------------------------------
@@ -750,21 +761,35 @@ __global__ void __launch_bounds__(64) NarrowphasePackedKernel(ModelView m, DataV
 // What stands between the dynamics and the row assembly - the bodies' poses, their boxes, the candidate pairs, the
 // manifolds - as one kernel, one wavefront an environment: four kernels of about a launch's time each become one, running
 // the same device code in the same order.  The general manifolds keep their candidate lists in scratch memory and, in
-// small worlds, several environments a wavefront, so with kManifolds false the kernel ends with the pairs: 13 us for the
-// three ops before them at 4096 walkers, 17 and two launches' gaps dispatched one by one (a step 353 -> 349 us).  A plan takes
+// small worlds, several environments a wavefront, so with kManifolds false the kernel ends with the pairs: the three
+// ops before them took 17 us and two launches' gaps at 4096 walkers, 13 as one (a step 353 -> 349 us).  A plan takes
 // this route when its op list holds the ops in a row (backend.hip).
+// A lane's bodies go from their pose to their box in its registers, and the boxes and the exclusions wait in LDS for the pairs,
+// whose walk leaves out the half of the grid that pairs nothing: 65536 humanoids 237 -> 182 us, 16384 boxes 19.7 -> 16.5, 333
+// humanoids 10.7 -> 9.7 (a dependent read of memory after the other is what bounds it; a step of 4096 walkers 341 -> 333 us).
+constexpr uint32_t kHeadExclusions = 512u;   // in LDS; the binary search of more reads memory
 template <bool kManifolds>
 __global__ void __launch_bounds__(kWave) CollisionHeadKernel(ModelView m, DataView d, BuildAabbsParams boxes, LbvhQueryPairsParams query,
                                                              NarrowphasePrimitivesParams narrow) {
+    extern __shared__ uint64_t lds64[];
     const uint32_t env = blockIdx.x, lane = threadIdx.x, nb = m.bodies_per_env;
+    const uint32_t held = m.excluded_pair_count <= kHeadExclusions ? m.excluded_pair_count : 0u;
+    Aabb* box = reinterpret_cast<Aabb*>(lds64 + held);
+    for (uint32_t e = lane; e < held; e += kWave) lds64[e] = m.excluded_pairs[e];
     const float* link_pose = d.link_pose + size_t{env} * m.links_per_env * 7u;
-    for (uint32_t b = lane; b < nb; b += kWave) sync_body_pose(m, d, env, b, link_pose);
-    __syncthreads();   // the poses are in memory for every lane
-    for (uint32_t b = lane; b < nb; b += kWave) build_aabb_of_body(m, d, boxes, env * nb + b);
+    for (uint32_t b = lane; b < nb; b += kWave) {
+        const uint32_t gid = env * nb + b;
+        Xf pose;
+        if (body_pose_of(m, b, link_pose, &pose)) store_xf(d.body_pose + size_t{gid} * 7u, pose);
+        else pose = load_xf(d.body_pose + size_t{gid} * 7u);
+        const Aabb mine = aabb_of_body(m, d, boxes, gid, b, pose);
+        store_aabb(d, gid, mine);
+        box[b] = mine;
+    }
     __syncthreads();
-    query_pairs_of_env(m, d, query, env, lane);
+    query_pairs_of_env(m, d, query, env, lane, [&](uint32_t b) { return box[b]; }, held != 0u ? lds64 : m.excluded_pairs);
     if constexpr (!kManifolds) return;
-    __syncthreads();
+    __syncthreads();   // the pairs and the poses are in memory for every lane
     narrowphase_of_env<true>(m, d, narrow, env, lane);
 }
 // math/cuda_vec_ops.cuh:150-183
@@ -1462,8 +1487,10 @@ Status OpCollisionHead(const ModelView& m, const DataView& d, const SyncLinkBody
         return Status::Unsupported;
     const bool manifolds = narrow != nullptr && m.max_points_per_slot <= 1u && narrow->env_count == E && narrow->bodies_per_env == nb &&
                            narrow->union_slot_count != 0u && narrow->rigid_slot_cap != 0u;
-    if (manifolds) hipLaunchKernelGGL(CollisionHeadKernel<true>, dim3(E), dim3(kWave), 0, stream, m, d, *boxes, *query, *narrow);
-    else hipLaunchKernelGGL(CollisionHeadKernel<false>, dim3(E), dim3(kWave), 0, stream, m, d, *boxes, *query, NarrowphasePrimitivesParams{});
+    const size_t lds = (m.excluded_pair_count <= kHeadExclusions ? m.excluded_pair_count : 0u) * sizeof(uint64_t) + size_t{nb} * sizeof(Aabb);
+    if (lds > 64u * 1024u) return Status::Unsupported;
+    if (manifolds) hipLaunchKernelGGL(CollisionHeadKernel<true>, dim3(E), dim3(kWave), lds, stream, m, d, *boxes, *query, *narrow);
+    else hipLaunchKernelGGL(CollisionHeadKernel<false>, dim3(E), dim3(kWave), lds, stream, m, d, *boxes, *query, NarrowphasePrimitivesParams{});
     *manifolds_done = manifolds;
     return hipGetLastError() == hipSuccess ? Status::Ok : Status::Failed;
 }
