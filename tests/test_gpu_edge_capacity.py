@@ -10,8 +10,8 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("rows,cols,bounds", [(7, 6, (14, 28, 42)), (3, 5, (14, 15, 15)), (2, 2, (4, 4, 4))])
 def test_environments_on_either_side_of_the_edge_capacities_match_the_oracle(oracle_py, device, rows, cols, bounds):
     """A raft of spheres over the plane, tilted or level: with 42 of them (168 heads) the solve sends environments of up to
-    14, of up to 28 and of more contact points to three launches of their own, with 15 to two, and four heads a point of
-    four spheres fit the fullest launch.  An environment's result is the oracle's, which knows no launches."""
+    14, of up to 28 and of more contact points to three launches of their own; with 15, whose 60 heads leave a compute unit
+    seven blocks of eight, and with four all go to one.  An environment's result is the oracle's, which knows no launches."""
     E = 96
     t = abi.Template()
     t.contact_cone = abi.CONE_PYRAMIDAL
