@@ -1129,17 +1129,16 @@ static const DynamicsEntry kDynamicsKernels[] = {
     NKH_DYNAMICS(28, 64), NKH_DYNAMICS(32, 64), NKH_DYNAMICS(36, 64), NKH_DYNAMICS(40, 64), NKH_DYNAMICS(44, 64), NKH_DYNAMICS(48, 64),
     NKH_DYNAMICS(52, 64), NKH_DYNAMICS(56, 64), NKH_DYNAMICS(60, 64), NKH_DYNAMICS(64, 64)};
 #undef NKH_DYNAMICS
-// Lanes an environment: all 64 while every environment fits the chip at once (ten workgroups a compute unit and more), when
-// the one chain an environment has is what counts and fewer lanes lengthen its sweeps; past that as few as hold its links
-// and coordinates.  When the line was drawn a step of 20011 arms (8 links, 7 coordinates) took 187 us with 64 lanes, 115
-// with 16 and 104 with 8 (92 since the sweeps read ahead; 181 with two wavefronts an environment before); 4000 arms 72, 60
-// and 59 us, 3000 56 us any way, 1000 47, 52 and 53; 4096 quadrupeds (13 links, 18 coordinates) 504 us with 64 and 496 with
-// 16, 16384 1308 and 1264, 1000 380 and 390.  Thirty-two lanes gain nothing: two environments of 31 links and 36 coordinates
-// ask for the LDS that two workgroups with 64 lanes each do (65536 humanoids 8435 and 8490 us).
-constexpr uint32_t kDynamicsResident = 3072u;
+// Lanes an environment: all 64 while the environments are few, when the one chain an environment has is what counts and fewer
+// lanes lengthen its sweeps; past that as few as hold its links and coordinates.  A step of 1000 arms (8 links, 7 coordinates)
+// takes 35.9 us with 64 lanes and 37.0 with 8, 1300 40.9 and 36.9, 2500 54.0 and 40.6; 1000 quadrupeds (13 links, 18
+// coordinates) 364 us with 64 and 373 with 16, 2500 399 and 400, 3000 400 and 391, 2000 walkers 261 and 256.  Thirty-two lanes
+// gain nothing: two environments of 31 links and 36 coordinates ask for the LDS that two workgroups with 64 lanes each do
+// (65536 humanoids 8435 and 8490 us).
+constexpr uint32_t kEightLanesFrom = 1152u, kSixteenLanesFrom = 2560u;   // environments
 static uint32_t DynamicsLanes(uint32_t links, uint32_t dof, uint32_t envs) {
-    if (envs < kDynamicsResident) return 64u;
-    return links <= 8u && dof <= 16u ? 8u : links <= 16u && dof <= 24u ? 16u : 64u;
+    if (links <= 8u && dof <= 16u) return envs < kEightLanesFrom ? 64u : 8u;
+    return links <= 16u && dof <= 24u && envs >= kSixteenLanesFrom ? 16u : 64u;
 }
 
 // LDS of a workgroup of `entry`, with a third wavefront's poses where it `places`
@@ -1174,8 +1173,8 @@ Status OpArticulationDynamics(const ModelView& m, const DataView& d, const void*
 }
 
 // The poses in the dynamics' launch: a launch and its gap less, and the sweep of the poses beside the dynamics' longer ones.
-// Always where environments share a wavefront or have few links (a step of 64 arms 37.3 -> 32.8 us, 2000 and 3500 49 -> 45,
-// 65536 229 -> 223; 4096 walkers 343 -> 339, 16384 quadrupeds 1240 -> 1243).  An environment a wavefront, up to six workgroups a compute unit:
+// Always where environments share a wavefront (a step of 3500 arms 49 -> 45 us, 65536 229 -> 223; 4096 walkers 343 -> 339, 16384
+// quadrupeds 1240 -> 1243).  An environment a wavefront (64 arms 37.3 -> 32.8 us), up to six workgroups a compute unit:
 // past that the third wavefront, which has a lane a link and waits on every depth, takes the others' turns (64 humanoids 517
 // -> 511 us, 1024 641 -> 637, 1500 621 -> 616, 1800 639 -> 645, 3000 714 -> 723, 65536 7818 -> 8180; 1800 quadrupeds 410 ->
 // 408, 2900 435 -> 440).  Not the 65 links of a rope, two a lane (256 of them 2321 -> 2288 us, 1000 2535 -> 2577).
@@ -1185,7 +1184,7 @@ bool PosesAndDynamicsServed(const ModelView& m, const FkWorldPosesParams* poses,
     if (poses->articulation_count != dynamics->articulation_count || poses->total_link_count != dynamics->total_link_count) return false;
     const DynamicsEntry* entry = DynamicsEntryOf(m, *dynamics);
     if (entry == nullptr || DynamicsBytes(m, *entry, true) > 160u * 1024u) return false;
-    return m.links_per_env <= entry->lanes && (m.links_per_env <= 8u || entry->lanes < uint32_t(kWave) || dynamics->articulation_count <= kPlacedBeside);
+    return m.links_per_env <= entry->lanes && (entry->lanes < uint32_t(kWave) || dynamics->articulation_count <= kPlacedBeside);
 }
 Status OpPosesAndDynamics(const ModelView& m, const DataView& d, const ArticulationDynamicsParams* dynamics, hipStream_t stream) {
     const DynamicsEntry* entry = DynamicsEntryOf(m, *dynamics);

@@ -1,5 +1,5 @@
 """The forward dynamics at its lane counts: 64 lanes an environment for small batches and large robots, 16 or 8 for large
-batches of small ones."""
+batches of small ones; and the launches that take the poses and the step's tail with it."""
 import numpy as np
 import pytest
 
@@ -33,10 +33,11 @@ def dynamics(device, tree, state, rows):
     (21, True, True, 4, 16),     # the most links and coordinates of a floating robot
     (16, False, True, 3, 17),    # sixty-four lanes whatever the batch
 ])
-@pytest.mark.parametrize("E", [3072, 3077])
+@pytest.mark.parametrize("E", [1152, 2560, 3077])
 def test_packed_environments_have_the_bits_they_have_alone(oracle_py, device, dof, floating, branched, limb_joints, links, E):
-    """From 3072 environments on a workgroup takes four or eight of them; the arithmetic is the same, so copies of 48 seeded
-    environments give in every place, also in a last workgroup that is not full, the bits that the 48 give alone."""
+    """From 1152 environments of up to eight links on, and 2560 of up to sixteen, a workgroup takes eight or four of them; the
+    arithmetic is the same, so copies of 48 seeded environments give in every place, also in a last workgroup that is not full,
+    the bits that the 48 give alone."""
     tree, _, state = tree_case(oracle_py, dof, floating, branched, seed=3 * dof + 1, E=48, limb_joints=limb_joints)
     assert tree.link_count == links
     rows = np.arange(E) % 48
