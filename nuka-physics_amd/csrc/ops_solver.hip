@@ -244,10 +244,12 @@ Status OpBlockDescentSolve(const ModelView& m, const DataView& d, const void* pa
     // lets more blocks share a compute unit, environments with few contact points go to a launch of that capacity:
     // a launch each for sixteen, twelve, eight, four and two blocks a unit, those the waves allow, before the full one.  Each launch takes the
     // environments whose contact points fall in its range; an environment's results do not depend on its launch.  It has to
-    // let twice as many blocks share a unit, for one launch waits for the other's longest environment: 4096 servo-driven
-    // humanoids take 2525 us a step in launches of eight and of seven blocks a unit and 1476 us in one of seven; humanoids
-    // under the pyramidal cone in launches of eight and five 506 us for 400 of them, 604 for 2500 and 771 for 6000, 339, 430
-    // and 756 in one of five; 4096 walkers in launches of eight, four, two and one 292 us, 685 in one of one.
+    // let half as many blocks again share a unit, for one launch waits for the other's longest environment: 4096 servo-driven
+    // humanoids take 2525 us a step in launches of eight and of seven blocks a unit and 1476 us in one of seven; 16384 walkers
+    // under the native laws 1.42 ms in launches of eight and five and 1.80 in one of five, 4096 0.58 and 0.67, 1000 0.47 either
+    // way.  Twice as many where a point is four heads, for a launch of as many heads then takes fewer of the environments:
+    // humanoids under the pyramidal cone in launches of eight and five blocks 506 us for 400 of them, 604 for 2500 and 771 for
+    // 6000, in one of five 338, 430 and 756; 4096 walkers in launches of eight, four, two and one 292 us, 685 in one of one.
     // A contact point is at most `a_point` heads, so `few` heads hold few / a_point points whatever their friction: four
     // edges a point under the pyramidal cone.  (While those worlds went to the one full launch, a walker's 304 heads left a
     // compute unit one block for environments of a handful of points: a step of 4096 with a twentieth reset 768 -> 438 us.)
@@ -258,7 +260,7 @@ Status OpBlockDescentSolve(const ModelView& m, const DataView& d, const void* pa
         for (const size_t blocks : {size_t{16u}, size_t{12u}, size_t{8u}, size_t{4u}, size_t{2u}}) {
             if (blocks > most_blocks) continue;                            // more blocks than the waves allow
             if (blocks_per_unit(staged) >= blocks) break;                  // the full capacity does as well,
-            if (blocks < 2u * blocks_per_unit(staged)) continue;           // or nearly: a launch more ends with a longest environment more
+            if (2u * blocks < (a_point == 1u ? 3u : 4u) * blocks_per_unit(staged)) continue;   // or nearly
             uint32_t few = staged;
             while (few > 8u && blocks_per_unit(few) < blocks) --few;
             const uint32_t points = few / a_point;
