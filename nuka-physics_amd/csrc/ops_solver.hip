@@ -140,6 +140,8 @@ const ReducedKernel kDenseKernels[] = {
 #define NKH_DENSE_BATCH 6144
 #endif
 constexpr uint32_t kDenseBatch = NKH_DENSE_BATCH;
+// Compute units, and the rounds of environments over them from which launches of fewer heads pay (OpBlockDescentSolve).
+constexpr size_t kUnits = 256u, kManyRounds = 9u;
 }  // namespace
 
 void InitSolverKernels() {
@@ -250,17 +252,23 @@ Status OpBlockDescentSolve(const ModelView& m, const DataView& d, const void* pa
     // way.  Twice as many where a point is four heads, for a launch of as many heads then takes fewer of the environments:
     // humanoids under the pyramidal cone in launches of eight and five blocks 506 us for 400 of them, 604 for 2500 and 771 for
     // 6000, in one of five 338, 430 and 756; 4096 walkers in launches of eight, four, two and one 292 us, 685 in one of one.
+    // What waiting for that other longest environment costs has to come back over the rounds of the full launch: those humanoids
+    // in launches of twelve and five 828 us for 6144 (under five rounds of 1280), 1037 for 8192, 1144 for 9500, 1351 for 11519
+    // and 3561 for 32768, in one of five 763, 980, 1117, 1355 and 3616.  Four times as many blocks make it good in fewer rounds:
+    // 1000 walkers, eight blocks for one and four rounds, 244 us in their launches and 289 in one.
     // A contact point is at most `a_point` heads, so `few` heads hold few / a_point points whatever their friction: four
     // edges a point under the pyramidal cone.  (While those worlds went to the one full launch, a walker's 304 heads left a
     // compute unit one block for environments of a handful of points: a step of 4096 with a twentieth reset 768 -> 438 us.)
     hipLaunchKernelGGL(OrderTilesKernel, dim3((p->env_count + kOrderEnvs - 1u) / kOrderEnvs), dim3(1024), 0, stream, d, p->env_count);
     uint32_t first_points = 0u;
     const uint32_t a_point = HeadsAPoint(m);
+    const bool few_rounds = p->env_count < kManyRounds * kUnits * blocks_per_unit(staged);
     if (p->contact_slots_per_env != 0u) {
         for (const size_t blocks : {size_t{16u}, size_t{12u}, size_t{8u}, size_t{4u}, size_t{2u}}) {
             if (blocks > most_blocks) continue;                            // more blocks than the waves allow
             if (blocks_per_unit(staged) >= blocks) break;                  // the full capacity does as well,
             if (2u * blocks < (a_point == 1u ? 3u : 4u) * blocks_per_unit(staged)) continue;   // or nearly
+            if (a_point != 1u && few_rounds && first_points == 0u && blocks < 4u * blocks_per_unit(staged)) break;   // too few rounds to split at all
             uint32_t few = staged;
             while (few > 8u && blocks_per_unit(few) < blocks) --few;
             const uint32_t points = few / a_point;

@@ -1,4 +1,6 @@
 """Worlds under the pyramidal cone of the compliant contact law, where a contact point is four heads of the solve."""
+import copy
+
 import numpy as np
 import pytest
 
@@ -47,3 +49,26 @@ def test_environments_on_either_side_of_the_edge_capacities_match_the_oracle(ora
     for name in ("qdot", "link_velocity", "base_pose"):
         error = per_env_error(world.download(name), oracle.download(name), E)
         assert error.max() <= 2e-4, (name, float(error.max()), int(counts[error.argmax()]))
+
+
+@pytest.mark.parametrize("E", [6144, 11519, 11520])
+def test_as_many_launches_as_the_environments_pay_for_give_the_same_bits(device, E):
+    """Humanoids go to one launch of five blocks a compute unit below nine rounds of 1280, and from there on to one of twelve for
+    those of few contact points ahead of it: copies of 48 environments have the bits that the 48 have alone."""
+    cfg = nk.synthetic.config(3, 48)
+    template, state = copy.deepcopy(cfg.template), cfg.state()
+    template.contact_cone = abi.CONE_PYRAMIDAL
+    for profile in template.profiles:
+        profile["law"] = abi.LAW_MUJOCO
+    out = []
+    for rows in (np.arange(48), np.arange(E) % 48):
+        world = nk.World(device, template, abi.world_desc(len(rows), cfg.dt, vel_iters=cfg.vel_iters))
+        world.set_state({name: values[rows] for name, values in state.items()})
+        world.step()
+        world.synchronize()
+        assert not world.download("env_status").any()
+        out.append({name: world.download(name).reshape(len(rows), -1) for name in ("contact_count", "qdot", "link_velocity", "lambda")})
+        world.close()
+    assert np.unique(out[0]["contact_count"]).size > 4
+    for name, alone in out[0].items():
+        assert np.array_equal(alone[np.arange(E) % 48], out[1][name]), name
