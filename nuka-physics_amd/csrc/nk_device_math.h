@@ -27,7 +27,10 @@ __device__ __forceinline__ V3 cross3(V3 a, V3 b) {
 // most one ulp off) by the residuals of its two neighbours; make_recip / div_by are the Newton reciprocal and the two
 // quotient corrections of the general division, so one reciprocal serves every quotient with the same divisor.  Both
 // give the bits of sqrtf and a / b whenever |x|, |a|, |b| and the result lie between 2^-90 and 2^90 (compared on the
-// device over 5e8 random operands each); outside that range they stay within an ulp.
+// device over 5e8 random operands each); outside that range they stay within an ulp while divisor and result are normal
+// numbers and the divisor is below 2^126.  A larger divisor's reciprocal, no normal number, counts as zero and so does the
+// quotient; a divisor that is infinite, subnormal or zero, or an infinite dividend, gives NaN (rsqrt_exact says what it does
+// about that).
 __device__ __forceinline__ float sqrt_rn_normal(float x) {
     const float s = __builtin_amdgcn_sqrtf(x);
     const float down = __uint_as_float(__float_as_uint(s) - 1u), up = __uint_as_float(__float_as_uint(s) + 1u);

@@ -255,7 +255,7 @@ template <int L, int K, int N>
 __device__ __forceinline__ void ldlt_pivots(uint32_t lane, float (&row)[N]) {
     if constexpr (K < N) {
         const float diagonal = fmaxf(group_value<L, K>(row[K]), 1.0e-6f);
-        const float lik = div_by(row[K], make_recip(diagonal));   // the quotient to the bit, masses lying far inside its range
+        const float lik = div_by(row[K], make_recip(diagonal));   // the quotient to the bit; zero where an armature past 2^126 holds the joint
         row[K] = lane > uint32_t(K) ? lik : (lane == uint32_t(K) ? diagonal : row[K]);
         subtract_products<L, (K + 1) / 4, K>(lik, diagonal, row);
         ldlt_pivots<L, K + 1>(lane, row);

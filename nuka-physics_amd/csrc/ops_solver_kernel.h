@@ -3218,7 +3218,7 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
             // (M^-1)_uu of every coordinate at once, lane = coordinate u: y = L^-1 e_u down the rows with the factor's entries the
             // same for every lane, and the ordered sum of y^2 / D, with the operations of the loop above (four coordinates a
             // pass of that loop took 40 k cycles of a servo-driven humanoid's set-up, this takes 9 k)
-            const Recip by_pivot = make_recip(pivot);   // the quotients to the bit wherever their sum can see them
+            const Recip by_pivot = make_recip(pivot);   // the quotients to the bit wherever their sum can see them, zero by pivots past 2^126
             float mine = 0.0f, y[N];
 #pragma unroll
             for (int i = 0; i < N; ++i) {
