@@ -310,7 +310,8 @@ nuka_result_t nuka_world_set_velocity_iterations(nuka_world_handle world, uint32
 nuka_result_t nuka_world_get_velocity_iterations(nuka_world_handle world, uint32_t* out_iterations);
 nuka_result_t nuka_world_synchronize(nuka_world_handle world);   /* nuka.h:376 */
 nuka_result_t nuka_world_reset(nuka_world_handle world);         /* nuka.h:380 */
-/* nuka.h:381-385: duplicates are ignored, count 0 is a no-op, an id out of range returns INVALID_ARG and changes nothing */
+/* nuka.h:381-385: duplicates are ignored, count 0 is a no-op, an id out of range returns INVALID_ARG and changes nothing.  Ordered
+ * on the world's stream behind what was submitted there, and finished when the call returns (it waits for the stream). */
 nuka_result_t nuka_world_reset_envs(nuka_world_handle world, const uint32_t* env_ids, uint32_t count);
 /* No counterpart in the reference.  nuka_world_reset_envs for callers that cannot allocate (tight serving loops,
  * harnesses that forbid hipMalloc): the same kernel and the same result, with the ids staged in a device array of

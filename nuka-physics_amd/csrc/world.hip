@@ -1302,7 +1302,7 @@ nuka_result_t nuka_world_reset_envs(nuka_world_handle world, const uint32_t* env
 
 // nuka_world_reset_envs for callers that cannot allocate: same kernel, same result, but the ids are staged in the
 // static device array (at most NUKA_RESET_ENVS_STATIC_MAX of them) and in a static host array, so the call takes no
-// device or host memory.  The array is shared by every call on one GPU: calls that overlap there race.
+// device or host memory.  The array is shared by every call on one GPU, which the lock lets in one at a time.
 nuka_result_t nuka_world_reset_envs_static(nuka_world_handle world, const uint32_t* env_ids, uint32_t count) {
     auto* w = reinterpret_cast<World*>(world);
     if (w == nullptr) return Error(NUKA_RESULT_NULL_HANDLE, "world is null");
