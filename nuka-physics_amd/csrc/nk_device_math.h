@@ -10,6 +10,14 @@
 
 namespace nkh {
 
+// Orders one wavefront's LDS writes before its later reads: its lanes run in step and the LDS takes a wavefront's
+// accesses in order, so only the compiler could move them - a fence of wavefront scope holds it without a wait
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 struct V3 { float x, y, z; };
 struct Q4 { float w, x, y, z; };
 struct Xf { V3 p; Q4 r; };

@@ -21,14 +21,6 @@ namespace {
 
 constexpr int kWave = 64;
 
-// Orders one wavefront's LDS writes before its later reads: its lanes run in step and the LDS takes a wavefront's
-// accesses in order, so only the compiler could move them - a fence of wavefront scope holds it without a wait
-__device__ __forceinline__ void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 __device__ __forceinline__ V3 load3(const float* p) { return V3{p[0], p[1], p[2]}; }
 
 // kinematics.cuh:25-42 JointRelativeFrame (revolute / prismatic / fixed)

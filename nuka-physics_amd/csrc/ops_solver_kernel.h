@@ -62,6 +62,15 @@ constexpr int WavesPerSimd(int width) { return width <= kTwoWaveWidth ? 2 : 1; }
 #endif
 #endif
 constexpr int kWidenAtUse = NKH_WIDEN_AT_USE;
+// Orders the block's LDS words between its lanes.  A block is one wavefront, whose LDS accesses are taken in order, so nothing
+// has to be waited for; a barrier of the workgroup waits for the writes all the same, some twenty times a Newton step (333
+// humanoids 567 -> 557 us, 4096 743 -> 732, 65536 7758 -> 7678).  A wide block keeps the barrier: without it reads move
+// up past it into registers the block does not have (8192 ropes 12.70 -> 12.86 ms).
+template <int N>
+__device__ __forceinline__ void lds_sync() {
+    if constexpr (N > kTwoWaveWidth) __syncthreads();
+    else wave_sync();
+}
 constexpr uint32_t kNewtonSteps = 16u;        // block_descent_dense.cuh:14
 constexpr uint32_t kLineSearchSteps = 32u;    // block_descent_dense.cuh:15
 constexpr float kLineTolerance = 1.0e-6f;     // block_descent_dense.cuh:17
@@ -610,7 +619,7 @@ __device__ __forceinline__ bool cholesky_solve(const Tile& c, float (&hrow)[N], 
         if (!valid) return false;
         PROF_BEGIN(c, 24);
         store_rows<N>(c.hfac, c.lane, hrow);
-        __syncthreads();
+        lds_sync<N>();
         PROF_END(c, 24);
         c.factor_current = true;
     } else {
@@ -627,7 +636,7 @@ __device__ __forceinline__ bool cholesky_solve(const Tile& c, float (&hrow)[N], 
         load_columns<N>(c.hfac, c.lane, col);
         *d_out = substitute<N>(hrow, col, inverse, c.lane < c.n ? g : 0.0f);
     }
-    __syncthreads();
+    lds_sync<N>();
     PROF_END(c, 15);
     return true;
 }
@@ -643,7 +652,7 @@ __device__ __forceinline__ bool factor_mass(Tile& c, const float (&mrow)[N]) {
     const bool valid = kLeavesFirst<N> ? factor_rows_up<N>(c.lane, row, &inverse, &root) : factor_rows<N>(c.lane, row, &inverse, &root);
     c.mass_inverse = inverse;
     store_rows<N>(c.mfac, c.lane, row);
-    __syncthreads();
+    lds_sync<N>();
     return valid;
 }
 template <int N>
@@ -1071,7 +1080,7 @@ __device__ __forceinline__ void add_heads_by_groups(const Tile& c, uint64_t head
 #pragma unroll
                 for (int q = 0; q < N / 4; ++q) words[q] = float4{hrow[4 * q], hrow[4 * q + 1], hrow[4 * q + 2], hrow[4 * q + 3]};
             }
-            __syncthreads();
+            lds_sync<N>();
             const float4* words = reinterpret_cast<const float4*>(exchange + column * uint32_t(N));
 #pragma unroll
             for (int q = 0; q < N / 4; ++q) {
@@ -1079,7 +1088,7 @@ __device__ __forceinline__ void add_heads_by_groups(const Tile& c, uint64_t head
                 if (group != 0u) continue;
                 hrow[4 * q] += w.x; hrow[4 * q + 1] += w.y; hrow[4 * q + 2] += w.z; hrow[4 * q + 3] += w.w;
             }
-            __syncthreads();
+            lds_sync<N>();
         }
     }
 }
@@ -1419,7 +1428,7 @@ __device__ __forceinline__ void sums_over_ways(const Tile& c, uint64_t heads, co
 #pragma unroll
             for (uint32_t e = 0u; e < 4u * kGroups; ++e) words[e * kStride + at] = v[e];
         }
-        __syncthreads();
+        lds_sync<int(kWave)>();
         const float* mine = words + (c.lane & 3u) * kStride;
         const uint32_t here = min(end - first, kHeads);
 #pragma unroll 2
@@ -1435,7 +1444,7 @@ __device__ __forceinline__ void sums_over_ways(const Tile& c, uint64_t heads, co
                 for (uint32_t g = 0u; g < uint32_t(kGroups); ++g) sum[g] = __builtin_amdgcn_mfma_f32_4x4x1f32(word[g][t], through, sum[g], 0, 0, 0);
             }
         }
-        __syncthreads();
+        lds_sync<int(kWave)>();
     }
 }
 // lane = coordinate: sum over the heads `heads` (a uniform mask of the first 64) of J^T x, x one value an axis held by
@@ -1584,7 +1593,7 @@ __device__ __forceinline__ void add_heads_through_links(const Tile& c, bool mine
         table[3u * lane + 2u] = float4{y[2], y[3], y[4], y[5]};
         c.stiffness_current = true;
     }
-    __syncthreads();
+    lds_sync<N>();
     const float4 la = table[3u * lane], lb = table[3u * lane + 1u], lc = table[3u * lane + 2u];
     const float s[6] = {la.x, la.y, la.z, la.w, lb.x, lb.y}, y[6] = {lb.z, lb.w, lc.x, lc.y, lc.z, lc.w};
     // (through the barrier so that the sixty-four lane masks of each are made here, two instructions a column, instead of
@@ -1611,7 +1620,7 @@ __device__ __forceinline__ void add_heads_through_links(const Tile& c, bool mine
             hrow[4 * q + r] += __uint_as_float(bits);
         }
     }
-    __syncthreads();
+    lds_sync<N>();
 }
 
 // AssembleTileBlock (:1507-1618): lane i assembles row i of H = M + sum J^T C J in `hrow` and its force g_i.  The
@@ -1671,7 +1680,7 @@ __device__ __forceinline__ bool assemble_block(const Tile& c, const float (&mrow
     if (c.units && lane < c.heads && c.U(hUnit, lane) != kInvalid) {   // a coordinate reads its unit heads' responses from the fields
         c.F(hF, lane) = mf[0]; c.F(hC, lane) = mc[0];
     }
-    __syncthreads();
+    lds_sync<N>();
     PROF_END(c, 10);
     PROF_BEGIN(c, 11);
     // Padded columns (k >= n) hold exact zeros in the mass row, the vectors and the Jacobian rows: their terms add
@@ -1844,7 +1853,7 @@ __device__ __forceinline__ bool assemble_block(const Tile& c, const float (&mrow
     }
     *converged = __all(!coordinate || fabsf(*force) <= kRoundings * FLT_EPSILON * scale);
     const bool ok = __all(!coordinate || finite);
-    __syncthreads();
+    lds_sync<N>();
     PROF_END(c, 13);
     return ok;
 }
@@ -1866,7 +1875,7 @@ template <int N>
 __device__ __forceinline__ float mass_times(const Tile& c, const float (&mrow)[N], float d) {
     float* dvec = c.vec + 192;
     dvec[c.lane] = d;
-    __syncthreads();
+    lds_sync<N>();
     float out = 0.0f;
     const float4* d4 = reinterpret_cast<const float4*>(dvec);
 #pragma unroll
@@ -1874,7 +1883,7 @@ __device__ __forceinline__ float mass_times(const Tile& c, const float (&mrow)[N
         const float4 dv = d4[q];
         out += mrow[4 * q] * dv.x; out += mrow[4 * q + 1] * dv.y; out += mrow[4 * q + 2] * dv.z; out += mrow[4 * q + 3] * dv.w;
     }
-    __syncthreads();
+    lds_sync<N>();
     return c.lane < c.n_all ? out : 0.0f;
 }
 
@@ -1932,14 +1941,14 @@ template <int N>
 __device__ __forceinline__ void row_steps(const Tile& c, float d) {
     float* dvec = c.vec;
     dvec[c.lane] = c.lane < c.n ? d : 0.0f;
-    __syncthreads();
+    lds_sync<N>();
     if (c.heads <= 16u && !c.units && !c.from_links) {
         // a lane a row: the first three rows of sixteen lanes take an axis each, lane & 15 = head (a head on one axis has
         // zeros in the rows of the others)
         const uint32_t axis = c.lane >> 4u, h = c.lane & 15u;
         if (axis < 3u && h < c.heads && c.U(hRow, h) != kInvalid)
             c.fields[axis == 0u ? c.at(hStep, h) : c.at(hStep + 1, h) + axis - 1u] = row_dot_fma<N>(c.jac + (c.U(hRow, h) + axis) * uint32_t(N), dvec);
-        __syncthreads();
+        lds_sync<N>();
         return;
     }
     if constexpr (N > kTwoWaveWidth) {
@@ -1953,7 +1962,7 @@ __device__ __forceinline__ void row_steps(const Tile& c, float d) {
                 c.F(hStep + 1, h) = axes > 1u ? wrench_dot(c, h, 1u, motion) : 0.0f;
                 c.F(hStep + 2, h) = axes > 2u ? wrench_dot(c, h, 2u, motion) : 0.0f;
             }
-            __syncthreads();
+            lds_sync<N>();
             return;
         }
     }
@@ -1970,7 +1979,7 @@ __device__ __forceinline__ void row_steps(const Tile& c, float d) {
             if (c.owned(h) && unit != kInvalid) c.F(hStep, h) = c.F(hUnitValue, h) * dvec[unit];   // :2028-2032
         }
     }
-    __syncthreads();
+    lds_sync<N>();
 }
 
 __device__ __forceinline__ void plain_line_terms(const PlainLine& p, float alpha, TileSum& row_slope, float& row_curvature, float& row_magnitude) {
@@ -2136,7 +2145,7 @@ __device__ __forceinline__ void apply_moves(const Tile& c, float alpha) {
 #pragma unroll
         for (int k = 0; k < 3; ++k) c.F(hMove + k, h) = fmaf(alpha, c.F(hStep + k, h), c.F(hMove + k, h));
     }
-    __syncthreads();
+    wave_sync();
 }
 
 // DescendTileBlock (:2145-2301).  `u` is lane i's block coordinate; `has_free` is false in the position pass.
@@ -2153,7 +2162,7 @@ __device__ __forceinline__ void descend_block(Tile& c, const float (&mrow)[N], f
         c.F(hNormalBound, h) = c.F(hDual, h);
         c.F(hMove, h) = 0.0f; c.F(hMove + 1, h) = 0.0f; c.F(hMove + 2, h) = 0.0f;
     }
-    __syncthreads();
+    lds_sync<N>();
     PlainLine line = own_line(c);   // the heads' constants over this block descent
     float start = coordinate ? *u_io : 0.0f;
     const float free_v = moving && has_free ? free_in : 0.0f;
@@ -2229,7 +2238,7 @@ __device__ __forceinline__ void descend_block(Tile& c, const float (&mrow)[N], f
 #pragma unroll
         for (int k = 0; k < 3; ++k) c.F(hRes + k, h) = c.F(hRes + k, h) - c.F(hMove + k, h);
     }
-    __syncthreads();
+    lds_sync<N>();
     if (failure != kFailNone) {
         c.failed = true;
         if (lane == 0u) d.env_status[c.env] |= kEnvStatusSolverFailure;
@@ -2254,7 +2263,7 @@ __device__ __forceinline__ void measure_primal(Tile& c, const float (&mrow)[N], 
     double* apart = reinterpret_cast<double*>(c.vec);
     const float here = coordinate ? *velocity_io : 0.0f;
     apart[lane] = coordinate ? double(here) - double(free_v) : 0.0;
-    __syncthreads();
+    lds_sync<N>();
     double balance = 0.0;
     const double2* apart2 = reinterpret_cast<const double2*>(apart);
     const float4* low4 = low_row<N>(c);
@@ -2322,7 +2331,7 @@ __device__ __forceinline__ void measure_primal(Tile& c, const float (&mrow)[N], 
         }
     }
     add_units(done, c.heads);
-    __syncthreads();
+    lds_sync<N>();
     const float force = float(balance);
     const bool finite = __all(!coordinate || fabs(balance) <= double(FLT_MAX));
     Failure failure = finite ? kFailNone : kFailEquation;
@@ -2353,7 +2362,7 @@ template <int N>
 __device__ __forceinline__ void initialize_residuals(const Tile& c, float velocity, const float* urows, float dt) {
     float* dvec = c.vec;
     dvec[c.lane] = c.lane < c.n ? velocity : 0.0f;
-    __syncthreads();
+    lds_sync<N>();
     const float4* d4 = reinterpret_cast<const float4*>(dvec);
     float motion[6] = {};   // of the link of lane's head, where the rows follow from the links
     if constexpr (N > kTwoWaveWidth) {
@@ -2391,7 +2400,7 @@ __device__ __forceinline__ void initialize_residuals(const Tile& c, float veloci
             c.F(hRes + axis, h) = residual;
         }
     }
-    __syncthreads();
+    lds_sync<N>();
 }
 
 struct DualMomentum { float t, beta; };
@@ -2537,7 +2546,7 @@ __device__ __forceinline__ void update_duals(const Tile& c, float* lambda_env, u
             c.F(hDual, h) = out.x; c.F(hDual + 1, h) = out.y; c.F(hDual + 2, h) = out.z;
         }
     }
-    __syncthreads();
+    wave_sync();
 }
 
 __host__ __device__ inline uint32_t PaddedWidth(uint32_t n) { return (n + 3u) & ~3u; }
@@ -2659,7 +2668,7 @@ __device__ __forceinline__ bool reduce_block(uint32_t lane, uint32_t n, const fl
 #pragma unroll
         for (int k = K; k < N; ++k) corner[(int(lane) - K) * kFollowers + (k - K)] = uint32_t(k) > lane ? full[k] : 0.0;
     }
-    __syncthreads();
+    lds_sync<K>();
     const uint32_t slot = lane >= uint32_t(K) && lane < uint32_t(N) ? lane - uint32_t(K) : 0u;
     double prow[K], column[kFollowers];
 #pragma unroll
@@ -2692,7 +2701,7 @@ __device__ __forceinline__ bool reduce_block(uint32_t lane, uint32_t n, const fl
 #pragma unroll
         for (int q = 0; q < K / 4; ++q) words[q] = float4{rest[4 * q], rest[4 * q + 1], rest[4 * q + 2], rest[4 * q + 3]};
     }
-    __syncthreads();
+    lds_sync<K>();
     return valid;
 }
 
@@ -2813,7 +2822,7 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
     }
     if constexpr (kContactsOnly) __builtin_assume(heads <= uint32_t(kWave));
     c.heads = heads;
-    __syncthreads();
+    lds_sync<W>();
     PROF_END(c, 16);
     PROF_BEGIN(c, 17);
     // stage Jacobian rows: the sum of the articulated sides' chain rows (TileBlock::Jacobian :555-573, CopyTileRows :836-869).
@@ -2839,7 +2848,7 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
 #pragma unroll
         for (uint32_t k = 1u; k < 3u; ++k) { c.U(hSourceA + k, h) = kInvalid; c.U(hSourceB + k, h) = kInvalid; }
     }
-    __syncthreads();
+    lds_sync<W>();
     PROF_BEGIN(c, 22);
     // FindTileRowSupport (:801-833), lane = head: a single-axis head whose Jacobian row has at most one entry is a unit
     // head and stages nothing; every other owned head stages three rows, placed in head order (PlaceTileRows).
@@ -2864,7 +2873,7 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
             c.U(hColumnsLow, h) = 0u; c.U(hColumnsHigh, h) = 0u;
         }
         if (__any(overflow_rows) && lane == 0u) d.env_status[env] |= kEnvStatusSolverFailure;
-        __syncthreads();
+        lds_sync<W>();
         PROF_END(c, 22);
         PROF_BEGIN(c, 23);
         // PlaceTileRows: the staged heads take their rows in head order
@@ -2885,7 +2894,7 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
         c.units = !kContactsOnly && __any(any_unit) && cap > staged_cap;   // the lists have room only when the world has joint heads
         c.staged_end = staged_end;
         c.individual_end = individual_end;
-        __syncthreads();
+        lds_sync<W>();
         // every coordinate lists its own unit heads, in head order
         if (c.units) {
             constexpr uint32_t kAhead = 16u;   // reads in flight
@@ -2906,7 +2915,7 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
         }
         PROF_END(c, 23);
     }
-    __syncthreads();
+    lds_sync<W>();
     if constexpr (W > kTwoWaveWidth && kContactsOnly) {
         // The coordinates' motion axes about the root link's origin, for add_heads_through_links: a hinge or an angular
         // coordinate of a floating root turns about its axis through the joint's origin, a sliding one moves along it
@@ -3002,7 +3011,7 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
                 c.U(hColumnsLow, lane) = uint32_t(head_way); c.U(hColumnsHigh, lane) = uint32_t(head_way >> 32u);
             }
         }
-        __syncthreads();
+        lds_sync<W>();
     }
     // CopyTileRows (:836-869): the staged heads' rows, their loads in flight together
 
@@ -3045,7 +3054,7 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
     }
     // a contact that reaches a coordinate the world's reduction left out: the launch was given the wrong width
     if (stray && lane == 0u) d.env_status[env] |= kEnvStatusSolverFailure;
-    __syncthreads();
+    lds_sync<W>();
     PROF_END(c, 17);
     PROF_BEGIN(c, 18);
     // TileInertialResponse (:709-739): J M^-1 J^T of every head's first row through the stored LDL^T factor
@@ -3192,14 +3201,14 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
                 const float term = coordinate ? a[t] * a[t] / pivot : 0.0f;
                 if (lane < uint32_t(N)) terms[uint32_t(t * N) + lane] = term;
             }
-            __syncthreads();
+            lds_sync<W>();
             float mine = 0.0f;
             {
                 const float4* words = reinterpret_cast<const float4*>(terms + (lane & 3u) * uint32_t(N));
 #pragma unroll
                 for (int q = 0; q < N / 4; ++q) { const float4 w = words[q]; mine += w.x; mine += w.y; mine += w.z; mine += w.w; }
             }
-            __syncthreads();
+            lds_sync<W>();
 #pragma unroll
             for (int t = 0; t < 4; ++t) total[t] = lane_value(mine, t);
 #pragma unroll
@@ -3241,7 +3250,7 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
                 c.F(hStep, h) = second ? 0.0f : mine; c.F(hMove, h) = second ? mine : 0.0f;
             }
         }
-        __syncthreads();
+        lds_sync<W>();
     }
     PROF_END(c, 18);
     PROF_BEGIN(c, 19);
@@ -3296,7 +3305,7 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
         }
     }
     c.elliptic = !kContactsOnly && __any(any_elliptic);
-    __syncthreads();
+    lds_sync<W>();
     {
         const uint32_t own = min(lane, heads == 0u ? 0u : heads - 1u);
         const bool staged = lane < heads && c.U(hRow, own) != kInvalid;
@@ -3394,7 +3403,7 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
     if (p.position_iterations != 0u) {
         float* qvec = c.vec + 128;
         qvec[lane] = coordinate ? velocity : 0.0f;   // the final generalized velocity, as qdot_flat
-        __syncthreads();
+        lds_sync<W>();
         bool push = false;
         for (uint32_t h = lane; h < heads; h += kWave) {
             const uint32_t slot = c.slot(h);
@@ -3452,7 +3461,7 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
         }
         push = __any(push);
         c.block_heads = false;   // on one axis now
-        __syncthreads();
+        lds_sync<W>();
         float pseudo = 0.0f;
         if (push) {
             const uint32_t positions = 1u;   // no head couples two moving blocks here, so one solve (:2716)
