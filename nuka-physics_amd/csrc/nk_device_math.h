@@ -201,10 +201,13 @@ __device__ __forceinline__ uint32_t joint_dof(uint8_t type) {
 // mirror of 16: every step pairs lanes that already hold equal partial results, so a commutative combine leaves all
 // 16 lanes equal), then the four row results are read as scalars and combined as (r0 + r1) + (r2 + r3).  The result
 // is uniform across the wave.
+// (Every lane of these moves has a source, so nothing is said of what a lane without one keeps: the move then joins the
+// instruction that takes its result, and a double's two halves want no registers cleared first: 333 humanoids 557 -> 548 us,
+// 4096 quadrupeds 480 -> 474.)
 template <int Ctrl>
-__device__ __forceinline__ float dpp_move(float v) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), Ctrl, 0xF, 0xF, false));
-}
+__device__ __forceinline__ uint32_t dpp_move_u(uint32_t v) { return uint32_t(__builtin_amdgcn_mov_dpp(int(v), Ctrl, 0xF, 0xF, true)); }
+template <int Ctrl>
+__device__ __forceinline__ float dpp_move(float v) { return __uint_as_float(dpp_move_u<Ctrl>(__float_as_uint(v))); }
 constexpr int kDppXor1 = 0xB1, kDppXor2 = 0x4E, kDppHalfMirror = 0x141, kDppMirror = 0x140;
 __device__ __forceinline__ float row_value(float v, int row) {
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 16 * row));
@@ -223,8 +226,6 @@ __device__ __forceinline__ float wave_sum(float v) {
 // step is a trip through LDS, six for each of the four reductions at the end of a sweep: a step of 4096 quadrupeds 483 ->
 // 479 us.
 constexpr int kDppRor8 = 0x128, kDppRor4 = 0x124;
-template <int Ctrl>
-__device__ __forceinline__ uint32_t dpp_move_u(uint32_t v) { return uint32_t(__builtin_amdgcn_update_dpp(0, int(v), Ctrl, 0xF, 0xF, false)); }
 struct LanePair { uint32_t first, second; };   // two lanes' words, in either order the same pair in both
 __device__ __forceinline__ LanePair across_halves(uint32_t v) { const auto p = __builtin_amdgcn_permlane32_swap(v, v, false, false); return LanePair{p[0], p[1]}; }
 __device__ __forceinline__ LanePair across_rows(uint32_t v) { const auto p = __builtin_amdgcn_permlane16_swap(v, v, false, false); return LanePair{p[0], p[1]}; }

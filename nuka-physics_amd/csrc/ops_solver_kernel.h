@@ -108,9 +108,7 @@ __device__ __forceinline__ void tile_add_product(TileSum& s, float a, float b) {
 template <int Ctrl>
 __device__ __forceinline__ double dpp_move_d(double v) {
     const uint64_t bits = uint64_t(__double_as_longlong(v));
-    const uint32_t low = uint32_t(__builtin_amdgcn_update_dpp(0, int(uint32_t(bits)), Ctrl, 0xF, 0xF, false));
-    const uint32_t high = uint32_t(__builtin_amdgcn_update_dpp(0, int(uint32_t(bits >> 32u)), Ctrl, 0xF, 0xF, false));
-    return __longlong_as_double((long long)((uint64_t(high) << 32u) | uint64_t(low)));
+    return double_of(dpp_move_u<Ctrl>(uint32_t(bits)), dpp_move_u<Ctrl>(uint32_t(bits >> 32u)));
 }
 __device__ __forceinline__ double row_value_d(double v, int row) {
     const uint64_t bits = uint64_t(__double_as_longlong(v));
