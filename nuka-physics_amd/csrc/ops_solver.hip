@@ -30,6 +30,8 @@ NKH_DECLARE_DENSE(4, 4) NKH_DECLARE_DENSE(8, 8) NKH_DECLARE_DENSE(12, 12) NKH_DE
 NKH_DECLARE_DENSE(24, 12) NKH_DECLARE_DENSE(28, 16) NKH_DECLARE_DENSE(32, 16) NKH_DECLARE_DENSE(36, 20) NKH_DECLARE_DENSE(40, 20)
 #undef NKH_DECLARE_DENSE
 }  // namespace dense
+__host__ __device__ uint32_t PackedEnvFloats(uint32_t staged);
+__global__ void PackedDescentKernel(ModelView, DataView, BlockDescentSolveParams, uint32_t, uint32_t);
 }  // namespace solver
 
 
@@ -190,7 +192,19 @@ static SolverKernel KernelOfWidth(const ModelView& m, bool contacts_only, uint32
             if (reduced.width == solver::PaddedWidth(m.dof) && reduced.reduced == width) return reduced.kernel;
     return kSolverKernels[contacts_only ? 1 : 0][solver::PaddedWidth(m.dof) / 4u - 1u];
 }
-// Blocks (one wavefront, one environment each) of a world's full-capacity solve launch that a compute unit holds at
+// Worlds whose environments are solved four a wavefront (ops_solver_packed.hip): contact heads only, no more of them and no
+// more coordinates than a row of sixteen lanes takes.  From a batch on that has wavefronts enough that way: a wavefront
+// of four takes longer than any of them alone, and 2048 free boxes step in 259 us one a wavefront, 324 packed (8192 342
+// and 339).
+constexpr uint32_t kPackedBatch = 8192u;
+static bool PackedSolverTakes(const ModelView& m, bool contacts_only, uint32_t staged, uint32_t env_count) {
+    return contacts_only && m.dof <= uint32_t(solver::kPackedWidth) && m.max_dof <= 16u && staged <= solver::kPackedHeads && env_count >= kPackedBatch;
+}
+// Environments that have a wavefront to themselves, the costliest: one a compute unit until the others' wavefronts take
+// longer than they do (16384 free boxes 429 us without them, 392 with; 65536 981 and 989).
+static uint32_t PackedAlone(uint32_t env_count) { return env_count < 3u * kPackedBatch ? uint32_t(kUnits) : 0u; }
+static size_t PackedLdsBytes(uint32_t staged) { return size_t{kPackedEnvs} * PackedEnvFloats(staged) * sizeof(float); }
+// Blocks (one wavefront each, one environment or four) of a world's full-capacity solve launch that a compute unit holds at
 // once, as the runtime's occupancy query answers for the kernel and the LDS the launch asks for; 0 without a solve.
 uint32_t SolverBlocksPerUnit(const ModelView& m, uint32_t env_count) {
     if (m.rows_per_env == 0u || m.dof == 0u) return 0u;
@@ -202,6 +216,13 @@ uint32_t SolverBlocksPerUnit(const ModelView& m, uint32_t env_count) {
     const size_t lds = size_t{solver::ReducedSolverLdsFloats(m.dof, width, staged + joint_heads, staged,
                                                              solver::RowsFromLinks(width, contacts_only, m.rows_from_links))} * sizeof(float);
     int blocks = 0;
+    if (PackedSolverTakes(m, contacts_only, staged, env_count)) {
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, reinterpret_cast<const void*>(PackedDescentKernel), solver::kWave, PackedLdsBytes(staged)) != hipSuccess) {
+            (void)hipGetLastError();
+            return 0u;
+        }
+        return uint32_t(std::max(blocks, 0));
+    }
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, reinterpret_cast<const void*>(KernelOfWidth(m, contacts_only, width, env_count)),
                                                      solver::kWave, lds) != hipSuccess) {
         (void)hipGetLastError();
@@ -260,6 +281,12 @@ Status OpBlockDescentSolve(const ModelView& m, const DataView& d, const void* pa
     // edges a point under the pyramidal cone.  (While those worlds went to the one full launch, a walker's 304 heads left a
     // compute unit one block for environments of a handful of points: a step of 4096 with a twentieth reset 768 -> 438 us.)
     hipLaunchKernelGGL(OrderTilesKernel, dim3((p->env_count + kOrderEnvs - 1u) / kOrderEnvs), dim3(1024), 0, stream, d, p->env_count);
+    if (PackedSolverTakes(m, contacts_only, staged, p->env_count)) {
+        const uint32_t alone = PackedAlone(p->env_count);
+        hipLaunchKernelGGL(PackedDescentKernel, dim3(alone + (p->env_count - alone + kPackedEnvs - 1u) / kPackedEnvs), dim3(solver::kWave),
+                           PackedLdsBytes(staged), stream, m, d, *p, staged, alone);
+        return hipGetLastError() == hipSuccess ? Status::Ok : Status::Failed;
+    }
     uint32_t first_points = 0u;
     const uint32_t a_point = HeadsAPoint(m);
     const bool few_rounds = p->env_count < kManyRounds * kUnits * blocks_per_unit(staged);

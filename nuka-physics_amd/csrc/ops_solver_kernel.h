@@ -62,6 +62,10 @@ constexpr int WavesPerSimd(int width) { return width <= kTwoWaveWidth ? 2 : 1; }
 #endif
 #endif
 constexpr int kWidenAtUse = NKH_WIDEN_AT_USE;
+// The blocks that are solved four a wavefront (ops_solver_packed.hip): the coordinates and heads a row of sixteen lanes takes
+constexpr int kPackedWidth = 8;
+constexpr uint32_t kPackedHeads = 16u, kPackedEnvs = 4u;
+constexpr int kPackedWaves = 3;   // a SIMD
 // Orders the block's LDS words between its lanes.  A block is one wavefront, whose LDS accesses are taken in order, so nothing
 // has to be waited for; a barrier of the workgroup waits for the writes all the same, some twenty times a Newton step (333
 // humanoids 567 -> 557 us, 4096 743 -> 732, 65536 7758 -> 7678).  A wide block keeps the barrier: without it reads move
