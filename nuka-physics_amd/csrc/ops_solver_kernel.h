@@ -247,27 +247,44 @@ __device__ __forceinline__ EllipticResponse elliptic_response(float cap, float c
     return EllipticResponse{float(cap * normal_scale), float(cap * tangent_scale * tangent / cy), float(cap * tangent_scale * tangent / cz),
                             float(normal_scale), float(tangent_scale)};
 }
-// EvaluateEllipticImpulse (augmented_row.hpp:58-80): the projection onto the friction cone in the metric that makes
-// its cross section a circle; curvature xx yy zz xy xz yz
-__device__ __forceinline__ void elliptic_impulse(V3 dual, float cap, float rx, float ry, float rz, float cn, float cy, float cz, float mu_first,
-                                                 float* f, float* cv) {
-    const EllipticResponse e = elliptic_response(cap, cn, cy, cz);
-    const float xx = fmaf(e.kx, rx, e.sx * dual.x), xy = fmaf(e.ky, ry, e.st * dual.y), xz = fmaf(e.kz, rz, e.st * dual.z);
-    const float root_x = sqrtf(e.kx), root_y = sqrtf(e.ky), root_z = sqrtf(e.kz);
-    const float m = mu_first * root_x / root_y;
-    const float p = xx / root_x, q1 = xy / root_y, q2 = xz / root_z;
+// What of EvaluateEllipticImpulse (augmented_row.hpp:58-80) depends on the row alone: the response, the roots of its residual
+// scales, the cone's slope in the metric that makes its cross section a circle, and 1 / (1 + slope^2).  A head keeps them from
+// its set-up on (three double-precision quotients and four roots, some 350 instructions, were made again at every probe of
+// a line: 3.0 k cycles a probe of the elliptic humanoid's longest environment, 1.2 k of a Coulomb one).
+struct EllipticCone { EllipticResponse e; float root_x, root_y, root_z, slope, share; };
+__device__ __forceinline__ EllipticCone elliptic_cone(float cap, float cn, float cy, float cz, float mu_first) {
+    EllipticCone k;
+    k.e = elliptic_response(cap, cn, cy, cz);
+    k.root_x = sqrtf(k.e.kx); k.root_y = sqrtf(k.e.ky); k.root_z = sqrtf(k.e.kz);
+    k.slope = mu_first * k.root_x / k.root_y;
+    k.share = 1.0f / (1.0f + k.slope * k.slope);
+    return k;
+}
+// The rest: the projection onto the friction cone; curvature xx yy zz xy xz yz.  Inside, outside and on the cone are
+// computed side by side and one is selected, so that a probe carries no branch; the quotients by one divisor share its reciprocal.
+struct EllipticLine { EllipticCone k; float scaled[3]; Recip by_x, by_y, by_z; };   // with the scaled duals, over a block descent
+__device__ __forceinline__ EllipticLine elliptic_line(const EllipticCone& k, V3 dual) {
+    return EllipticLine{k, {k.e.sx * dual.x, k.e.st * dual.y, k.e.st * dual.z}, make_recip(k.root_x), make_recip(k.root_y), make_recip(k.root_z)};
+}
+__device__ __forceinline__ void elliptic_impulse(const EllipticLine& l, float rx, float ry, float rz, float* f, float* cv) {
+    const EllipticResponse& e = l.k.e;
+    const float root_x = l.k.root_x, root_y = l.k.root_y, root_z = l.k.root_z, m = l.k.slope, a = l.k.share;
+    const float xx = fmaf(e.kx, rx, l.scaled[0]), xy = fmaf(e.ky, ry, l.scaled[1]), xz = fmaf(e.kz, rz, l.scaled[2]);
+    const float p = div_by(xx, l.by_x), q1 = div_by(xy, l.by_y), q2 = div_by(xz, l.by_z);
     const float t = hypotf(q1, q2);
-    f[0] = f[1] = f[2] = 0.0f;
-    cv[0] = cv[1] = cv[2] = cv[3] = cv[4] = cv[5] = 0.0f;
-    if (t <= m * p) { f[0] = xx; f[1] = xy; f[2] = xz; cv[0] = e.kx; cv[1] = e.ky; cv[2] = e.kz; return; }
-    if (m * t + p <= 0.0f) return;
-    const float a = 1.0f / (1.0f + m * m);
+    const bool inside = t <= m * p, outside = !inside && m * t + p <= 0.0f;
     const float projected = (p + m * t) * a;
-    const float u1 = q1 / t, u2 = q2 / t;
-    const float b = m * projected / t, along = m * m * a;
-    f[0] = projected * root_x; f[1] = m * projected * u1 * root_y; f[2] = m * projected * u2 * root_z;
-    cv[0] = e.kx * a; cv[1] = e.ky * (along * u1 * u1 + b * u2 * u2); cv[2] = e.kz * (along * u2 * u2 + b * u1 * u1);
-    cv[3] = root_x * root_y * m * a * u1; cv[4] = root_x * root_z * m * a * u2; cv[5] = root_y * root_z * (along - b) * u1 * u2;
+    const Recip by_t = make_recip(t);
+    const float u1 = div_by(q1, by_t), u2 = div_by(q2, by_t);
+    const float b = div_by(m * projected, by_t), along = m * m * a;
+    const auto one_of = [&](float within, float on) { return inside ? within : outside ? 0.0f : on; };
+    f[0] = one_of(xx, projected * root_x); f[1] = one_of(xy, m * projected * u1 * root_y); f[2] = one_of(xz, m * projected * u2 * root_z);
+    cv[0] = one_of(e.kx, e.kx * a);
+    cv[1] = one_of(e.ky, e.ky * (along * u1 * u1 + b * u2 * u2));
+    cv[2] = one_of(e.kz, e.kz * (along * u2 * u2 + b * u1 * u1));
+    cv[3] = one_of(0.0f, root_x * root_y * m * a * u1);
+    cv[4] = one_of(0.0f, root_x * root_z * m * a * u2);
+    cv[5] = one_of(0.0f, root_y * root_z * (along - b) * u1 * u2);
 }
 
 __device__ __forceinline__ uint32_t residual_bits(float value) { return __float_as_uint(value <= FLT_MAX ? fabsf(value) : FLT_MAX); }
@@ -295,6 +312,11 @@ constexpr uint32_t kUnowned = 0x80000000u;
 // is), so the first two words of hRelaxStep hold what it needs instead: the compliances of its two tangent rows.
 constexpr uint32_t kAxesElliptic = 4u;
 constexpr uint32_t hTangentCompliance = hRelaxStep;
+// ... and one of the first 64 its cone's constants (EllipticCone, ten words) in the rest of that state and where only heads
+// past the 64th and unit heads keep their curvature.
+constexpr uint32_t kConeWords = 10u;
+__device__ __forceinline__ constexpr uint32_t cone_field(uint32_t word) { return word < 5u ? hRelaxStep + 2u + word : hC + (word - 5u); }
+static_assert(hRelaxPoint == hRelaxStep + 4u && hC == hRelaxPoint + 3u, "five words of the relaxation state from its third on");
 __device__ __forceinline__ bool block_axes(uint32_t axes) { return axes >= 3u; }
 
 // A head on one axis uses the first component of every three-component field and none of the block-only fields;
@@ -389,6 +411,21 @@ struct Tile {
     __device__ __forceinline__ bool owned(uint32_t h) const { return (U(hSlot, h) & kUnowned) == 0u; }
 };
 
+// the cone of head h, which is under the elliptic cone
+__device__ __forceinline__ void keep_cone(const Tile& c, uint32_t h, const EllipticCone& k) {
+    const float words[kConeWords] = {k.e.kx, k.e.ky, k.e.kz, k.e.sx, k.e.st, k.root_x, k.root_y, k.root_z, k.slope, k.share};
+#pragma unroll
+    for (uint32_t w = 0u; w < kConeWords; ++w) c.F(cone_field(w), h) = words[w];
+}
+__device__ __forceinline__ EllipticCone cone_of(const Tile& c, uint32_t h) {
+    if (h >= uint32_t(kWave))
+        return elliptic_cone(c.F(hRho, h), c.F(hCompliance, h), c.F(hTangentCompliance, h), c.F(hTangentCompliance + 1, h), c.F(hMu1, h));
+    float w[kConeWords];
+#pragma unroll
+    for (uint32_t k = 0u; k < kConeWords; ++k) w[k] = c.F(cone_field(k), h);
+    return EllipticCone{EllipticResponse{w[0], w[1], w[2], w[3], w[4]}, w[5], w[6], w[7], w[8], w[9]};
+}
+
 // lane's row of Tile::low, as sixteen-byte words
 template <int N>
 __device__ __forceinline__ const float4* low_row(const Tile& c) { return reinterpret_cast<const float4*>(c.low + min(c.lane, uint32_t(N - 1)) * uint32_t(N)); }
@@ -397,9 +434,8 @@ __device__ __forceinline__ const float4* low_row(const Tile& c) { return reinter
 __device__ __forceinline__ void head_response(const Tile& c, uint32_t h, float mx, float my, float mz, float* f, float* cv) {
     const float rho = c.F(hRho, h);
     if (c.elliptic && c.U(hAxes, h) == kAxesElliptic) {   // block_descent.cu:1595-1601
-        elliptic_impulse(V3{c.F(hDual, h), c.F(hDual + 1, h), c.F(hDual + 2, h)}, rho, c.F(hRes, h) - mx, c.F(hRes + 1, h) - my,
-                         c.F(hRes + 2, h) - mz, c.F(hCompliance, h), c.F(hTangentCompliance, h), c.F(hTangentCompliance + 1, h),
-                         c.F(hMu1, h), f, cv);
+        elliptic_impulse(elliptic_line(cone_of(c, h), V3{c.F(hDual, h), c.F(hDual + 1, h), c.F(hDual + 2, h)}), c.F(hRes, h) - mx,
+                         c.F(hRes + 1, h) - my, c.F(hRes + 2, h) - mz, f, cv);
         return;
     }
     float ni, nc;
@@ -1100,7 +1136,7 @@ __device__ __forceinline__ void add_heads_by_groups(const Tile& c, uint64_t head
 struct HeadLine {
     uint32_t head;
     bool owned, contact, bounded, cone, elliptic;
-    float tangent_compliance[2], mu_first;
+    EllipticLine on_cone;   // of an elliptic head
     float rho, compliance, lower, upper, bound;
     Response response;
     TangentRatios ratios;
@@ -1115,7 +1151,7 @@ __device__ __forceinline__ HeadLine load_head_line(const Tile& c, uint32_t h) {
     if (!l.owned) return l;
     l.contact = block_axes(c.U(hAxes, h));
     l.elliptic = c.elliptic && c.U(hAxes, h) == kAxesElliptic;
-    if (l.elliptic) { l.tangent_compliance[0] = c.F(hTangentCompliance, h); l.tangent_compliance[1] = c.F(hTangentCompliance + 1, h); l.mu_first = c.F(hMu1, h); }
+    if (l.elliptic) l.on_cone = elliptic_line(cone_of(c, h), V3{c.F(hDual, h), c.F(hDual + 1, h), c.F(hDual + 2, h)});
     l.rho = c.F(hRho, h); l.compliance = c.F(hCompliance, h); l.lower = c.F(hLower, h); l.upper = c.F(hUpper, h);
     l.bound = c.F(hNormalBound, h);
     l.response = Response{c.F(hDualScale, h), c.F(hResidualScale, h)};
@@ -1160,8 +1196,7 @@ __device__ __forceinline__ void line_terms(const HeadLine& l, float alpha, TileS
     const float sx = l.step[0], sy = l.step[1], sz = l.step[2];
     float f[3] = {0.0f, 0.0f, 0.0f}, r[6] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
     if (l.elliptic) {
-        elliptic_impulse(V3{l.dual[0], l.dual[1], l.dual[2]}, l.rho, l.res[0] - fmaf(alpha, sx, l.move[0]), l.res[1] - fmaf(alpha, sy, l.move[1]),
-                         l.res[2] - fmaf(alpha, sz, l.move[2]), l.compliance, l.tangent_compliance[0], l.tangent_compliance[1], l.mu_first, f, r);
+        elliptic_impulse(l.on_cone, l.res[0] - fmaf(alpha, sx, l.move[0]), l.res[1] - fmaf(alpha, sy, l.move[1]), l.res[2] - fmaf(alpha, sz, l.move[2]), f, r);
         add_line_terms(f, r, sx, sy, sz, row_slope, row_curvature, row_magnitude);
         row_magnitude += line_noise(r, l.res[0], l.res[1], l.res[2], fmaf(alpha, sx, l.move[0]), fmaf(alpha, sy, l.move[1]), fmaf(alpha, sz, l.move[2]), sx, sy, sz);
         return;
@@ -1643,13 +1678,13 @@ __device__ __forceinline__ bool assemble_block(const Tile& c, const float (&mrow
     PROF_BEGIN(c, 10);
     // lane's own head (the first 64 heads) from its constants, without a branch; a lane without an owned head gets zeros
     float mf[3], mc[6], mn[3];
-    {
+    if (c.elliptic) head_terms(c, lane, mf, mc, mn);   // the cone's own response; the same values as below for every other head
+    else {
         refresh_moves(c, own);
         plain_response(own, own.move[0], own.move[1], own.move[2], mf, mc);
 #pragma unroll
         for (int k = 0; k < 3; ++k) mn[k] = fabsf(mf[k]) + mc[k] * (fabsf(own.res[k]) + fabsf(own.move[k]));
     }
-    if (c.elliptic) head_terms(c, lane, mf, mc, mn);   // the cone's own response; the same values as above for every other head
     // whether anything of the head is not zero (lanes from the heads' count on hold copies of the first sixteen heads when
     // there are no more than that)
     const auto bits = [](float v) { return __float_as_uint(v); };
@@ -1995,11 +2030,11 @@ __device__ __forceinline__ void plain_line_terms(const PlainLine& p, float alpha
     row_magnitude += fabsf(f[0] * sx) + fabsf(f[1] * sy) + fabsf(f[2] * sz) + line_noise(r, p.res[0], p.res[1], p.res[2], mx, my, mz, sx, sy, sz);
     row_curvature += r[0] * sx * sx + r[1] * sy * sy + r[2] * sz * sz + 2.0f * r[5] * sy * sz;
 }
-// The line search runs in one of four modes, the same for every probe of a solve: general (some head is under the elliptic
-// cone, or later heads need more than a number a field), plain with the terms in the first sixteen lanes (narrow), plain
-// over the whole wavefront, plain with the heads past the first 64 as numbers beside it (later).  The mode is a template
-// argument so that the probes carry no branch on it.
-enum LineMode : int { kLineGeneral = 0, kLineWide = 1, kLineNarrow = 2, kLineLater = 3 };
+// The line search runs in one of five modes, the same for every probe of a solve: general (some head is under the elliptic
+// cone, or later heads need more than a number a field), general with at most sixteen heads (cone), plain with the terms in
+// the first sixteen lanes (narrow), plain over the whole wavefront, plain with the heads past the first 64 as numbers beside
+// it (later).  The mode is a template argument so that the probes carry no branch on it.
+enum LineMode : int { kLineGeneral = 0, kLineWide = 1, kLineNarrow = 2, kLineLater = 3, kLineCone = 4 };
 template <LineMode kMode>
 __device__ __forceinline__ void line_derivatives(const Tile& c, const HeadLine& mine, const PlainLine& plain, const ScalarLine (&later)[kLaterHeads], float alpha,
                                  float inertial_slope, float inertial_curvature, float* slope, float* curvature, float* magnitude) {
@@ -2013,6 +2048,8 @@ __device__ __forceinline__ void line_derivatives(const Tile& c, const HeadLine& 
             const HeadLine extra = load_head_line(c, h);
             if (extra.owned) line_terms(extra, alpha, row_slope, row_curvature, row_magnitude);
         }
+    } else if constexpr (kMode == kLineCone) {
+        if (mine.owned) line_terms(mine, alpha, row_slope, row_curvature, row_magnitude);
     } else {
         plain_line_terms(plain, alpha, row_slope, row_curvature, row_magnitude);
         if constexpr (kMode == kLineLater) {
@@ -2035,33 +2072,34 @@ __device__ __forceinline__ void line_derivatives(const Tile& c, const HeadLine& 
         tile_add_product(total, alpha, inertial_curvature);
         tile_add(total, inertial_slope);
     }
-    if constexpr (kMode == kLineNarrow) {
+    if constexpr (kMode == kLineNarrow || kMode == kLineCone) {
         // with at most sixteen heads every term sits in the first row of lanes; (t + 0) + (0 + 0) is t, so the sums agree
         *slope = wave_total(total, true);
         *curvature = inertial_curvature + first_row_sum(row_curvature);
         *magnitude = fabsf(inertial_slope) + alpha * inertial_curvature + first_row_sum(row_magnitude);
     } else {
-        // the general mode takes the first-row sums too when its heads fit the first sixteen lanes
-        const bool narrow = c.heads <= 16u;
-        *slope = wave_total(total, narrow);
-        *curvature = inertial_curvature + (narrow ? first_row_sum(row_curvature) : wave_sum(row_curvature));
-        *magnitude = fabsf(inertial_slope) + alpha * inertial_curvature + (narrow ? first_row_sum(row_magnitude) : wave_sum(row_magnitude));
+        *slope = wave_total(total);
+        *curvature = inertial_curvature + wave_sum(row_curvature);
+        *magnitude = fabsf(inertial_slope) + alpha * inertial_curvature + wave_sum(row_magnitude);
     }
     PROF_END(c, 25);
 }
 
-// The search always evaluates the line at 0 and then at 1.  In the narrow mode the rows of sixteen lanes hold copies of
+// The search always evaluates the line at 0 and then at 1.  In the narrow and cone modes the rows of sixteen lanes hold copies of
 // the same heads (lane & 15) and the row sums stay within a row: the first row evaluates the line at 0 while the others
 // evaluate it at 1, one pass for both points with the numbers either gives alone.  Each point's sums come out in its
 // row's lanes.
 struct LinePoint { float slope, curvature, magnitude; };
-__device__ __forceinline__ void line_derivatives_pair(const Tile& c, const PlainLine& plain, float inertial_slope, float inertial_curvature,
+template <LineMode kMode>
+__device__ __forceinline__ void line_derivatives_pair(const Tile& c, const HeadLine& mine, const PlainLine& plain, float inertial_slope, float inertial_curvature,
                                                       LinePoint* at_zero, LinePoint* at_one) {
     PROF_COUNT(c, 1);
     const float alpha = c.lane < 16u ? 0.0f : 1.0f;
     TileSum row_slope{0.0};
     float row_curvature = 0.0f, row_magnitude = 0.0f;
-    plain_line_terms(plain, alpha, row_slope, row_curvature, row_magnitude);
+    if constexpr (kMode == kLineCone) {
+        if (mine.owned) line_terms(mine, alpha, row_slope, row_curvature, row_magnitude);
+    } else plain_line_terms(plain, alpha, row_slope, row_curvature, row_magnitude);
     TileSum total{-row_slope.value};
     if ((c.lane & 15u) == 0u) {
         tile_add_product(total, alpha, inertial_curvature);
@@ -2082,7 +2120,7 @@ __device__ __forceinline__ void line_derivatives_pair(const Tile& c, const Plain
 // SearchTileLine (:2089-2125)
 template <LineMode kMode>
 __device__ __forceinline__ float search_line_in(const Tile& c, PlainLine& plain, float inertial_slope, float inertial_curvature) {
-    constexpr bool kPaired = kMode == kLineNarrow;
+    constexpr bool kPaired = kMode == kLineNarrow || kMode == kLineCone;
     float slope = 0.0f, curvature = 0.0f, magnitude = 0.0f;
     HeadLine mine{};
     ScalarLine later[kLaterHeads] = {};
@@ -2092,6 +2130,7 @@ __device__ __forceinline__ float search_line_in(const Tile& c, PlainLine& plain,
             if (c.heads > kWave * (e + 1u)) later[e] = scalar_line(c, c.lane + kWave * (e + 1u));
     }
     if constexpr (kMode == kLineGeneral) mine = load_head_line(c, c.lane);
+    else if constexpr (kMode == kLineCone) mine = load_head_line(c, c.lane & 15u);
     else refresh_steps(c, plain);
     float low = 0.0f, high = 0.0f, alpha = 1.0f;
     bool bounded = false;
@@ -2115,7 +2154,7 @@ __device__ __forceinline__ float search_line_in(const Tile& c, PlainLine& plain,
     float answer = 0.0f;
     if constexpr (kPaired) {
         LinePoint at_zero, at_one;
-        line_derivatives_pair(c, plain, inertial_slope, inertial_curvature, &at_zero, &at_one);
+        line_derivatives_pair<kMode>(c, mine, plain, inertial_slope, inertial_curvature, &at_zero, &at_one);
         c.work += 1u;
         initial = at_zero.slope;
         if (!(initial < 0.0f)) return 0.0f;
@@ -2136,6 +2175,7 @@ __device__ __forceinline__ float search_line_in(const Tile& c, PlainLine& plain,
 }
 __device__ __forceinline__ float search_line(const Tile& c, PlainLine& line, float inertial_slope, float inertial_curvature) {
     if (c.scalar_later) return search_line_in<kLineLater>(c, line, inertial_slope, inertial_curvature);
+    if (c.elliptic && c.heads <= 16u) return search_line_in<kLineCone>(c, line, inertial_slope, inertial_curvature);
     if (c.heads > uint32_t(kWave) || c.elliptic) return search_line_in<kLineGeneral>(c, line, inertial_slope, inertial_curvature);
     if (c.heads <= 16u) return search_line_in<kLineNarrow>(c, line, inertial_slope, inertial_curvature);
     return search_line_in<kLineWide>(c, line, inertial_slope, inertial_curvature);
@@ -2427,11 +2467,12 @@ __device__ __forceinline__ void update_duals(const Tile& c, float* lambda_env, u
         V3 dual{normal, 0.0f, 0.0f};
         V3 rstep{0, 0, 0}, rpoint{0, 0, 0};
         float rweight = 0.0f;
-        float cone_y = 0.0f, cone_z = 0.0f;
+        EllipticResponse cone{};
         if (elliptic) {   // :2509-2510: the projection onto the elliptic cone as it is
-            cone_y = c.F(hTangentCompliance, h); cone_z = c.F(hTangentCompliance + 1, h);
+            const EllipticLine line = elliptic_line(cone_of(c, h), tdual);
+            cone = line.k.e;
             float f[3], cv[6];
-            elliptic_impulse(tdual, rho, residual.x, residual.y, residual.z, compliance, cone_y, cone_z, mu1, f, cv);
+            elliptic_impulse(line, residual.x, residual.y, residual.z, f, cv);
             dual = V3{f[0], f[1], f[2]};
         } else if (contact) {   // ProjectRowDual (block_descent.cu:799-804) with RelaxContactImpulse (augmented_row.hpp:128-138)
             float fy, fz, cyy, czz, cyz;
@@ -2466,9 +2507,7 @@ __device__ __forceinline__ void update_duals(const Tile& c, float* lambda_env, u
             step_tangent = hypotf(first, second);
         }
         if (!commit && response.residual_scale > 0.0f) step_normal = fabsf(dual.x - tdual.x) / response.residual_scale;
-        EllipticResponse cone{};
         if (elliptic) {   // EllipticMultiplierStep (augmented_row.hpp:104-108; :2516-2519)
-            cone = elliptic_response(rho, compliance, cone_y, cone_z);
             step_normal = fabsf(dual.x - tdual.x) / cone.kx;
             step_tangent = fmaxf(fabsf(dual.y - tdual.y) / cone.ky, fabsf(dual.z - tdual.z) / cone.kz);
         }
@@ -3303,6 +3342,7 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
             if (elliptic) {
                 c.F(hTangentCompliance, h) = urows[size_t{slot + stride} * kRowWords + 5u];
                 c.F(hTangentCompliance + 1, h) = urows[size_t{slot + 2u * stride} * kRowWords + 5u];
+                if (h < uint32_t(kWave)) keep_cone(c, h, elliptic_cone(rho, compliance, c.F(hTangentCompliance, h), c.F(hTangentCompliance + 1, h), row[8]));
             }
         }
     }
