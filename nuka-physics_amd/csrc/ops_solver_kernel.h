@@ -3445,6 +3445,16 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
     if (p.position_iterations != 0u) {
         float* qvec = c.vec + 128;
         qvec[lane] = coordinate ? velocity : 0.0f;   // the final generalized velocity, as qdot_flat
+        // The contact slots' first rows, for the heads to find their slot's; a slot without points is nobody's.  (Heads that walked
+        // the slots and their Jacobian rows in memory, a trip for every word, were 10 us of the pass's 30 with 4096
+        // quadrupeds; a world with compliant contacts, whose heads hardly ever ask, lists none.)
+        const uint32_t listed = m.any_mujoco != 0u ? 0u : min(S, 128u);
+        uint32_t* slot_rows = reinterpret_cast<uint32_t*>(c.vec);
+        for (uint32_t s = lane; s < listed; s += kWave) {
+            const size_t at = (size_t{env} * S + s) * 2u;
+            const uint32_t first = d.ucontact_row_range[at], points = d.ucontact_row_range[at + 1u];
+            slot_rows[s] = points > 0u ? first : kInvalid;
+        }
         lds_sync<W>();
         bool push = false;
         for (uint32_t h = lane; h < heads; h += kWave) {
@@ -3463,7 +3473,8 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
                     // the contact slot whose normal rows hold this row (MapRowContactsKernel, block_descent.cu:1756-1767)
                     const uint32_t group_first = __float_as_uint(row[1]), points = __float_as_uint(row[2]);
                     uint32_t contact = 0u;
-                    for (uint32_t s = 0u; s < S; ++s)
+                    for (uint32_t s = 0u; s < listed; ++s) contact = slot_rows[s] == group_first ? env * S + s : contact;
+                    for (uint32_t s = listed; s < S; ++s)
                         if (d.ucontact_row_range[(size_t{env} * S + s) * 2u] == group_first &&
                             d.ucontact_row_range[(size_t{env} * S + s) * 2u + 1u] > 0u) contact = env * S + s;
                     const size_t point = size_t{contact} * 4u + (slot - group_first) % points;
@@ -3472,13 +3483,24 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
                     const double correction = p.position_beta * fmax(depth, 0.0) + reserve;
                     const double target = fmin(depth, 0.0) + correction;
                     double vel = 0.0;   // RowVelocity (block_descent.cu:1051-1082) per articulated side
-                    const uint32_t kind_a = __float_as_uint(row[10]), kind_b = __float_as_uint(row[18]);
-                    if (kind_a == kSideArtic) {
+                    const uint32_t kind_a = __float_as_uint(row[10]), kind_b = __float_as_uint(row[18]), first = c.U(hRow, h);
+                    const bool apart = kind_a == kSideArtic && kind_b == kSideArtic && __float_as_uint(row[11]) != __float_as_uint(row[19]);
+                    if (!c.from_links && first != kInvalid && !apart) {
+                        // one owner: the staged row is the side's own (of two sides with one owner the first holds both), its
+                        // entries past the block zeros; each product is exact in double
+                        const float4* j4 = reinterpret_cast<const float4*>(c.jac + first * uint32_t(W)), *q4 = reinterpret_cast<const float4*>(qvec);
+#pragma unroll
+                        for (int q = 0; q < W / 4; ++q) {
+                            const float4 j = j4[q], v = q4[q];
+                            vel = fma(double(j.x), double(v.x), vel); vel = fma(double(j.y), double(v.y), vel);
+                            vel = fma(double(j.z), double(v.z), vel); vel = fma(double(j.w), double(v.w), vel);
+                        }
+                    } else if (kind_a == kSideArtic) {
                         double value = 0.0;
                         for (uint32_t k = 0u; k < n; ++k) value += double(d.chain_jacobian[size_t{slot} * md + k]) * qvec[k];
                         vel += value;
                     }
-                    if (kind_b == kSideArtic) {
+                    if (kind_b == kSideArtic && (c.from_links || first == kInvalid || apart)) {
                         double value = 0.0;
                         for (uint32_t k = 0u; k < n; ++k) value += double(d.chain_jacobian_b[size_t{slot} * md + k]) * qvec[k];
                         vel += value;
