@@ -726,9 +726,9 @@ __device__ __forceinline__ void add_columns(int q, const float* rows, float a0, 
 }
 // the same for a head on one axis, straight into the row
 template <int N>
-__device__ __forceinline__ void add_columns_single(int q, const float* rows, float a0, float (&hrow)[N]) {
+__device__ __forceinline__ void add_columns_single(int q, float x0, float a0, float (&hrow)[N]) {
     Vec4 term = {hrow[4 * q], hrow[4 * q + 1], hrow[4 * q + 2], hrow[4 * q + 3]};
-    term = __builtin_amdgcn_mfma_f32_4x4x1f32(rows[4 * q], a0, term, 0, 0, 0);
+    term = __builtin_amdgcn_mfma_f32_4x4x1f32(x0, a0, term, 0, 0, 0);
 #pragma unroll
     for (int r = 0; r < 4; ++r) hrow[4 * q + r] = term[r];
 }
@@ -768,11 +768,11 @@ __device__ __forceinline__ void add_head(const Tile& c, uint32_t h, bool coordin
             return;
         }
 #pragma unroll
-        for (int q = 0; q < kFirstColumns<N>; ++q) add_columns_single<N>(q, words, a0, hrow);
+        for (int q = 0; q < kFirstColumns<N>; ++q) add_columns_single<N>(q, words[4 * q], a0, hrow);
         if ((columns >> (4 * kFirstColumns<N>)) == 0ull) return;
 #pragma unroll
         for (int q = kFirstColumns<N>; q < N / 4; ++q)
-            if (((columns >> (4 * q)) & 0xFull) != 0ull) add_columns_single<N>(q, words, a0, hrow);
+            if (((columns >> (4 * q)) & 0xFull) != 0ull) add_columns_single<N>(q, words[4 * q], a0, hrow);
         return;
     }
     const float w1 = j0r[N + column], w2 = j0r[2 * N + column];
@@ -1019,11 +1019,15 @@ __device__ __forceinline__ void add_block_heads(const Tile& c, uint64_t heads, b
 // many-sphered feet, of which some do not converge within their sweeps, and an environment that has not converged hands
 // a last place of its Hessian on as the fourth decimal of its velocities.
 // Heads a pass: as many copies of the block's rows as fit the wavefront, kGroups<N> of them, a group of lanes kGroupLanes
-// wide each - or two where that takes as few passes, or the one that contributes.  The lanes of group k add head
-// `taken[k]` to rows of their own, which start at zero past the first group; a head's values come from its own lane
-// (lane = head) through the lane permute.  The groups' rows are added together at the end, in group order, through LDS
-// (hrows and hfac, which a changed Hessian frees), and stay in hrows.  With kRows false only the force and its scale are
-// taken: the Hessian of the last assembly stands.
+// wide each - or two where that takes as few passes, or the one that contributes.  The contributing heads are listed a lane
+// each once; in a pass the lanes of group k add the k-th head of the pass's to rows of their own, which start at zero past the
+// first group; a head's values come from its own lane (lane = head) through the lane permute.  The groups' rows are added
+// together at the end, in group order, through LDS (hrows and hfac, which a changed Hessian frees), and stay in hrows.  With
+// kRows false only the force and its scale are taken: the Hessian of the last assembly stands.
+//   Bound by the LDS trips of one wave, so a pass's words are asked for a pass ahead; a kernel of three waves a SIMD has no
+// registers for that, and its other waves fill the wait.  A pass of three heads took 1.25 k cycles while it found its heads
+// by scalar code, asked for the first row, the values and the words one behind the other and handed the rows over in two
+// exchanges: 333 humanoids 536 -> 510 us, 4096 722 -> 708, 65536 7630 -> 7500, the bits the same.
 template <int N>
 constexpr int kGroups = N <= 16 ? 4 : (N <= 20 ? 3 : 2);
 template <int N>
@@ -1054,10 +1058,14 @@ __device__ __forceinline__ void add_heads_by_groups(const Tile& c, uint64_t head
     static_assert(N <= 32, "two copies of the rows fit the wavefront");
     constexpr int G = kGroups<N>;
     const uint32_t lane = c.lane, group = lane / kGroupLanes<N>, row = lane - group * kGroupLanes<N>;
-    const int contributing = __popcll(heads);
-    const int taken_a_pass = contributing == 1 ? 1 : ((contributing + G - 1) / G < (contributing + 1) / 2 ? G : 2);
-    const bool single = contributing == 1 && c.U(hAxes, uint32_t(__builtin_ctzll(heads))) == 1u;
+    const uint32_t contributing = uint32_t(__popcll(heads));
+    const uint32_t taken_a_pass = contributing == 1u ? 1u : ((contributing + G - 1u) / G < (contributing + 1u) / 2u ? G : 2u);
+    const bool single = contributing == 1u && c.U(hAxes, uint32_t(__builtin_ctzll(heads))) == 1u;
     const uint32_t column = min(row, uint32_t(N - 1));
+    // the contributing heads in order, one a lane from lane 0 on, each with its first row
+    const uint32_t below = __builtin_amdgcn_mbcnt_hi(uint32_t(heads >> 32u), __builtin_amdgcn_mbcnt_lo(uint32_t(heads), 0u));
+    const uint32_t place = ((heads >> lane) & 1ull) != 0ull ? below : contributing + (lane - below);
+    const int listed = __builtin_amdgcn_ds_permute(int(4u * place), int((my_first << 8u) | lane));
     if (group != 0u) {
         if constexpr (kRows) {
 #pragma unroll
@@ -1065,66 +1073,90 @@ __device__ __forceinline__ void add_heads_by_groups(const Tile& c, uint64_t head
         }
         g.value = 0.0; scale = 0.0f;
     }
-    while (heads != 0ull) {
-        // what lanes without a head read: its rows are staged, and add_columns multiplies a word of theirs by zero, which must
-        // be a finite word
-        const uint32_t first = uint32_t(__builtin_ctzll(heads));
-        uint32_t mine = kInvalid;
+    // What a lane needs of its group's head in a pass; the next pass's words are on their way while this one's are worked on.
+    // Lanes without a head read the last one's: its rows are staged, and add_columns multiplies a word of theirs by zero, which
+    // must be a finite word.
+    struct Words { float f[3], noise[3], cv[4], j[3]; const float* rows; bool live; };
+    const auto fetch = [&](int entry, uint32_t rank) {
+        Words w;
+        const int source = (entry & 0xFF) * 4;
+        const float* rows = c.jac + (uint32_t(entry) >> 8u) * uint32_t(N);
+        w.live = group < taken_a_pass && rank < contributing && row < c.n;   // (the lanes past the last group have none)
 #pragma unroll
-        for (int k = 0; k < G; ++k) {
-            const uint32_t h = heads != 0ull && k < taken_a_pass ? uint32_t(__builtin_ctzll(heads)) : kInvalid;
-            if (k < taken_a_pass) heads &= heads - 1ull;   // zero stays zero
-            mine = group == uint32_t(k) ? h : mine;
-        }
-        const bool none = mine == kInvalid;   // also the lanes past the last group
-        const int source = int((none ? first : mine) * 4u);
-        const float* rows = c.jac + uint32_t(__builtin_amdgcn_ds_bpermute(source, int(my_first))) * uint32_t(N);
-        float f[3], noise[3];
-#pragma unroll
-        for (int k = 0; k < 3; ++k) { f[k] = lane_permute(source, mf[k]); noise[k] = lane_permute(source, mn[k]); }
-        const bool live = !none && row < c.n;
-        // (read whether or not the lane uses them: a read under a condition compiles to a branch a word)
-        const float w0 = rows[column], w1 = rows[N + column], w2 = rows[2 * N + column];
-        const float j0 = live ? w0 : 0.0f, j1 = live ? w1 : 0.0f, j2 = live ? w2 : 0.0f;
-        tile_add_product(g, j0, f[0]);
-        tile_add_product(g, j1, f[1]);
-        tile_add_product(g, j2, f[2]);
-        scale += (fabsf(j0) * noise[0] + fabsf(j1) * noise[1]) + fabsf(j2) * noise[2];
+        for (int k = 0; k < 3; ++k) w.j[k] = rows[uint32_t(k) * uint32_t(N) + column];
         if constexpr (kRows) {
-            float cv[6];
+            w.cv[0] = lane_permute(source, mc[0]); w.cv[1] = lane_permute(source, mc[1]);
+            w.cv[2] = lane_permute(source, mc[2]); w.cv[3] = lane_permute(source, mc[5]);
+            w.rows = rows + (lane & 3u);
+        }
 #pragma unroll
-            for (int k = 0; k < 6; ++k) cv[k] = lane_permute(source, mc[k]);
-            const float cxx = cv[0], cyy = cv[1], czz = cv[2], cxy = cv[3], cxz = cv[4], cyz = cv[5];
-            const float a0 = (j0 * cxx + j1 * cxy) + j2 * cxz;
-            const float a1 = (j1 * cyy + j2 * cyz) + j0 * cxy;
-            const float a2 = (j2 * czz + j1 * cyz) + j0 * cxz;
-            if (single) {
+        for (int k = 0; k < 3; ++k) { w.f[k] = lane_permute(source, mf[k]); w.noise[k] = lane_permute(source, mn[k]); }
+        return w;
+    };
+    const auto entry_of = [&](uint32_t rank) { return __builtin_amdgcn_ds_bpermute(int(4u * min(rank, contributing - 1u)), listed); };
+    const auto take = [&](const Words& w, bool alone) {
+        const float j0 = w.live ? w.j[0] : 0.0f, j1 = w.live ? w.j[1] : 0.0f, j2 = w.live ? w.j[2] : 0.0f;
+        if constexpr (kRows) {
+            // (no head of these worlds couples its normal axis to the others)
+            const float a0 = j0 * w.cv[0], a1 = j1 * w.cv[1] + j2 * w.cv[3], a2 = j2 * w.cv[2] + j1 * w.cv[3];
+            if (alone && single) {
 #pragma unroll
-                for (int q = 0; q < N / 4; ++q) add_columns_single<N>(q, rows + (lane & 3u), a0, hrow);
+                for (int q = 0; q < N / 4; ++q) add_columns_single<N>(q, w.rows[4 * q], a0, hrow);
             } else {
 #pragma unroll
-                for (int q = 0; q < N / 4; ++q) add_columns<N>(q, rows + (lane & 3u), a0, a1, a2, hrow);
+                for (int q = 0; q < N / 4; ++q) add_columns<N>(q, w.rows, a0, a1, a2, hrow);
             }
         }
+        tile_add_product(g, j0, w.f[0]);
+        tile_add_product(g, j1, w.f[1]);
+        tile_add_product(g, j2, w.f[2]);
+        scale += (fabsf(j0) * w.noise[0] + fabsf(j1) * w.noise[1]) + fabsf(j2) * w.noise[2];
+    };
+    uint32_t rank = group, done = 0u;
+    if constexpr (WavesPerSimd(N) > 2) {
+        for (; done < contributing; done += taken_a_pass, rank += taken_a_pass) take(fetch(entry_of(rank), rank), true);
+        if (contributing == 1u) return;
+    } else {
+        if (contributing == 1u) {
+            take(fetch(entry_of(rank), rank), true);
+            return;
+        }
+        Words even = fetch(entry_of(rank), rank), odd;
+        int entry = entry_of(rank + taken_a_pass);
+        const auto pass = [&](const Words& here, Words& next) {   // true after the last one
+            done += taken_a_pass; rank += taken_a_pass;
+            if (done < contributing) {
+                next = fetch(entry, rank);
+                entry = entry_of(rank + taken_a_pass);
+            }
+            take(here, false);
+            return done >= contributing;
+        };
+        while (!pass(even, odd) && !pass(odd, even)) {}
     }
-    if (contributing == 1) return;
     g.value = groups_sum<N>(lane, g.value); scale = groups_sum<N>(lane, scale);
     if constexpr (kRows) {
+        // the second group's rows by way of hrows, the third's by way of hfac, a fourth's behind them; what the lanes
+        // past the first group add to theirs is read by nobody
+        constexpr int kRound = 2;   // groups an exchange
 #pragma unroll
-        for (int k = 1; k < G; ++k) {
-            float* exchange = k % 2 == 1 ? c.hrows : c.hfac;
-            if (group == uint32_t(k) && row < uint32_t(N)) {
-                float4* words = reinterpret_cast<float4*>(exchange + row * uint32_t(N));
+        for (int k = 1; k < G; k += kRound) {
+            if (group - uint32_t(k) < uint32_t(kRound) && group < uint32_t(G) && row < uint32_t(N)) {
+                float4* to = reinterpret_cast<float4*>((group == uint32_t(k) ? c.hrows : c.hfac) + row * uint32_t(N));
 #pragma unroll
-                for (int q = 0; q < N / 4; ++q) words[q] = float4{hrow[4 * q], hrow[4 * q + 1], hrow[4 * q + 2], hrow[4 * q + 3]};
+                for (int q = 0; q < N / 4; ++q) to[q] = float4{hrow[4 * q], hrow[4 * q + 1], hrow[4 * q + 2], hrow[4 * q + 3]};
             }
             lds_sync<N>();
-            const float4* words = reinterpret_cast<const float4*>(exchange + column * uint32_t(N));
 #pragma unroll
-            for (int q = 0; q < N / 4; ++q) {
-                const float4 w = words[q];
-                if (group != 0u) continue;
-                hrow[4 * q] += w.x; hrow[4 * q + 1] += w.y; hrow[4 * q + 2] += w.z; hrow[4 * q + 3] += w.w;
+            for (int other = k; other < k + kRound && other < G; ++other) {
+                const float4* from = reinterpret_cast<const float4*>((other == k ? c.hrows : c.hfac) + column * uint32_t(N));
+#pragma unroll
+                for (int q = 0; q < N / 4; ++q) {
+                    const float4 w = from[q];
+                    const bool adds = G <= kRound + 1 || group == 0u;   // (a group that is still to hand its rows over keeps them)
+                    hrow[4 * q] += adds ? w.x : 0.0f; hrow[4 * q + 1] += adds ? w.y : 0.0f;
+                    hrow[4 * q + 2] += adds ? w.z : 0.0f; hrow[4 * q + 3] += adds ? w.w : 0.0f;
+                }
             }
             lds_sync<N>();
         }
