@@ -19,10 +19,17 @@ NKH_DECLARE_REDUCED(24, 12) NKH_DECLARE_REDUCED(28, 16) NKH_DECLARE_REDUCED(32, 
 NKH_DECLARE_REDUCED(44, 24) NKH_DECLARE_REDUCED(48, 24) NKH_DECLARE_REDUCED(52, 28) NKH_DECLARE_REDUCED(56, 28) NKH_DECLARE_REDUCED(60, 32)
 NKH_DECLARE_REDUCED(64, 32)
 #undef NKH_DECLARE_REDUCED
+// the same for worlds under the elliptic cone
+#define NKH_DECLARE_ELLIPTIC(N, K) \
+    extern template __global__ void BlockDescentTileKernel<N, true, K, true>(ModelView, DataView, BlockDescentSolveParams, uint32_t, uint32_t, uint32_t, uint32_t);
+NKH_DECLARE_ELLIPTIC(24, 12) NKH_DECLARE_ELLIPTIC(28, 16) NKH_DECLARE_ELLIPTIC(32, 16) NKH_DECLARE_ELLIPTIC(36, 20) NKH_DECLARE_ELLIPTIC(40, 20)
+NKH_DECLARE_ELLIPTIC(44, 24) NKH_DECLARE_ELLIPTIC(48, 24) NKH_DECLARE_ELLIPTIC(52, 28) NKH_DECLARE_ELLIPTIC(56, 28) NKH_DECLARE_ELLIPTIC(60, 32)
+NKH_DECLARE_ELLIPTIC(64, 32)
+#undef NKH_DECLARE_ELLIPTIC
 // The dense build of the same template (ops_solver_kernel.h compiled with NKH_SOLVER_DENSE: three or four waves a SIMD), for the
 // widths it is instantiated at in ops_solver_d*.hip.
 namespace dense {
-template <int N, bool kContactsOnly, int K = N>
+template <int N, bool kContactsOnly, int K = N, bool kElliptic = !kContactsOnly>
 __global__ void BlockDescentTileKernel(ModelView, DataView, BlockDescentSolveParams, uint32_t, uint32_t, uint32_t, uint32_t);
 #define NKH_DECLARE_DENSE(N, K) \
     extern template __global__ void BlockDescentTileKernel<N, true, K>(ModelView, DataView, BlockDescentSolveParams, uint32_t, uint32_t, uint32_t, uint32_t);
@@ -122,10 +129,21 @@ const SolverKernel kSolverKernels[2][16] = {{NKH_WIDTHS(false)}, {NKH_WIDTHS(tru
 // when no contact can reach a coordinate from that width on (ModelView::contact_dof_end).
 struct ReducedKernel { uint32_t width, reduced; SolverKernel kernel; };
 const ReducedKernel kReducedKernels[] = {
-    {24u, 12u, BlockDescentTileKernel<24, true, 12>}, {28u, 16u, BlockDescentTileKernel<28, true, 16>}, {32u, 16u, BlockDescentTileKernel<32, true, 16>},
-    {36u, 20u, BlockDescentTileKernel<36, true, 20>}, {40u, 20u, BlockDescentTileKernel<40, true, 20>}, {44u, 24u, BlockDescentTileKernel<44, true, 24>},
-    {48u, 24u, BlockDescentTileKernel<48, true, 24>}, {52u, 28u, BlockDescentTileKernel<52, true, 28>}, {56u, 28u, BlockDescentTileKernel<56, true, 28>},
-    {60u, 32u, BlockDescentTileKernel<60, true, 32>}, {64u, 32u, BlockDescentTileKernel<64, true, 32>}};
+    {24u, 12u, BlockDescentTileKernel<24, true, 12>}, {28u, 16u, BlockDescentTileKernel<28, true, 16>},
+    {32u, 16u, BlockDescentTileKernel<32, true, 16>}, {36u, 20u, BlockDescentTileKernel<36, true, 20>},
+    {40u, 20u, BlockDescentTileKernel<40, true, 20>}, {44u, 24u, BlockDescentTileKernel<44, true, 24>},
+    {48u, 24u, BlockDescentTileKernel<48, true, 24>}, {52u, 28u, BlockDescentTileKernel<52, true, 28>},
+    {56u, 28u, BlockDescentTileKernel<56, true, 28>}, {60u, 32u, BlockDescentTileKernel<60, true, 32>},
+    {64u, 32u, BlockDescentTileKernel<64, true, 32>}};
+// the same with the elliptic cone's response: 2048 humanoids under it 493 -> 408 us a step, by the general kernel at the full
+// width before
+const ReducedKernel kEllipticKernels[] = {
+    {24u, 12u, BlockDescentTileKernel<24, true, 12, true>}, {28u, 16u, BlockDescentTileKernel<28, true, 16, true>},
+    {32u, 16u, BlockDescentTileKernel<32, true, 16, true>}, {36u, 20u, BlockDescentTileKernel<36, true, 20, true>},
+    {40u, 20u, BlockDescentTileKernel<40, true, 20, true>}, {44u, 24u, BlockDescentTileKernel<44, true, 24, true>},
+    {48u, 24u, BlockDescentTileKernel<48, true, 24, true>}, {52u, 28u, BlockDescentTileKernel<52, true, 28, true>},
+    {56u, 28u, BlockDescentTileKernel<56, true, 28, true>}, {60u, 32u, BlockDescentTileKernel<60, true, 32, true>},
+    {64u, 32u, BlockDescentTileKernel<64, true, 32, true>}};
 // The dense kernels: (padded width of the block, width of the sweeps), contact heads only.
 const ReducedKernel kDenseKernels[] = {
     {4u, 4u, dense::BlockDescentTileKernel<4, true, 4>}, {8u, 8u, dense::BlockDescentTileKernel<8, true, 8>},
@@ -157,48 +175,56 @@ void InitSolverKernels() {
         (void)hipFuncSetAttribute(reinterpret_cast<const void*>(reduced.kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
         (void)hipGetLastError();
     }
+    for (const ReducedKernel& elliptic : kEllipticKernels) {
+        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(elliptic.kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+        (void)hipGetLastError();
+    }
     for (const ReducedKernel& dense : kDenseKernels) {
         (void)hipFuncSetAttribute(reinterpret_cast<const void*>(dense.kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
         (void)hipGetLastError();
     }
 }
 
+// The heads a world's solve meets: contact heads only, at most one a lane, plain or under the elliptic cone of the MuJoCo law
+// (which at the full width only the general kernel answers), or anything.
+enum class Heads { Any, Contacts, Elliptic };
+static Heads HeadsOf(const ModelView& m, uint32_t staged) {
+    const uint32_t joint_heads = m.joint_limit_rows + m.joint_friction_rows + m.joint_drive_rows;
+    if (joint_heads != 0u || staged > uint32_t(solver::kWave)) return Heads::Any;
+    return m.any_mujoco != 0u && m.contact_cone == 1u ? Heads::Elliptic : Heads::Contacts;
+}
 // The width the sweeps of a world's solve run at: its coordinates, or the K of a reduced block where no contact of the
 // world reaches the coordinates from K on and a kernel is compiled for that.
-static uint32_t SolverWorkingWidth(const ModelView& m, bool contacts_only) {
-    if (contacts_only)
+static uint32_t SolverWorkingWidth(const ModelView& m, Heads heads) {
+    if (heads != Heads::Any)
         for (const ReducedKernel& reduced : kReducedKernels)
             if (reduced.width == solver::PaddedWidth(m.dof) && m.contact_dof_end != 0u && m.contact_dof_end <= reduced.reduced &&
                 reduced.reduced <= m.dof) return reduced.reduced;   // (0: a host that did not say; the full width is always right)
     return m.dof;
 }
-// worlds whose heads are contact heads only, at most one a lane (the elliptic cone of the MuJoCo law is answered by the
-// general kernel only)
-static bool ContactHeadsOnly(const ModelView& m, uint32_t staged) {
-    const uint32_t joint_heads = m.joint_limit_rows + m.joint_friction_rows + m.joint_drive_rows;
-    return joint_heads == 0u && staged <= uint32_t(solver::kWave) && !(m.any_mujoco != 0u && m.contact_cone == 1u);
-}
 // `dense_out`: whether the kernel is a dense one
-static SolverKernel KernelOfWidth(const ModelView& m, bool contacts_only, uint32_t width, uint32_t env_count, bool* dense_out = nullptr) {
+static SolverKernel KernelOfWidth(const ModelView& m, Heads heads, uint32_t width, uint32_t env_count, bool* dense_out = nullptr) {
     if (dense_out != nullptr) *dense_out = false;
-    if (contacts_only && env_count >= kDenseBatch)
+    if (heads == Heads::Contacts && env_count >= kDenseBatch)
         for (const ReducedKernel& dense : kDenseKernels)
             if (dense.width == solver::PaddedWidth(m.dof) && dense.reduced == solver::PaddedWidth(width) && (width == m.dof || dense.reduced == width)) {
                 if (dense_out != nullptr) *dense_out = true;
                 return dense.kernel;
             }
-    if (width != m.dof)
-        for (const ReducedKernel& reduced : kReducedKernels)
+    if (width != m.dof) {
+        static_assert(sizeof(kReducedKernels) == sizeof(kEllipticKernels), "the same pairs of widths");
+        for (const ReducedKernel& reduced : heads == Heads::Elliptic ? kEllipticKernels : kReducedKernels)
             if (reduced.width == solver::PaddedWidth(m.dof) && reduced.reduced == width) return reduced.kernel;
-    return kSolverKernels[contacts_only ? 1 : 0][solver::PaddedWidth(m.dof) / 4u - 1u];
+    }
+    return kSolverKernels[heads == Heads::Contacts ? 1 : 0][solver::PaddedWidth(m.dof) / 4u - 1u];
 }
 // Worlds whose environments are solved four a wavefront (ops_solver_packed.hip): contact heads only, no more of them and no
 // more coordinates than a row of sixteen lanes takes.  From a batch on that has wavefronts enough that way: a wavefront
 // of four takes longer than any of them alone, and 2048 free boxes step in 259 us one a wavefront, 324 packed (8192 342
 // and 339).
 constexpr uint32_t kPackedBatch = 8192u;
-static bool PackedSolverTakes(const ModelView& m, bool contacts_only, uint32_t staged, uint32_t env_count) {
-    return contacts_only && m.dof <= uint32_t(solver::kPackedWidth) && m.max_dof <= 16u && staged <= solver::kPackedHeads && env_count >= kPackedBatch;
+static bool PackedSolverTakes(const ModelView& m, Heads heads, uint32_t staged, uint32_t env_count) {
+    return heads == Heads::Contacts && m.dof <= uint32_t(solver::kPackedWidth) && m.max_dof <= 16u && staged <= solver::kPackedHeads && env_count >= kPackedBatch;
 }
 // Environments that have a wavefront to themselves, the costliest: one a compute unit until the others' wavefronts take
 // longer than they do (16384 free boxes 429 us without them, 392 with; 65536 981 and 989).
@@ -211,19 +237,19 @@ uint32_t SolverBlocksPerUnit(const ModelView& m, uint32_t env_count) {
     const uint32_t staged = SolverHeadCapacity(m, std::max(m.contact_slots, 1u));
     if (staged == 0u) return 0u;
     const uint32_t joint_heads = m.joint_limit_rows + m.joint_friction_rows + m.joint_drive_rows;
-    const bool contacts_only = ContactHeadsOnly(m, staged);
-    const uint32_t width = SolverWorkingWidth(m, contacts_only);
+    const Heads heads = HeadsOf(m, staged);
+    const uint32_t width = SolverWorkingWidth(m, heads);
     const size_t lds = size_t{solver::ReducedSolverLdsFloats(m.dof, width, staged + joint_heads, staged,
-                                                             solver::RowsFromLinks(width, contacts_only, m.rows_from_links))} * sizeof(float);
+                                                             solver::RowsFromLinks(width, heads == Heads::Contacts, m.rows_from_links))} * sizeof(float);
     int blocks = 0;
-    if (PackedSolverTakes(m, contacts_only, staged, env_count)) {
+    if (PackedSolverTakes(m, heads, staged, env_count)) {
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, reinterpret_cast<const void*>(PackedDescentKernel), solver::kWave, PackedLdsBytes(staged)) != hipSuccess) {
             (void)hipGetLastError();
             return 0u;
         }
         return uint32_t(std::max(blocks, 0));
     }
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, reinterpret_cast<const void*>(KernelOfWidth(m, contacts_only, width, env_count)),
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, reinterpret_cast<const void*>(KernelOfWidth(m, heads, width, env_count)),
                                                      solver::kWave, lds) != hipSuccess) {
         (void)hipGetLastError();
         return 0u;
@@ -238,7 +264,7 @@ uint32_t SolverMassFactorFloats(const ModelView& m) {
 uint32_t SolverSweepWidth(const ModelView& m) {
     if (m.rows_per_env == 0u || m.dof == 0u) return m.dof;
     const uint32_t staged = SolverHeadCapacity(m, std::max(m.contact_slots, 1u));
-    return SolverWorkingWidth(m, staged != 0u && ContactHeadsOnly(m, staged));
+    return SolverWorkingWidth(m, staged != 0u ? HeadsOf(m, staged) : Heads::Any);
 }
 
 Status OpBlockDescentSolve(const ModelView& m, const DataView& d, const void* params, hipStream_t stream) {
@@ -250,14 +276,14 @@ Status OpBlockDescentSolve(const ModelView& m, const DataView& d, const void* pa
     const uint32_t staged = SolverHeadCapacity(m, p->contact_slots_per_env == 0u ? 1u : p->contact_slots_per_env);
     if (staged == 0u) return Status::InvalidArgument;
     const uint32_t joint_heads = m.joint_limit_rows + m.joint_friction_rows + m.joint_drive_rows;
-    const bool contacts_only = ContactHeadsOnly(m, staged);
-    const uint32_t width = SolverWorkingWidth(m, contacts_only);
+    const Heads heads = HeadsOf(m, staged);
+    const uint32_t width = SolverWorkingWidth(m, heads);
     const auto lds_bytes = [&](uint32_t contact_heads) {
         return size_t{solver::ReducedSolverLdsFloats(m.dof, width, contact_heads + joint_heads, contact_heads,
-                                                     solver::RowsFromLinks(width, contacts_only, m.rows_from_links))} * sizeof(float);
+                                                     solver::RowsFromLinks(width, heads == Heads::Contacts, m.rows_from_links))} * sizeof(float);
     };
     bool dense = false;
-    const SolverKernel kernel = KernelOfWidth(m, contacts_only, width, p->env_count, &dense);
+    const SolverKernel kernel = KernelOfWidth(m, heads, width, p->env_count, &dense);
     // blocks a compute unit holds at most, whatever their LDS: four a wave of a SIMD
     const int padded = int(solver::PaddedWidth(width));
     const size_t most_blocks = 4u * size_t(dense ? solver::DenseWavesPerSimd(padded) : solver::WavesPerSimd(padded));
@@ -281,7 +307,7 @@ Status OpBlockDescentSolve(const ModelView& m, const DataView& d, const void* pa
     // edges a point under the pyramidal cone.  (While those worlds went to the one full launch, a walker's 304 heads left a
     // compute unit one block for environments of a handful of points: a step of 4096 with a twentieth reset 768 -> 438 us.)
     hipLaunchKernelGGL(OrderTilesKernel, dim3((p->env_count + kOrderEnvs - 1u) / kOrderEnvs), dim3(1024), 0, stream, d, p->env_count);
-    if (PackedSolverTakes(m, contacts_only, staged, p->env_count)) {
+    if (PackedSolverTakes(m, heads, staged, p->env_count)) {
         const uint32_t alone = PackedAlone(p->env_count);
         hipLaunchKernelGGL(PackedDescentKernel, dim3(alone + (p->env_count - alone + kPackedEnvs - 1u) / kPackedEnvs), dim3(solver::kWave),
                            PackedLdsBytes(staged), stream, m, d, *p, staged, alone);

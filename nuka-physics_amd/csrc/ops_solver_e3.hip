@@ -1,0 +1,9 @@
+// Instantiations of the block-descent kernel for reduced blocks under the elliptic cone (contact heads only; full width, width of
+// the sweeps): 48/24, 52/28.
+#include "ops_solver_kernel.h"
+namespace nkh {
+namespace solver {
+template __global__ void BlockDescentTileKernel<48, true, 24, true>(ModelView, DataView, BlockDescentSolveParams, uint32_t, uint32_t, uint32_t, uint32_t);
+template __global__ void BlockDescentTileKernel<52, true, 28, true>(ModelView, DataView, BlockDescentSolveParams, uint32_t, uint32_t, uint32_t, uint32_t);
+}  // namespace solver
+}  // namespace nkh
