@@ -990,13 +990,13 @@ __device__ __forceinline__ void add_block_heads(const Tile& c, uint64_t heads, b
     };
     auto value_of = [&](float v, uint32_t h) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), int(h))); };
     uint32_t h = uint32_t(__builtin_ctzll(heads));
-    Words next = fetch(h);
-#pragma unroll 1
-    for (;;) {
+    // (two sets of words in turn: with one the compiler moves the reads of both places to where they meet, ahead of their use)
+    Words even = fetch(h), odd;
+    auto add = [&](const Words& w, Words& next) {   // true after the last head
         heads &= heads - 1ull;
-        const Words w = next;
         const uint32_t after = heads != 0ull ? uint32_t(__builtin_ctzll(heads)) : h;
         next = fetch(after);
+        __builtin_amdgcn_sched_barrier(0);
         float j[3];
 #pragma unroll
         for (int k = 0; k < 3; ++k) {
@@ -1011,9 +1011,11 @@ __device__ __forceinline__ void add_block_heads(const Tile& c, uint64_t heads, b
         const float a2 = (j[2] * czz + j[1] * cyz) + j[0] * cxz;
 #pragma unroll
         for (int q = 0; q < kFirst; ++q) add_columns<N>(q, w.x[q][0], w.x[q][1], w.x[q][2], a0, a1, a2, hrow);
-        if (heads == 0ull) break;
         h = after;
-    }
+        return heads == 0ull;
+    };
+#pragma unroll 1
+    while (!add(even, odd) && !add(odd, even)) {}
 }
 
 // A reduced block of plain contacts adds its heads to register rows instead, in an order of its own (below): its worlds are robots on two
