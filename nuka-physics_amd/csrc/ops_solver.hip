@@ -1,5 +1,5 @@
 // Launch side of the block-descent solve: head capacity, LDS sizing and the table of kernels, one per padded width.
-// The kernel template lives in ops_solver_kernel.h; its instantiations are spread over ops_solver_w*.hip (general)
+// The kernel template lives in ops_solver_kernel.h; its instantiations are spread over ops_solver_w*.hip, ops_solver_g*.hip (general)
 // and ops_solver_s*.hip (contact heads only) so that they compile in parallel.
 #include "ops_solver_kernel.h"
 
@@ -7,6 +7,7 @@ namespace nkh {
 namespace solver {
 #define NKH_DECLARE_WIDTH(N) \
     extern template __global__ void BlockDescentTileKernel<N, false>(ModelView, DataView, BlockDescentSolveParams, uint32_t, uint32_t, uint32_t, uint32_t); \
+    extern template __global__ void BlockDescentTileKernel<N, false, N, false>(ModelView, DataView, BlockDescentSolveParams, uint32_t, uint32_t, uint32_t, uint32_t); \
     extern template __global__ void BlockDescentTileKernel<N, true>(ModelView, DataView, BlockDescentSolveParams, uint32_t, uint32_t, uint32_t, uint32_t);
 NKH_DECLARE_WIDTH(4) NKH_DECLARE_WIDTH(8) NKH_DECLARE_WIDTH(12) NKH_DECLARE_WIDTH(16) NKH_DECLARE_WIDTH(20) NKH_DECLARE_WIDTH(24)
 NKH_DECLARE_WIDTH(28) NKH_DECLARE_WIDTH(32) NKH_DECLARE_WIDTH(36) NKH_DECLARE_WIDTH(40) NKH_DECLARE_WIDTH(44) NKH_DECLARE_WIDTH(48)
@@ -116,15 +117,26 @@ __global__ void __launch_bounds__(1024) OrderTilesKernel(DataView d, uint32_t en
 
 
 using SolverKernel = void (*)(ModelView, DataView, BlockDescentSolveParams, uint32_t, uint32_t, uint32_t, uint32_t);
-// Two instantiations per padded width: the general one, and the one for worlds whose heads are contact heads only,
-// at most one a lane.
-#define NKH_WIDTHS(V) \
-    BlockDescentTileKernel<4, V>, BlockDescentTileKernel<8, V>, BlockDescentTileKernel<12, V>, BlockDescentTileKernel<16, V>, \
-    BlockDescentTileKernel<20, V>, BlockDescentTileKernel<24, V>, BlockDescentTileKernel<28, V>, BlockDescentTileKernel<32, V>, \
-    BlockDescentTileKernel<36, V>, BlockDescentTileKernel<40, V>, BlockDescentTileKernel<44, V>, BlockDescentTileKernel<48, V>, \
-    BlockDescentTileKernel<52, V>, BlockDescentTileKernel<56, V>, BlockDescentTileKernel<60, V>, BlockDescentTileKernel<64, V>
-const SolverKernel kSolverKernels[2][16] = {{NKH_WIDTHS(false)}, {NKH_WIDTHS(true)}};
-#undef NKH_WIDTHS
+// Three instantiations per padded width, in the order of Heads: the general one without and with the elliptic cone's response
+// (whose functions and coupled curvatures the other then has no registers and lane reads for: four steps of 1000 servo-driven
+// quadrupeds 1934 -> 1880 us, 4096 servo-driven humanoids 1388 -> 1380), and the one for worlds whose heads
+// are contact heads only, at most one a lane.
+enum Heads : uint32_t { kAnyHeads, kAnyElliptic, kContactHeads, kContactElliptic };
+const SolverKernel kSolverKernels[3][16] = {
+    {BlockDescentTileKernel<4, false, 4, false>, BlockDescentTileKernel<8, false, 8, false>, BlockDescentTileKernel<12, false, 12, false>,
+     BlockDescentTileKernel<16, false, 16, false>, BlockDescentTileKernel<20, false, 20, false>, BlockDescentTileKernel<24, false, 24, false>,
+     BlockDescentTileKernel<28, false, 28, false>, BlockDescentTileKernel<32, false, 32, false>, BlockDescentTileKernel<36, false, 36, false>,
+     BlockDescentTileKernel<40, false, 40, false>, BlockDescentTileKernel<44, false, 44, false>, BlockDescentTileKernel<48, false, 48, false>,
+     BlockDescentTileKernel<52, false, 52, false>, BlockDescentTileKernel<56, false, 56, false>, BlockDescentTileKernel<60, false, 60, false>,
+     BlockDescentTileKernel<64, false, 64, false>},
+    {BlockDescentTileKernel<4, false>, BlockDescentTileKernel<8, false>, BlockDescentTileKernel<12, false>, BlockDescentTileKernel<16, false>,
+     BlockDescentTileKernel<20, false>, BlockDescentTileKernel<24, false>, BlockDescentTileKernel<28, false>, BlockDescentTileKernel<32, false>,
+     BlockDescentTileKernel<36, false>, BlockDescentTileKernel<40, false>, BlockDescentTileKernel<44, false>, BlockDescentTileKernel<48, false>,
+     BlockDescentTileKernel<52, false>, BlockDescentTileKernel<56, false>, BlockDescentTileKernel<60, false>, BlockDescentTileKernel<64, false>},
+    {BlockDescentTileKernel<4, true>, BlockDescentTileKernel<8, true>, BlockDescentTileKernel<12, true>, BlockDescentTileKernel<16, true>,
+     BlockDescentTileKernel<20, true>, BlockDescentTileKernel<24, true>, BlockDescentTileKernel<28, true>, BlockDescentTileKernel<32, true>,
+     BlockDescentTileKernel<36, true>, BlockDescentTileKernel<40, true>, BlockDescentTileKernel<44, true>, BlockDescentTileKernel<48, true>,
+     BlockDescentTileKernel<52, true>, BlockDescentTileKernel<56, true>, BlockDescentTileKernel<60, true>, BlockDescentTileKernel<64, true>}};
 // One reduced instantiation per padded width from 24 on: the sweeps run at about half the width.  A world takes it
 // when no contact can reach a coordinate from that width on (ModelView::contact_dof_end).
 struct ReducedKernel { uint32_t width, reduced; SolverKernel kernel; };
@@ -185,18 +197,18 @@ void InitSolverKernels() {
     }
 }
 
-// The heads a world's solve meets: contact heads only, at most one a lane, plain or under the elliptic cone of the MuJoCo law
-// (which at the full width only the general kernel answers), or anything.
-enum class Heads { Any, Contacts, Elliptic };
+// The heads a world's solve meets: anything or contact heads only, at most one a lane, either with or without the elliptic cone
+// of the MuJoCo law (contact heads under it take the general kernel at the full width).
 static Heads HeadsOf(const ModelView& m, uint32_t staged) {
     const uint32_t joint_heads = m.joint_limit_rows + m.joint_friction_rows + m.joint_drive_rows;
-    if (joint_heads != 0u || staged > uint32_t(solver::kWave)) return Heads::Any;
-    return m.any_mujoco != 0u && m.contact_cone == 1u ? Heads::Elliptic : Heads::Contacts;
+    const bool elliptic = m.any_mujoco != 0u && m.contact_cone == 1u;
+    if (joint_heads != 0u || staged > uint32_t(solver::kWave)) return elliptic ? kAnyElliptic : kAnyHeads;
+    return elliptic ? kContactElliptic : kContactHeads;
 }
 // The width the sweeps of a world's solve run at: its coordinates, or the K of a reduced block where no contact of the
 // world reaches the coordinates from K on and a kernel is compiled for that.
 static uint32_t SolverWorkingWidth(const ModelView& m, Heads heads) {
-    if (heads != Heads::Any)
+    if (heads == kContactHeads || heads == kContactElliptic)
         for (const ReducedKernel& reduced : kReducedKernels)
             if (reduced.width == solver::PaddedWidth(m.dof) && m.contact_dof_end != 0u && m.contact_dof_end <= reduced.reduced &&
                 reduced.reduced <= m.dof) return reduced.reduced;   // (0: a host that did not say; the full width is always right)
@@ -205,7 +217,7 @@ static uint32_t SolverWorkingWidth(const ModelView& m, Heads heads) {
 // `dense_out`: whether the kernel is a dense one
 static SolverKernel KernelOfWidth(const ModelView& m, Heads heads, uint32_t width, uint32_t env_count, bool* dense_out = nullptr) {
     if (dense_out != nullptr) *dense_out = false;
-    if (heads == Heads::Contacts && env_count >= kDenseBatch)
+    if (heads == kContactHeads && env_count >= kDenseBatch)
         for (const ReducedKernel& dense : kDenseKernels)
             if (dense.width == solver::PaddedWidth(m.dof) && dense.reduced == solver::PaddedWidth(width) && (width == m.dof || dense.reduced == width)) {
                 if (dense_out != nullptr) *dense_out = true;
@@ -213,10 +225,10 @@ static SolverKernel KernelOfWidth(const ModelView& m, Heads heads, uint32_t widt
             }
     if (width != m.dof) {
         static_assert(sizeof(kReducedKernels) == sizeof(kEllipticKernels), "the same pairs of widths");
-        for (const ReducedKernel& reduced : heads == Heads::Elliptic ? kEllipticKernels : kReducedKernels)
+        for (const ReducedKernel& reduced : heads == kContactElliptic ? kEllipticKernels : kReducedKernels)
             if (reduced.width == solver::PaddedWidth(m.dof) && reduced.reduced == width) return reduced.kernel;
     }
-    return kSolverKernels[heads == Heads::Contacts ? 1 : 0][solver::PaddedWidth(m.dof) / 4u - 1u];
+    return kSolverKernels[heads == kContactElliptic ? kAnyElliptic : heads][solver::PaddedWidth(m.dof) / 4u - 1u];
 }
 // Worlds whose environments are solved four a wavefront (ops_solver_packed.hip): contact heads only, no more of them and no
 // more coordinates than a row of sixteen lanes takes.  From a batch on that has wavefronts enough that way: a wavefront
@@ -224,7 +236,7 @@ static SolverKernel KernelOfWidth(const ModelView& m, Heads heads, uint32_t widt
 // and 339).
 constexpr uint32_t kPackedBatch = 8192u;
 static bool PackedSolverTakes(const ModelView& m, Heads heads, uint32_t staged, uint32_t env_count) {
-    return heads == Heads::Contacts && m.dof <= uint32_t(solver::kPackedWidth) && m.max_dof <= 16u && staged <= solver::kPackedHeads && env_count >= kPackedBatch;
+    return heads == kContactHeads && m.dof <= uint32_t(solver::kPackedWidth) && m.max_dof <= 16u && staged <= solver::kPackedHeads && env_count >= kPackedBatch;
 }
 // Environments that have a wavefront to themselves, the costliest: one a compute unit until the others' wavefronts take
 // longer than they do (16384 free boxes 429 us without them, 392 with; 65536 981 and 989).
@@ -240,7 +252,7 @@ uint32_t SolverBlocksPerUnit(const ModelView& m, uint32_t env_count) {
     const Heads heads = HeadsOf(m, staged);
     const uint32_t width = SolverWorkingWidth(m, heads);
     const size_t lds = size_t{solver::ReducedSolverLdsFloats(m.dof, width, staged + joint_heads, staged,
-                                                             solver::RowsFromLinks(width, heads == Heads::Contacts, m.rows_from_links))} * sizeof(float);
+                                                             solver::RowsFromLinks(width, heads == kContactHeads, m.rows_from_links))} * sizeof(float);
     int blocks = 0;
     if (PackedSolverTakes(m, heads, staged, env_count)) {
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, reinterpret_cast<const void*>(PackedDescentKernel), solver::kWave, PackedLdsBytes(staged)) != hipSuccess) {
@@ -264,7 +276,7 @@ uint32_t SolverMassFactorFloats(const ModelView& m) {
 uint32_t SolverSweepWidth(const ModelView& m) {
     if (m.rows_per_env == 0u || m.dof == 0u) return m.dof;
     const uint32_t staged = SolverHeadCapacity(m, std::max(m.contact_slots, 1u));
-    return SolverWorkingWidth(m, staged != 0u ? HeadsOf(m, staged) : Heads::Any);
+    return SolverWorkingWidth(m, staged != 0u ? HeadsOf(m, staged) : kAnyHeads);
 }
 
 Status OpBlockDescentSolve(const ModelView& m, const DataView& d, const void* params, hipStream_t stream) {
@@ -280,7 +292,7 @@ Status OpBlockDescentSolve(const ModelView& m, const DataView& d, const void* pa
     const uint32_t width = SolverWorkingWidth(m, heads);
     const auto lds_bytes = [&](uint32_t contact_heads) {
         return size_t{solver::ReducedSolverLdsFloats(m.dof, width, contact_heads + joint_heads, contact_heads,
-                                                     solver::RowsFromLinks(width, heads == Heads::Contacts, m.rows_from_links))} * sizeof(float);
+                                                     solver::RowsFromLinks(width, heads == kContactHeads, m.rows_from_links))} * sizeof(float);
     };
     bool dense = false;
     const SolverKernel kernel = KernelOfWidth(m, heads, width, p->env_count, &dense);

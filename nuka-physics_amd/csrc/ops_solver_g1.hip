@@ -1,0 +1,9 @@
+// Instantiations of the block-descent kernel (general variant without the elliptic cone) for padded widths 24, 28, 32.
+#include "ops_solver_kernel.h"
+namespace nkh {
+namespace solver {
+template __global__ void BlockDescentTileKernel<24, false, 24, false>(ModelView, DataView, BlockDescentSolveParams, uint32_t, uint32_t, uint32_t, uint32_t);
+template __global__ void BlockDescentTileKernel<28, false, 28, false>(ModelView, DataView, BlockDescentSolveParams, uint32_t, uint32_t, uint32_t, uint32_t);
+template __global__ void BlockDescentTileKernel<32, false, 32, false>(ModelView, DataView, BlockDescentSolveParams, uint32_t, uint32_t, uint32_t, uint32_t);
+}  // namespace solver
+}  // namespace nkh

@@ -1,0 +1,9 @@
+// Instantiations of the block-descent kernel (general variant without the elliptic cone) for padded widths 36, 40, 44.
+#include "ops_solver_kernel.h"
+namespace nkh {
+namespace solver {
+template __global__ void BlockDescentTileKernel<36, false, 36, false>(ModelView, DataView, BlockDescentSolveParams, uint32_t, uint32_t, uint32_t, uint32_t);
+template __global__ void BlockDescentTileKernel<40, false, 40, false>(ModelView, DataView, BlockDescentSolveParams, uint32_t, uint32_t, uint32_t, uint32_t);
+template __global__ void BlockDescentTileKernel<44, false, 44, false>(ModelView, DataView, BlockDescentSolveParams, uint32_t, uint32_t, uint32_t, uint32_t);
+}  // namespace solver
+}  // namespace nkh
