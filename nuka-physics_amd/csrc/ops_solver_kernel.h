@@ -2689,7 +2689,7 @@ __host__ __device__ inline uint32_t ReducedSolverLdsFloats(uint32_t full, uint32
 // The coordinates N-1 .. K are eliminated leaves first (FactorTileColumns' order): the lanes below K are left with
 // their rows of the Schur complement S = M_TT - M_TU M_UU^-1 M_UT and of U_TU = M_TU U_UU^-T, the followers with their
 // rows of the factor M_UU = U_UU U_UU^T.  P = M_UU^-1 M_UT = U_UU^-T U_TU^T then follows by forward substitution over the
-// followers in ascending order, its two operands passing through LDS to be read transposed.  On return a lane below K
+// followers in ascending order, a column of P a lane, which passes through LDS to be read by rows.  On return a lane below K
 // holds its row of S as the sum of two floats, mrow in registers and the second in LDS at `low` (read by low_row), a
 // follower its row of -P rounded to float in mrow.
 // Double because these rows stand in for the mass matrix over the whole solve: a Schur complement eliminated in
@@ -2741,42 +2741,50 @@ __device__ __forceinline__ bool reduce_block(uint32_t lane, uint32_t n, const fl
                 if (4 * q + t <= k - 1) full[4 * q + t] = fma(-full[k], u[t], full[4 * q + t]);
         }
     }
-    double* coupling = reinterpret_cast<double*>(lds);   // [follower][coordinate below K]: U_TU transposed
-    double* corner = coupling + kFollowers * K;           // [follower i][follower k]: U_UU[i][k], zero from the diagonal down
+    double* solved = reinterpret_cast<double*>(lds);      // [follower][coordinate below K]: what the substitution ends with
+    double* corner = solved + kFollowers * K;             // [follower i][follower k]: U_UU[i][k] right of the diagonal, 1 / U_UU[i][i] on it
+    if (lane >= uint32_t(K) && lane < uint32_t(N)) {
+#pragma unroll
+        for (int k = K; k < N; ++k) corner[(int(lane) - K) * kFollowers + (k - K)] = full[k];
+        corner[(int(lane) - K) * (kFollowers + 1)] = own_scale;
+    }
+    lds_sync<K>();
+    // lane = coordinate below K: its own entries of U_TU are a column of the coupling, and the substitution runs down them with the
+    // factor's rows the same for every lane, two entries a read.  (A lane a follower, column after column, each a chain of lane
+    // reads, took 1.3 k instructions where this takes 250: 65536 humanoids 7570 -> 7512 us, 4096 704 -> 699, the bits the same.)
+#pragma unroll
+    for (int j = 0; j < kFollowers; ++j) {
+        uint32_t from = uint32_t(j * kFollowers);
+        if (j > 0) asm volatile("" : "+v"(from) : "v"(full[K + j - 1]));   // (two rows' words in registers at a time, not all of them)
+        const double2* row = reinterpret_cast<const double2*>(corner + from);
+#pragma unroll
+        for (int q = j / 2; q < kFollowers / 2; ++q) {
+            const double2 u = row[q];
+            if (2 * q == j) full[K + j] *= u.x;
+            if (2 * q + 1 == j) full[K + j] *= u.y;
+            if (2 * q > j) full[K + 2 * q] = fma(u.x, -full[K + j], full[K + 2 * q]);
+            if (2 * q + 1 > j) full[K + 2 * q + 1] = fma(u.y, -full[K + j], full[K + 2 * q + 1]);
+        }
+    }
     if (lane < uint32_t(K)) {
 #pragma unroll
-        for (int k = K; k < N; ++k) coupling[(k - K) * K + int(lane)] = full[k];
-    } else if (lane < uint32_t(N)) {
-#pragma unroll
-        for (int k = K; k < N; ++k) corner[(int(lane) - K) * kFollowers + (k - K)] = uint32_t(k) > lane ? full[k] : 0.0;
+        for (int i = 0; i < kFollowers; ++i) solved[i * K + int(lane)] = full[K + i];
     }
     lds_sync<K>();
     const uint32_t slot = lane >= uint32_t(K) && lane < uint32_t(N) ? lane - uint32_t(K) : 0u;
-    double prow[K], column[kFollowers];
 #pragma unroll
     for (int q = 0; q < K / 2; ++q) {
-        const double2 v = reinterpret_cast<const double2*>(coupling + slot * uint32_t(K))[q];
-        prow[2 * q] = v.x; prow[2 * q + 1] = v.y;
-    }
-#pragma unroll
-    for (int i = 0; i < kFollowers; ++i) column[i] = corner[i * kFollowers + int(slot)];
-    // Column by column (the columns do not meet in the substitution).  A column of the coupling that is zero in every
-    // follower's row stays zero - a leg's coordinate and an arm's share no link - and is left out, on a uniform test.
-#pragma unroll
-    for (int c0 = 0; c0 < K; ++c0) {
-        if (__ballot(lane >= uint32_t(K) && lane < uint32_t(N) && prow[c0] != 0.0) == 0ull) continue;
-#pragma unroll
-        for (int i = K; i < N; ++i) {
-            const double y = lane_value_d(prow[c0] * own_scale, i);
-            prow[c0] = fma(column[i - K], -y, prow[c0]);   // (the column holds zeros for the followers up to i)
-        }
+        const double2 v = reinterpret_cast<const double2*>(solved + slot * uint32_t(K))[q];
+        full[2 * q] = lane >= uint32_t(K) ? -v.x : full[2 * q];
+        full[2 * q + 1] = lane >= uint32_t(K) ? -v.y : full[2 * q + 1];
     }
     float rest[K];
 #pragma unroll
     for (int k = 0; k < K; ++k) {
-        const double entry = lane < uint32_t(K) ? full[k] : (lane < n ? -(prow[k] * own_scale) : 0.0);
+        const double entry = lane < uint32_t(K) || lane < n ? full[k] : 0.0;
         mrow[k] = float(entry);
         rest[k] = float(entry - double(mrow[k]));
+        asm volatile("" : "+v"(mrow[k]));   // (or the double stays beside the float over the sweeps, in registers they need)
     }
     if (lane < uint32_t(K)) {   // (the scratch above has been read: its words may be these)
         float4* words = reinterpret_cast<float4*>(low + lane * uint32_t(K));
