@@ -1034,6 +1034,7 @@ __global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(kCom
         if (d.row_clear_extent != nullptr) d.row_clear_extent[env] = extent;
     }
     // padded generalized velocity tile (:200-214)
+    float free_velocity = 0.0f;   // of lane's coordinate
     if (lane < md) {
         float value = 0.0f;
         if (lane < m.dof) {
@@ -1041,6 +1042,7 @@ __global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(kCom
             value = c == kInvalid ? d.qdot[size_t{env} * nl + link] : d.link_velocity[(size_t{env} * nl + link) * 6u + c];
         }
         d.qdot_flat[size_t{env} * md + lane] = value;
+        free_velocity = value;
     }
     __syncthreads();
     // lane = DoF: the coordinate's axis, where it lies and whether it turns
@@ -1076,7 +1078,7 @@ __global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(kCom
     // contact rows (:453-801; speculative law, condim 3): a lane a slot where every slot has one point at most, else a
     // lane a (slot, point) - a slot's points share nothing but the slot's own values, which each of their lanes works
     // out for itself
-    uint32_t active_rows = 0u;
+    uint32_t active_rows = 0u, driven_points = 0u;
     bool invalid_endpoint = false;
     const uint32_t fan = __any(many) ? 4u : 1u;
     constexpr int kAxes = kCompliant ? 4 : 3;   // rows a point
@@ -1310,6 +1312,8 @@ __global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(kCom
                     if (links[0] != kInvalid) d.chain_jacobian[(size_t{env} * R + r) * md + lane] = entries[0];
                     if (links[1] != kInvalid) d.chain_jacobian_b[(size_t{env} * R + r) * md + lane] = entries[1];
                 }
+                // a point whose first row the free velocity drives into is one the solve will have to answer
+                if (axis == 0 && uniform_value(my_rhs[0], i) * p.dt > wave_sum((entries[0] + entries[1]) * free_velocity)) ++driven_points;
                 if constexpr (kCompliant) {
                     const float gain = uniform_value(my_gain[axis], i);
                     if (gain == 0.0f) continue;
@@ -1419,6 +1423,7 @@ __global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(kCom
     invalid_endpoint = __any(invalid_endpoint);
     if (lane == 0u) {
         d.row_count[env] = active_rows;
+        if (d.solver_cost != nullptr) d.solver_cost[env] = solve_cost_expected(d.solver_cost[env], driven_points);
         if (invalid_endpoint) d.env_status[env] |= kEnvStatusInvalidEndpoint;
     }
 }

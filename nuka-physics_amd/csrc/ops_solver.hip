@@ -69,7 +69,7 @@ namespace {
 using namespace solver;
 
 // OrderTilesKernel (block_descent_tile.cuh:3097-3121 orders tiles for its persistent kernel; here the order feeds the
-// grid): environments sorted by the work their previous solve took, costliest first, so that the few long solves
+// grid): environments sorted by the work their solve is taken to be (solve_cost), costliest first, so that the few long solves
 // start at once instead of trailing the launch.  Each of B workgroups sorts every B-th environment, a counting sort on a
 // 256-level key, and puts its i-th costliest to place i B + its own number: the costliest of all of them come first, then
 // the second ones.  The order inside a level is arbitrary, which changes when an environment runs and nothing it computes.
@@ -84,13 +84,14 @@ __global__ void __launch_bounds__(1024) OrderTilesKernel(DataView d, uint32_t en
     if (t == 0u) top = 0u;
     __syncthreads();
     const uint32_t mine = first + t * blocks, step = 1024u * blocks;
+    const auto cost_of = [&](uint32_t e) { return solve_cost(d.solver_cost[e]); };
     uint32_t largest = 0u;
-    for (uint32_t e = mine; e < env_count; e += step) largest = max(largest, d.solver_cost[e]);
+    for (uint32_t e = mine; e < env_count; e += step) largest = max(largest, cost_of(e));
     largest = wave_max_u(largest);
     if ((t & 63u) == 0u) atomicMax(&top, largest);
     __syncthreads();
     const uint32_t scale = top / 256u + 1u;
-    for (uint32_t e = mine; e < env_count; e += step) atomicAdd(&bins[255u - min(d.solver_cost[e] / scale, 255u)], 1u);
+    for (uint32_t e = mine; e < env_count; e += step) atomicAdd(&bins[255u - min(cost_of(e) / scale, 255u)], 1u);
     __syncthreads();
     // exclusive prefix of the 256 counts: a scan inside each of the first four wavefronts, then their totals
     __shared__ uint32_t wave_total[4];
@@ -112,7 +113,7 @@ __global__ void __launch_bounds__(1024) OrderTilesKernel(DataView d, uint32_t en
         bins[t] = before + through - count;
     }
     __syncthreads();
-    for (uint32_t e = mine; e < env_count; e += step) d.tile_order[atomicAdd(&bins[255u - min(d.solver_cost[e] / scale, 255u)], 1u) * blocks + first] = e;
+    for (uint32_t e = mine; e < env_count; e += step) d.tile_order[atomicAdd(&bins[255u - min(cost_of(e) / scale, 255u)], 1u) * blocks + first] = e;
 }
 
 

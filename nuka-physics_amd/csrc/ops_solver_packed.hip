@@ -840,8 +840,7 @@ PackedDescentKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint32_t
         d.solver_residual[size_t{env} * 4u + lane] = lane == 0u ? residual4[0] : lane == 1u ? residual4[1] : lane == 2u ? residual4[2] : residual4[3];
     if (lane == 0u) {
         d.vbd_velocity_sweep_count[env] = sweeps;
-        const uint32_t earlier = d.solver_cost[env];
-        d.solver_cost[env] = max(c.work, earlier - earlier / 4u);
+        d.solver_cost[env] = solve_cost_after(d.solver_cost[env], c.work);
     }
     if (lane < md) {   // (a block of at most W coordinates has no more words a row than lanes)
         d.solver_velocity[size_t{env} * md + lane] = coordinate ? velocity : 0.0f;
