@@ -23,6 +23,7 @@ NKH_DECLARE_REDUCED(64, 32)
 // the same for worlds under the elliptic cone
 #define NKH_DECLARE_ELLIPTIC(N, K) \
     extern template __global__ void BlockDescentTileKernel<N, true, K, true>(ModelView, DataView, BlockDescentSolveParams, uint32_t, uint32_t, uint32_t, uint32_t);
+NKH_DECLARE_ELLIPTIC(4, 4) NKH_DECLARE_ELLIPTIC(8, 8) NKH_DECLARE_ELLIPTIC(12, 12) NKH_DECLARE_ELLIPTIC(16, 16) NKH_DECLARE_ELLIPTIC(20, 20)
 NKH_DECLARE_ELLIPTIC(24, 12) NKH_DECLARE_ELLIPTIC(28, 16) NKH_DECLARE_ELLIPTIC(32, 16) NKH_DECLARE_ELLIPTIC(36, 20) NKH_DECLARE_ELLIPTIC(40, 20)
 NKH_DECLARE_ELLIPTIC(44, 24) NKH_DECLARE_ELLIPTIC(48, 24) NKH_DECLARE_ELLIPTIC(52, 28) NKH_DECLARE_ELLIPTIC(56, 28) NKH_DECLARE_ELLIPTIC(60, 32)
 NKH_DECLARE_ELLIPTIC(64, 32)
@@ -141,6 +142,12 @@ const SolverKernel kSolverKernels[3][16] = {
 // One reduced instantiation per padded width from 24 on: the sweeps run at about half the width.  A world takes it
 // when no contact can reach a coordinate from that width on (ModelView::contact_dof_end).
 struct ReducedKernel { uint32_t width, reduced; SolverKernel kernel; };
+// Contact heads under the elliptic cone at the full widths 4 to 20; wider ones that are not reduced take the general kernel
+// (the general kernel keeps what joint rows need: 4096 quadrupeds under the cone 363 -> 347 us a step, 16384 1150 -> 1096, 500 245
+// -> 234, the bits the same)
+const SolverKernel kEllipticFull[] = {BlockDescentTileKernel<4, true, 4, true>, BlockDescentTileKernel<8, true, 8, true>, BlockDescentTileKernel<12, true, 12, true>,
+                                      BlockDescentTileKernel<16, true, 16, true>, BlockDescentTileKernel<20, true, 20, true>};
+constexpr uint32_t kEllipticFullMost = 20u;
 const ReducedKernel kReducedKernels[] = {
     {24u, 12u, BlockDescentTileKernel<24, true, 12>}, {28u, 16u, BlockDescentTileKernel<28, true, 16>},
     {32u, 16u, BlockDescentTileKernel<32, true, 16>}, {36u, 20u, BlockDescentTileKernel<36, true, 20>},
@@ -188,6 +195,10 @@ void InitSolverKernels() {
         (void)hipFuncSetAttribute(reinterpret_cast<const void*>(reduced.kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
         (void)hipGetLastError();
     }
+    for (SolverKernel elliptic : kEllipticFull) {
+        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(elliptic), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+        (void)hipGetLastError();
+    }
     for (const ReducedKernel& elliptic : kEllipticKernels) {
         (void)hipFuncSetAttribute(reinterpret_cast<const void*>(elliptic.kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
         (void)hipGetLastError();
@@ -199,7 +210,7 @@ void InitSolverKernels() {
 }
 
 // The heads a world's solve meets: anything or contact heads only, at most one a lane, either with or without the elliptic cone
-// of the MuJoCo law (contact heads under it take the general kernel at the full width).
+// of the MuJoCo law (contact heads under it take the general kernel at full widths past 20).
 static Heads HeadsOf(const ModelView& m, uint32_t staged) {
     const uint32_t joint_heads = m.joint_limit_rows + m.joint_friction_rows + m.joint_drive_rows;
     const bool elliptic = m.any_mujoco != 0u && m.contact_cone == 1u;
@@ -229,6 +240,7 @@ static SolverKernel KernelOfWidth(const ModelView& m, Heads heads, uint32_t widt
         for (const ReducedKernel& reduced : heads == kContactElliptic ? kEllipticKernels : kReducedKernels)
             if (reduced.width == solver::PaddedWidth(m.dof) && reduced.reduced == width) return reduced.kernel;
     }
+    if (heads == kContactElliptic && solver::PaddedWidth(m.dof) <= kEllipticFullMost) return kEllipticFull[solver::PaddedWidth(m.dof) / 4u - 1u];
     return kSolverKernels[heads == kContactElliptic ? kAnyElliptic : heads][solver::PaddedWidth(m.dof) / 4u - 1u];
 }
 // Worlds whose environments are solved four a wavefront (ops_solver_packed.hip): contact heads only, no more of them and no
