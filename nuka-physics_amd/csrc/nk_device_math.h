@@ -286,24 +286,22 @@ __device__ __forceinline__ uint32_t opaque_word(uint32_t v) {
 __device__ __forceinline__ bool wave_all(bool p) { return __all(p); }
 __device__ __forceinline__ bool wave_any(bool p) { return __any(p); }
 
-// What the launch order of the solve goes by, a word an environment: the work of the last solves in its lower half (a decaying
-// maximum: an environment whose solves are long every other step or so keeps its early place), then a byte with the contact
-// points that its free velocity drove into ahead of the last solve and one with those it drives into ahead of the next.  The
-// work stands for a solve of as many points; where the number is another - another state, or none yet - the points do.  Of all
-// that is known ahead of a solve they say the most of its length (correlations of 0.73 to 0.90 between states that have nothing
-// to do with each other, 0.5 to 0.9 from step to step of one that goes on, where the last step's work has 0.6 to 0.9).  Nine
-// states in turn, a step, by the work alone and so: 4096 quadrupeds 590 -> 532 us, 4096 humanoids 1001 -> 802, servo-driven 2013
-// -> 1553, 16384 boxes 625 -> 447; five steps on from each 574 -> 548, 816 -> 714, 1497 -> 1375 and 636 -> 476 (the other gains
-// since then, a twentieth at most but for the boxes' third, among them).
-constexpr uint32_t kSolveCostMost = 0xFFFFu, kPointCost = 64u, kNoPointCost = 60u;
-__device__ __forceinline__ uint32_t solve_cost_expected(uint32_t word, uint32_t points) { return (word & 0xFFFFFFu) | (min(points, 255u) << 24u); }
-__device__ __forceinline__ uint32_t solve_cost_after(uint32_t word, uint32_t work) {
-    const uint32_t earlier = word & kSolveCostMost, points = word >> 24u;
-    return min(max(work, earlier - earlier / 4u), kSolveCostMost) | (points << 16u) | (points << 24u);
-}
-__device__ __forceinline__ uint32_t solve_cost(uint32_t word) {
-    const uint32_t work = word & kSolveCostMost, points = word >> 24u;
-    return work != 0u && ((word >> 16u) & 0xFFu) == points ? work : kNoPointCost + kPointCost * points;
+// What the launch order of the solve goes by, two words an environment.  DataView::solver_cost is the work of the last solves (a
+// decaying maximum: an environment whose solves are long every other step or so keeps its early place).  DataView::solver_points
+// holds the contact points that its free velocity drove into ahead of the last solve in its lower half, those it drives into ahead
+// of the next in its upper half.  The work stands for a solve of as many points; where the number is another - another state, or
+// none yet - the points do.  Of all that is known ahead of a solve they say the most of its length (correlations of 0.73 to 0.90
+// between states that have nothing to do with each other, 0.5 to 0.9 from step to step of one that goes on, where the last step's
+// work has 0.6 to 0.9).  Nine states in turn, a step, by the work alone and so: 4096 quadrupeds 590 -> 532 us, 4096 humanoids 1001
+// -> 802, servo-driven 2013 -> 1553, 16384 boxes 625 -> 447; five steps on from each 574 -> 548, 816 -> 714, 1497 -> 1375 and 636
+// -> 476 (the other gains since then, a twentieth at most but for the boxes' third, among them).
+constexpr uint32_t kMostPoints = 0xFFFFu, kPointCost = 64u, kNoPointCost = 60u;
+__device__ __forceinline__ uint32_t points_expected(uint32_t word, uint32_t points) { return (word & kMostPoints) | (min(points, kMostPoints) << 16u); }
+__device__ __forceinline__ uint32_t points_solved(uint32_t word) { return (word >> 16u) | (word & ~kMostPoints); }
+__device__ __forceinline__ uint32_t solve_cost_after(uint32_t earlier, uint32_t work) { return max(work, earlier - earlier / 4u); }
+__device__ __forceinline__ uint32_t solve_cost(uint32_t work, uint32_t word) {
+    const uint32_t points = word >> 16u;
+    return work != 0u && (word & kMostPoints) == points ? work : kNoPointCost + kPointCost * points;
 }
 
 }  // namespace nkh

@@ -1423,7 +1423,7 @@ __global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(kCom
     invalid_endpoint = __any(invalid_endpoint);
     if (lane == 0u) {
         d.row_count[env] = active_rows;
-        if (d.solver_cost != nullptr) d.solver_cost[env] = solve_cost_expected(d.solver_cost[env], driven_points);
+        if (d.solver_points != nullptr) d.solver_points[env] = points_expected(d.solver_points[env], driven_points);
         if (invalid_endpoint) d.env_status[env] |= kEnvStatusInvalidEndpoint;
     }
 }

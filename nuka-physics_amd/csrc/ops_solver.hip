@@ -85,7 +85,7 @@ __global__ void __launch_bounds__(1024) OrderTilesKernel(DataView d, uint32_t en
     if (t == 0u) top = 0u;
     __syncthreads();
     const uint32_t mine = first + t * blocks, step = 1024u * blocks;
-    const auto cost_of = [&](uint32_t e) { return solve_cost(d.solver_cost[e]); };
+    const auto cost_of = [&](uint32_t e) { return solve_cost(d.solver_cost[e], d.solver_points != nullptr ? d.solver_points[e] : 0u); };
     uint32_t largest = 0u;
     for (uint32_t e = mine; e < env_count; e += step) largest = max(largest, cost_of(e));
     largest = wave_max_u(largest);

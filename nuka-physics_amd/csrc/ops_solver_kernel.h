@@ -3469,6 +3469,7 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
     if (lane == 0u) {
         d.vbd_velocity_sweep_count[env] = sweeps;
         d.solver_cost[env] = solve_cost_after(d.solver_cost[env], c.work);   // the scheduling key of the next solves
+        if (d.solver_points != nullptr) d.solver_points[env] = points_solved(d.solver_points[env]);
     }
 #ifdef NKH_SOLVER_PROFILE
     PROF_END(c, 9);

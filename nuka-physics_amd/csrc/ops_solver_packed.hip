@@ -841,6 +841,7 @@ PackedDescentKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint32_t
     if (lane == 0u) {
         d.vbd_velocity_sweep_count[env] = sweeps;
         d.solver_cost[env] = solve_cost_after(d.solver_cost[env], c.work);
+        if (d.solver_points != nullptr) d.solver_points[env] = points_solved(d.solver_points[env]);
     }
     if (lane < md) {   // (a block of at most W coordinates has no more words a row than lanes)
         d.solver_velocity[size_t{env} * md + lane] = coordinate ? velocity : 0.0f;

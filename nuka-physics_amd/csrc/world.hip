@@ -378,7 +378,7 @@ struct Field { const char* name; Dtype dtype; uint32_t elem_bytes; size_t count;
     X(row_cj_link, kU32, E * R) X(row_cj_link_b, kU32, E * R) X(row_count, kU32, E) X(contact_count, kU32, E) \
     X(contact_row_extent, kU32, E * 2) X(row_clear_extent, kU32, E) X(env_status, kU32, E) X(vbd_velocity_sweep_count, kU32, E) \
     X(solver_residual, kF32, E * 4) X(solver_penalty, kF32, E * R) X(solver_velocity, kF32, E * md) X(solver_free, kF32, E * md) \
-    X(solver_cost, kU32, E) X(tile_order, kU32, E) X(row_unit, kU32, E * R) X(row_unit_value, kF32, E * R) \
+    X(solver_cost, kU32, E) X(tile_order, kU32, E) X(solver_points, kU32, E) X(row_unit, kU32, E * R) X(row_unit_value, kF32, E * R) \
     X(solver_mass_factor, kF32, E * mf) \
     X(body_invweight0, kF32, E * nb * 2) X(dof_invweight0, kF32, E * md) X(row_invweight, kF32, E * R) \
     X(row_reference_velocity_gain, kF32, E * R) X(step_qdot_flat, kF32, E * md) \
@@ -1359,7 +1359,7 @@ const char* ReferenceName(const char* name) {
     static const char* const renamed[][2] = {{"dof_link", "dof_to_link"}, {"dof_component", "dof_to_component"}};
     static const char* const own[] = {"joint_law", "link_push_order", "sweep_links", "link_dof", "link_dof_mask", "pairable_rows", "profile_mu",
                                       "profile_law", "profile_solref", "profile_solimp", "profile_margin", "profile_mix", "articulation_qdd",
-                                      "solver_penalty", "solver_velocity", "solver_free", "solver_cost", "tile_order", "row_unit",
+                                      "solver_penalty", "solver_velocity", "solver_free", "solver_cost", "tile_order", "solver_points", "row_unit",
                                       "row_unit_value", "solver_mass_factor", "contact_cache_match", "row_clear_extent"};
     for (const auto& pair : renamed) if (std::strcmp(name, pair[0]) == 0) return pair[1];
     for (const char* mine : own) if (std::strcmp(name, mine) == 0) return nullptr;
