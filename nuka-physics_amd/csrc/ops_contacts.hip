@@ -1312,8 +1312,12 @@ __global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(kCom
                     if (links[0] != kInvalid) d.chain_jacobian[(size_t{env} * R + r) * md + lane] = entries[0];
                     if (links[1] != kInvalid) d.chain_jacobian_b[(size_t{env} * R + r) * md + lane] = entries[1];
                 }
-                // a point whose first row the free velocity drives into is one the solve will have to answer
-                if (axis == 0 && uniform_value(my_rhs[0], i) * p.dt > wave_sum((entries[0] + entries[1]) * free_velocity)) ++driven_points;
+                // a point whose first row the free velocity drives into is one the solve will have to answer (a compliant row's
+                // right-hand side is still without its damping of the start velocity here)
+                if (axis == 0) {
+                    const float velocity = kCompliant ? fmaf(-p.dt * uniform_value(my_gain[0], i), start_velocity, free_velocity) : free_velocity;
+                    if (uniform_value(my_rhs[0], i) * p.dt > wave_sum((entries[0] + entries[1]) * velocity)) ++driven_points;
+                }
                 if constexpr (kCompliant) {
                     const float gain = uniform_value(my_gain[axis], i);
                     if (gain == 0.0f) continue;

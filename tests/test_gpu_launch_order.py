@@ -66,3 +66,36 @@ def test_the_work_field_holds_the_decaying_maximum_of_the_solves(device, index, 
         level = earlier[mine] // (earlier[mine].max() // 256 + 1)
         assert (mine % blocks == first).all() and (np.diff(level) <= 0).all()
     world.close()
+
+
+@pytest.mark.parametrize("index,law", [(2, "native"), (3, "native"), (2, "elliptic"), (3, "elliptic"), (2, "pyramidal"), (3, "pyramidal")])
+def test_the_counted_points_are_those_whose_first_row_the_free_velocity_drives_into(device, index, law):
+    """By the rows as the solve meets them: a compliant row's right-hand side includes the damping of the start velocity."""
+    E = 200
+    cfg = nk.synthetic.config(index, E)
+    if law != "native":
+        for profile in cfg.template.profiles:
+            profile["law"] = abi.LAW_MUJOCO
+        cfg.template.contact_cone = abi.CONE_ELLIPTIC if law == "elliptic" else abi.CONE_PYRAMIDAL
+    world = nk.World(device, cfg.template, abi.world_desc(E, cfg.dt, vel_iters=cfg.vel_iters))
+    world.set_state(cfg.state())
+    world.step()
+    world.synchronize()
+    R, S, md = world.rows_per_env, world.info.contact_slots_per_env, world.download("solver_free").size // E
+    words = world.download("urows").reshape(E, R, -1)
+    ranges = world.download("ucontact_row_range").reshape(E, S, 2).astype(np.int64)
+    jacobian = (world.download("chain_jacobian").reshape(E, R, md) + world.download("chain_jacobian_b").reshape(E, R, md)).astype(np.float64)
+    free = world.download("solver_free").reshape(E, md).astype(np.float64)
+    expect, clear = np.zeros(E, np.int64), np.ones(E, bool)
+    for env in range(E):
+        for first, count in ranges[env] - np.array([env * R, 0]):
+            for row in range(first, first + count):
+                if not words[env, row, 0].view(np.uint32) & 1:
+                    continue
+                terms = jacobian[env, row] * free[env]
+                gap = float(words[env, row, 4]) * cfg.dt - terms.sum()
+                expect[env] += gap > 0.0
+                clear[env] &= abs(gap) > 1e-5 * (1.0 + np.abs(terms).sum())   # (64 terms in single precision: below 64 / 2^24 of their size)
+    assert clear.mean() > 0.9 and expect.any()
+    assert np.array_equal((world.download("solver_points") >> 16)[clear], expect[clear])
+    world.close()
