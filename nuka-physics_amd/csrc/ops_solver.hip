@@ -77,7 +77,7 @@ using namespace solver;
 // One workgroup for all of them was bound by its LDS atomics: 80 us for 65536 environments, 22 for 16384 and 9.5 for 4096,
 // 7, 5 and 5 with one for every kOrderEnvs.
 constexpr uint32_t kOrderEnvs = 1024u;
-__global__ void __launch_bounds__(1024) OrderTilesKernel(DataView d, uint32_t env_count) {
+__global__ void __launch_bounds__(1024) OrderTilesKernel(DataView d, uint32_t env_count, bool by_points) {
     __shared__ uint32_t bins[256];
     __shared__ uint32_t top;
     const uint32_t t = threadIdx.x, first = blockIdx.x, blocks = gridDim.x;
@@ -85,7 +85,7 @@ __global__ void __launch_bounds__(1024) OrderTilesKernel(DataView d, uint32_t en
     if (t == 0u) top = 0u;
     __syncthreads();
     const uint32_t mine = first + t * blocks, step = 1024u * blocks;
-    const auto cost_of = [&](uint32_t e) { return solve_cost(d.solver_cost[e], d.solver_points != nullptr ? d.solver_points[e] : 0u); };
+    const auto cost_of = [&](uint32_t e) { return by_points ? solve_cost(d.solver_cost[e], d.solver_points[e]) : d.solver_cost[e]; };
     uint32_t largest = 0u;
     for (uint32_t e = mine; e < env_count; e += step) largest = max(largest, cost_of(e));
     largest = wave_max_u(largest);
@@ -331,7 +331,15 @@ Status OpBlockDescentSolve(const ModelView& m, const DataView& d, const void* pa
     // A contact point is at most `a_point` heads, so `few` heads hold few / a_point points whatever their friction: four
     // edges a point under the pyramidal cone.  (While those worlds went to the one full launch, a walker's 304 heads left a
     // compute unit one block for environments of a handful of points: a step of 4096 with a twentieth reset 768 -> 438 us.)
-    hipLaunchKernelGGL(OrderTilesKernel, dim3((p->env_count + kOrderEnvs - 1u) / kOrderEnvs), dim3(1024), 0, stream, d, p->env_count);
+    // Whether the order goes by the counted points in a state that is new.  Under the pyramidal cone the points say how many heads an
+    // environment has and little of its Newton steps - some of any count take three times the others' - so that the many-headed
+    // ones together ahead of the rest start those later than any order would: four states in turn, by the work alone and by the
+    // points, 4096 humanoids 583 and 623 us, 2500 433 and 464, 16384 1855 and 1876, 6000 quadrupeds 462 and 472, 12288 boxes 359 and
+    // 370.  Not so where a full launch leaves a compute unit fewer blocks than it has SIMDs, which the few environments of many
+    // points have to themselves: 4096 walkers (one block) 305 and 289, 8192 464 and 442.
+    const uint32_t a_point = HeadsAPoint(m);
+    const bool by_points = d.solver_points != nullptr && (a_point == 1u || blocks_per_unit(staged) < 4u);
+    hipLaunchKernelGGL(OrderTilesKernel, dim3((p->env_count + kOrderEnvs - 1u) / kOrderEnvs), dim3(1024), 0, stream, d, p->env_count, by_points);
     if (PackedSolverTakes(m, heads, staged, p->env_count)) {
         const uint32_t alone = PackedAlone(p->env_count);
         hipLaunchKernelGGL(PackedDescentKernel, dim3(alone + (p->env_count - alone + kPackedEnvs - 1u) / kPackedEnvs), dim3(solver::kWave),
@@ -339,7 +347,6 @@ Status OpBlockDescentSolve(const ModelView& m, const DataView& d, const void* pa
         return hipGetLastError() == hipSuccess ? Status::Ok : Status::Failed;
     }
     uint32_t first_points = 0u;
-    const uint32_t a_point = HeadsAPoint(m);
     const bool few_rounds = p->env_count < kManyRounds * kUnits * blocks_per_unit(staged);
     if (p->contact_slots_per_env != 0u) {
         for (const size_t blocks : {size_t{16u}, size_t{12u}, size_t{8u}, size_t{4u}, size_t{2u}}) {

@@ -99,3 +99,27 @@ def test_the_counted_points_are_those_whose_first_row_the_free_velocity_drives_i
     assert clear.mean() > 0.9 and expect.any()
     assert np.array_equal((world.download("solver_points") >> 16)[clear], expect[clear])
     world.close()
+
+
+@pytest.mark.parametrize("law", ["native", "pyramidal"])
+def test_a_new_state_is_ordered_by_its_points_but_under_the_pyramidal_cone(device, law):
+    """There the points say little of a solve's length: the order stays that of the work."""
+    E = 300
+    cfg = nk.synthetic.config(2, E)
+    if law == "pyramidal":
+        for profile in cfg.template.profiles:
+            profile["law"] = abi.LAW_MUJOCO
+        cfg.template.contact_cone = abi.CONE_PYRAMIDAL
+    world = nk.World(device, cfg.template, abi.world_desc(E, cfg.dt, vel_iters=cfg.vel_iters))
+    world.set_state(cfg.state())
+    work = (np.random.default_rng(7).permutation(E) + 1) * 16
+    world.upload("solver_cost", work.astype(np.uint32))
+    world.upload("solver_points", np.full(E, 0xFFFF, np.uint32))   # no state has so many
+    world.step()
+    world.synchronize()
+    order, points = world.download("tile_order"), world.download("solver_points") >> 16
+    assert np.array_equal(np.sort(order), np.arange(E)) and len(np.unique(points)) > 2
+    by = work if law == "pyramidal" else points
+    level = by[order].astype(np.int64) // (work.max() // 256 + 1 if law == "pyramidal" else 1)
+    assert (np.diff(level) <= 0).all()
+    world.close()
