@@ -245,11 +245,17 @@ static SolverKernel KernelOfWidth(const ModelView& m, Heads heads, uint32_t widt
 }
 // Worlds whose environments are solved four a wavefront (ops_solver_packed.hip): contact heads only, no more of them and no
 // more coordinates than a row of sixteen lanes takes.  From a batch on that has wavefronts enough that way: a wavefront
-// of four takes longer than any of them alone, and 2048 free boxes step in 259 us one a wavefront, 324 packed (8192 342
-// and 339).
-constexpr uint32_t kPackedBatch = 8192u;
+// of four takes longer than any of them alone, and 2048 free boxes step in 259 us one a wavefront, 324 packed (8192 345
+// and 339).  Sixteen heads take 24.8 KB of LDS a wavefront, six of them a compute unit, where four take 10.5 KB and the registers
+// allow twelve: a body of eight coordinates on sixteen points still gains from 8192 on (732 -> 635 us; 1292 -> 1078 at 16384), its
+// sweeps are long.  A free body's four points under the pyramidal cone, sixteen heads of short sweeps, gain from half as many again:
+// 8192 boxes 271 and 290, 9216 289 and 302, 10240 302 and 312, 11264 322 and 298, 12288 339 and 321, 16384 411 and 363.  With eight
+// heads or fewer, or on a tree, that cone gains from 8192 on too (capsules 223 and 223, four-point trees 243 and 236).
+constexpr uint32_t kPackedBatch = 8192u, kPackedEdgesBatch = kPackedBatch + kPackedBatch / 2u;
 static bool PackedSolverTakes(const ModelView& m, Heads heads, uint32_t staged, uint32_t env_count) {
-    return heads == kContactHeads && m.dof <= uint32_t(solver::kPackedWidth) && m.max_dof <= 16u && staged <= solver::kPackedHeads && env_count >= kPackedBatch;
+    const bool edges = m.free_body != 0u && HeadsAPoint(m) != 1u && staged > 8u;
+    return heads == kContactHeads && m.dof <= uint32_t(solver::kPackedWidth) && m.max_dof <= 16u && staged <= solver::kPackedHeads &&
+        env_count >= (edges ? kPackedEdgesBatch : kPackedBatch);
 }
 // Environments that have a wavefront to themselves, the costliest: one a compute unit until the others' wavefronts take
 // longer than they do (16384 free boxes 429 us without them, 392 with; 65536 981 and 989).

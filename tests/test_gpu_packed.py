@@ -26,8 +26,9 @@ def copies_alike(big, name, E, count):
     return batch[:E]
 
 
-# a last wavefront of one, two and three environments, and batches with and without environments that go alone
-@pytest.mark.parametrize("count", [8193, 8194, 8195, 24576, 24577])
+# a last wavefront of one, two and three environments, and batches with and without environments that go alone; under the
+# pyramidal cone the last batch that does not go four a wavefront and the first ones that do
+@pytest.mark.parametrize("count", [8193, 8194, 8195, 12287, 12288, 12289, 12290, 12291, 24576, 24577])
 @pytest.mark.parametrize("law", ["native", "pyramidal"])
 def test_free_boxes_four_a_wavefront(device, count, law):
     E = 60
@@ -73,3 +74,15 @@ def test_small_trees_four_a_wavefront(oracle_py, device, dof, floating):
         error = per_env_error(copies_alike(big, name, E, count), small.download(name), E).max()
         assert error <= bar(sens, "lambda" if name == "lambda" else "velocity"), (name, error)
     small.close(); big.close()
+
+
+@pytest.mark.parametrize("count,packed", [(8192, False), (12287, False), (12288, True)])
+def test_boxes_under_the_pyramidal_cone_go_four_a_wavefront_in_larger_batches(device, count, packed):
+    """Six of the wavefronts of four fit a compute unit; they pay from 12288 environments on."""
+    t = box_template(half=(0.2, 0.15, 0.1), mass=3.0, diag=(0.03, 0.04, 0.05), mu=0.6)
+    for profile in t.profiles:
+        profile["law"] = abi.LAW_MUJOCO
+    t.contact_cone = abi.CONE_PYRAMIDAL
+    world = nk.World(device, t, abi.world_desc(count, 1.0 / 240.0, vel_iters=8, contact_margin=0.02))
+    assert (world.info.solver_blocks_per_cu == 6) == packed
+    world.close()
