@@ -62,6 +62,10 @@ __device__ __forceinline__ float div_by(float a, Recip d) {
     return fmaf(e, d.value, q);
 }
 
+// The same with the division's own last instruction, which gives what the division gives for a divisor or a dividend that is zero,
+// infinite or NaN
+__device__ __forceinline__ float quotient_by(float a, Recip d) { return __builtin_amdgcn_div_fixupf(div_by(a, d), d.divisor, a); }
+
 // Full-precision reciprocal square root: v_rsq_f32 alone is 1 ulp-approximate, sqrt then divide is exact-rounded.  The bits of
 // 1.0f / sqrtf(x) for x between 2^-90 and 2^90 - squared lengths of axes, normals and quaternions - in a third of its
 // instructions, which stand twice on the chain from a link's pose to its child's.  Outside that range the division's own last
@@ -69,7 +73,7 @@ __device__ __forceinline__ float div_by(float a, Recip d) {
 // square of an orientation or axis past 1.8e19 as a diverged environment has one; infinity for zero, NaN for NaN.
 __device__ __forceinline__ float rsqrt_exact(float x) {
     const Recip root = make_recip(sqrt_rn_normal(x));
-    return __builtin_amdgcn_div_fixupf(div_by(1.0f, root), root.divisor, 1.0f);
+    return quotient_by(1.0f, root);
 }
 
 __device__ __forceinline__ Xf load_xf(const float* p) { return Xf{V3{p[0], p[1], p[2]}, Q4{p[3], p[4], p[5], p[6]}}; }

@@ -261,7 +261,8 @@ __device__ __forceinline__ EllipticCone elliptic_cone(float cap, float cn, float
     return k;
 }
 // The rest: the projection onto the friction cone; curvature xx yy zz xy xz yz.  Inside, outside and on the cone are
-// computed side by side and one is selected, so that a probe carries no branch; the quotients by one divisor share its reciprocal.
+// computed side by side and one is selected, so that a probe carries no branch; the quotients by one divisor share its reciprocal
+// and are finished as the division's are, so that they hold over the whole range of the operands.
 struct EllipticLine { EllipticCone k; float scaled[3]; Recip by_x, by_y, by_z; };   // with the scaled duals, over a block descent
 __device__ __forceinline__ EllipticLine elliptic_line(const EllipticCone& k, V3 dual) {
     return EllipticLine{k, {k.e.sx * dual.x, k.e.st * dual.y, k.e.st * dual.z}, make_recip(k.root_x), make_recip(k.root_y), make_recip(k.root_z)};
@@ -270,13 +271,17 @@ __device__ __forceinline__ void elliptic_impulse(const EllipticLine& l, float rx
     const EllipticResponse& e = l.k.e;
     const float root_x = l.k.root_x, root_y = l.k.root_y, root_z = l.k.root_z, m = l.k.slope, a = l.k.share;
     const float xx = fmaf(e.kx, rx, l.scaled[0]), xy = fmaf(e.ky, ry, l.scaled[1]), xz = fmaf(e.kz, rz, l.scaled[2]);
-    const float p = div_by(xx, l.by_x), q1 = div_by(xy, l.by_y), q2 = div_by(xz, l.by_z);
+    const float p = quotient_by(xx, l.by_x), q1 = quotient_by(xy, l.by_y), q2 = quotient_by(xz, l.by_z);
     const float t = hypotf(q1, q2);
     const bool inside = t <= m * p, outside = !inside && m * t + p <= 0.0f;
     const float projected = (p + m * t) * a;
-    const Recip by_t = make_recip(t);
-    const float u1 = div_by(q1, by_t), u2 = div_by(q2, by_t);
-    const float b = div_by(m * projected, by_t), along = m * m * a;
+    // (t has any size down to a subnormal number, whose reciprocal is none: its exponent comes off it and off the dividends, which
+    // are no larger on the cone)
+    const int exponent = -__builtin_amdgcn_frexp_expf(t);
+    const Recip by_t = make_recip(__builtin_ldexpf(t, exponent));
+    const auto over_t = [&](float v) { return quotient_by(__builtin_ldexpf(v, exponent), by_t); };
+    const float u1 = over_t(q1), u2 = over_t(q2);
+    const float b = over_t(m * projected), along = m * m * a;
     const auto one_of = [&](float within, float on) { return inside ? within : outside ? 0.0f : on; };
     f[0] = one_of(xx, projected * root_x); f[1] = one_of(xy, m * projected * u1 * root_y); f[2] = one_of(xz, m * projected * u2 * root_z);
     cv[0] = one_of(e.kx, e.kx * a);
