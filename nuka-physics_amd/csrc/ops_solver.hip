@@ -119,7 +119,8 @@ __global__ void __launch_bounds__(1024) OrderTilesKernel(DataView d, uint32_t en
 
 
 using SolverKernel = void (*)(ModelView, DataView, BlockDescentSolveParams, uint32_t, uint32_t, uint32_t, uint32_t);
-// Three instantiations per padded width, in the order of Heads: the general one without and with the elliptic cone's response
+// Three instantiations per padded width, in the order of the first three of Heads (contact heads under the elliptic cone have the two
+// tables after it): the general one without and with the elliptic cone's response
 // (whose functions and coupled curvatures the other then has no registers and lane reads for: four steps of 1000 servo-driven
 // quadrupeds 1934 -> 1880 us, 4096 servo-driven humanoids 1388 -> 1380), and the one for worlds whose heads
 // are contact heads only, at most one a lane.

@@ -1084,7 +1084,7 @@ __device__ __forceinline__ void add_heads_by_groups(const Tile& c, uint64_t head
     // What a lane needs of its group's head in a pass; the next pass's words are on their way while this one's are worked on.
     // Lanes without a head read the last one's: its rows are staged, and add_columns multiplies a word of theirs by zero, which
     // must be a finite word.
-    struct Words { float f[3], noise[3], cv[6], j[3]; const float* rows; bool live; };
+    struct Words { float f[3], noise[3], cv[4], j[3]; const float* rows; bool live; };   // cv: xx yy zz yz
     const auto fetch = [&](int entry, uint32_t rank) {
         Words w;
         const int source = (entry & 0xFF) * 4;
@@ -1094,7 +1094,8 @@ __device__ __forceinline__ void add_heads_by_groups(const Tile& c, uint64_t head
         for (int k = 0; k < 3; ++k) w.j[k] = rows[uint32_t(k) * uint32_t(N) + column];
         if constexpr (kRows) {
 #pragma unroll
-            for (int k = 0; k < 6; ++k) w.cv[k] = k < 3 || k > 4 || c.elliptic ? lane_permute(source, mc[k]) : 0.0f;
+            for (int k = 0; k < 3; ++k) w.cv[k] = lane_permute(source, mc[k]);
+            w.cv[3] = lane_permute(source, mc[5]);
             w.rows = rows + (lane & 3u);
         }
 #pragma unroll
@@ -1105,12 +1106,7 @@ __device__ __forceinline__ void add_heads_by_groups(const Tile& c, uint64_t head
     const auto take = [&](const Words& w, bool alone) {
         const float j0 = w.live ? w.j[0] : 0.0f, j1 = w.live ? w.j[1] : 0.0f, j2 = w.live ? w.j[2] : 0.0f;
         if constexpr (kRows) {
-            float a0 = j0 * w.cv[0], a1 = j1 * w.cv[1] + j2 * w.cv[5], a2 = j2 * w.cv[2] + j1 * w.cv[5];
-            if (c.elliptic) {   // no other head couples its normal axis to the tangents
-                a0 = (a0 + j1 * w.cv[3]) + j2 * w.cv[4];
-                a1 = a1 + j0 * w.cv[3];
-                a2 = a2 + j0 * w.cv[4];
-            }
+            const float a0 = j0 * w.cv[0], a1 = j1 * w.cv[1] + j2 * w.cv[3], a2 = j2 * w.cv[2] + j1 * w.cv[3];   // (no plain head couples its normal to a tangent)
             if (alone && single) {
 #pragma unroll
                 for (int q = 0; q < N / 4; ++q) add_columns_single<N>(q, w.rows[4 * q], a0, hrow);
