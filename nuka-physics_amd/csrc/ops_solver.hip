@@ -84,15 +84,15 @@ __global__ void __launch_bounds__(1024) OrderTilesKernel(DataView d, uint32_t en
     if (t < 256u) bins[t] = 0u;
     if (t == 0u) top = 0u;
     __syncthreads();
-    const uint32_t mine = first + t * blocks, step = 1024u * blocks;
-    const auto cost_of = [&](uint32_t e) { return by_points ? solve_cost(d.solver_cost[e], d.solver_points[e]) : d.solver_cost[e]; };
-    uint32_t largest = 0u;
-    for (uint32_t e = mine; e < env_count; e += step) largest = max(largest, cost_of(e));
-    largest = wave_max_u(largest);
+    const uint32_t mine = first + t * blocks;   // (no workgroup has more environments than threads)
+    const bool there = mine < env_count;
+    uint32_t cost = 0u;
+    if (there) cost = by_points ? solve_cost(d.solver_cost[mine], d.solver_points[mine]) : d.solver_cost[mine];
+    const uint32_t largest = wave_max_u(cost);
     if ((t & 63u) == 0u) atomicMax(&top, largest);
     __syncthreads();
-    const uint32_t scale = top / 256u + 1u;
-    for (uint32_t e = mine; e < env_count; e += step) atomicAdd(&bins[255u - min(cost_of(e) / scale, 255u)], 1u);
+    const uint32_t level = 255u - min(cost / (top / 256u + 1u), 255u);
+    if (there) atomicAdd(&bins[level], 1u);
     __syncthreads();
     // exclusive prefix of the 256 counts: a scan inside each of the first four wavefronts, then their totals
     __shared__ uint32_t wave_total[4];
@@ -114,7 +114,7 @@ __global__ void __launch_bounds__(1024) OrderTilesKernel(DataView d, uint32_t en
         bins[t] = before + through - count;
     }
     __syncthreads();
-    for (uint32_t e = mine; e < env_count; e += step) d.tile_order[atomicAdd(&bins[255u - min(cost_of(e) / scale, 255u)], 1u) * blocks + first] = e;
+    if (there) d.tile_order[atomicAdd(&bins[level], 1u) * blocks + first] = mine;
 }
 
 
