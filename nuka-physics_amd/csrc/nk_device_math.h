@@ -37,8 +37,8 @@ __device__ __forceinline__ V3 cross3(V3 a, V3 b) {
 // give the bits of sqrtf and a / b whenever |x|, |a|, |b| and the result lie between 2^-90 and 2^90 (compared on the
 // device over 5e8 random operands each); outside that range they stay within an ulp while divisor and result are normal
 // numbers and the divisor is below 2^126.  A larger divisor's reciprocal, no normal number, counts as zero and so does the
-// quotient; a divisor that is infinite, subnormal or zero, or an infinite dividend, gives NaN (rsqrt_exact says what it does
-// about that).
+// quotient; a divisor that is infinite, subnormal or zero, or an infinite dividend, gives NaN (quotient_by is for callers that
+// may meet those).
 __device__ __forceinline__ float sqrt_rn_normal(float x) {
     const float s = __builtin_amdgcn_sqrtf(x);
     const float down = __uint_as_float(__float_as_uint(s) - 1u), up = __uint_as_float(__float_as_uint(s) + 1u);
@@ -62,8 +62,8 @@ __device__ __forceinline__ float div_by(float a, Recip d) {
     return fmaf(e, d.value, q);
 }
 
-// The same with the division's own last instruction, which gives what the division gives for a divisor or a dividend that is zero,
-// infinite or NaN
+// div_by with the division's own last instruction, which gives what the division gives for a divisor or a dividend that is zero,
+// infinite or NaN.  (A subnormal divisor's reciprocal is none: a caller that may have one takes its exponent off first.)
 __device__ __forceinline__ float quotient_by(float a, Recip d) { return __builtin_amdgcn_div_fixupf(div_by(a, d), d.divisor, a); }
 
 // Full-precision reciprocal square root: v_rsq_f32 alone is 1 ulp-approximate, sqrt then divide is exact-rounded.  The bits of

@@ -246,12 +246,13 @@ static SolverKernel KernelOfWidth(const ModelView& m, Heads heads, uint32_t widt
 }
 // Worlds whose environments are solved four a wavefront (ops_solver_packed.hip): contact heads only, no more of them and no
 // more coordinates than a row of sixteen lanes takes.  From a batch on that has wavefronts enough that way: a wavefront
-// of four takes longer than any of them alone, and 2048 free boxes step in 259 us one a wavefront, 324 packed (8192 345
-// and 339).  Sixteen heads take 24.8 KB of LDS a wavefront, six of them a compute unit, where four take 10.5 KB and the registers
-// allow twelve: a body of eight coordinates on sixteen points still gains from 8192 on (732 -> 635 us; 1292 -> 1078 at 16384), its
-// sweeps are long.  A free body's four points under the pyramidal cone, sixteen heads of short sweeps, gain from half as many again:
-// 8192 boxes 271 and 290, 9216 289 and 302, 10240 302 and 312, 11264 322 and 298, 12288 339 and 321, 16384 411 and 363.  With eight
-// heads or fewer, or on a tree, that cone gains from 8192 on too (capsules 223 and 223, four-point trees 243 and 236).
+// of four takes longer than any of them alone: 4096 free boxes step in 269 us one a wavefront and 295 packed, 8192 in 336
+// and 339 (374 and 364 where every state is new), 16384 in 526 and 418.
+//   Sixteen heads take 24.8 KB of LDS a wavefront, six of them a compute unit, where four take 10.5 KB and the registers allow
+// twelve: a body of eight coordinates on sixteen points still gains from 8192 on (732 -> 635 us; 1292 -> 1078 at 16384), its sweeps
+// are long.  A free body's four points under the pyramidal cone, sixteen heads of short sweeps, gain from half as many again:
+// 8192 boxes 271 and 290, 9216 289 and 302, 10240 302 and 312, 11264 322 and 298, 12288 339 and 321, 16384 411 and 363.  With
+// eight heads or fewer, or on a tree, that cone gains from 8192 on too (capsules 223 and 223, four-point trees 243 and 236).
 constexpr uint32_t kPackedBatch = 8192u, kPackedEdgesBatch = kPackedBatch + kPackedBatch / 2u;
 static bool PackedSolverTakes(const ModelView& m, Heads heads, uint32_t staged, uint32_t env_count) {
     const bool edges = m.free_body != 0u && HeadsAPoint(m) != 1u && staged > 8u;
@@ -259,7 +260,7 @@ static bool PackedSolverTakes(const ModelView& m, Heads heads, uint32_t staged, 
         env_count >= (edges ? kPackedEdgesBatch : kPackedBatch);
 }
 // Environments that have a wavefront to themselves, the costliest: one a compute unit until the others' wavefronts take
-// longer than they do (16384 free boxes 429 us without them, 392 with; 65536 981 and 989).
+// longer than they do (12288 free boxes 395 us without them, 368 with, 16384 444 and 418, 24576 475 and 477, 65536 976 and 989).
 static uint32_t PackedAlone(uint32_t env_count) { return env_count < 3u * kPackedBatch ? uint32_t(kUnits) : 0u; }
 static size_t PackedLdsBytes(uint32_t staged) { return size_t{kPackedEnvs} * PackedEnvFloats(staged) * sizeof(float); }
 // Blocks (one wavefront each, one environment or four) of a world's full-capacity solve launch that a compute unit holds at

@@ -30,8 +30,9 @@ namespace solver {
 // This header compiles two ways.  Plainly, a block of up to kTwoWaveWidth coordinates runs two waves a SIMD with up to 256
 // registers each.  With NKH_SOLVER_DENSE defined (ops_solver_d*.hip) everything below sits in namespace `dense` and a block
 // of up to twenty coordinates is compiled for three waves a SIMD, of up to eight for four (DenseWavesPerSimd): 168 or 128
-// registers, a few dozen values a lane in scratch memory at some widths, the same arithmetic.  A long environment runs a tenth slower that way and a full machine gets a tenth
-// more done, so the launcher takes the dense kernels for batches that fill the machine several times over.
+// registers, up to fifteen values a lane in scratch memory at some widths (60 bytes at 36/20 and 40/20, 28 at 28/16 and 32/16, 12 at 20),
+// the same arithmetic.  A long environment runs a tenth slower that way and a full machine gets a tenth more done, so the
+// launcher takes the dense kernels for batches that fill the machine several times over.
 #ifdef NKH_SOLVER_DENSE
 namespace dense {
 #endif
@@ -44,7 +45,8 @@ constexpr int kWave = 64;
 constexpr int kTwoWaveWidth = NKH_TWO_WAVE_WIDTH;
 // Waves per SIMD of the dense build at widths it is instantiated at: four where 128 registers hold the block without
 // scratch memory (eight coordinates need 126, twelve spill 12 bytes a lane), else three.  A step of 16384 free boxes
-// (six coordinates) 642 -> 588 us, of 65536 2128 -> 1904 us, with a fourth wave.
+// (six coordinates) 642 -> 588 us, of 65536 2128 -> 1904 us, with a fourth wave, while batches of that size took these
+// kernels; blocks of up to eight coordinates take them from 6144 to 8191 environments now, or with more than sixteen heads.
 constexpr int DenseWavesPerSimd(int width) { return width <= 8 ? 4 : width <= 20 ? 3 : 0; }
 #ifdef NKH_SOLVER_DENSE
 constexpr int WavesPerSimd(int width) { return DenseWavesPerSimd(width) != 0 ? DenseWavesPerSimd(width) : (width <= kTwoWaveWidth ? 2 : 1); }
@@ -68,8 +70,9 @@ constexpr uint32_t kPackedHeads = 16u, kPackedEnvs = 4u;
 constexpr int kPackedWaves = 3;   // a SIMD
 // Orders the block's LDS words between its lanes.  A block is one wavefront, whose LDS accesses are taken in order, so nothing
 // has to be waited for; a barrier of the workgroup waits for the writes all the same, some twenty times a Newton step (333
-// humanoids 567 -> 557 us, 4096 743 -> 732, 65536 7758 -> 7678).  A wide block keeps the barrier: without it reads move
-// up past it into registers the block does not have (8192 ropes 12.70 -> 12.86 ms).
+// humanoids 567 -> 557 us, 4096 743 -> 732, 65536 7758 -> 7678).  A wide block keeps the barrier where matrix rows are read
+// behind it: without it those reads move up past it into registers the block does not have (8192 ropes 12.70 -> 12.86 ms).  Where a
+// loop over heads has written their fields (apply_moves, update_duals) the fence is taken at every width.
 template <int N>
 __device__ __forceinline__ void lds_sync() {
     if constexpr (N > kTwoWaveWidth) __syncthreads();
