@@ -565,8 +565,8 @@ typedef struct nuka_world_info_t {
     uint32_t solver_width;
     /* one-wavefront blocks of the contact solve's full-capacity launch that a compute unit (four SIMDs) holds at once,
      * by the runtime's occupancy query for that kernel and its LDS (a world of 6144 environments or more takes the
-     * kernels built for three waves a SIMD where there is one for its width: 12 instead of 8); 0 for a world without
-     * a contact solve */
+     * kernels built for three waves a SIMD where there is one for its width: 12 instead of 8; one of small blocks puts four
+     * environments into a wavefront from 8192 on); 0 for a world without a contact solve */
     uint32_t solver_blocks_per_cu;
 } nuka_world_info_t;
 nuka_result_t nuka_world_get_info(nuka_world_handle world, nuka_world_info_t* out);

@@ -13,10 +13,12 @@
 // The arithmetic is that of the narrow block (BlockDescentTileKernel<8, true>) operation for operation, sums in the same
 // order, so an environment of up to four heads ends with the same bits; with more of them, of which some contribute
 // nothing, the other kernel's passes take them in another grouping.
-//   Bound by vector issue (22 k instructions a wavefront of four free boxes, where one takes 12.4 k in the other kernel) and,
-// below 32768 boxes, by the longest wavefronts: the four of one do not take their line searches and sweeps alike, which is
-// why the costliest go alone (PackedAlone).  A step of 8192 free boxes 342 -> 339 us, 16384 537 -> 392, 32768 924 -> 558,
-// 65536 1725 -> 981.  Four waves a SIMD, the rest in scratch memory: 16384 527, 65536 1250; two: 439 and 1145.
+//   Bound by vector issue (20 k instructions a wavefront of 16384 free boxes, of which 256 go alone, where one environment takes
+// 12.4 k in the other kernel) and, below 32768 boxes, by the longest wavefronts: the four of one do not take their line searches
+// and sweeps alike, which is why the costliest go alone (PackedAlone).  A step of 8192 free boxes in the other kernel and so 336 and
+// 339 us (374 and 364 where every state is new), 16384 526 and 418, 32768 915 and 564, 65536 1678 and 979.  Three waves a SIMD, 60
+// bytes a lane in scratch memory; with four and the rest in scratch memory 16384 527 and 65536 1250, with two 439 and 1145, where
+// three took 392 and 981.
 // Replaces what ops_solver_kernel.h replaces (block_descent_tile.cuh), whose line numbers stand there.
 #include "ops_solver_kernel.h"
 
