@@ -11,8 +11,10 @@
 // order (sorted by cost) makes much alike.
 //
 // The arithmetic is that of the narrow block (BlockDescentTileKernel<8, true>) operation for operation, sums in the same
-// order, so an environment of up to four heads ends with the same bits; with more of them, of which some contribute
-// nothing, the other kernel's passes take them in another grouping.
+// order, but for where a head stands in the four partial sums of a force: the other kernel places the heads that contribute one
+// behind the other, this one every head by its number.  An environment of up to four heads ends with the same bits unless three of
+// them contribute and one of the first two does not; then, and with more heads, the last place of a force may differ (in 24 steps of
+// 9001 boxes coming to rest one velocity did, by one).
 //   Bound by vector issue (20 k instructions a wavefront of 16384 free boxes, of which 256 go alone, where one environment takes
 // 12.4 k in the other kernel) and, below 32768 boxes, by the longest wavefronts: the four of one do not take their line searches
 // and sweeps alike, which is why the costliest go alone (PackedAlone).  A step of 8192 free boxes in the other kernel and so 336 and

@@ -52,7 +52,7 @@ def test_free_boxes_four_a_wavefront(device, count, law):
         assert (world.download("contact_count") > 0).mean() >= 0.4
         world.close()
     for name, value in after[E].items():
-        if law == "native" or value.dtype != np.float32:   # four heads: the same bits
+        if law == "native" or value.dtype != np.float32:   # four heads, none of these states groups their sums otherwise: the same bits
             assert np.array_equal(value, after[count][name]), name
         else:   # the same sums in another grouping; three steps
             assert per_env_error(value, after[count][name], E, floor=1e-2).max() <= 3e-4, name
