@@ -1061,6 +1061,8 @@ __global__ void __launch_bounds__(3 * kWave) ArticulationDynamicsKernel(ModelVie
     step_tail_of_block<G>(m, d, t, env_count, lds);
 }
 
+#include "ops_chain_kernel.h"
+
 // The instantiation for `lanes` lanes an environment and the number of its workgroups
 #define NKH_LAUNCH_LANES(lanes, kernel, envs, threads, lds_words_an_env, stream, ...)                                                          \
     do {                                                                                                                                       \
@@ -1182,6 +1184,11 @@ Status OpPosesAndDynamics(const ModelView& m, const DataView& d, const Articulat
     const DynamicsEntry* entry = DynamicsEntryOf(m, *dynamics);
     return entry == nullptr ? Status::InvalidArgument : LaunchDynamics(m, d, *dynamics, *entry, true, StepTail{}, stream);
 }
+// Serial chains go a lane an environment (ChainStepKernel): as many depths as links, parents ahead of their children (the cook
+// refuses others), is link l on link l - 1; no floating base.
+static bool ChainServed(const ModelView& m, const ArticulationDynamicsParams& dynamics) {
+    return m.links_per_env <= kChainLinks && m.max_depth + 1u == m.links_per_env && m.floating_root == 0u && m.max_dof <= kChainLinks && dynamics.articulation_count >= kChainFrom;
+}
 // The step's tail in the dynamics' launch, up to five workgroups a compute unit: past that the shorter kernels fill the chip
 // better than one whose workgroups hold the dynamics' LDS to the end (a step of 64 arms 32.8 -> 30.6 us, 1000 37.8 -> 35.4, 8000
 // in 1000 workgroups 51.0 -> 46.7, 12000 67.2 -> 67.5, 20011 86 -> 88, 65536 223 -> 234).
@@ -1191,6 +1198,7 @@ bool StepServed(const ModelView& m, const ArticulationDynamicsParams& dynamics, 
     StepTail tail;
     const DynamicsEntry* entry = DynamicsEntryOf(m, dynamics);
     if (entry == nullptr || !StepTailOf(m, integrate, poses, twists, bodies, &tail) || poses->articulation_count != dynamics.articulation_count) return false;
+    if (ChainServed(m, dynamics)) return true;
     return uint64_t{dynamics.articulation_count} * entry->lanes <= uint64_t{kTailWorkgroups} * kWave;
 }
 Status OpStep(const ModelView& m, const DataView& d, const ArticulationDynamicsParams* dynamics, const IntegratePositionParams* integrate,
@@ -1198,6 +1206,11 @@ Status OpStep(const ModelView& m, const DataView& d, const ArticulationDynamicsP
     const DynamicsEntry* entry = DynamicsEntryOf(m, *dynamics);
     StepTail tail;
     if (entry == nullptr || !StepTailOf(m, integrate, poses, twists, bodies, &tail)) return Status::InvalidArgument;
+    if (ChainServed(m, *dynamics)) {
+        hipLaunchKernelGGL(ChainStepKernel, dim3((dynamics->articulation_count + kWave - 1u) / kWave), dim3(kChainWaves * kWave), ChainLdsWords(m.links_per_env, m.max_dof) * sizeof(float), stream, m, d,
+                           *dynamics, dynamics->articulation_count, tail);
+        return hipGetLastError() == hipSuccess ? Status::Ok : Status::Failed;
+    }
     return LaunchDynamics(m, d, *dynamics, *entry, true, tail, stream);
 }
 
@@ -1433,6 +1446,8 @@ void InitArticulationKernels() {
         (void)hipFuncSetAttribute(reinterpret_cast<const void*>(entry.kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
         (void)hipGetLastError();
     }
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(ChainStepKernel), hipFuncAttributeMaxDynamicSharedMemorySize, int(ChainLdsWords(kChainLinks, kChainLinks) * sizeof(float)));
+    (void)hipGetLastError();
 }
 
 // ApplyAffineDriveKernel (articulation.cu:836-940): one thread per link turns the controller fields into an affine

@@ -1,0 +1,71 @@
+"""Serial chains of up to eight links without rows, a lane an environment: a step against the general kernels' ops and, with
+them, against the double-precision oracle."""
+import numpy as np
+import pytest
+
+from conftest import nk, relative_error
+
+abi = nk.abi
+pytestmark = pytest.mark.gpu
+FIELDS = ("m", "m_factor", "articulation_bias", "articulation_qdd", "qdot", "qddot", "q", "link_velocity", "link_acceleration", "link_pose", "body_pose")
+OPS = ("FkWorldPoses", "ApplyDrives", "ArticulationDynamics", "IntegrateVelocity", "IntegratePosition", "FkWorldPoses", "FkLinkVelocities", "SyncLinkBodyPose")
+
+
+def chain(links, kinds, g):
+    """`links` links one on the other, the joints' types in turn `kinds`; frames, axes and inertias in general position."""
+    t = abi.Template()
+    for k in range(links):
+        rotation = g.normal(size=4)
+        kind = kinds[k % len(kinds)]
+        t.add_link(kind, k - 1 if k else None, axis=tuple(g.normal(size=3)), local_pos=tuple(g.normal(0.0, 0.15, 3)), local_rot=tuple(rotation / np.linalg.norm(rotation)),
+                   mass=g.uniform(0.2, 2.0), diag_inertia=tuple(g.uniform(2e-3, 2e-2, 3)), com=tuple(g.normal(0.0, 0.05, 3)), damping=0.1, armature=0.02,
+                   stiffness=0.5)
+    for link in range(links):
+        t.add_body(abi.ROLE_LINK_BODY, link=link, kind=abi.SHAPE_NONE, contype=0, conaffinity=0)
+    return t
+
+
+R, P, F = abi.JOINT_REVOLUTE, abi.JOINT_PRISMATIC, abi.JOINT_FIXED
+
+
+@pytest.mark.parametrize("links,kinds", [(1, (R,)), (1, (P,)), (2, (F, R)), (5, (P, R)), (7, (R, P, F)), (8, (F, R, R, R, R, R, R, R)), (8, (R,)), (8, (R, F, P))])
+@pytest.mark.parametrize("E,wrench", [(64, True), (65, False), (333, True)])
+def test_a_chain_steps_like_the_ops_and_as_near_the_double_step(oracle_py, device, links, kinds, E, wrench):
+    """Two steps.  A field of the one-lane walk is within single precision's rounding over eight links of the general kernels' (they
+    differ in fused products and the order of sums: 1e-5 of the field's norm, ten times what is seen), and no further than 1.5 times
+    as far from the double-precision step, or under 5e-7 of the norm, where single values' last places decide."""
+    g = np.random.default_rng(10 * links + len(kinds))
+    t = chain(links, kinds, g)
+    jointed = np.array([link["joint_type"] != F for link in t.links])
+    state = {name: (g.normal(0.0, sigma, (E, links)) * jointed).astype(np.float32) for name, sigma in (("q", 1.0), ("qdot", 1.0), ("tau", 2.0))}
+    base = np.zeros((E, 7), np.float32)
+    base[:, 3] = 1.0
+    state.update(base_pose=base, root_twist=np.zeros((E, 6), np.float32))
+    pushes = g.normal(0.0, 1.0, (E, links, 6)).astype(np.float32) * (g.random((E, links, 1)) < 0.2)
+    desc = abi.world_desc(E, 1.0 / 240.0)
+    worlds = [nk.World(device, t, desc), nk.World(device, t, desc), oracle_py.OracleWorld(t, desc, threads=4, double=True)]
+    out = []
+    for kind, w in zip(("ops", "step", "double"), worlds):
+        w.set_state(state)
+        for _ in range(2):
+            if wrench:
+                w.upload("link_wrench", pushes)
+            if kind == "ops":
+                for op in OPS:
+                    w.op(op)
+            else:
+                w.step()
+        if kind != "double":
+            w.synchronize()
+        if kind == "step":
+            assert not np.any(w.download("link_wrench"))
+        out.append({name: w.download(name).astype(np.float64).reshape(E, -1) for name in FIELDS if kind != "double" or name not in ("m_factor", "body_pose")})
+        w.close()
+    ops, step, double = out
+    assert np.abs(ops["articulation_qdd"]).max() > 0.1 and np.isfinite(step["link_pose"]).all()
+    for name in FIELDS:
+        assert relative_error(step[name], ops[name]) <= 1e-5, (name, relative_error(step[name], ops[name]))
+        if name in double:
+            scale = np.linalg.norm(double[name]) + 1e-30
+            mine, general = np.linalg.norm(step[name] - double[name]) / scale, np.linalg.norm(ops[name] - double[name]) / scale
+            assert mine <= max(1.5 * general, 5e-7), (name, mine, general)
