@@ -88,10 +88,8 @@ constexpr float kPenaltyConditionCap = 1.0e2f;   // block_descent.cu:71
 constexpr uint32_t kUnitSlots = 6u;
 // contributing heads from which a wide block takes the heads' curvature by way of the links (add_heads_through_links)
 constexpr uint32_t kLinkHeads = 4u;
-// words a head of Tile::wrench: 3 x 6 wrench components, the two words of its way to the root, one more for an odd stride
-constexpr uint32_t kWrenchStride = 21u;
-// words a component of Tile::motions: sixteen-byte words, the components of four lanes in different banks
-constexpr uint32_t kMotionStride = 68u;
+// words a head of Tile::wrench: 3 x 6 wrench components, one more for an odd stride
+constexpr uint32_t kWrenchStride = 19u;
 
 // Phase timers for development builds (-DNKH_SOLVER_PROFILE): cycles per phase and event counts per environment,
 // written over the environment's solver_penalty words at the end of the solve.
@@ -390,7 +388,7 @@ struct Tile {
     bool failed;
     // what add_heads_through_links needs (wide blocks only)
     bool from_links;          // the block keeps no contact rows: their entries follow from `wrench` and `axes` wherever a row is read
-    float* wrench;            // cap x kWrenchStride: a head's three rows as wrenches about `pivot`, then its way to the root (two words)
+    float* wrench;            // cap x kWrenchStride: a head's three rows as wrenches about `pivot` (its way to the root takes the words of its column mask)
     bool through_links;       // every staged head acts on the block through one link: the heads' curvature may go by way of the links
     float* axes;              // 64 x 12: a coordinate's motion axis about `pivot`, then the contact stiffness it carries times that axis
     uint32_t path_low, path_high;     // lane = coordinate: the coordinates on the way from its link to the root, itself included
@@ -398,8 +396,6 @@ struct Tile {
     uint32_t over_low, over_high;     // the heads whose way to the root passes through lane's coordinate
     bool over_runs;                   // those are neighbours in the list of heads, for every coordinate (a chain, or limbs in turn)
     bool way_runs;                    // and every head's way to the root is a run of coordinates (a chain)
-    float* spread;            // from_links: 8 x 68 words, what the lanes hand each other as heads and take as coordinates
-    float* motions;           // from_links: 8 x 68 words, the coordinates' motion axes once more, component by component (two of them idle)
     mutable bool stiffness_current;   // no head's curvature has changed since the stiffness in `axes` was summed
     V3 pivot;                 // the point the axes and the heads' wrenches are taken about: the root link's origin
     const float* rows;        // the environment-major row records and row points of device memory
@@ -1446,6 +1442,26 @@ struct LaneRun {   // the lanes of a mask that are one run
     }
 };
 
+// What lanes of coordinates and lanes of heads hand each other on the matrix cores, without a word through LDS.
+// v_mfma_f32_4x4x1 takes the four lanes of block q for every block's left side (cbsz 4, abid q).  Where those four
+// lanes hold one value each - the motion axes of four coordinates - their registers serve as they are.  Where a lane holds four
+// values that belong side by side - four components of one head - each four lanes transpose theirs first: four products with
+// unit vectors, exact.  (Through LDS, a table a use, a wait a group of columns and 4.9 KB a block: a step of 8192 ropes
+// 12.49 ms, as it is 12.28, bit for bit.)
+struct FourUnits {
+    float one[4];   // one[k]: one in the lanes of place k among their four, else zero
+    __device__ __forceinline__ explicit FourUnits(uint32_t lane) {
+#pragma unroll
+        for (uint32_t k = 0u; k < 4u; ++k) one[k] = (lane & 3u) == k ? 1.0f : 0.0f;
+    }
+    // entry t of a lane of place k: v[k] of its four's lane of place t
+    __device__ __forceinline__ Vec4 transposed(const float (&v)[4]) const {
+        Vec4 out = {};
+#pragma unroll
+        for (uint32_t k = 0u; k < 4u; ++k) out = __builtin_amdgcn_mfma_f32_4x4x1f32(v[k], one[k], out, 0, 0, 0);
+        return out;
+    }
+};
 // Blocks that keep no contact rows (Tile::from_links).  Entry j of a head's row is s_j . w where j lies on the head's
 // way to the root, s_j the coordinate's motion axis (Tile::axes) and w the row's wrench (Tile::wrench); elsewhere zero.
 // lane = head: the motion of the head's link, sum over the coordinates j on its way of s_j x_j, for a vector x in LDS.
@@ -1462,9 +1478,8 @@ __device__ __forceinline__ void link_motion(const Tile& c, uint64_t way, const f
         return;
     }
     // Every lane of the wavefront, those without a head with a way of none: v_mfma_f32_4x4x1 takes a coordinate's axis, a
-    // component a lane of four, against the lane's own weight, and register r of a lane is the sum of component r - the
-    // multiply-adds that six vector instructions and two sixteen-byte reads a coordinate made before, bit for bit.
-    const Vec4* words = reinterpret_cast<const Vec4*>(c.motions + (c.lane & 3u) * kMotionStride);
+    // component a lane of four, against the lane's own weight, and register r of a lane is the sum of component r.
+    const float* words = c.axes + (c.lane & 3u);
     const Vec4* x4 = reinterpret_cast<const Vec4*>(x);
     const uint32_t on_low = uint32_t(way), on_high = uint32_t(way >> 32u);
     Vec4 low = {}, high = {};
@@ -1472,13 +1487,13 @@ __device__ __forceinline__ void link_motion(const Tile& c, uint64_t way, const f
     // block does not have
 #pragma unroll 2
     for (uint32_t q = 0u; q < uint32_t(N / 4); ++q) {
-        const Vec4 xs = x4[q], first = words[q], last = words[kMotionStride + q];
+        const Vec4 xs = x4[q];
         const uint32_t four = q < 8u ? on_low >> (4u * q) : on_high >> (4u * q - 32u);
 #pragma unroll
         for (uint32_t t = 0u; t < 4u; ++t) {
             const float on = kept_if(four, t, xs[t]);
-            low = __builtin_amdgcn_mfma_f32_4x4x1f32(first[t], on, low, 0, 0, 0);
-            high = __builtin_amdgcn_mfma_f32_4x4x1f32(last[t], on, high, 0, 0, 0);   // (and two components nobody reads)
+            low = __builtin_amdgcn_mfma_f32_4x4x1f32(words[12u * (4u * q + t)], on, low, 0, 0, 0);
+            high = __builtin_amdgcn_mfma_f32_4x4x1f32(words[12u * (4u * q + t) + 4u], on, high, 0, 0, 0);   // (and two components nobody reads)
         }
     }
     motion[0] = low[0]; motion[1] = low[1]; motion[2] = low[2]; motion[3] = low[3]; motion[4] = high[0]; motion[5] = high[1];
@@ -1489,43 +1504,37 @@ __device__ __forceinline__ float wrench_dot(const Tile& c, uint32_t h, uint32_t 
     return fmaf(w[5], motion[5], fmaf(w[4], motion[4], fmaf(w[3], motion[3], fmaf(w[2], motion[2], fmaf(w[1], motion[1], w[0] * motion[0])))));
 }
 __device__ __forceinline__ uint64_t way_of(const Tile& c, uint32_t h) {
-    const uint32_t* w = reinterpret_cast<const uint32_t*>(c.wrench + h * kWrenchStride + 18u);
-    return (uint64_t(w[1]) << 32u) | uint64_t(w[0]);
+    return (uint64_t(c.U(hColumnsHigh, h)) << 32u) | uint64_t(c.U(hColumnsLow, h));
 }
 // lane = head holds 4 kGroups values; lane = coordinate comes back with their sums over the heads of `heads` (a uniform mask of
-// the first 64) whose way holds the coordinate, added to `sum` in head order.  The values go through LDS (`words`,
-// 4 kGroups x (kHeads + 4) of them) kHeads heads at a time, and v_mfma_f32_4x4x1 multiplies a head's four words of a group, a
-// lane of four each, with the coordinates' own ones and zeros: an instruction a head and group, each the four
-// multiply-adds by one or zero it replaces with their lane reads.  The lanes of heads outside `heads` hold zeros.
-template <int kGroups, uint32_t kHeads>
-__device__ __forceinline__ void sums_over_ways(const Tile& c, uint64_t heads, const float (&v)[4 * kGroups], float* words, Vec4 (&sum)[kGroups]) {
-    constexpr uint32_t kStride = kHeads + 4u;   // sixteen-byte words, the four lanes' in different banks
-    const uint32_t end = heads == 0ull ? 0u : uint32_t(64 - __builtin_clzll(heads));
-#pragma unroll 1
-    for (uint32_t first = 0u; first < end; first += kHeads) {
-        const uint32_t at = c.lane - first;
-        if (at < kHeads) {
+// the first 64) whose way holds the coordinate, added to `sum` in head order: an instruction a head and group, a head's four
+// values of a group, a lane of four each, against the coordinates' own ones and zeros.  The lanes of heads outside `heads`
+// hold zeros.
+template <int Q, int kGroups>
+__device__ __forceinline__ void add_over_ways(uint32_t over_low, uint32_t over_high, uint64_t heads, const Vec4 (&words)[kGroups], Vec4 (&sum)[kGroups]) {
+    if constexpr (Q < int(kWave) / 4) {
+        if constexpr (Q % 4 == 0) if ((heads >> (4 * Q)) == 0ull) return;
+        const uint32_t over = Q < 8 ? over_low : over_high;
 #pragma unroll
-            for (uint32_t e = 0u; e < 4u * kGroups; ++e) words[e * kStride + at] = v[e];
+        for (uint32_t t = 0u; t < 4u; ++t) {
+            const float through = kept_if(over, (4u * uint32_t(Q) + t) & 31u, 1.0f);
+#pragma unroll
+            for (uint32_t g = 0u; g < uint32_t(kGroups); ++g) sum[g] = __builtin_amdgcn_mfma_f32_4x4x1f32(words[g][t], through, sum[g], 4, Q, 0);
         }
-        lds_sync<int(kWave)>();
-        const float* mine = words + (c.lane & 3u) * kStride;
-        const uint32_t here = min(end - first, kHeads);
-#pragma unroll 2
-        for (uint32_t h = 0u; h < here; h += 4u) {
-            const uint32_t four = first + h < 32u ? c.over_low >> (first + h) : c.over_high >> (first + h - 32u);
-            Vec4 word[kGroups];
-#pragma unroll
-            for (uint32_t g = 0u; g < uint32_t(kGroups); ++g) word[g] = *reinterpret_cast<const Vec4*>(mine + 4u * g * kStride + h);
-#pragma unroll
-            for (uint32_t t = 0u; t < 4u; ++t) {
-                const float through = kept_if(four, t, 1.0f);
-#pragma unroll
-                for (uint32_t g = 0u; g < uint32_t(kGroups); ++g) sum[g] = __builtin_amdgcn_mfma_f32_4x4x1f32(word[g][t], through, sum[g], 0, 0, 0);
-            }
-        }
-        lds_sync<int(kWave)>();
+        add_over_ways<Q + 1>(over_low, over_high, heads, words, sum);
     }
+}
+template <int kGroups>
+__device__ __forceinline__ void sums_over_ways(const Tile& c, uint64_t heads, const float (&v)[4 * kGroups], Vec4 (&sum)[kGroups]) {
+    const FourUnits units(c.lane);
+    Vec4 words[kGroups];
+#pragma unroll
+    for (uint32_t g = 0u; g < uint32_t(kGroups); ++g) {
+        const float four[4] = {v[4u * g], v[4u * g + 1u], v[4u * g + 2u], v[4u * g + 3u]};
+        words[g] = units.transposed(four);
+    }
+    // (through the barrier so that the sixty-four ones and zeros are made here, not ahead of the sweeps and kept)
+    add_over_ways<0>(opaque_word(c.over_low), opaque_word(c.over_high), heads, words, sum);
 }
 // lane = coordinate: sum over the heads `heads` (a uniform mask of the first 64) of J^T x, x one value an axis held by
 // lane = head, in double: the heads' wrenches weighted by x summed over the heads whose way holds the coordinate, then
@@ -1570,7 +1579,7 @@ __device__ __forceinline__ double rows_transposed_times(const Tile& c, uint64_t 
                 for (int k = 0; k < 6; ++k) carried[k] = fma(through, lane_value_d(wide[k], first + t), carried[k]);
             }
         }
-        if constexpr (kScale) sums_over_ways<2, 64u>(c, heads, bound, c.spread, carried_bound);
+        if constexpr (kScale) sums_over_ways<2>(c, heads, bound, carried_bound);
     }
     const float4* table = reinterpret_cast<const float4*>(c.axes);
     const float4 a = table[3u * lane], b = table[3u * lane + 1u];
@@ -1601,9 +1610,26 @@ __device__ __forceinline__ double rows_transposed_times(const Tile& c, uint64_t 
 // run on the matrix cores with the multiply-adds of the vector form, bit for bit; while no curvature has changed the
 // stiffness of the last assembly, left in the table beside the axes, stands.  A
 // step of 8192 ropes: 22.1 -> 18.5 ms with the sums of rows_transposed_times and link_motion in the same form.
-// heads a pass of the stiffness sums: 24 words a head (21 and padding), within the factor's place
-template <int N>
-constexpr uint32_t kLinkPass = FactorFloats(N) >= 24u * 68u ? 64u : (FactorFloats(N) >= 24u * 36u ? 32u : 16u);
+// columns 4 Q .. on of lane's row: (K_i s_i) . s_j and (K_j s_j) . s_i, each the stiffness-times-axis of the coordinate
+// further from the root first, four columns an instruction and component
+template <int Q, int N>
+__device__ __forceinline__ void add_link_columns(const float (&s)[6], const float (&y)[6], const uint32_t (&path)[2], const uint32_t (&under)[2], float (&hrow)[N]) {
+    if constexpr (Q < N / 4) {
+        Vec4 mine_first = {}, other_first = {};
+#pragma unroll
+        for (int t = 0; t < 6; ++t) {
+            mine_first = __builtin_amdgcn_mfma_f32_4x4x1f32(s[t], y[t], mine_first, 4, Q, 0);
+            other_first = __builtin_amdgcn_mfma_f32_4x4x1f32(y[t], s[t], other_first, 4, Q, 0);
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const uint32_t at = uint32_t(4 * Q + r) & 31u;
+            const uint32_t bits = (bit_spread(path[Q / 8], at) & __float_as_uint(mine_first[r])) | (bit_spread(under[Q / 8], at) & __float_as_uint(other_first[r]));
+            hrow[4 * Q + r] += __uint_as_float(bits);
+        }
+        add_link_columns<Q + 1>(s, y, path, under, hrow);
+    }
+}
 template <int N>
 __device__ __forceinline__ void add_heads_through_links(const Tile& c, bool mine, const float (&mc)[6], float (&hrow)[N]) {
     const uint32_t lane = c.lane;
@@ -1649,11 +1675,9 @@ __device__ __forceinline__ void add_heads_through_links(const Tile& c, bool mine
                 for (int t = r; t < 6; ++t) k[e++] = (w[0][r] * u[0][t] + w[1][r] * u[1][t]) + w[2][r] * u[2][t];
             }
         }
-        // lane = coordinate: the stiffness of every head whose way to the root passes through it.  By way of the factor's
-        // place, which a changed Hessian frees; where the factor still stood it is made again.
-        c.factor_current = false;
+        // lane = coordinate: the stiffness of every head whose way to the root passes through it
         Vec4 carried[6] = {};
-        sums_over_ways<6, kLinkPass<N>>(c, __ballot(mine), k, c.hfac, carried);
+        sums_over_ways<6>(c, __ballot(mine), k, carried);
         const float4 a = table[3u * lane], b = table[3u * lane + 1u];
         const float s[6] = {a.x, a.y, a.z, a.w, b.x, b.y};
         float y[6];
@@ -1673,34 +1697,13 @@ __device__ __forceinline__ void add_heads_through_links(const Tile& c, bool mine
         table[3u * lane + 2u] = float4{y[2], y[3], y[4], y[5]};
         c.stiffness_current = true;
     }
-    lds_sync<N>();
     const float4 la = table[3u * lane], lb = table[3u * lane + 1u], lc = table[3u * lane + 2u];
     const float s[6] = {la.x, la.y, la.z, la.w, lb.x, lb.y}, y[6] = {lb.z, lb.w, lc.x, lc.y, lc.z, lc.w};
     // (through the barrier so that the sixty-four lane masks of each are made here, two instructions a column, instead of
     // ahead of the sweeps and kept in scalar registers the kernel does not have)
     const uint32_t path[2] = {opaque_word(c.path_low), opaque_word(c.path_high)};
     const uint32_t under[2] = {opaque_word(c.under_low) & ~path[0], opaque_word(c.under_high) & ~path[1]};
-#pragma unroll
-    for (int q = 0; q < N / 4; ++q) {
-        // (K_i s_i) . s_j and (K_j s_j) . s_i, each the stiffness-times-axis of the coordinate further from the root first:
-        // four columns an instruction and component, v_mfma_f32_4x4x1 with the columns' words a lane of four each
-        const float4* column = table + 3u * (4u * uint32_t(q) + (lane & 3u));
-        const float4 a = column[0], b = column[1], d = column[2];
-        const float cs[6] = {a.x, a.y, a.z, a.w, b.x, b.y}, cy[6] = {b.z, b.w, d.x, d.y, d.z, d.w};
-        Vec4 mine_first = {}, other_first = {};
-#pragma unroll
-        for (int t = 0; t < 6; ++t) {
-            mine_first = __builtin_amdgcn_mfma_f32_4x4x1f32(cs[t], y[t], mine_first, 0, 0, 0);
-            other_first = __builtin_amdgcn_mfma_f32_4x4x1f32(cy[t], s[t], other_first, 0, 0, 0);
-        }
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const uint32_t at = uint32_t(4 * q + r) & 31u;
-            const uint32_t bits = (bit_spread(path[q / 8], at) & __float_as_uint(mine_first[r])) | (bit_spread(under[q / 8], at) & __float_as_uint(other_first[r]));
-            hrow[4 * q + r] += __uint_as_float(bits);
-        }
-    }
-    lds_sync<N>();
+    add_link_columns<0>(s, y, path, under, hrow);
 }
 
 // AssembleTileBlock (:1507-1618): lane i assembles row i of H = M + sum J^T C J in `hrow` and its force g_i.  The
@@ -2671,14 +2674,12 @@ __host__ __device__ inline bool RowsFromLinks(uint32_t n, bool contacts_only, ui
 __host__ __device__ inline uint32_t RowFloats(uint32_t N, uint32_t staged, bool from_links) {
     return from_links ? (kWrenchStride * staged + 3u) & ~3u : 3u * staged * N;
 }
-// what a block that keeps no contact rows sums over its heads' ways through LDS (Tile::spread), and Tile::motions
-__host__ __device__ inline uint32_t SpreadFloats(bool from_links) { return from_links ? 16u * kMotionStride : 0u; }
 __host__ __device__ inline uint32_t SolverLdsFloats(uint32_t n, uint32_t cap, uint32_t staged, bool from_links = false, bool reduced = false) {
     const uint32_t N = PaddedWidth(n);
     // the per-coordinate unit lists exist only when some head beyond the staged ones can be listed; without joint rows
     // the block keeps the footprint that lets eight of them share a compute unit's LDS
     return FactorRegionFloats(n) + RowFloats(N, staged, from_links) + HeadFieldFloats(cap, staged) + 256u +
-           UnitListFloats(cap, staged) + LinkAxisFloats(n) + SpreadFloats(from_links) + KeptRowFloats(n, reduced);
+           UnitListFloats(cap, staged) + LinkAxisFloats(n) + KeptRowFloats(n, reduced);
 }
 __host__ __device__ inline uint32_t ReducedSolverLdsFloats(uint32_t full, uint32_t reduced, uint32_t cap, uint32_t staged, bool from_links = false) {
     const uint32_t solve = SolverLdsFloats(reduced, cap, staged, from_links, reduced < full), scratch = ReductionScratchFloats(full, reduced);
@@ -2863,8 +2864,6 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
     c.unit_lists = true; c.unit_count = 0u; c.unit_most = 0u; c.staged_end = 0u; c.individual_end = 0u;
     c.through_links = false; c.over_runs = false; c.way_runs = false;
     c.axes = c.vec + 256 + UnitListFloats(cap, staged_cap);   // a wide block's; a narrow one keeps rows here
-    c.spread = c.axes + 12u * uint32_t(kWave);   // a block without contact rows has it, and the next
-    c.motions = c.spread + 8u * kMotionStride;
     c.path_low = c.path_high = c.under_low = c.under_high = c.over_low = c.over_high = 0u;
     c.stiffness_current = false;
     c.rows = d.urows; c.row_point_a = d.row_cj_point; c.row_point_b = d.row_cj_point_b;
@@ -3047,10 +3046,6 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
         table[3u * lane] = float4{axis[0], axis[1], axis[2], axis[3]};
         table[3u * lane + 1u] = float4{axis[4], axis[5], 0.0f, 0.0f};
         table[3u * lane + 2u] = float4{0.0f, 0.0f, 0.0f, 0.0f};
-        if (c.from_links) {
-#pragma unroll
-            for (uint32_t k = 0u; k < 6u; ++k) c.motions[k * kMotionStride + lane] = axis[k];
-        }
         c.path_low = uint32_t(path); c.path_high = uint32_t(path >> 32u);
         uint64_t head_way = 0ull;   // lane = head: the way to the root of the one side that moves
         if (lane < heads) {
@@ -3100,8 +3095,6 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
 #pragma unroll
                     for (int t = 0; t < 6; ++t) record[6u * a + uint32_t(t)] = w[t];
                 }
-                reinterpret_cast<uint32_t*>(record)[18] = uint32_t(head_way);
-                reinterpret_cast<uint32_t*>(record)[19] = uint32_t(head_way >> 32u);
                 c.U(hColumnsLow, lane) = uint32_t(head_way); c.U(hColumnsHigh, lane) = uint32_t(head_way >> 32u);
             }
         }
