@@ -13,9 +13,16 @@ NKH_DECLARE_WIDTH(4) NKH_DECLARE_WIDTH(8) NKH_DECLARE_WIDTH(12) NKH_DECLARE_WIDT
 NKH_DECLARE_WIDTH(28) NKH_DECLARE_WIDTH(32) NKH_DECLARE_WIDTH(36) NKH_DECLARE_WIDTH(40) NKH_DECLARE_WIDTH(44) NKH_DECLARE_WIDTH(48)
 NKH_DECLARE_WIDTH(52) NKH_DECLARE_WIDTH(56) NKH_DECLARE_WIDTH(60) NKH_DECLARE_WIDTH(64)
 #undef NKH_DECLARE_WIDTH
+// with a queue
+#define NKH_DECLARE_QUEUE(N) \
+    extern template __global__ void BlockDescentTileKernel<N, false, N, false, true>(ModelView, DataView, BlockDescentSolveParams, uint32_t, uint32_t, uint32_t, uint32_t);
+NKH_DECLARE_QUEUE(4) NKH_DECLARE_QUEUE(8) NKH_DECLARE_QUEUE(12) NKH_DECLARE_QUEUE(16) NKH_DECLARE_QUEUE(20) NKH_DECLARE_QUEUE(24) NKH_DECLARE_QUEUE(28)
+NKH_DECLARE_QUEUE(32) NKH_DECLARE_QUEUE(36)
+#undef NKH_DECLARE_QUEUE
 // reduced blocks (contact heads only): width N with the sweeps K wide
 #define NKH_DECLARE_REDUCED(N, K) \
-    extern template __global__ void BlockDescentTileKernel<N, true, K>(ModelView, DataView, BlockDescentSolveParams, uint32_t, uint32_t, uint32_t, uint32_t);
+    extern template __global__ void BlockDescentTileKernel<N, true, K>(ModelView, DataView, BlockDescentSolveParams, uint32_t, uint32_t, uint32_t, uint32_t); \
+    extern template __global__ void BlockDescentTileKernel<N, true, K, false, true>(ModelView, DataView, BlockDescentSolveParams, uint32_t, uint32_t, uint32_t, uint32_t);
 NKH_DECLARE_REDUCED(24, 12) NKH_DECLARE_REDUCED(28, 16) NKH_DECLARE_REDUCED(32, 16) NKH_DECLARE_REDUCED(36, 20) NKH_DECLARE_REDUCED(40, 20)
 NKH_DECLARE_REDUCED(44, 24) NKH_DECLARE_REDUCED(48, 24) NKH_DECLARE_REDUCED(52, 28) NKH_DECLARE_REDUCED(56, 28) NKH_DECLARE_REDUCED(60, 32)
 NKH_DECLARE_REDUCED(64, 32)
@@ -31,7 +38,7 @@ NKH_DECLARE_ELLIPTIC(64, 32)
 // The dense build of the same template (ops_solver_kernel.h compiled with NKH_SOLVER_DENSE: three or four waves a SIMD), for the
 // widths it is instantiated at in ops_solver_d*.hip.
 namespace dense {
-template <int N, bool kContactsOnly, int K = N, bool kElliptic = !kContactsOnly>
+template <int N, bool kContactsOnly, int K = N, bool kElliptic = !kContactsOnly, bool kQueue = true>
 __global__ void BlockDescentTileKernel(ModelView, DataView, BlockDescentSolveParams, uint32_t, uint32_t, uint32_t, uint32_t);
 #define NKH_DECLARE_DENSE(N, K) \
     extern template __global__ void BlockDescentTileKernel<N, true, K>(ModelView, DataView, BlockDescentSolveParams, uint32_t, uint32_t, uint32_t, uint32_t);
@@ -39,6 +46,17 @@ NKH_DECLARE_DENSE(4, 4) NKH_DECLARE_DENSE(8, 8) NKH_DECLARE_DENSE(12, 12) NKH_DE
 NKH_DECLARE_DENSE(24, 12) NKH_DECLARE_DENSE(28, 16) NKH_DECLARE_DENSE(32, 16) NKH_DECLARE_DENSE(36, 20) NKH_DECLARE_DENSE(40, 20)
 #undef NKH_DECLARE_DENSE
 }  // namespace dense
+// The paired build (NKH_SOLVER_PAIRED, ops_solver_p*.hip): wide blocks of contact heads without contact rows, two waves a SIMD.
+namespace paired {
+template <int N, bool kContactsOnly, int K = N, bool kElliptic = !kContactsOnly, bool kQueue = false>
+__global__ void BlockDescentTileKernel(ModelView, DataView, BlockDescentSolveParams, uint32_t, uint32_t, uint32_t, uint32_t);
+#define NKH_DECLARE_PAIRED(N) \
+    extern template __global__ void BlockDescentTileKernel<N, true>(ModelView, DataView, BlockDescentSolveParams, uint32_t, uint32_t, uint32_t, uint32_t);
+NKH_DECLARE_PAIRED(40) NKH_DECLARE_PAIRED(44) NKH_DECLARE_PAIRED(48) NKH_DECLARE_PAIRED(52) NKH_DECLARE_PAIRED(56) NKH_DECLARE_PAIRED(60)
+NKH_DECLARE_PAIRED(64)
+#undef NKH_DECLARE_PAIRED
+uint32_t BlockFloats(uint32_t n, uint32_t staged);   // words of LDS
+}  // namespace paired
 __host__ __device__ uint32_t PackedEnvFloats(uint32_t staged);
 __global__ void PackedDescentKernel(ModelView, DataView, BlockDescentSolveParams, uint32_t, uint32_t);
 }  // namespace solver
@@ -84,6 +102,7 @@ __global__ void __launch_bounds__(1024) OrderTilesKernel(DataView d, uint32_t en
     if (t < 256u) bins[t] = 0u;
     if (t == 0u) top = 0u;
     __syncthreads();
+    if (first == 0u && t == 0u && d.solver_queue != nullptr) *d.solver_queue = 0u;   // the next launch's first place
     const uint32_t mine = first + t * blocks;   // (no workgroup has more environments than threads)
     const bool there = mine < env_count;
     uint32_t cost = 0u;
@@ -142,7 +161,7 @@ const SolverKernel kSolverKernels[3][16] = {
      BlockDescentTileKernel<52, true>, BlockDescentTileKernel<56, true>, BlockDescentTileKernel<60, true>, BlockDescentTileKernel<64, true>}};
 // One reduced instantiation per padded width from 24 on: the sweeps run at about half the width.  A world takes it
 // when no contact can reach a coordinate from that width on (ModelView::contact_dof_end).
-struct ReducedKernel { uint32_t width, reduced; SolverKernel kernel; };
+struct ReducedKernel { uint32_t width, reduced; SolverKernel kernel, queue; };   // queue: the instantiation with one, if any
 // Contact heads under the elliptic cone at the full widths 4 to 20; wider ones that are not reduced take the general kernel
 // (the general kernel keeps what joint rows need: 4096 quadrupeds under the cone 363 -> 347 us a step, 16384 1150 -> 1096, 500 245
 // -> 234, the bits the same)
@@ -150,28 +169,28 @@ const SolverKernel kEllipticFull[] = {BlockDescentTileKernel<4, true, 4, true>, 
                                       BlockDescentTileKernel<16, true, 16, true>, BlockDescentTileKernel<20, true, 20, true>};
 constexpr uint32_t kEllipticFullMost = 20u;
 const ReducedKernel kReducedKernels[] = {
-    {24u, 12u, BlockDescentTileKernel<24, true, 12>}, {28u, 16u, BlockDescentTileKernel<28, true, 16>},
-    {32u, 16u, BlockDescentTileKernel<32, true, 16>}, {36u, 20u, BlockDescentTileKernel<36, true, 20>},
-    {40u, 20u, BlockDescentTileKernel<40, true, 20>}, {44u, 24u, BlockDescentTileKernel<44, true, 24>},
-    {48u, 24u, BlockDescentTileKernel<48, true, 24>}, {52u, 28u, BlockDescentTileKernel<52, true, 28>},
-    {56u, 28u, BlockDescentTileKernel<56, true, 28>}, {60u, 32u, BlockDescentTileKernel<60, true, 32>},
-    {64u, 32u, BlockDescentTileKernel<64, true, 32>}};
+    {24u, 12u, BlockDescentTileKernel<24, true, 12>, BlockDescentTileKernel<24, true, 12, false, true>}, {28u, 16u, BlockDescentTileKernel<28, true, 16>, BlockDescentTileKernel<28, true, 16, false, true>},
+    {32u, 16u, BlockDescentTileKernel<32, true, 16>, BlockDescentTileKernel<32, true, 16, false, true>}, {36u, 20u, BlockDescentTileKernel<36, true, 20>, BlockDescentTileKernel<36, true, 20, false, true>},
+    {40u, 20u, BlockDescentTileKernel<40, true, 20>, BlockDescentTileKernel<40, true, 20, false, true>}, {44u, 24u, BlockDescentTileKernel<44, true, 24>, BlockDescentTileKernel<44, true, 24, false, true>},
+    {48u, 24u, BlockDescentTileKernel<48, true, 24>, BlockDescentTileKernel<48, true, 24, false, true>}, {52u, 28u, BlockDescentTileKernel<52, true, 28>, BlockDescentTileKernel<52, true, 28, false, true>},
+    {56u, 28u, BlockDescentTileKernel<56, true, 28>, BlockDescentTileKernel<56, true, 28, false, true>}, {60u, 32u, BlockDescentTileKernel<60, true, 32>, BlockDescentTileKernel<60, true, 32, false, true>},
+    {64u, 32u, BlockDescentTileKernel<64, true, 32>, BlockDescentTileKernel<64, true, 32, false, true>}};
 // the same with the elliptic cone's response: 2048 humanoids under it 493 -> 408 us a step, by the general kernel at the full
 // width before
 const ReducedKernel kEllipticKernels[] = {
-    {24u, 12u, BlockDescentTileKernel<24, true, 12, true>}, {28u, 16u, BlockDescentTileKernel<28, true, 16, true>},
-    {32u, 16u, BlockDescentTileKernel<32, true, 16, true>}, {36u, 20u, BlockDescentTileKernel<36, true, 20, true>},
-    {40u, 20u, BlockDescentTileKernel<40, true, 20, true>}, {44u, 24u, BlockDescentTileKernel<44, true, 24, true>},
-    {48u, 24u, BlockDescentTileKernel<48, true, 24, true>}, {52u, 28u, BlockDescentTileKernel<52, true, 28, true>},
-    {56u, 28u, BlockDescentTileKernel<56, true, 28, true>}, {60u, 32u, BlockDescentTileKernel<60, true, 32, true>},
-    {64u, 32u, BlockDescentTileKernel<64, true, 32, true>}};
+    {24u, 12u, BlockDescentTileKernel<24, true, 12, true>, nullptr}, {28u, 16u, BlockDescentTileKernel<28, true, 16, true>, nullptr},
+    {32u, 16u, BlockDescentTileKernel<32, true, 16, true>, nullptr}, {36u, 20u, BlockDescentTileKernel<36, true, 20, true>, nullptr},
+    {40u, 20u, BlockDescentTileKernel<40, true, 20, true>, nullptr}, {44u, 24u, BlockDescentTileKernel<44, true, 24, true>, nullptr},
+    {48u, 24u, BlockDescentTileKernel<48, true, 24, true>, nullptr}, {52u, 28u, BlockDescentTileKernel<52, true, 28, true>, nullptr},
+    {56u, 28u, BlockDescentTileKernel<56, true, 28, true>, nullptr}, {60u, 32u, BlockDescentTileKernel<60, true, 32, true>, nullptr},
+    {64u, 32u, BlockDescentTileKernel<64, true, 32, true>, nullptr}};
 // The dense kernels: (padded width of the block, width of the sweeps), contact heads only.
 const ReducedKernel kDenseKernels[] = {
-    {4u, 4u, dense::BlockDescentTileKernel<4, true, 4>}, {8u, 8u, dense::BlockDescentTileKernel<8, true, 8>},
-    {12u, 12u, dense::BlockDescentTileKernel<12, true, 12>}, {16u, 16u, dense::BlockDescentTileKernel<16, true, 16>},
-    {20u, 20u, dense::BlockDescentTileKernel<20, true, 20>}, {24u, 12u, dense::BlockDescentTileKernel<24, true, 12>},
-    {28u, 16u, dense::BlockDescentTileKernel<28, true, 16>}, {32u, 16u, dense::BlockDescentTileKernel<32, true, 16>},
-    {36u, 20u, dense::BlockDescentTileKernel<36, true, 20>}, {40u, 20u, dense::BlockDescentTileKernel<40, true, 20>}};
+    {4u, 4u, dense::BlockDescentTileKernel<4, true, 4>, dense::BlockDescentTileKernel<4, true, 4>}, {8u, 8u, dense::BlockDescentTileKernel<8, true, 8>, dense::BlockDescentTileKernel<8, true, 8>},
+    {12u, 12u, dense::BlockDescentTileKernel<12, true, 12>, dense::BlockDescentTileKernel<12, true, 12>}, {16u, 16u, dense::BlockDescentTileKernel<16, true, 16>, dense::BlockDescentTileKernel<16, true, 16>},
+    {20u, 20u, dense::BlockDescentTileKernel<20, true, 20>, dense::BlockDescentTileKernel<20, true, 20>}, {24u, 12u, dense::BlockDescentTileKernel<24, true, 12>, dense::BlockDescentTileKernel<24, true, 12>},
+    {28u, 16u, dense::BlockDescentTileKernel<28, true, 16>, dense::BlockDescentTileKernel<28, true, 16>}, {32u, 16u, dense::BlockDescentTileKernel<32, true, 16>, dense::BlockDescentTileKernel<32, true, 16>},
+    {36u, 20u, dense::BlockDescentTileKernel<36, true, 20>, dense::BlockDescentTileKernel<36, true, 20>}, {40u, 20u, dense::BlockDescentTileKernel<40, true, 20>, dense::BlockDescentTileKernel<40, true, 20>}};
 // Batches from this many environments on take a dense kernel where there is one: twice the 3072 wave slots three waves
 // a SIMD make of 256 compute units.  A dense wave runs slower than a two-wave one (fewer registers, some spilled), so
 // below that the launch is over sooner with the two-wave kernel: its length is then the longest environment's, not the
@@ -181,6 +200,20 @@ const ReducedKernel kDenseKernels[] = {
 #define NKH_DENSE_BATCH 6144
 #endif
 constexpr uint32_t kDenseBatch = NKH_DENSE_BATCH;
+// The general kernels without the elliptic cone that run two waves a SIMD, with a queue.
+const SolverKernel kQueueKernels[] = {BlockDescentTileKernel<4, false, 4, false, true>, BlockDescentTileKernel<8, false, 8, false, true>,
+                                      BlockDescentTileKernel<12, false, 12, false, true>, BlockDescentTileKernel<16, false, 16, false, true>,
+                                      BlockDescentTileKernel<20, false, 20, false, true>, BlockDescentTileKernel<24, false, 24, false, true>,
+                                      BlockDescentTileKernel<28, false, 28, false, true>, BlockDescentTileKernel<32, false, 32, false, true>,
+                                      BlockDescentTileKernel<36, false, 36, false, true>};
+// The paired kernels: the seven padded widths from 40 on.
+const SolverKernel kPairedKernels[] = {paired::BlockDescentTileKernel<40, true>, paired::BlockDescentTileKernel<44, true>, paired::BlockDescentTileKernel<48, true>,
+                                       paired::BlockDescentTileKernel<52, true>, paired::BlockDescentTileKernel<56, true>, paired::BlockDescentTileKernel<60, true>,
+                                       paired::BlockDescentTileKernel<64, true>};
+// Batches from this many environments on take a paired kernel where there is one: as many as it holds at once.  Below, an
+// environment with a SIMD to itself is over sooner (ropes, the plain and the paired kernel: 1024 2.36 and 2.53 ms a step, 1536 2.85
+// and 3.08, 1792 3.03 and 3.10, 2048 3.33 and 3.23, 4096 6.22 and 5.08, 8192 12.22 and 9.90).
+constexpr uint32_t kPairedBatch = 2048u;
 // Compute units, and the rounds of environments over them from which launches of fewer heads pay (OpBlockDescentSolve).
 constexpr size_t kUnits = 256u, kManyRounds = 9u;
 }  // namespace
@@ -208,7 +241,20 @@ void InitSolverKernels() {
         (void)hipFuncSetAttribute(reinterpret_cast<const void*>(dense.kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
         (void)hipGetLastError();
     }
+    for (const ReducedKernel& reduced : kReducedKernels) {
+        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(reduced.queue), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+        (void)hipGetLastError();
+    }
+    for (SolverKernel queue : kQueueKernels) {
+        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(queue), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+        (void)hipGetLastError();
+    }
+    for (SolverKernel paired : kPairedKernels) {
+        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(paired), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+        (void)hipGetLastError();
+    }
 }
+
 
 // The heads a world's solve meets: anything or contact heads only, at most one a lane, either with or without the elliptic cone
 // of the MuJoCo law (contact heads under it take the general kernel at full widths past 20).
@@ -227,22 +273,32 @@ static uint32_t SolverWorkingWidth(const ModelView& m, Heads heads) {
                 reduced.reduced <= m.dof) return reduced.reduced;   // (0: a host that did not say; the full width is always right)
     return m.dof;
 }
-// `dense_out`: whether the kernel is a dense one
-static SolverKernel KernelOfWidth(const ModelView& m, Heads heads, uint32_t width, uint32_t env_count, bool* dense_out = nullptr) {
-    if (dense_out != nullptr) *dense_out = false;
+// The kernel of a world's solve, the same with a queue, where there is one, and how many of its waves share a SIMD
+struct ChosenKernel { SolverKernel kernel, queue; int waves; bool paired; };
+static ChosenKernel KernelOfWidth(const ModelView& m, Heads heads, uint32_t width, uint32_t env_count) {
+    const uint32_t padded = solver::PaddedWidth(m.dof);
+    const int waves = solver::WavesPerSimd(int(solver::PaddedWidth(width)));
     if (heads == kContactHeads && env_count >= kDenseBatch)
         for (const ReducedKernel& dense : kDenseKernels)
-            if (dense.width == solver::PaddedWidth(m.dof) && dense.reduced == solver::PaddedWidth(width) && (width == m.dof || dense.reduced == width)) {
-                if (dense_out != nullptr) *dense_out = true;
-                return dense.kernel;
-            }
+            if (dense.width == padded && dense.reduced == solver::PaddedWidth(width) && (width == m.dof || dense.reduced == width))
+                return {dense.kernel, dense.queue, solver::DenseWavesPerSimd(int(dense.reduced)), false};
+    if (width == m.dof && env_count >= kPairedBatch && solver::RowsFromLinks(width, heads == kContactHeads, m.rows_from_links))
+        return {kPairedKernels[padded / 4u - 10u], nullptr, 2, true};
     if (width != m.dof) {
         static_assert(sizeof(kReducedKernels) == sizeof(kEllipticKernels), "the same pairs of widths");
         for (const ReducedKernel& reduced : heads == kContactElliptic ? kEllipticKernels : kReducedKernels)
-            if (reduced.width == solver::PaddedWidth(m.dof) && reduced.reduced == width) return reduced.kernel;
+            if (reduced.width == padded && reduced.reduced == width) return {reduced.kernel, reduced.queue, waves, false};
     }
-    if (heads == kContactElliptic && solver::PaddedWidth(m.dof) <= kEllipticFullMost) return kEllipticFull[solver::PaddedWidth(m.dof) / 4u - 1u];
-    return kSolverKernels[heads == kContactElliptic ? kAnyElliptic : heads][solver::PaddedWidth(m.dof) / 4u - 1u];
+    if (heads == kContactElliptic && padded <= kEllipticFullMost) return {kEllipticFull[padded / 4u - 1u], nullptr, waves, false};
+    return {kSolverKernels[heads == kContactElliptic ? kAnyElliptic : heads][padded / 4u - 1u],
+            heads == kAnyHeads && padded <= uint32_t(solver::kTwoWaveWidth) ? kQueueKernels[padded / 4u - 1u] : nullptr, waves, false};
+}
+// LDS of a block of that kernel with room for so many contact heads
+static size_t BlockLdsBytes(const ModelView& m, Heads heads, uint32_t width, const ChosenKernel& chosen, uint32_t staged) {
+    const uint32_t joint_heads = m.joint_limit_rows + m.joint_friction_rows + m.joint_drive_rows;
+    return sizeof(float) * (chosen.paired ? paired::BlockFloats(m.dof, staged)
+                                          : solver::ReducedSolverLdsFloats(m.dof, width, staged + joint_heads, staged,
+                                                                           solver::RowsFromLinks(width, heads == kContactHeads, m.rows_from_links)));
 }
 // Worlds whose environments are solved four a wavefront (ops_solver_packed.hip): contact heads only, no more of them and no
 // more coordinates than a row of sixteen lanes takes.  From a batch on that has wavefronts enough that way: a wavefront
@@ -269,11 +325,8 @@ uint32_t SolverBlocksPerUnit(const ModelView& m, uint32_t env_count) {
     if (m.rows_per_env == 0u || m.dof == 0u) return 0u;
     const uint32_t staged = SolverHeadCapacity(m, std::max(m.contact_slots, 1u));
     if (staged == 0u) return 0u;
-    const uint32_t joint_heads = m.joint_limit_rows + m.joint_friction_rows + m.joint_drive_rows;
     const Heads heads = HeadsOf(m, staged);
     const uint32_t width = SolverWorkingWidth(m, heads);
-    const size_t lds = size_t{solver::ReducedSolverLdsFloats(m.dof, width, staged + joint_heads, staged,
-                                                             solver::RowsFromLinks(width, heads == kContactHeads, m.rows_from_links))} * sizeof(float);
     int blocks = 0;
     if (PackedSolverTakes(m, heads, staged, env_count)) {
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, reinterpret_cast<const void*>(PackedDescentKernel), solver::kWave, PackedLdsBytes(staged)) != hipSuccess) {
@@ -282,8 +335,9 @@ uint32_t SolverBlocksPerUnit(const ModelView& m, uint32_t env_count) {
         }
         return uint32_t(std::max(blocks, 0));
     }
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, reinterpret_cast<const void*>(KernelOfWidth(m, heads, width, env_count)),
-                                                     solver::kWave, lds) != hipSuccess) {
+    const ChosenKernel chosen = KernelOfWidth(m, heads, width, env_count);
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, reinterpret_cast<const void*>(chosen.kernel), solver::kWave,
+                                                     BlockLdsBytes(m, heads, width, chosen, staged)) != hipSuccess) {
         (void)hipGetLastError();
         return 0u;
     }
@@ -292,7 +346,7 @@ uint32_t SolverBlocksPerUnit(const ModelView& m, uint32_t env_count) {
 uint32_t SolverMassFactorFloats(const ModelView& m) {
     if (m.rows_per_env == 0u || m.dof == 0u) return 0u;
     const uint32_t width = SolverSweepWidth(m);
-    return solver::MassFactorInMemory(width) ? solver::FactorFloats(solver::PaddedWidth(width)) : 0u;
+    return solver::MassFactorInMemory(width) ? solver::MassFactorFloats(solver::PaddedWidth(width)) : 0u;
 }
 uint32_t SolverSweepWidth(const ModelView& m) {
     if (m.rows_per_env == 0u || m.dof == 0u) return m.dof;
@@ -311,15 +365,11 @@ Status OpBlockDescentSolve(const ModelView& m, const DataView& d, const void* pa
     const uint32_t joint_heads = m.joint_limit_rows + m.joint_friction_rows + m.joint_drive_rows;
     const Heads heads = HeadsOf(m, staged);
     const uint32_t width = SolverWorkingWidth(m, heads);
-    const auto lds_bytes = [&](uint32_t contact_heads) {
-        return size_t{solver::ReducedSolverLdsFloats(m.dof, width, contact_heads + joint_heads, contact_heads,
-                                                     solver::RowsFromLinks(width, heads == kContactHeads, m.rows_from_links))} * sizeof(float);
-    };
-    bool dense = false;
-    const SolverKernel kernel = KernelOfWidth(m, heads, width, p->env_count, &dense);
+    const ChosenKernel chosen = KernelOfWidth(m, heads, width, p->env_count);
+    const SolverKernel kernel = chosen.kernel;
+    const auto lds_bytes = [&](uint32_t contact_heads) { return BlockLdsBytes(m, heads, width, chosen, contact_heads); };
     // blocks a compute unit holds at most, whatever their LDS: four a wave of a SIMD
-    const int padded = int(solver::PaddedWidth(width));
-    const size_t most_blocks = 4u * size_t(dense ? solver::DenseWavesPerSimd(padded) : solver::WavesPerSimd(padded));
+    const size_t most_blocks = 4u * size_t(chosen.waves);
     const auto blocks_per_unit = [&](uint32_t contact_heads) { return std::min<size_t>(most_blocks, (160u * 1024u) / lds_bytes(contact_heads)); };
     // The LDS a block needs grows with the contact heads it can stage, and a scene's slots (every pair that may ever
     // touch, at its largest manifold) outnumber the contacts an environment usually has.  Where a smaller capacity
@@ -371,8 +421,16 @@ Status OpBlockDescentSolve(const ModelView& m, const DataView& d, const void* pa
             first_points = points + 1u;
         }
     }
-    hipLaunchKernelGGL(kernel, dim3(p->env_count), dim3(solver::kWave), lds_bytes(staged), stream, m, d, *p, staged + joint_heads, staged,
-                       first_points, kInvalid);
+    // One launch of more blocks than the machine holds takes as many as it holds, and a queue (ops_solver_kernel.h).  Steps from the same
+    // state, and from eight states in turn: 4096 humanoids 682 -> 672 and 800 -> 777 us, 65536 7540 -> 7353 and 7620 -> 7320; 4096 servo-driven
+    // ones 1351 -> 1320 and 1551 -> 1508, 16384 4715 -> 4534; 65536 quadrupeds 4547 -> 4459 and 4580 -> 4457.  Blocks of contact heads that are
+    // neither reduced nor dense, and those under the elliptic cone, have no kernel for it (4096 quadrupeds 466 and 466, 531 -> 521 in turn; under
+    // the cone 595 -> 592), and paired blocks lose by it: eight that start together are better there than eight at any
+    // time (8192 ropes 9.87 ms and 10.06).  Nor where the points send environments to several launches, whose blocks are mostly over at once.
+    const size_t held = kUnits * blocks_per_unit(staged);
+    const bool queued = chosen.queue != nullptr && first_points == 0u && d.solver_queue != nullptr && p->env_count > held;
+    hipLaunchKernelGGL(queued ? chosen.queue : kernel, dim3(queued ? uint32_t(held) : p->env_count), dim3(solver::kWave), lds_bytes(staged), stream, m, d, *p, staged + joint_heads,
+                       staged, queued ? uint32_t(held) : first_points, queued ? kQueued : kInvalid);
     return hipGetLastError() == hipSuccess ? Status::Ok : Status::Failed;
 }
 

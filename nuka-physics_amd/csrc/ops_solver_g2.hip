@@ -3,6 +3,7 @@
 namespace nkh {
 namespace solver {
 template __global__ void BlockDescentTileKernel<36, false, 36, false>(ModelView, DataView, BlockDescentSolveParams, uint32_t, uint32_t, uint32_t, uint32_t);
+template __global__ void BlockDescentTileKernel<36, false, 36, false, true>(ModelView, DataView, BlockDescentSolveParams, uint32_t, uint32_t, uint32_t, uint32_t);
 template __global__ void BlockDescentTileKernel<40, false, 40, false>(ModelView, DataView, BlockDescentSolveParams, uint32_t, uint32_t, uint32_t, uint32_t);
 template __global__ void BlockDescentTileKernel<44, false, 44, false>(ModelView, DataView, BlockDescentSolveParams, uint32_t, uint32_t, uint32_t, uint32_t);
 }  // namespace solver

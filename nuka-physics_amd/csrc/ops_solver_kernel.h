@@ -27,14 +27,29 @@
 
 namespace nkh {
 namespace solver {
-// This header compiles two ways.  Plainly, a block of up to kTwoWaveWidth coordinates runs two waves a SIMD with up to 256
+// This header compiles three ways.  Plainly, a block of up to kTwoWaveWidth coordinates runs two waves a SIMD with up to 256
 // registers each.  With NKH_SOLVER_DENSE defined (ops_solver_d*.hip) everything below sits in namespace `dense` and a block
 // of up to twenty coordinates is compiled for three waves a SIMD, of up to eight for four (DenseWavesPerSimd): 168 or 128
-// registers, up to fifteen values a lane in scratch memory at some widths (60 bytes at 36/20 and 40/20, 28 at 28/16 and 32/16, 12 at 20),
+// registers, up to twenty values a lane in scratch memory at some widths (80 bytes at 36/20, 76 at 40/20, 36 at 28/16 and 32/16, 12 at 20 and 24/12),
 // the same arithmetic.  A long environment runs a tenth slower that way and a full machine gets a tenth more done, so the
 // launcher takes the dense kernels for batches that fill the machine several times over.
+//   With NKH_SOLVER_PAIRED defined (ops_solver_p*.hip) it sits in namespace `paired`: wide blocks of contact heads without contact
+// rows (Tile::from_links), two waves a SIMD.  A wide wave alone on its SIMD issues an instruction in less than half of its cycles, whatever
+// it waits for, and what kept a second one away was LDS, 28 KB a block, not registers: 256 hold the sweeps' rows with some
+// eighty values a Newton step in scratch memory.  The build keeps no factor in LDS - the substitution hands its columns round
+// eight at a time (substitute_by_turns) and a Hessian met again is factored again - and no field that such a head has
+// no use for: 20.4 KB, eight blocks a compute unit, and the bits of the plain build (8192 ropes 12.2 -> 9.7 ms a step).
 #ifdef NKH_SOLVER_DENSE
 namespace dense {
+constexpr bool kDense = true;
+#else
+constexpr bool kDense = false;
+#endif
+#ifdef NKH_SOLVER_PAIRED
+namespace paired {
+constexpr bool kPaired = true;
+#else
+constexpr bool kPaired = false;
 #endif
 
 constexpr int kWave = 64;
@@ -51,7 +66,7 @@ constexpr int DenseWavesPerSimd(int width) { return width <= 8 ? 4 : width <= 20
 #ifdef NKH_SOLVER_DENSE
 constexpr int WavesPerSimd(int width) { return DenseWavesPerSimd(width) != 0 ? DenseWavesPerSimd(width) : (width <= kTwoWaveWidth ? 2 : 1); }
 #else
-constexpr int WavesPerSimd(int width) { return width <= kTwoWaveWidth ? 2 : 1; }
+constexpr int WavesPerSimd(int width) { return width <= kTwoWaveWidth || kPaired ? 2 : 1; }
 #endif
 // From this width on a block widens its mass rows to double where it uses them; below it the widened rows are kept over
 // the solve (two registers an entry), which pays while they fit.  In the dense build's 168 registers they never do:
@@ -301,13 +316,15 @@ enum HeadField : uint32_t {
     hSlot,               // the head's row of the environment-major records; kUnowned beside it: the head acts on nothing
     hStride, hAxes, hRho, hCompliance, hLower, hUpper, hMu1, hMu2, hNormalBound,
     hRes, hDual = hRes + 3, hMove = hDual + 3, hStep = hMove + 3, hBase = hStep + 3, hDualScale = hBase + 3, hResidualScale,
-    hRelaxStep, hRelaxWeight = hRelaxStep + 3, hRelaxPoint, hC = hRelaxPoint + 3, hColumnsLow = hC + 6, hColumnsHigh,
+    hRelaxStep, hRelaxWeight = hRelaxStep + 3, hRelaxPoint, hC = hRelaxPoint + 3, hColumnsLow = hC + (kPaired ? 0 : 6), hColumnsHigh,
     hRow,                // first of the head's three staged Jacobian rows; kInvalid for a unit head
     hSecond,             // the side that moves is the row's second
-    hUnit,               // the one coordinate a unit head acts on; kInvalid for a staged head
-    hUnitValue,          // its Jacobian entry there
-    hFieldCount
+    hUnit = hSecond + (kPaired ? 0 : 1),      // the one coordinate a unit head acts on; kInvalid for a staged head
+    hUnitValue = hUnit + (kPaired ? 0 : 1),   // its Jacobian entry there
+    hFieldCount = hUnitValue + 1
 };
+// (paired: a contact head's curvature is in its lane's registers, and no head is a unit head: neither has words, nothing reads or
+// writes them)
 // Fields that share their words: the rows' sources are done with when a head's residual and base are first written, and an
 // assembly's impulses when the next steps are.
 constexpr uint32_t hSourceA = hRes, hSourceB = hBase, hF = hStep;
@@ -343,7 +360,7 @@ __host__ __device__ constexpr uint32_t narrow_below(uint32_t f) {
     return clamped_span(f, hStride, hAxes + 1) + clamped_span(f, hMu1, hNormalBound + 1) +
            clamped_span(f, hRes + 1, hRes + 3) + clamped_span(f, hDual + 1, hDual + 3) + clamped_span(f, hMove + 1, hMove + 3) +
            clamped_span(f, hStep + 1, hStep + 3) + clamped_span(f, hBase + 1, hBase + 3) + clamped_span(f, hRelaxStep, hC) +
-           clamped_span(f, hC + 1, hC + 6) + clamped_span(f, hColumnsLow, hSecond + 1);
+           (kPaired ? 0u : clamped_span(f, hC + 1, hC + 6)) + clamped_span(f, hColumnsLow, hSecond + 1);
 }
 __host__ __device__ constexpr bool narrow_field(uint32_t f) { return narrow_below(f + 1u) != narrow_below(f); }
 constexpr uint32_t kNarrowFields = narrow_below(hFieldCount);
@@ -359,10 +376,10 @@ struct Tile {
     uint32_t n_all;   // n, or past it the coordinates that follow the block's own (a reduced block, described above mass_times)
     float tolerance;
     float* mfac;     // FactorFloats(N) words: Cholesky factor of the mass matrix (rows; columns are read transposed); device memory for a wide block
-    float* hfac;     // FactorFloats(N) words: Cholesky factor of the current Newton Hessian
+    float* hfac;     // FactorFloats(N) words: Cholesky factor of the current Newton Hessian (paired: none)
     float* jac;      // 3 * staged capacity rows x ldj, ldj = N
     float* fields;   // cap x kWideStride, then (narrow + 1) x kNarrowStride
-    float* vec;      // 4 x 64 scratch vectors, 16-byte aligned
+    float* vec;      // 4 x 64 scratch vectors (paired: kTurnFloats words), 16-byte aligned
     float* hrows;    // blocks of at most 32 coordinates: N x N words, the Hessian of the last assembly in full
     float* low;      // a reduced block: N x N words, the second floats of its mass rows
     float mass_inverse;   // 1 / diagonal of the mass factor, lane = row
@@ -593,6 +610,47 @@ __device__ __forceinline__ float substitute_up(uint32_t lane, const float (&row)
     return r * inverse;
 }
 
+// The same from the rows alone: the lanes of eight rows at a time put them into `turn`, where every lane finds its
+// column's eight words, the next eight under way while these are used.  A block's LDS accesses are taken in order: nothing is
+// waited for but the words.  72 writes of sixteen bytes where a stored factor takes 64 of four, and a quarter of its LDS.  Lanes
+// ahead of the eight find what an earlier turn left: their own entries have been taken (`solved`) by then.
+constexpr uint32_t kTurnRows = 8u, kTurnStride = 68u, kTurnFloats = kTurnRows * kTurnStride;   // (the eight rows' words in different banks)
+template <int First, int N>
+__device__ __forceinline__ void take_turn(uint32_t lane, const float (&row)[N], float* turn, float (&u)[kTurnRows]) {
+    if ((lane >> 3u) == uint32_t(First) / kTurnRows) {
+        float4* words = reinterpret_cast<float4*>(turn + (lane & 7u) * kTurnStride);
+#pragma unroll
+        for (int q = First / 4; q < N / 4; ++q) words[q] = float4{row[4 * q], row[4 * q + 1], row[4 * q + 2], row[4 * q + 3]};
+    }
+    wave_sync();
+#pragma unroll
+    for (int t = 0; t < int(kTurnRows); ++t) u[t] = First + t < N ? turn[uint32_t(t) * kTurnStride + lane] : 0.0f;   // U[j][lane], zero up to the diagonal
+    wave_sync();
+}
+template <int First, int N>
+__device__ __forceinline__ void substitute_turns(uint32_t lane, const float (&row)[N], float* turn, float inverse, const float (&u)[kTurnRows], float& r, float& solved) {
+    if constexpr (First < N) {
+        float next[kTurnRows];
+        if constexpr (First + int(kTurnRows) < N) take_turn<First + int(kTurnRows)>(lane, row, turn, next);
+#pragma unroll
+        for (int t = 0; t < int(kTurnRows); ++t)
+            if (First + t < N) r = fmaf(u[t], -lane_value(r * inverse, First + t), r);
+        solved = (lane >> 3u) == uint32_t(First) / kTurnRows ? r * inverse : solved;
+        substitute_turns<First + int(kTurnRows)>(lane, row, turn, inverse, next, r, solved);
+    }
+}
+template <int N>
+__device__ __forceinline__ float substitute_by_turns(uint32_t lane, const float (&row)[N], float* turn, float inverse, float g) {
+    lane = local_lane(lane);
+    float r = g, solved = 0.0f, u[kTurnRows];
+    take_turn<0>(lane, row, turn, u);
+#pragma unroll
+    for (int j = N - 1; j >= 0; --j) r = fmaf(row[j], -lane_value(r * inverse, j), r);
+    r *= inverse;
+    substitute_turns<0>(lane, row, turn, inverse, u, r, solved);
+    return lane < uint32_t(N) ? solved : 0.0f;
+}
+
 // SolveTileBlock (:1647-1666): forward with the factor's rows, backward with its columns (col[j] = L_j,lane), both zero
 // from the diagonal on.
 template <int N>
@@ -642,6 +700,29 @@ __device__ __forceinline__ void load_rows(const float* a, uint32_t lane, float (
 #pragma unroll
     for (int k = 0; k < N; ++k) row[k] = diagonal[max(k - int(from), 0)];
 }
+// A leaves-first factor in device memory four columns at a time, the rows down to the diagonal side by side: words that
+// neighbouring lanes read and write together, sixteen bytes a lane.  (Rows one after the other, packed, are 64 words of 64
+// different lines a lane; with them and the transposed reads the mass solves were a tenth of the solve of 8192 ropes.)
+__host__ __device__ constexpr uint32_t quads_before(uint32_t q) { return 8u * q * (q + 1u); }
+template <int N>
+__device__ __forceinline__ void store_quads(float* a, uint32_t lane, const float (&row)[N]) {
+    lane = local_lane(lane);
+#pragma unroll
+    for (int q = 0; q < N / 4; ++q)
+        if (lane <= 4u * uint32_t(q) + 3u)
+            reinterpret_cast<float4*>(a + quads_before(uint32_t(q)))[lane] = float4{row[4 * q], row[4 * q + 1], row[4 * q + 2], row[4 * q + 3]};
+}
+template <int N>
+__device__ __forceinline__ void load_quads(const float* a, uint32_t lane, float (&row)[N]) {
+    lane = local_lane(lane);
+#pragma unroll
+    for (int q = 0; q < N / 4; ++q) {   // lanes below the diagonal read the last row's words, zeros
+        const float4 w = reinterpret_cast<const float4*>(a + quads_before(uint32_t(q)))[min(lane, 4u * uint32_t(q) + 3u)];
+        row[4 * q] = w.x; row[4 * q + 1] = w.y; row[4 * q + 2] = w.z; row[4 * q + 3] = w.w;
+    }
+}
+// words of device memory an environment's mass factor takes in a wide block, by rows or by fours
+__host__ __device__ constexpr uint32_t MassFactorFloats(uint32_t N) { return FactorFloats(N) > quads_before(N / 4u) ? FactorFloats(N) : quads_before(N / 4u); }
 template <int N>
 __device__ __forceinline__ void load_columns(const float* a, uint32_t lane, float (&col)[N]) {
     lane = local_lane(lane);
@@ -655,6 +736,14 @@ __device__ __forceinline__ void load_columns(const float* a, uint32_t lane, floa
 template <int N, bool kFollow>
 __device__ __forceinline__ bool cholesky_solve(const Tile& c, float (&hrow)[N], float g, float* d_out) {
     float inverse = 0.0f;
+    if constexpr (kPaired) {
+        if (!factor_rows_up<N>(c.lane, hrow, &inverse, &c.factor_root)) return false;
+        if (c.factor_current) inverse = 1.0f / c.factor_root;   // the Hessian is the one factored last: as a kept factor answers
+        c.factor_current = true;
+        *d_out = substitute_by_turns<N>(c.lane, hrow, c.vec, inverse, c.lane < c.n ? g : 0.0f);
+        lds_sync<N>();
+        return true;
+    }
     if (!c.factor_current) {   // otherwise the Hessian is the one factored last: its factor is still in hfac
         PROF_BEGIN(c, 14);
         const bool valid = kLeavesFirst<N> ? factor_rows_up<N>(c.lane, hrow, &inverse, &c.factor_root) : factor_rows<N>(c.lane, hrow, &inverse, &c.factor_root);
@@ -694,13 +783,18 @@ __device__ __forceinline__ bool factor_mass(Tile& c, const float (&mrow)[N]) {
     float inverse = 0.0f, root = 0.0f;
     const bool valid = kLeavesFirst<N> ? factor_rows_up<N>(c.lane, row, &inverse, &root) : factor_rows<N>(c.lane, row, &inverse, &root);
     c.mass_inverse = inverse;
-    store_rows<N>(c.mfac, c.lane, row);
+    if constexpr (kPaired) store_quads<N>(c.mfac, c.lane, row);
+    else store_rows<N>(c.mfac, c.lane, row);
     lds_sync<N>();
     return valid;
 }
 template <int N>
 __device__ __forceinline__ float solve_tile_mass(const Tile& c, float force) {
     float row[N];
+    if constexpr (kPaired) {
+        load_quads<N>(c.mfac, c.lane, row);
+        return substitute_by_turns<N>(c.lane, row, c.vec, c.mass_inverse, c.lane < c.n ? force : 0.0f);
+    }
     load_rows<N>(c.mfac, c.lane, row);
     if constexpr (kLeavesFirst<N>) return substitute_up<N>(c.lane, row, c.mfac, c.mass_inverse, c.lane < c.n ? force : 0.0f);
     float col[N];
@@ -2459,7 +2553,7 @@ __device__ __forceinline__ void initialize_residuals(const Tile& c, float veloci
     }
     for (uint32_t h = c.lane; h < c.heads; h += kWave) {
         const uint32_t slot = c.slot(h), stride = c.U(hStride, h), axes = c.U(hAxes, h);
-        const uint32_t unit = c.U(hUnit, h), first = c.U(hRow, h);
+        const uint32_t unit = kPaired ? kInvalid : c.U(hUnit, h), first = c.U(hRow, h);
         if (unit != kInvalid || first == kInvalid) {   // one coordinate (or none): every other product is an exact zero
             const float along = unit != kInvalid ? c.F(hUnitValue, h) * dvec[unit] : 0.0f;
             c.F(hRes, h) = urows[size_t{slot} * kRowWords + 4u] * dt - (0.0f + along);
@@ -2644,6 +2738,7 @@ __host__ __device__ inline uint32_t PaddedWidth(uint32_t n) { return (n + 3u) & 
 // (DataView::solver_mass_factor), so that two of them fit a compute unit's LDS.
 __host__ __device__ inline bool MassFactorInMemory(uint32_t n) { return PaddedWidth(n) > uint32_t(kTwoWaveWidth); }
 __host__ __device__ inline uint32_t FactorRegionFloats(uint32_t n) {
+    if (kPaired) return 0u;
     const uint32_t N = PaddedWidth(n);
     return (MassFactorInMemory(n) ? 1u : 2u) * FactorFloats(N);   // a multiple of 4
 }
@@ -2660,6 +2755,7 @@ __host__ __device__ inline uint32_t KeptRowFloats(uint32_t n, bool reduced) {
     const uint32_t N = PaddedWidth(n);
     return N > 32u ? 0u : (reduced ? 2u : 1u) * N * N;
 }
+constexpr uint32_t kVectorFloats = kPaired ? kTurnFloats : 4u * uint32_t(kWave);   // Tile::vec
 // the coordinates' lists of their unit heads, sixteen bits a place
 __host__ __device__ inline uint32_t UnitListFloats(uint32_t cap, uint32_t staged) { return cap > staged ? kUnitSlots * uint32_t(kWave) / 2u : 0u; }
 __host__ __device__ inline uint32_t HeadFieldFloats(uint32_t cap, uint32_t narrow) {
@@ -2678,7 +2774,7 @@ __host__ __device__ inline uint32_t SolverLdsFloats(uint32_t n, uint32_t cap, ui
     const uint32_t N = PaddedWidth(n);
     // the per-coordinate unit lists exist only when some head beyond the staged ones can be listed; without joint rows
     // the block keeps the footprint that lets eight of them share a compute unit's LDS
-    return FactorRegionFloats(n) + RowFloats(N, staged, from_links) + HeadFieldFloats(cap, staged) + 256u +
+    return FactorRegionFloats(n) + RowFloats(N, staged, from_links) + HeadFieldFloats(cap, staged) + kVectorFloats +
            UnitListFloats(cap, staged) + LinkAxisFloats(n) + KeptRowFloats(n, reduced);
 }
 __host__ __device__ inline uint32_t ReducedSolverLdsFloats(uint32_t full, uint32_t reduced, uint32_t cap, uint32_t staged, bool from_links = false) {
@@ -2802,24 +2898,47 @@ __device__ __forceinline__ bool reduce_block(uint32_t lane, uint32_t n, const fl
 
 // K < N is a reduced block (described above mass_times): no contact of the world reaches the coordinates K..n-1, which are
 // eliminated once in the set-up, and the sweeps run K wide.  K is a multiple of 4 with K <= n, contact heads only.
-template <int N, bool kContactsOnly, int K = N, bool kElliptic = !kContactsOnly>
+//   An environment a block, or (kQueue, every dense instantiation), where environments outnumber the blocks the machine holds at once,
+// as many blocks as it holds, each of which takes the next place of the launch order (DataView::solver_queue, cleared by the order's
+// launch) when it is done.  Blocks of a launch are handed out in turns to the parts of the machine, and one whose part is full holds up those
+// behind it: with solves of unequal length a launch of 8192 blocks kept four fifths of the places busy.  The first places are the
+// blocks' own, so that the costliest environments start where a launch of all of them would start them.  Instantiations of their own,
+// for what a solve keeps in registers over the loop costs the others a per cent (4096 walkers 304 -> 308 us a step).
+constexpr uint32_t kQueued = kInvalid - 1u;   // in the place of a launch's largest number of points: points_lo blocks and a queue
+struct SolveArguments { ModelView m; DataView d; BlockDescentSolveParams p; };   // the first of the kernel's arguments as they lie in memory
+template <int N, bool kContactsOnly, int K = N, bool kElliptic = !kContactsOnly, bool kQueue = kDense>
 __global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(WavesPerSimd(K), WavesPerSimd(K))))
-BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint32_t cap, uint32_t staged_cap, uint32_t points_lo,
-                       uint32_t points_hi) {
+BlockDescentTileKernel(ModelView model, DataView data, BlockDescentSolveParams params, uint32_t cap, uint32_t staged_cap, uint32_t lowest,
+                       uint32_t highest) {
     constexpr bool kReduced = K < N;
     constexpr int W = K;   // the width of the sweeps
     static_assert(K % 4 == 0 && K <= N && (!kReduced || kContactsOnly), "a reduced block holds contact heads only");
     extern __shared__ __align__(16) float lds[];
-    const uint32_t env = d.tile_order[blockIdx.x], lane = threadIdx.x;
+    uint32_t place = blockIdx.x;
+environment:
+    auto arguments = (const __attribute__((address_space(4))) SolveArguments*)__builtin_amdgcn_kernarg_segment_ptr();
+    uint32_t lane = threadIdx.x;
+    if constexpr (kQueue) {
+        // They come anew for every environment: what follows from them would otherwise be made once, ahead of the loop, and kept in
+        // registers that a solve does not have.
+        lane = 0u;
+        asm volatile("" : "+s"(arguments), "+s"(lane));
+        lane = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, lane));
+    }
+    const ModelView& m = kQueue ? ((const SolveArguments*)arguments)->m : model;
+    const DataView& d = kQueue ? ((const SolveArguments*)arguments)->d : data;
+    const BlockDescentSolveParams& p = kQueue ? ((const SolveArguments*)arguments)->p : params;
+    const uint32_t env = d.tile_order[place];
     // A world whose contact slots outnumber the contacts it usually has is solved by two launches of different LDS
     // capacity; each takes the environments whose contact points fall in its range and leaves the others at once.
-    if (points_lo != 0u || points_hi != kInvalid) {
+    if (!(kQueue && highest == kQueued) && (lowest != 0u || highest != kInvalid)) {
         const uint32_t points = d.contact_count[env];
-        if (points < points_lo || points > points_hi) return;
+        if (points < lowest || points > highest) return;
     }
     const uint32_t R = p.rows_per_env, md = p.max_dof, n = m.dof, nl = m.links_per_env, S = p.contact_slots_per_env;
     // A narrow block would leave registers free and let more waves share a SIMD than the launch is sized for; one name of
-    // the last register holds the kernel to its two (dense build: three or four) waves.
+    // the last register holds the kernel to its two (dense build: three or four) waves.  (Behind the place's own words, which
+    // are scalar reads only ahead of it.)
     if constexpr (WavesPerSimd(W) == 4) asm volatile("" ::: "v127");
     else if constexpr (WavesPerSimd(W) == 3) asm volatile("" ::: "v163");
     else if constexpr (WavesPerSimd(W) == 2) asm volatile("" ::: "v255");
@@ -2837,18 +2956,19 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
     PROF_BEGIN(c, 9);
     PROF_BEGIN(c, 0);
     if constexpr (W > kTwoWaveWidth) {
-        c.mfac = d.solver_mass_factor + size_t{env} * FactorFloats(uint32_t(W));
+        c.mfac = d.solver_mass_factor + size_t{env} * MassFactorFloats(uint32_t(W));
         c.hfac = lds;
     } else {
         c.mfac = lds;
         c.hfac = c.mfac + FactorFloats(uint32_t(W));
     }
-    c.from_links = RowsFromLinks(uint32_t(W), kContactsOnly, m.rows_from_links);
+    c.from_links = kPaired || RowsFromLinks(uint32_t(W), kContactsOnly, m.rows_from_links);
     c.jac = lds + FactorRegionFloats(uint32_t(W));
     c.wrench = c.jac;   // one or the other
     c.fields = c.jac + RowFloats(uint32_t(W), staged_cap, c.from_links);
     c.vec = c.fields + HeadFieldFloats(cap, staged_cap);
-    c.hrows = c.vec + 256 + UnitListFloats(cap, staged_cap);
+    if constexpr (kPaired) c.hfac = c.vec;   // what the set-up passes through the factor's place
+    c.hrows = c.vec + kVectorFloats + UnitListFloats(cap, staged_cap);
     c.low = c.hrows + uint32_t(W) * uint32_t(W);
     // The block's mass rows: lane's row of M, or in a reduced block lane's row of the Schur complement (lanes below K)
     // and of -P (the followers).
@@ -2860,10 +2980,10 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
         PROF_END(c, 30);
     }
     if (lane < kNarrowFields) c.fields[kWideStride * cap + staged_cap * kNarrowStride + lane] = 0.0f;   // what a narrow field reads beyond its heads
-    c.unit_list = reinterpret_cast<uint16_t*>(c.vec + 256);
+    c.unit_list = reinterpret_cast<uint16_t*>(c.vec + kVectorFloats);
     c.unit_lists = true; c.unit_count = 0u; c.unit_most = 0u; c.staged_end = 0u; c.individual_end = 0u;
     c.through_links = false; c.over_runs = false; c.way_runs = false;
-    c.axes = c.vec + 256 + UnitListFloats(cap, staged_cap);   // a wide block's; a narrow one keeps rows here
+    c.axes = c.vec + kVectorFloats + UnitListFloats(cap, staged_cap);   // a wide block's; a narrow one keeps rows here
     c.path_low = c.path_high = c.under_low = c.under_high = c.over_low = c.over_high = 0u;
     c.stiffness_current = false;
     c.rows = d.urows; c.row_point_a = d.row_cj_point; c.row_point_b = d.row_cj_point_b;
@@ -2962,7 +3082,8 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
             float unit_value = 0.0f;
             if (owned && single_axis && d.row_unit[slot] != kInvalid) { unit = d.row_unit[slot]; unit_value = d.row_unit_value[slot]; }
             else if (owned && h >= staged_cap) { overflow_rows = true; unit = 0u; }   // no room for its rows: it acts on nothing, and the solve is flagged
-            c.U(hUnit, h) = unit; c.F(hUnitValue, h) = unit_value; c.U(hRow, h) = owned && unit == kInvalid ? 0u : kInvalid;
+            if constexpr (!kPaired) { c.U(hUnit, h) = unit; c.F(hUnitValue, h) = unit_value; }
+            c.U(hRow, h) = owned && unit == kInvalid ? 0u : kInvalid;
             c.U(hColumnsLow, h) = 0u; c.U(hColumnsHigh, h) = 0u;
         }
         if (__any(overflow_rows) && lane == 0u) d.env_status[env] |= kEnvStatusSolverFailure;
@@ -3478,7 +3599,7 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
         // launch slot and the wave's first and last moment on the constant 100 MHz clock, as raw words
         d.solver_penalty[size_t{env} * R + 30] = __uint_as_float(uint32_t(prof_wall_start));
         d.solver_penalty[size_t{env} * R + 31] = __uint_as_float(uint32_t(wall_clock64()));
-        d.solver_penalty[size_t{env} * R + 32] = __uint_as_float(blockIdx.x);
+        d.solver_penalty[size_t{env} * R + 32] = __uint_as_float(place);
     }
 #endif
     // the block velocities persist for the next solve's carried start
@@ -3602,8 +3723,20 @@ BlockDescentTileKernel(ModelView m, DataView d, BlockDescentSolveParams p, uint3
             else d.link_velocity_pseudo[(lbase + my_link) * 6u + my_component] = pseudo;
         }
     }
+    if constexpr (kQueue) {
+        if (highest != kQueued) return;
+        uint32_t taken = 0u;
+        if (lane == 0u) taken = atomicAdd(d.solver_queue, 1u);
+        place = lowest + uint32_t(__builtin_amdgcn_readfirstlane(int(taken)));
+        if (place >= p.env_count) return;
+        __syncthreads();
+        goto environment;
+    }
 }
 
+#ifdef NKH_SOLVER_PAIRED
+}  // namespace paired
+#endif
 #ifdef NKH_SOLVER_DENSE
 }  // namespace dense
 #endif

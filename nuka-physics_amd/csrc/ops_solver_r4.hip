@@ -3,5 +3,6 @@
 namespace nkh {
 namespace solver {
 template __global__ void BlockDescentTileKernel<64, true, 32>(ModelView, DataView, BlockDescentSolveParams, uint32_t, uint32_t, uint32_t, uint32_t);
+template __global__ void BlockDescentTileKernel<64, true, 32, false, true>(ModelView, DataView, BlockDescentSolveParams, uint32_t, uint32_t, uint32_t, uint32_t);
 }  // namespace solver
 }  // namespace nkh

@@ -924,7 +924,8 @@ nuka_result_t CreateWorld(nuka_device_handle device, const nuka_template_desc_t*
 #define X(name, dtype, count) Place<int>(w.fields, #name, dtype, size_t(count), &cursor, false);
         NKH_DATA_FIELDS(X)
 #undef X
-        w.arena_bytes = cursor;
+        const size_t queue_at = (cursor + 255u) & ~size_t{255u};   // the solve's queue, behind the fields
+        w.arena_bytes = queue_at + 256u;
         uint8_t status = 0u;
         nuka_phi_buffer_type* type = BackendDeviceBufferType(w.device->backend);
         w.arena = reinterpret_cast<nuka_phi_buffer_type_head*>(type)->iface->alloc(type, w.arena_bytes, &status);
@@ -950,6 +951,7 @@ nuka_result_t CreateWorld(nuka_device_handle device, const nuka_template_desc_t*
 #define X(name, dtype, count) { const Field& fld = w.fields[f++]; w.data.name = reinterpret_cast<decltype(w.data.name)>(base + fld.offset); }
         NKH_DATA_FIELDS(X)
 #undef X
+        w.data.solver_queue = reinterpret_cast<uint32_t*>(base + queue_at);
         // initial state: identity poses, cooked static poses, no rows
         {
             std::vector<float> base_pose(E * 7u, 0.0f), link_pose(E * nl * 7u, 0.0f), body_pose(E * nb * 7u, 0.0f);

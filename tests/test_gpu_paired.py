@@ -1,0 +1,65 @@
+"""A solve's result is the environment's own, whatever kernel and launch its batch takes: wide blocks two a SIMD, launches of as
+many blocks as the machine holds."""
+import numpy as np
+import pytest
+
+from conftest import nk
+from trees import tree_case
+
+abi = nk.abi
+pytestmark = pytest.mark.gpu
+FIELDS = ("q", "qdot", "link_velocity", "lambda", "vbd_velocity_sweep_count", "env_status", "solver_residual")
+
+
+def repeated(state, E):
+    return {name: np.ascontiguousarray(np.asarray(v)[np.arange(E) % len(v)]) for name, v in state.items()}
+
+
+def batches_agree(device, template, desc_of, state, small, large, steps=2):
+    """The environments of a large batch, the small one's over and over, step as the small one's do, bit for bit."""
+    few, many = nk.World(device, template, desc_of(small)), nk.World(device, template, desc_of(large))
+    few.set_state(state)
+    many.set_state(repeated(state, large))
+    for _ in range(steps):
+        few.step()
+        many.step()
+    few.synchronize()
+    many.synchronize()
+    assert (few.download("contact_count") > 0).any()
+    for name in FIELDS:
+        a, b = few.download(name).reshape(small, -1), many.download(name).reshape(large, -1)
+        assert np.array_equal(b.view(np.uint32), a.view(np.uint32)[np.arange(large) % small]), name
+    blocks = few.info.solver_blocks_per_cu, many.info.solver_blocks_per_cu
+    few.close()
+    many.close()
+    return blocks
+
+
+@pytest.mark.parametrize("dof,floating,branched,limb_joints", [
+    (37, False, True, 2), (40, False, False, 7), (44, True, True, 3), (50, True, True, 2), (53, False, True, 4), (57, True, False, 7),
+    (61, False, True, 2), (64, False, True, 3),
+])
+def test_wide_trees_two_a_simd_step_as_one_a_simd(oracle_py, device, dof, floating, branched, limb_joints):
+    """Every padded width, with coordinates that fill it and that do not, ways and heads that are runs of lanes and that are not."""
+    small, large = 48, 2049
+    tree, _, state = tree_case(oracle_py, dof, floating, branched, seed=5 * dof, E=small, limb_joints=limb_joints)
+    blocks = batches_agree(device, tree.template, lambda E: abi.world_desc(E, 1.0 / 240.0, vel_iters=6), state, small, large)
+    assert blocks[0] <= 4 < blocks[1]
+
+
+def test_ropes_two_a_simd_step_as_one_a_simd(device):
+    cfg = nk.synthetic.config(5, 64)
+    blocks = batches_agree(device, cfg.template, lambda E: abi.world_desc(E, cfg.dt, vel_iters=cfg.vel_iters), cfg.state(), 64, 2111)
+    assert blocks == (4, 8)
+
+
+@pytest.mark.parametrize("index,driven,large", [(2, False, 2049), (2, False, 6144 + 1), (3, False, 2600), (3, True, 1900)])
+def test_environments_past_the_blocks_held_step_as_the_first(device, index, driven, large):
+    """Two-wave, dense and general kernels with more environments than blocks: the ones that wait in the queue, one at the least."""
+    cfg = nk.synthetic.config(index, 150)
+    template = cfg.template
+    if driven:
+        for link in template.links:
+            if link["joint_type"] == abi.JOINT_REVOLUTE:
+                link["frictionloss"] = 0.1
+    batches_agree(device, template, lambda E: abi.world_desc(E, cfg.dt, vel_iters=cfg.vel_iters), cfg.state(), 150, large, steps=3)
