@@ -818,19 +818,19 @@ __device__ __forceinline__ uint32_t contact_row_bound(uint32_t previous, uint32_
 // nk/solve/collidable_owner.hpp:25-62 for one articulation per environment
 __device__ uint32_t resolve_side(const ModelView& m, uint32_t env, uint32_t collidable, int32_t body_id, uint32_t* index,
                                  uint32_t* link) {
+    // (two rounds of reads, whatever the answer: read under the answer's conditions they are four, one behind the other)
+    const bool within = collidable < m.bodies_per_env;
+    const uint32_t own = within ? collidable : 0u;
+    const uint32_t proxy = m.body_collidable_body[own];
+    const bool proxied = proxy != kInvalid;
+    const uint32_t body = proxied && proxy < m.bodies_per_env ? proxy : own;
+    const uint32_t further = m.body_collidable_body[body], l = m.body_to_link[body], articulation = m.body_to_articulation[body];
     *index = kInvalid; *link = kInvalid;
-    if (collidable >= m.bodies_per_env) return kInvalid;
-    uint32_t body = collidable;
+    if (!within) return kInvalid;
     if (body_id < 0) return kSideStatic;
-    const uint32_t proxy = m.body_collidable_body[body];
-    if (proxy != kInvalid) {
-        if (proxy >= m.bodies_per_env) return kInvalid;
-        body = proxy;
-        if (m.body_collidable_body[body] != kInvalid) return kInvalid;
-    }
-    const uint32_t l = m.body_to_link[body];
+    if (proxied && (proxy >= m.bodies_per_env || further != kInvalid)) return kInvalid;
     if (l == kInvalid) { *index = env * m.bodies_per_env + body; return kSideRigid; }
-    if (l >= m.links_per_env || m.body_to_articulation[body] >= 1u) return kInvalid;
+    if (l >= m.links_per_env || articulation >= 1u) return kInvalid;
     *link = env * m.links_per_env + l; *index = env;
     return kSideArtic;
 }
@@ -964,16 +964,30 @@ __device__ __forceinline__ float uniform_value(float v, uint32_t lane) {   // `l
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), int(lane)));
 }
 
+// lane's value and those of the lanes before it
+__device__ __forceinline__ uint32_t wave_running_sum(uint32_t v) {
+    const auto add = [&](auto from, auto rows) { v += uint32_t(__builtin_amdgcn_update_dpp(0, int(v), decltype(from)::value, decltype(rows)::value, 0xF, true)); };
+    using std::integral_constant;
+    const integral_constant<int, 0xF> all{};
+    add(integral_constant<int, 0x111>{}, all); add(integral_constant<int, 0x112>{}, all);   // within sixteen lanes
+    add(integral_constant<int, 0x114>{}, all); add(integral_constant<int, 0x118>{}, all);
+    add(integral_constant<int, 0x142>{}, integral_constant<int, 0xA>{});   // lane 15 of a row to the next row,
+    add(integral_constant<int, 0x143>{}, integral_constant<int, 0xC>{});   // lane 31 to the upper two
+    return v;
+}
+
 // ---- AssembleRows: one wavefront per environment (assemble_rows.cu:325-394, 200-214, 406-801, 122-186) ----
 // A lane a contact point, 64 points at a time: it writes the point's rows, and then the points go by in turn, lane = DoF,
 // with what their rows share - links, point, directions - handed round as lane reads, so that the moment arm of a point is
 // formed once for its rows and nothing of a row waits in LDS (ten words a row slot were 42 KB of it for 64 slots, three
 // blocks a compute unit).  Two instantiations: worlds without compliant contacts need neither their spring-dampers and pyramids
-// nor the registers these take, and run six waves a SIMD where the others run four.
+// nor the registers these take, and run six waves a SIMD where the others run four.  It is a chain of reads and of the points'
+// arithmetic: what a point and a coordinate need is read ahead of the first write, which no read can be moved past, in three rounds
+// where there were seven (4096 humanoids 30.4 -> 28.7 us, 65536 329 -> 306, 8192 ropes 360 -> 322, 16384 boxes 54 -> 50).
 __host__ __device__ inline uint32_t AssembleTermStride(uint32_t md) { return md | 1u; }   // rows of terms in different banks
 constexpr uint32_t kTermRows = 32u;   // sixteen rows, both sides
 __host__ __device__ inline uint32_t AssembleLdsWords(uint32_t slots, uint32_t links, uint32_t md, bool compliant) {
-    return 2u * slots + 2u * links + (compliant ? kTermRows * AssembleTermStride(md) : 0u);
+    return 4u * slots + 2u * links + (compliant ? kTermRows * AssembleTermStride(md) : 0u);
 }
 template <bool kCompliant>
 __global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(kCompliant ? 4 : 6, kCompliant ? 4 : 6))) AssembleRowsKernel(ModelView m, DataView d, AssembleRowsParams p) {
@@ -984,56 +998,15 @@ __global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(kCom
     uint64_t* link_mask = reinterpret_cast<uint64_t*>(lds_u);
     uint32_t* range_first = lds_u + 2u * nl;   // S
     uint32_t* range_points = range_first + S;   // S
-    float* terms = reinterpret_cast<float*>(range_points + S);   // kTermRows rows of what a compliant row's start velocity sums
+    uint16_t* listed = reinterpret_cast<uint16_t*>(range_points + S);   // 4 S: the environment's points, 4 slot + point
+    float* terms = reinterpret_cast<float*>(range_points + 3u * S);   // kTermRows rows of what a compliant row's start velocity sums
     for (uint32_t l = lane; l < nl; l += kWave) link_mask[l] = m.link_dof_mask[l];
     Row* rows = reinterpret_cast<Row*>(d.urows) + size_t{env} * R;
     float* lambda = d.lambda + size_t{env} * R;
     float* pen = d.row_penetration + size_t{env} * R;
     uint32_t* cj_link = d.row_cj_link + size_t{env} * R, *cj_link_b = d.row_cj_link_b + size_t{env} * R;
     float* cj_point = d.row_cj_point + size_t{env} * R * 3u, *cj_point_b = d.row_cj_point_b + size_t{env} * R * 3u;
-    // row ranges: exclusive prefix of the slots' point counts, four rows a point (:336-360)
-    const uint32_t previous_extent = d.contact_row_extent[2u * env + 1u];
-    uint32_t carry = 0u, extent = 1u;
-    bool many = false;   // some slot has more than one point
-    for (uint32_t base = 0u; base < S; base += kWave) {
-        const uint32_t slot = base + lane;
-        const uint32_t points = slot < S ? d.ucontact_count[size_t{env} * S + slot] : 0u;
-        uint32_t through = points;
-#pragma unroll
-        for (int o = 1; o < kWave; o <<= 1) {
-            const uint32_t other = __shfl_up(through, o, kWave);
-            if (int(lane) >= o) through += other;
-        }
-        if (slot < S) {
-            const uint32_t first = (carry + through - points) * kRowsPerPoint;
-            range_first[slot] = first; range_points[slot] = points;
-            many = many || points > 1u;
-            d.ucontact_row_range[(size_t{env} * S + slot) * 2u] = env * R + first;
-            d.ucontact_row_range[(size_t{env} * S + slot) * 2u + 1u] = points;
-            if (first < contact_row_bound(previous_extent, 1u, CR)) d.contact_material[size_t{env} * S + slot] = 0ull;   // :358
-            if (points > 0u) extent = max(extent, first + points * kRowsPerPoint + 1u);
-        }
-        carry += __shfl(through, kWave - 1, kWave);
-    }
-    extent = wave_max_u(extent);
-    // Rows below the previous and current extents are cleared (:366-394); the impulses by the previous extent, which a restore
-    // zeroes since it brings impulses back, the rest by what this world's own steps have left in memory, which a restore
-    // does not touch: 192 flags cleared, a line of memory each, were 197 us of the 641 us this kernel took at 65536 humanoids
-    // stepped from a checkpoint.
-    // (a caller that binds its own buffers may leave the field out: the previous extent then bounds both)
-    const uint32_t left = d.row_clear_extent != nullptr ? d.row_clear_extent[env] : previous_extent;
-    const uint32_t impulse_bound = contact_row_bound(previous_extent, 1u, CR), clear_bound = contact_row_bound(left, 1u, CR);
-    for (uint32_t local = lane; local < impulse_bound; local += kWave) lambda[local] = 0.0f;
-    for (uint32_t local = lane; local < clear_bound; local += kWave) {
-        pen[local] = 0.0f; cj_link[local] = kInvalid; cj_link_b[local] = kInvalid;
-        rows[local].flags = 0u;
-    }
-    if (lane == 0u) {
-        d.contact_row_extent[2u * env] = previous_extent;
-        d.contact_row_extent[2u * env + 1u] = extent;
-        if (d.row_clear_extent != nullptr) d.row_clear_extent[env] = extent;
-    }
-    // padded generalized velocity tile (:200-214)
+    // What a coordinate's lane needs, ahead of everything that is written: no read waits behind a write that way.
     float free_velocity = 0.0f;   // of lane's coordinate
     if (lane < md) {
         float value = 0.0f;
@@ -1041,10 +1014,8 @@ __global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(kCom
             const uint32_t link = m.dof_link[lane], c = m.dof_component[lane];
             value = c == kInvalid ? d.qdot[size_t{env} * nl + link] : d.link_velocity[(size_t{env} * nl + link) * 6u + c];
         }
-        d.qdot_flat[size_t{env} * md + lane] = value;
         free_velocity = value;
     }
-    __syncthreads();
     // lane = DoF: the coordinate's axis, where it lies and whether it turns
     V3 axis_world{0, 0, 0}, origin{0, 0, 0};
     uint32_t mode = 0u;   // 0 none, 1 revolute, 2 prismatic, 3 base angular, 4 base linear
@@ -1074,15 +1045,54 @@ __global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(kCom
         }
     }
     const float start_velocity = kCompliant && m.any_mujoco != 0u && lane < md ? d.step_qdot_flat[size_t{env} * md + lane] : 0.0f;
+    // row ranges: exclusive prefix of the slots' point counts, four rows a point (:336-360)
+    const uint32_t previous_extent = d.contact_row_extent[2u * env + 1u];
+    uint32_t carry = 0u, extent = 1u;
+    for (uint32_t base = 0u; base < S; base += kWave) {
+        const uint32_t slot = base + lane;
+        const uint32_t points = slot < S ? d.ucontact_count[size_t{env} * S + slot] : 0u;
+        const uint32_t through = wave_running_sum(points);
+        if (slot < S) {
+            const uint32_t first = (carry + through - points) * kRowsPerPoint;
+            range_first[slot] = first; range_points[slot] = points;
+            for (uint32_t point = 0u, at = carry + through - points; point < points && at < 4u * S; ++point, ++at)
+                listed[at] = uint16_t(point < 4u ? 4u * slot + point : 0xFFFFu);   // (a manifold has no more than four)
+            d.ucontact_row_range[(size_t{env} * S + slot) * 2u] = env * R + first;
+            d.ucontact_row_range[(size_t{env} * S + slot) * 2u + 1u] = points;
+            if (first < contact_row_bound(previous_extent, 1u, CR)) d.contact_material[size_t{env} * S + slot] = 0ull;   // :358
+            if (points > 0u) extent = max(extent, first + points * kRowsPerPoint + 1u);
+        }
+        carry += uint32_t(__builtin_amdgcn_readlane(int(through), int(kWave) - 1));
+    }
+    const uint32_t items = min(carry, 4u * S);
+    extent = wave_max_u(extent);
+    // Rows below the previous and current extents are cleared (:366-394); the impulses by the previous extent, which a restore
+    // zeroes since it brings impulses back, the rest by what this world's own steps have left in memory, which a restore
+    // does not touch: 192 flags cleared, a line of memory each, were 197 us of the 641 us this kernel took at 65536 humanoids
+    // stepped from a checkpoint.
+    // (a caller that binds its own buffers may leave the field out: the previous extent then bounds both)
+    const uint32_t left = d.row_clear_extent != nullptr ? d.row_clear_extent[env] : previous_extent;
+    const uint32_t impulse_bound = contact_row_bound(previous_extent, 1u, CR), clear_bound = contact_row_bound(left, 1u, CR);
+    for (uint32_t local = lane; local < impulse_bound; local += kWave) lambda[local] = 0.0f;
+    for (uint32_t local = lane; local < clear_bound; local += kWave) {
+        pen[local] = 0.0f; cj_link[local] = kInvalid; cj_link_b[local] = kInvalid;
+        rows[local].flags = 0u;
+    }
+    if (lane == 0u) {
+        d.contact_row_extent[2u * env] = previous_extent;
+        d.contact_row_extent[2u * env + 1u] = extent;
+        if (d.row_clear_extent != nullptr) d.row_clear_extent[env] = extent;
+    }
+    if (lane < md) d.qdot_flat[size_t{env} * md + lane] = free_velocity;   // :200-214
+    __syncthreads();
     auto uniform_word = [](uint32_t v, uint32_t from) { return uint32_t(__builtin_amdgcn_readlane(int(v), int(from))); };
-    // contact rows (:453-801; speculative law, condim 3): a lane a slot where every slot has one point at most, else a
-    // lane a (slot, point) - a slot's points share nothing but the slot's own values, which each of their lanes works
-    // out for itself
+    // contact rows (:453-801; speculative law, condim 3): a lane a point the environment has - a slot's points share nothing but the
+    // slot's own values, which each of their lanes works out for itself.  (A lane a slot's every place, 304 of them for 76 slots of
+    // four, was five passes for a handful of points.)
     uint32_t active_rows = 0u, driven_points = 0u;
     bool invalid_endpoint = false;
-    const uint32_t fan = __any(many) ? 4u : 1u;
     constexpr int kAxes = kCompliant ? 4 : 3;   // rows a point
-    for (uint32_t chunk = 0u; chunk < S * fan; chunk += kWave) {
+    for (uint32_t chunk = 0u; chunk < items; chunk += kWave) {
         // what the chain Jacobians need of lane's point: its first row and the stride of its rows, which of them it has, its
         // links, whether they have one owner, the point, the rows' directions (side A's; side B's are their negatives) and
         // a compliant row's gain on the start velocity along it
@@ -1092,15 +1102,18 @@ __global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(kCom
 #pragma unroll
         for (int axis = 0; axis < kAxes; ++axis) { my_dir[axis] = V3{0, 0, 0}; my_gain[axis] = 0.0f; my_rhs[axis] = 0.0f; }
         const auto emit_point = [&]() {
-        const uint32_t item = chunk + lane;
-        if (item >= S * fan) return;
-        const uint32_t slot = item / fan, own_point = item - slot * fan;
-        const size_t gid = size_t{env} * S + slot;
+        const uint32_t item = chunk + lane, entry = item < items ? listed[item] : 0xFFFFu;
+        if (entry == 0xFFFFu) return;
+        const uint32_t slot = entry / 4u, own_point = entry & 3u;
+        const size_t gid = size_t{env} * S + slot, mp = gid * 4u + own_point;
         const uint32_t base = range_first[slot], P = range_points[slot];
-        if (own_point >= P) return;
         const bool slot_lane = own_point == 0u;   // the one lane that writes what belongs to the slot as a whole
         uint32_t n_active = P;
-        const uint32_t local_a = d.ucontact_a[gid * 4u], local_b = d.ucontact_b[gid * 4u];
+        // (all that is read of the point, ahead of what is written)
+        const uint32_t local_a = d.ucontact_a[gid * 4u], local_b = d.ucontact_b[gid * 4u], law = d.ucontact_law[gid];
+        const V3 raw{d.ucontact_normal[3u * mp], d.ucontact_normal[3u * mp + 1u], d.ucontact_normal[3u * mp + 2u]};
+        const V3 place{d.ucontact_point[3u * mp], d.ucontact_point[3u * mp + 1u], d.ucontact_point[3u * mp + 2u]};
+        const float penetration = d.ucontact_depth[mp];
         ShapeRow sa{}, sb{};
         sa.body_id = sb.body_id = -1; sa.profile = sb.profile = kInvalid;
         if (local_a < m.bodies_per_env) sa = load_shape(m.shape_table, local_a);
@@ -1115,7 +1128,6 @@ __global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(kCom
         if (kind_a == kSideStatic) idx_a = kInvalid;
         if (kind_b == kSideStatic) idx_b = kInvalid;
         // the two sides' profiles merged (:540-594; scene/contact_filter.hpp:100-137); a side without one has the defaults
-        const uint32_t law = d.ucontact_law[gid];
         const bool mujoco = kCompliant && law == kContactLawCompliant;   // :480
         float side_a[14], side_b[14], merged[12];
         profile_terms(m, sa.profile, side_a); profile_terms(m, sb.profile, side_b);
@@ -1141,22 +1153,20 @@ __global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(kCom
         if (pyramidal && sb.kind == 1u && sa.kind == 3u) frame_axis = make_prim(sb, load_xf(d.body_pose + (size_t{env} * m.bodies_per_env + local_b) * 7u)).cz;
         {
             const uint32_t pt = own_point;
-            const size_t mp = gid * 4u + pt;
             // the velocity laws keep every point; a compliant point lives inside its margin (:625-626)
-            const bool live = pt < n_active && pt < 4u && (!mujoco || d.ucontact_depth[mp] + margin > 0.0f);
+            const bool live = pt < n_active && pt < 4u && (!mujoco || penetration + margin > 0.0f);
             // the rows' directions as four values selected by the row's place, not an array indexed by it: an array
             // indexed at run time lives in scratch memory, and every row would wait on it
             V3 n{0, 0, 1}, point{0, 0, 0}, dir0{0, 0, 0}, dir1{0, 0, 0}, dir2{0, 0, 0}, dir3{0, 0, 0};
             V3 t0{1, 0, 0}, t1{0, 1, 0};
             float d0 = 0.0f;
             if (live) {
-                const V3 raw{d.ucontact_normal[3u * mp], d.ucontact_normal[3u * mp + 1u], d.ucontact_normal[3u * mp + 2u]};
                 const float len = sqrtf(raw.x * raw.x + raw.y * raw.y + raw.z * raw.z);
                 n = len < 1e-12f ? V3{0, 0, 0} : V3{raw.x / len, raw.y / len, raw.z / len};
-                point = V3{d.ucontact_point[3u * mp], d.ucontact_point[3u * mp + 1u], d.ucontact_point[3u * mp + 2u]};
+                point = place;
                 if (kCompliant && pyramidal) mujoco_contact_frame(raw, frame_axis, &t0, &t1);
                 else contact_tangent_basis(raw, &t0, &t1);
-                d0 = d.ucontact_depth[mp];
+                d0 = penetration;
             }
             // a pyramid has four scalar rows a point along n +- mu t (:651-690); the other cones a normal and two tangents
             const uint32_t row_count = pyramidal ? 4u : 3u;
