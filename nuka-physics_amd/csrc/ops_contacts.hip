@@ -982,7 +982,8 @@ __device__ __forceinline__ uint32_t wave_running_sum(uint32_t v) {
 // with what their rows share - links, point, directions - handed round as lane reads, so that the moment arm of a point is
 // formed once for its rows and nothing of a row waits in LDS (ten words a row slot were 42 KB of it for 64 slots, three
 // blocks a compute unit).  Two instantiations: worlds without compliant contacts need neither their spring-dampers and pyramids
-// nor the registers these take, and run six waves a SIMD where the others run four.  It is a chain of reads and of the points'
+// nor the registers these take, and run six waves a SIMD where the others run four.  A third gives an environment `G` lanes of a
+// wavefront (AssembleTakesEight): a free body's four points and six coordinates kept six lanes of 64 at work.  It is a chain of reads and of the points'
 // arithmetic: what a point and a coordinate need is read ahead of the first write, which no read can be moved past, in three rounds
 // where there were seven (4096 humanoids 30.4 -> 28.7 us, 65536 329 -> 306, 8192 ropes 360 -> 322, 16384 boxes 54 -> 50).
 __host__ __device__ inline uint32_t AssembleTermStride(uint32_t md) { return md | 1u; }   // rows of terms in different banks
@@ -990,10 +991,19 @@ constexpr uint32_t kTermRows = 32u;   // sixteen rows, both sides
 __host__ __device__ inline uint32_t AssembleLdsWords(uint32_t slots, uint32_t links, uint32_t md, bool compliant) {
     return 4u * slots + 2u * links + (compliant ? kTermRows * AssembleTermStride(md) : 0u);
 }
-template <bool kCompliant>
-__global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(kCompliant ? 4 : 6, kCompliant ? 4 : 6))) AssembleRowsKernel(ModelView m, DataView d, AssembleRowsParams p) {
+template <bool kCompliant, int G = 64>
+__global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(kCompliant || G < 64 ? 4 : 6, kCompliant || G < 64 ? 4 : 6))) AssembleRowsKernel(ModelView m, DataView d, AssembleRowsParams p) {
     extern __shared__ __align__(8) uint32_t lds_u[];
-    const uint32_t env = blockIdx.x, lane = threadIdx.x;
+    static_assert(G == 64 || !kCompliant, "environments share a wavefront in worlds under the native laws");
+    const uint32_t env = G == 64 ? blockIdx.x : blockIdx.x * uint32_t(kWave / G) + threadIdx.x / G, lane = G == 64 ? threadIdx.x : threadIdx.x % G;
+    // what the lanes of an environment hand each other
+    const auto read = [](uint32_t v, uint32_t from) { return G == 64 ? uint32_t(__builtin_amdgcn_readlane(int(v), int(from))) : uint32_t(__shfl(int(v), int(from), G)); };
+    const auto read_value = [&](float v, uint32_t from) { return __uint_as_float(read(__float_as_uint(v), from)); };
+    const auto over_lanes = [](auto v, auto&& join) {   // (fewer than 64)
+#pragma unroll
+        for (int o = 1; o < G; o <<= 1) v = join(v, decltype(v)(__shfl_xor(v, o, G)));
+        return v;
+    };
     const uint32_t R = p.rows_per_env, S = p.union_slot_count, CR = p.contact_rows_per_env, md = p.max_dof, nl = m.links_per_env;
     // nl: the coordinates on each link's path to the root; a point asks for its links' masks and would wait on the table each time
     uint64_t* link_mask = reinterpret_cast<uint64_t*>(lds_u);
@@ -1001,7 +1011,8 @@ __global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(kCom
     uint32_t* range_points = range_first + S;   // S
     uint16_t* listed = reinterpret_cast<uint16_t*>(range_points + S);   // 4 S: the environment's points, 4 slot + point
     float* terms = reinterpret_cast<float*>(range_points + 3u * S);   // kTermRows rows of what a compliant row's start velocity sums
-    for (uint32_t l = lane; l < nl; l += kWave) link_mask[l] = m.link_dof_mask[l];
+    for (uint32_t l = threadIdx.x; l < nl; l += kWave) link_mask[l] = m.link_dof_mask[l];
+    if (G < 64 && env >= p.env_count) return;
     Row* rows = reinterpret_cast<Row*>(d.urows) + size_t{env} * R;
     float* lambda = d.lambda + size_t{env} * R;
     float* pen = d.row_penetration + size_t{env} * R;
@@ -1048,25 +1059,39 @@ __global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(kCom
     const float start_velocity = kCompliant && m.any_mujoco != 0u && lane < md ? d.step_qdot_flat[size_t{env} * md + lane] : 0.0f;
     // row ranges: exclusive prefix of the slots' point counts, four rows a point (:336-360)
     const uint32_t previous_extent = d.contact_row_extent[2u * env + 1u];
-    uint32_t carry = 0u, extent = 1u;
-    for (uint32_t base = 0u; base < S; base += kWave) {
+    uint32_t carry = 0u, extent = 1u, own_first = 0u, own_points = 0u;
+    for (uint32_t base = 0u; base < S; base += kWave) {   // (fewer than 64 lanes hold all the slots)
         const uint32_t slot = base + lane;
         const uint32_t points = slot < S ? d.ucontact_count[size_t{env} * S + slot] : 0u;
-        const uint32_t through = wave_running_sum(points);
+        uint32_t through = points;
+        if constexpr (G == 64) through = wave_running_sum(points);
+        else {
+#pragma unroll
+            for (int o = 1; o < G; o <<= 1) {
+                const uint32_t other = uint32_t(__shfl_up(int(through), o, G));
+                if (int(lane) >= o) through += other;
+            }
+        }
         if (slot < S) {
             const uint32_t first = (carry + through - points) * kRowsPerPoint;
-            range_first[slot] = first; range_points[slot] = points;
-            for (uint32_t point = 0u, at = carry + through - points; point < points && at < 4u * S; ++point, ++at)
-                listed[at] = uint16_t(point < 4u ? 4u * slot + point : 0xFFFFu);   // (a manifold has no more than four)
+            own_first = first; own_points = points;
+            if constexpr (G == 64) {
+                range_first[slot] = first; range_points[slot] = points;
+                for (uint32_t point = 0u, at = carry + through - points; point < points && at < 4u * S; ++point, ++at)
+                    listed[at] = uint16_t(point < 4u ? 4u * slot + point : 0xFFFFu);   // (a manifold has no more than four)
+            }
             d.ucontact_row_range[(size_t{env} * S + slot) * 2u] = env * R + first;
             d.ucontact_row_range[(size_t{env} * S + slot) * 2u + 1u] = points;
             if (first < contact_row_bound(previous_extent, 1u, CR)) d.contact_material[size_t{env} * S + slot] = 0ull;   // :358
             if (points > 0u) extent = max(extent, first + points * kRowsPerPoint + 1u);
         }
-        carry += uint32_t(__builtin_amdgcn_readlane(int(through), int(kWave) - 1));
+        carry += read(through, uint32_t(G) - 1u);
     }
-    const uint32_t items = min(carry, 4u * S);
-    extent = wave_max_u(extent);
+    // one pass for a lane a place, where there are no more of them than lanes
+    const uint32_t fan = m.max_points_per_slot == 1u ? 1u : kPointsPerSlot, items = G == 64 ? min(carry, 4u * S) : S * fan;
+    const auto larger = [](uint32_t x, uint32_t y) { return max(x, y); };
+    if constexpr (G == 64) extent = wave_max_u(extent);
+    else extent = over_lanes(extent, larger);
     // Rows below the previous and current extents are cleared (:366-394); the impulses by the previous extent, which a restore
     // zeroes since it brings impulses back, the rest by what this world's own steps have left in memory, which a restore
     // does not touch: 192 flags cleared, a line of memory each, were 197 us of the 641 us this kernel took at 65536 humanoids
@@ -1074,8 +1099,8 @@ __global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(kCom
     // (a caller that binds its own buffers may leave the field out: the previous extent then bounds both)
     const uint32_t left = d.row_clear_extent != nullptr ? d.row_clear_extent[env] : previous_extent;
     const uint32_t impulse_bound = contact_row_bound(previous_extent, 1u, CR), clear_bound = contact_row_bound(left, 1u, CR);
-    for (uint32_t local = lane; local < impulse_bound; local += kWave) lambda[local] = 0.0f;
-    for (uint32_t local = lane; local < clear_bound; local += kWave) {
+    for (uint32_t local = lane; local < impulse_bound; local += G) lambda[local] = 0.0f;
+    for (uint32_t local = lane; local < clear_bound; local += G) {
         pen[local] = 0.0f; cj_link[local] = kInvalid; cj_link_b[local] = kInvalid;
         rows[local].flags = 0u;
     }
@@ -1086,10 +1111,13 @@ __global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(kCom
     }
     if (lane < md) d.qdot_flat[size_t{env} * md + lane] = free_velocity;   // :200-214
     __syncthreads();
-    auto uniform_word = [](uint32_t v, uint32_t from) { return uint32_t(__builtin_amdgcn_readlane(int(v), int(from))); };
     // contact rows (:453-801; speculative law, condim 3): a lane a point the environment has - a slot's points share nothing but the
     // slot's own values, which each of their lanes works out for itself.  (A lane a slot's every place, 304 of them for 76 slots of
     // four, was five passes for a handful of points.)
+    const auto sum_of = [&](float v) {
+        if constexpr (G == 64) return wave_sum(v);
+        else return over_lanes(v, [](float x, float y) { return x + y; });
+    };
     uint32_t active_rows = 0u, driven_points = 0u;
     bool invalid_endpoint = false;
     constexpr int kAxes = kCompliant ? 4 : 3;   // rows a point
@@ -1102,12 +1130,17 @@ __global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(kCom
         float my_gain[kAxes], my_rhs[kAxes];
 #pragma unroll
         for (int axis = 0; axis < kAxes; ++axis) { my_dir[axis] = V3{0, 0, 0}; my_gain[axis] = 0.0f; my_rhs[axis] = 0.0f; }
+        uint32_t place_first = 0u, place_points = 0u;   // of lane's place, where there is a lane a place
+        if constexpr (G < 64) { place_first = read(own_first, lane / fan); place_points = read(own_points, lane / fan); }
         const auto emit_point = [&]() {
-        const uint32_t item = chunk + lane, entry = item < items ? listed[item] : 0xFFFFu;
-        if (entry == 0xFFFFu) return;
-        const uint32_t slot = entry / 4u, own_point = entry & 3u;
+        uint32_t slot = lane / fan, own_point = lane - slot * fan;
+        if constexpr (G == 64) {
+            const uint32_t item = chunk + lane, entry = item < items ? listed[item] : 0xFFFFu;
+            if (entry == 0xFFFFu) return;
+            slot = entry / 4u; own_point = entry & 3u;
+        } else if (slot >= S || own_point >= place_points) return;
         const size_t gid = size_t{env} * S + slot, mp = gid * 4u + own_point;
-        const uint32_t base = range_first[slot], P = range_points[slot];
+        const uint32_t base = G == 64 ? range_first[slot] : place_first, P = G == 64 ? range_points[slot] : place_points;
         const bool slot_lane = own_point == 0u;   // the one lane that writes what belongs to the slot as a whole
         uint32_t n_active = P;
         // (all that is read of the point, ahead of what is written)
@@ -1289,22 +1322,25 @@ __global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(kCom
             __syncthreads();
             staged_terms = 0u;
         };
-        for (uint64_t rest = __ballot(my_axes != 0u && (my_link[0] != kInvalid || my_link[1] != kInvalid)); rest != 0ull; rest &= rest - 1ull) {
+        // (the wavefront's points, or the places of every environment that shares it side by side)
+        uint64_t rest = G == 64 ? __ballot(my_axes != 0u && (my_link[0] != kInvalid || my_link[1] != kInvalid)) : (uint64_t{1} << items) - 1ull;
+        for (; rest != 0ull; rest &= rest - 1ull) {
             const uint32_t i = uint32_t(__builtin_ctzll(rest));
-            const uint32_t links[2] = {uniform_word(my_link[0], i), uniform_word(my_link[1], i)}, axes = uniform_word(my_axes, i);
-            const uint32_t first_row = uniform_word(my_row, i), stride = uniform_word(my_stride, i), merge = uniform_word(my_merge, i);
-            const V3 point{uniform_value(my_point.x, i), uniform_value(my_point.y, i), uniform_value(my_point.z, i)};
+            const uint32_t links[2] = {read(my_link[0], i), read(my_link[1], i)}, axes = read(my_axes, i);
+            if (G < 64 && (axes == 0u || (links[0] == kInvalid && links[1] == kInvalid))) continue;
+            const uint32_t first_row = read(my_row, i), stride = read(my_stride, i), merge = read(my_merge, i);
+            const V3 point{read_value(my_point.x, i), read_value(my_point.y, i), read_value(my_point.z, i)};
             const V3 arm = cross3(axis_world, sub3(point, origin));
             bool on_path[2];
 #pragma unroll
             for (int side = 0; side < 2; ++side) {
-                const uint64_t mask = (uint64_t(uniform_word(my_mask[side][1], i)) << 32u) | uint64_t(uniform_word(my_mask[side][0], i));
+                const uint64_t mask = (uint64_t(read(my_mask[side][1], i)) << 32u) | uint64_t(read(my_mask[side][0], i));
                 on_path[side] = lane < m.dof && ((mask >> lane) & 1ull) != 0ull;
             }
 #pragma unroll
             for (int axis = 0; axis < kAxes; ++axis) {
                 if (((axes >> axis) & 1u) == 0u) continue;
-                const V3 dir_a{uniform_value(my_dir[axis].x, i), uniform_value(my_dir[axis].y, i), uniform_value(my_dir[axis].z, i)};
+                const V3 dir_a{read_value(my_dir[axis].x, i), read_value(my_dir[axis].y, i), read_value(my_dir[axis].z, i)};
                 float entries[2] = {0.0f, 0.0f};
 #pragma unroll
                 for (int side = 0; side < 2; ++side) {
@@ -1326,11 +1362,11 @@ __global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(kCom
                 // a point whose first row the free velocity drives into is one the solve will have to answer (a compliant row's
                 // right-hand side is still without its damping of the start velocity here)
                 if (axis == 0) {
-                    const float velocity = kCompliant ? fmaf(-p.dt * uniform_value(my_gain[0], i), start_velocity, free_velocity) : free_velocity;
-                    if (uniform_value(my_rhs[0], i) * p.dt > wave_sum((entries[0] + entries[1]) * velocity)) ++driven_points;
+                    const float velocity = kCompliant ? fmaf(-p.dt * read_value(my_gain[0], i), start_velocity, free_velocity) : free_velocity;
+                    if (read_value(my_rhs[0], i) * p.dt > sum_of((entries[0] + entries[1]) * velocity)) ++driven_points;
                 }
                 if constexpr (kCompliant) {
-                    const float gain = uniform_value(my_gain[axis], i);
+                    const float gain = read_value(my_gain[axis], i);
                     if (gain == 0.0f) continue;
                     if (lane < md) {
 #pragma unroll
@@ -1338,7 +1374,7 @@ __global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(kCom
                             terms[(16u * side + staged_terms) * AssembleTermStride(md) + lane] = entries[side] * start_velocity;
                     }
                     if (lane == staged_terms) {
-                        term_row = r; term_rhs = uniform_value(my_rhs[axis], i); term_gain = gain;
+                        term_row = r; term_rhs = read_value(my_rhs[axis], i); term_gain = gain;
                         term_sides[0] = links[0] != kInvalid; term_sides[1] = links[1] != kInvalid;
                     }
                     if (++staged_terms == kTermRows / 2u) add_velocities();
@@ -1351,7 +1387,7 @@ __global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(kCom
     // and upper limit (two a link), dry friction, drive.  Each acts on one coordinate, J = +-e_joint; the rest of
     // its Jacobian row is never written and stays at the zeros it was allocated with.  A MuJoCo-sourced joint gets its
     // limit and friction rows as compliant rows (margin, solref, solimp at the coordinate's reference weight).
-    {
+    if constexpr (G == 64) {
         const uint32_t limit_rows = p.joint_limit_rows_per_env, friction_rows = p.joint_friction_rows_per_env;
         const uint32_t joint_slots = limit_rows + friction_rows + p.joint_drive_rows_per_env;
         const size_t lbase = size_t{env} * nl;
@@ -1434,8 +1470,9 @@ __global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(kCom
             rows[rs] = row;
         }
     }
-    active_rows = uint32_t(wave_sum(float(active_rows)));
-    invalid_endpoint = __any(invalid_endpoint);
+    active_rows = uint32_t(sum_of(float(active_rows)));
+    if constexpr (G == 64) invalid_endpoint = __any(invalid_endpoint);
+    else invalid_endpoint = over_lanes(invalid_endpoint ? 1u : 0u, larger) != 0u;
     if (lane == 0u) {
         d.row_count[env] = active_rows;
         if (d.solver_points != nullptr) d.solver_points[env] = points_expected(d.solver_points[env], driven_points);
@@ -1520,6 +1557,17 @@ Status OpNarrowphaseHeightfield(const ModelView&, const DataView&, const void* p
 }
 
 
+// Eight lanes an environment where they are one for every coordinate and for every place of a point, in worlds under the native
+// laws without joint rows, from a batch on that leaves the machine wavefronts enough: free boxes (six coordinates, one slot of four
+// points), the kernel at 16384 50 us with 64 lanes and 24 with eight; a step of 256 210 and 214 us, of 1024 246 and 246, of 2048 250 and 247,
+// of 4096 313 and 303, of 16384 395 and 367, of 65536 982 and 872.  Thirty-two lanes gain nothing: 4096 quadrupeds (18 coordinates, four slots)
+// 468 and 469, 16384 1220 and 1238.
+constexpr uint32_t kAssembleEightFrom = 2048u;
+static bool AssembleTakesEight(const ModelView& m, const AssembleRowsParams& p) {
+    const uint32_t places = p.union_slot_count * (m.max_points_per_slot == 1u ? 1u : kPointsPerSlot);
+    return m.any_mujoco == 0u && p.joint_limit_rows_per_env + p.joint_friction_rows_per_env + p.joint_drive_rows_per_env == 0u && places <= 8u &&
+        p.max_dof <= 8u && p.env_count >= kAssembleEightFrom;
+}
 Status OpAssembleRows(const ModelView& m, const DataView& d, const void* params, hipStream_t stream) {
     const auto* p = static_cast<const AssembleRowsParams*>(params);
     if (p == nullptr) return Status::Failed;
@@ -1530,6 +1578,10 @@ Status OpAssembleRows(const ModelView& m, const DataView& d, const void* params,
         return Status::InvalidArgument;
     const bool compliant = m.any_mujoco != 0u;
     const size_t lds = size_t{AssembleLdsWords(p->union_slot_count, m.links_per_env, p->max_dof, compliant)} * sizeof(uint32_t);
+    if (AssembleTakesEight(m, *p)) {
+        hipLaunchKernelGGL((AssembleRowsKernel<false, 8>), dim3((p->env_count + 7u) / 8u), dim3(kWave), lds, stream, m, d, *p);
+        return hipGetLastError() == hipSuccess ? Status::Ok : Status::Failed;
+    }
     hipLaunchKernelGGL(compliant ? AssembleRowsKernel<true> : AssembleRowsKernel<false>, dim3(p->env_count), dim3(kWave), lds, stream, m, d, *p);
     return hipGetLastError() == hipSuccess ? Status::Ok : Status::Failed;
 }

@@ -1,5 +1,5 @@
-"""A solve's result is the environment's own, whatever kernel and launch its batch takes: wide blocks two a SIMD, launches of as
-many blocks as the machine holds."""
+"""A step's result is the environment's own, whatever kernels and launches its batch takes: wide blocks two a SIMD, launches of as
+many blocks as the machine holds, row assemblies of eight environments a wavefront."""
 import numpy as np
 import pytest
 
@@ -15,7 +15,7 @@ def repeated(state, E):
     return {name: np.ascontiguousarray(np.asarray(v)[np.arange(E) % len(v)]) for name, v in state.items()}
 
 
-def batches_agree(device, template, desc_of, state, small, large, steps=2):
+def batches_agree(device, template, desc_of, state, small, large, steps=2, fields=FIELDS):
     """The environments of a large batch, the small one's over and over, step as the small one's do, bit for bit."""
     few, many = nk.World(device, template, desc_of(small)), nk.World(device, template, desc_of(large))
     few.set_state(state)
@@ -26,9 +26,9 @@ def batches_agree(device, template, desc_of, state, small, large, steps=2):
     few.synchronize()
     many.synchronize()
     assert (few.download("contact_count") > 0).any()
-    for name in FIELDS:
+    for name in fields:
         a, b = few.download(name).reshape(small, -1), many.download(name).reshape(large, -1)
-        assert np.array_equal(b.view(np.uint32), a.view(np.uint32)[np.arange(large) % small]), name
+        assert np.array_equal(b.view(np.uint8), a.view(np.uint8)[np.arange(large) % small]), name
     blocks = few.info.solver_blocks_per_cu, many.info.solver_blocks_per_cu
     few.close()
     many.close()
@@ -63,3 +63,17 @@ def test_environments_past_the_blocks_held_step_as_the_first(device, index, driv
             if link["joint_type"] == abi.JOINT_REVOLUTE:
                 link["frictionloss"] = 0.1
     batches_agree(device, template, lambda E: abi.world_desc(E, cfg.dt, vel_iters=cfg.vel_iters), cfg.state(), 150, large, steps=3)
+
+
+@pytest.mark.parametrize("large", [2048, 2051])
+def test_boxes_whose_rows_are_assembled_eight_a_wavefront_step_as_alone(device, large):
+    """Four-point manifolds that come and go: some environments have no point, some a few."""
+    cfg = nk.synthetic.config(6, 70)
+    state = cfg.state()
+    state["base_pose"] = state["base_pose"].copy()
+    state["base_pose"][::3, 2] += np.linspace(0.0, 0.03, len(state["base_pose"][::3]), dtype=np.float32)
+    state["base_pose"][1::5, 4] += 0.08
+    state["base_pose"][:, 3:] /= np.linalg.norm(state["base_pose"][:, 3:], axis=1, keepdims=True)
+    batches_agree(device, cfg.template, lambda E: abi.world_desc(E, cfg.dt, vel_iters=cfg.vel_iters), state, 70, large, steps=4,
+                  fields=("lambda", "chain_jacobian", "chain_jacobian_b", "row_penetration", "row_cj_point", "ucontact_count", "row_count",
+                          "contact_material", "body_linear_velocity", "body_angular_velocity", "base_pose", "env_status", "qdot_flat"))
