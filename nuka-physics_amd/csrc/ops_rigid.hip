@@ -151,13 +151,17 @@ __device__ FreeRotation solve_free_rotation(V3 w0, V3 inv_i, float dt) {
     return out;
 }
 
+// A body a lane, a wavefront a workgroup: 16384 bodies in workgroups of four filled 64 of 256 compute units (15.0 us, 10.5 so; the
+// positions, whose registers the larger workgroup bounds, 12.5 and 19.9).
+constexpr uint32_t kBodyThreads = 64u;   // of the velocities
+
 // BodyIntegrateVelocityKernel (articulation.cu:1019-1049): the world inverse inertia at the step's pose, gravity and the
 // applied force on the linear velocity, the applied torque on the angular velocity (`link_wrench`: force and torque
 // about the centre of mass in world axes, cleared here).  Then the block the solve descends on (InitializeRigidBlock,
 // block_descent_rigid.cuh:4-48): the mass matrix diag(m, m, m) with the inverse of the world inverse inertia, its
 // L D L^T factor (FactorMass, articulation_mass.cuh:269-335, right-looking) for the heads' inertial response, and the six
 // coordinates in the link's twist words.
-__global__ void __launch_bounds__(256) BodyIntegrateVelocityKernel(ModelView m, DataView d, IntegrateVelocityParams p, uint32_t env_count) {
+__global__ void __launch_bounds__(kBodyThreads) BodyIntegrateVelocityKernel(ModelView m, DataView d, IntegrateVelocityParams p, uint32_t env_count) {
     const uint32_t env = blockIdx.x * blockDim.x + threadIdx.x;
     if (env >= env_count) return;
     const size_t body = size_t{env} * m.bodies_per_env + m.link_body[0];   // the body's row among the environment's bodies
@@ -275,7 +279,7 @@ __global__ void __launch_bounds__(256) BodyIntegratePositionKernel(ModelView m, 
 Status BodyIntegrateVelocity(const ModelView& m, const DataView& d, const IntegrateVelocityParams& p, hipStream_t stream) {
     if (m.links_per_env != 1u || m.dof != 6u || m.max_dof < 6u || p.articulation_count == 0u) return Status::InvalidArgument;
     const uint32_t E = p.articulation_count;
-    hipLaunchKernelGGL(BodyIntegrateVelocityKernel, dim3((E + 255u) / 256u), dim3(256), 0, stream, m, d, p, E);
+    hipLaunchKernelGGL(BodyIntegrateVelocityKernel, dim3((E + kBodyThreads - 1u) / kBodyThreads), dim3(kBodyThreads), 0, stream, m, d, p, E);
     return hipGetLastError() == hipSuccess ? Status::Ok : Status::Failed;
 }
 Status BodyIntegratePosition(const ModelView& m, const DataView& d, const IntegratePositionParams& p, hipStream_t stream) {
