@@ -294,7 +294,9 @@ __device__ __forceinline__ void store_tile(const TilePlace& place, float* out, c
         if (wide == 1u) {
             if (!kLower || j <= i) out[e] = word(i, j);
         } else if (!kLower || j + 3u <= i) {
-            reinterpret_cast<float4*>(out)[e] = float4{word(i, j), word(i, j + 1u), word(i, j + 2u), word(i, j + 3u)};
+            const float* four = A + i * ld + j;
+            reinterpret_cast<float4*>(out)[e] = n == stride ? float4{four[0], four[1], four[2], four[3]}   // (nothing is past the matrix)
+                                                            : float4{word(i, j), word(i, j + 1u), word(i, j + 2u), word(i, j + 3u)};
         } else {
             for (uint32_t t = 0u; j + t <= i; ++t) out[i * stride + j + t] = word(i, j + t);
         }
@@ -850,10 +852,15 @@ __device__ __forceinline__ void dynamics_of_block(const ModelView& m, const Data
         // compiles to a branch a word)
         const uint32_t ll = local_lane(ml);
         const uint32_t from = (ll < n ? ll : 0u) * ld;
+        if (n == uint32_t(N)) {   // a lane past the matrix holds its first row, which nothing reads
 #pragma unroll
-        for (int k = 0; k < N; ++k) {
-            const float word = w.A[from + (uint32_t(k) < n ? uint32_t(k) : 0u)];
-            row[k] = ll < n && uint32_t(k) < n ? word : (ll == uint32_t(k) ? 1.0f : 0.0f);
+            for (int k = 0; k < N; ++k) row[k] = w.A[from + uint32_t(k)];
+        } else {
+#pragma unroll
+            for (int k = 0; k < N; ++k) {
+                const float word = w.A[from + (uint32_t(k) < n ? uint32_t(k) : 0u)];
+                row[k] = ll < n && uint32_t(k) < n ? word : (ll == uint32_t(k) ? 1.0f : 0.0f);
+            }
         }
     }
     ldlt_pivots<int(kRowLanes), 0>(local_lane(ml), row);
@@ -875,7 +882,7 @@ __device__ __forceinline__ void dynamics_of_block(const ModelView& m, const Data
 #pragma unroll
         for (int i = 0; i < N; ++i) {
             const float word = w.A[(uint32_t(i) < n ? uint32_t(i) : 0u) * ld + (ll < n ? ll : 0u)];
-            col[i] = ll < uint32_t(i) && uint32_t(i) < n ? word : 0.0f;
+            col[i] = uint32_t(i) < n ? word : 0.0f;   // (taken by the lanes ahead of the diagonal alone)
         }
         forward_rows<int(kRowLanes), 0>(ll, n, row, &x);
         if (ll < n) x = x / w.A[ll * ld + ll];

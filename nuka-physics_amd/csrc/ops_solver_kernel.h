@@ -36,7 +36,7 @@ namespace solver {
 //   With NKH_SOLVER_PAIRED defined (ops_solver_p*.hip) it sits in namespace `paired`: wide blocks of contact heads without contact
 // rows (Tile::from_links), two waves a SIMD.  A wide wave alone on its SIMD issues an instruction in less than half of its cycles, whatever
 // it waits for, and what kept a second one away was LDS, 28 KB a block, not registers: 256 hold the sweeps' rows with some
-// eighty values a Newton step in scratch memory.  The build keeps no factor in LDS - the substitution hands its columns round
+// forty values a Newton step in scratch memory.  The build keeps no factor in LDS - the substitution hands its columns round
 // eight at a time (substitute_by_turns) and a Hessian met again is factored again - and no field that such a head has
 // no use for: 20.4 KB, eight blocks a compute unit, and the bits of the plain build (8192 ropes 12.2 -> 9.7 ms a step).
 #ifdef NKH_SOLVER_DENSE
