@@ -1059,8 +1059,11 @@ __global__ void __launch_bounds__(2 * kWave) StepTailKernel(ModelView m, DataVie
 }
 // Where nothing stands between the dynamics and the step's tail, as in a world without rows, the workgroup goes on with its own
 // environments: their state is its own.
+// (Two waves a SIMD at the least, of the five or so that registers allow: a kernel that may have the whole register file gets its matrix
+// products in the half of it that other instructions cannot name, and reads each of them back - 630 of 9500 at 36 coordinates.  65536
+// humanoids 1064 -> 1030 us, 4096 95.1 -> 91.7, 8192 ropes 962 -> 919, 4096 quadrupeds 38.8 -> 38.3.)
 template <int N, int G>
-__global__ void __launch_bounds__(3 * kWave) ArticulationDynamicsKernel(ModelView m, DataView d, ArticulationDynamicsParams p, uint32_t env_count, StepTail t) {
+__global__ void __launch_bounds__(3 * kWave) __attribute__((amdgpu_waves_per_eu(2))) ArticulationDynamicsKernel(ModelView m, DataView d, ArticulationDynamicsParams p, uint32_t env_count, StepTail t) {
     extern __shared__ float lds[];
     dynamics_of_block<N, G>(m, d, p, env_count, lds);
     if (t.runs == 0u) return;
