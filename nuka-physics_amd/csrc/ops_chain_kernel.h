@@ -22,9 +22,10 @@ constexpr uint32_t kChainFrom = 64u;   // environments
 // a link's constants in LDS
 enum ChainWord : uint32_t {
     cRotation = 0u,       // the joint's frame in the parent: nine words, row-major
-    cTurns = 9u,          // 1 where the joint turns, else 0
+    cTurns = 9u,          // whether the joint turns, as a word
     cOffset = 12u,        // ... and its origin
     cSlide = 16u,         // what a slider's coordinate adds to it
+    cSlides = 19u,        // whether it does, as a word
     cAxis = 20u,          // unit axis, zero for none
     cAngular = 24u,       // motion subspace
     cLinear = 28u,
@@ -32,7 +33,6 @@ enum ChainWord : uint32_t {
     cDamping = 53u, cArmature, cStiffness, cReference,
     cQuat = 57u,
     cDof = 61u,           // as a word; kInvalid where the joint has none
-    cType = 62u,
     kChainWords = 64u
 };
 struct ChainMotion { V3 w, v; };                        // angular, linear
@@ -141,13 +141,20 @@ __device__ __forceinline__ void chain_rotation(const float* link, float s, float
 #pragma unroll
     for (int e = 0; e < 9; ++e) r[e] = out[e];
 }
-__device__ __forceinline__ V3 chain_offset(const float* link, float q) { return fma3(chain_vector(link + cSlide), q, chain_vector(link + cOffset)); }
+// A coordinate counts where the joint has a use for it and not otherwise: it is selected, for zero times a word that is not
+// finite is not zero
+__device__ __forceinline__ bool chain_flag(const float* link, uint32_t word) { return __float_as_uint(link[word]) != 0u; }
+__device__ __forceinline__ float chain_angle(const float* link, float q) { return chain_flag(link, cTurns) ? q : 0.0f; }
+__device__ __forceinline__ V3 chain_offset(const float* link, float q) {
+    const V3 origin = chain_vector(link + cOffset), moved = fma3(chain_vector(link + cSlide), q, origin);
+    return chain_flag(link, cSlides) ? moved : origin;
+}
 // joint_relative_frame from the link's constants and the sine and the cosine of half the angle
 __device__ __forceinline__ Xf chain_place(const float* link, float q, float s, float c) {
     Xf place{chain_offset(link, q), Q4{link[cQuat], link[cQuat + 1], link[cQuat + 2], link[cQuat + 3]}};
     const V3 n = chain_vector(link + cAxis);
     const Q4 turned = qnormalize_le(qmul(place.r, Q4{c, n.x * s, n.y * s, n.z * s}), 1.0e-12f);
-    if (link[cTurns] != 0.0f) place.r = turned;
+    if (chain_flag(link, cTurns)) place.r = turned;
     return place;
 }
 // consecutive words of a lane's own, sixteen bytes at a time from any word on
@@ -248,7 +255,8 @@ ChainStepKernel(ModelView m, DataView d, ArticulationDynamicsParams p, uint32_t 
             const V3 subspace = directed ? axis : authored;   // (motion_subspace keeps an axis too short to normalise)
             const V3 angular = type == kRevolute ? subspace : still.w, linear = type == kPrismatic ? subspace : still.w;
             mat3_from_quat(local.r, link + cRotation);
-            link[cTurns] = type == kRevolute && directed ? 1.0f : 0.0f;
+            link[cTurns] = __uint_as_float(type == kRevolute && directed ? 1u : 0u);
+            link[cSlides] = __uint_as_float(type == kPrismatic ? 1u : 0u);
             const auto put = [&](uint32_t at, V3 v) { link[at] = v.x; link[at + 1u] = v.y; link[at + 2u] = v.z; };
             put(cOffset, offset); put(cSlide, slide); put(cAxis, axis); put(cAngular, angular); put(cLinear, linear);
             const float* inertia = m.link_inertia + 36u * lane;
@@ -286,7 +294,7 @@ ChainStepKernel(ModelView m, DataView d, ArticulationDynamicsParams p, uint32_t 
     for (uint32_t l = wave; l < nl; l += kChainWaves) {
         const float* link = links + l * kChainWords;
         float s, c, r[9];
-        sincosf(link[cTurns] * q[l * kWave], &s, &c);
+        sincosf(chain_angle(link, q[l * kWave]), &s, &c);
         chain_rotation(link, s, c, r);
 #pragma unroll
         for (int e = 0; e < 9; ++e) rotation[(l * 9u + uint32_t(e)) * kWave] = r[e];
@@ -459,7 +467,7 @@ ChainStepKernel(ModelView m, DataView d, ArticulationDynamicsParams p, uint32_t 
         const bool moves = dof != kInvalid && p.integrate_velocity != 0u;   // uniform
         if (moves) rate = fmaf(dt, solved, rate);
         const float to = fmaf(tail.integrate.pos_pass != 0u ? rate + d.qdot_pseudo[lbase + l] : rate, tail.integrate.dt, q[l * kWave]);
-        const float angle = links[l * kChainWords + cTurns] * to;
+        const float angle = chain_angle(links + l * kChainWords, to);
         float s, c, half_s, half_c;
         sincosf(angle, &s, &c);
         sincosf(0.5f * angle, &half_s, &half_c);

@@ -69,3 +69,41 @@ def test_a_chain_steps_like_the_ops_and_as_near_the_double_step(oracle_py, devic
             scale = np.linalg.norm(double[name]) + 1e-30
             mine, general = np.linalg.norm(step[name] - double[name]) / scale, np.linalg.norm(ops[name] - double[name]) / scale
             assert mine <= max(1.5 * general, 5e-7), (name, mine, general)
+
+
+@pytest.mark.parametrize("kinds", [(R, F, P, R, F), (F, P, R, F, R, R, P, F)])
+def test_a_coordinate_counts_where_its_joint_has_a_use_for_it(device, kinds):
+    """A fixed link's coordinate that is not finite reaches its own word and nothing else; a joint's reaches what it reaches in the
+    general kernels' ops."""
+    E, links = 70, len(kinds)
+    g = np.random.default_rng(links)
+    t = chain(links, kinds, g)
+    jointed = np.array([kind != F for kind in kinds])
+    state = {name: (g.normal(0.0, sigma, (E, links)) * jointed).astype(np.float32) for name, sigma in (("q", 1.0), ("qdot", 1.0), ("tau", 2.0))}
+    base = np.zeros((E, 7), np.float32)
+    base[:, 3] = 1.0
+    state.update(base_pose=base, root_twist=np.zeros((E, 6), np.float32))
+    fixed, moving = np.flatnonzero(~jointed), np.flatnonzero(jointed)
+    for env, value in ((3, np.nan), (5, np.inf), (9, -np.inf), (69, np.nan)):
+        state["q"][env, fixed] = value
+    for k, link in enumerate(moving):
+        state["q"][20 + 2 * k, link], state["q"][21 + 2 * k, link] = np.inf, np.nan
+    out = []
+    for kind in ("ops", "step"):
+        w = nk.World(device, t, abi.world_desc(E, 1.0 / 240.0))
+        w.set_state(state)
+        if kind == "ops":
+            for op in OPS:
+                w.op(op)
+        else:
+            w.step()
+        w.synchronize()
+        out.append({name: w.download(name).astype(np.float64).reshape(E, -1) for name in FIELDS})
+        w.close()
+    ops, step = out
+    for name in FIELDS:
+        assert np.array_equal(np.isfinite(step[name]), np.isfinite(ops[name])), name
+        unused = np.zeros(links, bool) if name != "q" else ~jointed
+        assert np.isfinite(step[name][[3, 5, 9, 69]][:, ~np.resize(unused, step[name].shape[1])]).all(), name
+        whole = np.isfinite(ops[name])
+        assert relative_error(step[name][whole], ops[name][whole]) <= 1e-5, name
