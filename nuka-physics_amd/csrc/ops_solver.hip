@@ -346,7 +346,7 @@ uint32_t SolverBlocksPerUnit(const ModelView& m, uint32_t env_count) {
 uint32_t SolverMassFactorFloats(const ModelView& m) {
     if (m.rows_per_env == 0u || m.dof == 0u) return 0u;
     const uint32_t width = SolverSweepWidth(m);
-    return solver::MassFactorInMemory(width) ? solver::MassFactorFloats(solver::PaddedWidth(width)) : 0u;
+    return solver::MassFactorInMemory(width) ? solver::FactorFloats(solver::PaddedWidth(width)) : 0u;
 }
 uint32_t SolverSweepWidth(const ModelView& m) {
     if (m.rows_per_env == 0u || m.dof == 0u) return m.dof;

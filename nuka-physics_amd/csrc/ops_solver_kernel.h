@@ -700,29 +700,39 @@ __device__ __forceinline__ void load_rows(const float* a, uint32_t lane, float (
 #pragma unroll
     for (int k = 0; k < N; ++k) row[k] = diagonal[max(k - int(from), 0)];
 }
-// A leaves-first factor in device memory four columns at a time, the rows down to the diagonal side by side: words that
-// neighbouring lanes read and write together, sixteen bytes a lane.  (Rows one after the other, packed, are 64 words of 64
-// different lines a lane; with them and the transposed reads the mass solves were a tenth of the solve of 8192 ropes.)
-__host__ __device__ constexpr uint32_t quads_before(uint32_t q) { return 8u * q * (q + 1u); }
+// A leaves-first factor in device memory four columns at a time, its rows side by side: words that neighbouring lanes read and
+// write together, sixteen bytes a lane.  (Rows one after the other, packed, are 64 words of 64 different lines a lane; with them
+// and the transposed reads the mass solves were a tenth of the solve of 8192 ropes.)  It takes no more words than the
+// packed rows, whose room a caller gives: a quad's last two rows hold one entry between them, which goes behind all of them
+// with four zeros that the lanes past a quad's rows read.
+__host__ __device__ constexpr uint32_t quads_before(uint32_t q) { return 8u * q * q; }   // 4 q + 2 rows of four words a quad
 template <int N>
 __device__ __forceinline__ void store_quads(float* a, uint32_t lane, const float (&row)[N]) {
+    static_assert(quads_before(N / 4) + 4u + N / 4 <= FactorFloats(N), "no more than the packed rows");
     lane = local_lane(lane);
+    float last = 0.0f;   // of a quad's third row, its entry
 #pragma unroll
-    for (int q = 0; q < N / 4; ++q)
-        if (lane <= 4u * uint32_t(q) + 3u)
-            reinterpret_cast<float4*>(a + quads_before(uint32_t(q)))[lane] = float4{row[4 * q], row[4 * q + 1], row[4 * q + 2], row[4 * q + 3]};
+    for (int q = 0; q < N / 4; ++q) {
+        const float4 words{row[4 * q], row[4 * q + 1], row[4 * q + 2], row[4 * q + 3]};
+        if (lane <= 4u * uint32_t(q) + 1u) reinterpret_cast<float4*>(a + quads_before(uint32_t(q)))[lane] = words;
+        last = lane == 4u * uint32_t(q) + 2u ? words.w : last;
+    }
+    float* behind = a + quads_before(uint32_t(N / 4));
+    if (lane < 4u) behind[lane] = 0.0f;
+    if ((lane & 3u) == 2u && lane < uint32_t(N)) behind[4u + lane / 4u] = last;
 }
 template <int N>
 __device__ __forceinline__ void load_quads(const float* a, uint32_t lane, float (&row)[N]) {
     lane = local_lane(lane);
+    const float last = a[quads_before(uint32_t(N / 4)) + 4u + min(lane, uint32_t(N - 1)) / 4u];
+    const float4* words = reinterpret_cast<const float4*>(a);
 #pragma unroll
-    for (int q = 0; q < N / 4; ++q) {   // lanes below the diagonal read the last row's words, zeros
-        const float4 w = reinterpret_cast<const float4*>(a + quads_before(uint32_t(q)))[min(lane, 4u * uint32_t(q) + 3u)];
-        row[4 * q] = w.x; row[4 * q + 1] = w.y; row[4 * q + 2] = w.z; row[4 * q + 3] = w.w;
+    for (int q = 0; q < N / 4; ++q) {
+        const float4 w = words[lane <= 4u * uint32_t(q) + 1u ? quads_before(uint32_t(q)) / 4u + lane : quads_before(uint32_t(N / 4)) / 4u];
+        row[4 * q] = w.x; row[4 * q + 1] = w.y; row[4 * q + 2] = w.z;
+        row[4 * q + 3] = lane == 4u * uint32_t(q) + 2u ? last : w.w;
     }
 }
-// words of device memory an environment's mass factor takes in a wide block, by rows or by fours
-__host__ __device__ constexpr uint32_t MassFactorFloats(uint32_t N) { return FactorFloats(N) > quads_before(N / 4u) ? FactorFloats(N) : quads_before(N / 4u); }
 template <int N>
 __device__ __forceinline__ void load_columns(const float* a, uint32_t lane, float (&col)[N]) {
     lane = local_lane(lane);
@@ -2956,7 +2966,7 @@ environment:
     PROF_BEGIN(c, 9);
     PROF_BEGIN(c, 0);
     if constexpr (W > kTwoWaveWidth) {
-        c.mfac = d.solver_mass_factor + size_t{env} * MassFactorFloats(uint32_t(W));
+        c.mfac = d.solver_mass_factor + size_t{env} * FactorFloats(uint32_t(W));
         c.hfac = lds;
     } else {
         c.mfac = lds;

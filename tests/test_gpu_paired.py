@@ -47,6 +47,29 @@ def test_wide_trees_two_a_simd_step_as_one_a_simd(oracle_py, device, dof, floati
     assert blocks[0] <= 4 < blocks[1]
 
 
+@pytest.mark.parametrize("dof,large", [(40, 2049), (44, 2049), (64, 2049), (64, 70)])
+def test_a_wide_blocks_mass_factor_takes_the_packed_rows_room(oracle_py, device, dof, large):
+    """n (n + 1) / 2 words of the padded width, a multiple of four: what a caller that binds its own memory gives for it, whichever
+    build solves.  The paired build's words past its factor stay as they are."""
+    tree, _, state = tree_case(oracle_py, dof, True, True, seed=5 * dof, E=48, limb_joints=3)
+    w = nk.World(device, tree.template, abi.world_desc(large, 1.0 / 240.0, vel_iters=2))
+    room = (dof * (dof + 1) // 2 + 3) // 4 * 4
+    assert w.download("solver_mass_factor").size == large * room
+    assert (w.info.solver_blocks_per_cu > 4) == (large >= 2048)
+    words = np.full((large, room), 7.0, np.float32)
+    w.upload("solver_mass_factor", words)
+    w.set_state(repeated(state, large))
+    w.step()
+    w.synchronize()
+    words = w.download("solver_mass_factor").reshape(large, room)
+    if large >= 2048:   # 8 quads^2 words by fours, four zeros, a word a quad
+        quads = dof // 4
+        used = 8 * quads * quads + 4 + quads
+        assert (words[:, used:] == 7.0).all() and not (words[:, :used] == 7.0).any()
+        assert not words[:, 8 * quads * quads:8 * quads * quads + 4].any()
+    w.close()
+
+
 def test_ropes_two_a_simd_step_as_one_a_simd(device):
     cfg = nk.synthetic.config(5, 64)
     blocks = batches_agree(device, cfg.template, lambda E: abi.world_desc(E, cfg.dt, vel_iters=cfg.vel_iters), cfg.state(), 64, 2111)
