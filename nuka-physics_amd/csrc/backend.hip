@@ -235,10 +235,16 @@ Status DispatchNext(Backend* be, const ModelView& m, const DataView& d, const nu
     return DispatchOn(be, m, d, calls[0]);
 }
 
+// A host's view: what its storage holds in the queue's place, which is no field, is not handed to a kernel.
+DataView HostView(const nuka_phi_data_view* d) {
+    DataView data = *reinterpret_cast<const DataView*>(d);
+    data.solver_queue = nullptr;
+    return data;
+}
+
 uint8_t BeDispatch(nuka_phi_backend* b, const nuka_phi_model_view* m, const nuka_phi_data_view* d, const nuka_phi_op_call* call) {
     if (b == nullptr || m == nullptr || d == nullptr || call == nullptr) return uint8_t(Status::InvalidArgument);
-    return uint8_t(DispatchOn(reinterpret_cast<Backend*>(b), *reinterpret_cast<const ModelView*>(m),
-                              *reinterpret_cast<const DataView*>(d), *call));
+    return uint8_t(DispatchOn(reinterpret_cast<Backend*>(b), *reinterpret_cast<const ModelView*>(m), HostView(d), *call));
 }
 
 uint8_t BeSynchronize(nuka_phi_backend* b, nuka_phi_execution_error* error) {
@@ -272,13 +278,7 @@ uint32_t DirectKernels(hipGraph_t graph, hipKernelNodeParams (&kernels)[2]) {
 
 // A plan is the op list captured once into a HIP graph on the backend's stream (cuda_backend.cu:245-361).  Ops
 // launch kernels only - no memsets or allocations - so the captured graph holds kernel nodes alone.
-nuka_phi_plan* BePlanCreate(nuka_phi_backend* b, const nuka_phi_model_view* m, const nuka_phi_data_view* d,
-                            const nuka_phi_op_call* calls, int n_calls, nuka_phi_execution_error* error) {
-    auto* be = reinterpret_cast<Backend*>(b);
-    if (m == nullptr || d == nullptr || calls == nullptr || n_calls <= 0) {
-        Fail(error, Status::InvalidArgument, uint16_t(NkOp::Count), 0, "plan_create: empty op list");
-        return nullptr;
-    }
+Plan* CreatePlan(Backend* be, const ModelView& model, const DataView& data, const nuka_phi_op_call* calls, int n_calls, nuka_phi_execution_error* error) {
     for (int i = 0; i < n_calls; ++i)
         if (calls[i].op >= uint16_t(NkOp::Count) || g_ops[calls[i].op] == nullptr) {
             Fail(error, Status::Unsupported, calls[i].op, 0, "plan_create: op not supported by the HIP backend");
@@ -288,8 +288,6 @@ nuka_phi_plan* BePlanCreate(nuka_phi_backend* b, const nuka_phi_model_view* m, c
     if (e != hipSuccess) { Fail(error, Status::Failed, uint16_t(NkOp::Count), int(e), hipGetErrorString(e)); return nullptr; }
     Status status = Status::Ok;
     uint16_t failed = uint16_t(NkOp::Count);
-    const ModelView& model = *reinterpret_cast<const ModelView*>(m);
-    const DataView& data = *reinterpret_cast<const DataView*>(d);
     for (int i = 0, served = 0; i < n_calls && status == Status::Ok; i += served) {
         status = DispatchNext(be, model, data, calls + i, n_calls - i, &served);
         if (status != Status::Ok) failed = calls[i].op;
@@ -314,7 +312,15 @@ nuka_phi_plan* BePlanCreate(nuka_phi_backend* b, const nuka_phi_model_view* m, c
     auto* plan = new Plan{graph, exec, nodes, n_calls, {}, 0u};
     plan->direct_count = DirectKernels(graph, plan->direct);
     (void)hipGetLastError();
-    return reinterpret_cast<nuka_phi_plan*>(plan);
+    return plan;
+}
+nuka_phi_plan* BePlanCreate(nuka_phi_backend* b, const nuka_phi_model_view* m, const nuka_phi_data_view* d,
+                            const nuka_phi_op_call* calls, int n_calls, nuka_phi_execution_error* error) {
+    if (m == nullptr || d == nullptr || calls == nullptr || n_calls <= 0) {
+        Fail(error, Status::InvalidArgument, uint16_t(NkOp::Count), 0, "plan_create: empty op list");
+        return nullptr;
+    }
+    return reinterpret_cast<nuka_phi_plan*>(CreatePlan(reinterpret_cast<Backend*>(b), *reinterpret_cast<const ModelView*>(m), HostView(d), calls, n_calls, error));
 }
 
 uint8_t BePlanExecute(nuka_phi_backend* b, nuka_phi_plan* p, nuka_phi_execution_error* error) {
@@ -460,6 +466,9 @@ void* CreateBackend(int device, void* borrowed_stream) {
 
 Status BackendDispatchNext(void* backend, const ModelView& m, const DataView& d, const nuka_phi_op_call* calls, int n, int* served) {
     return DispatchNext(static_cast<Backend*>(backend), m, d, calls, n, served);
+}
+nuka_phi_plan* BackendPlanCreate(void* backend, const ModelView& m, const DataView& d, const nuka_phi_op_call* calls, int n, nuka_phi_execution_error* error) {
+    return reinterpret_cast<nuka_phi_plan*>(CreatePlan(static_cast<Backend*>(backend), m, d, calls, n, error));
 }
 hipStream_t BackendStream(void* backend) { return static_cast<Backend*>(backend)->stream; }
 nuka_phi_buffer_type* BackendDeviceBufferType(void* backend) { return reinterpret_cast<nuka_phi_buffer_type*>(&static_cast<Backend*>(backend)->device_type); }

@@ -175,7 +175,7 @@ struct DataView {
     uint32_t *solver_points;                // the points an environment's solves answer, which the order goes by in a new state (solve_cost, nk_device_math.h); may be left out
     uint32_t *row_unit;                     // per row: the one coordinate a single-coordinate row acts on, ~0u otherwise
     float *row_unit_value;                  // its Jacobian entry there
-    uint32_t *solver_queue;                 // one word: places of tile_order a solve's launch has handed out; not a field, may be left out
+    uint32_t *solver_queue;                 // one word: places of tile_order a solve's launch has handed out; a world's own, no field: not taken from a host's storage
     // sums over the substeps of one step (fields.yaml:627-632), written by AccumulateStep
     uint32_t *step_env_status;
     float *step_link_impulse, *step_link_moment, *step_joint_limit_impulse;

@@ -760,8 +760,7 @@ nuka_result_t PreparePlan(World& w) {
     if (w.plan != nullptr) return NUKA_RESULT_OK;
     nuka_phi_execution_error error{};
     ++w.capture_attempts;
-    w.plan = w.be->plan_create(w.backend, reinterpret_cast<const nuka_phi_model_view*>(&w.model),
-                               reinterpret_cast<const nuka_phi_data_view*>(&w.data), w.calls.data(), int(w.calls.size()), &error);
+    w.plan = BackendPlanCreate(w.device->backend, w.model, w.data, w.calls.data(), int(w.calls.size()), &error);
     if (w.plan == nullptr) { w.last_error = error; return Error(MapStatus(error.status), std::string("graph capture failed: ") + error.message); }
     return NUKA_RESULT_OK;
 }
