@@ -210,10 +210,13 @@ const SolverKernel kQueueKernels[] = {BlockDescentTileKernel<4, false, 4, false,
 const SolverKernel kPairedKernels[] = {paired::BlockDescentTileKernel<40, true>, paired::BlockDescentTileKernel<44, true>, paired::BlockDescentTileKernel<48, true>,
                                        paired::BlockDescentTileKernel<52, true>, paired::BlockDescentTileKernel<56, true>, paired::BlockDescentTileKernel<60, true>,
                                        paired::BlockDescentTileKernel<64, true>};
-// Batches from this many environments on take a paired kernel where there is one: as many as it holds at once.  Below, an
-// environment with a SIMD to itself is over sooner (ropes, the plain and the paired kernel: 1024 2.36 and 2.53 ms a step, 1536 2.85
-// and 3.08, 1792 3.03 and 3.10, 2048 3.33 and 3.23, 4096 6.22 and 5.08, 8192 12.22 and 9.90).
-constexpr uint32_t kPairedBatch = 2048u;
+// Batches from this many environments on take a paired kernel where there is one.  Below, an environment with a SIMD to itself is over
+// sooner.  With as many heads as coordinates or more it is as many as the machine holds at once that way: ropes of 40 to 64 links, all of them
+// on the ground, take 0.83 to 0.85 of the plain kernel's step for 2048, 0.87 to 0.92 for 3072 (64 links: 1024 2.36 and 2.53 ms, plain and
+// paired, 1536 2.85 and 3.08, 2048 3.33 and 3.23 in steps in a row, 8192 12.22 and 9.90).  With fewer, a block is a shorter one and waits less
+// for its matrix products: 26 trees of 37 to 64 coordinates and 2 to 40 heads take 0.83 to 1.18 of the plain kernel's step for 2048, 0.74 to
+// 1.07 for 3072, the plain kernel's third round, and 0.77 to 0.96 for 3328.
+constexpr uint32_t kPairedBatch = 2048u, kPairedFewHeads = 3328u;
 // Compute units, and the rounds of environments over them from which launches of fewer heads pay (OpBlockDescentSolve).
 constexpr size_t kUnits = 256u, kManyRounds = 9u;
 }  // namespace
@@ -275,14 +278,14 @@ static uint32_t SolverWorkingWidth(const ModelView& m, Heads heads) {
 }
 // The kernel of a world's solve, the same with a queue, where there is one, and how many of its waves share a SIMD
 struct ChosenKernel { SolverKernel kernel, queue; int waves; bool paired; };
-static ChosenKernel KernelOfWidth(const ModelView& m, Heads heads, uint32_t width, uint32_t env_count) {
+static ChosenKernel KernelOfWidth(const ModelView& m, Heads heads, uint32_t width, uint32_t env_count, uint32_t staged) {
     const uint32_t padded = solver::PaddedWidth(m.dof);
     const int waves = solver::WavesPerSimd(int(solver::PaddedWidth(width)));
     if (heads == kContactHeads && env_count >= kDenseBatch)
         for (const ReducedKernel& dense : kDenseKernels)
             if (dense.width == padded && dense.reduced == solver::PaddedWidth(width) && (width == m.dof || dense.reduced == width))
                 return {dense.kernel, dense.queue, solver::DenseWavesPerSimd(int(dense.reduced)), false};
-    if (width == m.dof && env_count >= kPairedBatch && solver::RowsFromLinks(width, heads == kContactHeads, m.rows_from_links))
+    if (width == m.dof && env_count >= (staged >= m.dof ? kPairedBatch : kPairedFewHeads) && solver::RowsFromLinks(width, heads == kContactHeads, m.rows_from_links))
         return {kPairedKernels[padded / 4u - 10u], nullptr, 2, true};
     if (width != m.dof) {
         static_assert(sizeof(kReducedKernels) == sizeof(kEllipticKernels), "the same pairs of widths");
@@ -335,7 +338,7 @@ uint32_t SolverBlocksPerUnit(const ModelView& m, uint32_t env_count) {
         }
         return uint32_t(std::max(blocks, 0));
     }
-    const ChosenKernel chosen = KernelOfWidth(m, heads, width, env_count);
+    const ChosenKernel chosen = KernelOfWidth(m, heads, width, env_count, staged);
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, reinterpret_cast<const void*>(chosen.kernel), solver::kWave,
                                                      BlockLdsBytes(m, heads, width, chosen, staged)) != hipSuccess) {
         (void)hipGetLastError();
@@ -365,7 +368,7 @@ Status OpBlockDescentSolve(const ModelView& m, const DataView& d, const void* pa
     const uint32_t joint_heads = m.joint_limit_rows + m.joint_friction_rows + m.joint_drive_rows;
     const Heads heads = HeadsOf(m, staged);
     const uint32_t width = SolverWorkingWidth(m, heads);
-    const ChosenKernel chosen = KernelOfWidth(m, heads, width, p->env_count);
+    const ChosenKernel chosen = KernelOfWidth(m, heads, width, p->env_count, staged);
     const SolverKernel kernel = chosen.kernel;
     const auto lds_bytes = [&](uint32_t contact_heads) { return BlockLdsBytes(m, heads, width, chosen, contact_heads); };
     // blocks a compute unit holds at most, whatever their LDS: four a wave of a SIMD

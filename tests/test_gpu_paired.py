@@ -41,13 +41,13 @@ def batches_agree(device, template, desc_of, state, small, large, steps=2, field
 ])
 def test_wide_trees_two_a_simd_step_as_one_a_simd(oracle_py, device, dof, floating, branched, limb_joints):
     """Every padded width, with coordinates that fill it and that do not, ways and heads that are runs of lanes and that are not."""
-    small, large = 48, 2049
+    small, large = 48, 3329   # (fewer heads than coordinates: paired from 3328 environments on)
     tree, _, state = tree_case(oracle_py, dof, floating, branched, seed=5 * dof, E=small, limb_joints=limb_joints)
     blocks = batches_agree(device, tree.template, lambda E: abi.world_desc(E, 1.0 / 240.0, vel_iters=6), state, small, large)
     assert blocks[0] <= 4 < blocks[1]
 
 
-@pytest.mark.parametrize("dof,large", [(40, 2049), (44, 2049), (64, 2049), (64, 70)])
+@pytest.mark.parametrize("dof,large", [(40, 3328), (44, 3333), (64, 3329), (64, 3327)])
 def test_a_wide_blocks_mass_factor_takes_the_packed_rows_room(oracle_py, device, dof, large):
     """n (n + 1) / 2 words of the padded width, a multiple of four: what a caller that binds its own memory gives for it, whichever
     build solves.  The paired build's words past its factor stay as they are."""
@@ -55,14 +55,14 @@ def test_a_wide_blocks_mass_factor_takes_the_packed_rows_room(oracle_py, device,
     w = nk.World(device, tree.template, abi.world_desc(large, 1.0 / 240.0, vel_iters=2))
     room = (dof * (dof + 1) // 2 + 3) // 4 * 4
     assert w.download("solver_mass_factor").size == large * room
-    assert (w.info.solver_blocks_per_cu > 4) == (large >= 2048)
+    assert (w.info.solver_blocks_per_cu > 4) == (large >= 3328)
     words = np.full((large, room), 7.0, np.float32)
     w.upload("solver_mass_factor", words)
     w.set_state(repeated(state, large))
     w.step()
     w.synchronize()
     words = w.download("solver_mass_factor").reshape(large, room)
-    if large >= 2048:   # 8 quads^2 words by fours, four zeros, a word a quad
+    if large >= 3328:   # 8 quads^2 words by fours, four zeros, a word a quad
         quads = dof // 4
         used = 8 * quads * quads + 4 + quads
         assert (words[:, used:] == 7.0).all() and not (words[:, :used] == 7.0).any()
@@ -70,10 +70,12 @@ def test_a_wide_blocks_mass_factor_takes_the_packed_rows_room(oracle_py, device,
     w.close()
 
 
-def test_ropes_two_a_simd_step_as_one_a_simd(device):
+@pytest.mark.parametrize("large,held", [(2111, 8), (2047, 4)])
+def test_ropes_two_a_simd_step_as_one_a_simd(device, large, held):
+    """As many heads as coordinates: paired from 2048 environments on."""
     cfg = nk.synthetic.config(5, 64)
-    blocks = batches_agree(device, cfg.template, lambda E: abi.world_desc(E, cfg.dt, vel_iters=cfg.vel_iters), cfg.state(), 64, 2111)
-    assert blocks == (4, 8)
+    blocks = batches_agree(device, cfg.template, lambda E: abi.world_desc(E, cfg.dt, vel_iters=cfg.vel_iters), cfg.state(), 64, large)
+    assert blocks == (4, held)
 
 
 @pytest.mark.parametrize("index,driven,large", [(2, False, 2049), (2, False, 6144 + 1), (3, False, 2600), (3, True, 1900)])
