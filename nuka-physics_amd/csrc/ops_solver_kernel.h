@@ -1568,6 +1568,20 @@ struct FourUnits {
 };
 // Blocks that keep no contact rows (Tile::from_links).  Entry j of a head's row is s_j . w where j lies on the head's
 // way to the root, s_j the coordinate's motion axis (Tile::axes) and w the row's wrench (Tile::wrench); elsewhere zero.
+// columns 4 Q .. on: their coordinates' axes, transposed, against the lane's own weights
+template <int Q, int N>
+__device__ __forceinline__ void add_motions(uint32_t on_low, uint32_t on_high, const Vec4& first, const Vec4& last, const float* x, Vec4& low, Vec4& high) {
+    if constexpr (Q < N / 4) {
+        const Vec4 xs = reinterpret_cast<const Vec4*>(x)[Q];
+#pragma unroll
+        for (uint32_t t = 0u; t < 4u; ++t) {
+            const float on = kept_if(Q < 8 ? on_low : on_high, (4u * uint32_t(Q) + t) & 31u, xs[t]);
+            low = __builtin_amdgcn_mfma_f32_4x4x1f32(first[t], on, low, 4, Q, 0);
+            high = __builtin_amdgcn_mfma_f32_4x4x1f32(last[t], on, high, 4, Q, 0);   // (and two components nobody reads)
+        }
+        add_motions<Q + 1, N>(on_low, on_high, first, last, x, low, high);
+    }
+}
 // lane = head: the motion of the head's link, sum over the coordinates j on its way of s_j x_j, for a vector x in LDS.
 template <int N>
 __device__ __forceinline__ void link_motion(const Tile& c, uint64_t way, const float* x, float (&motion)[6]) {
@@ -1582,24 +1596,15 @@ __device__ __forceinline__ void link_motion(const Tile& c, uint64_t way, const f
         return;
     }
     // Every lane of the wavefront, those without a head with a way of none: v_mfma_f32_4x4x1 takes a coordinate's axis, a
-    // component a lane of four, against the lane's own weight, and register r of a lane is the sum of component r.
-    const float* words = c.axes + (c.lane & 3u);
-    const Vec4* x4 = reinterpret_cast<const Vec4*>(x);
-    const uint32_t on_low = uint32_t(way), on_high = uint32_t(way >> 32u);
+    // component a lane of four, against the lane's own weight, and register r of a lane is the sum of component r.  (The axes word by
+    // word from the table in LDS: 2048 trees of 64 coordinates in limbs of three 1938 us a step, as it is 1793.)
+    const FourUnits units(c.lane);
+    const float4* table = reinterpret_cast<const float4*>(c.axes);
+    const float4 a = table[3u * c.lane], b = table[3u * c.lane + 1u];
+    const float four[4] = {a.x, a.y, a.z, a.w}, two[4] = {b.x, b.y, 0.0f, 0.0f};
+    const Vec4 first = units.transposed(four), last = units.transposed(two);
     Vec4 low = {}, high = {};
-    // a loop that stays a loop: unrolled, all of the table is fetched ahead of the first product, into registers the
-    // block does not have
-#pragma unroll 2
-    for (uint32_t q = 0u; q < uint32_t(N / 4); ++q) {
-        const Vec4 xs = x4[q];
-        const uint32_t four = q < 8u ? on_low >> (4u * q) : on_high >> (4u * q - 32u);
-#pragma unroll
-        for (uint32_t t = 0u; t < 4u; ++t) {
-            const float on = kept_if(four, t, xs[t]);
-            low = __builtin_amdgcn_mfma_f32_4x4x1f32(words[12u * (4u * q + t)], on, low, 0, 0, 0);
-            high = __builtin_amdgcn_mfma_f32_4x4x1f32(words[12u * (4u * q + t) + 4u], on, high, 0, 0, 0);   // (and two components nobody reads)
-        }
-    }
+    add_motions<0, N>(opaque_word(uint32_t(way)), opaque_word(uint32_t(way >> 32u)), first, last, x, low, high);
     motion[0] = low[0]; motion[1] = low[1]; motion[2] = low[2]; motion[3] = low[3]; motion[4] = high[0]; motion[5] = high[1];
 }
 // lane = head: row `axis` of head h times the vector whose link motion is `motion`
