@@ -107,3 +107,41 @@ def test_a_coordinate_counts_where_its_joint_has_a_use_for_it(device, kinds):
         assert np.isfinite(step[name][[3, 5, 9, 69]][:, ~np.resize(unused, step[name].shape[1])]).all(), name
         whole = np.isfinite(ops[name])
         assert relative_error(step[name][whole], ops[name][whole]) <= 1e-5, name
+
+
+@pytest.mark.parametrize("bodies", [3, 70, 300])
+def test_a_chains_bodies_follow_their_links(device, bodies):
+    """Rows that follow a link as they are, from a place of their own on it, and rows that stand still, more of them than lanes and than
+    a workgroup has: the ops' poses, and the cooked ones where nothing moves."""
+    E, links = 70, 5
+    g = np.random.default_rng(bodies)
+    t = chain(links, (R, P, F, R), g)
+    roles = g.integers(0, 3, bodies)
+    for role in roles:
+        place = dict(kind=abi.SHAPE_SPHERE, params=(0.1, 0, 0, 0), local_pos=tuple(g.normal(size=3)), contype=0, conaffinity=0)
+        if role == 0:
+            t.add_body(abi.ROLE_STATIC, **place)
+        else:
+            t.add_body(abi.ROLE_PROXY, link=int(g.integers(links)), **place)
+    jointed = np.array([link["joint_type"] != F for link in t.links])
+    state = {name: (g.normal(0.0, 1.0, (E, links)) * jointed).astype(np.float32) for name in ("q", "qdot", "tau")}
+    base = np.zeros((E, 7), np.float32)
+    base[:, 3] = 1.0
+    state.update(base_pose=base, root_twist=np.zeros((E, 6), np.float32))
+    out = []
+    for kind in ("ops", "step"):
+        w = nk.World(device, t, abi.world_desc(E, 1.0 / 240.0))
+        w.set_state(state)
+        before = w.download("body_pose").reshape(E, -1, 7)
+        if kind == "ops":
+            for op in OPS:
+                w.op(op)
+        else:
+            w.step()
+        w.synchronize()
+        out.append(w.download("body_pose").reshape(E, -1, 7).astype(np.float64))
+        w.close()
+    ops, step = out
+    still = np.concatenate([np.zeros(links, bool), roles == 0])
+    assert np.array_equal(step[:, still], before[:, still]) and not np.array_equal(step[:, ~still], before[:, ~still])
+    assert relative_error(step, ops) <= 1e-5
