@@ -15,9 +15,11 @@
 // (X = [[E, 0], [-E t x, E]]) and inertias kept symmetric, half the instructions of the general kernel's products; the results
 // differ from its in their last places and lie as near a double-precision step.
 constexpr uint32_t kChainLinks = 8u;
-// From a wavefront's lanes full on: the kernel takes as long for one environment as for sixty-four (the step's launch for 64 arms of
-// eight links 21.7 us by the general kernel, 19.7 by this one; for 20011, with the tail's own launch, 76.5 and 28.0).
-constexpr uint32_t kChainFrom = 64u;   // environments
+// From so many environments on: the kernel takes as long for one of them as for sixty-four, so that no fewer are worth it, and a longer
+// chain is a longer walk for its one lane while the general kernel's lanes still fill an idle machine (a step, general kernel and this one:
+// five links, 64 environments 21.4 and 19.1 us; six, 64 22.6 and 21.5, 256 22.2 and 21.8; seven, 64 23.9 and 24.0, 256 23.4 and 24.3, 320
+// 24.8 and 24.3; eight, 64 25.1 and 26.5, 512 26.0 and 27.1, 576 27.8 and 27.1, 1024 29.4 and 27.3).
+__host__ __device__ constexpr uint32_t ChainFrom(uint32_t links) { return links <= 6u ? 64u : 256u * (links - 6u) + 1u; }
 
 // a link's constants in LDS
 enum ChainWord : uint32_t {

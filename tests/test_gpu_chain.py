@@ -1,5 +1,6 @@
-"""Serial chains of up to eight links without rows, a lane an environment: a step against the general kernels' ops and, with
-them, against the double-precision oracle."""
+"""Serial chains of up to eight links without rows, a lane an environment from a batch on: a step against the general kernels' ops
+and, with them, against the double-precision oracle.  The one-lane walk's results are its own in their last places; below its batch a
+step is the ops', bit for bit."""
 import numpy as np
 import pytest
 
@@ -28,12 +29,18 @@ def chain(links, kinds, g):
 R, P, F = abi.JOINT_REVOLUTE, abi.JOINT_PRISMATIC, abi.JOINT_FIXED
 
 
+def fewest(links):
+    """The batch from which a chain of so many links is a lane an environment."""
+    return 64 if links <= 6 else 256 * (links - 6) + 1
+
+
 @pytest.mark.parametrize("links,kinds", [(1, (R,)), (1, (P,)), (2, (F, R)), (5, (P, R)), (7, (R, P, F)), (8, (F, R, R, R, R, R, R, R)), (8, (R,)), (8, (R, F, P))])
 @pytest.mark.parametrize("E,wrench", [(64, True), (65, False), (333, True)])
 def test_a_chain_steps_like_the_ops_and_as_near_the_double_step(oracle_py, device, links, kinds, E, wrench):
-    """Two steps.  A field of the one-lane walk is within single precision's rounding over eight links of the general kernels' (they
-    differ in fused products and the order of sums: 1e-5 of the field's norm, ten times what is seen), and no further than 1.5 times
-    as far from the double-precision step, or under 5e-7 of the norm, where single values' last places decide."""
+    """Two steps, from the fewest environments on.  A field of the one-lane walk is within single precision's rounding over eight links of
+    the general kernels' (they differ in fused products and the order of sums: 1e-5 of the field's norm, ten times what is seen), and no
+    further than 1.5 times as far from the double-precision step, or under 5e-7 of the norm, where single values' last places decide."""
+    E = E - 64 + fewest(links)
     g = np.random.default_rng(10 * links + len(kinds))
     t = chain(links, kinds, g)
     jointed = np.array([link["joint_type"] != F for link in t.links])
@@ -62,6 +69,7 @@ def test_a_chain_steps_like_the_ops_and_as_near_the_double_step(oracle_py, devic
         out.append({name: w.download(name).astype(np.float64).reshape(E, -1) for name in FIELDS if kind != "double" or name not in ("m_factor", "body_pose")})
         w.close()
     ops, step, double = out
+    assert links < 5 or any(not np.array_equal(step[name], ops[name]) for name in FIELDS)   # the one-lane walk's
     assert np.abs(ops["articulation_qdd"]).max() > 0.1 and np.isfinite(step["link_pose"]).all()
     for name in FIELDS:
         assert relative_error(step[name], ops[name]) <= 1e-5, (name, relative_error(step[name], ops[name]))
@@ -71,11 +79,39 @@ def test_a_chain_steps_like_the_ops_and_as_near_the_double_step(oracle_py, devic
             assert mine <= max(1.5 * general, 5e-7), (name, mine, general)
 
 
+@pytest.mark.parametrize("links,E", [(1, 63), (6, 63), (7, 64), (7, 256), (8, 512)])
+def test_below_its_batch_a_step_is_the_ops(device, links, E):
+    """The general kernels in one launch and one by one, and the environments of a smaller batch among a larger's."""
+    t = chain(links, (R, P, R), np.random.default_rng(links))
+    g = np.random.default_rng(E)
+    state = {name: g.normal(0.0, 1.0, (E, links)).astype(np.float32) for name in ("q", "qdot", "tau")}
+    base = np.zeros((E, 7), np.float32)
+    base[:, 3] = 1.0
+    state.update(base_pose=base, root_twist=np.zeros((E, 6), np.float32))
+    out = []
+    for kind, envs in (("ops", E), ("step", E), ("step", 17)):
+        w = nk.World(device, t, abi.world_desc(envs, 1.0 / 240.0))
+        w.set_state({name: v[:envs] for name, v in state.items()})
+        for _ in range(2):
+            if kind == "ops":
+                for op in OPS:
+                    w.op(op)
+            else:
+                w.step()
+        w.synchronize()
+        out.append({name: w.download(name).reshape(envs, -1) for name in FIELDS})
+        w.close()
+    for name in FIELDS:
+        assert np.array_equal(out[0][name].view(np.uint8), out[1][name].view(np.uint8)), name
+        assert np.array_equal(out[2][name].view(np.uint8), out[1][name][:17].view(np.uint8)), name
+
+
 @pytest.mark.parametrize("kinds", [(R, F, P, R, F), (F, P, R, F, R, R, P, F)])
 def test_a_coordinate_counts_where_its_joint_has_a_use_for_it(device, kinds):
     """A fixed link's coordinate that is not finite reaches its own word and nothing else; a joint's reaches what it reaches in the
     general kernels' ops."""
-    E, links = 70, len(kinds)
+    links = len(kinds)
+    E = fewest(links) + 6
     g = np.random.default_rng(links)
     t = chain(links, kinds, g)
     jointed = np.array([kind != F for kind in kinds])
