@@ -323,8 +323,8 @@ enum HeadField : uint32_t {
     hUnitValue = hUnit + (kPaired ? 0 : 1),   // its Jacobian entry there
     hFieldCount = hUnitValue + 1
 };
-// (paired: a contact head's curvature is in its lane's registers, and no head is a unit head: neither has words, nothing reads or
-// writes them)
+// (paired: a contact head's curvature is in its lane's registers, and no head is a unit head: neither has words, and what reads
+// or writes them stands behind kPaired or Tile::units)
 // Fields that share their words: the rows' sources are done with when a head's residual and base are first written, and an
 // assembly's impulses when the next steps are.
 constexpr uint32_t hSourceA = hRes, hSourceB = hBase, hF = hStep;
@@ -3115,10 +3115,12 @@ environment:
             if (stage) c.U(hRow, h) = 3u * (staged + uint32_t(__popcll(mask & ((uint64_t{1} << lane) - 1ull))));   // no more than h
             staged += uint32_t(__popcll(mask));
             if (mask != 0ull) staged_end = base + uint32_t(64 - __builtin_clzll(mask));
-            any_unit = any_unit || (h < heads && c.U(hUnit, h) != kInvalid);
-            // heads that need a response of their own: staged ones, and unit heads whose entry is not +-1
-            const uint64_t own = __ballot(h < heads && (c.U(hUnit, h) == kInvalid || fabsf(c.F(hUnitValue, h)) != 1.0f));
-            if (own != 0ull) individual_end = base + uint32_t(64 - __builtin_clzll(own));
+            if constexpr (!kPaired) {
+                any_unit = any_unit || (h < heads && c.U(hUnit, h) != kInvalid);
+                // heads that need a response of their own: staged ones, and unit heads whose entry is not +-1
+                const uint64_t own = __ballot(h < heads && (c.U(hUnit, h) == kInvalid || fabsf(c.F(hUnitValue, h)) != 1.0f));
+                if (own != 0ull) individual_end = base + uint32_t(64 - __builtin_clzll(own));
+            }
         }
         c.units = !kContactsOnly && __any(any_unit) && cap > staged_cap;   // the lists have room only when the world has joint heads
         c.staged_end = staged_end;
@@ -3393,8 +3395,8 @@ environment:
                     apart[t] = __float_as_uint(row[11]) != __float_as_uint(row[19]);
                 }
                 second[t] = artic_b && !artic_a;
-                const uint32_t first = c.U(hRow, h), unit = c.U(hUnit, h);
-                const float unit_value = c.F(hUnitValue, h);
+                const uint32_t first = c.U(hRow, h), unit = kPaired ? kInvalid : c.U(hUnit, h);
+                const float unit_value = kPaired ? 0.0f : c.F(hUnitValue, h);
                 skip[t] = share_units && unit != kInvalid && fabsf(unit_value) == 1.0f && !apart[t];
                 if (coordinate && (artic_a || artic_b) && !apart[t] && !skip[t]) {
                     if (W > kTwoWaveWidth && c.from_links) {   // the first row's entry: the coordinate's axis against the row's wrench
