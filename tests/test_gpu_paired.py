@@ -1,4 +1,4 @@
-"""A step's result is the environment's own, whatever kernels and launches its batch takes: wide blocks two a SIMD, launches of as
+"""An environment's solve and its rows are its own, whatever kernels and launches its batch takes: wide blocks two a SIMD, launches of as
 many blocks as the machine holds, row assemblies of eight environments a wavefront."""
 import numpy as np
 import pytest
@@ -8,6 +8,7 @@ from trees import tree_case
 
 abi = nk.abi
 pytestmark = pytest.mark.gpu
+SOLVER_FAILURE = 1 << 13
 FIELDS = ("q", "qdot", "link_velocity", "lambda", "vbd_velocity_sweep_count", "env_status", "solver_residual")
 
 
@@ -15,8 +16,9 @@ def repeated(state, E):
     return {name: np.ascontiguousarray(np.asarray(v)[np.arange(E) % len(v)]) for name, v in state.items()}
 
 
-def batches_agree(device, template, desc_of, state, small, large, steps=2, fields=FIELDS):
-    """The environments of a large batch, the small one's over and over, step as the small one's do, bit for bit."""
+def batches_agree(device, template, desc_of, state, small, large, steps=2, fields=FIELDS, failing=None, width=None):
+    """The environments of a large batch, the small one's over and over, step as the small one's do, bit for bit; those whose solve
+    fails (`failing`, of the small batch) are flagged, and what becomes of them is nobody's concern."""
     few, many = nk.World(device, template, desc_of(small)), nk.World(device, template, desc_of(large))
     few.set_state(state)
     many.set_state(repeated(state, large))
@@ -28,7 +30,11 @@ def batches_agree(device, template, desc_of, state, small, large, steps=2, field
     assert (few.download("contact_count") > 0).any()
     for name in fields:
         a, b = few.download(name).reshape(small, -1), many.download(name).reshape(large, -1)
-        assert np.array_equal(b.view(np.uint8), a.view(np.uint8)[np.arange(large) % small]), name
+        kept = np.ones(small, bool) if failing is None else ~failing
+        assert np.array_equal(b.view(np.uint8)[np.resize(kept, large)], a.view(np.uint8)[np.arange(large) % small][np.resize(kept, large)]), name
+        if name == "env_status":
+            assert np.array_equal((b[:, 0] & SOLVER_FAILURE) != 0, np.resize(~kept, large))
+    assert width is None or many.info.solver_width == width
     blocks = few.info.solver_blocks_per_cu, many.info.solver_blocks_per_cu
     few.close()
     many.close()
@@ -78,16 +84,43 @@ def test_ropes_two_a_simd_step_as_one_a_simd(device, large, held):
     assert blocks == (4, held)
 
 
-@pytest.mark.parametrize("index,driven,large", [(2, False, 2049), (2, False, 6144 + 1), (3, False, 2600), (3, True, 1900)])
-def test_environments_past_the_blocks_held_step_as_the_first(device, index, driven, large):
-    """Two-wave, dense and general kernels with more environments than blocks: the ones that wait in the queue, one at the least."""
+def with_dry_friction(template):
+    for link in template.links:
+        if link["joint_type"] == abi.JOINT_REVOLUTE:
+            link["frictionloss"] = 0.1
+    return template
+
+
+# Blocks with joint rows (general), blocks whose sweeps are narrower than their coordinates (reduced) and batches of 6144 on (dense) of more
+# environments than the machine holds blocks: the launches that have a queue.  The second number is the width of the sweeps.
+@pytest.mark.parametrize("index,width,driven,large", [(2, 18, True, 2100), (2, 18, False, 6145), (3, 20, False, 2600), (3, 36, True, 2600)])
+@pytest.mark.parametrize("sick", [False, True])
+def test_environments_past_the_blocks_held_step_as_the_first(device, index, width, driven, large, sick):
+    """Those that wait in the queue, one at the least; also behind environments whose velocity is no number, which leave their block's
+    LDS to the next as the failed solve left it."""
     cfg = nk.synthetic.config(index, 150)
-    template = cfg.template
-    if driven:
-        for link in template.links:
-            if link["joint_type"] == abi.JOINT_REVOLUTE:
-                link["frictionloss"] = 0.1
-    batches_agree(device, template, lambda E: abi.world_desc(E, cfg.dt, vel_iters=cfg.vel_iters), cfg.state(), 150, large, steps=3)
+    template, state = with_dry_friction(cfg.template) if driven else cfg.template, cfg.state()
+    failing = np.arange(150) % 4 == 1
+    if sick:
+        state["root_twist"] = np.where(failing[:, None], np.float32(np.nan), state["root_twist"]).astype(np.float32)
+    blocks = batches_agree(device, template, lambda E: abi.world_desc(E, cfg.dt, vel_iters=cfg.vel_iters), state, 150, large, steps=1 if sick else 3,
+                           failing=failing if sick else None, width=width)
+    assert large > 256 * blocks[1]
+
+
+@pytest.mark.parametrize("dof,width,floating,limb_joints,sphere_limbs,driven,large", [
+    (3, 3, False, 7, None, True, 2100), (7, 7, False, 3, None, True, 2100), (11, 11, True, 3, None, True, 2100), (14, 14, True, 3, None, True, 2100),
+    (23, 23, True, 3, None, True, 2100), (26, 26, True, 3, None, True, 2100), (32, 32, True, 3, None, True, 2100),
+    (24, 12, True, 3, 2, False, 2100), (27, 16, True, 3, 2, False, 2100), (32, 16, True, 5, 2, False, 2100), (40, 20, True, 7, 2, False, 2100),
+    (44, 24, True, 7, 2, False, 2100), (48, 24, True, 7, 2, False, 2100), (51, 28, True, 7, 3, False, 2100), (56, 28, True, 7, 3, False, 2100),
+    (60, 32, True, 7, 3, False, 2100), (64, 32, True, 7, 3, False, 2100), (24, 12, True, 3, 2, False, 6200), (8, 8, False, 3, None, False, 6200),
+])
+def test_trees_past_the_blocks_held_step_as_the_first(oracle_py, device, dof, width, floating, limb_joints, sphere_limbs, driven, large):
+    """The same at the padded widths that the configurations leave out."""
+    tree, _, state = tree_case(oracle_py, dof, floating, True, seed=7 * dof, E=48, limb_joints=limb_joints, sphere_limbs=sphere_limbs)
+    template = with_dry_friction(tree.template) if driven else tree.template
+    blocks = batches_agree(device, template, lambda E: abi.world_desc(E, 1.0 / 240.0, vel_iters=6), state, 48, large, width=width)
+    assert large > 256 * blocks[1]
 
 
 @pytest.mark.parametrize("large", [2048, 2051])
