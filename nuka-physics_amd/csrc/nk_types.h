@@ -86,6 +86,8 @@ struct ModelView {
     // 1: the template's one link is a free rigid body, stepped by the rigid-body ops (ops_rigid.hip): its six coordinates
     // are its linear velocity and its angular velocity about the centre of mass, in world axes
     uint32_t free_body;
+    // 1: link l hangs from link l - 1 by a hinge, a slider or nothing that moves, the first from the ground (0: not known)
+    uint32_t serial_chain;
     const uint8_t* joint_type;
     const uint32_t* parent_link;
     const float* joint_axis;

@@ -1194,10 +1194,10 @@ Status OpPosesAndDynamics(const ModelView& m, const DataView& d, const Articulat
     const DynamicsEntry* entry = DynamicsEntryOf(m, *dynamics);
     return entry == nullptr ? Status::InvalidArgument : LaunchDynamics(m, d, *dynamics, *entry, true, StepTail{}, stream);
 }
-// Serial chains go a lane an environment (ChainStepKernel): as many depths as links, parents ahead of their children (the cook
-// refuses others), is link l on link l - 1; no floating base.
+// Serial chains go a lane an environment (ChainStepKernel), where the host says that the links are one (a chain's depths alone
+// do not say that link l hangs from link l - 1)
 static bool ChainServed(const ModelView& m, const ArticulationDynamicsParams& dynamics) {
-    return m.links_per_env <= kChainLinks && m.max_depth + 1u == m.links_per_env && m.floating_root == 0u && m.max_dof <= kChainLinks && dynamics.articulation_count >= ChainFrom(m.links_per_env);
+    return m.serial_chain != 0u && m.links_per_env <= kChainLinks && m.max_dof <= kChainLinks && dynamics.articulation_count >= ChainFrom(m.links_per_env);
 }
 // The step's tail in the dynamics' launch, up to five workgroups a compute unit: past that the shorter kernels fill the chip
 // better than one whose workgroups hold the dynamics' LDS to the end (a step of 64 arms 32.8 -> 30.6 us, 1000 37.8 -> 35.4, 8000

@@ -347,9 +347,11 @@ void Cook(const nuka_template_desc_t& d, HostModel* out) {
         for (uint32_t k = 0u; k < nv; ++k) if ((mask >> k) & 1ull) c.contact_dof_end = std::max(c.contact_dof_end, k + 1u);
     }
     c.rows_from_links = link_pairs ? 0u : 1u;
+    c.serial_chain = 1u;
     for (uint32_t l = 0u; l < nl; ++l) {
         const uint8_t type = m.joint_type[l];
         if (!(type == kRevolute || type == kPrismatic || type == kFixed || (type == kFloatingBase && l == 0u))) c.rows_from_links = 0u;
+        if (!(type == kRevolute || type == kPrismatic || type == kFixed) || m.parent_link[l] != (l == 0u ? kInvalid : l - 1u)) c.serial_chain = 0u;
     }
     c.excluded_pair_count = uint32_t(m.excluded_pairs.size());
     // rows whose type and affinity masks are both empty pass the filter with no partner (shape_kind.hpp:26-33): the pair
@@ -1459,7 +1461,7 @@ int nuka_hip_model_view_set_count(nuka_phi_model_view* model, const char* name, 
     COUNT(links_per_env) COUNT(bodies_per_env) COUNT(dof) COUNT(max_dof) COUNT(max_depth) COUNT(contact_slots) COUNT(rows_per_env)
     COUNT(contact_rows_per_env) COUNT(profile_count) COUNT(floating_root) COUNT(max_points_per_slot) COUNT(excluded_pair_count)
     COUNT(sweep_passes) COUNT(pairable_count) COUNT(contact_dof_end) COUNT(rows_from_links) COUNT(joint_limit_rows) COUNT(joint_friction_rows) COUNT(joint_drive_rows)
-    COUNT(drive_mode) COUNT(any_mujoco) COUNT(contact_cone) COUNT(integrator) COUNT(free_body)
+    COUNT(drive_mode) COUNT(any_mujoco) COUNT(contact_cone) COUNT(integrator) COUNT(free_body) COUNT(serial_chain)
 #undef COUNT
     return -1;
 }
