@@ -12,15 +12,16 @@ FIELDS = ("m", "m_factor", "articulation_bias", "articulation_qdd", "qdot", "qdd
 OPS = ("FkWorldPoses", "ApplyDrives", "ArticulationDynamics", "IntegrateVelocity", "IntegratePosition", "FkWorldPoses", "FkLinkVelocities", "SyncLinkBodyPose")
 
 
-def chain(links, kinds, g):
-    """`links` links one on the other, the joints' types in turn `kinds`; frames, axes and inertias in general position."""
+def chain(links, kinds, g, flat=None):
+    """`links` links one on the other, the joints' types in turn `kinds`; frames, axes, inertias and the joints' own terms in general
+    position.  Link `flat` has an axis of zeros."""
     t = abi.Template()
     for k in range(links):
         rotation = g.normal(size=4)
         kind = kinds[k % len(kinds)]
-        t.add_link(kind, k - 1 if k else None, axis=tuple(g.normal(size=3)), local_pos=tuple(g.normal(0.0, 0.15, 3)), local_rot=tuple(rotation / np.linalg.norm(rotation)),
-                   mass=g.uniform(0.2, 2.0), diag_inertia=tuple(g.uniform(2e-3, 2e-2, 3)), com=tuple(g.normal(0.0, 0.05, 3)), damping=0.1, armature=0.02,
-                   stiffness=0.5)
+        t.add_link(kind, k - 1 if k else None, axis=(0, 0, 0) if k == flat else tuple(g.normal(size=3)), local_pos=tuple(g.normal(0.0, 0.15, 3)), local_rot=tuple(rotation / np.linalg.norm(rotation)),
+                   mass=g.uniform(0.2, 2.0), diag_inertia=tuple(g.uniform(2e-3, 2e-2, 3)), com=tuple(g.normal(0.0, 0.05, 3)), damping=g.uniform(0.05, 0.3),
+                   armature=g.uniform(0.01, 0.05), stiffness=g.uniform(0.2, 1.0), spring_ref=g.normal(0.0, 0.5))
     for link in range(links):
         t.add_body(abi.ROLE_LINK_BODY, link=link, kind=abi.SHAPE_NONE, contype=0, conaffinity=0)
     return t
@@ -38,22 +39,25 @@ def fewest(links):
 @pytest.mark.parametrize("E,wrench", [(64, True), (65, False), (333, True)])
 def test_a_chain_steps_like_the_ops_and_as_near_the_double_step(oracle_py, device, links, kinds, E, wrench):
     """Two steps, from the fewest environments on.  A field of the one-lane walk is within single precision's rounding over eight links of
-    the general kernels' (they differ in fused products and the order of sums: 1e-5 of the field's norm, ten times what is seen), and no
-    further than 1.5 times as far from the double-precision step, or under 5e-7 of the norm, where single values' last places decide."""
+    the general kernels' (they differ in fused products and the order of sums: 1e-5 of the field's norm, ten times what is seen; what
+    follows from the accelerations within what two factorings of n coordinates may differ by, 2 n cond(M) 2^-24, where that is more), and
+    no further than 1.5 times as far from the double-precision step, or under 5e-7 of the norm, where single values' last places decide."""
     E = E - 64 + fewest(links)
     g = np.random.default_rng(10 * links + len(kinds))
-    t = chain(links, kinds, g)
+    t = chain(links, kinds, g, flat=3 if links == 5 else None)
     jointed = np.array([link["joint_type"] != F for link in t.links])
     state = {name: (g.normal(0.0, sigma, (E, links)) * jointed).astype(np.float32) for name, sigma in (("q", 1.0), ("qdot", 1.0), ("tau", 2.0))}
-    base = np.zeros((E, 7), np.float32)
-    base[:, 3] = 1.0
+    base = g.normal(size=(E, 7)).astype(np.float32)   # (of no concern to a root that stands still)
+    base[:, 3:] /= np.linalg.norm(base[:, 3:], axis=1, keepdims=True)
     state.update(base_pose=base, root_twist=np.zeros((E, 6), np.float32))
+    gravity_force = g.normal(0.0, 1.0, (E, links)).astype(np.float32)
     pushes = g.normal(0.0, 1.0, (E, links, 6)).astype(np.float32) * (g.random((E, links, 1)) < 0.2)
     desc = abi.world_desc(E, 1.0 / 240.0)
     worlds = [nk.World(device, t, desc), nk.World(device, t, desc), oracle_py.OracleWorld(t, desc, threads=4, double=True)]
     out = []
     for kind, w in zip(("ops", "step", "double"), worlds):
         w.set_state(state)
+        w.upload("joint_gravity_force", gravity_force)
         for _ in range(2):
             if wrench:
                 w.upload("link_wrench", pushes)
@@ -71,8 +75,11 @@ def test_a_chain_steps_like_the_ops_and_as_near_the_double_step(oracle_py, devic
     ops, step, double = out
     assert links < 5 or any(not np.array_equal(step[name], ops[name]) for name in FIELDS)   # the one-lane walk's
     assert np.abs(ops["articulation_qdd"]).max() > 0.1 and np.isfinite(step["link_pose"]).all()
+    n = int(jointed.sum())
+    solved = 2 * n * np.linalg.cond(double["m"].reshape(E, n, n)).max() * 2.0 ** -24
     for name in FIELDS:
-        assert relative_error(step[name], ops[name]) <= 1e-5, (name, relative_error(step[name], ops[name]))
+        bound = 1e-5 if name in ("m", "m_factor", "articulation_bias") else max(1e-5, solved)
+        assert relative_error(step[name], ops[name]) <= bound, (name, relative_error(step[name], ops[name]), bound)
         if name in double:
             scale = np.linalg.norm(double[name]) + 1e-30
             mine, general = np.linalg.norm(step[name] - double[name]) / scale, np.linalg.norm(ops[name] - double[name]) / scale

@@ -16,7 +16,7 @@ def repeated(state, E):
     return {name: np.ascontiguousarray(np.asarray(v)[np.arange(E) % len(v)]) for name, v in state.items()}
 
 
-def batches_agree(device, template, desc_of, state, small, large, steps=2, fields=FIELDS, failing=None, width=None):
+def batches_agree(device, template, desc_of, state, small, large, steps=2, fields=FIELDS, failing=None, width=None, slots=False):
     """The environments of a large batch, the small one's over and over, step as the small one's do, bit for bit; those whose solve
     fails (`failing`, of the small batch) are flagged, and what becomes of them is nobody's concern."""
     few, many = nk.World(device, template, desc_of(small)), nk.World(device, template, desc_of(large))
@@ -36,9 +36,10 @@ def batches_agree(device, template, desc_of, state, small, large, steps=2, field
             assert np.array_equal((b[:, 0] & SOLVER_FAILURE) != 0, np.resize(~kept, large))
     assert width is None or many.info.solver_width == width
     blocks = few.info.solver_blocks_per_cu, many.info.solver_blocks_per_cu
+    held = few.info.contact_slots_per_env
     few.close()
     many.close()
-    return blocks
+    return held if slots else blocks
 
 
 @pytest.mark.parametrize("dof,floating,branched,limb_joints", [
@@ -135,3 +136,42 @@ def test_boxes_whose_rows_are_assembled_eight_a_wavefront_step_as_alone(device, 
     batches_agree(device, cfg.template, lambda E: abi.world_desc(E, cfg.dt, vel_iters=cfg.vel_iters), state, 70, large, steps=4,
                   fields=("lambda", "chain_jacobian", "chain_jacobian_b", "row_penetration", "row_cj_point", "ucontact_count", "row_count",
                           "contact_material", "body_linear_velocity", "body_angular_velocity", "base_pose", "env_status", "qdot_flat"))
+
+
+ROW_FIELDS = ("lambda", "chain_jacobian", "chain_jacobian_b", "row_penetration", "row_cj_point", "row_cj_point_b", "row_cj_link", "ucontact_count", "row_count",
+              "contact_material", "env_status", "qdot_flat", "q", "qdot", "link_velocity", "contact_row_extent")
+
+
+@pytest.mark.parametrize("dof,floating,branched,limb_joints,sphere_pairs", [
+    (8, False, True, 2, False), (7, True, False, 7, False), (6, False, False, 7, False), (2, False, False, 2, False), (4, False, True, 2, True), (8, True, True, 1, True),
+])
+def test_trees_whose_rows_are_assembled_eight_a_wavefront_step_as_alone(oracle_py, device, dof, floating, branched, limb_joints, sphere_pairs):
+    """One point a slot, up to eight slots; spheres of different limbs too, whose rows have the articulation on both sides."""
+    small = 70
+    tree, _, state = tree_case(oracle_py, dof, floating, branched, seed=11 * dof, E=small, limb_joints=limb_joints, sphere_pairs=sphere_pairs)
+    slots = batches_agree(device, tree.template, lambda E: abi.world_desc(E, 1.0 / 240.0, vel_iters=6, contact_margin=0.1), state, small, 2051, steps=3, fields=ROW_FIELDS,
+                          slots=True)
+    assert 1 <= slots <= 8
+
+
+def test_two_boxes_on_a_tree_whose_rows_are_assembled_eight_a_wavefront_step_as_alone(device):
+    """Two slots of four points each, a root and the link on its hinge: every lane a place."""
+    small, g = 70, np.random.default_rng(3)
+    t = abi.Template()
+    t.add_link(abi.JOINT_FLOATING, None, mass=3.0, diag_inertia=(0.03, 0.04, 0.05))
+    t.add_link(abi.JOINT_REVOLUTE, 0, axis=(0, 1, 0), local_pos=(0.35, 0, 0), mass=1.0, diag_inertia=(0.01, 0.01, 0.01), armature=0.02)
+    profile = t.add_profile(0.6)
+    t.add_body(abi.ROLE_STATIC, kind=abi.SHAPE_PLANE, contype=2, conaffinity=1, profile=profile)
+    for link, half in ((0, (0.15, 0.1, 0.1)), (1, (0.1, 0.1, 0.1))):
+        t.add_body(abi.ROLE_LINK_BODY, link=link, kind=abi.SHAPE_NONE, contype=0, conaffinity=0)
+        t.add_body(abi.ROLE_PROXY, link=link, kind=abi.SHAPE_BOX, params=(*half, 0), contype=1, conaffinity=2, profile=profile)
+    t.max_contacts_per_env = 2
+    base = np.zeros((small, 7), np.float32)
+    base[:, 2] = 0.1 + g.uniform(-0.004, 0.02, small)
+    base[:, 3] = 1.0
+    base[:, 4:] = 0.5 * g.normal(0.0, 0.02, (small, 3))
+    base[:, 3:] /= np.linalg.norm(base[:, 3:], axis=1, keepdims=True)
+    state = dict(q=np.stack([np.zeros(small), g.normal(0.0, 0.05, small)], 1).astype(np.float32), qdot=np.zeros((small, 2), np.float32), tau=np.zeros((small, 2), np.float32),
+                 base_pose=base, root_twist=g.normal(0.0, 0.3, (small, 6)).astype(np.float32))
+    slots = batches_agree(device, t, lambda E: abi.world_desc(E, 1.0 / 240.0, vel_iters=8, contact_margin=0.02), state, small, 2051, steps=4, fields=ROW_FIELDS, slots=True)
+    assert slots == 2
