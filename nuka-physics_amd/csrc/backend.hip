@@ -259,7 +259,7 @@ uint8_t BeSynchronize(nuka_phi_backend* b, nuka_phi_execution_error* error) {
 
 // The kernels of a captured graph of one or two, in their order, with the parameters the graph keeps (they live as long as it
 // does): such a plan is executed by launching them.  A graph's launch leaves the stream idle for some 8 us, whatever it holds,
-// a kernel's does not (a step of 64 arms, one kernel, 31.1 -> 25.5 us; 20011, 40.7 -> 35.2).  From three kernels on the gain is
+// a kernel's does not (a step of 64 arms, one kernel, 30.5 -> 24.7 us; 20011, 41.0 -> 35.7).  From three kernels on the gain is
 // the same 5 us and the host's work is more, which shows where it starts a step on an idle device (1000 servo-driven quadrupeds,
 // four steps of eleven kernels, 1815 us by the graph and 1845 kernel by kernel).
 uint32_t DirectKernels(hipGraph_t graph, hipKernelNodeParams (&kernels)[2]) {
@@ -300,18 +300,19 @@ Plan* CreatePlan(Backend* be, const ModelView& model, const DataView& data, cons
         Fail(error, status != Status::Ok ? status : Status::Failed, failed, int(e), "plan_create: capture failed");
         return nullptr;
     }
-    hipGraphExec_t exec = nullptr;
-    e = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
+    size_t nodes = 0u;
+    (void)hipGraphGetNodes(graph, nullptr, &nodes);
+    auto* plan = new Plan{graph, nullptr, nodes, n_calls, {}, 0u};
+    plan->direct_count = DirectKernels(graph, plan->direct);
+    (void)hipGetLastError();
+    if (plan->direct_count != 0u) return plan;   // (no exec, for nothing would launch it)
+    e = hipGraphInstantiate(&plan->exec, graph, nullptr, nullptr, 0);
     if (e != hipSuccess) {
         (void)hipGraphDestroy(graph);
+        delete plan;
         Fail(error, Status::Failed, uint16_t(NkOp::Count), int(e), hipGetErrorString(e));
         return nullptr;
     }
-    size_t nodes = 0u;
-    (void)hipGraphGetNodes(graph, nullptr, &nodes);
-    auto* plan = new Plan{graph, exec, nodes, n_calls, {}, 0u};
-    plan->direct_count = DirectKernels(graph, plan->direct);
-    (void)hipGetLastError();
     return plan;
 }
 nuka_phi_plan* BePlanCreate(nuka_phi_backend* b, const nuka_phi_model_view* m, const nuka_phi_data_view* d,
@@ -351,7 +352,7 @@ uint8_t BePlanExecuteRepeated(nuka_phi_backend* b, nuka_phi_plan* p, uint32_t co
 void BePlanFree(nuka_phi_backend*, nuka_phi_plan* p) {
     auto* plan = reinterpret_cast<Plan*>(p);
     if (plan == nullptr) return;
-    (void)hipGraphExecDestroy(plan->exec);
+    if (plan->exec != nullptr) (void)hipGraphExecDestroy(plan->exec);
     (void)hipGraphDestroy(plan->graph);
     delete plan;
 }
