@@ -430,8 +430,12 @@ Status OpBlockDescentSolve(const ModelView& m, const DataView& d, const void* pa
     // neither reduced nor dense, and those under the elliptic cone, have no kernel for it (4096 quadrupeds 466 and 466, 531 -> 521 in turn; under
     // the cone 595 -> 592), and paired blocks lose by it: eight that start together are better there than eight at any
     // time (8192 ropes 9.87 ms and 10.06).  Nor where the points send environments to several launches, whose blocks are mostly over at once.
+    // From a third more environments than blocks on: of fewer most blocks take none from it, and the kernel that has it is a little the
+    // slower (twenty trees of every width that has one, as many blocks as are held and a queue against a block an environment: just past the
+    // blocks held 0.99 to 1.01 of the step, a quarter past them 0.99 to 1.01, half 0.99 to 1.02, three quarters 0.92 to 1.02, twice 0.96 to 1.00,
+    // eight times 0.85 to 0.96).
     const size_t held = kUnits * blocks_per_unit(staged);
-    const bool queued = chosen.queue != nullptr && first_points == 0u && d.solver_queue != nullptr && p->env_count > held;
+    const bool queued = chosen.queue != nullptr && first_points == 0u && d.solver_queue != nullptr && p->env_count > held + held / 3u;
     hipLaunchKernelGGL(queued ? chosen.queue : kernel, dim3(queued ? uint32_t(held) : p->env_count), dim3(solver::kWave), lds_bytes(staged), stream, m, d, *p, staged + joint_heads,
                        staged, queued ? uint32_t(held) : first_points, queued ? kQueued : kInvalid);
     return hipGetLastError() == hipSuccess ? Status::Ok : Status::Failed;

@@ -92,9 +92,9 @@ def with_dry_friction(template):
     return template
 
 
-# Blocks with joint rows (general), blocks whose sweeps are narrower than their coordinates (reduced) and batches of 6144 on (dense) of more
-# environments than the machine holds blocks: the launches that have a queue.  The second number is the width of the sweeps.
-@pytest.mark.parametrize("index,width,driven,large", [(2, 18, True, 2100), (2, 18, False, 6145), (3, 20, False, 2600), (3, 36, True, 2600)])
+# Blocks with joint rows (general), blocks whose sweeps are narrower than their coordinates (reduced) and batches of 6144 on (dense) of over a third
+# more environments than the machine holds blocks: the launches that have a queue.  The second number is the width of the sweeps.
+@pytest.mark.parametrize("index,width,driven,large", [(2, 18, True, 2740), (2, 18, False, 6145), (3, 20, False, 2740), (3, 36, True, 2740)])
 @pytest.mark.parametrize("sick", [False, True])
 def test_environments_past_the_blocks_held_step_as_the_first(device, index, width, driven, large, sick):
     """Those that wait in the queue, one at the least; also behind environments whose velocity is no number, which leave their block's
@@ -106,22 +106,22 @@ def test_environments_past_the_blocks_held_step_as_the_first(device, index, widt
         state["root_twist"] = np.where(failing[:, None], np.float32(np.nan), state["root_twist"]).astype(np.float32)
     blocks = batches_agree(device, template, lambda E: abi.world_desc(E, cfg.dt, vel_iters=cfg.vel_iters), state, 150, large, steps=1 if sick else 3,
                            failing=failing if sick else None, width=width)
-    assert large > 256 * blocks[1]
+    assert large > 256 * blocks[1] * 4 // 3   # (the queue's)
 
 
 @pytest.mark.parametrize("dof,width,floating,limb_joints,sphere_limbs,driven,large", [
-    (3, 3, False, 7, None, True, 2100), (7, 7, False, 3, None, True, 2100), (11, 11, True, 3, None, True, 2100), (14, 14, True, 3, None, True, 2100),
-    (23, 23, True, 3, None, True, 2100), (26, 26, True, 3, None, True, 2100), (32, 32, True, 3, None, True, 2100),
-    (24, 12, True, 3, 2, False, 2100), (27, 16, True, 3, 2, False, 2100), (32, 16, True, 5, 2, False, 2100), (40, 20, True, 7, 2, False, 2100),
-    (44, 24, True, 7, 2, False, 2100), (48, 24, True, 7, 2, False, 2100), (51, 28, True, 7, 3, False, 2100), (56, 28, True, 7, 3, False, 2100),
-    (60, 32, True, 7, 3, False, 2100), (64, 32, True, 7, 3, False, 2100), (24, 12, True, 3, 2, False, 6200), (8, 8, False, 3, None, False, 6200),
+    (3, 3, False, 7, None, True, 2740), (7, 7, False, 3, None, True, 2740), (11, 11, True, 3, None, True, 2740), (14, 14, True, 3, None, True, 2740),
+    (23, 23, True, 3, None, True, 2740), (26, 26, True, 3, None, True, 2740), (32, 32, True, 3, None, True, 2740),
+    (24, 12, True, 3, 2, False, 2740), (27, 16, True, 3, 2, False, 2740), (32, 16, True, 5, 2, False, 2740), (40, 20, True, 7, 2, False, 2740),
+    (44, 24, True, 7, 2, False, 2740), (48, 24, True, 7, 2, False, 2740), (51, 28, True, 7, 3, False, 2740), (56, 28, True, 7, 3, False, 2740),
+    (60, 32, True, 7, 3, False, 2740), (64, 32, True, 7, 3, False, 2740), (24, 12, True, 3, 2, False, 6200), (8, 8, False, 3, None, False, 6200),
 ])
 def test_trees_past_the_blocks_held_step_as_the_first(oracle_py, device, dof, width, floating, limb_joints, sphere_limbs, driven, large):
     """The same at the padded widths that the configurations leave out."""
     tree, _, state = tree_case(oracle_py, dof, floating, True, seed=7 * dof, E=48, limb_joints=limb_joints, sphere_limbs=sphere_limbs)
     template = with_dry_friction(tree.template) if driven else tree.template
     blocks = batches_agree(device, template, lambda E: abi.world_desc(E, 1.0 / 240.0, vel_iters=6), state, 48, large, width=width)
-    assert large > 256 * blocks[1]
+    assert large > 256 * blocks[1] * 4 // 3   # (the queue's)
 
 
 @pytest.mark.parametrize("large", [2048, 2051])
