@@ -1035,6 +1035,7 @@ __global__ void __launch_bounds__(kWave) FkLinkVelocitiesKernel(ModelView m, Dat
 // `G` lanes of two wavefronts an environment: four kernels that each take about the time of a launch become one, running
 // the same device code in the same order (IntegratePosition, FkWorldPoses, FkLinkVelocities, SyncLinkBodyPose).  A plan
 // takes this route when its op list holds the four in a row (backend.hip); an op dispatched by itself runs its own kernel.
+// (The whole step of a serial chain may be other code, with other last places: ops_chain_kernel.h.)
 struct StepTail { IntegratePositionParams integrate; uint32_t runs, sync_bodies; };
 template <int G>
 __device__ __forceinline__ void step_tail_of_block(const ModelView& m, const DataView& d, const StepTail& t, uint32_t env_count, float* lds) {

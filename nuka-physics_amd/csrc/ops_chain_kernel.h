@@ -14,6 +14,7 @@
 // compute unit that LDS holds.  Products and sums are fused, transforms applied by their rotation and offset
 // (X = [[E, 0], [-E t x, E]]) and inertias kept symmetric, half the instructions of the general kernel's products; the results
 // differ from its in their last places and lie as near a double-precision step.
+// Eight: 78 KB of LDS, two workgroups a compute unit; nine links take 86 KB, one.
 constexpr uint32_t kChainLinks = 8u;
 // From so many environments on: the kernel takes as long for one of them as for sixty-four, so that no fewer are worth it, and a longer
 // chain is a longer walk for its one lane while the general kernel's lanes still fill an idle machine (a step, general kernel and this one:

@@ -537,7 +537,9 @@ def test_reset_envs_restores_the_selected_environments_only(device):
 @pytest.mark.parametrize("index,E", [(3, 512), (1, 64), (5, 64)])
 def test_a_plan_steps_bit_for_bit_like_the_ops_one_by_one(device, index, E):
     """A plan may run neighbouring ops as one launch (the four after the solve); whatever it merges, the state after
-    any number of steps must be the state the ops leave when each is dispatched by itself."""
+    any number of steps must be the state that eager stepping leaves, which merges them too, and, where a step is the ops' kernels, the
+    state they leave when each is dispatched by itself (serial chains without rows have a walk of their own from a batch on:
+    test_gpu_chain.py)."""
     cfg = nk.synthetic.config(index, E)
     hashes = []
     fields = {}
