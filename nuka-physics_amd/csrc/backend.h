@@ -13,7 +13,8 @@ void* CreateBackend(int device, void* borrowed_stream);
 hipStream_t BackendStream(void* backend);
 // one launch for the first op of the list, or for the first few where a merged kernel runs them (`served` of them), as in a plan
 Status BackendDispatchNext(void* backend, const ModelView& m, const DataView& d, const nuka_phi_op_call* calls, int n, int* served);
-// plan_create on a world's own views, which have a queue (DataView::solver_queue); a host's, through the seam, have none
+// dispatch and plan_create on a world's own views, which have a queue (DataView::solver_queue); a host's, through the seam, have none
+Status BackendDispatch(void* backend, const ModelView& m, const DataView& d, const nuka_phi_op_call& call);
 nuka_phi_plan* BackendPlanCreate(void* backend, const ModelView& m, const DataView& d, const nuka_phi_op_call* calls, int n, nuka_phi_execution_error* error);
 nuka_phi_buffer_type* BackendDeviceBufferType(void* backend);
 nuka_phi_buffer_type* BackendHostBufferType(void* backend);

@@ -468,6 +468,7 @@ void* CreateBackend(int device, void* borrowed_stream) {
 Status BackendDispatchNext(void* backend, const ModelView& m, const DataView& d, const nuka_phi_op_call* calls, int n, int* served) {
     return DispatchNext(static_cast<Backend*>(backend), m, d, calls, n, served);
 }
+Status BackendDispatch(void* backend, const ModelView& m, const DataView& d, const nuka_phi_op_call& call) { return DispatchOn(static_cast<Backend*>(backend), m, d, call); }
 nuka_phi_plan* BackendPlanCreate(void* backend, const ModelView& m, const DataView& d, const nuka_phi_op_call* calls, int n, nuka_phi_execution_error* error) {
     return reinterpret_cast<nuka_phi_plan*>(CreatePlan(static_cast<Backend*>(backend), m, d, calls, n, error));
 }

@@ -1015,8 +1015,7 @@ nuka_result_t CreateWorld(nuka_device_handle device, const nuka_template_desc_t*
                                                      {uint16_t(NkOp::ReferenceWeights), &w.p_reference_weights}};
             for (const nuka_phi_op_call& call : at_creation) {
                 if (call.op == uint16_t(NkOp::SyncLinkBodyPose) && nb == 0u) continue;
-                const uint8_t status = w.be->dispatch(w.backend, reinterpret_cast<const nuka_phi_model_view*>(&w.model),
-                                                      reinterpret_cast<const nuka_phi_data_view*>(&w.data), &call);
+                const uint8_t status = uint8_t(BackendDispatch(w.device->backend, w.model, w.data, call));
                 if (status != uint8_t(Status::Ok)) return Error(MapStatus(status), "reference weights failed");
             }
             if (w.be->synchronize(w.backend, nullptr) != uint8_t(Status::Ok)) return Error(NUKA_RESULT_DEVICE_ERROR, "device error in the reference weights");
@@ -1346,8 +1345,7 @@ nuka_result_t nuka_world_dispatch_op(nuka_world_handle world, uint16_t op, uint3
     if (op == uint16_t(NkOp::ReferenceWeights)) params = &w->p_reference_weights;
     if (params == nullptr) return Error(NUKA_RESULT_NOT_SUPPORTED, "op is not part of this world's pipeline");
     const nuka_phi_op_call call{op, params};
-    const uint8_t status = w->be->dispatch(w->backend, reinterpret_cast<const nuka_phi_model_view*>(&w->model),
-                                           reinterpret_cast<const nuka_phi_data_view*>(&w->data), &call);
+    const uint8_t status = uint8_t(BackendDispatch(w->device->backend, w->model, w->data, call));
     if (status != uint8_t(Status::Ok)) return Error(MapStatus(status), std::string("dispatch failed: ") + OpName(static_cast<NkOp>(op)));
     return NUKA_RESULT_OK;
 }
@@ -1544,8 +1542,7 @@ nuka_result_t DemandReadout(World& w, const Field& f) {
     if (!wanted || w.contact_readout_demanded || w.model.contact_slots == 0u) return NUKA_RESULT_OK;
     if (w.be->synchronize(w.backend, nullptr) != uint8_t(Status::Ok)) return Error(NUKA_RESULT_DEVICE_ERROR, "device error before the readout");
     const nuka_phi_op_call call{uint16_t(NkOp::ReadoutContactWrench), &w.p_readout_contacts};
-    const uint8_t status = w.be->dispatch(w.backend, reinterpret_cast<const nuka_phi_model_view*>(&w.model),
-                                          reinterpret_cast<const nuka_phi_data_view*>(&w.data), &call);
+    const uint8_t status = uint8_t(BackendDispatch(w.device->backend, w.model, w.data, call));
     if (status != uint8_t(Status::Ok)) return Error(MapStatus(status), "contact readout failed");
     if (w.be->synchronize(w.backend, nullptr) != uint8_t(Status::Ok)) return Error(NUKA_RESULT_DEVICE_ERROR, "device error in the readout");
     w.contact_readout_demanded = true;
@@ -1912,8 +1909,7 @@ nuka_result_t nuka_world_profile_ops(nuka_world_handle world, nuka_checkpoint_ha
         if (from != nullptr && (result = nuka_world_checkpoint_restore(world, from)) != NUKA_RESULT_OK) break;
         w->be->event_record(w->backend, events[0]);
         for (size_t i = 0u; i < n; ++i) {
-            const uint8_t status = w->be->dispatch(w->backend, reinterpret_cast<const nuka_phi_model_view*>(&w->model),
-                                                   reinterpret_cast<const nuka_phi_data_view*>(&w->data), &w->calls[i]);
+            const uint8_t status = uint8_t(BackendDispatch(w->device->backend, w->model, w->data, w->calls[i]));
             if (status != uint8_t(Status::Ok)) { result = Error(MapStatus(status), "profile dispatch failed"); break; }
             w->be->event_record(w->backend, events[i + 1u]);
         }
@@ -2249,8 +2245,7 @@ nuka_result_t nuka_world_forward_kinematics(nuka_world_handle world) {
     const nuka_phi_op_call fk{uint16_t(NkOp::FkWorldPoses), &w->p_fk}, sync{uint16_t(NkOp::SyncLinkBodyPose), &w->p_sync};
     for (const nuka_phi_op_call* call : {&fk, &sync}) {
         if (call == &sync && w->model.bodies_per_env == 0u) break;
-        const uint8_t status = w->be->dispatch(w->backend, reinterpret_cast<const nuka_phi_model_view*>(&w->model),
-                                               reinterpret_cast<const nuka_phi_data_view*>(&w->data), call);
+        const uint8_t status = uint8_t(BackendDispatch(w->device->backend, w->model, w->data, *call));
         if (status != uint8_t(Status::Ok)) return Error(MapStatus(status), std::string("dispatch failed: ") + OpName(static_cast<NkOp>(call->op)));
     }
     return NUKA_RESULT_OK;
